@@ -58,7 +58,9 @@ extern "C" int s3r_compressed_attn_topk(const void* q, const void* k, const void
                 "s3r_compressed_attn_topk: fused selection needs bf16/fp16, head_dim 64, 16-byte aligned tensors; "
                 "pass a scores buffer for other shapes");
   if (!o) return fail(S3R_ERR_UNSUPPORTED, "s3r_compressed_attn_topk: indices without the attention output need the MFMA path");
-  int rc = launch_attn_simple(p, dtype, /*select=*/false, stream);
+  const bool f32_ok = dtype == S3R_F32 && D == 64 && softmax_scale > 0.f && skn > 0 && svn > 0 && skn < (1 << 20) && svn < (1 << 20) &&
+                      vec_ok(k, es, skb, skh, skn) && vec_ok(v, es, svb, svh, svn) && vec_ok(o, es, sob, soh, som);
+  int rc = f32_ok ? launch_attn_f32(p, /*select=*/false, stream) : launch_attn_simple(p, dtype, /*select=*/false, stream);
   if (rc != S3R_OK) return rc;
   if (topk_idx != nullptr) rc = s3r_topk_rows(scores, topk_idx, (int64_t)B * H * Lq, Lk, Lk, K, stream);
   return rc;
@@ -195,6 +197,10 @@ static int select_attn_impl(const char* who, const void* q, const void* k, const
   }
   if (mfma_ok) return launch_select_pipe(p, dtype, stream);
   if (b16_ok) return launch_select_b16(p, dtype, stream);
+  const bool f32_ok = dtype == S3R_F32 && D == 64 && (block == 64 || block == 32 || block == 16) && K <= 64 && softmax_scale > 0.f &&
+                      skn > 0 && svn > 0 && skn < (1 << 20) && svn < (1 << 20) &&
+                      vec_ok(k, es, skb, skh, skn) && vec_ok(v, es, svb, svh, svn) && vec_ok(o, es, sob, soh, son);
+  if (f32_ok) return launch_attn_f32(p, /*select=*/true, stream);
   return launch_attn_simple(p, dtype, /*select=*/true, stream);
 }
 

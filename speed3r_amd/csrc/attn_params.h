@@ -36,6 +36,7 @@ struct AttnParams {
 // row-wise top-k; causal_lq > 0: row r (query r % causal_lq) ranks only its first min((q/64 + 1) * 64, cols) columns
 int launch_topk_rows(const float* scores, int32_t* idx, int64_t rows, int cols, int64_t row_stride, int K, int64_t causal_lq, void* stream);
 int launch_attn_simple(const AttnParams& p, int dtype, bool select, void* stream);
+int launch_attn_f32(const AttnParams& p, bool select, void* stream);  // fp32, head_dim 64, blocks of 16, 32 or 64 tokens
 int launch_select_pipe(const AttnParams& p, int dtype, void* stream);
 int launch_select_b16(const AttnParams& p, int dtype, void* stream);  // block 16
 int launch_compressed_mfma(const AttnParams& p, int dtype, void* stream);

@@ -1,7 +1,7 @@
 // Generic (any I/O dtype, head_dim <= 64) attention kernel for both branches.
 //
-// This is the fp32-I/O instance of the path and the fallback for shapes the MFMA kernels do
-// not cover (block < 64, head_dim < 64).  One 256-thread workgroup owns one query block
+// This is the fallback for shapes the MFMA kernels do not cover (blocks of 4 tokens, head_dim < 64, unaligned tensors,
+// the causal variant).  One 256-thread workgroup owns one query block
 // (64 rows for the compressed branch, `block` rows for the selection branch) of one head.
 // Thread (r, g) owns query row r and a quarter of the columns: key columns g, g+4, ... of the
 // score tile and head_dim slice [16g, 16g+16) of the output.  The query row lives in
