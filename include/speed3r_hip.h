@@ -232,6 +232,54 @@ int s3r_qkv_prepass(const void* q, const void* k, const void* v, void* q_out, vo
                     int64_t sxb, int64_t sxh, int64_t sxn, int64_t spb, int64_t spn, int dtype, void* stream);
 
 /*
+ * The same pass with everything the layer needs of it, in an argument block:
+ *   q_out, k_out (both or neither): the full-token q and k after norm and rotation, contiguous [B,H,N,64].
+ *   q_pool, k_pool, v_pool (all or none): the block means, contiguous [B,H,ceil(N/block),64]; with finish_pooled q_pool and
+ *     k_pool are normalised and rotated too, at the truncated mean position of their block's tokens (the reference's pooled
+ *     tokens, pi3/models/layers/sparse_attention.py:97-110); q_raw, k_raw (optional): their values before that.
+ *   positions: (y,x) pairs, int32 or int64 (positions_int64), strides in elements, or NULL.
+ *   cos_table, sin_table: [table_rows,16] in the I/O dtype as in s3r_norm_rope.  inv_freq (optional, [16] fp32): positions
+ *     at or beyond table_rows get cosine and sine of round(position * inv_freq); without it they are clamped.
+ *   norm parameters in the I/O dtype, or fp32 with norm_fp32 (used unrounded).
+ */
+typedef struct s3r_prepass_args {
+  const void *q, *k, *v;
+  void *q_out, *k_out;
+  void *q_pool, *k_pool, *v_pool;
+  void *q_raw, *k_raw;
+  const void* positions;
+  const void *cos_table, *sin_table;
+  const float* inv_freq;
+  const void *q_norm_weight, *q_norm_bias, *k_norm_weight, *k_norm_bias;
+  int64_t N, stride_b, stride_h, stride_n, pos_stride_b, pos_stride_n;
+  int B, H, head_dim, block, table_rows, positions_int64, norm_fp32, finish_pooled, dtype;
+  float eps;
+} s3r_prepass_args;
+
+int s3r_layer_prepass(const s3r_prepass_args* args, void* stream);
+
+/*
+ * Gradient of that pass (bf16/fp16, blocks of at most 64 tokens): from the gradients of q_out, k_out, v [B,H,N,64] and of
+ * the finished q_pool, k_pool, v_pool (all contiguous, I/O dtype) those of the raw projection, written through
+ * dx_q, dx_k, dx_v with the strides of q, k, v, and, where there is a norm, norm_grads [4,64] fp32: q_norm weight, bias,
+ * k_norm weight, bias.  args as in the forward call (its outputs q_raw, k_raw are read); workspace: fp32
+ * [workspace_rows,256] (768 rows fill the chip), any contents.
+ */
+int s3r_layer_prepass_bwd(const s3r_prepass_args* args, const void* dq, const void* dk, const void* dv, const void* dq_pool,
+                          const void* dk_pool, const void* dv_pool, void* dx_q, void* dx_k, void* dx_v, float* norm_grads,
+                          float* workspace, int workspace_rows, void* stream);
+
+/*
+ * Gradient of the gated merge (bf16/fp16, head_dim 64): dout [B,N,H*64], o_cmp [B,H,ceil(N/block),64], o_sel [B,H,N,64]
+ * contiguous, gate [B,H,N,2] with strides sgb,sgh,sgn (pair contiguous) -> d_o_cmp, d_o_sel (as o_cmp, o_sel), d_gate
+ * [B,N,H,2], and the row sums delta_cmp = <d_o_cmp, o_cmp> [B,H,ceil(N/block)], delta_sel = <d_o_sel, o_sel> [B,H,N] (fp32)
+ * that s3r_attn_bwd takes.  Sums in fp32, every result rounded once.
+ */
+int s3r_gated_merge_bwd(const void* dout, const void* o_cmp, const void* o_sel, const void* gate, void* d_o_cmp, void* d_o_sel,
+                        void* d_gate, float* delta_cmp, float* delta_sel, int B, int H, int64_t N, int D, int block,
+                        int64_t sgb, int64_t sgh, int64_t sgn, int dtype, void* stream);
+
+/*
  * LayerNorm over the channels of token rows:  y[r,:] = (x[r,:] - mean_r) * rstd_r * w + b, fp32 statistics, one
  * rounding to the I/O dtype.  Replaces, for inference, the nn.LayerNorm modules in front of the attention layers and
  * the MLPs (norm1 / norm2, pi3/models/layers/block.py:281,296,312,315).

@@ -42,6 +42,9 @@ SIGNATURES = {
                               c_int, c_int, c_int64, c_int, *_i64x3, c_int64, c_int64, c_int, c_void_p]),
     "s3r_qkv_prepass": (c_int, [c_void_p] * 8 + [c_void_p, c_void_p, c_void_p, c_int] + [c_void_p] * 4 + [c_float, c_int, c_int, c_int64,
                                 c_int, c_int, *_i64x3, c_int64, c_int64, c_int, c_void_p]),
+    "s3r_layer_prepass": (c_int, [c_void_p, c_void_p]),
+    "s3r_layer_prepass_bwd": (c_int, [c_void_p] * 12 + [c_int, c_void_p]),
+    "s3r_gated_merge_bwd": (c_int, [c_void_p] * 9 + [c_int, c_int, c_int64, c_int, c_int, *_i64x3, c_int, c_void_p]),
     "s3r_layer_norm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int, c_int64, c_int64, c_int, c_void_p]),
     "s3r_gated_merge": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int, c_int,
                                 *_i64x3, *_i64x3, *_i64x3, c_int, c_void_p]),
@@ -52,6 +55,18 @@ SIGNATURES = {
                      + [c_int, c_int, c_int64, c_int64, c_int, c_int, c_int]
                      + _i64x3 * 8 + [c_float, c_int, c_void_p]),
 }
+
+
+class PrepassArgs(ctypes.Structure):
+    """``s3r_prepass_args`` of include/speed3r_hip.h, field by field."""
+    _fields_ = ([(n, c_void_p) for n in ("q", "k", "v", "q_out", "k_out", "q_pool", "k_pool", "v_pool", "q_raw", "k_raw", "positions",
+                                         "cos_table", "sin_table", "inv_freq", "q_norm_weight", "q_norm_bias", "k_norm_weight",
+                                         "k_norm_bias")]
+                + [(n, c_int64) for n in ("N", "stride_b", "stride_h", "stride_n", "pos_stride_b", "pos_stride_n")]
+                + [(n, c_int) for n in ("B", "H", "head_dim", "block", "table_rows", "positions_int64", "norm_fp32", "finish_pooled",
+                                        "dtype")]
+                + [("eps", c_float)])
+
 
 _lib = None
 

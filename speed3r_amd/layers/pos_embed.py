@@ -18,10 +18,21 @@ class RoPE2D(nn.Module):
         super().__init__()
         self.base = freq
         self.F0 = F0
-        # number of rows of the cos/sin tables the fused kernel reads; 0: sized from the positions of every call
-        # (one device synchronisation per call, like the reference's ``positions.max()``)
+        # number of rows of the cos/sin tables the fused kernels read, and so a bound of the coordinates (larger ones are
+        # clamped); 0: no bound, coordinates beyond DEFAULT_ROWS are rotated by angles the kernels evaluate themselves
         self.max_positions = max_positions
         self._tables = {}
+
+    DEFAULT_ROWS = 64   # table rows where no bound of the coordinates is given (the kernels hold so many in LDS)
+
+    def fused_tables(self, head_dim: int, n_pos, device, dtype):
+        """``(cos, sin, inv_freq)`` for the fused kernels: tables of ``n_pos`` (default: ``max_positions``) rows and no
+        ``inv_freq`` (coordinates beyond them are clamped), or, without a bound, default tables and the frequencies that
+        give every further coordinate its own angle; no look at the positions, no device synchronisation."""
+        rows = n_pos or self.max_positions
+        if rows:
+            return *self.tables(head_dim, rows, device, dtype), None
+        return *self.tables(head_dim, self.DEFAULT_ROWS, device, dtype), self.inv_freq(head_dim, device)
 
     def tables(self, head_dim: int, n_pos: int, device, dtype):
         """cos, sin ``[n_pos, head_dim // 4]`` in ``dtype``: row p holds cos/sin of the angles ``p * inv_freq`` after
@@ -29,10 +40,18 @@ class RoPE2D(nn.Module):
         key = (head_dim, n_pos, str(device), dtype)
         if key not in self._tables:
             half = head_dim // 2
-            inv_freq = 1.0 / (self.base ** (torch.arange(0, half, 2, device=device, dtype=torch.float32) / half))
+            inv_freq = self.inv_freq(head_dim, device)
             t = torch.arange(n_pos, device=device, dtype=torch.float32)
-            ang = torch.einsum("i,j->ij", t, inv_freq).to(dtype)
+            ang = (t[:, None] * inv_freq).to(dtype)   # (a plain product: fp32 under autocast too)
             self._tables[key] = (ang.cos().contiguous(), ang.sin().contiguous())
+        return self._tables[key]
+
+    def inv_freq(self, head_dim: int, device) -> torch.Tensor:
+        """fp32 ``[head_dim // 4]``: the angle of position p is ``p * inv_freq`` (before its rounding to the tokens' dtype)."""
+        key = (head_dim, str(device))
+        if key not in self._tables:
+            half = head_dim // 2
+            self._tables[key] = 1.0 / (self.base ** (torch.arange(0, half, 2, device=device, dtype=torch.float32) / half))
         return self._tables[key]
 
     def _cos_sin(self, pos1d: torch.Tensor, half: int, dtype: torch.dtype):

@@ -8,9 +8,9 @@ Differences, all on the host side of the operator boundary:
 * q, k, v are handed to the kernels as strided views of the packed projection (no ``.contiguous()`` copies),
   pooling reads the packed projection directly, and the gated merge runs in the selection kernel's epilogue
   (or in its own kernel where that is not built), writing ``[B, N, C]`` for ``proj``;
-* when a gradient is wanted (grad mode on and the input or a parameter requires grad) the layer runs as a
-  differentiable composition instead: the two attention operators with their backward kernels (bf16/fp16,
-  head_dim 64, blocks of 64 or 16 tokens), pooling, norm/RoPE and merge as torch expressions;
+* when a gradient is wanted (grad mode on and the input or a parameter requires grad) the layer runs as projections
+  around one differentiable operator with a backward of kernels (bf16/fp16, head_dim 64, blocks of 64 or 16 tokens; see
+  ``_forward_with_grad`` for the rest);
 * ``N`` need not be a multiple of the block: the last block pools its valid tokens, its keys beyond ``N`` are
   masked and its query rows beyond ``N`` do not exist (the reference raises for such ``N``);
 * the top-k count, 32 in the reference, is a constructor argument.
@@ -97,32 +97,30 @@ class SparseFlashAttentionRope(nn.Module):
     def _norm_rope(self, t: Tensor, norm: nn.Module, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
         return norm_rope_fused_or_eager(t, norm, self.rope, pos, n_pos)
 
-    def _prepass(self, qkv: Tensor, h: int, block: int, pos: Optional[Tensor], n_pos: Optional[int] = None):
-        """The fused pre-pass where its conditions hold (those of ``norm_rope_fused_or_eager`` for both norms), else None."""
+    def _fused_args(self, qkv: Tensor, pos: Optional[Tensor], n_pos: Optional[int] = None):
+        """``(pos, cos, sin, inv_freq, q_ln, k_ln, eps)`` for the kernels that take qk-norm and RoPE with the packed
+        projection, or None where their conditions do not hold (those of ``norm_rope_fused_or_eager`` for both norms)."""
         def plain(norm):
             return isinstance(norm, nn.Identity) or (type(norm) is nn.LayerNorm and norm.elementwise_affine)
         same_kind = isinstance(self.q_norm, nn.Identity) == isinstance(self.k_norm, nn.Identity)
-        if not (qkv.is_cuda and plain(self.q_norm) and plain(self.k_norm) and same_kind and (pos is None or isinstance(self.rope, RoPE2D))):
+        if not (qkv.is_cuda and qkv.shape[-1] == 192 * self.num_heads and plain(self.q_norm) and plain(self.k_norm) and same_kind
+                and (pos is None or isinstance(self.rope, RoPE2D))):
             return None
-        if isinstance(self.q_norm, nn.Identity) and pos is None:   # nothing to do to q and k: the kernels read the projection in place
-            return None
-        if block < 32:   # many pooled tokens: the index kernel is long and starts earlier behind the separate pooling kernel,
-            return None  # beside the norm/RoPE kernels (measured at 266 496 tokens, block 16: 10.9 against 11.2 ms per layer)
-        cos = sin = None
-        if pos is not None:
-            rows = n_pos or self.rope.max_positions or int(pos.max()) + 1
-            cos, sin = self.rope.tables(64, rows, qkv.device, qkv.dtype)
         ln = isinstance(self.q_norm, nn.LayerNorm)
         if ln and self.q_norm.eps != self.k_norm.eps:
             return None
-        return ops.qkv_prepass(qkv, h, block, pos, cos, sin,
-                               (self.q_norm.weight, self.q_norm.bias) if ln else None,
-                               (self.k_norm.weight, self.k_norm.bias) if ln else None, self.q_norm.eps if ln else 0.0)
+        cos = sin = inv_freq = None
+        if pos is not None:
+            cos, sin, inv_freq = self.rope.fused_tables(64, n_pos, qkv.device, qkv.dtype)
+        return (pos, cos, sin, inv_freq, (self.q_norm.weight, self.q_norm.bias) if ln else None,
+                (self.k_norm.weight, self.k_norm.bias) if ln else None, self.q_norm.eps if ln else 0.0)
 
     def _forward_with_grad(self, x: Tensor, xpos: Optional[Tensor]) -> Tensor:
-        """The same layer as a differentiable composition (training): the two attention operators carry their own
-        backward kernels; pooling, qk-norm/RoPE and the gated merge run as the torch expressions of the reference
-        (sparse_attention.py:97-110,120-136), whose gradients autograd provides."""
+        """The same layer for training.  Between its projections it is one differentiable operator whose forward and
+        backward are kernels (``ops.layer_core_autograd``).  Where that is not built (another norm or rope module, blocks of
+        128 or 256 tokens): a composition in which the two attention operators carry their own backward kernels and pooling,
+        qk-norm/RoPE and the gated merge run as the torch expressions of the reference (sparse_attention.py:97-110,120-136),
+        whose gradients autograd provides."""
         b, n, c = x.shape
         h = self.num_heads
         d = c // h
@@ -130,6 +128,16 @@ class SparseFlashAttentionRope(nn.Module):
         nc = -(-n // block)
         qkv = self.qkv(x)
         gate = self.gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)              # [B, H, N, 2]
+        use_pos = xpos is not None and self.rope is not None
+        fused = self._fused_args(qkv, xpos if use_pos else None)
+        if fused is not None and self.topk in (1, 2, 4, 8, 16, 32, 64):
+            pos, cos, sin, inv_freq, q_ln, k_ln, eps = fused
+            core = ops.layer_core_autograd(qkv, gate, h, block, self.topk, pos, cos, sin, inv_freq, q_ln, k_ln, eps)
+            if core is not None:
+                out, idx = core
+                if self.keep_topk_idx:
+                    self.last_topk_idx = idx
+                return self.proj_drop(self.proj(out))
         q, k, v = qkv.view(b, n, 3, h, d).permute(2, 0, 3, 1, 4).unbind(0)    # each [B, H, N, D]
 
         def pool(t):  # block means; a ragged tail block averages its valid tokens
@@ -145,7 +153,6 @@ class SparseFlashAttentionRope(nn.Module):
             t = norm(t).to(t.dtype)
             return self.rope(t, pos) if pos is not None else t
 
-        use_pos = xpos is not None and self.rope is not None
         pos_c = block_positions(xpos, block) if use_pos else None
         q_c, k_c, v_c = pool(q), pool(k), pool(v)
         q_c, k_c = norm_rope(q_c, self.q_norm, pos_c), norm_rope(k_c, self.k_norm, pos_c)
@@ -177,21 +184,28 @@ class SparseFlashAttentionRope(nn.Module):
 
         use_pos = xpos is not None and self.rope is not None
         pos = xpos if use_pos else None
-        # One pass over the packed projection: block means of the raw q, k, v (compressed branch) and norm + RoPE of
-        # the full-token q and k (selection branch), each input row read once.  Where that kernel is not built
-        # (head_dim other than 64, another norm or rope module): pooling kernel, then norm/RoPE per tensor.
-        pre = self._prepass(qkv, h, block, pos, n_pos)
-        self.last_prepass = pre is not None
-        if pre is not None:
-            q, k, v, q_c, k_c, v_c = pre
+        # One pass over the packed projection: block means of the raw q, k, v, normalised and rotated at the block
+        # positions (compressed branch), and norm + RoPE of the full-token q and k (selection branch), each input row read
+        # once.  Where that kernel is not built (head_dim other than 64, another norm or rope module): pooling kernel, then
+        # norm/RoPE per tensor.  16-token blocks take the pass in two launches: the block means first, so that the index
+        # kernel, long for so many pooled tokens, starts while the full tokens are still to come.
+        fused = self._fused_args(qkv, pos, n_pos)
+        q = k = v = None
+        self.last_prepass = False
+        if fused is not None and (pos is not None or fused[4] is not None):   # (else q and k are read in place)
+            args = (pos, fused[1], fused[2], *fused[4:])
+            self.last_prepass = block >= 32
+            if self.last_prepass:
+                q, k, v, q_c, k_c, v_c = ops.qkv_prepass(qkv, h, block, *args, pooled="final", inv_freq=fused[3])
+            else:
+                q_c, k_c, v_c = ops.qkv_prepass(qkv, h, block, *args, tokens=False, pooled="final", inv_freq=fused[3])
         else:
             q_c, k_c, v_c = ops.pool_qkv_packed(qkv, h, block)
-        # compressed branch: pooled raw projections -> norm -> RoPE at block positions -> attention + top-k
-        pos_c = block_positions(xpos, block) if use_pos else None
-        q_c, k_c = self._norm_rope(q_c, self.q_norm, pos_c, n_pos), self._norm_rope(k_c, self.k_norm, pos_c, n_pos)
+            pos_c = block_positions(xpos, block) if use_pos else None
+            q_c, k_c = self._norm_rope(q_c, self.q_norm, pos_c, n_pos), self._norm_rope(k_c, self.k_norm, pos_c, n_pos)
         # the index kernel needs pooled q and k only and its result is first read by the selection kernel: where
         # it is a kernel of its own it runs on a second stream, beside the compressed attention (and the norm/RoPE of
-        # the full tokens where they are separate kernels)
+        # the full tokens where they come after it)
         side = x.is_cuda and ops._two_kernel_compressed(q_c, self.topk)
         if side:
             idx, join = ops.topk_indices_on_side_stream(q_c, k_c, self.topk)
@@ -199,7 +213,9 @@ class SparseFlashAttentionRope(nn.Module):
         else:
             o_c, idx = flash_attn_topk_func(q_c, k_c, v_c, self.topk)
 
-        if pre is None:  # selection branch on strided views of the projection; norm/RoPE make q, k contiguous
+        if q is None and fused is not None and (pos is not None or fused[4] is not None):
+            q, k, v = ops.qkv_prepass(qkv, h, 64, *args, pooled=None, inv_freq=fused[3])
+        elif q is None:  # selection branch on strided views of the projection; norm/RoPE make q, k contiguous
             q, k, v = qkv.view(b, n, 3, h, d).permute(2, 0, 3, 1, 4).unbind(0)   # each [B, H, N, D]
             q, k = self._norm_rope(q, self.q_norm, pos, n_pos), self._norm_rope(k, self.k_norm, pos, n_pos)
         if side:

@@ -10,6 +10,7 @@ dimension; indices are int32 ``[B, H, n_query_blocks, K]`` in block units.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 import os
 from typing import Optional, Tuple
@@ -332,51 +333,79 @@ def norm_rope(x: torch.Tensor, positions: Optional[torch.Tensor], cos_tab: Optio
     return y
 
 
-def qkv_prepass(qkv: torch.Tensor, num_heads: int, block: int, positions: Optional[torch.Tensor],
-                cos_tab: Optional[torch.Tensor], sin_tab: Optional[torch.Tensor],
-                q_ln: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None,
-                k_ln: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None, eps: float = 1e-5):
-    """The layer's pre-pass over the packed projection ``[B, N, 3*H*64]`` (layout ``(qkv h d)``) in one kernel:
-    returns ``(q, k, v, q_c, k_c, v_c)`` -- q, k ``[B,H,N,64]`` contiguous after LayerNorm (``q_ln``/``k_ln`` = (weight,
-    bias) or None) and RoPE2D at ``positions`` (None: no rotation), v the strided view of the projection, and the
-    block means of the RAW q, k, v ``[B,H,ceil(N/block),64]``.  Same bits as :func:`pool_qkv_packed` followed by
-    :func:`norm_rope` on q and k.  Returns None when the library has no kernel for the shape (head_dim other than 64)."""
-    _need_device(qkv)
-    _forward_only(qkv)
+def _prepass_args(qkv: torch.Tensor, h: int, block: int, positions, cos_tab, sin_tab, q_ln, k_ln, eps: float, inv_freq=None):
+    """Argument block of the passes over the packed projection, with its inputs filled in, and the tensors it points to."""
     b, n, c3 = qkv.shape
-    d = c3 // (3 * num_heads)
-    if d != 64 or c3 != 3 * num_heads * 64 or qkv.stride(-1) != 1:
-        return None
-    assert (q_ln is None) == (k_ln is None), "q and k are normalised together or not at all"
-    h = num_heads
-    q, k, v = qkv.view(b, n, 3, h, d).permute(2, 0, 3, 1, 4).unbind(0)   # each [B,H,N,D], common strides
-    nc = -(-n // block)
-    q_out, k_out = (torch.empty((b, h, n, d), dtype=qkv.dtype, device=qkv.device) for _ in range(2))
-    qc, kc, vc = (torch.empty((b, h, nc, d), dtype=qkv.dtype, device=qkv.device) for _ in range(3))
-    pos32 = None
-    p = 0
+    es = qkv.element_size()
+    base = qkv.data_ptr()
+    a = _lib.PrepassArgs(q=base, k=base + h * 64 * es, v=base + 2 * h * 64 * es, N=n, stride_b=qkv.stride(0), stride_h=64,
+                         stride_n=qkv.stride(1), B=b, H=h, head_dim=64, block=block, eps=eps, dtype=_code(qkv))
+    keep = []
     if positions is not None:
         assert positions.shape == (b, n, 2), f"positions shape {tuple(positions.shape)} != {(b, n, 2)}"
         assert cos_tab is not None and sin_tab is not None and cos_tab.shape == sin_tab.shape and cos_tab.shape[1] == 16
         assert cos_tab.dtype == qkv.dtype and sin_tab.dtype == qkv.dtype, "tables must have the tokens' dtype"
-        pos32 = positions.to(device=qkv.device, dtype=torch.int32).contiguous()
+        if positions.dtype not in (torch.int64, torch.int32) or positions.device != qkv.device or positions.stride(2) != 1:
+            positions = positions.to(device=qkv.device, dtype=torch.int32).contiguous()
         cos_tab, sin_tab = cos_tab.contiguous(), sin_tab.contiguous()
-        p = cos_tab.shape[0]
+        keep += [positions, cos_tab, sin_tab]
+        a.positions, a.positions_int64 = positions.data_ptr(), positions.dtype == torch.int64
+        a.pos_stride_b, a.pos_stride_n = positions.stride(0), positions.stride(1)
+        a.cos_table, a.sin_table, a.table_rows = cos_tab.data_ptr(), sin_tab.data_ptr(), cos_tab.shape[0]
+        if inv_freq is not None:
+            a.inv_freq = inv_freq.data_ptr()
+    if q_ln is not None:
+        params = [*q_ln, *k_ln]
+        # fp32 parameters of 16-bit tokens (autocast) are used as they are, any others in the tokens' dtype
+        as_fp32 = all(t is None or t.dtype == torch.float32 for t in params)
+        dtype = torch.float32 if as_fp32 else qkv.dtype
+        params = [t.detach().to(dtype).contiguous() if t is not None else None for t in params]
+        keep += params
+        a.norm_fp32 = as_fp32
+        a.q_norm_weight, a.q_norm_bias, a.k_norm_weight, a.k_norm_bias = (t.data_ptr() if t is not None else None for t in params)
+    return a, keep
 
-    def par(t):
-        return t.detach().to(qkv.dtype).contiguous() if t is not None else None
 
-    qw, qb = (par(q_ln[0]), par(q_ln[1])) if q_ln is not None else (None, None)
-    kw, kb = (par(k_ln[0]), par(k_ln[1])) if k_ln is not None else (None, None)
-    ptr = lambda t: t.data_ptr() if t is not None else None
+def qkv_prepass(qkv: torch.Tensor, num_heads: int, block: int, positions: Optional[torch.Tensor],
+                cos_tab: Optional[torch.Tensor], sin_tab: Optional[torch.Tensor],
+                q_ln: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None,
+                k_ln: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None, eps: float = 1e-5, *,
+                tokens: bool = True, pooled: Optional[str] = "raw", keep_raw: bool = False, inv_freq: Optional[torch.Tensor] = None):
+    """The layer's pre-pass over the packed projection ``[B, N, 3*H*64]`` (layout ``(qkv h d)``) in one kernel:
+    returns ``(q, k, v, q_c, k_c, v_c)`` -- q, k ``[B,H,N,64]`` contiguous after LayerNorm (``q_ln``/``k_ln`` = (weight,
+    bias) or None) and RoPE2D at ``positions`` (None: no rotation), v the strided view of the projection, and the
+    block means of the RAW q, k, v ``[B,H,ceil(N/block),64]``.  Same bits as :func:`pool_qkv_packed` followed by
+    :func:`norm_rope` on q and k.  Returns None when the library has no kernel for the shape (head_dim other than 64).
+
+    ``pooled="final"``: q_c and k_c are normalised and rotated too, at the truncated mean position of their block
+    (:func:`norm_rope` at ``block_positions``); ``keep_raw`` then appends their raw values to the result.
+    ``pooled=None``: q, k, v only; ``tokens=False``: the block means only.  ``inv_freq`` ([16] fp32): positions beyond the
+    tables are rotated by their own angles instead of being clamped to the last row."""
+    _need_device(qkv)
+    _forward_only(qkv)
+    b, n, c3 = qkv.shape
+    h = num_heads
+    if c3 != 3 * h * 64 or qkv.stride(-1) != 1 or qkv.stride(1) < c3:
+        return None
+    assert (q_ln is None) == (k_ln is None), "q and k are normalised together or not at all"
+    assert pooled in ("raw", "final", None) and (tokens or pooled)
+    a, keep = _prepass_args(qkv, h, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq)
+    out = ()
+    if tokens:
+        q_out, k_out = qkv.new_empty((2, b, h, n, 64)).unbind(0)
+        a.q_out, a.k_out = q_out.data_ptr(), k_out.data_ptr()
+        out = (q_out, k_out, qkv.as_strided((b, h, n, 64), (qkv.stride(0), 64, qkv.stride(1), 1), qkv.storage_offset() + 2 * h * 64))
+    if pooled:
+        means = qkv.new_empty((5 if keep_raw else 3, b, h, -(-n // block), 64)).unbind(0)
+        a.q_pool, a.k_pool, a.v_pool = (t.data_ptr() for t in means[:3])
+        a.finish_pooled = pooled == "final"
+        if keep_raw:
+            a.q_raw, a.k_raw = means[3].data_ptr(), means[4].data_ptr()
+        out += means
     with torch.cuda.device(qkv.device):
-        rc = _lib.lib().s3r_qkv_prepass(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), q_out.data_ptr(), k_out.data_ptr(), qc.data_ptr(), kc.data_ptr(),
-            vc.data_ptr(), ptr(pos32), ptr(cos_tab) if pos32 is not None else None, ptr(sin_tab) if pos32 is not None else None, p,
-            ptr(qw), ptr(qb), ptr(kw), ptr(kb), float(eps), b, h, n, d, block, q.stride(0), q.stride(1), q.stride(2),
-            pos32.stride(0) if pos32 is not None else 0, pos32.stride(1) if pos32 is not None else 0, _code(qkv), _stream(qkv))
-    _lib.check(rc, "s3r_qkv_prepass")
-    return q_out, k_out, v, qc, kc, vc
+        rc = _lib.lib().s3r_layer_prepass(ctypes.byref(a), _stream(qkv))
+    _lib.check(rc, "s3r_layer_prepass")
+    return out
 
 
 def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], eps: float) -> Optional[torch.Tensor]:
@@ -591,6 +620,92 @@ class _CompressedAttnFn(torch.autograd.Function):
         dq, dk, dv = attn_bwd(q, k, v, o, dout, lse, None, 64, ctx.scale,
                               need_dq=ctx.needs_input_grad[0], need_dkv=ctx.needs_input_grad[1] or ctx.needs_input_grad[2])
         return dq, dk, dv, None, None, None   # (the reference's backward does not know of `causal` either, :653-666)
+
+
+def gated_merge_bwd(dout: torch.Tensor, o_cmp: torch.Tensor, o_sel: torch.Tensor, gate: torch.Tensor, block: int):
+    """Gradient of :func:`gated_merge` (bf16/fp16, head_dim 64): ``(d_o_cmp, d_o_sel, d_gate, delta_cmp, delta_sel)``, d_gate
+    as the ``[B,H,N,2]`` view of a ``[B,N,H,2]`` tensor, the deltas as :func:`attn_bwd` takes them."""
+    b, h, n, d = o_sel.shape
+    dout, o_cmp, o_sel, gate = dout.contiguous(), o_cmp.contiguous(), o_sel.contiguous(), _last_contig(gate)
+    d_oc, d_os = torch.empty_like(o_cmp), torch.empty_like(o_sel)
+    d_gate = gate.new_empty((b, n, h, 2))
+    delta_c = torch.empty(o_cmp.shape[:3], dtype=torch.float32, device=gate.device)
+    delta_s = torch.empty((b, h, n), dtype=torch.float32, device=gate.device)
+    with torch.cuda.device(gate.device):
+        rc = _lib.lib().s3r_gated_merge_bwd(
+            dout.data_ptr(), o_cmp.data_ptr(), o_sel.data_ptr(), gate.data_ptr(), d_oc.data_ptr(), d_os.data_ptr(), d_gate.data_ptr(),
+            delta_c.data_ptr(), delta_s.data_ptr(), b, h, n, d, block, gate.stride(0), gate.stride(1), gate.stride(2), _code(gate), _stream(gate))
+    _lib.check(rc, "s3r_gated_merge_bwd")
+    return d_oc, d_os, d_gate.permute(0, 2, 1, 3), delta_c, delta_s
+
+
+PREPASS_BWD_ROWS = 768   # workgroups of the projection's backward pass that hold parameter sums: three per CU
+
+
+def qkv_prepass_bwd(qkv: torch.Tensor, num_heads: int, block: int, positions, cos_tab, sin_tab, q_ln, k_ln, eps: float, raw, grads,
+                    inv_freq=None):
+    """Gradient of :func:`qkv_prepass` with ``pooled="final"``: ``raw`` = the raw (q_c, k_c), ``grads`` = the gradients of
+    (q, k, v, q_c, k_c, v_c).  Returns ``(d_qkv, d_norm)``, d_norm ``[4,64]`` fp32 (q weight, q bias, k weight, k bias) or
+    None without a norm."""
+    a, keep = _prepass_args(qkv, num_heads, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq)
+    a.q_raw, a.k_raw = (t.data_ptr() for t in raw)
+    grads = [t.contiguous() for t in grads]
+    d_qkv = torch.empty_strided(qkv.shape, qkv.stride(), dtype=qkv.dtype, device=qkv.device)
+    off = [d_qkv.data_ptr() + i * num_heads * 64 * d_qkv.element_size() for i in range(3)]
+    d_norm = work = None
+    if q_ln is not None:
+        work = torch.empty((PREPASS_BWD_ROWS + 1, 256), dtype=torch.float32, device=qkv.device)
+        d_norm = work[PREPASS_BWD_ROWS].view(4, 64)
+    with torch.cuda.device(qkv.device):
+        rc = _lib.lib().s3r_layer_prepass_bwd(ctypes.byref(a), *(t.data_ptr() for t in grads), *off,
+                                              d_norm.data_ptr() if d_norm is not None else None,
+                                              work.data_ptr() if work is not None else None, PREPASS_BWD_ROWS, _stream(qkv))
+    _lib.check(rc, "s3r_layer_prepass_bwd")
+    return d_qkv, d_norm
+
+
+class _LayerCoreFn(torch.autograd.Function):
+    """Everything of the layer between its projections, ``(packed qkv, gate, qk-norm parameters) -> ([B,N,C], indices)``
+    (pi3/models/layers/sparse_attention.py:97-136): the forward kernels of the inference route with their log-sum-exps,
+    and a backward of kernels only.  Between the two the I/O-dtype tensors that a kernel reads again are kept."""
+
+    @staticmethod
+    def forward(ctx, qkv, gate, q_w, q_b, k_w, k_b, xpos, cos, sin, inv_freq, heads, block, topk, eps):
+        q_ln, k_ln = ((q_w, q_b), (k_w, k_b)) if q_w is not None else (None, None)
+        with torch.no_grad():
+            q, k, v, q_c, k_c, v_c, q_raw, k_raw = qkv_prepass(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, pooled="final",
+                                                               keep_raw=True, inv_freq=inv_freq)
+            o_c, idx, lse_c = compressed_attn_topk(q_c, k_c, v_c, topk, return_lse=True)
+            o_s, lse = select_attn(q, k, v, idx, block, return_lse=True)
+            out = gated_merge(o_c, o_s, gate, block)
+        ctx.save_for_backward(qkv, gate, q_w, q_b, k_w, k_b, xpos, cos, sin, inv_freq, q, k, q_c, k_c, v_c, q_raw, k_raw, o_c, lse_c, o_s, lse, idx)
+        ctx.args = heads, block, eps
+        ctx.mark_non_differentiable(idx)
+        return out, idx
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dout, _didx):
+        qkv, gate, q_w, q_b, k_w, k_b, xpos, cos, sin, inv_freq, q, k, q_c, k_c, v_c, q_raw, k_raw, o_c, lse_c, o_s, lse, idx = ctx.saved_tensors
+        heads, block, eps = ctx.args
+        b, n, _ = qkv.shape
+        v = qkv.as_strided((b, heads, n, 64), (qkv.stride(0), 64, qkv.stride(1), 1), qkv.storage_offset() + 2 * heads * 64)
+        d_oc, d_os, d_gate, delta_c, delta_s = gated_merge_bwd(dout, o_c, o_s, gate, block)
+        pooled = attn_bwd(q_c, k_c, v_c, o_c, d_oc, lse_c, delta=delta_c)
+        full = attn_bwd(q, k, v, o_s, d_os, lse, idx, block, delta=delta_s)
+        q_ln, k_ln = ((q_w, q_b), (k_w, k_b)) if q_w is not None else (None, None)
+        d_qkv, d_norm = qkv_prepass_bwd(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, (q_raw, k_raw), (*full, *pooled), inv_freq)
+        params = [d_norm[i].to(t.dtype) if t is not None else None for i, t in enumerate((q_w, q_b, k_w, k_b))]
+        return d_qkv, d_gate, *params, *([None] * 8)
+
+
+def layer_core_autograd(qkv: torch.Tensor, gate: torch.Tensor, heads: int, block: int, topk: int, xpos, cos, sin, inv_freq, q_ln, k_ln, eps: float):
+    """``(out [B,N,C], indices)`` of the layer between its projections, differentiable in qkv, gate and the norm parameters,
+    or None where the kernels are not built (bf16/fp16, head_dim 64, blocks of 64 or 16 tokens)."""
+    if qkv.dtype not in (torch.bfloat16, torch.float16) or gate.dtype != qkv.dtype or qkv.shape[-1] != 3 * heads * 64 or block not in (64, 16) \
+            or not qkv.is_contiguous():
+        return None
+    return _LayerCoreFn.apply(qkv, gate, *(q_ln or (None, None)), *(k_ln or (None, None)), xpos, cos, sin, inv_freq, heads, block, topk, eps)
 
 
 def _wants_grad(*ts: torch.Tensor) -> bool:
