@@ -67,9 +67,8 @@ __global__ __launch_bounds__(256) void merge_bwd_kernel(const T* __restrict__ do
       }
     }
   }
-  for (int off = LPR; off < 64; off <<= 1)
 #pragma unroll
-    for (int i = 0; i < VEC; i++) acc[i] += __shfl_xor(acc[i], off);
+  for (int i = 0; i < VEC; i++) acc[i] = across_groups<LPR>(acc[i]);
   uint4 out;
   float dc = 0.f;
 #pragma unroll
@@ -233,9 +232,8 @@ __global__ __launch_bounds__(256, 3) void prepass_bwd_kernel(PrepassParams p, Pr
     // parameter sums: over the row groups of a wave, then over the four waves through LDS (the tables are done with)
 #pragma unroll
     for (int k = 0; k < 4; k++)
-      for (int off = LPR; off < 64; off <<= 1)
 #pragma unroll
-        for (int i = 0; i < VEC; i++) sums[k][i] += __shfl_xor(sums[k][i], off);
+      for (int i = 0; i < VEC; i++) sums[k][i] = across_groups<LPR>(sums[k][i]);
     __syncthreads();
     if (r0 == 0) {
 #pragma unroll

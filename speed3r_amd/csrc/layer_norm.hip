@@ -35,8 +35,7 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const T* __restrict__ x
       s += v[i][j];
     }
   }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) s += __shfl_xor(s, off);
+  s = group_sum<64>(s);
   const float mean = s / (float)C;
   float q = 0.f;
 #pragma unroll
@@ -45,8 +44,7 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const T* __restrict__ x
 #pragma unroll
       for (int j = 0; j < VEC; j++) q += (v[i][j] - mean) * (v[i][j] - mean);
     }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) q += __shfl_xor(q, off);
+  q = group_sum<64>(q);
   const float rstd = 1.0f / sqrtf(q / (float)C + eps);
   T* yr = y + row * sy;
 #pragma unroll

@@ -9,6 +9,29 @@
 
 namespace s3r {
 
+// acc: sums of the wave's row groups (lpr lanes a row) -> the mean over cnt rows in every group; same pairs of addends
+// whichever way the groups are folded
+template <int VEC> __device__ __forceinline__ void fold_mean(float (&acc)[VEC], int lpr, int cnt) {
+  if (lpr == 8 || lpr == 16) {  // (wave-uniform) rows of 64 values: no LDS crossbar
+#pragma unroll
+    for (int i = 0; i < VEC; i++) acc[i] = lpr == 8 ? across_groups<8>(acc[i]) : across_groups<16>(acc[i]);
+  } else {
+    for (int off = lpr; off < 64; off <<= 1) {
+#pragma unroll
+      for (int i = 0; i < VEC; i++) acc[i] += __shfl_xor(acc[i], off);
+    }
+  }
+  const float c = (float)cnt;
+  if ((cnt & (cnt - 1)) == 0) {  // (wave-uniform) a power of two: its reciprocal is exact and the product the quotient
+    const float inv = 1.0f / c;
+#pragma unroll
+    for (int i = 0; i < VEC; i++) acc[i] *= inv;
+  } else {
+#pragma unroll
+    for (int i = 0; i < VEC; i++) acc[i] /= c;
+  }
+}
+
 template <typename T, int U>
 __global__ __launch_bounds__(256) void pool_mean_kernel(
     const T* __restrict__ x, T* __restrict__ y, int H, int64_t N, int D, int block, int64_t Nc,
@@ -53,16 +76,12 @@ __global__ __launch_bounds__(256) void pool_mean_kernel(
       for (int i = 0; i < VEC; i++) acc[i] += keep ? to_f32(e[i]) : 0.f;
     }
   }
-  for (int off = lpr; off < 64; off <<= 1) {
-#pragma unroll
-    for (int i = 0; i < VEC; i++) acc[i] += __shfl_xor(acc[i], off);
-  }
+  fold_mean(acc, lpr, nvalid);
   if (r0 == 0) {
     uint4 raw;
     T* e = reinterpret_cast<T*>(&raw);
-    const float cnt = (float)nvalid;
 #pragma unroll
-    for (int i = 0; i < VEC; i++) e[i] = from_f32<T>(acc[i] / cnt);
+    for (int i = 0; i < VEC; i++) e[i] = from_f32<T>(acc[i]);
     *reinterpret_cast<uint4*>(y + b * syb + h * syh + j * syn + dc * VEC) = raw;
   }
 }
@@ -114,16 +133,12 @@ __global__ __launch_bounds__(256) void pool_mean_group_kernel(
 #pragma unroll
       for (int i = 0; i < VEC; i++) acc[i] += keep ? to_f32(e[i]) : 0.f;
     }
-    for (int off = lpr; off < 64; off <<= 1) {
-#pragma unroll
-      for (int i = 0; i < VEC; i++) acc[i] += __shfl_xor(acc[i], off);
-    }
+    fold_mean(acc, lpr, nval[g] > 0 ? nval[g] : 1);
     if (r0 == 0 && nval[g] > 0) {
       uint4 out;
       T* e = reinterpret_cast<T*>(&out);
-      const float cnt = (float)nval[g];
 #pragma unroll
-      for (int i = 0; i < VEC; i++) e[i] = from_f32<T>(acc[i] / cnt);
+      for (int i = 0; i < VEC; i++) e[i] = from_f32<T>(acc[i]);
       *reinterpret_cast<uint4*>(y + b * syb + h * syh + (jg * G + g) * syn + dc * VEC) = out;
     }
   }

@@ -84,7 +84,7 @@ template <typename T> struct RotLane {
 __device__ __forceinline__ int block_position(int pos_sum, float cnt, int half) {
 #pragma unroll
   for (int off = 2; off < 64; off <<= 1) pos_sum += __shfl_xor(pos_sum, off);
-  return (int)((float)__shfl(pos_sum, half) / cnt);
+  return (int)((float)(half ? __builtin_amdgcn_readlane(pos_sum, 1) : __builtin_amdgcn_readlane(pos_sum, 0)) / cnt);
 }
 
 template <int VEC> __device__ __forceinline__ void load_row(const float* src, float (&x)[VEC]) {

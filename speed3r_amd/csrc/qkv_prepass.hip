@@ -32,12 +32,8 @@ __global__ __launch_bounds__(256, 4) void qkv_prepass_kernel(PrepassParams p, in
   constexpr int RPW = 64 / LPR;      // rows per wave-wide step
   extern __shared__ __align__(16) float staged[];
   const int lane = threadIdx.x & 63;
-  if constexpr (NORM || ROT) {
-    stage_tables<T>(p, staged);
-    __syncthreads();
-  }
-  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= total) return;
+  const int64_t w_own = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t w = w_own < total ? w_own : total - 1;  // (a wave past the end leaves after the workgroup's barrier)
   // heads fastest: the waves that run side by side read neighbouring 128-byte pieces of the same token rows of the
   // packed projection (one head each), not rows 3*H*128 bytes apart
   const int h = (int)(w % p.H);
@@ -77,7 +73,30 @@ __global__ __launch_bounds__(256, 4) void qkv_prepass_kernel(PrepassParams p, in
     nk = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.k + off));
     if constexpr (POOL) nv = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.v + off));
   };
-  if constexpr (ROWS) request(0);
+  u32x4 first[ROWS ? 1 : 12];  // block means alone: the rows of the first four steps
+  if constexpr (ROWS) {
+    request(0);
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int rr = u * RPW + r0;
+      const int64_t off = in_off + (t0 + (rr < nvalid ? rr : nvalid - 1)) * p.sxn;
+      if (u * RPW < nvalid) {
+        first[3 * u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.q + off));
+        first[3 * u + 1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.k + off));
+        first[3 * u + 2] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.v + off));
+      }
+    }
+    if constexpr (ROT) {
+      for (int t = 0; t < nvalid; t += 64) fetch_positions(t);
+    }
+  }
+  // the first rows are on their way while the workgroup stages its tables
+  if constexpr (NORM || ROT) {
+    stage_tables<T>(p, staged);
+    __syncthreads();
+  }
+  if (w_own >= total) return;
   // one wave-wide step; WHOLE: all its rows are inside the block (no row to keep out of the sums and the stores)
   auto step = [&](int rbase, auto whole_tag) {
     constexpr bool WHOLE = decltype(whole_tag)::value;
@@ -125,19 +144,17 @@ __global__ __launch_bounds__(256, 4) void qkv_prepass_kernel(PrepassParams p, in
     one(lk, ak, 2, ko);
   };
   if constexpr (!ROWS) {  // the sums alone: four steps' rows in flight
-    if constexpr (ROT) {
-      for (int t = 0; t < nvalid; t += 64) fetch_positions(t);
-    }
     for (int rbase = 0; rbase < nvalid; rbase += 4 * RPW) {
-      u32x4 rq[4], rk[4], rv[4];
+      if (rbase > 0) {
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int rr = rbase + u * RPW + r0;
-        if (rbase + u * RPW < nvalid) {
+        for (int u = 0; u < 4; u++) {
+          const int rr = rbase + u * RPW + r0;
           const int64_t off = in_off + (t0 + (rr < nvalid ? rr : nvalid - 1)) * p.sxn;
-          rq[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.q + off));
-          rk[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.k + off));
-          rv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.v + off));
+          if (rbase + u * RPW < nvalid) {
+            first[3 * u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.q + off));
+            first[3 * u + 1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.k + off));
+            first[3 * u + 2] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const T*)p.v + off));
+          }
         }
       }
 #pragma unroll
@@ -145,9 +162,9 @@ __global__ __launch_bounds__(256, 4) void qkv_prepass_kernel(PrepassParams p, in
         if (rbase + u * RPW + r0 < nvalid) {
 #pragma unroll
           for (int i = 0; i < VEC; i++) {
-            aq[i] += to_f32(reinterpret_cast<const T*>(&rq[u])[i]);
-            ak[i] += to_f32(reinterpret_cast<const T*>(&rk[u])[i]);
-            av[i] += to_f32(reinterpret_cast<const T*>(&rv[u])[i]);
+            aq[i] += to_f32(reinterpret_cast<const T*>(&first[3 * u])[i]);
+            ak[i] += to_f32(reinterpret_cast<const T*>(&first[3 * u + 1])[i]);
+            av[i] += to_f32(reinterpret_cast<const T*>(&first[3 * u + 2])[i]);
           }
         }
       }
@@ -158,45 +175,58 @@ __global__ __launch_bounds__(256, 4) void qkv_prepass_kernel(PrepassParams p, in
     else step(rbase, std::false_type{});
   }
   if constexpr (POOL) {
-    // block means: fold the row groups, divide by the number of valid tokens
-    for (int off = LPR; off < 64; off <<= 1) {
-#pragma unroll
-      for (int i = 0; i < VEC; i++) {
-        aq[i] += __shfl_xor(aq[i], off);
-        ak[i] += __shfl_xor(ak[i], off);
-        av[i] += __shfl_xor(av[i], off);
-      }
-    }
-    const float cnt = (float)nvalid;
-    const int64_t o = ((b * p.H + h) * Nc + j) * D + lr * VEC;
-    auto put = [&](void* dst, const float (&x)[VEC]) {
-      uint4 r;
-#pragma unroll
-      for (int i = 0; i < VEC; i++) reinterpret_cast<T*>(&r)[i] = from_f32<T>(x[i]);
-      if (r0 == 0) *reinterpret_cast<uint4*>((T*)dst + o) = r;
-    };
+    // Block means: fold the row groups, divide by the number of valid tokens.  The row groups share the rest of the work:
+    // even ones go on with q, odd ones with k (one pass of norm and rotation for both; with 16-token blocks this tail is
+    // as long as the block's two steps), the third stores v.
+    const bool odd = (r0 & 1) != 0;
+    float x[VEC];
 #pragma unroll
     for (int i = 0; i < VEC; i++) {
-      aq[i] = round_to<T>(aq[i] / cnt);
-      ak[i] = round_to<T>(ak[i] / cnt);
-      av[i] = round_to<T>(av[i] / cnt);
+      const float mine = odd ? ak[i] : aq[i], other = odd ? aq[i] : ak[i];
+      if constexpr (LPR == 8) {
+        x[i] = mine + lane_xor<8>(other);
+        av[i] = sum_step<8>(av[i]);
+        x[i] = sum_step<32>(sum_step<16>(x[i]));
+      } else {
+        x[i] = mine + lane_xor<16>(other);
+        av[i] = sum_step<16>(av[i]);
+        x[i] = sum_step<32>(x[i]);
+      }
+      av[i] = LPR == 8 ? sum_step<32>(sum_step<16>(av[i])) : sum_step<32>(av[i]);
     }
-    put(p.vc, av);
-    if (p.q_raw != nullptr) put(p.q_raw, aq);
-    if (p.k_raw != nullptr) put(p.k_raw, ak);
+    const float cnt = (float)nvalid;
+    if ((nvalid & (nvalid - 1)) == 0) {  // (wave-uniform) a power of two: its reciprocal is exact and the product the quotient
+      const float inv = 1.0f / cnt;
+#pragma unroll
+      for (int i = 0; i < VEC; i++) {
+        x[i] = round_to<T>(x[i] * inv);
+        av[i] = round_to<T>(av[i] * inv);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < VEC; i++) {
+        x[i] = round_to<T>(x[i] / cnt);
+        av[i] = round_to<T>(av[i] / cnt);
+      }
+    }
+    const int64_t o = ((b * p.H + h) * Nc + j) * D + lr * VEC;
+    auto put = [&](void* dst, const float (&y)[VEC]) {
+      uint4 r;
+#pragma unroll
+      for (int i = 0; i < VEC; i++) reinterpret_cast<T*>(&r)[i] = from_f32<T>(y[i]);
+      *reinterpret_cast<uint4*>((T*)dst + o) = r;
+    };
+    if (r0 == 2) put(p.vc, av);
+    void* const raw = odd ? p.k_raw : p.q_raw;
+    if (r0 < 2 && raw != nullptr) put(raw, x);
     if (p.finish) {  // the means as tokens of the compressed branch: norm, rotation at the truncated mean position
-      TablePtr tab = {};
+      if constexpr (NORM) norm_row<T>(p, staged, x, odd ? 2 : 0, lr);
       if constexpr (ROT) {
         const int pc = block_position(pos_sum, cnt, rl.half);
-        tab = table_ptr<T>(p, staged, rl, pc, __any(pc >= p.staged_rows), !rl.second);
+        rotate_row<T>(x, table_ptr<T>(p, staged, rl, pc, __any(pc >= p.staged_rows), !rl.second));
       }
-      if constexpr (NORM) norm_row<T>(p, staged, aq, 0, lr);
-      if constexpr (ROT) rotate_row<T>(aq, tab);
-      if constexpr (NORM) norm_row<T>(p, staged, ak, 2, lr);
-      if constexpr (ROT) rotate_row<T>(ak, tab);
     }
-    put(p.qc, aq);
-    put(p.kc, ak);
+    if (r0 < 2) put(odd ? p.kc : p.qc, x);
   }
 }
 

@@ -99,25 +99,52 @@ constexpr int kWave = 64;
 // the row bits, and row bit 4 and above do not enter: k_swizzle(r + 8) = k_swizzle(r) ^ k_swizzle(8) for r < 8.
 __device__ __forceinline__ constexpr int k_swizzle(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
 
-// Value held by lane ^ MASK.  Masks 1 and 2 stay inside a quad and ride on the DPP operand path of an ordinary move
-// (no LDS crossbar); masks up to 16 use the swizzle unit without an address register; larger ones the general permute.
+// Value held by lane ^ MASK.  Masks 1, 2 and 8 ride on the DPP operand path of an ordinary move
+// (no LDS crossbar); the others up to 16 use the swizzle unit without an address register; larger ones the general permute.
 template <int MASK> __device__ __forceinline__ float lane_xor(float x) {
   static_assert(MASK > 0 && MASK < 64 && (MASK & (MASK - 1)) == 0, "one bit of the lane number");
   const int v = __float_as_int(x);
   if constexpr (MASK == 1) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));       // quad_perm [1,0,3,2]
   else if constexpr (MASK == 2) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));  // quad_perm [2,3,0,1]
+  else if constexpr (MASK == 8) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x128, 0xF, 0xF, false));  // row_ror:8
   else if constexpr (MASK < 32) return __int_as_float(__builtin_amdgcn_ds_swizzle(v, (MASK << 10) | 0x1F));       // bit mode: and 0x1f, xor MASK
   else return __shfl_xor(x, MASK);
 }
+// One butterfly step of a sum: x + x of lane ^ MASK, for MASK = 1, 2, ..., N / 2 in this order.  No step uses the LDS
+// crossbar: after the steps below it all lanes of a quad (half row) hold the same value, so the mirror of a half row (row)
+// hands out what lane ^ 4 (^ 8) holds; whole rows and halves of the wave are exchanged by the permlane swaps.
+template <int MASK> __device__ __forceinline__ float sum_step(float x) {
+  static_assert(MASK > 0 && MASK < 64 && (MASK & (MASK - 1)) == 0, "one bit of the lane number");
+  const int v = __float_as_int(x);
+  if constexpr (MASK < 4) {
+    return x + lane_xor<MASK>(x);
+  } else if constexpr (MASK == 4) {
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));  // row_half_mirror
+  } else if constexpr (MASK == 8) {
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x128, 0xF, 0xF, false));  // row_ror:8 (= lane ^ 8, from any start)
+  } else if constexpr (MASK == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+}
 // sum over the aligned group of N lanes (a power of two) the lane belongs to
 template <int N> __device__ __forceinline__ float group_sum(float s) {
-  if constexpr (N >= 2) s += lane_xor<1>(s);
-  if constexpr (N >= 4) s += lane_xor<2>(s);
-  if constexpr (N >= 8) s += lane_xor<4>(s);
-  if constexpr (N >= 16) s += lane_xor<8>(s);
-  if constexpr (N >= 32) s += lane_xor<16>(s);
-  if constexpr (N >= 64) s += lane_xor<32>(s);
+  if constexpr (N >= 2) s = sum_step<1>(s);
+  if constexpr (N >= 4) s = sum_step<2>(s);
+  if constexpr (N >= 8) s = sum_step<4>(s);
+  if constexpr (N >= 16) s = sum_step<8>(s);
+  if constexpr (N >= 32) s = sum_step<16>(s);
+  if constexpr (N >= 64) s = sum_step<32>(s);
   return s;
+}
+// sum over the lanes lane ^ k N of the wave (N = 8 or 16: the row groups of a pass over 16-bit or fp32 rows of 64 values)
+template <int N> __device__ __forceinline__ float across_groups(float s) {
+  static_assert(N == 8 || N == 16, "row groups of 8 or 16 lanes");
+  if constexpr (N == 8) s = sum_step<8>(s);
+  return sum_step<32>(sum_step<16>(s));
 }
 
 }  // namespace s3r
