@@ -6,7 +6,10 @@
 // The 32x32x16 MFMA wants 32 keys and 32 queries per tile, a list entry offers 16 keys for 16 queries.  Two walks:
 //  * union walk (default): the wave walks the UNION of its four lists, two distinct key blocks per tile, all 64
 //    queries scored against both (neighbouring query blocks list mostly the same blocks, so most quadrants are
-//    useful); walk list built first, then a software pipeline over (tile, query half) units, see the kernel body;
+//    useful); walk list built first, then a software pipeline over (tile, query half) units, see the kernel body.
+//    Where the lists share little (a layer on features without a common scene: 90 to 105 distinct blocks of 128
+//    entries, where a video's q, k give 38) half of those units score blocks that nobody of the half lists: each half
+//    of the wave then walks its own union, decided per wave;
 //  * pair walk (S3R_B16_KERNEL=pairs, cross-check, and tensors beyond 4 GB per head): a tile pairs TWO query blocks
 //    with ONE list entry of each, rows 0-15 of the key half tile hold the block the first query block lists at
 //    position i, rows 16-31 the block the second one lists at position i; S^T = K Q^T then has two useful 16x16
@@ -33,6 +36,13 @@ constexpr int kHalfBytes = 32 * 128;
 // (measured on the walk before the pipeline: 4 waves 1.71 ms, 2: 1.50 ms, 1: 1.42 ms at 266 496 tokens, top-32).
 constexpr int kWaves = S3R_B16_WAVES;
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr int kHalfList = 132;  // places of a half's own list (2 x 64 entries; an even number: entries are read in pairs)
+// One walk per half where the longer half's list has at most this share of the distinct blocks of all four lists.  A unit
+// costs the same either way and there are 2 max(n0, n1) of them instead of 2 n; the walks per half fetch n0 + n1 blocks
+// instead of n.  Thresholds from 60 to 100 % measured (us, top-32): lists of 98 distinct blocks at 32 256 tokens 271 without,
+// 248 / 246 / 246 at 60 / 70 / 90 %; 105 at 8 064 tokens 83 without, 74 / 68.5 / 68.5; lists of 38 (halves 35) at 266 496
+// tokens 1 010 without, 985 / 980 / 980, and 1 230 at 100 %, where the walks per half fetch everything twice for nothing.
+constexpr int kSplitNum = 4, kSplitDen = 5;
 typedef std::integral_constant<int, 0> H0;
 typedef std::integral_constant<int, 1> H1;
 
@@ -248,7 +258,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
 #pragma unroll
     for (int qt = 0; qt < 2; qt++)
       lanes_any[qt] = (__ballot(my_idx[2 * qt] >= 0) ? 0x0000FFFF0000FFFFull : 0ull) | (__ballot(my_idx[2 * qt + 1] >= 0) ? 0xFFFF0000FFFF0000ull : 0ull);
-    __shared__ __attribute__((aligned(16))) int2 lds_walk[kWaves][264];  // up to 4 x 64 entries and the end mark
+    __shared__ __attribute__((aligned(16))) int2 lds_walk[kWaves][2 * kHalfList];  // up to 4 x 64 entries and the end mark
     int2* const walk = lds_walk[wave];
     const int32_t ragged_blk = (N & 15) ? (int32_t)(N >> 4) : -2;  // the block that ends before its 16th row ...
     const int ragged_last = (int)(N & 15) - 1;
@@ -259,6 +269,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
     // then the occupied slots are compacted into the list, eight slots per lane, positions from ballots.  The list's
     // order is the table's, which is as good as any.
     int n_union = 0;
+    int half_tiles = 0;  // tiles per half where each half walks its own union; 0: one walk for both
     uint32_t cnt_bits = 0;
     {
       int32_t* const hkey = reinterpret_cast<int32_t*>(k_buf[0]);          // [512]
@@ -287,18 +298,41 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
       const int4 c0 = reinterpret_cast<const int4*>(hcnt)[2 * lane], c1 = reinterpret_cast<const int4*>(hcnt)[2 * lane + 1];
       const int32_t ks8[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
       const int32_t cs8[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-      uint32_t pos = 0;  // occupied slots of the lanes below
+      uint32_t pos = 0, pos0 = 0, pos1 = 0;  // occupied slots of the lanes below: all, with a count of half 0, of half 1
+      int n_half[2] = {0, 0};
 #pragma unroll
       for (int s8 = 0; s8 < 8; s8++) {
-        const uint64_t m = __ballot(ks8[s8] >= 0);
+        const uint64_t m0 = __ballot((cs8[s8] & 0xffff) != 0), m1 = __ballot(((uint32_t)cs8[s8] >> 16) != 0), m = m0 | m1;
         pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, pos));
+        pos0 = __builtin_amdgcn_mbcnt_hi((uint32_t)(m0 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m0, pos0));
+        pos1 = __builtin_amdgcn_mbcnt_hi((uint32_t)(m1 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m1, pos1));
         n_union += __popcll(m);
+        n_half[0] += __popcll(m0);
+        n_half[1] += __popcll(m1);
         cnt_bits |= (uint32_t)cs8[s8];
       }
+      // Lists that share little: one walk per half (a half without a list of its own keeps to the common walk).
+      const int longer = n_half[0] > n_half[1] ? n_half[0] : n_half[1];
+      if (n_half[0] > 0 && n_half[1] > 0 && longer * kSplitDen <= n_union * kSplitNum) half_tiles = (longer + 1) >> 1;
+      if (half_tiles == 0) {
 #pragma unroll
-      for (int s8 = 0; s8 < 8; s8++)
-        if (ks8[s8] >= 0) walk[pos++] = make_int2(ks8[s8], cs8[s8]);
-      if (lane == 0) walk[n_union] = make_int2(-1, 0);
+        for (int s8 = 0; s8 < 8; s8++)
+          if (ks8[s8] >= 0) walk[pos++] = make_int2(ks8[s8], cs8[s8]);
+        if (lane == 0) walk[n_union] = make_int2(-1, 0);
+      } else {
+        pos1 += kHalfList;
+#pragma unroll
+        for (int s8 = 0; s8 < 8; s8++) {
+          if ((cs8[s8] & 0xffff) != 0) walk[pos0++] = make_int2(ks8[s8], cs8[s8]);
+          if (((uint32_t)cs8[s8] >> 16) != 0) walk[pos1++] = make_int2(ks8[s8], cs8[s8]);
+        }
+        // the shorter list, and an odd one, goes on with its first block, counted by nobody
+#pragma unroll
+        for (int qt = 0; qt < 2; qt++) {
+          const int first = walk[qt * kHalfList].x;
+          for (int i = n_half[qt] + lane; i < 2 * half_tiles; i += 64) walk[qt * kHalfList + i] = make_int2(first, 0);
+        }
+      }
       cnt_bits = __any((cnt_bits & 0xfefefefeu) != 0) ? 2u : 0u;
       cnt_bits |= ragged_cnts;
     }
@@ -525,11 +559,92 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
       exps_tail(H1{});
     };
 
-    const int ntiles = (n_union + 1) >> 1;
+    // One walk per half: unit u = tile u >> 1 of half u & 1's own list, K and V tiles of its own in the buffers of its half.
+    // On entry of phase u (half QT): st[QT] = its scores; ak = K(u+1); vfr = V(u-1); pf[other] = probabilities of unit u-1.
+    // Transfers are issued in the fixed order K(u+3), V(u+1), K(u+4), V(u+2), four instructions each, so that twelve
+    // lie behind the ones a phase waits for.  (av, bv): the blocks of unit u+1; nx: the pending read of unit u+4's.
+    auto phase = [&](auto qt_tag, uint32_t ca, uint32_t cb, int32_t av, int32_t bv, const int4& nx,
+                     int32_t& a4, uint32_t& ca4, int32_t& b4, uint32_t& cb4) {
+      constexpr int QT = decltype(qt_tag)::value;
+      typedef std::integral_constant<int, QT ^ 1> O;
+      pre(qt_tag, ca, cb);
+      static_for<8>([&](auto j_tag) {
+        constexpr int j = decltype(j_tag)::value;
+        if constexpr (j == 1) {
+          __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): V(u-1) is in registers
+          dma_v(O{}, av, bv);                  // V(u+1) over V(u-1)
+        }
+        if constexpr (j == 4) {
+          __builtin_amdgcn_s_waitcnt(0x0F7C);  // vmcnt(12): K(u+2) has landed
+          load_k(qt_tag);
+        }
+        if constexpr (j == 7) {
+          __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): K(u+2) is in registers
+          lookup_take(nx, a4, ca4, b4, cb4);
+          dma_k(qt_tag, a4, b4);               // K(u+4) over K(u+2)
+        }
+        if constexpr (j < 4) mma_s(O{}, j_tag);
+        else mma_pv(O{}, std::integral_constant<int, j - 4>{});
+        exps(qt_tag, j_tag);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      exps_tail(qt_tag);
+      __builtin_amdgcn_s_waitcnt(0x0F7C);  // vmcnt(12): V(u) has landed
+      load_v(qt_tag);
+    };
+    auto half_lookup = [&](auto qt_tag, int tau) -> int4 {
+      constexpr int QT = decltype(qt_tag)::value;
+      int4 v = make_int4(-1, 0, -1, 0);
+      if (tau < half_tiles) v = *reinterpret_cast<const int4*>(walk + QT * kHalfList + 2 * tau);
+      return v;
+    };
+
+    const int ntiles = half_tiles > 0 ? 0 : (n_union + 1) >> 1;
     for (int pass = 0; pass < 2; pass++) {
       exact = pass == 1;
       settled[0] = lanes_any[0] == 0;
       settled[1] = lanes_any[1] == 0;
+      if (half_tiles > 0) {
+        int32_t a00, b00, a10, b10, a01, b01, a11, b11, a4, b4;  // blocks and counts of (half, tile t or t + 1)
+        uint32_t ca00, cb00, ca10, cb10, ca01, cb01, ca11, cb11, ca4, cb4;
+        lookup_take(half_lookup(H0{}, 0), a00, ca00, b00, cb00);
+        lookup_take(half_lookup(H1{}, 0), a10, ca10, b10, cb10);
+        lookup_take(half_lookup(H0{}, 1), a01, ca01, b01, cb01);
+        lookup_take(half_lookup(H1{}, 1), a11, ca11, b11, cb11);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): (second walk) the first walk's last reads are done
+        dma_k(H0{}, a00, b00);
+        dma_k(H1{}, a10, b10);
+        __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): K(0) has landed
+        load_k(H0{});
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        dma_k(H0{}, a01, b01);
+        dma_v(H0{}, a00, b00);
+        static_for<4>([&](auto ks_tag) { mma_s(H0{}, ks_tag); });
+        __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): K(1) has landed
+        load_k(H1{});
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        dma_k(H1{}, a11, b11);
+#pragma unroll
+        for (int jj = 0; jj < 2; jj++) {  // nothing before unit 0: its PV slots add zero
+#pragma unroll
+          for (int e = 0; e < 8; e++) pf[1][jj][e] = (E)0.f;
+#pragma unroll
+          for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) vfr[jj][dt][e] = (E)0.f;
+        }
+        for (int t = 0; t < half_tiles; t++) {
+          int4 nx = half_lookup(H0{}, t + 2);
+          phase(H0{}, ca00, cb00, a10, b10, nx, a4, ca4, b4, cb4);
+          a00 = a01; b00 = b01; ca00 = ca01; cb00 = cb01;
+          a01 = a4; b01 = b4; ca01 = ca4; cb01 = cb4;
+          nx = half_lookup(H1{}, t + 2);
+          phase(H1{}, ca10, cb10, a00, b00, nx, a4, ca4, b4, cb4);
+          a10 = a11; b10 = b11; ca10 = ca11; cb10 = cb11;
+          a11 = a4; b11 = b4; ca11 = ca4; cb11 = cb4;
+        }
+        static_for<4>([&](auto i_tag) { mma_pv(H1{}, i_tag); });  // PV of the last unit
+      }
       if (ntiles > 0) {
         int32_t a0, b0, a1, b1, a2, b2, a3, b3;  // blocks and counts of tiles t .. t+3
         uint32_t ca0, cb0, ca1, cb1, ca2, cb2, ca3, cb3;
