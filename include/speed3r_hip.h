@@ -290,6 +290,22 @@ int s3r_layer_norm(const void* x, void* y, const void* w, const void* b, float e
                    int64_t sx, int64_t sy, int dtype, void* stream);
 
 /*
+ * Residual and the norm behind it:  s[r,:] = x[r,:] + gamma * a[r,:] rounded to the I/O dtype, y = LayerNorm(s) as
+ * s3r_layer_norm computes it.  The add (LayerScale with gamma, pi3/models/layers/block.py:281,296) and the next norm
+ * in one pass.  x, a, s, y: contiguous [rows, C], s and y apart from x and a; gamma, w, b: [C], gamma and b may be NULL.
+ */
+int s3r_add_layer_norm(const void* x, const void* a, const void* gamma, void* s, void* y, const void* w, const void* b, float eps,
+                       int64_t rows, int C, int dtype, void* stream);
+
+/*
+ * The layer's gate  out[r,:] = sigmoid(x[r,:] W^T + bias)  (pi3/models/layers/sparse_attention.py:88,127); fp32 sums, the
+ * product with its bias and the sigmoid each rounded to the I/O dtype.
+ *   x: contiguous [rows, C], w: contiguous [O, C], bias: [O] or NULL, out: contiguous [rows, O]; bf16 / fp16, C a multiple of
+ *   256 up to 1024, O even, up to 32.
+ */
+int s3r_gate(const void* x, const void* w, const void* bias, void* out, int64_t rows, int C, int O, int dtype, void* stream);
+
+/*
  * Gated merge of the two branches, written in the [B,N,H*D] layout the output projection
  * reads:  out[b,n,h*D+d] = gate[b,h,n,0]*o_cmp[b,h,n/block,d] + gate[b,h,n,1]*o_sel[b,h,n,d].
  * Replaces the einops/broadcast expression in pi3/models/layers/sparse_attention.py:127-136.

@@ -52,6 +52,25 @@ def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Ten
     return rope(t, pos) if pos is not None else t
 
 
+def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Optional[int] = None):
+    """``(pos, cos, sin, inv_freq, q_ln, k_ln, eps)`` for the kernels that take qk-norm and RoPE with the packed
+    projection, or None where their conditions do not hold (those of ``norm_rope_fused_or_eager`` for both norms)."""
+    def plain(norm):
+        return isinstance(norm, nn.Identity) or (type(norm) is nn.LayerNorm and norm.elementwise_affine)
+    same_kind = isinstance(attn.q_norm, nn.Identity) == isinstance(attn.k_norm, nn.Identity)
+    if not (qkv.is_cuda and qkv.shape[-1] == 192 * attn.num_heads and plain(attn.q_norm) and plain(attn.k_norm) and same_kind
+            and (pos is None or isinstance(attn.rope, RoPE2D))):
+        return None
+    ln = isinstance(attn.q_norm, nn.LayerNorm)
+    if ln and attn.q_norm.eps != attn.k_norm.eps:
+        return None
+    cos = sin = inv_freq = None
+    if pos is not None:
+        cos, sin, inv_freq = attn.rope.fused_tables(64, n_pos, qkv.device, qkv.dtype)
+    return (pos, cos, sin, inv_freq, (attn.q_norm.weight, attn.q_norm.bias) if ln else None,
+            (attn.k_norm.weight, attn.k_norm.bias) if ln else None, attn.q_norm.eps if ln else 0.0)
+
+
 class SparseFlashAttentionRope(nn.Module):
     def __init__(
         self,
@@ -97,23 +116,18 @@ class SparseFlashAttentionRope(nn.Module):
     def _norm_rope(self, t: Tensor, norm: nn.Module, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
         return norm_rope_fused_or_eager(t, norm, self.rope, pos, n_pos)
 
-    def _fused_args(self, qkv: Tensor, pos: Optional[Tensor], n_pos: Optional[int] = None):
-        """``(pos, cos, sin, inv_freq, q_ln, k_ln, eps)`` for the kernels that take qk-norm and RoPE with the packed
-        projection, or None where their conditions do not hold (those of ``norm_rope_fused_or_eager`` for both norms)."""
-        def plain(norm):
-            return isinstance(norm, nn.Identity) or (type(norm) is nn.LayerNorm and norm.elementwise_affine)
-        same_kind = isinstance(self.q_norm, nn.Identity) == isinstance(self.k_norm, nn.Identity)
-        if not (qkv.is_cuda and qkv.shape[-1] == 192 * self.num_heads and plain(self.q_norm) and plain(self.k_norm) and same_kind
-                and (pos is None or isinstance(self.rope, RoPE2D))):
-            return None
-        ln = isinstance(self.q_norm, nn.LayerNorm)
-        if ln and self.q_norm.eps != self.k_norm.eps:
-            return None
-        cos = sin = inv_freq = None
-        if pos is not None:
-            cos, sin, inv_freq = self.rope.fused_tables(64, n_pos, qkv.device, qkv.dtype)
-        return (pos, cos, sin, inv_freq, (self.q_norm.weight, self.q_norm.bias) if ln else None,
-                (self.k_norm.weight, self.k_norm.bias) if ln else None, self.q_norm.eps if ln else 0.0)
+    def _gate(self, x: Tensor) -> Tensor:
+        """``self.gate(x)`` for inference: one kernel where it is the plain pair of modules it was built as (their calls
+        carry nothing else: no hooks, no autocast, no replaced module)."""
+        def plain(m, kind):
+            return type(m) is kind and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+        if x.is_cuda and plain(self.gate, nn.Sequential) and len(self.gate) == 2 and plain(self.gate[0], nn.Linear) \
+                and plain(self.gate[1], nn.Sigmoid) and not torch.is_autocast_enabled("cuda") and "forward" not in self.gate[0].__dict__ \
+                and not (nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks):
+            out = ops.gate(x, self.gate[0].weight, self.gate[0].bias)
+            if out is not None:
+                return out
+        return self.gate(x)
 
     def _forward_with_grad(self, x: Tensor, xpos: Optional[Tensor]) -> Tensor:
         """The same layer for training.  Between its projections it is one differentiable operator whose forward and
@@ -129,7 +143,7 @@ class SparseFlashAttentionRope(nn.Module):
         qkv = self.qkv(x)
         gate = self.gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)              # [B, H, N, 2]
         use_pos = xpos is not None and self.rope is not None
-        fused = self._fused_args(qkv, xpos if use_pos else None)
+        fused = fused_qk_args(self, qkv, xpos if use_pos else None)
         if fused is not None and self.topk in (1, 2, 4, 8, 16, 32, 64):
             pos, cos, sin, inv_freq, q_ln, k_ln, eps = fused
             core = ops.layer_core_autograd(qkv, gate, h, block, self.topk, pos, cos, sin, inv_freq, q_ln, k_ln, eps)
@@ -180,7 +194,7 @@ class SparseFlashAttentionRope(nn.Module):
         block = self.block_size ** 2
 
         qkv = self.qkv(x)                                              # [B, N, 3C], layout (qkv h d)
-        gate = self.gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)       # [B, H, N, 2], strided view
+        gate = self._gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)      # [B, H, N, 2], strided view
 
         use_pos = xpos is not None and self.rope is not None
         pos = xpos if use_pos else None
@@ -189,7 +203,7 @@ class SparseFlashAttentionRope(nn.Module):
         # once.  Where that kernel is not built (head_dim other than 64, another norm or rope module): pooling kernel, then
         # norm/RoPE per tensor.  16-token blocks take the pass in two launches: the block means first, so that the index
         # kernel, long for so many pooled tokens, starts while the full tokens are still to come.
-        fused = self._fused_args(qkv, pos, n_pos)
+        fused = fused_qk_args(self, qkv, pos, n_pos)
         q = k = v = None
         self.last_prepass = False
         if fused is not None and (pos is not None or fused[4] is not None):   # (else q and k are read in place)

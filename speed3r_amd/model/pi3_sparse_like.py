@@ -36,7 +36,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from ..layers import RoPE2D, SparseFlashAttentionRope
-from ..layers.sparse_attention import norm_rope_fused_or_eager
+from ..layers.sparse_attention import fused_qk_args, norm_rope_fused_or_eager
 from ..sparse_attn import ops
 from .token_order import tile_major, tile_major_inverse
 
@@ -72,6 +72,18 @@ def token_norm(norm: nn.LayerNorm, x: Tensor) -> Tensor:
     return norm(x)
 
 
+def add_and_norm(x: Tensor, scale: nn.Module, branch: Tensor, norm: Optional[nn.LayerNorm]):
+    """``(s, norm(s))`` of the residual sum ``s = x + scale(branch)``: one pass for inference on the GPU (``norm=None``:
+    ``(s, None)``)."""
+    scaled = isinstance(scale, LayerScale)
+    if norm is not None and x.is_cuda and not torch.is_grad_enabled() and norm.elementwise_affine:
+        out = ops.add_layer_norm(x, branch, scale.gamma if scaled else None, norm.weight, norm.bias, norm.eps)
+        if out is not None:
+            return out
+    s = scale.add_to(x, branch) if scaled else x + branch
+    return s, token_norm(norm, s) if norm is not None else None
+
+
 class DenseAttentionRope(nn.Module):
     """Dense attention inside each sequence of the batch (one frame), optional qk-norm and RoPE2D."""
 
@@ -92,9 +104,17 @@ class DenseAttentionRope(nn.Module):
     def forward(self, x: Tensor, attn_bias=None, xpos: Optional[Tensor] = None, n_pos: Optional[int] = None) -> Tensor:
         b, n, c = x.shape
         h = self.num_heads
-        q, k, v = self.qkv(x).view(b, n, 3, h, c // h).permute(2, 0, 3, 1, 4).unbind(0)
+        qkv = self.qkv(x)
         pos = xpos if self.rope is not None else None
-        q, k = self._norm_rope(q, self.q_norm, pos, n_pos), self._norm_rope(k, self.k_norm, pos, n_pos)
+        fused = fused_qk_args(self, qkv, pos, n_pos) if not torch.is_grad_enabled() else None
+        qkv_out = None
+        if fused is not None and (pos is not None or fused[4] is not None):   # one pass over the projection for q and k
+            qkv_out = ops.qkv_prepass(qkv, h, 64, *fused[:3], *fused[4:], pooled=None, inv_freq=fused[3])
+        if qkv_out is not None:
+            q, k, v = qkv_out
+        else:
+            q, k, v = qkv.view(b, n, 3, h, c // h).permute(2, 0, 3, 1, 4).unbind(0)
+            q, k = self._norm_rope(q, self.q_norm, pos, n_pos), self._norm_rope(k, self.k_norm, pos, n_pos)
         if x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and c // h == 64 and not torch.is_grad_enabled():
             # the package's dense flash kernel (the compressed branch's attention), written straight into [B,N,H,D]
             o = torch.empty((b, n, h, c // h), dtype=x.dtype, device=x.device)
@@ -116,10 +136,28 @@ class Block(nn.Module):
         self.ls2 = LayerScale(dim, init_values) if init_values else nn.Identity()
 
     def forward(self, x: Tensor, xpos: Optional[Tensor] = None, n_pos: Optional[int] = None) -> Tensor:
-        a = self.attn(token_norm(self.norm1, x), xpos=xpos, n_pos=n_pos)
-        x = self.ls1.add_to(x, a) if isinstance(self.ls1, LayerScale) else x + a
-        m = self.mlp(token_norm(self.norm2, x))
-        return self.ls2.add_to(x, m) if isinstance(self.ls2, LayerScale) else x + m
+        return self._run(x, token_norm(self.norm1, x), None, xpos, n_pos)[0]
+
+    def step(self, x: Tensor, normed: Tensor, next_norm: Optional[nn.LayerNorm], xpos: Optional[Tensor] = None,
+             n_pos: Optional[int] = None):
+        """The block on ``x`` with ``normed = norm1(x)`` at hand: its output and, for the module behind it, ``next_norm`` of
+        that output (each residual sum meets its norm in one pass).  A block with hooks is called as a module."""
+        if self._forward_hooks or self._forward_pre_hooks:
+            x = self(x, xpos=xpos, n_pos=n_pos)
+            return x, token_norm(next_norm, x) if next_norm is not None else None
+        return self._run(x, normed, next_norm, xpos, n_pos)
+
+    def _run(self, x, normed, next_norm, xpos, n_pos):
+        x, y = add_and_norm(x, self.ls1, self.attn(normed, xpos=xpos, n_pos=n_pos), self.norm2)
+        return add_and_norm(x, self.ls2, self.mlp(y), next_norm)
+
+
+def run_blocks(blocks, x: Tensor, last_norm: Optional[nn.LayerNorm], **kw):
+    """``blocks`` in sequence: the last one's output and ``last_norm`` of it (None without)."""
+    y = token_norm(blocks[0].norm1, x) if len(blocks) else token_norm(last_norm, x) if last_norm is not None else None
+    for i, blk in enumerate(blocks):
+        x, y = blk.step(x, y, blocks[i + 1].norm1 if i + 1 < len(blocks) else last_norm, **kw)
+    return x, y
 
 
 class PatchEncoder(nn.Module):
@@ -153,9 +191,7 @@ class PatchEncoder(nn.Module):
         x = F.linear(x, self.patch_embed.weight.reshape(self.patch_embed.out_channels, -1), self.patch_embed.bias)
         x = torch.cat((self.cls_token.expand(f, -1, -1), x), dim=1) + self._pos(gh, gw)
         x = torch.cat((x[:, :1], self.register_tokens.expand(f, -1, -1), x[:, 1:]), dim=1)
-        for blk in self.blocks:
-            x = blk(x)
-        return token_norm(self.norm, x)[:, 1 + self.register_tokens.shape[1]:]
+        return run_blocks(self.blocks, x, self.norm)[1][:, 1 + self.register_tokens.shape[1]:]
 
 
 class HeadDecoder(nn.Module):
@@ -166,10 +202,7 @@ class HeadDecoder(nn.Module):
         self.linear_out = nn.Linear(dim, out_dim)
 
     def forward(self, x: Tensor, xpos: Tensor, n_pos: Optional[int] = None) -> Tensor:
-        x = self.project(x)
-        for blk in self.blocks:
-            x = blk(x, xpos=xpos, n_pos=n_pos)
-        return self.linear_out(x)
+        return self.linear_out(run_blocks(self.blocks, self.project(x), None, xpos=xpos, n_pos=n_pos)[0])
 
 
 class PixelShuffleHead(nn.Module):
@@ -261,11 +294,16 @@ class Pi3SparseLike(nn.Module):
             x, pos_dec = tile_major(x, gh, gw, self.tile), tile_major(pos, gh, gw, self.tile)
         else:
             pos_dec = pos
-        local_out = None
-        for local_blk, global_blk in zip(self.local_decoder, self.global_decoder):
-            x = local_blk(x, xpos=pos_dec, n_pos=n_pos)
+        local_out = normed = None
+        for i, (local_blk, global_blk) in enumerate(zip(self.local_decoder, self.global_decoder)):
+            if normed is None:
+                normed = token_norm(local_blk.norm1, x)
+            x, normed = local_blk.step(x, normed, global_blk.norm1, xpos=pos_dec, n_pos=n_pos)
             local_out = x
-            x = global_blk(x.reshape(b, f * t, -1), xpos=pos_dec.reshape(b, f * t, 2), n_pos=n_pos).reshape(b * f, t, -1)
+            flat = (b, f * t, -1)                                                  # the global block sees one sequence
+            x, normed = global_blk.step(x.reshape(flat), normed.reshape(flat), self.local_decoder[i + 1].norm1
+                                        if i + 1 < len(self.local_decoder) else None, xpos=pos_dec.reshape(b, f * t, 2), n_pos=n_pos)
+            x, normed = x.reshape(b * f, t, -1), normed.reshape(b * f, t, -1) if normed is not None else None
         feat = torch.cat((local_out, x), dim=-1)
         if tiled:                                                                  # the heads see row-major tokens again
             feat = tile_major_inverse(feat, gh, gw, self.tile)

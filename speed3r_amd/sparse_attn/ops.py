@@ -432,6 +432,51 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     return y.view(x.shape)
 
 
+def add_layer_norm(x: torch.Tensor, a: torch.Tensor, gamma: Optional[torch.Tensor], weight: torch.Tensor, bias: Optional[torch.Tensor],
+                   eps: float) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """``(s, layer_norm(s))`` of ``s = x + gamma * a`` (``gamma=None``: ``x + a``) in one pass (inference); the bits of the sum
+    followed by :func:`layer_norm`.  Returns None where that has no kernel, or where the tensors' types or forms differ."""
+    _need_device(x)
+    _forward_only(x, a)
+    c = x.shape[-1]
+    vec = 16 // x.element_size()
+    if x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or c % vec or c // vec > 512 or x.numel() == 0:
+        return None
+    params = [t for t in (gamma, weight, bias) if t is not None]
+    if x.shape != a.shape or any(t.shape != (c,) or not t.is_contiguous() for t in params) or not (x.is_contiguous() and a.is_contiguous()):
+        return None
+    if any(t.dtype != x.dtype or t.device != x.device or t.data_ptr() % 16 for t in (x, a, *params)):
+        return None
+    s, y = torch.empty_like(x), torch.empty_like(x)
+    with torch.cuda.device(x.device):
+        rc = _lib.lib().s3r_add_layer_norm(x.data_ptr(), a.data_ptr(), gamma.data_ptr() if gamma is not None else None, s.data_ptr(),
+                                           y.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
+                                           float(eps), x.numel() // c, c, _code(x), _stream(x))
+    _lib.check(rc, "s3r_add_layer_norm")
+    return s, y
+
+
+def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """``sigmoid(F.linear(x, weight, bias))`` for the few outputs of the layer's gate, in one pass over ``x`` (inference).
+
+    Returns None where the library has no kernel (bf16/fp16, channels a multiple of 256 up to 1024, an even number of
+    outputs up to 32, contiguous 16-byte aligned tensors of one dtype)."""
+    _need_device(x)
+    _forward_only(x, weight)
+    c, o = x.shape[-1], weight.shape[0]
+    ts = [t for t in (x, weight, bias) if t is not None]
+    if x.dtype not in (torch.bfloat16, torch.float16) or c % 256 or c > 1024 or o > 32 or o % 2 or x.numel() == 0 or weight.shape != (o, c):
+        return None
+    if any(t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
+        return None
+    out = x.new_empty((*x.shape[:-1], o))
+    with torch.cuda.device(x.device):
+        rc = _lib.lib().s3r_gate(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                                 x.numel() // c, c, o, _code(x), _stream(x))
+    _lib.check(rc, "s3r_gate")
+    return out
+
+
 def select_attn_merge(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, idx: torch.Tensor, o_cmp: torch.Tensor,
                       gate: torch.Tensor, block: int, softmax_scale: Optional[float] = None) -> Optional[torch.Tensor]:
     """``select_attn`` with ``gated_merge`` in its epilogue -> ``[B,N,H*D]``; bit-identical to the two calls, without the
