@@ -39,11 +39,11 @@ class RoPE2D(nn.Module):
         their rounding to ``dtype`` (the reference's table, pos_embed.py:121-131, without the duplicated half)."""
         key = (head_dim, n_pos, str(device), dtype)
         if key not in self._tables:
-            half = head_dim // 2
             inv_freq = self.inv_freq(head_dim, device)
-            t = torch.arange(n_pos, device=device, dtype=torch.float32)
-            ang = (t[:, None] * inv_freq).to(dtype)   # (a plain product: fp32 under autocast too)
-            self._tables[key] = (ang.cos().contiguous(), ang.sin().contiguous())
+            with torch.inference_mode(False), torch.no_grad():   # kept for training calls too, which save them
+                t = torch.arange(n_pos, device=device, dtype=torch.float32)
+                ang = (t[:, None] * inv_freq).to(dtype)   # (a plain product: fp32 under autocast too)
+                self._tables[key] = (ang.cos().contiguous(), ang.sin().contiguous())
         return self._tables[key]
 
     def inv_freq(self, head_dim: int, device) -> torch.Tensor:
@@ -51,7 +51,8 @@ class RoPE2D(nn.Module):
         key = (head_dim, str(device))
         if key not in self._tables:
             half = head_dim // 2
-            self._tables[key] = 1.0 / (self.base ** (torch.arange(0, half, 2, device=device, dtype=torch.float32) / half))
+            with torch.inference_mode(False), torch.no_grad():
+                self._tables[key] = 1.0 / (self.base ** (torch.arange(0, half, 2, device=device, dtype=torch.float32) / half))
         return self._tables[key]
 
     def _cos_sin(self, pos1d: torch.Tensor, half: int, dtype: torch.dtype):

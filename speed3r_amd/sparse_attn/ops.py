@@ -750,6 +750,8 @@ def layer_core_autograd(qkv: torch.Tensor, gate: torch.Tensor, heads: int, block
     if qkv.dtype not in (torch.bfloat16, torch.float16) or gate.dtype != qkv.dtype or qkv.shape[-1] != 3 * heads * 64 or block not in (64, 16) \
             or not qkv.is_contiguous():
         return None
+    if xpos is not None and xpos.is_inference():   # (such a tensor can't be saved for the backward)
+        xpos = xpos.clone()
     return _LayerCoreFn.apply(qkv, gate, *(q_ln or (None, None)), *(k_ln or (None, None)), xpos, cos, sin, inv_freq, heads, block, topk, eps)
 
 

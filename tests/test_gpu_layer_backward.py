@@ -3,7 +3,7 @@ through the torch expressions in fp64 (needs an MI355X)."""
 import pytest
 import torch
 
-from speed3r_amd.layers import RoPE2D, block_positions
+from speed3r_amd.layers import RoPE2D, SparseFlashAttentionRope, block_positions
 from speed3r_amd.sparse_attn import ops
 
 pytestmark = pytest.mark.gpu
@@ -123,3 +123,20 @@ def test_finished_block_means_and_split_passes(dtype, n, block, high):
              *ops.qkv_prepass(qkv, h, block, pos, cos, sin, *ln, 1e-6, tokens=False, pooled="final", inv_freq=inv))
     for a, w in zip(split, got):
         assert torch.equal(a, w)
+
+
+def test_training_after_inference_mode():
+    """Tables laid out, and positions made, in inference mode serve a training call (whose backward saves them)."""
+    torch.manual_seed(0)
+    layer = SparseFlashAttentionRope(128, num_heads=2, qkv_bias=True, qk_norm=True, rope=RoPE2D(100.0), block_size=8, topk=2).to(DEV, torch.bfloat16)
+    x = torch.randn((1, 130, 128), device=DEV, dtype=torch.bfloat16)
+    with torch.inference_mode():
+        pos = torch.randint(0, 30, (1, 130, 2), device=DEV)
+        layer(x, xpos=pos)
+    got = torch.autograd.grad(layer(x, xpos=pos).float().square().sum(), list(layer.parameters()))
+    layer.rope._tables.clear()
+    want = torch.autograd.grad(layer(x, xpos=pos.clone()).float().square().sum(), list(layer.parameters()))
+    assert all(torch.isfinite(g).all() for g in got)
+    assert torch.equal(layer(x, xpos=pos), layer(x, xpos=pos.clone()))
+    # two runs of the same kernels: the bits may differ only where a reduction's order does (one rounding of the result)
+    assert all(_close(g, w, torch.bfloat16, steps=1) for g, w in zip(got, want))

@@ -117,3 +117,11 @@ def test_patch_embedding_as_one_gemm_equals_the_convolution():
     f, gh, gw = 2, 3, 2
     x = torch.cat((enc.cls_token.expand(f, -1, -1), want), dim=1) + enc._pos(gh, gw)
     assert torch.allclose(got, enc.norm(x)[:, 1:], atol=1e-5)
+
+
+def test_rotation_tables_made_in_inference_mode_serve_training():
+    """The tables outlive the call that lays them out: autograd must be able to save them later."""
+    rope = RoPE2D(100.0)
+    with torch.inference_mode():
+        tables = rope.fused_tables(64, None, torch.device("cpu"), torch.bfloat16)
+    assert not any(t.is_inference() for t in tables)
