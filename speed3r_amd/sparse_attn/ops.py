@@ -10,6 +10,7 @@ dimension; indices are int32 ``[B, H, n_query_blocks, K]`` in block units.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
 import os
@@ -36,8 +37,19 @@ def _need_device(*ts: torch.Tensor) -> None:
             raise RuntimeError("speed3r_amd operators run on HIP device tensors only (got a CPU tensor)")
 
 
+# A short call is bound by the host: a stream object and a device guard per launch were 20 of the 280 us of two views
+# through the layer and 16 of the 137 us of one view through the operators.  The raw stream is asked for directly, and the
+# guard is entered only where another device is current.
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """Makes ``device`` the current one for a launch."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def _last_contig(t: torch.Tensor) -> torch.Tensor:
@@ -61,7 +73,7 @@ def pool_mean(x: torch.Tensor, block: int) -> torch.Tensor:
     b, h, n, d = x.shape
     nc = -(-n // block)
     y = torch.empty((b, h, nc, d), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.lib().s3r_pool_mean(x.data_ptr(), y.data_ptr(), b, h, n, d, block,
                                       x.stride(0), x.stride(1), x.stride(2),
                                       y.stride(0), y.stride(1), y.stride(2), _code(x), _stream(x))
@@ -132,7 +144,7 @@ def compressed_attn_topk(q: torch.Tensor, k: torch.Tensor, v: Optional[torch.Ten
             scores = torch.full((b, h, lq, lk), float("nan"), dtype=torch.float32, device=q.device) if return_scores \
                 else torch.empty((b, h, lq, lk), dtype=torch.float32, device=q.device)
         st3 = lambda t: (t.stride(0), t.stride(1), t.stride(2))
-        with torch.cuda.device(q.device):
+        with _on(q.device):
             rc = _lib.lib().s3r_compressed_attn_topk_causal(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr() if lse is not None else None,
                 idx.data_ptr() if idx is not None else None, scores.data_ptr() if scores is not None else None,
@@ -173,7 +185,7 @@ def compressed_attn_topk(q: torch.Tensor, k: torch.Tensor, v: Optional[torch.Ten
     st3 = lambda t: (t.stride(0), t.stride(1), t.stride(2))
 
     def launch(q_, o_, lse_, idx_, scores_, rows):
-        with torch.cuda.device(q.device):
+        with _on(q.device):
             rc = _lib.lib().s3r_compressed_attn_topk(
                 q_.data_ptr(), k.data_ptr(), None if indices_only else v.data_ptr(), None if indices_only else o_.data_ptr(),
                 lse_.data_ptr() if lse_ is not None else None,
@@ -221,7 +233,7 @@ def topk_rows(scores: torch.Tensor, k: int) -> torch.Tensor:
     cols = scores.shape[-1]
     rows = scores.numel() // cols
     idx = torch.empty((*scores.shape[:-1], k), dtype=torch.int32, device=scores.device)
-    with torch.cuda.device(scores.device):
+    with _on(scores.device):
         rc = _lib.lib().s3r_topk_rows(scores.data_ptr(), idx.data_ptr(), rows, cols, cols, k, _stream(scores))
     _lib.check(rc, "s3r_topk_rows")
     return idx
@@ -259,7 +271,7 @@ def select_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, idx: torch.Te
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
     o = torch.empty_like(q, memory_format=torch.contiguous_format)
     lse = torch.empty((b, h, n), dtype=torch.float32, device=q.device) if return_lse else None
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         rc = _lib.lib().s3r_select_attn(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), idx.data_ptr(), o.data_ptr(),
             lse.data_ptr() if lse is not None else None,
@@ -286,7 +298,7 @@ def gated_merge(o_cmp: torch.Tensor, o_sel: torch.Tensor, gate: torch.Tensor, bl
     assert o_cmp.shape == (b, h, nc, d), f"o_cmp shape {tuple(o_cmp.shape)} != {(b, h, nc, d)}"
     assert gate.shape == (b, h, n, 2), f"gate shape {tuple(gate.shape)} != {(b, h, n, 2)}"
     out = torch.empty((b, n, h * d), dtype=o_sel.dtype, device=o_sel.device)
-    with torch.cuda.device(o_sel.device):
+    with _on(o_sel.device):
         rc = _lib.lib().s3r_gated_merge(
             o_cmp.data_ptr(), o_sel.data_ptr(), gate.data_ptr(), out.data_ptr(), b, h, n, d, block,
             o_cmp.stride(0), o_cmp.stride(1), o_cmp.stride(2), o_sel.stride(0), o_sel.stride(1), o_sel.stride(2),
@@ -321,7 +333,7 @@ def norm_rope(x: torch.Tensor, positions: Optional[torch.Tensor], cos_tab: Optio
     w = ln_weight.detach().to(x.dtype).contiguous() if ln_weight is not None else None
     bias = ln_bias.detach().to(x.dtype).contiguous() if (ln_bias is not None and w is not None) else None
     y = torch.empty((b, h, n, d), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.lib().s3r_norm_rope(
             x.data_ptr(), y.data_ptr(), pos32.data_ptr() if pos32 is not None else None,
             cos_tab.data_ptr() if pos32 is not None else None, sin_tab.data_ptr() if pos32 is not None else None, p,
@@ -402,7 +414,7 @@ def qkv_prepass(qkv: torch.Tensor, num_heads: int, block: int, positions: Option
         if keep_raw:
             a.q_raw, a.k_raw = means[3].data_ptr(), means[4].data_ptr()
         out += means
-    with torch.cuda.device(qkv.device):
+    with _on(qkv.device):
         rc = _lib.lib().s3r_layer_prepass(ctypes.byref(a), _stream(qkv))
     _lib.check(rc, "s3r_layer_prepass")
     return out
@@ -425,7 +437,7 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     w = weight.detach().to(x.dtype).contiguous()
     b = bias.detach().to(x.dtype).contiguous() if bias is not None else None
     y = torch.empty_like(x2)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.lib().s3r_layer_norm(x2.data_ptr(), y.data_ptr(), w.data_ptr(), b.data_ptr() if b is not None else None,
                                        float(eps), x2.shape[0], c, x2.stride(0), y.stride(0), _code(x), _stream(x))
     _lib.check(rc, "s3r_layer_norm")
@@ -448,7 +460,7 @@ def add_layer_norm(x: torch.Tensor, a: torch.Tensor, gamma: Optional[torch.Tenso
     if any(t.dtype != x.dtype or t.device != x.device or t.data_ptr() % 16 for t in (x, a, *params)):
         return None
     s, y = torch.empty_like(x), torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.lib().s3r_add_layer_norm(x.data_ptr(), a.data_ptr(), gamma.data_ptr() if gamma is not None else None, s.data_ptr(),
                                            y.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
                                            float(eps), x.numel() // c, c, _code(x), _stream(x))
@@ -470,7 +482,7 @@ def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) ->
     if any(t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
         return None
     out = x.new_empty((*x.shape[:-1], o))
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.lib().s3r_gate(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
                                  x.numel() // c, c, o, _code(x), _stream(x))
     _lib.check(rc, "s3r_gate")
@@ -500,7 +512,7 @@ def select_attn_merge(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, idx: to
         return None
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
     out = torch.empty((b, n, h * d), dtype=q.dtype, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         rc = _lib.lib().s3r_select_attn_merge(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), idx.data_ptr(), o_cmp.data_ptr(), gate.data_ptr(), out.data_ptr(),
             b, h, n, d, block, idx.shape[3],
@@ -533,7 +545,7 @@ def key_block_lists(idx: torch.Tensor, n_key_blocks: int) -> Tuple[torch.Tensor,
     b, h, nqb, kk = idx.shape
     lists = torch.empty((b, h, nqb * kk), dtype=torch.int32, device=idx.device)
     off = torch.empty((b, h, n_key_blocks + 1), dtype=torch.int32, device=idx.device)
-    with torch.cuda.device(idx.device):
+    with _on(idx.device):
         rc = _lib.lib().s3r_key_block_lists(idx.data_ptr(), lists.data_ptr(), off.data_ptr(), b, h, nqb, kk, n_key_blocks,
                                             idx.stride(0), idx.stride(1), idx.stride(2), nqb * kk, _stream(idx))
     _lib.check(rc, "s3r_key_block_lists")
@@ -564,7 +576,7 @@ def attn_bwd_delta(o: torch.Tensor, dout: torch.Tensor) -> torch.Tensor:
     o, dout = _last_contig(o), _last_contig(dout)
     b, h, n, d = o.shape
     delta = torch.empty((b, h, n), dtype=torch.float32, device=o.device)
-    with torch.cuda.device(o.device):
+    with _on(o.device):
         rc = _lib.lib().s3r_attn_bwd_delta(o.data_ptr(), dout.data_ptr(), delta.data_ptr(), b, h, n, d,
                                            o.stride(0), o.stride(1), o.stride(2),
                                            dout.stride(0), dout.stride(1), dout.stride(2), _code(o), _stream(o))
@@ -611,7 +623,7 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     def st(t):
         return (t.stride(0), t.stride(1), t.stride(2)) if t is not None else (0, 0, 0)
 
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         rc = _lib.lib().s3r_attn_bwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), lse.data_ptr(), delta.data_ptr(),
             idx.data_ptr() if idx is not None else None,
@@ -676,7 +688,7 @@ def gated_merge_bwd(dout: torch.Tensor, o_cmp: torch.Tensor, o_sel: torch.Tensor
     d_gate = gate.new_empty((b, n, h, 2))
     delta_c = torch.empty(o_cmp.shape[:3], dtype=torch.float32, device=gate.device)
     delta_s = torch.empty((b, h, n), dtype=torch.float32, device=gate.device)
-    with torch.cuda.device(gate.device):
+    with _on(gate.device):
         rc = _lib.lib().s3r_gated_merge_bwd(
             dout.data_ptr(), o_cmp.data_ptr(), o_sel.data_ptr(), gate.data_ptr(), d_oc.data_ptr(), d_os.data_ptr(), d_gate.data_ptr(),
             delta_c.data_ptr(), delta_s.data_ptr(), b, h, n, d, block, gate.stride(0), gate.stride(1), gate.stride(2), _code(gate), _stream(gate))
@@ -701,7 +713,7 @@ def qkv_prepass_bwd(qkv: torch.Tensor, num_heads: int, block: int, positions, co
     if q_ln is not None:
         work = torch.empty((PREPASS_BWD_ROWS + 1, 256), dtype=torch.float32, device=qkv.device)
         d_norm = work[PREPASS_BWD_ROWS].view(4, 64)
-    with torch.cuda.device(qkv.device):
+    with _on(qkv.device):
         rc = _lib.lib().s3r_layer_prepass_bwd(ctypes.byref(a), *(t.data_ptr() for t in grads), *off,
                                               d_norm.data_ptr() if d_norm is not None else None,
                                               work.data_ptr() if work is not None else None, PREPASS_BWD_ROWS, _stream(qkv))
