@@ -218,9 +218,9 @@ class SparseFlashAttentionRope(nn.Module):
             pos_c = block_positions(xpos, block) if use_pos else None
             q_c, k_c = self._norm_rope(q_c, self.q_norm, pos_c, n_pos), self._norm_rope(k_c, self.k_norm, pos_c, n_pos)
         # the index kernel needs pooled q and k only and its result is first read by the selection kernel: where
-        # it is a kernel of its own it runs on a second stream, beside the compressed attention (and the norm/RoPE of
+        # it is a kernel of its own, and long enough, it runs on a second stream, beside the compressed attention (and the norm/RoPE of
         # the full tokens where they come after it)
-        side = x.is_cuda and ops._two_kernel_compressed(q_c, self.topk)
+        side = x.is_cuda and ops._indices_beside(q_c, self.topk)
         if side:
             idx, join = ops.topk_indices_on_side_stream(q_c, k_c, self.topk)
             o_c, _ = ops.compressed_attn_topk(q_c, k_c, v_c, None)

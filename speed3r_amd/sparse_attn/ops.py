@@ -810,6 +810,20 @@ def _two_kernel_compressed(q: torch.Tensor, topk: int, block: int = 1) -> bool:
             and -(-q.shape[2] // block) <= (1 << 21) and _lib.lib_has_fused_topk())
 
 
+# Pooled rows (B * H * blocks) from which the index kernel goes on a stream of its own.  The two events and the change of
+# stream cost the host 60 to 80 us and the kernels behind them a wait between queues; what there is to hide is the dense
+# sweep's 12 to 16 us and the norm/RoPE pass.  us per call, two streams / one, 16 heads: layer, two views at 16-token blocks
+# (126 pooled tokens) 259 / 183, eight views (504) 286 / 253, 16 (1 008) 384 / 400, 32 (2 016) 701 / 747; operators, one view
+# (63) 118 / 61, eight (504) 131 / 122, 16 (1 008) 147 / 146; at 64-token blocks 8 frames (130) 127 / 94, 32 (518) 259 / 254.
+SIDE_STREAM_ROWS = 16 * 512
+
+
+def _indices_beside(q: torch.Tensor, topk: int, block: int = 1) -> bool:
+    """True where the index kernel runs on the side stream (arguments as for :func:`_two_kernel_compressed`)."""
+    rows = q.shape[0] * q.shape[1] * -(-q.shape[2] // block)
+    return rows > SIDE_STREAM_ROWS and _two_kernel_compressed(q, topk, block)
+
+
 def topk_indices_on_side_stream(qc: torch.Tensor, kc: torch.Tensor, topk: int, softmax_scale: Optional[float] = None):
     """Launch the index kernel (top-k columns of the raw scores ``qc kc^T``, no score buffer) on the device's side
     stream, ordered after the work already queued on the current stream.  Returns ``(idx, join)``; call ``join()``
@@ -840,7 +854,7 @@ def sparse_global_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g
     The merge runs in the selection kernel's epilogue where the library offers it (same bits either way);
     ``return_parts`` needs the selection output and therefore runs the two operators separately.
 
-    ``overlap`` (default: on where it applies): the indices need pooled q and k only, the compressed attention output
+    ``overlap`` (default: on from ``SIDE_STREAM_ROWS`` pooled rows; True: wherever it applies): the indices need pooled q and k only, the compressed attention output
     is not read before the merge.  Where the two come from different kernels (no score buffer), the index kernel runs
     on a second stream next to the pooling of v and the compressed attention (same kernels, same results; only the
     schedule differs).  The index kernel alone leaves most of the chip idle below a few thousand pooled tokens (one
@@ -858,7 +872,7 @@ def sparse_global_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g
 
     mark("start")
     if overlap is not False and materialize_scores is not True and not return_parts and q.is_cuda \
-            and _two_kernel_compressed(q, topk, block):
+            and (_two_kernel_compressed if overlap else _indices_beside)(q, topk, block):
         qc, kc = pool_mean(q, block), pool_mean(k, block)
         idx, join = topk_indices_on_side_stream(qc, kc, topk, softmax_scale)
         vc = pool_mean(v, block)

@@ -251,3 +251,15 @@ def test_layer_takes_the_one_pass_route_where_it_is_built():
         m3 = SparseFlashAttentionRope(dim=128, num_heads=2, qk_norm=True, rope=RoPE2D(100.0), block_size=4, topk=4).to(torch.bfloat16).to(DEV).eval()
         m3(x, xpos=pos)                         # 16-token blocks: separate kernels, the index kernel starts earlier
         assert m3.last_prepass is False and m3.last_path == "fused-merge"
+
+
+@pytest.mark.parametrize("n,block,topk", [(8192, 16, 32), (8193, 16, 32), (8207, 16, 4), (100, 64, 2)])
+def test_operators_give_the_same_bits_on_one_stream_and_on_two(n, block, topk):
+    """Around the line where the index kernel moves to a stream of its own (512 blocks x 16 heads), and below it."""
+    import speed3r_amd as s3r
+
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn((1, 16, n, 64), generator=g).to(torch.bfloat16).cuda() for _ in range(3))
+    gate = torch.rand((1, 16, n, 2), generator=g).to(torch.bfloat16).cuda()
+    got = [s3r.sparse_global_attention(q, k, v, gate, block, topk, overlap=o) for o in (None, True, False)]
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
