@@ -36,12 +36,14 @@ constexpr int kHalfBytes = 32 * 128;
 // (measured on the walk before the pipeline: 4 waves 1.71 ms, 2: 1.50 ms, 1: 1.42 ms at 266 496 tokens, top-32).
 constexpr int kWaves = S3R_B16_WAVES;
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr int kHalfList = 132;  // places of a half's own list (2 x 64 entries; an even number: entries are read in pairs)
+constexpr int kHalfList = 132;  // places of a half's own list (2 x 64 entries and a gap; an even number: entries are read in pairs)
 // One walk per half where the longer half's list has at most this share of the distinct blocks of all four lists.  A unit
 // costs the same either way and there are 2 max(n0, n1) of them instead of 2 n; the walks per half fetch n0 + n1 blocks
 // instead of n.  Thresholds from 60 to 100 % measured (us, top-32): lists of 98 distinct blocks at 32 256 tokens 271 without,
 // 248 / 246 / 246 at 60 / 70 / 90 %; 105 at 8 064 tokens 83 without, 74 / 68.5 / 68.5; lists of 38 (halves 35) at 266 496
 // tokens 1 010 without, 985 / 980 / 980, and 1 230 at 100 %, where the walks per half fetch everything twice for nothing.
+// (Measured with references from the walk's own tiles.  Those of the common walk's, which make the results of both the
+// same bits, cost 1 us at 2 016 tokens and 3 at 32 256: 39.4 and 254 us, 41.8 and 273 without the walk per half.)
 constexpr int kSplitNum = 4, kSplitDen = 5;
 typedef std::integral_constant<int, 0> H0;
 typedef std::integral_constant<int, 1> H1;
@@ -86,12 +88,20 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
   // The four index rows of the group, one entry per lane.  They head the longest dependency chain of the start-up
   // (rows -> walk list -> first tiles): their loads go first, ahead of the Q rows in the memory queue.
   int32_t my_idx[4];
+  auto read_lists = [&]() {
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int qb = grp * 4 + j;
-    my_idx[j] = -1;
-    if (qb < nqb && lane < p.K) my_idx[j] = __builtin_nontemporal_load(p.idx + ((int64_t)b * p.sib + (int64_t)h * p.sih + (int64_t)qb * p.sim + lane));
-  }
+    for (int j = 0; j < 4; j++) {
+      const int qb = grp * 4 + j;
+      my_idx[j] = -1;
+      if (qb < nqb && lane < p.K) my_idx[j] = __builtin_nontemporal_load(p.idx + ((int64_t)b * p.sib + (int64_t)h * p.sih + (int64_t)qb * p.sim + lane));
+    }
+  };
+  auto drop_invalid = [&]() {
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (my_idx[j] < 0 || (int64_t)my_idx[j] * 16 >= N) my_idx[j] = -1;
+  };
+  read_lists();
   __builtin_amdgcn_sched_barrier(0);
   // B operand Q: lane = query row, head_dim chunk hh + 2 ks
   V8 bq[2][4];
@@ -106,9 +116,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
       bq[qt][ks] = as_v8<E>(f);
     }
   }
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-    if (my_idx[j] < 0 || (int64_t)my_idx[j] * 16 >= N) my_idx[j] = -1;
+  drop_invalid();
 
   f32x16 ot[2][2];  // O^T [dt][qt]
 #pragma unroll
@@ -244,8 +252,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
   if constexpr (UNION) {
     // Neighbouring query blocks list mostly the same key blocks.  The wave therefore walks the UNION of its four
     // lists: a tile is two distinct key blocks A, B (rows 0-15, 16-31), fetched once, and every one of the 64 queries
-    // whose block lists A (B) uses its 16 scores against A (B).  The visiting order differs from the lists' order,
-    // which changes fp32 summation order only.
+    // whose block lists A (B) uses its 16 scores against A (B).  The visiting order differs from the lists' order: it
+    // decides the fp32 summation order and, through the tile that a query's softmax reference is taken from, against
+    // what its probabilities are rounded to the I/O dtype.  The walk per half visits in the common walk's order and
+    // takes its references, so that both give the same bits.
     //
     // 1. The walk list is built first, in LDS: entry n holds a distinct block and four count bytes (how often query
     //    block j lists it; 0: not at all, above 1: a duplicated entry, which attends the block that often).
@@ -270,14 +280,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
     // order is the table's, which is as good as any.
     int n_union = 0;
     int half_tiles = 0;  // tiles per half where each half walks its own union; 0: one walk for both
-    uint32_t cnt_bits = 0;
-    {
+    bool dup = false;    // some list names a block more than once (wave-uniform)
+    auto build_walk = [&](bool may_split) {
       int32_t* const hkey = reinterpret_cast<int32_t*>(k_buf[0]);          // [512]
       uint32_t* const hcnt = reinterpret_cast<uint32_t*>(k_buf[0] + 2048);  // [512]
       reinterpret_cast<int4*>(hkey)[lane] = make_int4(-1, -1, -1, -1);
       reinterpret_cast<int4*>(hkey)[lane + 64] = make_int4(-1, -1, -1, -1);
       reinterpret_cast<int4*>(hcnt)[lane] = make_int4(0, 0, 0, 0);
       reinterpret_cast<int4*>(hcnt)[lane + 64] = make_int4(0, 0, 0, 0);
+      ragged_cnts = 0;
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const int32_t e = my_idx[j];
@@ -298,8 +309,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
       const int4 c0 = reinterpret_cast<const int4*>(hcnt)[2 * lane], c1 = reinterpret_cast<const int4*>(hcnt)[2 * lane + 1];
       const int32_t ks8[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
       const int32_t cs8[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+      uint32_t cnt_bits = 0;
       uint32_t pos = 0, pos0 = 0, pos1 = 0;  // occupied slots of the lanes below: all, with a count of half 0, of half 1
       int n_half[2] = {0, 0};
+      n_union = 0;
 #pragma unroll
       for (int s8 = 0; s8 < 8; s8++) {
         const uint64_t m0 = __ballot((cs8[s8] & 0xffff) != 0), m1 = __ballot(((uint32_t)cs8[s8] >> 16) != 0), m = m0 | m1;
@@ -312,31 +325,76 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
         cnt_bits |= (uint32_t)cs8[s8];
       }
       // Lists that share little: one walk per half (a half without a list of its own keeps to the common walk).
-      const int longer = n_half[0] > n_half[1] ? n_half[0] : n_half[1];
-      if (n_half[0] > 0 && n_half[1] > 0 && longer * kSplitDen <= n_union * kSplitNum) half_tiles = (longer + 1) >> 1;
-      if (half_tiles == 0) {
+      int longer = n_half[0] > n_half[1] ? n_half[0] : n_half[1];
+      const bool split = may_split && n_half[0] > 0 && n_half[1] > 0 && longer * kSplitDen <= n_union * kSplitNum;
+      if (!split) {
+        half_tiles = 0;
 #pragma unroll
         for (int s8 = 0; s8 < 8; s8++)
           if (ks8[s8] >= 0) walk[pos++] = make_int2(ks8[s8], cs8[s8]);
         if (lane == 0) walk[n_union] = make_int2(-1, 0);
       } else {
+        // The halves' lists keep the order of the common one, so that every sum adds up in its order.  The count bytes that
+        // belong to the other half hold the block's tile of the common walk: `pre` takes a query's reference over the
+        // blocks of ONE such tile, as the common walk does, so that the result is the same whichever way is taken.
         pos1 += kHalfList;
 #pragma unroll
         for (int s8 = 0; s8 < 8; s8++) {
-          if ((cs8[s8] & 0xffff) != 0) walk[pos0++] = make_int2(ks8[s8], cs8[s8]);
-          if (((uint32_t)cs8[s8] >> 16) != 0) walk[pos1++] = make_int2(ks8[s8], cs8[s8]);
+          const uint32_t c = (uint32_t)cs8[s8], tile = pos >> 1;
+          if ((c & 0xffff) != 0) walk[pos0++] = make_int2(ks8[s8], (int32_t)((c & 0xffffu) | (tile << 16)));
+          if ((c >> 16) != 0) walk[pos1++] = make_int2(ks8[s8], (int32_t)((c & 0xffff0000u) | tile));
+          pos += c != 0;
         }
-        // the shorter list, and an odd one, goes on with its first block, counted by nobody
+        // Two blocks of one common tile that are the first ones of a query block's list must meet in a tile here too.  A
+        // list's first place is even; where the half's other query block begins at an odd place with such a pair, a place
+        // that counts for nobody goes in front of it.
+        int2 e[2][2];     // [half][places lane and 64 + lane]
+        int behind[2][2];  // counts at the next place
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+          for (int qt = 0; qt < 2; qt++) {
+            e[qt][u] = walk[qt * kHalfList + 64 * u + lane];
+            behind[qt][u] = walk[qt * kHalfList + 64 * u + lane + 1].y;
+          }
+        const int2 head[2] = {walk[0], walk[kHalfList]};
 #pragma unroll
         for (int qt = 0; qt < 2; qt++) {
-          const int first = walk[qt * kHalfList].x;
-          for (int i = n_half[qt] + lane; i < 2 * half_tiles; i += 64) walk[qt * kHalfList + i] = make_int2(first, 0);
+          const int n = n_half[qt];
+          int gap = -1;
+#pragma unroll
+          for (int j = 0; j < 2; j++) {
+            const uint32_t byte = 0xffu << (16 * qt + 8 * j);
+            int u = 0;
+            uint64_t has = __ballot(lane < n && ((uint32_t)e[qt][0].y & byte) != 0);
+            uint64_t pair = __ballot(lane + 1 < n && (((e[qt][0].y ^ behind[qt][0]) >> (qt ? 0 : 16)) & 0xffff) == 0 && ((uint32_t)behind[qt][0] & byte) != 0);
+            if (has == 0 && n > 64) {
+              u = 1;
+              has = __ballot(64 + lane < n && ((uint32_t)e[qt][1].y & byte) != 0);
+              pair = __ballot(65 + lane < n && (((e[qt][1].y ^ behind[qt][1]) >> (qt ? 0 : 16)) & 0xffff) == 0 && ((uint32_t)behind[qt][1] & byte) != 0);
+            }
+            const uint64_t first = has & -has;
+            if ((first & pair & 0xAAAAAAAAAAAAAAAAull) != 0) gap = 64 * u + __builtin_ctzll(first);
+          }
+          if (gap >= 0) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+              const int i = 64 * u + lane;
+              if (i >= gap && i < n) walk[qt * kHalfList + i + 1] = e[qt][u];
+            }
+            if (lane == 0) walk[qt * kHalfList + gap] = make_int2(head[qt].x, 0);
+            n_half[qt]++;
+          }
         }
+        longer = n_half[0] > n_half[1] ? n_half[0] : n_half[1];
+        half_tiles = (longer + 1) >> 1;
+        // the shorter list, and an odd one, goes on with its first block, counted by nobody
+#pragma unroll
+        for (int qt = 0; qt < 2; qt++)
+          for (int i = n_half[qt] + lane; i < 2 * half_tiles; i += 64) walk[qt * kHalfList + i] = make_int2(head[qt].x, 0);
       }
-      cnt_bits = __any((cnt_bits & 0xfefefefeu) != 0) ? 2u : 0u;
-      cnt_bits |= ragged_cnts;
-    }
-    const bool dup = (cnt_bits & 0xfefefefeu) != 0;  // some list names a block more than once (wave-uniform)
+      dup = __any((cnt_bits & 0xfefefefeu) != 0) || (ragged_cnts & 0xfefefefeu) != 0;
+    };
     // tile tau = entries 2 tau, 2 tau + 1 of the walk list (-1 / no counts beyond its end): the read is issued early
     // and its result taken where it is needed
     auto lookup_issue = [&](int tau) -> int4 {
@@ -440,8 +498,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
     // holds a block of its list and then stays (softmax is shift invariant), so later tiles need no maximum, no
     // comparison and no pass over the accumulators; probabilities may exceed 1, and a row sum that ends up huge or
     // not finite sends the group through a second walk with the running maximum (exact == true).
-    auto pre = [&](auto qt_tag, uint32_t ca, uint32_t cb) {
+    // SPLIT: the walk per half, whose tiles may pair blocks of two tiles of the common walk: those of the first one count.
+    auto pre = [&](auto qt_tag, uint32_t ca, uint32_t cb, auto split_tag) {
       constexpr int QT = decltype(qt_tag)::value;
+      constexpr bool SPLIT = decltype(split_tag)::value;
       const uint32_t pa = (ca >> (16 * QT)) & 0xffffu, pb = (cb >> (16 * QT)) & 0xffffu;  // the half's two query blocks
       const int wa = (int)(mine ? pa >> 8 : pa & 0xffu), wb = (int)(mine ? pb >> 8 : pb & 0xffu);
       if (exact || !settled[QT]) {  // (wave-uniform) once every query with a list has its reference, none of this runs
@@ -453,7 +513,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
             mxa = fmaxf(mxa, st[QT][r]);
             mxb = fmaxf(mxb, st[QT][8 + r]);
           }
-          float mx = fmaxf(wa ? mxa : -INFINITY, wb ? mxb : -INFINITY);
+          const bool one_tile = !SPLIT || (((ca ^ cb) >> (QT ? 0 : 16)) & 0xffffu) == 0;
+          float mx = fmaxf(wa ? mxa : -INFINITY, wb && (one_tile || !wa) ? mxb : -INFINITY);
           mx = xh_max(mx) * sl2;
           const float m_new = (exact || unset) ? fmaxf(m_i[QT], mx) : m_i[QT];
           if (__any(m_new != m_i[QT])) {
@@ -528,7 +589,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
                     int32_t& a3, uint32_t& ca3, int32_t& b3, uint32_t& cb3) {
       constexpr int P = decltype(par_tag)::value;
       typedef std::integral_constant<int, P ^ 1> Q;
-      pre(H0{}, ca, cb);
+      pre(H0{}, ca, cb, std::false_type{});
       static_for<8>([&](auto j_tag) {  // exponentials of (t, 0); scores of (t, 1); PV of (t-1, 1)
         constexpr int j = decltype(j_tag)::value;
         if constexpr (j == 4) {
@@ -542,7 +603,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
       });
       exps_tail(H0{});
       load_v(par_tag);  // V(t)
-      pre(H1{}, ca, cb);
+      pre(H1{}, ca, cb, std::false_type{});
       static_for<8>([&](auto j_tag) {  // exponentials of (t, 1); scores of (t+1, 0); PV of (t, 0)
         constexpr int j = decltype(j_tag)::value;
         if constexpr (j == 2) {
@@ -567,7 +628,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
                      int32_t& a4, uint32_t& ca4, int32_t& b4, uint32_t& cb4) {
       constexpr int QT = decltype(qt_tag)::value;
       typedef std::integral_constant<int, QT ^ 1> O;
-      pre(qt_tag, ca, cb);
+      pre(qt_tag, ca, cb, std::true_type{});
       static_for<8>([&](auto j_tag) {
         constexpr int j = decltype(j_tag)::value;
         if constexpr (j == 1) {
@@ -599,9 +660,19 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
       return v;
     };
 
-    const int ntiles = half_tiles > 0 ? 0 : (n_union + 1) >> 1;
     for (int pass = 0; pass < 2; pass++) {
       exact = pass == 1;
+      if (pass == 0 || half_tiles > 0) {  // the second walk is always the common one
+        if (pass == 1) {
+          read_lists();
+          drop_invalid();
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): the first walk's transfers and reads are done
+          asm volatile("" ::: "memory");
+        }
+        build_walk(pass == 0);
+      }
+      const int ntiles = half_tiles > 0 ? 0 : (n_union + 1) >> 1;
       settled[0] = lanes_any[0] == 0;
       settled[1] = lanes_any[1] == 0;
       if (half_tiles > 0) {
@@ -706,7 +777,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void select_b16_kernel(AttnParams p
 #pragma unroll
           for (int j = 0; j < 8; j++)
             if (4 * hh + 8 * (j >> 2) + (j & 3) > ragged_last) st[QT][j] = -INFINITY;
-          pre(qt_tag, ragged_cnts, 0u);
+          pre(qt_tag, ragged_cnts, 0u, std::false_type{});
           static_for<8>([&](auto j_tag) { exps(qt_tag, j_tag); });
           exps_tail(qt_tag);
           static_for<4>([&](auto i_tag) { mma_pv(qt_tag, i_tag); });

@@ -72,3 +72,49 @@ def test_block16_split_walk_handles_scores_far_above_the_reference(gain):
     o = s3r.select_attn(q.to(DEV), kk.to(DEV), v.to(DEV), idx.to(DEV), 16)
     assert torch.isfinite(o.float()).all()
     assert max_abs(o, oracle.select_attention(q, kk, v, idx, 16, out_dtype=torch.float32)) <= 2e-2
+
+
+def _same_union_lists(n, h, k, seed, keep, last=False, duplicates=False):
+    """Two sets of lists with the same union (2k blocks) per group of four query blocks and the same lists for half ``keep``
+    of it.  Each half names 1.5k blocks in the first set; in the second the other half names the whole union, so that the
+    group keeps to the common walk.  No two blocks of a union share a slot of the kernel's table, so that the order of the
+    walk does not depend on which list names a block first."""
+    g = torch.Generator().manual_seed(seed)
+    nb, nqb = n // 16, -(-n // 16)
+    slot = [(e * 0x9E3779B1 % 2 ** 32) >> 23 for e in range(nb)]
+    lists = torch.full((2, 1, h, nqb, k), -1, dtype=torch.int32)
+    for head in range(h):
+        for grp in range(-(-nqb // 4)):
+            by_slot = {slot[e]: e for e in torch.randperm(nb, generator=g).tolist()}
+            union = torch.tensor(list(by_slot.values()), dtype=torch.int32)[:2 * k]
+            named = {keep: (union[:3 * k // 2],) * 2, 1 - keep: (union[k // 2:], union)}
+            for half, both in named.items():
+                for which, blocks in enumerate(both):
+                    blocks = blocks[torch.randperm(len(blocks), generator=torch.Generator().manual_seed(grp))]
+                    parts = blocks[:k], torch.cat((blocks[k:], blocks[:k // 4 if len(blocks) < 2 * k else 0]))
+                    for j, part in enumerate(parts):
+                        m = 4 * grp + 2 * half + j
+                        if m < nqb:
+                            lists[which, 0, head, m, :len(part)] = part
+                            if j == 1 and half == keep and last:
+                                lists[which, 0, head, m, -1] = nqb - 1
+                            if j == 1 and half == keep and duplicates:
+                                lists[which, 0, head, m, -2] = part[0]
+    return lists
+
+
+@pytest.mark.parametrize("dtype,size", [(torch.bfloat16, 1.0), (torch.float16, 1.0), (torch.float16, 3.5), (torch.bfloat16, 9.0)])
+@pytest.mark.parametrize("keep", [0, 1])
+@pytest.mark.parametrize("n,k,extra", [(4096, 32, {}), (4105, 32, {"last": True}), (2048, 16, {"duplicates": True}), (8192, 64, {})])
+def test_block16_result_does_not_depend_on_the_walk(dtype, size, keep, n, k, extra):
+    """A half's queries get the same bits from the walk per half and from the common walk over the same union: the same
+    order of additions, and each query's softmax reference from the same blocks.  ``size`` 3.5 and 9: row sums beyond the
+    bound, the groups start over with the running maximum."""
+    h = 2
+    lists = _same_union_lists(n, h, k, n + keep, keep, **extra)
+    g = torch.Generator().manual_seed(n + k)
+    q, kk, v = ((torch.randn((1, h, n, 64), generator=g) * s).to(dtype).to(DEV) for s in (size, size, 1.0))
+    (o, lse), (o_common, lse_common) = (s3r.select_attn(q, kk, v, idx.to(DEV), 16, return_lse=True) for idx in lists)
+    rows = (torch.arange(n) // 32 % 2 == keep) & (torch.arange(n) < n // 64 * 64)    # of whole groups
+    assert torch.equal(o[:, :, rows], o_common[:, :, rows])
+    assert torch.equal(lse[:, :, rows], lse_common[:, :, rows])
