@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256, 3) void prepass_bwd_kernel(PrepassParams p, Pr
       pos_lo = load_pos(p, b, t0 + (ta < nvalid ? ta : nvalid - 1), lane & 1);
       pos_hi = load_pos(p, b, t0 + (tb < nvalid ? tb : nvalid - 1), lane & 1);
       const int pc = block_position((ta < nvalid ? pos_lo : 0) + (tb < nvalid ? pos_hi : 0), (float)nvalid, rl.half);
-      tab = table_ptr<T>(p, staged, rl, pc, __any(pc >= p.staged_rows), rl.second);
+      tab = table_ptr<T>(p, staged, rl, pc, rl.second);
     }
     // what every token of the block gets through its mean (all row groups compute it, the first one counts)
     float mean_grad[3][VEC];
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256, 3) void prepass_bwd_kernel(PrepassParams p, Pr
         const int slot = 2 * rcl + rl.half;
         const int from_lo = __shfl(pos_lo, slot & 63), from_hi = __shfl(pos_hi, slot & 63);
         const int pp = slot < 64 ? from_lo : from_hi;
-        tab = table_ptr<T>(p, staged, rl, pp, __any(pp >= p.staged_rows), rl.second);
+        tab = table_ptr<T>(p, staged, rl, pp, rl.second);
       }
       u32x4 rx[2], rd[3];
       if constexpr (NORM) {

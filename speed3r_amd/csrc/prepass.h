@@ -115,24 +115,23 @@ template <typename T, int VEC> __device__ __forceinline__ void norm_row(const Pr
 }
 
 // Where the lane reads the VEC cosines and sines of its frequencies at position pp: the staged tables or, for positions
-// beyond them (far, wave-uniform: some lane has one), a slot of its own in LDS that is filled here.  Pointers instead of
-// values keep the rare case out of the registers of the common one (with both in registers the pass spills).
+// outside of them (negative ones too; rare), a slot of its own in LDS that is filled here.  Called by whole waves.  Pointers
+// instead of values keep the rare case out of the registers of the common one (with both in registers the pass spills).
 struct TablePtr {
   const float *c, *s;
 };
 template <typename T>
-__device__ __forceinline__ TablePtr table_ptr(const PrepassParams& p, float* staged, const RotLane<T>& rl, int pp, bool far, bool minus_sine) {
+__device__ __forceinline__ TablePtr table_ptr(const PrepassParams& p, float* staged, const RotLane<T>& rl, int pp, bool minus_sine) {
   constexpr int VEC = RotLane<T>::VEC;
-  pp = pp < 0 ? 0 : pp;
-  const int lp = pp < p.staged_rows ? pp : p.staged_rows - 1;
+  const bool outside = (uint32_t)pp >= (uint32_t)p.staged_rows;
   TablePtr t;
-  t.c = staged + lp * 16 + rl.f0;
+  t.c = staged + (outside ? 0 : pp) * 16 + rl.f0;
   t.s = t.c + (minus_sine ? 2 : 1) * p.staged_rows * 16;
-  if (far) {
-    if (pp >= p.staged_rows) {
+  if (__any(outside)) {
+    if (outside) {
       float* const slot = staged + (3 * p.staged_rows * 16 + 4 * 64) + threadIdx.x * (2 * VEC);
-      const int64_t row = (int64_t)(pp < p.P ? pp : p.P - 1) * 16 + rl.f0;
       if (pp < p.P || p.inv_freq == nullptr) {
+        const int64_t row = (int64_t)(pp < 0 ? 0 : pp < p.P ? pp : p.P - 1) * 16 + rl.f0;
         const uint4 c = *reinterpret_cast<const uint4*>((const T*)p.cos_tab + row), sv = *reinterpret_cast<const uint4*>((const T*)p.sin_tab + row);
 #pragma unroll
         for (int i = 0; i < VEC; i++) {

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256, 4) void qkv_prepass_kernel(PrepassParams p, in
       pp = slot < 64 ? from_lo : from_hi;
     }
     TablePtr tab = {};
-    if constexpr (ROT && ROWS) tab = table_ptr<T>(p, staged, rl, pp, __any(pp >= p.staged_rows), !rl.second);
+    if constexpr (ROT && ROWS) tab = table_ptr<T>(p, staged, rl, pp, !rl.second);
     if constexpr (POOL) {
 #pragma unroll
       for (int i = 0; i < VEC; i++) av[i] += keep ? to_f32(reinterpret_cast<const T*>(&lv)[i]) : 0.f;
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256, 4) void qkv_prepass_kernel(PrepassParams p, in
       if constexpr (NORM) norm_row<T>(p, staged, x, odd ? 2 : 0, lr);
       if constexpr (ROT) {
         const int pc = block_position(pos_sum, cnt, rl.half);
-        rotate_row<T>(x, table_ptr<T>(p, staged, rl, pc, __any(pc >= p.staged_rows), !rl.second));
+        rotate_row<T>(x, table_ptr<T>(p, staged, rl, pc, !rl.second));
       }
     }
     if (r0 < 2) put(odd ? p.kc : p.qc, x);

@@ -140,3 +140,32 @@ def test_training_after_inference_mode():
     assert torch.equal(layer(x, xpos=pos), layer(x, xpos=pos.clone()))
     # two runs of the same kernels: the bits may differ only where a reduction's order does (one rounding of the result)
     assert all(_close(g, w, torch.bfloat16, steps=1) for g, w in zip(got, want))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,block,low,high", [(33, 16, -9, 0), (64, 16, -3, 4), (200, 64, -70, 0), (130, 64, -5, 70), (130, 256, -4, 2)])
+@pytest.mark.parametrize("bound", [None, 3])
+def test_positions_below_zero_take_the_first_table_row(dtype, n, block, low, high, bound):
+    """Tokens' and block means' positions below zero, in one coordinate or both, are clamped like those beyond a bounded
+    table: the bits of the norm + RoPE kernel, in one launch and in two (which holds no tables in LDS)."""
+    b, h = 2, 3
+    g = torch.Generator().manual_seed(n - low)
+    qkv = (torch.randn((b, n, 3 * h * 64), generator=g) * 0.7).to(dtype).to(DEV)
+    pos = torch.randint(low, high, (b, n, 2), generator=g)
+    pos[0, :, 1] = pos[0, :, 1].abs()
+    pos = pos.to(DEV)
+    ln = [((1 + 0.3 * torch.randn(64, generator=g)).to(dtype).to(DEV), (0.2 * torch.randn(64, generator=g)).to(dtype).to(DEV)) for _ in range(2)]
+    rope = RoPE2D(100.0)
+    cos, sin, inv = rope.fused_tables(64, bound, qkv.device, dtype)
+    full = rope.tables(64, bound or 128, qkv.device, dtype)
+    q, k, v = qkv.view(b, n, 3, h, 64).permute(2, 0, 3, 1, 4).unbind(0)
+    raw, pc = ops.pool_qkv_packed(qkv, h, block), block_positions(pos, block)
+    want = (*(ops.norm_rope(t, pos, *full, *l, 1e-6) for t, l in zip((q, k), ln)), v,
+            *(ops.norm_rope(t, pc, *full, *l, 1e-6) for t, l in zip(raw, ln)), raw[2])
+    args = pos, cos, sin, *ln, 1e-6
+    one = ops.qkv_prepass(qkv, h, block, *args, pooled="final", inv_freq=inv)
+    two = (*ops.qkv_prepass(qkv, h, 64, *args, pooled=None, inv_freq=inv),
+           *ops.qkv_prepass(qkv, h, block, *args, tokens=False, pooled="final", inv_freq=inv))
+    for got in (one, two):
+        for i, (a, w) in enumerate(zip(got, want)):
+            assert torch.equal(a, w), i
