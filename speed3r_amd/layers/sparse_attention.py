@@ -27,6 +27,15 @@ from ..sparse_attn.flash_attention_topk import flash_attn_topk_func
 from .pos_embed import RoPE2D, block_positions
 
 
+def calls_forward_only(m: nn.Module, kind: type) -> bool:
+    """Whether calling ``m`` runs ``kind.forward`` and nothing else: exactly of that type, ``forward`` not replaced, not
+    compiled, no hooks of its own and no global ones.  A kernel may only then stand in for the call."""
+    g = nn.modules.module
+    return type(m) is kind and "forward" not in m.__dict__ and m._compiled_call_impl is None and not (
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or g._global_forward_hooks
+        or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks)
+
+
 def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
     """qk-norm, cast and RoPE of one ``[B,H,N,D]`` tensor (reference sparse_attention.py:103-110,120-124): one fused
     kernel where it is built -- a tensor on the GPU, head_dim 64, ``nn.Identity`` or an affine ``nn.LayerNorm`` of

@@ -36,7 +36,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from ..layers import RoPE2D, SparseFlashAttentionRope
-from ..layers.sparse_attention import fused_qk_args, norm_rope_fused_or_eager
+from ..layers.sparse_attention import calls_forward_only, fused_qk_args, norm_rope_fused_or_eager
 from ..sparse_attn import ops
 from .token_order import tile_major, tile_major_inverse
 
@@ -138,26 +138,32 @@ class Block(nn.Module):
     def forward(self, x: Tensor, xpos: Optional[Tensor] = None, n_pos: Optional[int] = None) -> Tensor:
         return self._run(x, token_norm(self.norm1, x), None, xpos, n_pos)[0]
 
-    def step(self, x: Tensor, normed: Tensor, next_norm: Optional[nn.LayerNorm], xpos: Optional[Tensor] = None,
-             n_pos: Optional[int] = None):
-        """The block on ``x`` with ``normed = norm1(x)`` at hand: its output and, for the module behind it, ``next_norm`` of
-        that output (each residual sum meets its norm in one pass).  A block with hooks is called as a module."""
-        if self._forward_hooks or self._forward_pre_hooks:
-            x = self(x, xpos=xpos, n_pos=n_pos)
-            return x, token_norm(next_norm, x) if next_norm is not None else None
-        return self._run(x, normed, next_norm, xpos, n_pos)
-
-    def _run(self, x, normed, next_norm, xpos, n_pos):
+    def _run(self, x, normed, next_norm, xpos=None, n_pos=None):
+        """The block on ``x`` with ``normed = norm1(x)`` at hand: its output and ``next_norm`` of that (None without)."""
         x, y = add_and_norm(x, self.ls1, self.attn(normed, xpos=xpos, n_pos=n_pos), self.norm2)
         return add_and_norm(x, self.ls2, self.mlp(y), next_norm)
 
 
+def takes_normed(blk: nn.Module) -> bool:
+    """Whether ``blk`` may be handed ``norm1`` of its input from the block before it: for inference, where calling the
+    module would run ``Block.forward`` and nothing else."""
+    return not torch.is_grad_enabled() and calls_forward_only(blk, Block)
+
+
+def run_block(blk: nn.Module, x: Tensor, normed: Optional[Tensor], next_norm: Optional[nn.LayerNorm], **kw):
+    """One block of a sequence: its output and, where it could be had in the pass over the residual sum, ``next_norm`` of
+    that output (else None).  ``normed``: ``norm1(x)`` if the block before it gave it."""
+    if takes_normed(blk):
+        return blk._run(x, token_norm(blk.norm1, x) if normed is None else normed, next_norm, **kw)
+    return blk(x, **kw), None
+
+
 def run_blocks(blocks, x: Tensor, last_norm: Optional[nn.LayerNorm], **kw):
     """``blocks`` in sequence: the last one's output and ``last_norm`` of it (None without)."""
-    y = token_norm(blocks[0].norm1, x) if len(blocks) else token_norm(last_norm, x) if last_norm is not None else None
-    for i, blk in enumerate(blocks):
-        x, y = blk.step(x, y, blocks[i + 1].norm1 if i + 1 < len(blocks) else last_norm, **kw)
-    return x, y
+    y = None
+    for blk, after in zip(blocks, [*list(blocks)[1:], None]):
+        x, y = run_block(blk, x, y, last_norm if after is None else after.norm1 if takes_normed(after) else None, **kw)
+    return x, token_norm(last_norm, x) if y is None and last_norm is not None else y
 
 
 class PatchEncoder(nn.Module):
@@ -295,15 +301,15 @@ class Pi3SparseLike(nn.Module):
         else:
             pos_dec = pos
         local_out = normed = None
-        for i, (local_blk, global_blk) in enumerate(zip(self.local_decoder, self.global_decoder)):
-            if normed is None:
-                normed = token_norm(local_blk.norm1, x)
-            x, normed = local_blk.step(x, normed, global_blk.norm1, xpos=pos_dec, n_pos=n_pos)
-            local_out = x
-            flat = (b, f * t, -1)                                                  # the global block sees one sequence
-            x, normed = global_blk.step(x.reshape(flat), normed.reshape(flat), self.local_decoder[i + 1].norm1
-                                        if i + 1 < len(self.local_decoder) else None, xpos=pos_dec.reshape(b, f * t, 2), n_pos=n_pos)
-            x, normed = x.reshape(b * f, t, -1), normed.reshape(b * f, t, -1) if normed is not None else None
+        blocks = [blk for pair in zip(self.local_decoder, self.global_decoder) for blk in pair]
+        for i, blk in enumerate(blocks):
+            # a global block sees the frames of a batch as one sequence
+            shape, p = ((b * f, t, -1), pos_dec) if i % 2 == 0 else ((b, f * t, -1), pos_dec.reshape(b, f * t, 2))
+            after = blocks[i + 1] if i + 1 < len(blocks) and takes_normed(blocks[i + 1]) else None
+            x, normed = run_block(blk, x.reshape(shape), normed.reshape(shape) if normed is not None else None,
+                                  after.norm1 if after is not None else None, xpos=p, n_pos=n_pos)
+            local_out = x if i % 2 == 0 else local_out
+        x = x.reshape(b * f, t, -1)
         feat = torch.cat((local_out, x), dim=-1)
         if tiled:                                                                  # the heads see row-major tokens again
             feat = tile_major_inverse(feat, gh, gw, self.tile)

@@ -7,6 +7,7 @@ import torch
 import oracle
 from speed3r_amd.layers import RoPE2D, SparseFlashAttentionRope
 from speed3r_amd.model import Pi3SparseLike
+from speed3r_amd.model.pi3_sparse_like import Block
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -226,3 +227,20 @@ def test_end_to_end_workload_in_the_reference_setting_100_frames_504x392():
     assert torch.allclose(rot @ rot.transpose(-1, -2), torch.eye(3, dtype=torch.float64, device=DEV).expand(frames, 3, 3), atol=1e-4)
     del m, out
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(token_order="tile", num_register=0, grid=(4, 8))])
+def test_blocks_called_as_modules_give_the_bits_of_the_chained_passes(kw):
+    """A hook on every block has the blocks called one by one; without, each residual sum and the next block's norm are
+    one pass."""
+    m = _randomised_small_model(seed=3, **kw).to(torch.bfloat16).to(DEV)
+    imgs = torch.rand((1, 5, 3, 14 * m.encoder.grid[0], 14 * m.encoder.grid[1]), device=DEV)
+    with torch.no_grad():
+        want = m(imgs, return_features=True)
+        calls = []
+        for module in m.modules():
+            if isinstance(module, Block):
+                module.register_forward_hook(lambda *a: calls.append(1))
+        got = m(imgs, return_features=True)
+    assert len(calls) == 2 + 4 + 3
+    assert all(torch.equal(got[k], want[k]) for k in want)
