@@ -25,14 +25,14 @@ class RoPE2D(nn.Module):
 
     DEFAULT_ROWS = 64   # table rows where no bound of the coordinates is given (the kernels hold so many in LDS)
 
-    def fused_tables(self, head_dim: int, n_pos, device, dtype):
+    def fused_tables(self, head_dim: int, n_pos, device, dtype, bounded: bool = True):
         """``(cos, sin, inv_freq)`` for the fused kernels: tables of ``n_pos`` (default: ``max_positions``) rows and no
         ``inv_freq`` (coordinates beyond them are clamped), or, without a bound, default tables and the frequencies that
-        give every further coordinate its own angle; no look at the positions, no device synchronisation."""
-        rows = n_pos or self.max_positions
-        if rows:
-            return *self.tables(head_dim, rows, device, dtype), None
-        return *self.tables(head_dim, self.DEFAULT_ROWS, device, dtype), self.inv_freq(head_dim, device)
+        give every further coordinate its own angle; no look at the positions, no device synchronisation.
+        ``bounded=False``: the frequencies beside tables of ``n_pos`` rows too, like the module's own angles."""
+        rows = n_pos or (self.max_positions if bounded else 0)
+        inv_freq = None if bounded and rows else self.inv_freq(head_dim, device)
+        return *self.tables(head_dim, rows or self.DEFAULT_ROWS, device, dtype), inv_freq
 
     def tables(self, head_dim: int, n_pos: int, device, dtype):
         """cos, sin ``[n_pos, head_dim // 4]`` in ``dtype``: row p holds cos/sin of the angles ``p * inv_freq`` after

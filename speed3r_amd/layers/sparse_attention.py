@@ -61,9 +61,10 @@ def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Ten
     return rope(t, pos) if pos is not None else t
 
 
-def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Optional[int] = None):
+def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Optional[int] = None, training: bool = False):
     """``(pos, cos, sin, inv_freq, q_ln, k_ln, eps)`` for the kernels that take qk-norm and RoPE with the packed
-    projection, or None where their conditions do not hold (those of ``norm_rope_fused_or_eager`` for both norms)."""
+    projection, or None where their conditions do not hold (those of ``norm_rope_fused_or_eager`` for both norms).
+    ``training``: in the place of the modules' own calls, which know no bound of the positions."""
     def plain(norm):
         return isinstance(norm, nn.Identity) or (type(norm) is nn.LayerNorm and norm.elementwise_affine)
     same_kind = isinstance(attn.q_norm, nn.Identity) == isinstance(attn.k_norm, nn.Identity)
@@ -75,7 +76,7 @@ def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Op
         return None
     cos = sin = inv_freq = None
     if pos is not None:
-        cos, sin, inv_freq = attn.rope.fused_tables(64, n_pos, qkv.device, qkv.dtype)
+        cos, sin, inv_freq = attn.rope.fused_tables(64, n_pos, qkv.device, qkv.dtype, bounded=not training)
     return (pos, cos, sin, inv_freq, (attn.q_norm.weight, attn.q_norm.bias) if ln else None,
             (attn.k_norm.weight, attn.k_norm.bias) if ln else None, attn.q_norm.eps if ln else 0.0)
 
@@ -138,7 +139,7 @@ class SparseFlashAttentionRope(nn.Module):
                 return out
         return self.gate(x)
 
-    def _forward_with_grad(self, x: Tensor, xpos: Optional[Tensor]) -> Tensor:
+    def _forward_with_grad(self, x: Tensor, xpos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
         """The same layer for training.  Between its projections it is one differentiable operator whose forward and
         backward are kernels (``ops.layer_core_autograd``).  Where that is not built (another norm or rope module, blocks of
         128 or 256 tokens): a composition in which the two attention operators carry their own backward kernels and pooling,
@@ -152,7 +153,7 @@ class SparseFlashAttentionRope(nn.Module):
         qkv = self.qkv(x)
         gate = self.gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)              # [B, H, N, 2]
         use_pos = xpos is not None and self.rope is not None
-        fused = fused_qk_args(self, qkv, xpos if use_pos else None)
+        fused = fused_qk_args(self, qkv, xpos if use_pos else None, n_pos, training=True)
         if fused is not None and self.topk in (1, 2, 4, 8, 16, 32, 64):
             pos, cos, sin, inv_freq, q_ln, k_ln, eps = fused
             core = ops.layer_core_autograd(qkv, gate, h, block, self.topk, pos, cos, sin, inv_freq, q_ln, k_ln, eps)
@@ -193,10 +194,11 @@ class SparseFlashAttentionRope(nn.Module):
     def forward(self, x: Tensor, attn_bias=None, xpos: Optional[Tensor] = None, n_pos: Optional[int] = None) -> Tensor:
         """``n_pos`` (optional, beyond the reference's signature): an upper bound, exclusive, of the coordinates in
         ``xpos`` for this call; sizes the fused kernels' cos/sin tables without a device synchronisation and without
-        touching state shared between calls."""
+        touching state shared between calls.  Larger coordinates are clamped to it for inference; a training call gives
+        them their own angles."""
         if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters())):
             self.last_path = "autograd"
-            return self._forward_with_grad(x, xpos)
+            return self._forward_with_grad(x, xpos, n_pos)
         b, n, c = x.shape
         h = self.num_heads
         d = c // h

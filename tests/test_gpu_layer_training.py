@@ -1,0 +1,67 @@
+"""The layer's training route against the same layer composed of torch modules (needs an MI355X)."""
+import pytest
+import torch
+from torch import nn
+
+from speed3r_amd.layers import RoPE2D, SparseFlashAttentionRope
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+DIM, HEADS = 128, 2
+
+
+class TorchRope(nn.Module):
+    """RoPE2D as a module of another type: the layer composes torch expressions around it."""
+
+    def __init__(self, rope):
+        super().__init__()
+        self.rope = rope
+
+    def forward(self, tokens, positions):
+        return self.rope(tokens, positions)
+
+
+def _layer(rope, block_size=8, seed=0, dtype=torch.bfloat16, topk=4):
+    torch.manual_seed(seed)
+    m = SparseFlashAttentionRope(DIM, num_heads=HEADS, qkv_bias=True, qk_norm=True, rope=rope, block_size=block_size, topk=topk)
+    with torch.no_grad():
+        m.gate[0].weight.normal_(0, 0.05)
+        for norm in (m.q_norm, m.k_norm):
+            norm.weight.uniform_(0.5, 1.5)
+            norm.bias.normal_(0, 0.1)
+    return m.to(DEV, dtype)
+
+
+def _step(m, x, pos, dout, **kw):
+    """{name: tensor} of the output, the input's gradient and every parameter's."""
+    x = x.detach().requires_grad_()
+    out = m(x, xpos=pos, **kw)
+    names, params = zip(*m.named_parameters())
+    grads = torch.autograd.grad(out, (x, *params), dout, allow_unused=True)
+    return {"out": out.detach(), "x": grads[0], **dict(zip(names, grads[1:]))}
+
+
+def _inputs(n, b=1, high=40, seed=1, low=0, dtype=torch.bfloat16):
+    g = torch.Generator().manual_seed(seed)
+    x, dout = (torch.randn((b, n, DIM), generator=g).to(DEV, dtype) for _ in range(2))
+    return x, torch.randint(low, high, (b, n, 2), generator=g).to(DEV), dout
+
+
+def _same(got, want):
+    """Two 16-bit evaluations of the same sums: a chain of at most a dozen roundings to 2^-9, some of them of terms that
+    cancel to a fifth: 5e-2 of the tensor's norm.  Positions that are off by one change it by more than a third."""
+    assert got.keys() == want.keys()
+    for k in want:
+        assert got[k].dtype == want[k].dtype and got[k].shape == want[k].shape, k
+        assert torch.isfinite(got[k]).all(), k
+        diff, size = (got[k].double() - want[k].double()).norm(), want[k].double().norm()
+        assert diff <= 5e-2 * size, (k, float(diff / size))
+
+
+@pytest.mark.parametrize("block_size,n", [(8, 256), (8, 200), (4, 60)])
+@pytest.mark.parametrize("n_pos", [None, 41, 8])
+def test_training_rotates_by_every_position_whatever_the_tables(block_size, n, n_pos):
+    """Positions beyond a rope module's ``max_positions`` and beyond a call's ``n_pos`` keep their own angles in training."""
+    x, pos, dout = _inputs(n, high=41)
+    got = _step(_layer(RoPE2D(100.0, max_positions=8), block_size), x, pos, dout, n_pos=n_pos)
+    _same(got, _step(_layer(TorchRope(RoPE2D(100.0)), block_size), x, pos, dout))
