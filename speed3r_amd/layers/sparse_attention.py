@@ -64,12 +64,14 @@ def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Ten
 def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Optional[int] = None, training: bool = False):
     """``(pos, cos, sin, inv_freq, q_ln, k_ln, eps)`` for the kernels that take qk-norm and RoPE with the packed
     projection, or None where their conditions do not hold (those of ``norm_rope_fused_or_eager`` for both norms).
-    ``training``: in the place of the modules' own calls, which know no bound of the positions."""
+    ``training``: in the place of the modules' own calls, which know no bound of the positions and must do nothing else."""
     def plain(norm):
+        if training and not (calls_forward_only(norm, nn.Identity) or calls_forward_only(norm, nn.LayerNorm)):
+            return False
         return isinstance(norm, nn.Identity) or (type(norm) is nn.LayerNorm and norm.elementwise_affine)
     same_kind = isinstance(attn.q_norm, nn.Identity) == isinstance(attn.k_norm, nn.Identity)
     if not (qkv.is_cuda and qkv.shape[-1] == 192 * attn.num_heads and plain(attn.q_norm) and plain(attn.k_norm) and same_kind
-            and (pos is None or isinstance(attn.rope, RoPE2D))):
+            and (pos is None or (calls_forward_only(attn.rope, RoPE2D) if training else isinstance(attn.rope, RoPE2D)))):
         return None
     ln = isinstance(attn.q_norm, nn.LayerNorm)
     if ln and attn.q_norm.eps != attn.k_norm.eps:

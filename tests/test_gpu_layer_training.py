@@ -65,3 +65,52 @@ def test_training_rotates_by_every_position_whatever_the_tables(block_size, n, n
     x, pos, dout = _inputs(n, high=41)
     got = _step(_layer(RoPE2D(100.0, max_positions=8), block_size), x, pos, dout, n_pos=n_pos)
     _same(got, _step(_layer(TorchRope(RoPE2D(100.0)), block_size), x, pos, dout))
+
+
+class _ScaledRope(RoPE2D):
+    def forward(self, tokens, positions):
+        return super().forward(tokens, 2 * positions)
+
+
+@pytest.mark.parametrize("what", ["q_norm hook", "k_norm pre-hook", "backward hook", "rope hook", "global hook", "rope subclass", "replaced forward"])
+def test_training_calls_norms_and_rope_that_do_more_than_their_forward(what):
+    """Hooks fire once for the tokens and once for the block means, and what they return counts."""
+    x, pos, dout = _inputs(200)
+    calls = []
+
+    def scaled(mod, args, out):
+        calls.append(1)
+        return 0.5 * out
+
+    def change(m):
+        if what == "q_norm hook":
+            return [m.q_norm.register_forward_hook(scaled)]
+        if what == "k_norm pre-hook":
+            return [m.k_norm.register_forward_pre_hook(lambda mod, args: (calls.append(1), (args[0] + 0.5,))[1])]
+        if what == "backward hook":
+            return [m.q_norm.register_full_backward_hook(lambda *a: calls.append(1))]
+        if what == "rope hook":
+            return [m.rope.register_forward_hook(scaled)]
+        if what == "global hook":
+            return [nn.modules.module.register_module_forward_hook(
+                lambda mod, args, out: scaled(mod, args, out) if isinstance(mod, nn.LayerNorm) else None)]
+        if what == "rope subclass":
+            m.rope = TorchRope(_ScaledRope(100.0)) if isinstance(m.rope, TorchRope) else _ScaledRope(100.0)
+        else:
+            m.q_norm.forward = lambda t: nn.functional.layer_norm(t, (64,))
+        return []
+
+    results = []
+    for rope in (RoPE2D(100.0), TorchRope(RoPE2D(100.0))):
+        m = _layer(rope)
+        calls.clear()
+        handles = change(m)
+        try:
+            results.append((_step(m, x, pos, dout), len(calls)))
+        finally:
+            for handle in handles:
+                handle.remove()
+    (got, fired), (want, expected) = results
+    assert fired == expected
+    want, got = ({k: v for k, v in d.items() if v is not None} for d in (want, got))
+    _same(got, want)
