@@ -114,3 +114,10 @@ def test_training_calls_norms_and_rope_that_do_more_than_their_forward(what):
     assert fired == expected
     want, got = ({k: v for k, v in d.items() if v is not None} for d in (want, got))
     _same(got, want)
+
+
+@pytest.mark.parametrize("shape", [(1, 200, 2), (3, 200, 2), (3, 1, 2), (1, 1, 2)])
+def test_training_broadcasts_positions_over_the_batch(shape):
+    x, _, dout = _inputs(200, b=3)
+    pos = torch.randint(0, 40, shape, generator=torch.Generator().manual_seed(2)).to(DEV)
+    _same(_step(_layer(RoPE2D(100.0)), x, pos, dout), _step(_layer(TorchRope(RoPE2D(100.0))), x, pos, dout))
