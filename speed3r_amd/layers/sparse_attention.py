@@ -73,8 +73,8 @@ def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Op
     if not (qkv.is_cuda and qkv.shape[-1] == 192 * attn.num_heads and plain(attn.q_norm) and plain(attn.k_norm) and same_kind
             and (pos is None or (calls_forward_only(attn.rope, RoPE2D) if training else isinstance(attn.rope, RoPE2D)))):
         return None
-    if training and pos is not None:   # (a rope module takes one set of positions for all sequences, and more)
-        if pos.shape not in (qkv.shape[:2] + (2,), (1, qkv.shape[1], 2)):
+    if training and pos is not None:   # (a rope module takes one set of positions for all sequences, fractional ones, and more)
+        if pos.is_floating_point() or pos.shape not in (qkv.shape[:2] + (2,), (1, qkv.shape[1], 2)):
             return None
         pos = pos.expand(*qkv.shape[:2], 2)
     ln = isinstance(attn.q_norm, nn.LayerNorm)

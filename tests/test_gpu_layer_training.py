@@ -121,3 +121,12 @@ def test_training_broadcasts_positions_over_the_batch(shape):
     x, _, dout = _inputs(200, b=3)
     pos = torch.randint(0, 40, shape, generator=torch.Generator().manual_seed(2)).to(DEV)
     _same(_step(_layer(RoPE2D(100.0)), x, pos, dout), _step(_layer(TorchRope(RoPE2D(100.0))), x, pos, dout))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int32, torch.int16, torch.uint8])
+@pytest.mark.parametrize("block_size", [8, 4])
+def test_training_with_positions_of_any_type(dtype, block_size):
+    """Fractional positions have their own angles (block means take the truncated mean, like the others)."""
+    x, pos, dout = _inputs(200, high=30)
+    pos = (pos.float() + 0.5).to(dtype) if dtype.is_floating_point else pos.to(dtype)
+    _same(_step(_layer(RoPE2D(100.0), block_size, topk=16), x, pos, dout), _step(_layer(TorchRope(RoPE2D(100.0)), block_size, topk=16), x, pos, dout))
