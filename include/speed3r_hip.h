@@ -239,7 +239,8 @@ int s3r_qkv_prepass(const void* q, const void* k, const void* v, void* q_out, vo
  *     tokens, pi3/models/layers/sparse_attention.py:97-110); q_raw, k_raw (optional): their values before that.
  *   positions: (y,x) pairs, int32 or int64 (positions_int64), strides in elements, or NULL.
  *   cos_table, sin_table: [table_rows,16] in the I/O dtype as in s3r_norm_rope.  inv_freq (optional, [16] fp32): positions
- *     at or beyond table_rows get cosine and sine of round(position * inv_freq); without it they are clamped.
+ *     at or beyond table_rows get cosine and sine of round(position * inv_freq); without it they are clamped.  Positions below
+ *     zero are clamped too, or, with inv_freq and signed_positions, get their own angles like those.
  *   norm parameters in the I/O dtype, or fp32 with norm_fp32 (used unrounded).
  */
 typedef struct s3r_prepass_args {
@@ -252,7 +253,7 @@ typedef struct s3r_prepass_args {
   const float* inv_freq;
   const void *q_norm_weight, *q_norm_bias, *k_norm_weight, *k_norm_bias;
   int64_t N, stride_b, stride_h, stride_n, pos_stride_b, pos_stride_n;
-  int B, H, head_dim, block, table_rows, positions_int64, norm_fp32, finish_pooled, dtype;
+  int B, H, head_dim, block, table_rows, positions_int64, norm_fp32, finish_pooled, signed_positions, dtype;
   float eps;
 } s3r_prepass_args;
 

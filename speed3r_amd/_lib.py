@@ -66,7 +66,7 @@ class PrepassArgs(ctypes.Structure):
                                          "k_norm_bias")]
                 + [(n, c_int64) for n in ("N", "stride_b", "stride_h", "stride_n", "pos_stride_b", "pos_stride_n")]
                 + [(n, c_int) for n in ("B", "H", "head_dim", "block", "table_rows", "positions_int64", "norm_fp32", "finish_pooled",
-                                        "dtype")]
+                                        "signed_positions", "dtype")]
                 + [("eps", c_float)])
 
 

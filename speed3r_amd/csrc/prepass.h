@@ -2,6 +2,7 @@
 // and LayerNorm parameters staged in LDS, the row transforms.
 #pragma once
 #include "s3r_common.h"
+#include <climits>
 #include <type_traits>
 
 namespace s3r {
@@ -17,6 +18,7 @@ struct PrepassParams {
   const void *qn_w, *qn_b, *kn_w, *kn_b;  // LayerNorm(64) parameters (nullptr weights: no norm) in T, or fp32 (ln_f32)
   float eps;
   int pos64, ln_f32, finish;    // finish: qc, kc after norm and rotation
+  int lowest;                   // positions below are taken as this: 0, or the lowest there is (own angles below zero too)
   int P, staged_rows;           // rows of the tables; the first staged_rows of them are held in LDS
   int B, H, block;
   int64_t N, sxb, sxh, sxn, spb, spn;
@@ -35,7 +37,7 @@ inline PrepassParams prepass_params(const s3r_prepass_args& a) {
   p.q_raw = a.q_raw; p.k_raw = a.k_raw; p.pos = a.positions; p.pos64 = a.positions_int64;
   p.cos_tab = a.cos_table; p.sin_tab = a.sin_table; p.inv_freq = a.inv_freq; p.P = a.table_rows;
   p.qn_w = a.q_norm_weight; p.qn_b = a.q_norm_bias; p.kn_w = a.k_norm_weight; p.kn_b = a.k_norm_bias; p.ln_f32 = a.norm_fp32; p.eps = a.eps;
-  p.finish = a.finish_pooled; p.B = a.B; p.H = a.H; p.N = a.N; p.block = a.block;
+  p.finish = a.finish_pooled; p.lowest = a.inv_freq != nullptr && a.signed_positions ? INT_MIN : 0; p.B = a.B; p.H = a.H; p.N = a.N; p.block = a.block;
   p.sxb = a.stride_b; p.sxh = a.stride_h; p.sxn = a.stride_n; p.spb = a.pos_stride_b; p.spn = a.pos_stride_n;
   return p;
 }
@@ -115,7 +117,7 @@ template <typename T, int VEC> __device__ __forceinline__ void norm_row(const Pr
 }
 
 // Where the lane reads the VEC cosines and sines of its frequencies at position pp: the staged tables or, for positions
-// outside of them (negative ones too; rare), a slot of its own in LDS that is filled here.  Called by whole waves.  Pointers
+// outside of them (rare; below zero too unless they are clamped to it), a slot of its own in LDS that is filled here.  Called by whole waves.  Pointers
 // instead of values keep the rare case out of the registers of the common one (with both in registers the pass spills).
 struct TablePtr {
   const float *c, *s;
@@ -123,6 +125,7 @@ struct TablePtr {
 template <typename T>
 __device__ __forceinline__ TablePtr table_ptr(const PrepassParams& p, float* staged, const RotLane<T>& rl, int pp, bool minus_sine) {
   constexpr int VEC = RotLane<T>::VEC;
+  pp = pp < p.lowest ? p.lowest : pp;
   const bool outside = (uint32_t)pp >= (uint32_t)p.staged_rows;
   TablePtr t;
   t.c = staged + (outside ? 0 : pp) * 16 + rl.f0;
@@ -130,8 +133,8 @@ __device__ __forceinline__ TablePtr table_ptr(const PrepassParams& p, float* sta
   if (__any(outside)) {
     if (outside) {
       float* const slot = staged + (3 * p.staged_rows * 16 + 4 * 64) + threadIdx.x * (2 * VEC);
-      if (pp < p.P || p.inv_freq == nullptr) {
-        const int64_t row = (int64_t)(pp < 0 ? 0 : pp < p.P ? pp : p.P - 1) * 16 + rl.f0;
+      if ((uint32_t)pp < (uint32_t)p.P || p.inv_freq == nullptr) {
+        const int64_t row = (int64_t)(pp < p.P ? pp : p.P - 1) * 16 + rl.f0;
         const uint4 c = *reinterpret_cast<const uint4*>((const T*)p.cos_tab + row), sv = *reinterpret_cast<const uint4*>((const T*)p.sin_tab + row);
 #pragma unroll
         for (int i = 0; i < VEC; i++) {

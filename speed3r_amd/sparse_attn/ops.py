@@ -345,7 +345,7 @@ def norm_rope(x: torch.Tensor, positions: Optional[torch.Tensor], cos_tab: Optio
     return y
 
 
-def _prepass_args(qkv: torch.Tensor, h: int, block: int, positions, cos_tab, sin_tab, q_ln, k_ln, eps: float, inv_freq=None):
+def _prepass_args(qkv: torch.Tensor, h: int, block: int, positions, cos_tab, sin_tab, q_ln, k_ln, eps: float, inv_freq=None, signed=False):
     """Argument block of the passes over the packed projection, with its inputs filled in, and the tensors it points to."""
     b, n, c3 = qkv.shape
     es = qkv.element_size()
@@ -365,7 +365,7 @@ def _prepass_args(qkv: torch.Tensor, h: int, block: int, positions, cos_tab, sin
         a.pos_stride_b, a.pos_stride_n = positions.stride(0), positions.stride(1)
         a.cos_table, a.sin_table, a.table_rows = cos_tab.data_ptr(), sin_tab.data_ptr(), cos_tab.shape[0]
         if inv_freq is not None:
-            a.inv_freq = inv_freq.data_ptr()
+            a.inv_freq, a.signed_positions = inv_freq.data_ptr(), signed
     if q_ln is not None:
         params = [*q_ln, *k_ln]
         # fp32 parameters of 16-bit tokens (autocast) are used as they are, any others in the tokens' dtype
@@ -382,7 +382,8 @@ def qkv_prepass(qkv: torch.Tensor, num_heads: int, block: int, positions: Option
                 cos_tab: Optional[torch.Tensor], sin_tab: Optional[torch.Tensor],
                 q_ln: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None,
                 k_ln: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None, eps: float = 1e-5, *,
-                tokens: bool = True, pooled: Optional[str] = "raw", keep_raw: bool = False, inv_freq: Optional[torch.Tensor] = None):
+                tokens: bool = True, pooled: Optional[str] = "raw", keep_raw: bool = False, inv_freq: Optional[torch.Tensor] = None,
+                signed: bool = False):
     """The layer's pre-pass over the packed projection ``[B, N, 3*H*64]`` (layout ``(qkv h d)``) in one kernel:
     returns ``(q, k, v, q_c, k_c, v_c)`` -- q, k ``[B,H,N,64]`` contiguous after LayerNorm (``q_ln``/``k_ln`` = (weight,
     bias) or None) and RoPE2D at ``positions`` (None: no rotation), v the strided view of the projection, and the
@@ -392,7 +393,8 @@ def qkv_prepass(qkv: torch.Tensor, num_heads: int, block: int, positions: Option
     ``pooled="final"``: q_c and k_c are normalised and rotated too, at the truncated mean position of their block
     (:func:`norm_rope` at ``block_positions``); ``keep_raw`` then appends their raw values to the result.
     ``pooled=None``: q, k, v only; ``tokens=False``: the block means only.  ``inv_freq`` ([16] fp32): positions beyond the
-    tables are rotated by their own angles instead of being clamped to the last row."""
+    tables are rotated by their own angles instead of being clamped to the last row, with ``signed`` those below zero too
+    (else: row 0)."""
     _need_device(qkv)
     _forward_only(qkv)
     b, n, c3 = qkv.shape
@@ -401,7 +403,7 @@ def qkv_prepass(qkv: torch.Tensor, num_heads: int, block: int, positions: Option
         return None
     assert (q_ln is None) == (k_ln is None), "q and k are normalised together or not at all"
     assert pooled in ("raw", "final", None) and (tokens or pooled)
-    a, keep = _prepass_args(qkv, h, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq)
+    a, keep = _prepass_args(qkv, h, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq, signed)
     out = ()
     if tokens:
         q_out, k_out = qkv.new_empty((2, b, h, n, 64)).unbind(0)
@@ -700,11 +702,11 @@ PREPASS_BWD_ROWS = 768   # workgroups of the projection's backward pass that hol
 
 
 def qkv_prepass_bwd(qkv: torch.Tensor, num_heads: int, block: int, positions, cos_tab, sin_tab, q_ln, k_ln, eps: float, raw, grads,
-                    inv_freq=None):
+                    inv_freq=None, signed: bool = False):
     """Gradient of :func:`qkv_prepass` with ``pooled="final"``: ``raw`` = the raw (q_c, k_c), ``grads`` = the gradients of
     (q, k, v, q_c, k_c, v_c).  Returns ``(d_qkv, d_norm)``, d_norm ``[4,64]`` fp32 (q weight, q bias, k weight, k bias) or
     None without a norm."""
-    a, keep = _prepass_args(qkv, num_heads, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq)
+    a, keep = _prepass_args(qkv, num_heads, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq, signed)
     a.q_raw, a.k_raw = (t.data_ptr() for t in raw)
     grads = [t.contiguous() for t in grads]
     d_qkv = torch.empty_strided(qkv.shape, qkv.stride(), dtype=qkv.dtype, device=qkv.device)
@@ -731,7 +733,7 @@ class _LayerCoreFn(torch.autograd.Function):
         q_ln, k_ln = ((q_w, q_b), (k_w, k_b)) if q_w is not None else (None, None)
         with torch.no_grad():
             q, k, v, q_c, k_c, v_c, q_raw, k_raw = qkv_prepass(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, pooled="final",
-                                                               keep_raw=True, inv_freq=inv_freq)
+                                                               keep_raw=True, inv_freq=inv_freq, signed=True)
             o_c, idx, lse_c = compressed_attn_topk(q_c, k_c, v_c, topk, return_lse=True)
             o_s, lse = select_attn(q, k, v, idx, block, return_lse=True)
             out = gated_merge(o_c, o_s, gate, block)
@@ -751,7 +753,7 @@ class _LayerCoreFn(torch.autograd.Function):
         pooled = attn_bwd(q_c, k_c, v_c, o_c, d_oc, lse_c, delta=delta_c)
         full = attn_bwd(q, k, v, o_s, d_os, lse, idx, block, delta=delta_s)
         q_ln, k_ln = ((q_w, q_b), (k_w, k_b)) if q_w is not None else (None, None)
-        d_qkv, d_norm = qkv_prepass_bwd(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, (q_raw, k_raw), (*full, *pooled), inv_freq)
+        d_qkv, d_norm = qkv_prepass_bwd(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, (q_raw, k_raw), (*full, *pooled), inv_freq, signed=True)
         params = [d_norm[i].to(t.dtype) if t is not None else None for i, t in enumerate((q_w, q_b, k_w, k_b))]
         return d_qkv, d_gate, *params, *([None] * 8)
 

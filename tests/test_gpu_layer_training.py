@@ -130,3 +130,9 @@ def test_training_with_positions_of_any_type(dtype, block_size):
     x, pos, dout = _inputs(200, high=30)
     pos = (pos.float() + 0.5).to(dtype) if dtype.is_floating_point else pos.to(dtype)
     _same(_step(_layer(RoPE2D(100.0), block_size, topk=16), x, pos, dout), _step(_layer(TorchRope(RoPE2D(100.0)), block_size, topk=16), x, pos, dout))
+
+
+@pytest.mark.parametrize("block_size,low,high", [(8, -20, 20), (4, -90, -60), (8, -1, 1), (4, -3, 90)])
+def test_training_with_positions_below_zero(block_size, low, high):
+    x, pos, dout = _inputs(200, low=low, high=high)
+    _same(_step(_layer(RoPE2D(100.0), block_size, topk=16), x, pos, dout), _step(_layer(TorchRope(RoPE2D(100.0)), block_size, topk=16), x, pos, dout))
