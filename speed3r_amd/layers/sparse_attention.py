@@ -133,13 +133,10 @@ class SparseFlashAttentionRope(nn.Module):
         return norm_rope_fused_or_eager(t, norm, self.rope, pos, n_pos)
 
     def _gate(self, x: Tensor) -> Tensor:
-        """``self.gate(x)`` for inference: one kernel where it is the plain pair of modules it was built as (their calls
-        carry nothing else: no hooks, no autocast, no replaced module)."""
-        def plain(m, kind):
-            return type(m) is kind and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
-        if x.is_cuda and plain(self.gate, nn.Sequential) and len(self.gate) == 2 and plain(self.gate[0], nn.Linear) \
-                and plain(self.gate[1], nn.Sigmoid) and not torch.is_autocast_enabled("cuda") and "forward" not in self.gate[0].__dict__ \
-                and not (nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks):
+        """``self.gate(x)`` for inference: one kernel where it is the plain pair of modules it was built as, whose calls run
+        nothing but their ``forward``, and outside of autocast."""
+        if x.is_cuda and calls_forward_only(self.gate, nn.Sequential) and len(self.gate) == 2 and calls_forward_only(self.gate[0], nn.Linear) \
+                and calls_forward_only(self.gate[1], nn.Sigmoid) and not torch.is_autocast_enabled("cuda"):
             out = ops.gate(x, self.gate[0].weight, self.gate[0].bias)
             if out is not None:
                 return out

@@ -263,3 +263,47 @@ def test_operators_give_the_same_bits_on_one_stream_and_on_two(n, block, topk):
     gate = torch.rand((1, 16, n, 2), generator=g).to(torch.bfloat16).cuda()
     got = [s3r.sparse_global_attention(q, k, v, gate, block, topk, overlap=o) for o in (None, True, False)]
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+def _layer_and_input(block_size, rope, n=200, seed=0, dim=256):
+    torch.manual_seed(seed)
+    m = SparseFlashAttentionRope(dim=dim, num_heads=dim // 64, qkv_bias=True, qk_norm=True, rope=rope, block_size=block_size, topk=2)
+    with torch.no_grad():
+        m.gate[0].weight.normal_(0, 0.1)
+    return m.to(torch.bfloat16).to(DEV).eval(), torch.randn(1, n, dim, device=DEV).to(torch.bfloat16)
+
+
+class _Calls(torch.nn.Module):
+    """Calls the module it is given: a type of its own around the same call."""
+
+    def __init__(self, module):
+        super().__init__()
+        self.module = module
+
+    def forward(self, *args):
+        return self.module(*args)
+
+
+@pytest.mark.parametrize("what", ["sigmoid", "sequential", "linear", "compiled", "global backward hook"])
+def test_gate_modules_that_do_more_than_their_forward_are_called(what):
+    m, x = _layer_and_input(8, None)
+    gate, handles, calls = m.gate, [], []
+    if what == "sigmoid":
+        gate[1].forward = lambda t: 0.5 * torch.sigmoid(t)
+    elif what == "sequential":
+        gate.forward = lambda t: torch.tanh(gate[0](t))
+    elif what == "linear":
+        gate[0].forward = lambda t: torch.nn.functional.linear(t, 2 * gate[0].weight, gate[0].bias)
+    elif what == "compiled":
+        gate[0]._compiled_call_impl = lambda t: calls.append(1) or torch.nn.functional.linear(t, -gate[0].weight, gate[0].bias)
+    else:
+        handles = [torch.nn.modules.module.register_module_full_backward_pre_hook(lambda *a: None)]
+    try:
+        with torch.no_grad():
+            got = m(x)
+            fired = len(calls)
+            m.gate = _Calls(gate)
+            assert torch.equal(got, m(x)) and fired * 2 == len(calls) and bool(fired) == (what == "compiled")
+    finally:
+        for handle in handles:
+            handle.remove()
