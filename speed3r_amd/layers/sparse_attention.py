@@ -70,7 +70,7 @@ def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Op
             return False
         return isinstance(norm, nn.Identity) or (type(norm) is nn.LayerNorm and norm.elementwise_affine)
     same_kind = isinstance(attn.q_norm, nn.Identity) == isinstance(attn.k_norm, nn.Identity)
-    if not (qkv.is_cuda and qkv.shape[-1] == 192 * attn.num_heads and plain(attn.q_norm) and plain(attn.k_norm) and same_kind
+    if not (qkv.is_cuda and ops.prepass_takes(qkv, attn.num_heads) and plain(attn.q_norm) and plain(attn.k_norm) and same_kind
             and (pos is None or (calls_forward_only(attn.rope, RoPE2D) if training else isinstance(attn.rope, RoPE2D)))):
         return None
     if training and pos is not None:   # (a rope module takes one set of positions for all sequences, fractional ones, and more)

@@ -345,9 +345,14 @@ def norm_rope(x: torch.Tensor, positions: Optional[torch.Tensor], cos_tab: Optio
     return y
 
 
+def prepass_takes(qkv: torch.Tensor, num_heads: int) -> bool:
+    """Whether the passes over the packed projection are built for it: heads of 64, rows of adjacent values that do not overlap."""
+    return qkv.shape[-1] == 192 * num_heads and qkv.stride(-1) == 1 and qkv.stride(1) >= qkv.shape[-1]
+
+
 def _prepass_args(qkv: torch.Tensor, h: int, block: int, positions, cos_tab, sin_tab, q_ln, k_ln, eps: float, inv_freq=None, signed=False):
     """Argument block of the passes over the packed projection, with its inputs filled in, and the tensors it points to."""
-    b, n, c3 = qkv.shape
+    b, n = qkv.shape[:2]
     es = qkv.element_size()
     base = qkv.data_ptr()
     a = _lib.PrepassArgs(q=base, k=base + h * 64 * es, v=base + 2 * h * 64 * es, N=n, stride_b=qkv.stride(0), stride_h=64,
@@ -388,7 +393,7 @@ def qkv_prepass(qkv: torch.Tensor, num_heads: int, block: int, positions: Option
     returns ``(q, k, v, q_c, k_c, v_c)`` -- q, k ``[B,H,N,64]`` contiguous after LayerNorm (``q_ln``/``k_ln`` = (weight,
     bias) or None) and RoPE2D at ``positions`` (None: no rotation), v the strided view of the projection, and the
     block means of the RAW q, k, v ``[B,H,ceil(N/block),64]``.  Same bits as :func:`pool_qkv_packed` followed by
-    :func:`norm_rope` on q and k.  Returns None when the library has no kernel for the shape (head_dim other than 64).
+    :func:`norm_rope` on q and k.  Returns None where the library has no kernel for it (:func:`prepass_takes`).
 
     ``pooled="final"``: q_c and k_c are normalised and rotated too, at the truncated mean position of their block
     (:func:`norm_rope` at ``block_positions``); ``keep_raw`` then appends their raw values to the result.
@@ -397,9 +402,9 @@ def qkv_prepass(qkv: torch.Tensor, num_heads: int, block: int, positions: Option
     (else: row 0)."""
     _need_device(qkv)
     _forward_only(qkv)
-    b, n, c3 = qkv.shape
+    b, n = qkv.shape[:2]
     h = num_heads
-    if c3 != 3 * h * 64 or qkv.stride(-1) != 1 or qkv.stride(1) < c3:
+    if not prepass_takes(qkv, h):
         return None
     assert (q_ln is None) == (k_ln is None), "q and k are normalised together or not at all"
     assert pooled in ("raw", "final", None) and (tokens or pooled)

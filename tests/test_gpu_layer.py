@@ -307,3 +307,19 @@ def test_gate_modules_that_do_more_than_their_forward_are_called(what):
     finally:
         for handle in handles:
             handle.remove()
+
+
+class _TransposedLinear(torch.nn.Linear):
+    def forward(self, x):
+        return super().forward(x).transpose(1, 2).contiguous().transpose(1, 2)
+
+
+@pytest.mark.parametrize("block_size", [8, 4])
+@pytest.mark.parametrize("with_pos", [True, False])
+def test_layer_takes_a_projection_in_any_layout(block_size, with_pos):
+    m, x = _layer_and_input(block_size, RoPE2D(100.0))
+    pos = torch.randint(0, 30, (1, 200, 2), device=DEV) if with_pos else None
+    with torch.no_grad():
+        want = m(x, xpos=pos)
+        m.qkv.__class__ = _TransposedLinear
+        assert torch.equal(m(x, xpos=pos), want)
