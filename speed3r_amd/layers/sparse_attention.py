@@ -82,6 +82,8 @@ def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Op
         return None
     cos = sin = inv_freq = None
     if pos is not None:
+        if not training and type(attn.rope).tables is not RoPE2D.tables and not (n_pos or attn.rope.max_positions):
+            n_pos = int(pos.max()) + 1   # (the kernels' own angles are RoPE2D's: tables of another kind hold every position)
         cos, sin, inv_freq = attn.rope.fused_tables(64, n_pos, qkv.device, qkv.dtype, bounded=not training)
     return (pos, cos, sin, inv_freq, (attn.q_norm.weight, attn.q_norm.bias) if ln else None,
             (attn.k_norm.weight, attn.k_norm.bias) if ln else None, attn.q_norm.eps if ln else 0.0)

@@ -323,3 +323,22 @@ def test_layer_takes_a_projection_in_any_layout(block_size, with_pos):
         want = m(x, xpos=pos)
         m.qkv.__class__ = _TransposedLinear
         assert torch.equal(m(x, xpos=pos), want)
+
+
+class _HalfAngles(RoPE2D):
+    """Tables of its own, as a subclass that stretches its positions lays them out."""
+
+    def tables(self, head_dim, n_pos, device, dtype):
+        t = torch.arange(n_pos, device=device, dtype=torch.float32)[:, None] / 2
+        ang = (t * self.inv_freq(head_dim, device)).to(dtype)
+        return ang.cos().contiguous(), ang.sin().contiguous()
+
+
+@pytest.mark.parametrize("block_size", [8, 4])
+def test_a_rope_with_tables_of_its_own_rotates_every_position_by_them(block_size):
+    """Positions up to 100, with a bound given for the call and without one."""
+    m, x = _layer_and_input(block_size, _HalfAngles(100.0))
+    pos = torch.randint(0, 101, (1, 200, 2), generator=torch.Generator().manual_seed(1))
+    pos[0, 7] = 100
+    with torch.no_grad():
+        assert torch.equal(m(x, xpos=pos.to(DEV)), m(x, xpos=pos.to(DEV), n_pos=101))
