@@ -37,7 +37,7 @@ class RoPE2D(nn.Module):
     def tables(self, head_dim: int, n_pos: int, device, dtype):
         """cos, sin ``[n_pos, head_dim // 4]`` in ``dtype``: row p holds cos/sin of the angles ``p * inv_freq`` after
         their rounding to ``dtype`` (the reference's table, pos_embed.py:121-131, without the duplicated half)."""
-        key = (head_dim, n_pos, str(device), dtype)
+        key = (self.base, head_dim, n_pos, str(device), dtype)
         if key not in self._tables:
             inv_freq = self.inv_freq(head_dim, device)
             with torch.inference_mode(False), torch.no_grad():   # kept for training calls too, which save them
@@ -48,7 +48,7 @@ class RoPE2D(nn.Module):
 
     def inv_freq(self, head_dim: int, device) -> torch.Tensor:
         """fp32 ``[head_dim // 4]``: the angle of position p is ``p * inv_freq`` (before its rounding to the tokens' dtype)."""
-        key = (head_dim, str(device))
+        key = (self.base, head_dim, str(device))
         if key not in self._tables:
             half = head_dim // 2
             with torch.inference_mode(False), torch.no_grad():

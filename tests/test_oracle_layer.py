@@ -125,3 +125,12 @@ def test_rotation_tables_made_in_inference_mode_serve_training():
     with torch.inference_mode():
         tables = rope.fused_tables(64, None, torch.device("cpu"), torch.bfloat16)
     assert not any(t.is_inference() for t in tables)
+
+
+def test_rotation_tables_follow_a_changed_base():
+    rope = RoPE2D(100.0)
+    rope.tables(64, 8, "cpu", torch.float32), rope.inv_freq(64, "cpu")
+    rope.base = 1000.0
+    fresh = RoPE2D(1000.0)
+    assert torch.equal(rope.inv_freq(64, "cpu"), fresh.inv_freq(64, "cpu"))
+    assert all(torch.equal(a, b) for a, b in zip(rope.tables(64, 8, "cpu", torch.float32), fresh.tables(64, 8, "cpu", torch.float32)))
