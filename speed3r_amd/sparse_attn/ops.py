@@ -686,11 +686,16 @@ class _CompressedAttnFn(torch.autograd.Function):
         return dq, dk, dv, None, None, None   # (the reference's backward does not know of `causal` either, :653-666)
 
 
+def _at_16_bytes(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """``t`` or, where it does not start at a multiple of 16 bytes (a view of a flat buffer), a copy that does."""
+    return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
+
+
 def gated_merge_bwd(dout: torch.Tensor, o_cmp: torch.Tensor, o_sel: torch.Tensor, gate: torch.Tensor, block: int):
     """Gradient of :func:`gated_merge` (bf16/fp16, head_dim 64): ``(d_o_cmp, d_o_sel, d_gate, delta_cmp, delta_sel)``, d_gate
     as the ``[B,H,N,2]`` view of a ``[B,N,H,2]`` tensor, the deltas as :func:`attn_bwd` takes them."""
     b, h, n, d = o_sel.shape
-    dout, o_cmp, o_sel, gate = dout.contiguous(), o_cmp.contiguous(), o_sel.contiguous(), _last_contig(gate)
+    dout, o_cmp, o_sel, gate = _at_16_bytes(dout.contiguous()), o_cmp.contiguous(), o_sel.contiguous(), _last_contig(gate)
     d_oc, d_os = torch.empty_like(o_cmp), torch.empty_like(o_sel)
     d_gate = gate.new_empty((b, n, h, 2))
     delta_c = torch.empty(o_cmp.shape[:3], dtype=torch.float32, device=gate.device)
@@ -767,11 +772,12 @@ def layer_core_autograd(qkv: torch.Tensor, gate: torch.Tensor, heads: int, block
     """``(out [B,N,C], indices)`` of the layer between its projections, differentiable in qkv, gate and the norm parameters,
     or None where the kernels are not built (bf16/fp16, head_dim 64, blocks of 64 or 16 tokens)."""
     if qkv.dtype not in (torch.bfloat16, torch.float16) or gate.dtype != qkv.dtype or qkv.shape[-1] != 3 * heads * 64 or block not in (64, 16) \
-            or not qkv.is_contiguous():
+            or not qkv.is_contiguous() or qkv.data_ptr() % 16:
         return None
     if xpos is not None and xpos.is_inference():   # (such a tensor can't be saved for the backward)
         xpos = xpos.clone()
-    return _LayerCoreFn.apply(qkv, gate, *(q_ln or (None, None)), *(k_ln or (None, None)), xpos, cos, sin, inv_freq, heads, block, topk, eps)
+    params = [_at_16_bytes(t) for t in (*(q_ln or (None, None)), *(k_ln or (None, None)))]
+    return _LayerCoreFn.apply(qkv, gate, *params, xpos, cos, sin, inv_freq, heads, block, topk, eps)
 
 
 def _wants_grad(*ts: torch.Tensor) -> bool:

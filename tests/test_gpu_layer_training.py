@@ -136,3 +136,40 @@ def test_training_with_positions_of_any_type(dtype, block_size):
 def test_training_with_positions_below_zero(block_size, low, high):
     x, pos, dout = _inputs(200, low=low, high=high)
     _same(_step(_layer(RoPE2D(100.0), block_size, topk=16), x, pos, dout), _step(_layer(TorchRope(RoPE2D(100.0)), block_size, topk=16), x, pos, dout))
+
+
+def _flat_norms(m):
+    """The norm parameters as views of one flat buffer, none of them at a multiple of 16 bytes."""
+    flat = torch.cat([torch.zeros(1, dtype=m.q_norm.weight.dtype, device=DEV)] + [t.detach() for norm in (m.q_norm, m.k_norm) for t in (norm.weight, norm.bias)])
+    views = flat[1:].split(64)
+    for i, norm in enumerate((m.q_norm, m.k_norm)):
+        norm.weight, norm.bias = nn.Parameter(views[2 * i]), nn.Parameter(views[2 * i + 1])
+    assert all(t.data_ptr() % 16 for t in (*m.q_norm.parameters(), *m.k_norm.parameters()))
+    return m
+
+
+@pytest.mark.parametrize("norm_dtype", [torch.bfloat16, torch.float32])
+def test_training_with_norm_parameters_off_a_16_byte_boundary(norm_dtype):
+    x, pos, dout = _inputs(200)
+    results = []
+    for rope in (RoPE2D(100.0), TorchRope(RoPE2D(100.0))):
+        m = _layer(rope)
+        m.q_norm.to(norm_dtype), m.k_norm.to(norm_dtype)
+        _flat_norms(m)
+        if norm_dtype == torch.float32:
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                results.append(_step(m, x, pos, dout))
+        else:
+            results.append(_step(m, x, pos, dout))
+    _same(*results)
+
+
+def test_training_with_an_output_gradient_off_a_16_byte_boundary():
+    x, pos, dout = _inputs(200)
+    odd = torch.empty(dout.numel() + 1, dtype=dout.dtype, device=DEV)[1:].view(dout.shape).copy_(dout)
+    results = []
+    for grad in (odd, dout):
+        m = _layer(RoPE2D(100.0))
+        m.proj = nn.Identity()
+        results.append(_step(m, x, pos, grad))
+    assert all(torch.equal(results[0][k], results[1][k]) for k in results[1])
