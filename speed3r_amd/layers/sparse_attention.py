@@ -146,27 +146,41 @@ class SparseFlashAttentionRope(nn.Module):
 
     def _forward_with_grad(self, x: Tensor, xpos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
         """The same layer for training.  Between its projections it is one differentiable operator whose forward and
-        backward are kernels (``ops.layer_core_autograd``).  Where that is not built (another norm or rope module, blocks of
+        backward are kernels (``ops.layer_core_autograd``; where only the gate is trained, the attention without gradients
+        and the merge as a torch expression).  Where that is not built (another norm or rope module, blocks of
         128 or 256 tokens): a composition in which the two attention operators carry their own backward kernels and pooling,
         qk-norm/RoPE and the gated merge run as the torch expressions of the reference (sparse_attention.py:97-110,120-136),
         whose gradients autograd provides."""
         b, n, c = x.shape
         h = self.num_heads
-        d = c // h
         block = self.block_size ** 2
-        nc = -(-n // block)
         qkv = self.qkv(x)
         gate = self.gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)              # [B, H, N, 2]
         use_pos = xpos is not None and self.rope is not None
         fused = fused_qk_args(self, qkv, xpos if use_pos else None, n_pos, training=True)
+        branches = None
         if fused is not None and self.topk in (1, 2, 4, 8, 16, 32, 64):
             pos, cos, sin, inv_freq, q_ln, k_ln, eps = fused
             core = ops.layer_core_autograd(qkv, gate, h, block, self.topk, pos, cos, sin, inv_freq, q_ln, k_ln, eps)
             if core is not None:
-                out, idx = core
+                *branches, idx = core
                 if self.keep_topk_idx:
                     self.last_topk_idx = idx
-                return self.proj_drop(self.proj(out))
+                if len(branches) == 1:
+                    return self.proj_drop(self.proj(branches[0]))
+        o_c, o_s = branches if branches is not None else self._branches_with_grad(qkv, xpos if use_pos else None)
+        blk = torch.arange(n, device=x.device) // block
+        out = gate[..., 0:1] * o_c[:, :, blk] + gate[..., 1:2] * o_s           # [B, H, N, D]
+        out = out.permute(0, 2, 1, 3).reshape(b, n, c)
+        return self.proj_drop(self.proj(out))
+
+    def _branches_with_grad(self, qkv: Tensor, xpos: Optional[Tensor]):
+        """Outputs of the two attention branches as a composition of torch expressions around the attention operators."""
+        b, n, c3 = qkv.shape
+        h = self.num_heads
+        d = c3 // (3 * h)
+        block = self.block_size ** 2
+        nc = -(-n // block)
         q, k, v = qkv.view(b, n, 3, h, d).permute(2, 0, 3, 1, 4).unbind(0)    # each [B, H, N, D]
 
         def pool(t):  # block means; a ragged tail block averages its valid tokens
@@ -182,19 +196,14 @@ class SparseFlashAttentionRope(nn.Module):
             t = norm(t).to(t.dtype)
             return self.rope(t, pos) if pos is not None else t
 
-        pos_c = block_positions(xpos, block) if use_pos else None
+        pos_c = block_positions(xpos, block) if xpos is not None else None
         q_c, k_c, v_c = pool(q), pool(k), pool(v)
         q_c, k_c = norm_rope(q_c, self.q_norm, pos_c), norm_rope(k_c, self.k_norm, pos_c)
         o_c, idx = flash_attn_topk_func(q_c, k_c, v_c, self.topk)
         if self.keep_topk_idx:
             self.last_topk_idx = idx
-        pos = xpos if use_pos else None
-        q, k = norm_rope(q, self.q_norm, pos), norm_rope(k, self.k_norm, pos)
-        o_s = ops.select_attn_autograd(q, k, v, idx, block)
-        blk = torch.arange(n, device=x.device) // block
-        out = gate[..., 0:1] * o_c[:, :, blk] + gate[..., 1:2] * o_s           # [B, H, N, D]
-        out = out.permute(0, 2, 1, 3).reshape(b, n, c)
-        return self.proj_drop(self.proj(out))
+        q, k = norm_rope(q, self.q_norm, xpos), norm_rope(k, self.k_norm, xpos)
+        return o_c, ops.select_attn_autograd(q, k, v, idx, block)
 
     def forward(self, x: Tensor, attn_bias=None, xpos: Optional[Tensor] = None, n_pos: Optional[int] = None) -> Tensor:
         """``n_pos`` (optional, beyond the reference's signature): an upper bound, exclusive, of the coordinates in

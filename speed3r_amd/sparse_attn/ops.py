@@ -770,13 +770,21 @@ class _LayerCoreFn(torch.autograd.Function):
 
 def layer_core_autograd(qkv: torch.Tensor, gate: torch.Tensor, heads: int, block: int, topk: int, xpos, cos, sin, inv_freq, q_ln, k_ln, eps: float):
     """``(out [B,N,C], indices)`` of the layer between its projections, differentiable in qkv, gate and the norm parameters,
-    or None where the kernels are not built (bf16/fp16, head_dim 64, blocks of 64 or 16 tokens)."""
+    or None where the kernels are not built (bf16/fp16, head_dim 64, blocks of 64 or 16 tokens).  Where only the gate
+    wants a gradient: ``(o_cmp, o_sel, indices)``, constants of the merge, whose gradient is a product of torch."""
     if qkv.dtype not in (torch.bfloat16, torch.float16) or gate.dtype != qkv.dtype or qkv.shape[-1] != 3 * heads * 64 or block not in (64, 16) \
             or not qkv.is_contiguous() or qkv.data_ptr() % 16:
         return None
     if xpos is not None and xpos.is_inference():   # (such a tensor can't be saved for the backward)
         xpos = xpos.clone()
     params = [_at_16_bytes(t) for t in (*(q_ln or (None, None)), *(k_ln or (None, None)))]
+    if not _wants_grad(qkv, *params):
+        q_ln, k_ln = (params[:2], params[2:]) if q_ln is not None else (None, None)
+        with torch.no_grad():
+            q, k, v, q_c, k_c, v_c = qkv_prepass(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, pooled="final", inv_freq=inv_freq, signed=True)
+            o_c, idx = compressed_attn_topk(q_c, k_c, v_c, topk)
+            o_s = select_attn(q, k, v, idx, block)
+            return (o_c, o_s, idx) if gate.requires_grad else (gated_merge(o_c, o_s, gate, block), idx)
     return _LayerCoreFn.apply(qkv, gate, *params, xpos, cos, sin, inv_freq, heads, block, topk, eps)
 
 

@@ -173,3 +173,26 @@ def test_training_with_an_output_gradient_off_a_16_byte_boundary():
         m.proj = nn.Identity()
         results.append(_step(m, x, pos, grad))
     assert all(torch.equal(results[0][k], results[1][k]) for k in results[1])
+
+
+def test_training_of_the_gate_alone_runs_no_attention_backward(monkeypatch):
+    """Nothing but the gate wants a gradient: the attention's is not computed, and the gate's is what it is in full
+    training; a second derivative goes through it like through any product."""
+    from speed3r_amd.sparse_attn import ops
+
+    x, pos, dout = _inputs(200)
+    want = _step(_layer(RoPE2D(100.0)), x, pos, dout)
+    m = _layer(RoPE2D(100.0)).requires_grad_(False)
+    m.gate.requires_grad_(True)
+    ran = []
+    for name in ("attn_bwd", "qkv_prepass_bwd", "key_block_lists"):
+        real = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *a, _real=real, _name=name, **kw: (ran.append(_name), _real(*a, **kw))[1])
+    out = m(x, xpos=pos)
+    params = list(m.gate.parameters())
+    got = torch.autograd.grad(out, params, dout, create_graph=True)
+    assert ran == []
+    _same({"weight": got[0].detach(), "bias": got[1].detach(), "out": out.detach()},
+          {"weight": want["gate.0.weight"], "bias": want["gate.0.bias"], "out": want["out"]})
+    second = torch.autograd.grad(sum(g.float().square().sum() for g in got), params)
+    assert all(torch.isfinite(t).all() and t.abs().max() > 0 for t in second)
