@@ -723,8 +723,8 @@ def qkv_prepass_bwd(qkv: torch.Tensor, num_heads: int, block: int, positions, co
     off = [d_qkv.data_ptr() + i * num_heads * 64 * d_qkv.element_size() for i in range(3)]
     d_norm = work = None
     if q_ln is not None:
-        work = torch.empty((PREPASS_BWD_ROWS + 1, 256), dtype=torch.float32, device=qkv.device)
-        d_norm = work[PREPASS_BWD_ROWS].view(4, 64)
+        work = torch.empty((PREPASS_BWD_ROWS, 256), dtype=torch.float32, device=qkv.device)
+        d_norm = torch.empty((4, 64), dtype=torch.float32, device=qkv.device)
     with _on(qkv.device):
         rc = _lib.lib().s3r_layer_prepass_bwd(ctypes.byref(a), *(t.data_ptr() for t in grads), *off,
                                               d_norm.data_ptr() if d_norm is not None else None,
@@ -764,7 +764,8 @@ class _LayerCoreFn(torch.autograd.Function):
         full = attn_bwd(q, k, v, o_s, d_os, lse, idx, block, delta=delta_s)
         q_ln, k_ln = ((q_w, q_b), (k_w, k_b)) if q_w is not None else (None, None)
         d_qkv, d_norm = qkv_prepass_bwd(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, (q_raw, k_raw), (*full, *pooled), inv_freq, signed=True)
-        params = [d_norm[i].to(t.dtype) if t is not None else None for i, t in enumerate((q_w, q_b, k_w, k_b))]
+        # (tensors of their own: autograd keeps what it is given as .grad)
+        params = [d_norm[i].to(t.dtype, copy=True) if t is not None else None for i, t in enumerate((q_w, q_b, k_w, k_b))]
         return d_qkv, d_gate, *params, *([None] * 8)
 
 

@@ -196,3 +196,17 @@ def test_training_of_the_gate_alone_runs_no_attention_backward(monkeypatch):
           {"weight": want["gate.0.weight"], "bias": want["gate.0.bias"], "out": want["out"]})
     second = torch.autograd.grad(sum(g.float().square().sum() for g in got), params)
     assert all(torch.isfinite(t).all() and t.abs().max() > 0 for t in second)
+
+
+@pytest.mark.parametrize("norm_dtype", [torch.bfloat16, torch.float32])
+def test_norm_gradients_share_no_storage(norm_dtype):
+    """Each gradient a tensor of its own, nothing of the kernels' workspace behind it."""
+    x, pos, dout = _inputs(200)
+    m = _layer(RoPE2D(100.0))
+    m.q_norm.to(norm_dtype), m.k_norm.to(norm_dtype)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        out = m(x, xpos=pos)
+    out.backward(dout)
+    grads = [t.grad for norm in (m.q_norm, m.k_norm) for t in norm.parameters()]
+    assert all(g.dtype == norm_dtype and g.untyped_storage().nbytes() == g.numel() * g.element_size() for g in grads)
+    assert len({g.untyped_storage().data_ptr() for g in grads}) == 4
