@@ -76,7 +76,8 @@ def add_and_norm(x: Tensor, scale: nn.Module, branch: Tensor, norm: Optional[nn.
     """``(s, norm(s))`` of the residual sum ``s = x + scale(branch)``: one pass for inference on the GPU (``norm=None``:
     ``(s, None)``)."""
     scaled = isinstance(scale, LayerScale)
-    if norm is not None and x.is_cuda and not torch.is_grad_enabled() and norm.elementwise_affine:
+    plain = not scaled or (type(scale) is LayerScale and "add_to" not in vars(scale))
+    if plain and norm is not None and x.is_cuda and not torch.is_grad_enabled() and norm.elementwise_affine and x.dtype == norm.weight.dtype:
         out = ops.add_layer_norm(x, branch, scale.gamma if scaled else None, norm.weight, norm.bias, norm.eps)
         if out is not None:
             return out
