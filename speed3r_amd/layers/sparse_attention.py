@@ -128,7 +128,8 @@ class SparseFlashAttentionRope(nn.Module):
         self.topk = topk
         self.keep_topk_idx = False   # debugging aid: keep the last forward's block indices in ``last_topk_idx``
         self.last_topk_idx = None
-        self.last_prepass = None     # whether the last forward used the one-pass kernel over the packed projection
+        self.last_prepass = None     # whether the last forward took q, k and the block means from one launch over the packed projection
+        self.last_passes = None      # its launches over the projection: 1, 2 (block means, then q and k) or 0 (kernels per tensor)
         self.last_path = None        # which route the last forward took: "fused-merge", "two-operators" or "autograd"
 
     def _norm_rope(self, t: Tensor, norm: nn.Module, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
@@ -230,10 +231,11 @@ class SparseFlashAttentionRope(nn.Module):
         # kernel, long for so many pooled tokens, starts while the full tokens are still to come.
         fused = fused_qk_args(self, qkv, pos, n_pos)
         q = k = v = None
-        self.last_prepass = False
+        self.last_prepass, self.last_passes = False, 0
         if fused is not None and (pos is not None or fused[4] is not None):   # (else q and k are read in place)
             args = (pos, fused[1], fused[2], *fused[4:])
             self.last_prepass = block >= 32
+            self.last_passes = 1 if self.last_prepass else 2
             if self.last_prepass:
                 q, k, v, q_c, k_c, v_c = ops.qkv_prepass(qkv, h, block, *args, pooled="final", inv_freq=fused[3])
             else:

@@ -47,3 +47,16 @@ def test_fp32_compressed_scores_and_attention(lq, lk):
     assert torch.equal(idx, s3r.topk_rows(s, topk))
     o3 = s3r.compressed_attn_topk(q.to(DEV), kd, vd, topk, softmax_scale=3.0 / math.sqrt(64))[0]
     assert max_abs(o3, oracle.compressed_attention(q, k, v, softmax_scale=3.0 / math.sqrt(64), out_dtype=torch.float32)[0]) <= 3e-5
+
+
+@pytest.mark.parametrize("lq,lk", [(64, 33), (131, 131), (1, 300)])
+def test_fp32_scores_have_the_generic_kernels_bits(lq, lk):
+    """The same tensors at addresses that are no multiples of 16 bytes go through the generic kernel."""
+    g = torch.Generator().manual_seed(lq)
+    q, k, v = (torch.randn((1, 3, n, 64), generator=g).to(DEV) for n in (lq, lk, lk))
+
+    def off(t):
+        return torch.empty(t.numel() + 1, device=DEV)[1:].view(t.shape).copy_(t)
+
+    s = s3r.compressed_attn_topk(q, k, v, 1, return_scores=True)[2]
+    assert torch.equal(s, s3r.compressed_attn_topk(off(q), off(k), off(v), 1, return_scores=True)[2])

@@ -152,10 +152,9 @@ def test_layer_gradients_match_autograd_through_the_oracle(n, block_size, topk):
                                                         (77, 16, False, True), (130, 64, True, False), (5, 64, True, True)])
 @pytest.mark.parametrize("k_bias", [False, True])
 def test_one_pass_over_the_packed_projection_equals_pooling_then_norm_rope(dtype, n, block, with_norm, with_pos, k_bias):
-    """s3r_qkv_prepass (block means of raw q, k, v + LayerNorm + RoPE of q and k in one pass) against s3r_pool_mean on
-    the packed projection followed by s3r_norm_rope on q and k: the same bits, ragged last blocks included.  With both
-    LayerNorm biases and positions (``k_bias``) the kernel runs the instance the layer module launches, in which norm,
-    biases and rotation are compile-time facts; without the k bias the general one."""
+    """s3r_layer_prepass (block means of raw q, k, v + LayerNorm + RoPE of q and k in one pass) against s3r_pool_mean on
+    the packed projection followed by s3r_norm_rope on q and k: the same bits, ragged last blocks included, with and
+    without the k bias (a missing one is staged as zeros)."""
     from speed3r_amd.sparse_attn import ops
     b, h = 2, 3
     g = torch.Generator().manual_seed(n + block)
@@ -178,11 +177,11 @@ def test_one_pass_over_the_packed_projection_equals_pooling_then_norm_rope(dtype
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows", [165, 166, 400])
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 165, 166, 400])
 def test_one_pass_with_rotation_tables_around_the_lds_limit(dtype, rows):
-    """The layer's instance keeps fp32 copies of the rotation tables in LDS while three tables of ``rows`` x 16 values
-    and the LayerNorm rows fit 32 KB (165 rows do, 166 do not); beyond that it reads the caller's tables as before.
-    Both sides of the limit give the bits of pooling followed by s3r_norm_rope, positions up to the last row included."""
+    """The first 64 rows of the rotation tables are held in LDS as fp32; a lane whose position lies in a later row reads
+    that from the caller's tables.  Both sides of the limit give the bits of pooling followed by s3r_norm_rope, positions
+    up to the last row included."""
     from speed3r_amd.sparse_attn import ops
     b, h, n, block = 1, 2, 700, 64
     g = torch.Generator().manual_seed(rows)
@@ -249,7 +248,7 @@ def test_layer_takes_the_one_pass_route_where_it_is_built():
         m2(x)                                   # no norm, no positions: nothing to do to q and k, no pre-pass
         assert m2.last_prepass is False
         m3 = SparseFlashAttentionRope(dim=128, num_heads=2, qk_norm=True, rope=RoPE2D(100.0), block_size=4, topk=4).to(torch.bfloat16).to(DEV).eval()
-        m3(x, xpos=pos)                         # 16-token blocks: separate kernels, the index kernel starts earlier
+        m3(x, xpos=pos)                         # 16-token blocks: the pass in two launches, the index kernel between them
         assert m3.last_prepass is False and m3.last_path == "fused-merge"
 
 
@@ -342,3 +341,38 @@ def test_a_rope_with_tables_of_its_own_rotates_every_position_by_them(block_size
     pos[0, 7] = 100
     with torch.no_grad():
         assert torch.equal(m(x, xpos=pos.to(DEV)), m(x, xpos=pos.to(DEV), n_pos=101))
+
+
+def test_last_passes_counts_the_launches_over_the_projection():
+    """One where the blocks are long, two (block means, then tokens) at 16-token blocks, none where the pass is not built."""
+    pos = torch.randint(0, 30, (1, 200, 2), device=DEV)
+    for block_size, rope, passes in ((8, RoPE2D(100.0), 1), (4, RoPE2D(100.0), 2), (4, _Calls(RoPE2D(100.0)), 0)):
+        m, x = _layer_and_input(block_size, rope)
+        with torch.no_grad():
+            m(x, xpos=pos)
+        assert m.last_passes == passes and m.last_path == "fused-merge"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,block", [(130, 64), (77, 16), (320, 64)])
+def test_one_pass_entry_point_with_plain_arguments(dtype, n, block):
+    """s3r_qkv_prepass itself (int32 positions, tables and norm parameters in the tensors' type) against s3r_pool_mean and
+    s3r_norm_rope: the same bits."""
+    from speed3r_amd import _lib
+    from speed3r_amd.sparse_attn import ops
+    b, h = 2, 3
+    g = torch.Generator().manual_seed(n)
+    qkv = (torch.randn((b, n, 3 * h * 64), generator=g) * 0.7).to(dtype).to(DEV)
+    pos = torch.randint(0, 40, (b, n, 2), generator=g, dtype=torch.int32).to(DEV)
+    cos, sin = RoPE2D(freq=100.0).tables(64, 40, DEV, dtype)
+    ln = [torch.randn(64, generator=g).to(dtype).to(DEV) for _ in range(4)]
+    nc = -(-n // block)
+    outs = [torch.empty((b, h, rows, 64), dtype=dtype, device=DEV) for rows in (n, n, nc, nc, nc)]
+    q, k, v = qkv.view(b, n, 3, h, 64).permute(2, 0, 3, 1, 4).unbind(0)
+    rc = _lib.lib().s3r_qkv_prepass(q.data_ptr(), k.data_ptr(), v.data_ptr(), *(t.data_ptr() for t in outs), pos.data_ptr(), cos.data_ptr(),
+                                    sin.data_ptr(), 40, *(t.data_ptr() for t in ln), 1e-6, b, h, n, 64, block, *q.stride()[:3],
+                                    *pos.stride()[:2], ops._code(qkv), torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "s3r_qkv_prepass")
+    want = (ops.norm_rope(q, pos, cos, sin, ln[0], ln[1], 1e-6), ops.norm_rope(k, pos, cos, sin, ln[2], ln[3], 1e-6), *ops.pool_qkv_packed(qkv, h, block))
+    for got, w in zip(outs, want):
+        assert torch.equal(got, w)

@@ -210,3 +210,21 @@ def test_norm_gradients_share_no_storage(norm_dtype):
     grads = [t.grad for norm in (m.q_norm, m.k_norm) for t in norm.parameters()]
     assert all(g.dtype == norm_dtype and g.untyped_storage().nbytes() == g.numel() * g.element_size() for g in grads)
     assert len({g.untyped_storage().data_ptr() for g in grads}) == 4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("block_size,n,topk", [(8, 200, 2), (8, 256, 4), (4, 200, 8), (4, 250, 16)])
+def test_mixed_precision_training_step(dtype, block_size, n, topk):
+    """fp32 weights and inputs under autocast, two sequences, whole and ragged last blocks: every gradient in its
+    parameter's type, against the composition of torch modules."""
+    x, pos, dout = _inputs(n, b=2, dtype=torch.float32, high=30)
+    results = []
+    for rope in (RoPE2D(100.0), TorchRope(RoPE2D(100.0))):
+        m = _layer(rope, block_size, dtype=torch.float32, topk=topk)
+        m.keep_topk_idx = True
+        with torch.autocast("cuda", dtype=dtype):
+            results.append((_step(m, x, pos, dout.to(dtype)), m.last_topk_idx))
+    (got, idx), (want, want_idx) = results
+    assert (idx == want_idx).float().mean() >= 0.98   # (scores a rounding apart can change places)
+    assert all(got[k].dtype == torch.float32 for k in got if k != "out") and got["out"].dtype == dtype
+    _same(got, want)
