@@ -26,7 +26,8 @@ struct PrepassParams {
 
 // Table rows held in LDS as fp32 (cosine, sine and minus sine: 192 bytes per row).  64 rows = 12 KB: every frame of up
 // to 64 patches a side; further rows are read from the caller's tables.  A workgroup copies all of them, so that more
-// rows than a call has positions would cost time.
+// rows than a call has positions would cost time.  Against up to 165 rows in LDS (as many as four resident workgroups hold
+// without the lanes' slots), 100 000 tokens x 16 heads, bf16: 209 us / 206 us at 100 positions a side, 225 / 222 at 164.
 constexpr int kStagedRows = 64;
 // tables, parameter rows and, with a rotation, the lanes' slots (64 bytes each at most)
 inline size_t staged_bytes(int rows, bool rot) { return ((size_t)3 * rows * 16 + 4 * 64) * sizeof(float) + (rot ? 256 * 64 : 0); }
