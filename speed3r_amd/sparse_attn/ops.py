@@ -484,7 +484,8 @@ def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) ->
     _forward_only(x, weight)
     c, o = x.shape[-1], weight.shape[0]
     ts = [t for t in (x, weight, bias) if t is not None]
-    if x.dtype not in (torch.bfloat16, torch.float16) or c % 256 or c > 1024 or o > 32 or o % 2 or x.numel() == 0 or weight.shape != (o, c):
+    if x.dtype not in (torch.bfloat16, torch.float16) or c % 256 or c > 1024 or o > 32 or o % 2 or x.numel() == 0 or weight.shape != (o, c) \
+            or (bias is not None and bias.shape != (o,)):
         return None
     if any(t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
         return None

@@ -35,6 +35,7 @@ def test_gate_has_no_kernel_for_other_forms():
     assert ops.gate(x.t()[:256], w[:, :4], None) is None
     assert ops.gate(x, torch.zeros((34, 1024), dtype=torch.bfloat16, device=DEV), None) is None
     assert ops.gate(x[:0], w, None) is None
+    assert ops.gate(x, w, w[0, :1]) is None   # (a bias that torch spreads over the outputs)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
