@@ -37,23 +37,31 @@ class RoPE2D(nn.Module):
     def tables(self, head_dim: int, n_pos: int, device, dtype):
         """cos, sin ``[n_pos, head_dim // 4]`` in ``dtype``: row p holds cos/sin of the angles ``p * inv_freq`` after
         their rounding to ``dtype`` (the reference's table, pos_embed.py:121-131, without the duplicated half)."""
-        key = (self.base, head_dim, n_pos, str(device), dtype)
-        if key not in self._tables:
-            inv_freq = self.inv_freq(head_dim, device)
-            with torch.inference_mode(False), torch.no_grad():   # kept for training calls too, which save them
-                t = torch.arange(n_pos, device=device, dtype=torch.float32)
-                ang = (t[:, None] * inv_freq).to(dtype)   # (a plain product: fp32 under autocast too)
-                self._tables[key] = (ang.cos().contiguous(), ang.sin().contiguous())
-        return self._tables[key]
+        def lay_out():
+            t = torch.arange(n_pos, device=device, dtype=torch.float32)
+            ang = (t[:, None] * self.inv_freq(head_dim, device)).to(dtype)   # (a plain product: fp32 under autocast too)
+            return ang.cos().contiguous(), ang.sin().contiguous()
+        return self._kept((self.base, head_dim, n_pos, str(device), dtype), lay_out)
 
     def inv_freq(self, head_dim: int, device) -> torch.Tensor:
         """fp32 ``[head_dim // 4]``: the angle of position p is ``p * inv_freq`` (before its rounding to the tokens' dtype)."""
-        key = (self.base, head_dim, str(device))
-        if key not in self._tables:
+        def lay_out():
             half = head_dim // 2
-            with torch.inference_mode(False), torch.no_grad():
-                self._tables[key] = 1.0 / (self.base ** (torch.arange(0, half, 2, device=device, dtype=torch.float32) / half))
-        return self._tables[key]
+            return (1.0 / (self.base ** (torch.arange(0, half, 2, device=device, dtype=torch.float32) / half)),)
+        return self._kept((self.base, head_dim, str(device)), lay_out)[0]
+
+    def _kept(self, key, lay_out):
+        """The tensors of ``key``, laid out once for every later call, whichever its stream or mode."""
+        if key in self._tables:
+            return self._tables[key]
+        with torch.inference_mode(False), torch.no_grad():   # kept for training calls too, which save them
+            made = lay_out()
+        if made[0].is_cuda:
+            if torch.cuda.is_current_stream_capturing():     # they get their values when the graph runs, and go with it
+                return made
+            torch.cuda.current_stream(made[0].device).synchronize()
+        self._tables[key] = made
+        return made
 
     def _cos_sin(self, pos1d: torch.Tensor, half: int, dtype: torch.dtype):
         # pos1d [B, N] integer coordinates -> cos, sin [B, 1, N, half] with the two quarters holding the same angles

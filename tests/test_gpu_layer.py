@@ -376,3 +376,18 @@ def test_one_pass_entry_point_with_plain_arguments(dtype, n, block):
     want = (ops.norm_rope(q, pos, cos, sin, ln[0], ln[1], 1e-6), ops.norm_rope(k, pos, cos, sin, ln[2], ln[3], 1e-6), *ops.pool_qkv_packed(qkv, h, block))
     for got, w in zip(outs, want):
         assert torch.equal(got, w)
+
+
+def test_rotation_tables_laid_out_while_a_graph_is_captured_are_not_kept():
+    """They have no values before the graph runs."""
+    rope, fresh = RoPE2D(100.0), RoPE2D(100.0)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        inside = (*rope.tables(64, 64, DEV, torch.bfloat16), rope.inv_freq(64, DEV))
+    outside = (*rope.tables(64, 64, DEV, torch.bfloat16), rope.inv_freq(64, DEV))
+    want = (*fresh.tables(64, 64, DEV, torch.bfloat16), fresh.inv_freq(64, DEV))
+    assert all(torch.equal(a, b) for a, b in zip(outside, want))
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(inside, want))
