@@ -299,6 +299,17 @@ int s3r_add_layer_norm(const void* x, const void* a, const void* gamma, void* s,
                        int64_t rows, int C, int dtype, void* stream);
 
 /*
+ * A linear layer of the inference paths  y[r,:] = act(x[r,:] W^T + bias)  (the projections around the attention,
+ * pi3/models/layers/sparse_attention.py:93,140, and the MLPs); fp32 sums, bias and activation in fp32, one rounding.
+ *   x: [M, K], w: [N, K], y: [M, N] with row strides ldx, ldw, ldy (elements); bias: [N] or NULL; bf16 / fp16, K a multiple of
+ *   128, N of 8; x, w, y and their rows multiples of 16 bytes, bias of 8.
+ */
+#define S3R_ACT_NONE 0
+#define S3R_ACT_GELU 1 /* exact: x/2 (1 + erf(x / sqrt 2)) */
+int s3r_linear(const void* x, const void* w, const void* bias, void* y, int64_t M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
+               int activation, int dtype, void* stream);
+
+/*
  * The layer's gate  out[r,:] = sigmoid(x[r,:] W^T + bias)  (pi3/models/layers/sparse_attention.py:88,127); fp32 sums, the
  * product with its bias and the sigmoid each rounded to the I/O dtype.
  *   x: contiguous [rows, C], w: contiguous [O, C], bias: [O] or NULL, out: contiguous [rows, O]; bf16 / fp16, C a multiple of

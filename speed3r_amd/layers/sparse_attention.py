@@ -36,6 +36,24 @@ def calls_forward_only(m: nn.Module, kind: type) -> bool:
         or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks)
 
 
+def takes_kernels(x: Tensor) -> bool:
+    """Whether a call on ``x`` is an ordinary one: a tensor on the GPU, without autocast, tracing, compilation or a transform
+    (vmap, forward-mode derivatives) that has to see the torch operations."""
+    return x.is_cuda and type(x) is Tensor and not torch.is_autocast_enabled("cuda") and torch._C._functorch.peek_interpreter_stack() is None \
+        and torch.autograd.forward_ad._current_level < 0 and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+
+
+def linear(m: nn.Linear, x: Tensor, gelu: bool = False) -> Tensor:
+    """``m(x)``, with ``gelu`` followed by ``F.gelu``: for inference one kernel where calling ``m`` would run
+    ``nn.Linear.forward`` and nothing else, the modules otherwise."""
+    if takes_kernels(x) and calls_forward_only(m, nn.Linear) and ops.linear_pays(x.numel() // x.shape[-1], *m.weight.shape) and type(m.weight) is nn.Parameter \
+            and not (torch.is_grad_enabled() and (x.requires_grad or m.weight.requires_grad or (m.bias is not None and m.bias.requires_grad))):
+        out = ops.linear(x, m.weight, m.bias, gelu)
+        if out is not None:
+            return out
+    return nn.functional.gelu(m(x)) if gelu else m(x)
+
+
 def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
     """qk-norm, cast and RoPE of one ``[B,H,N,D]`` tensor (reference sparse_attention.py:103-110,120-124): one fused
     kernel where it is built -- a tensor on the GPU, head_dim 64, ``nn.Identity`` or an affine ``nn.LayerNorm`` of
@@ -219,7 +237,7 @@ class SparseFlashAttentionRope(nn.Module):
         d = c // h
         block = self.block_size ** 2
 
-        qkv = self.qkv(x)                                              # [B, N, 3C], layout (qkv h d)
+        qkv = linear(self.qkv, x)                                      # [B, N, 3C], layout (qkv h d)
         gate = self._gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)      # [B, H, N, 2], strided view
 
         use_pos = xpos is not None and self.rope is not None
@@ -270,5 +288,5 @@ class SparseFlashAttentionRope(nn.Module):
             self.last_path = "two-operators"
             out = ops.gated_merge(o_c, ops.select_attn(q, k, v, idx, block), gate, block)
 
-        out = self.proj(out)
+        out = linear(self.proj, out)
         return self.proj_drop(out)

@@ -21,7 +21,8 @@ pi3/models/layers/transformer_head.py (head decoders, linear pixel-shuffle head)
   the head decoders (:265-269), global attention over 16-token blocks = 4 x 4 patch tiles with the 32 best blocks
   (sparse_attention.py:73,98,112).  The patch grid must split into 4 x 4 tiles (frames of 56-pixel multiples).
 
-All dense GEMMs are library calls (torch on rocBLAS/hipBLASLt); the frame-local dense attentions run on the package's
+The linear layers run on the package's kernel (GELU of the MLPs in its epilogue) for bf16/fp16 inference where their sizes
+allow, else on library calls, as do the patch embedding and the pixel-shuffle heads; the frame-local dense attentions run on the package's
 dense flash kernel (the one behind the compressed branch) for bf16/fp16 inference with head_dim 64, else on
 scaled_dot_product_attention.
 Inference only: call under ``torch.no_grad()`` with the module in one dtype (bf16).
@@ -36,7 +37,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from ..layers import RoPE2D, SparseFlashAttentionRope
-from ..layers.sparse_attention import calls_forward_only, fused_qk_args, norm_rope_fused_or_eager
+from ..layers.sparse_attention import calls_forward_only, fused_qk_args, linear, norm_rope_fused_or_eager
 from ..sparse_attn import ops
 from .token_order import tile_major, tile_major_inverse
 
@@ -48,7 +49,7 @@ class Mlp(nn.Module):
         self.fc2 = nn.Linear(hidden, dim)
 
     def forward(self, x: Tensor) -> Tensor:
-        return self.fc2(F.gelu(self.fc1(x)))
+        return linear(self.fc2, linear(self.fc1, x, gelu=True))
 
 
 class LayerScale(nn.Module):
@@ -105,7 +106,7 @@ class DenseAttentionRope(nn.Module):
     def forward(self, x: Tensor, attn_bias=None, xpos: Optional[Tensor] = None, n_pos: Optional[int] = None) -> Tensor:
         b, n, c = x.shape
         h = self.num_heads
-        qkv = self.qkv(x)
+        qkv = linear(self.qkv, x)
         pos = xpos if self.rope is not None else None
         fused = fused_qk_args(self, qkv, pos, n_pos) if not torch.is_grad_enabled() else None
         qkv_out = None
@@ -120,7 +121,7 @@ class DenseAttentionRope(nn.Module):
             # the package's dense flash kernel (the compressed branch's attention), written straight into [B,N,H,D]
             o = torch.empty((b, n, h, c // h), dtype=x.dtype, device=x.device)
             ops.compressed_attn_topk(q, k, v, None, out=o.permute(0, 2, 1, 3))
-            return self.proj(o.view(b, n, c))
+            return linear(self.proj, o.view(b, n, c))
         o = F.scaled_dot_product_attention(q, k, v)
         return self.proj(o.transpose(1, 2).reshape(b, n, c))
 
@@ -209,7 +210,7 @@ class HeadDecoder(nn.Module):
         self.linear_out = nn.Linear(dim, out_dim)
 
     def forward(self, x: Tensor, xpos: Tensor, n_pos: Optional[int] = None) -> Tensor:
-        return self.linear_out(run_blocks(self.blocks, self.project(x), None, xpos=xpos, n_pos=n_pos)[0])
+        return linear(self.linear_out, run_blocks(self.blocks, linear(self.project, x), None, xpos=xpos, n_pos=n_pos)[0])
 
 
 class PixelShuffleHead(nn.Module):

@@ -475,6 +475,35 @@ def add_layer_norm(x: torch.Tensor, a: torch.Tensor, gamma: Optional[torch.Tenso
     return s, y
 
 
+# Where the layers leave a product to the library (us on the device, library / kernel): few rows, a handful of tiles
+# (256 x 1024 x 1024 5.5 / 8.7, 1 041 x 1024 x 1024 9.0 / 9.2, 2 016 x 1024 x 1024 10.4 / 9.7), and a long K with fewer tiles than
+# CUs, which the library splits (2 016 x 1024 x 4096 28 / 40, 4 032 x 1024 x 4096 43.5 / 43.7).
+def linear_pays(rows: int, n: int, k: int) -> bool:
+    return rows >= 1024 and (k <= 1024 or -(-rows // 128) * -(-n // 128) >= 256)
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], gelu: bool = False) -> Optional[torch.Tensor]:
+    """``F.linear(x, weight, bias)``, with ``gelu`` followed by ``F.gelu``, in one kernel (inference).
+
+    Returns None where the library has no kernel (bf16/fp16, inputs a multiple of 128, outputs of 8, 16-byte aligned tensors
+    of one dtype with adjacent values and rows of one stride)."""
+    _need_device(x)
+    _forward_only(x, weight)
+    k, n = x.shape[-1], weight.shape[0]
+    ts = [t for t in (x, weight, bias) if t is not None]
+    if x.dtype not in (torch.bfloat16, torch.float16) or k % 128 or n % 8 or x.numel() == 0 or weight.shape != (n, k) or k > 1 << 20 or n > 1 << 20 \
+            or (bias is not None and bias.shape != (n,)):
+        return None
+    if any(t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
+        return None
+    out = x.new_empty((*x.shape[:-1], n))
+    with _on(x.device):
+        rc = _lib.lib().s3r_linear(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                                   x.numel() // k, n, k, k, k, n, 1 if gelu else 0, _code(x), _stream(x))
+    _lib.check(rc, "s3r_linear")
+    return out
+
+
 def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """``sigmoid(F.linear(x, weight, bias))`` for the few outputs of the layer's gate, in one pass over ``x`` (inference).
 
