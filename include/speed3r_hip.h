@@ -310,6 +310,18 @@ int s3r_linear(const void* x, const void* w, const void* bias, void* y, int64_t 
                int activation, int dtype, void* stream);
 
 /*
+ * s3r_linear and s3r_layer_prepass in one: the layer's projection  [q | k | v] = x W^T + bias  and, of it,
+ * q and k after LayerNorm and RoPE2D, v, and the finished block means (sparse_attention.py:93-110,115-124).
+ *   x: [B*N, C] rows of stride ldx, w: [3*C, C] of stride ldw, bias: [3*C] or NULL, C = 64 H; v_out: contiguous [B,H,N,64];
+ *   a: as for s3r_layer_prepass (q, k, v and the strides are not read): q_out, k_out, positions and tables are required,
+ *   the three means and the norms optional; means only with norms, `finish_pooled` and without q_raw, k_raw.
+ * bf16 / fp16, an even number of heads, block 16 or 64; several sequences: 256 tokens or more each, with means a multiple of
+ * the block.  Rounding: the projection to the I/O dtype, then once at the end (s3r_layer_prepass also rounds in between).
+ */
+int s3r_qkv_project(const void* x, const void* w, const void* bias, int64_t ldx, int64_t ldw, void* v_out, const struct s3r_prepass_args* a,
+                    void* stream);
+
+/*
  * The layer's gate  out[r,:] = sigmoid(x[r,:] W^T + bias)  (pi3/models/layers/sparse_attention.py:88,127); fp32 sums, the
  * product with its bias and the sigmoid each rounded to the I/O dtype.
  *   x: contiguous [rows, C], w: contiguous [O, C], bias: [O] or NULL, out: contiguous [rows, O]; bf16 / fp16, C a multiple of

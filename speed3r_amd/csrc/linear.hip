@@ -2,13 +2,13 @@
 // function) in the epilogue.  bf16 / fp16, matrix-core bound; the tile is linear_tile.h's.
 //
 // Persistent workgroups.  256 x 256 tiles, one workgroup per CU, where these fill the chip; 128 x 128 tiles, two workgroups
-// per CU, where they do not.  Against the library's product on the same card (us, with bias; and with bias and GELU,
+// per CU, where they do not.  us, this / the library's product on the same card (with bias; and with bias and GELU,
 // where the library's product is followed by a pass over its output):
-//   104 100 x 3072 x 1024     546 / 616     650 / 869
-//     8 064 x 4096 x 1024      56 /  56      66 /  86
-//     8 064 x 3072 x 1024      49 /  54
+//   104 100 x 3072 x 1024     520 / 610     626 / 860
+//     8 064 x 4096 x 1024      58 /  57      68 /  87
+//     8 064 x 1024 x 4096      55 /  58
 //     8 064 x 1024 x 1024      18.5 / 21.3
-//     2 016 x 1024 x 1024       9.7 / 19.8
+//     2 016 x 1024 x 1024       9.7 / 10.4 on the device, 9.7 / 19.8 with the host's share
 // What bounds the large tile: 81 % of the cycles inside the sweep over K are products (8192^3), at the clock the power limit
 // leaves; with K = 1024 the epilogue takes a sixth of a tile.
 #include "linear_tile.h"
@@ -87,15 +87,10 @@ __global__ __launch_bounds__(256, WPS) void linear_kernel(LinearParams p) {
   for (int i = 0; i < Tl::NL; i++) tl.move(lx1, lw1, kb, i);
   tl.begin(lx0, lw0);
   for (;;) {
+    uint2 cb[T];  // this tile's bias (nb moves on to the next tile's)
 #pragma unroll
-    for (int c = 0; c < T; c++) {
-      union { uint2 u; E e[4]; } b;
-      b.u = nb[c];
-#pragma unroll
-      for (int t = 0; t < T; t++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) tl.acc[c][t][i] = (float)b.e[i];
-    }
+    for (int c = 0; c < T; c++) cb[c] = nb[c];
+    tl.clear();
     tl.before_products();
     int left = p.K >> 6;  // even
     do {
@@ -117,6 +112,14 @@ __global__ __launch_bounds__(256, WPS) void linear_kernel(LinearParams p) {
     const int och = n * BN + tl.wn * 16 * T + pc * 8;
     const uint32_t yo = och < p.N ? (uint32_t)(tl.wm * 16 * T + pr) * row_bytes + (uint32_t)och * 2 : 0x80000000u;
     unsigned char* const mine = lst + tl.wave * (2 * kStage);
+    float bias[T][4];  // added last, as the library's product does: the same bits where that does not split K
+#pragma unroll
+    for (int c = 0; c < T; c++) {
+      union { uint2 u; E e[4]; } b;
+      b.u = cb[c];
+#pragma unroll
+      for (int i = 0; i < 4; i++) bias[c][i] = (float)b.e[i];
+    }
 #pragma unroll
     for (int t = 0; t < T; t++) {
       unsigned char* const buf = mine + (t & 1) * kStage;
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(256, WPS) void linear_kernel(LinearParams p) {
         union { V2 v[2]; uint2 u; } o;
 #pragma unroll
         for (int r = 0; r < 2; r++) {
-          float a = tl.acc[c][t][2 * r], b = tl.acc[c][t][2 * r + 1];
+          float a = tl.acc[c][t][2 * r] + bias[c][2 * r], b = tl.acc[c][t][2 * r + 1] + bias[c][2 * r + 1];
           if constexpr (GELU) {
             a = gelu(a);
             b = gelu(b);
@@ -147,16 +150,6 @@ __global__ __launch_bounds__(256, WPS) void linear_kernel(LinearParams p) {
     walk.locate(walk.at, m, n);
   }
   __builtin_amdgcn_s_waitcnt(0x0070);  // no transfer may still write LDS when the wave ends
-}
-
-// Tiles of 256 or of 128.  Time of a round of tiles in steps of the large tile: its K / 64 and 4 for the epilogue; a round
-// of the small ones (two per CU) takes 0.61 of that, half a round (one per CU) 0.36: measured at 2 016 to 104 100 rows, 1024 to
-// 4096 channels; the choice is the faster one at all of them.
-static bool large_tiles(int64_t M, int N) {
-  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256), small = ((M + 127) / 128) * ((N + 127) / 128);
-  const double t_big = (double)((big + 255) / 256);
-  const double t_small = small <= 256 ? 0.36 : 0.61 * (double)((small + 511) / 512);
-  return t_big <= t_small;
 }
 
 template <typename E> static void launch_linear(LinearParams& p, bool act, hipStream_t st) {

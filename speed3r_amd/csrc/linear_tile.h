@@ -27,18 +27,23 @@ __device__ __forceinline__ void to_lds16(const void* base, void* dst, uint32_t v
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0x7fffffff, 0x00020000);
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
 }
-// 16 bytes to base + off unless that lies at or beyond `bytes`
+// 16 bytes to base + off unless that lies at or beyond `bytes`; non-temporal, so that what is written does not push the X and W
+// rows of the tiles to come out of the L2 (104 100 x 3072 x 1024: 546 -> 520 us; the projection with its epilogue 722 -> 697)
 __device__ __forceinline__ void store16_if(void* base, uint32_t bytes, uint32_t off, const uint4& v) {
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
-  __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4*>(&v), rs, off, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4*>(&v), rs, off, 0, 2);
 }
 
-template <typename E> __device__ __forceinline__ void mma_acc(typename Mma<E>::V8 a, typename Mma<E>::V8 b, f32x4& c);
-template <> __device__ __forceinline__ void mma_acc<bf16_t>(bf16x8 a, bf16x8 b, f32x4& c) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-template <> __device__ __forceinline__ void mma_acc<f16_t>(f16x8 a, f16x8 b, f32x4& c) {
-  asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+// Accumulators in the AGPR half of the register file where they fill it (with two waves per SIMD the compiler would split
+// the file in halves for 64 of them).
+template <typename E, bool AGPR> __device__ __forceinline__ void mma_acc(typename Mma<E>::V8 a, typename Mma<E>::V8 b, f32x4& c) {
+  if constexpr (std::is_same<E, bf16_t>::value) {
+    if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+  } else {
+    if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+  }
 }
 
 // LDS row map: rows of 128 bytes (64 values of K), chunk c of row r at chunk position c ^ swizzle(r)
@@ -69,6 +74,7 @@ struct TileWalk {
 template <typename E, int TT, int TC> struct Tile {
   typedef typename Mma<E>::V8 V8;
   static constexpr int BM = 32 * TT, BN = 32 * TC;  // two waves by two
+  static constexpr bool kAgpr = TT * TC == 64;
   static constexpr int NL = TT + TC;                // fragments of a half step; transfers of a step, per wave
   static constexpr int NM = TT * TC;                // products of a half step
   // spacing in sixteenths of a product: reads of the first half step; transfers, and reads, of the second
@@ -128,6 +134,9 @@ template <typename E, int TT, int TC> struct Tile {
     __builtin_amdgcn_s_waitcnt(0x0F70 | (NL & 15) | ((NL >> 4) << 14));  // the first step has landed
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
+    read_first(x0, w0);
+  }
+  template <typename P8> __device__ __forceinline__ void read_first(P8* x0, P8* w0) {
 #pragma unroll
     for (int r = 0; r < NL; r++) read(P, x0, w0, 0, r);
   }
@@ -139,7 +148,7 @@ template <typename E, int TT, int TC> struct Tile {
 #pragma unroll
       for (int r = 0; r < NL; r++)
         if (r * kRead1 / 16 == j) read(Q, lx, lw, 1, r);
-      mma_acc<E>(P.w[j / TT], P.x[j % TT], acc[j / TT][j % TT]);
+      mma_acc<E, kAgpr>(P.w[j / TT], P.x[j % TT], acc[j / TT][j % TT]);
       __builtin_amdgcn_sched_barrier(0);
     }
     // the buffer's last reads are in registers and the other buffer's transfers have landed, in every wave
@@ -153,9 +162,17 @@ template <typename E, int TT, int TC> struct Tile {
         if (r * kMove2 / 16 == j) move(lx, lw, kb, r);
         if (r * kRead2 / 16 + kRead2At == j) read(P, ox, ow, 0, r);
       }
-      mma_acc<E>(Q.w[j / TT], Q.x[j % TT], acc[j / TT][j % TT]);
+      mma_acc<E, kAgpr>(Q.w[j / TT], Q.x[j % TT], acc[j / TT][j % TT]);
       __builtin_amdgcn_sched_barrier(0);
     }
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int c = 0; c < TC; c++)
+#pragma unroll
+      for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[c][t][i] = 0.f;
   }
   // Around the products written out the compiler knows of no hazards: accumulators written by vector instructions are given
   // time before the first product reads them, the last products time before vector instructions read theirs.
@@ -171,9 +188,22 @@ template <typename E, int TT, int TC> struct Tile {
 #pragma unroll
     for (int c = 0; c < TC; c++)
 #pragma unroll
-      for (int t = 0; t < TT; t++) asm volatile("" : "+a"(acc[c][t]));
+      for (int t = 0; t < TT; t++) {
+        if constexpr (kAgpr) asm volatile("" : "+a"(acc[c][t]));
+        else asm volatile("" : "+v"(acc[c][t]));
+      }
   }
 };
+
+// Tiles of 256 or of 128.  Time of a round of tiles in steps of the large tile: its K / 64 and 4 for the epilogue; a round
+// of the small ones (two per CU) takes 0.61 of that, half a round (one per CU) 0.36: measured at 2 016 to 104 100 rows, 1024 to
+// 4096 channels; the choice is the faster one at all of them.
+inline bool large_tiles(int64_t M, int N) {
+  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256), small = ((M + 127) / 128) * ((N + 127) / 128);
+  const double t_big = (double)((big + 255) / 256);
+  const double t_small = small <= 256 ? 0.36 : 0.61 * (double)((small + 511) / 512);
+  return t_big <= t_small;
+}
 
 }  // namespace lin
 }  // namespace s3r

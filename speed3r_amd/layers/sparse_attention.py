@@ -43,15 +43,32 @@ def takes_kernels(x: Tensor) -> bool:
         and torch.autograd.forward_ad._current_level < 0 and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
 
 
+def linear_takes(m: nn.Linear, x: Tensor) -> bool:
+    """Whether a kernel may stand in for ``m(x)``: an ordinary call for inference of a module that would run
+    ``nn.Linear.forward`` and nothing else, on enough rows."""
+    return takes_kernels(x) and calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter and x.shape[-1] == m.weight.shape[1] \
+        and ops.linear_pays(x.numel() // max(x.shape[-1], 1), *m.weight.shape) \
+        and not (torch.is_grad_enabled() and (x.requires_grad or m.weight.requires_grad or (m.bias is not None and m.bias.requires_grad)))
+
+
 def linear(m: nn.Linear, x: Tensor, gelu: bool = False) -> Tensor:
-    """``m(x)``, with ``gelu`` followed by ``F.gelu``: for inference one kernel where calling ``m`` would run
-    ``nn.Linear.forward`` and nothing else, the modules otherwise."""
-    if takes_kernels(x) and calls_forward_only(m, nn.Linear) and ops.linear_pays(x.numel() // x.shape[-1], *m.weight.shape) and type(m.weight) is nn.Parameter \
-            and not (torch.is_grad_enabled() and (x.requires_grad or m.weight.requires_grad or (m.bias is not None and m.bias.requires_grad))):
+    """``m(x)``, with ``gelu`` followed by ``F.gelu``: one kernel where :func:`linear_takes` says so, else the modules."""
+    if linear_takes(m, x):
         out = ops.linear(x, m.weight, m.bias, gelu)
         if out is not None:
             return out
     return nn.functional.gelu(m(x)) if gelu else m(x)
+
+
+def project(attn: nn.Module, x: Tensor, pos: Optional[Tensor], n_pos: Optional[int], block: int, pooled: bool):
+    """The projection of an attention layer with all that follows it row by row (``ops.qkv_project``), or None where the
+    kernel does not take the layer or does not stand in for its modules (then: ``linear`` and the passes over its result)."""
+    if pos is None or not linear_takes(attn.qkv, x) or pos.is_floating_point():
+        return None
+    fused = fused_qk_args(attn, x, pos, n_pos, takes=x.dim() == 3 and x.shape[-1] == 64 * attn.num_heads)
+    if fused is None or fused[0].shape != (*x.shape[:2], 2):
+        return None
+    return ops.qkv_project(x, attn.qkv.weight, attn.qkv.bias, attn.num_heads, block, *fused[:3], *fused[4:], pooled=pooled, inv_freq=fused[3])
 
 
 def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
@@ -79,16 +96,20 @@ def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Ten
     return rope(t, pos) if pos is not None else t
 
 
-def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Optional[int] = None, training: bool = False):
+def fused_qk_args(attn: nn.Module, qkv: Tensor, pos: Optional[Tensor], n_pos: Optional[int] = None, training: bool = False,
+                  takes: Optional[bool] = None):
     """``(pos, cos, sin, inv_freq, q_ln, k_ln, eps)`` for the kernels that take qk-norm and RoPE with the packed
     projection, or None where their conditions do not hold (those of ``norm_rope_fused_or_eager`` for both norms).
+    ``takes``: whether the kernel takes ``qkv`` (default: a packed projection, ``ops.prepass_takes``).
     ``training``: in the place of the modules' own calls, which know no bound of the positions and must do nothing else."""
     def plain(norm):
         if training and not (calls_forward_only(norm, nn.Identity) or calls_forward_only(norm, nn.LayerNorm)):
             return False
         return isinstance(norm, nn.Identity) or (type(norm) is nn.LayerNorm and norm.elementwise_affine)
     same_kind = isinstance(attn.q_norm, nn.Identity) == isinstance(attn.k_norm, nn.Identity)
-    if not (qkv.is_cuda and ops.prepass_takes(qkv, attn.num_heads) and plain(attn.q_norm) and plain(attn.k_norm) and same_kind
+    if takes is None:
+        takes = qkv.is_cuda and ops.prepass_takes(qkv, attn.num_heads)
+    if not (takes and plain(attn.q_norm) and plain(attn.k_norm) and same_kind
             and (pos is None or (calls_forward_only(attn.rope, RoPE2D) if training else isinstance(attn.rope, RoPE2D)))):
         return None
     if training and pos is not None:   # (a rope module takes one set of positions for all sequences, fractional ones, and more)
@@ -237,20 +258,24 @@ class SparseFlashAttentionRope(nn.Module):
         d = c // h
         block = self.block_size ** 2
 
-        qkv = linear(self.qkv, x)                                      # [B, N, 3C], layout (qkv h d)
-        gate = self._gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)      # [B, H, N, 2], strided view
-
         use_pos = xpos is not None and self.rope is not None
         pos = xpos if use_pos else None
-        # One pass over the packed projection: block means of the raw q, k, v, normalised and rotated at the block
+        # The projection and all that follows it row by row in one kernel, where that takes the layer.  Else one pass over the
+        # packed projection: block means of the raw q, k, v, normalised and rotated at the block
         # positions (compressed branch), and norm + RoPE of the full-token q and k (selection branch), each input row read
         # once.  Where that kernel is not built (head_dim other than 64, another norm or rope module): pooling kernel, then
         # norm/RoPE per tensor.  16-token blocks take the pass in two launches: the block means first, so that the index
         # kernel, long for so many pooled tokens, starts while the full tokens are still to come.
-        fused = fused_qk_args(self, qkv, pos, n_pos)
-        q = k = v = None
+        q = k = v = fused = qkv = None
         self.last_prepass, self.last_passes = False, 0
-        if fused is not None and (pos is not None or fused[4] is not None):   # (else q and k are read in place)
+        projected = project(self, x, pos, n_pos, block, True)
+        if projected is None:
+            qkv = linear(self.qkv, x)                                  # [B, N, 3C], layout (qkv h d)
+            fused = fused_qk_args(self, qkv, pos, n_pos)
+        if projected is not None:
+            q, k, v, q_c, k_c, v_c = projected
+            self.last_prepass, self.last_passes = True, 1
+        elif fused is not None and (pos is not None or fused[4] is not None):   # (else q and k are read in place)
             args = (pos, fused[1], fused[2], *fused[4:])
             self.last_prepass = block >= 32
             self.last_passes = 1 if self.last_prepass else 2
@@ -271,6 +296,7 @@ class SparseFlashAttentionRope(nn.Module):
             o_c, _ = ops.compressed_attn_topk(q_c, k_c, v_c, None)
         else:
             o_c, idx = flash_attn_topk_func(q_c, k_c, v_c, self.topk)
+        gate = self._gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)      # [B, H, N, 2], strided view
 
         if q is None and fused is not None and (pos is not None or fused[4] is not None):
             q, k, v = ops.qkv_prepass(qkv, h, 64, *args, pooled=None, inv_freq=fused[3])

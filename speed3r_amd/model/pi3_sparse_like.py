@@ -37,7 +37,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from ..layers import RoPE2D, SparseFlashAttentionRope
-from ..layers.sparse_attention import calls_forward_only, fused_qk_args, linear, norm_rope_fused_or_eager
+from ..layers.sparse_attention import calls_forward_only, fused_qk_args, linear, norm_rope_fused_or_eager, project
 from ..sparse_attn import ops
 from .token_order import tile_major, tile_major_inverse
 
@@ -106,14 +106,15 @@ class DenseAttentionRope(nn.Module):
     def forward(self, x: Tensor, attn_bias=None, xpos: Optional[Tensor] = None, n_pos: Optional[int] = None) -> Tensor:
         b, n, c = x.shape
         h = self.num_heads
-        qkv = linear(self.qkv, x)
         pos = xpos if self.rope is not None else None
-        fused = fused_qk_args(self, qkv, pos, n_pos) if not torch.is_grad_enabled() else None
-        qkv_out = None
-        if fused is not None and (pos is not None or fused[4] is not None):   # one pass over the projection for q and k
-            qkv_out = ops.qkv_prepass(qkv, h, 64, *fused[:3], *fused[4:], pooled=None, inv_freq=fused[3])
-        if qkv_out is not None:
-            q, k, v = qkv_out
+        projected = project(self, x, pos, n_pos, 64, False) if not torch.is_grad_enabled() else None
+        if projected is None:
+            qkv = linear(self.qkv, x)
+            fused = fused_qk_args(self, qkv, pos, n_pos) if not torch.is_grad_enabled() else None
+            if fused is not None and (pos is not None or fused[4] is not None):   # one pass over the projection for q and k
+                projected = ops.qkv_prepass(qkv, h, 64, *fused[:3], *fused[4:], pooled=None, inv_freq=fused[3])
+        if projected is not None:
+            q, k, v = projected
         else:
             q, k, v = qkv.view(b, n, 3, h, c // h).permute(2, 0, 3, 1, 4).unbind(0)
             q, k = self._norm_rope(q, self.q_norm, pos, n_pos), self._norm_rope(k, self.k_norm, pos, n_pos)

@@ -504,6 +504,43 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     return out
 
 
+def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], num_heads: int, block: int, positions: torch.Tensor,
+                cos_tab: torch.Tensor, sin_tab: torch.Tensor, q_ln=None, k_ln=None, eps: float = 1e-5, *, pooled: bool,
+                inv_freq: Optional[torch.Tensor] = None):
+    """:func:`linear` with the weights of the packed projection and :func:`qkv_prepass` of its result (``pooled``: with
+    ``pooled="final"``, else without means) in one kernel: ``(q, k, v[, q_c, k_c, v_c])``, all contiguous.  The projection is
+    rounded, then once at the end (the pass rounds after the norm and inside the rotation too).
+
+    Returns None where the library has no kernel: bf16/fp16, head_dim 64, an even number of heads, contiguous 16-byte
+    aligned tensors of one dtype; means with norms and over blocks of 16 or 64 tokens only; several sequences of 256 tokens or
+    more each, with means a multiple of the block."""
+    _need_device(x)
+    _forward_only(x, weight)
+    b, n, c = x.shape
+    h = num_heads
+    ts = [t for t in (x, weight, bias) if t is not None]
+    if x.dtype not in (torch.bfloat16, torch.float16) or c != 64 * h or h % 2 or c > 1 << 18 or x.numel() == 0 or b * n > 1 << 30 \
+            or weight.shape != (3 * c, c) or (bias is not None and bias.shape != (3 * c,)):
+        return None
+    if any(t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
+        return None
+    if pooled and (q_ln is None or block not in (16, 64)) or b > 1 and (n < 256 or h * n * 128 > 0x70000000 or pooled and n % block):
+        return None
+    a, keep = _prepass_args(x, h, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq)
+    q, k, v = x.new_empty((3, b, h, n, 64)).unbind(0)
+    a.q_out, a.k_out = q.data_ptr(), k.data_ptr()
+    means = ()
+    if pooled:
+        means = x.new_empty((3, b, h, -(-n // block), 64)).unbind(0)
+        a.q_pool, a.k_pool, a.v_pool = (t.data_ptr() for t in means)
+        a.finish_pooled = True
+    with _on(x.device):
+        rc = _lib.lib().s3r_qkv_project(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, c, c, v.data_ptr(),
+                                        ctypes.byref(a), _stream(x))
+    _lib.check(rc, "s3r_qkv_project")
+    return (q, k, v, *means)
+
+
 def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """``sigmoid(F.linear(x, weight, bias))`` for the few outputs of the layer's gate, in one pass over ``x`` (inference).
 
