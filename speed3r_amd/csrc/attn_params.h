@@ -39,6 +39,9 @@ int launch_attn_simple(const AttnParams& p, int dtype, bool select, void* stream
 int launch_attn_f32(const AttnParams& p, bool select, void* stream);  // fp32, head_dim 64, blocks of 16, 32 or 64 tokens
 int launch_select_pipe(const AttnParams& p, int dtype, void* stream);
 int launch_select_b16(const AttnParams& p, int dtype, void* stream);  // block 16
+constexpr int64_t kMostKeys = 1216;
+bool topk_lds_pays(const AttnParams& p);  // top-k indices alone: at most kMostKeys keys, and not too many rows
+int launch_topk_lds(const AttnParams& p, int dtype, void* stream);
 int launch_compressed_mfma(const AttnParams& p, int dtype, void* stream);
 
 }  // namespace s3r

@@ -723,6 +723,7 @@ int launch_compressed_mfma(const AttnParams& p, int dtype, void* stream) {
     }
     if (rc != S3R_OK) return rc;
   }
+  if (p.topk_idx != nullptr && topk_lds_pays(p)) return launch_topk_lds(p, dtype, stream);
   if (p.topk_idx != nullptr) return dtype == S3R_BF16 ? cmp::launch_e<bf16_t>(p, true, st) : cmp::launch_e<f16_t>(p, true, st);
   return S3R_OK;
 }

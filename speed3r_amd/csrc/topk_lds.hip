@@ -1,0 +1,268 @@
+// Exact top-k block indices of the compressed branch for up to 2496 pooled keys (flash_attention_topk.py:101-157): the scores
+// of 16 query rows against all keys stay in LDS, and a row is selected by one wave that sees all of it.
+//
+// The two-sweep kernel (compressed_mfma.hip) meets at a barrier per 64 keys and folds queues of survivors into register lists;
+// with few tiles its chains of barriers, LDS round trips and folds are all there is (63 tiles, top-32: 124 us, 2 % of the
+// matrix rate).  Here:
+//   * Scores: S^T = K Q^T with v_mfma_f32_32x32x16 as there, same operands in the same order, so the scores are the same bits.  A
+//     workgroup has 16 rows, so half of the 32 query columns repeat the other half: the products are a fiftieth of the work.  The
+//     eight waves share the key tiles; operands come straight from memory (each is used once per workgroup), four tiles in
+//     flight per wave.
+//   * Selection: a wave reads a row, 4 neighbouring columns per lane and 256-column piece, into registers.  The K-th largest of
+//     256 group maxima (a lane's four columns modulo 4: neighbours in different groups, since large scores come in runs) is a
+//     lower bound of the row's K-th largest score; the search for it looks at the upper 24 bits of the sortable pattern only (its result may only be lower).  Scores at or above it, K to 1.4 K of them as a
+//     rule, are gathered in the row's own LDS space, one per lane, and ranked by counting: lane l compares its key with every
+//     other one.  No chain of exchanges, no sort.
+//   * More than 64 candidates (ties; a row of equal scores): K times the largest key below the last one, from the registers.
+// Order, fillers and NaN as in the two-sweep kernel: descending (sortable score, lowest column first), NaN never chosen, Lk - 1
+// in slots that nothing fills.
+//
+// us on the device, two-sweep kernel / this, 16 heads, as many rows as keys: 126 keys, top-32 16 / 8; 504, top-32 40 / 13; 1 041,
+// top-16 46 / 35; 1 200, top-32 66 / 39.  Bound: the vector instructions of the selection, about 700 per row at 1 041 keys.
+//
+// Up to kMostKeys keys two workgroups fit a CU (78 KB each).  With more keys one does, and the two phases have nobody to hide
+// behind: 2 016 keys, top-32, 95 / 112.  With more than kMostGroups workgroups the two-sweep kernel, which shares its key tiles
+// among more rows, is no longer bound by latency: 24 heads of 1 041 47 / 48, 32 of them 53 / 58, 48 of 756 44 / 46.
+#include "select_common.h"
+#include "attn_params.h"
+
+namespace s3r {
+namespace tkl {
+using namespace sel;
+
+constexpr int kRows = 16, kWaves = 8;
+
+__device__ __forceinline__ float sortable_to_float(uint32_t k) {  // the inverse of sortable_key
+  return __uint_as_float(k ^ ((k & 0x80000000u) ? 0x80000000u : 0xFFFFFFFFu));
+}
+
+template <typename E, int NC>  // NC: pieces of 256 columns
+__global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, int groups, int total) {
+  typedef typename Mma<E>::V8 V8;
+  // rows of the scores, 4 mod 64 values apart: what 16 lanes on 16 rows touch lies in different banks
+  constexpr int stride = (NC == 5 ? (int)kMostKeys : 256 * NC) + 4;
+  __shared__ __attribute__((aligned(16))) float sc[kRows * stride];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int hh = lane >> 5, c = lane & 31;
+  // the row groups of a head run on one XCD, whose L2 then holds its keys
+  const int xcd = blockIdx.x & 7, per = total >> 3, rem = total & 7;
+  const int vid = xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  const int bh = vid / groups, g = vid - bh * groups;
+  const int b = bh / p.H, h = bh - b * p.H;
+  const int Lk = (int)p.Lk, q0 = g * kRows;
+  const int rows = (int)p.Lq - q0 < kRows ? (int)p.Lq - q0 : kRows;
+  const E* const kp = (const E*)p.k + (int64_t)b * p.skb + (int64_t)h * p.skh;
+
+  // ---- scores ----
+  {
+    const int qr = (c & 15) < rows ? (c & 15) : rows - 1;
+    const E* const qp = (const E*)p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh + (int64_t)(q0 + qr) * p.sqm + hh * 8;
+    Frag qf[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) qf[ks].u = *reinterpret_cast<const uint4*>(qp + ks * 16);
+    const int tiles = (Lk + 31) >> 5;
+    // The keys come with lane-linear loads, all of a wave's tiles on their way at once (lane = key takes the address unit 64
+    // cycles per instruction instead of 18), and go through LDS into operand order: 16 keys of 128 bytes fit the columns that a
+    // tile's scores will take, so a tile's keys use its own columns and the wave's next ones.
+    const int lr = lane >> 3, lc = lane & 7;
+    u32x4 kv[NC][4];
+#pragma unroll
+    for (int u = 0; u < NC; u++)
+      if (wave + u * kWaves < tiles) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int key = (wave + u * kWaves) * 32 + 8 * i + lr;
+          kv[u][i] = *reinterpret_cast<const u32x4*>(kp + (int64_t)(key < Lk ? key : Lk - 1) * p.skn + lc * 8);
+        }
+      }
+    constexpr int held = (stride - 4) >> 5;  // tiles that the score rows have columns for
+#pragma unroll
+    for (int u = 0; u < NC; u++) {
+      const int t = wave + u * kWaves;
+      if (t < tiles) {
+        char* const own = reinterpret_cast<char*>(sc + t * 32);
+        char* const put = own + lr * stride * 4 + lc * 16;
+        const char* const get = own + (c & 15) * stride * 4 + hh * 16;
+        u32x4 kf[4];
+        *reinterpret_cast<u32x4*>(put) = kv[u][0];
+        *reinterpret_cast<u32x4*>(put + 8 * stride * 4) = kv[u][1];
+        if (t + kWaves < held) {
+          *reinterpret_cast<u32x4*>(put + kWaves * 128) = kv[u][2];
+          *reinterpret_cast<u32x4*>(put + kWaves * 128 + 8 * stride * 4) = kv[u][3];
+#pragma unroll
+          for (int ks = 0; ks < 4; ks++) kf[ks] = *reinterpret_cast<const u32x4*>(get + (c < 16 ? 0 : kWaves * 128) + ks * 32);
+        } else {  // the wave's last tile: its own columns twice
+          u32x4 lo[4];
+#pragma unroll
+          for (int ks = 0; ks < 4; ks++) lo[ks] = *reinterpret_cast<const u32x4*>(get + ks * 32);
+          *reinterpret_cast<u32x4*>(put) = kv[u][2];
+          *reinterpret_cast<u32x4*>(put + 8 * stride * 4) = kv[u][3];
+#pragma unroll
+          for (int ks = 0; ks < 4; ks++) {
+            const u32x4 hi = *reinterpret_cast<const u32x4*>(get + ks * 32);
+            kf[ks] = c < 16 ? lo[ks] : hi;
+          }
+        }
+        f32x16 acc;
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[r] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) acc = Mma<E>::mma(__builtin_bit_cast(V8, kf[ks]), as_v8<E>(qf[ks]), acc);
+        if (c < kRows) {
+          float* const dst = sc + c * stride + t * 32 + 4 * hh;  // rows 8 j + 4 hh + i of the tile
+#pragma unroll
+          for (int j = 0; j < 4; j++) *reinterpret_cast<float4*>(dst + 8 * j) = make_float4(acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]);
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- selection ----
+  const int K = p.K;
+  constexpr int G = 4;               // groups of scores per lane: neighbouring columns in different ones
+  constexpr int R = kRows / kWaves;  // rows of a wave, side by side: each hides the other's waits
+  float v[R][NC][4];
+  float* row[R];
+  uint32_t t[R];
+  uint32_t gk[R][G];  // largest score of a group, sortable
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int q = wave * R + r;
+    row[r] = sc + (q < rows ? q : rows - 1) * stride;  // (rows behind the last one repeat it and store nothing)
+    float mx[G];
+#pragma unroll
+    for (int e = 0; e < G; e++) mx[e] = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const int col = (i * 64 + lane) * 4;
+      const float4 x = *reinterpret_cast<const float4*>(row[r] + (col < Lk ? col : 0));
+      v[r][i][0] = x.x; v[r][i][1] = x.y; v[r][i][2] = x.z; v[r][i][3] = x.w;
+      if (i * 256 + 256 > Lk) {  // beyond the keys: NaN, which no comparison lets pass
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[r][i][e] = col + e < Lk ? v[r][i][e] : __uint_as_float(0x7fc00000u);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) mx[e % G] = fmaxf(mx[e % G], v[r][i][e]);  // (passes over NaN)
+    }
+#pragma unroll
+    for (int e = 0; e < G; e++) gk[r][e] = sortable_key(mx[e]);
+    t[r] = 0;
+  }
+#pragma unroll
+  for (int bit = 31; bit >= 8; bit--)
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const uint32_t cand = t[r] | (1u << bit);
+      int cnt = 0;
+#pragma unroll
+      for (int e = 0; e < G; e++) cnt += (int)__popcll(__ballot(gk[r][e] >= cand));
+      t[r] = cnt >= K ? cand : t[r];
+    }
+  // candidates, packed to the front of the row's space (its scores are in registers): pattern and column
+  float bound[R];
+  int mine[R], n[R];  // where a lane's first one goes; the number of all
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    bound[r] = t[r] <= 0x007FFFFFu ? -INFINITY : sortable_to_float(t[r]);  // (below the pattern of -inf lie NaNs)
+    mine[r] = 0;
+#pragma unroll
+    for (int i = 0; i < NC; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) mine[r] += v[r][i][e] >= bound[r] ? 1 : 0;
+    int s = mine[r];  // inclusive sum over the lanes below: rows of 16, then across them
+#define S3R_STEP(ctrl, rows_on) s += __builtin_amdgcn_update_dpp(0, s, ctrl, rows_on, 0xF, false)
+    S3R_STEP(0x111, 0xF);  // row_shr:1
+    S3R_STEP(0x112, 0xF);  // row_shr:2
+    S3R_STEP(0x114, 0xF);  // row_shr:4
+    S3R_STEP(0x118, 0xF);  // row_shr:8
+    S3R_STEP(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+    S3R_STEP(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+#undef S3R_STEP
+    n[r] = __builtin_amdgcn_readlane(s, 63);
+    mine[r] = s - mine[r];
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (n[r] <= 64 && wave * R + r < rows) {
+      uint2* at = reinterpret_cast<uint2*>(row[r]) + mine[r];
+#pragma unroll
+      for (int i = 0; i < NC; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (v[r][i][e] >= bound[r]) *at++ = make_uint2(__float_as_uint(v[r][i][e]), (uint32_t)((i * 64 + lane) * 4 + e));
+    }
+  uint64_t key[R];
+  uint32_t col[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {  // one candidate per lane, as a key, back to where the others read it
+    const uint2 x = reinterpret_cast<const uint2*>(row[r])[lane < n[r] ? lane : 0];
+    col[r] = x.y;
+    key[r] = lane < n[r] ? ((uint64_t)sortable_key(__uint_as_float(x.x)) << 32) | ((uint32_t)(Lk - 1) - x.y) : 0;
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (n[r] <= 64 && wave * R + r < rows) reinterpret_cast<uint64_t*>(row[r])[lane] = key[r];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if (wave * R + r >= rows) break;
+    int32_t* const out = p.topk_idx + ((int64_t)bh * p.Lq + q0 + wave * R + r) * K;
+    if (n[r] <= 64) {
+      int rank = 0;
+      for (int j = 0; j < n[r]; j += 8) {  // (keys behind the last one are 0: above nothing)
+        const ulonglong2* const o = reinterpret_cast<const ulonglong2*>(row[r]) + j / 2;
+        ulonglong2 w[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) w[u] = o[u];
+#pragma unroll
+        for (int u = 0; u < 4; u++) rank += (w[u].x > key[r] ? 1 : 0) + (w[u].y > key[r] ? 1 : 0);
+      }
+      if (lane < n[r] && rank < K) out[rank] = (int32_t)col[r];
+      if (lane >= n[r] && lane < K) out[lane] = Lk - 1;
+    } else {
+      uint64_t last = ~0ull;
+#pragma unroll 1
+      for (int k = 0; k < K; k++) {
+        uint64_t best = 0;
+#pragma unroll
+        for (int i = 0; i < NC; i++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const uint64_t x = ((uint64_t)sortable_key(v[r][i][e]) << 32) | (uint32_t)(Lk - 1 - ((i * 64 + lane) * 4 + e));
+            best = v[r][i][e] >= bound[r] && x < last && x > best ? x : best;
+          }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const uint64_t other = ((uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)(best >> 32), off) << 32) | (uint32_t)__shfl_xor((int)(uint32_t)best, off);
+          best = other > best ? other : best;
+        }
+        last = best;
+        if (lane == 0) out[k] = Lk - 1 - (int)(uint32_t)best;
+      }
+    }
+  }
+}
+
+template <typename E> static int launch(const AttnParams& p, hipStream_t st) {
+  const int64_t groups = (p.Lq + kRows - 1) / kRows, total = groups * p.B * p.H;
+#define S3R_TKL(NC) hipLaunchKernelGGL((topk_lds_kernel<E, NC>), dim3((unsigned)total), dim3(64 * kWaves), 0, st, p, (int)groups, (int)total)
+  if (p.Lk <= 256) S3R_TKL(1);
+  else if (p.Lk <= 512) S3R_TKL(2);
+  else if (p.Lk <= 768) S3R_TKL(3);
+  else if (p.Lk <= 1024) S3R_TKL(4);
+  else S3R_TKL(5);
+#undef S3R_TKL
+  return check_launch("topk_lds_kernel");
+}
+
+}  // namespace tkl
+
+constexpr int64_t kMostGroups = 1536;
+
+bool topk_lds_pays(const AttnParams& p) { return p.Lk <= kMostKeys && (p.Lq + tkl::kRows - 1) / tkl::kRows * p.B * p.H <= kMostGroups; }
+
+int launch_topk_lds(const AttnParams& p, int dtype, void* stream) {
+  return dtype == S3R_BF16 ? tkl::launch<bf16_t>(p, (hipStream_t)stream) : tkl::launch<f16_t>(p, (hipStream_t)stream);
+}
+
+}  // namespace s3r
