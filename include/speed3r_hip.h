@@ -316,10 +316,13 @@ int s3r_linear(const void* x, const void* w, const void* bias, void* y, int64_t 
  *   a: as for s3r_layer_prepass (q, k, v and the strides are not read): q_out, k_out, positions and tables are required,
  *   the three means and the norms optional; means only with norms, `finish_pooled` and without q_raw, k_raw.
  * bf16 / fp16, an even number of heads, block 16 or 64; several sequences: 256 tokens or more each, with means a multiple of
- * the block.  Rounding: the projection to the I/O dtype, then once at the end (s3r_layer_prepass also rounds in between).
+ * the block.  gate_out (or NULL): [B*N, gate_outputs], what s3r_gate gives for x, gate_w ([gate_outputs, C]) and gate_bias (or
+ * NULL); a multiple of 4 outputs up to 32.  Rounding: the projection to the I/O dtype, then once at the end (s3r_layer_prepass also rounds in between).
  */
 int s3r_qkv_project(const void* x, const void* w, const void* bias, int64_t ldx, int64_t ldw, void* v_out, const struct s3r_prepass_args* a,
-                    void* stream);
+                    const void* gate_w, const void* gate_bias, void* gate_out, int gate_outputs, void* stream);
+/* Whether s3r_qkv_project computes the gate of `rows` = B*N rows and H heads in time that it leaves idle (else s3r_gate is as good). */
+int s3r_qkv_project_gate_rides(int64_t rows, int H);
 
 /*
  * The layer's gate  out[r,:] = sigmoid(x[r,:] W^T + bias)  (pi3/models/layers/sparse_attention.py:88,127); fp32 sums, the

@@ -7,6 +7,8 @@
 // The accumulator layout suits it: a lane holds 4 consecutive channels of one token in each of the head's
 // four 16 x 16 tiles, so the row sums of the norm take two exchanges per 16 values, the rotation partner (16 channels away)
 // sits in the same lane, and 16 tokens' sums for the means are one reduction over 16 lanes.
+// The layer's gate, sigmoid(x W^T + b) with 2 outputs per head (sparse_attention.py:88,127), is 32 more columns: thin tiles for the
+// workgroups that the last round of tiles leaves idle.
 // us, library product + pass / this: 104 100 tokens (64-token blocks) 610 + 207 / 697, 32 256 (16-token blocks) 165 + 81 / 222,
 // 8 x 1 008 without means 57 + 20 / 57, 2 016 (16-token blocks) 21 + 23 / 28.
 //
@@ -34,6 +36,9 @@ struct ProjectParams {
   const float* inv_freq;
   const void* ln[4];  // q norm weight, bias, k norm weight, bias
   float eps;
+  const void *gate_w, *gate_b;  // optional: gate_out [M, O] = sigmoid(x gate_w^T + gate_b)
+  void* gate_out;
+  int O;
 };
 
 // (cos, sin) pairs of the I/O type, 16 frequencies per position; chunk of 4 frequencies c of row r at c ^ ((r >> 2) & 3), so
@@ -82,9 +87,9 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
   __shared__ __attribute__((aligned(16))) int lfar[2][4];  // per wave: a position it handed out lies outside of the staged rows
   __shared__ __attribute__((aligned(16))) E lbias[2][BN];  // the bias of its channels
   TileWalk walk(p.mt, p.nt);
-  if (walk.at >= walk.count) return;
-  Tl tl;
   const int tid = threadIdx.x;
+  if (walk.at < walk.count) {
+  Tl tl;
   for (int i = tid; i < p.staged_rows * 16; i += 256)
     ltab[table_at(i >> 4, (i & 15) >> 2) + (i & 3)] = pack_pair<E>(((const E*)p.cos_tab)[i], ((const E*)p.sin_tab)[i]);
   if constexpr (NORM) {
@@ -377,8 +382,51 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
     walk.locate(walk.at, m, n);
     tl.read_first(lx0, lw0);  // (the last step has read it too: 64 registers that the epilogue needs more)
   }
+  }
   __builtin_amdgcn_s_waitcnt(0x0070);  // no transfer may still write LDS when the wave ends
+  if (p.gate_out == nullptr) return;
+
+  // ---- the gate: tiles of BM tokens x 32 outputs, for the workgroups that have one tile less than others (gate_rides) ----
+  typedef Tile<E, T, 1> Gt;
+  const int xcd = blockIdx.x & 7;
+  const int from = (int)((int64_t)p.mt * xcd / 8), thin = (int)((int64_t)p.mt * (xcd + 1) / 8) - from;
+  const int full = walk.count % walk.slots, idle = walk.slots - full;
+  Gt gt;
+  for (int i = (int)(blockIdx.x >> 3) - full; i >= 0 && i < thin; i += idle) {
+    const int r0 = (from + i) * BM, rows = p.M - r0 < BM ? p.M - r0 : BM;
+    __syncthreads();  // every wave is done with the LDS buffers
+    gt.aim((const E*)p.x + r0 * p.ldx, p.ldx, rows, (const E*)p.gate_w, p.K, p.O);
+#pragma unroll
+    for (int t = 0; t < Gt::NL; t++) gt.move(lx0, lw0, 0, t);
+#pragma unroll
+    for (int t = 0; t < Gt::NL; t++) gt.move(lx1, lw1, 128, t);
+    gt.begin(lx0, lw0);
+    gt.clear();
+    gt.before_products();
+    const int last = p.K * 2 - 128;
+    for (int kb = 256; kb < p.K * 2 + 256; kb += 256) {  // (beyond the end the last step is requested again)
+      gt.step(lx0, lw0, lx1, lw1, kb < last ? kb : last);
+      gt.step(lx1, lw1, lx0, lw0, kb + 128 < last ? kb + 128 : last);
+    }
+    gt.after_products();
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the requests beyond the end have landed
+    const int o = gt.wn * 16 + 4 * gt.g4;
+    if (o < p.O) {
+      float bias[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) bias[e] = p.gate_b != nullptr ? (float)((const E*)p.gate_b)[o + e] : 0.f;
+#pragma unroll
+      for (int t = 0; t < T; t++) {
+        const int row = gt.wm * WROWS + t * 16 + gt.c16;
+        union { E e[4]; uint2 u; } g;  // rounding points of the two modules: the product with its bias, then the sigmoid
+#pragma unroll
+        for (int e = 0; e < 4; e++) g.e[e] = (E)(1.f / (1.f + expf(-round_to<E>(gt.acc[0][t][e] + bias[e]))));
+        if (row < rows) *reinterpret_cast<uint2*>((E*)p.gate_out + (int64_t)(r0 + row) * p.O + o) = g.u;
+      }
+    }
+  }
 }
+
 
 // Norm and rotation of the block means in place, at the truncated mean positions of their blocks: 8 lanes a row, 8 rows a wave,
 // q and k; the pass's functions and rounding points.  The selection ranks products of these: other roundings are other
@@ -433,14 +481,33 @@ template <typename E> static void launch_finish(const s3r_prepass_args& a, int64
   hipLaunchKernelGGL((finish_means_kernel<E>), dim3((unsigned)((2 * groups + 3) / 4)), dim3(256), (unsigned)staged_bytes(0, true), st, p, Nc, groups);
 }
 
+// a wave of the large tile holds two heads: both of q, of k or of v
+static bool large_project(int64_t M, int C) { return C % 128 == 0 && large_tiles(M, 3 * C); }
+
+// Whether the gate costs nothing beside the projection: every XCD has two workgroups without a tile in the last round for each three
+// of its thin tiles.  One takes half the time of a tile (short steps: it waits for its rows at each); more of them, or any on
+// workgroups with a tile of their own, prolong the kernel, while the gate's own kernel can run beside the index kernel
+// (layer, us, apart / here: 25 212 tokens 379 / 358, 2 016 131 / 124; 104 100, two per workgroup, 1 547 / 1 555, 32 256, four, 665 / 690).
+static bool gate_rides(int64_t M, int C) {
+  const bool large = large_project(M, C);
+  const int b = large ? 256 : 128, most = large ? 256 : 512;
+  const int64_t mt = (M + b - 1) / b, tiles = mt * ((3 * C + b - 1) / b);
+  if (tiles + mt <= most) return true;  // (as many workgroups as tiles of both kinds)
+  for (int xcd = 0; xcd < 8; xcd++) {
+    const int64_t count = tiles / 8 + (xcd < tiles % 8 ? 1 : 0), thin = mt * (xcd + 1) / 8 - mt * xcd / 8;
+    if (2 * thin > 3 * (most / 8 - count % (most / 8))) return false;
+  }
+  return true;
+}
+
 template <typename E, bool NORM, int POOL> static void launch_project(ProjectParams& p, hipStream_t st) {
-  // a wave of the large tile holds two heads: both of q, of k or of v
-  const bool large = p.C % 128 == 0 && large_tiles(p.M, 3 * p.C);
+  const bool large = large_project(p.M, p.C);
   const int b = large ? 256 : 128;
   p.mt = (p.M + b - 1) / b;
   p.nt = (3 * p.C + b - 1) / b;
-  const int64_t tiles = (int64_t)p.mt * p.nt, most = large ? 256 : 512;
-  const dim3 grid((unsigned)(tiles < most ? tiles : most)), blk(256);
+  const int64_t tiles = (int64_t)p.mt * p.nt + (p.gate_out != nullptr ? p.mt : 0), most = large ? 256 : 512;
+  // (gate: every XCD, which has its share of the thin tiles, needs a workgroup)
+  const dim3 grid((unsigned)(tiles >= most ? most : p.gate_out != nullptr && tiles < 8 ? 8 : tiles)), blk(256);
   if (large) hipLaunchKernelGGL((project_kernel<E, 8, NORM, POOL, 1>), grid, blk, 0, st, p);
   else hipLaunchKernelGGL((project_kernel<E, 4, NORM, POOL, 2>), grid, blk, 0, st, p);
 }
@@ -457,8 +524,10 @@ template <typename E> static void launch_project(ProjectParams& p, int pool, hip
 
 using namespace s3r;
 
+extern "C" int s3r_qkv_project_gate_rides(int64_t rows, int H) { return rows > 0 && H > 0 && H <= (1 << 20) / 192 && rows <= (1 << 30) && lin::gate_rides(rows, 64 * H); }
+
 extern "C" int s3r_qkv_project(const void* x, const void* w, const void* bias, int64_t ldx, int64_t ldw, void* v_out, const s3r_prepass_args* a,
-                               void* stream) {
+                               const void* gate_w, const void* gate_bias, void* gate_out, int gate_outputs, void* stream) {
   if (!a || !x || !w || !v_out || !a->q_out || !a->k_out || !a->positions || !a->cos_table || !a->sin_table)
     return fail(S3R_ERR_BAD_ARG, "s3r_qkv_project: null pointer");
   if (a->B <= 0 || a->H <= 0 || a->N <= 0 || a->table_rows <= 0) return fail(S3R_ERR_BAD_ARG, "s3r_qkv_project: non-positive size");
@@ -484,7 +553,15 @@ extern "C" int s3r_qkv_project(const void* x, const void* w, const void* bias, i
     if (!aligned16(ptr)) return fail(S3R_ERR_BAD_ARG, "s3r_qkv_project: pointers must be multiples of 16 bytes");
   if (ldx % 8 || ldw % 8 || (reinterpret_cast<uintptr_t>(bias) & 7u))
     return fail(S3R_ERR_BAD_ARG, "s3r_qkv_project: rows must be multiples of 16 bytes, the bias of 8");
+  if (gate_out != nullptr) {
+    if (!gate_w) return fail(S3R_ERR_BAD_ARG, "s3r_qkv_project: null pointer");
+    if (gate_outputs <= 0 || gate_outputs > 32 || gate_outputs % 4)
+      return fail(S3R_ERR_UNSUPPORTED, "s3r_qkv_project: %d gate outputs (built for a multiple of 4 up to 32)", gate_outputs);
+    if (!aligned16(gate_w) || (reinterpret_cast<uintptr_t>(gate_out) & 7u))
+      return fail(S3R_ERR_BAD_ARG, "s3r_qkv_project: the gate's weight must be a multiple of 16 bytes, its output of 8");
+  }
   lin::ProjectParams p = {};
+  p.gate_w = gate_w; p.gate_b = gate_bias; p.gate_out = gate_out; p.O = gate_outputs;
   p.x = x; p.w = w; p.bias = bias; p.ldx = ldx; p.ldw = ldw;
   p.M = (int)M; p.N = (int)a->N; p.K = C; p.C = C; p.H = a->H; p.Nc = pool ? (int)((a->N + a->block - 1) / a->block) : 0;
   p.q = a->q_out; p.k = a->k_out; p.v = v_out; p.qc = a->q_pool; p.kc = a->k_pool; p.vc = a->v_pool;

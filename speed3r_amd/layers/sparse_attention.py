@@ -60,15 +60,17 @@ def linear(m: nn.Linear, x: Tensor, gelu: bool = False) -> Tensor:
     return nn.functional.gelu(m(x)) if gelu else m(x)
 
 
-def project(attn: nn.Module, x: Tensor, pos: Optional[Tensor], n_pos: Optional[int], block: int, pooled: bool):
-    """The projection of an attention layer with all that follows it row by row (``ops.qkv_project``), or None where the
-    kernel does not take the layer or does not stand in for its modules (then: ``linear`` and the passes over its result)."""
+def project(attn: nn.Module, x: Tensor, pos: Optional[Tensor], n_pos: Optional[int], block: int, pooled: bool, gate=None):
+    """The projection of an attention layer with all that follows it row by row, and the layer's gate (weight, bias) beside it
+    (``ops.qkv_project``), or None where the kernel does not take the layer or does not stand in for its modules (then:
+    ``linear`` and the passes over its result)."""
     if pos is None or not linear_takes(attn.qkv, x) or pos.is_floating_point():
         return None
     fused = fused_qk_args(attn, x, pos, n_pos, takes=x.dim() == 3 and x.shape[-1] == 64 * attn.num_heads)
     if fused is None or fused[0].shape != (*x.shape[:2], 2):
         return None
-    return ops.qkv_project(x, attn.qkv.weight, attn.qkv.bias, attn.num_heads, block, *fused[:3], *fused[4:], pooled=pooled, inv_freq=fused[3])
+    return ops.qkv_project(x, attn.qkv.weight, attn.qkv.bias, attn.num_heads, block, *fused[:3], *fused[4:], pooled=pooled, inv_freq=fused[3],
+                           gate=gate)
 
 
 def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
@@ -174,11 +176,14 @@ class SparseFlashAttentionRope(nn.Module):
     def _norm_rope(self, t: Tensor, norm: nn.Module, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
         return norm_rope_fused_or_eager(t, norm, self.rope, pos, n_pos)
 
+    def _plain_gate(self) -> bool:
+        """Whether the gate is the plain pair of modules it was built as, whose calls run nothing but their ``forward``."""
+        return calls_forward_only(self.gate, nn.Sequential) and len(self.gate) == 2 and calls_forward_only(self.gate[0], nn.Linear) \
+            and calls_forward_only(self.gate[1], nn.Sigmoid)
+
     def _gate(self, x: Tensor) -> Tensor:
-        """``self.gate(x)`` for inference: one kernel where it is the plain pair of modules it was built as, whose calls run
-        nothing but their ``forward``, and outside of autocast."""
-        if x.is_cuda and calls_forward_only(self.gate, nn.Sequential) and len(self.gate) == 2 and calls_forward_only(self.gate[0], nn.Linear) \
-                and calls_forward_only(self.gate[1], nn.Sigmoid) and not torch.is_autocast_enabled("cuda"):
+        """``self.gate(x)`` for inference: one kernel where it is plain, and outside of autocast."""
+        if x.is_cuda and self._plain_gate() and not torch.is_autocast_enabled("cuda"):
             out = ops.gate(x, self.gate[0].weight, self.gate[0].bias)
             if out is not None:
                 return out
@@ -268,12 +273,14 @@ class SparseFlashAttentionRope(nn.Module):
         # kernel, long for so many pooled tokens, starts while the full tokens are still to come.
         q = k = v = fused = qkv = None
         self.last_prepass, self.last_passes = False, 0
-        projected = project(self, x, pos, n_pos, block, True)
+        gate = None
+        projected = project(self, x, pos, n_pos, block, True, (self.gate[0].weight, self.gate[0].bias) if self._plain_gate() else None)
         if projected is None:
             qkv = linear(self.qkv, x)                                  # [B, N, 3C], layout (qkv h d)
             fused = fused_qk_args(self, qkv, pos, n_pos)
         if projected is not None:
-            q, k, v, q_c, k_c, v_c = projected
+            q, k, v, q_c, k_c, v_c = projected[:6]
+            gate = projected[6] if len(projected) > 6 else None
             self.last_prepass, self.last_passes = True, 1
         elif fused is not None and (pos is not None or fused[4] is not None):   # (else q and k are read in place)
             args = (pos, fused[1], fused[2], *fused[4:])
@@ -296,7 +303,7 @@ class SparseFlashAttentionRope(nn.Module):
             o_c, _ = ops.compressed_attn_topk(q_c, k_c, v_c, None)
         else:
             o_c, idx = flash_attn_topk_func(q_c, k_c, v_c, self.topk)
-        gate = self._gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)      # [B, H, N, 2], strided view
+        gate = (self._gate(x) if gate is None else gate).view(b, n, h, 2).permute(0, 2, 1, 3)   # [B, H, N, 2], strided view
 
         if q is None and fused is not None and (pos is not None or fused[4] is not None):
             q, k, v = ops.qkv_prepass(qkv, h, 64, *args, pooled=None, inv_freq=fused[3])

@@ -506,10 +506,12 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
 
 def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], num_heads: int, block: int, positions: torch.Tensor,
                 cos_tab: torch.Tensor, sin_tab: torch.Tensor, q_ln=None, k_ln=None, eps: float = 1e-5, *, pooled: bool,
-                inv_freq: Optional[torch.Tensor] = None):
+                inv_freq: Optional[torch.Tensor] = None, gate: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None):
     """:func:`linear` with the weights of the packed projection and :func:`qkv_prepass` of its result (``pooled``: with
-    ``pooled="final"``, else without means) in one kernel: ``(q, k, v[, q_c, k_c, v_c])``, all contiguous.  The projection is
-    rounded, then once at the end (the pass rounds after the norm and inside the rotation too).
+    ``pooled="final"``, else without means) in one kernel: ``(q, k, v[, q_c, k_c, v_c][, gates])``, all contiguous.  The projection
+    is rounded, then once at the end (the pass rounds after the norm and inside the rotation too).  ``gate``: (weight, bias) of
+    :func:`gate`, whose result ``[B,N,O]`` is then the last one, or None where its outputs are not a multiple of 4 up to 32 or
+    the kernel has no idle time for it.
 
     Returns None where the library has no kernel: bf16/fp16, head_dim 64, an even number of heads, contiguous 16-byte
     aligned tensors of one dtype; means with norms and over blocks of 16 or 64 tokens only; several sequences of 256 tokens or
@@ -534,11 +536,20 @@ def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
         means = x.new_empty((3, b, h, -(-n // block), 64)).unbind(0)
         a.q_pool, a.k_pool, a.v_pool = (t.data_ptr() for t in means)
         a.finish_pooled = True
+    gates, gate_args = (), (None, None, None, 0)
+    if gate is not None:
+        gw, gb = gate
+        gts = [t for t in gate if t is not None]
+        takes = _lib.lib().s3r_qkv_project_gate_rides(b * n, h) and gw.shape[0] % 4 == 0 and gw.shape[0] <= 32 and gw.shape[1:] == (c,) and (gb is None or gb.shape == gw.shape[:1]) \
+            and all(t.dtype == x.dtype and t.device == x.device and t.is_contiguous() for t in gts) and gw.data_ptr() % 16 == 0
+        gates = (x.new_empty((b, n, gw.shape[0])) if takes else None,)
+        if takes:
+            gate_args = (gw.data_ptr(), gb.data_ptr() if gb is not None else None, gates[0].data_ptr(), gw.shape[0])
     with _on(x.device):
         rc = _lib.lib().s3r_qkv_project(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, c, c, v.data_ptr(),
-                                        ctypes.byref(a), _stream(x))
+                                        ctypes.byref(a), *gate_args, _stream(x))
     _lib.check(rc, "s3r_qkv_project")
-    return (q, k, v, *means)
+    return (q, k, v, *means, *gates)
 
 
 def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:

@@ -4,6 +4,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from speed3r_amd import _lib
 from speed3r_amd.layers import RoPE2D
 from speed3r_amd.sparse_attn import ops
 
@@ -103,6 +104,32 @@ def test_project_without_means_or_norm_and_at_far_positions(n):
                     g, e = g.float(), e.float()
                     assert ((g - e).abs() <= 2.0 ** -8 * (4 * 1.42 * e.abs().amax(-1, keepdim=True) + 2 * e.abs())).all()
                     assert (g - e).norm() <= 4e-3 * e.norm()
+
+
+# thin tiles of the gate: fewer tiles than XCDs, as many workgroups as tiles, a last round of tiles with idle workgroups, of the
+# large and of the small tile
+@pytest.mark.parametrize("n,h", [(1, 2), (130, 2), (2016, 16), (25212, 16), (65536, 2), (30000, 6), (21600, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_project_with_the_gate(n, h, dtype):
+    x, w, bias, pos, ln = _case(1, n, h, dtype, seed=n)
+    c = 64 * h
+    gw, gb = (torch.randn(2 * h, c, device=DEV) / c ** 0.5).to(dtype), torch.randn(2 * h, device=DEV).to(dtype)
+    cos, sin = RoPE2D(100.0).tables(64, 40, x.device, dtype)
+    plain = ops.qkv_project(x, w, bias, h, 64, pos, cos, sin, *ln, 1e-6, pooled=True)
+    step = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    rides = bool(_lib.lib().s3r_qkv_project_gate_rides(n, h))
+    assert rides or n == 21600
+    for b in (gb, None):
+        got = ops.qkv_project(x, w, bias, h, 64, pos, cos, sin, *ln, 1e-6, pooled=True, gate=(gw, b))
+        assert (got[6] is not None) == rides
+        if not rides:
+            continue
+        assert all(torch.equal(a, e) for a, e in zip(got, plain))
+        z = x.double() @ gw.double().t() + (b.double() if b is not None else 0)
+        # half a step of the product (a whole one where fp32 sums round it the other way) through a slope of at most 1/4,
+        # half a step of the result
+        assert ((got[6].double() - z.sigmoid()).abs() <= step * (2 * z.abs() * 0.25 + z.sigmoid()) + 1e-6).all()
+    assert ops.qkv_project(x, w, bias, h, 64, pos, cos, sin, *ln, 1e-6, pooled=True, gate=(gw[:3], None))[6] is None
 
 
 def test_project_keeps_infinities_to_their_rows_and_blocks():
