@@ -310,6 +310,17 @@ int s3r_linear(const void* x, const void* w, const void* bias, void* y, int64_t 
                int activation, int dtype, void* stream);
 
 /*
+ * Gradients of a linear layer's parameters over many rows:  dw = dy^T x [N, C],  db = the sums of dy over the rows [N], or NULL;
+ * fp32 sums, one rounding, the same bits for the same inputs.
+ *   dy: [M, N], x: [M, C] with row strides lddy, ldx (elements); dw, db contiguous; workspace: as many floats as
+ *   s3r_linear_wgrad_workspace says; bf16 / fp16, N and C multiples of 8, C > 768 with db; dy, x, dw, the workspace and the rows of
+ *   dy and x multiples of 16 bytes.
+ */
+int64_t s3r_linear_wgrad_workspace(int64_t M, int N, int C, int64_t lddy, int64_t ldx);
+int s3r_linear_wgrad(const void* dy, const void* x, void* dw, void* db, float* workspace, int64_t M, int N, int C, int64_t lddy, int64_t ldx,
+                     int dtype, void* stream);
+
+/*
  * s3r_linear and s3r_layer_prepass in one: the layer's projection  [q | k | v] = x W^T + bias  and, of it,
  * q and k after LayerNorm and RoPE2D, v, and the finished block means (sparse_attention.py:93-110,115-124).
  *   x: [B*N, C] rows of stride ldx, w: [3*C, C] of stride ldw, bias: [3*C] or NULL, C = 64 H; v_out: contiguous [B,H,N,64];

@@ -37,10 +37,8 @@ def calls_forward_only(m: nn.Module, kind: type) -> bool:
 
 
 def takes_kernels(x: Tensor) -> bool:
-    """Whether a call on ``x`` is an ordinary one: a tensor on the GPU, without autocast, tracing, compilation or a transform
-    (vmap, forward-mode derivatives) that has to see the torch operations."""
-    return x.is_cuda and type(x) is Tensor and not torch.is_autocast_enabled("cuda") and torch._C._functorch.peek_interpreter_stack() is None \
-        and torch.autograd.forward_ad._current_level < 0 and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+    """Whether a call on ``x`` is an ordinary one (:func:`ops.ordinary`), without autocast."""
+    return not torch.is_autocast_enabled("cuda") and ops.ordinary(x)
 
 
 def linear_takes(m: nn.Linear, x: Tensor) -> bool:
@@ -51,8 +49,23 @@ def linear_takes(m: nn.Linear, x: Tensor) -> bool:
         and not (torch.is_grad_enabled() and (x.requires_grad or m.weight.requires_grad or (m.bias is not None and m.bias.requires_grad)))
 
 
+def linear_trains(m: nn.Linear, x: Tensor) -> bool:
+    """Whether ``ops.linear_autograd`` may stand in for ``m(x)``: an ordinary call, with or without autocast, in a 16-bit type, of
+    a module that would run ``nn.Linear.forward`` and nothing else, on so many rows that the kernel for the weight's gradient
+    is the faster one."""
+    dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
+    return torch.is_grad_enabled() and calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter and m.weight.requires_grad \
+        and dtype in (torch.bfloat16, torch.float16) and x.shape[-1] == m.weight.shape[1] and ops.ordinary(x) \
+        and all(t is None or t.dtype in (torch.float32, torch.bfloat16, torch.float16) for t in (x, m.weight, m.bias)) \
+        and ops.linear_wgrad_pays(x.numel() // max(x.shape[-1], 1))
+
+
 def linear(m: nn.Linear, x: Tensor, gelu: bool = False) -> Tensor:
-    """``m(x)``, with ``gelu`` followed by ``F.gelu``: one kernel where :func:`linear_takes` says so, else the modules."""
+    """``m(x)``, with ``gelu`` followed by ``F.gelu``: one kernel where :func:`linear_takes` says so, the product with a kernel for
+    the parameters' gradients where :func:`linear_trains` does, else the modules."""
+    if linear_trains(m, x):
+        out = ops.linear_autograd(x, m.weight, m.bias)
+        return nn.functional.gelu(out) if gelu else out
     if linear_takes(m, x):
         out = ops.linear(x, m.weight, m.bias, gelu)
         if out is not None:
@@ -199,8 +212,12 @@ class SparseFlashAttentionRope(nn.Module):
         b, n, c = x.shape
         h = self.num_heads
         block = self.block_size ** 2
-        qkv = self.qkv(x)
-        gate = self.gate(x).view(b, n, h, 2).permute(0, 2, 1, 3)              # [B, H, N, 2]
+        plain_gate = self._plain_gate()
+        if plain_gate and linear_trains(self.qkv, x) and linear_trains(self.gate[0], x):
+            x = ops.autocast_once(x)
+        qkv = linear(self.qkv, x)
+        gate = torch.sigmoid(linear(self.gate[0], x)) if plain_gate else self.gate(x)
+        gate = gate.view(b, n, h, 2).permute(0, 2, 1, 3)                      # [B, H, N, 2]
         use_pos = xpos is not None and self.rope is not None
         fused = fused_qk_args(self, qkv, xpos if use_pos else None, n_pos, training=True)
         branches = None
@@ -212,12 +229,12 @@ class SparseFlashAttentionRope(nn.Module):
                 if self.keep_topk_idx:
                     self.last_topk_idx = idx
                 if len(branches) == 1:
-                    return self.proj_drop(self.proj(branches[0]))
+                    return self.proj_drop(linear(self.proj, branches[0]))
         o_c, o_s = branches if branches is not None else self._branches_with_grad(qkv, xpos if use_pos else None)
         blk = torch.arange(n, device=x.device) // block
         out = gate[..., 0:1] * o_c[:, :, blk] + gate[..., 1:2] * o_s           # [B, H, N, D]
         out = out.permute(0, 2, 1, 3).reshape(b, n, c)
-        return self.proj_drop(self.proj(out))
+        return self.proj_drop(linear(self.proj, out))
 
     def _branches_with_grad(self, qkv: Tensor, xpos: Optional[Tensor]):
         """Outputs of the two attention branches as a composition of torch expressions around the attention operators."""

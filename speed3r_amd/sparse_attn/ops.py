@@ -504,6 +504,88 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     return out
 
 
+def ordinary(x: torch.Tensor) -> bool:
+    """Whether a call on ``x`` is an ordinary one: a tensor on the GPU, without tracing, compilation or a transform (vmap,
+    forward-mode derivatives) that has to see the torch operations."""
+    return x.is_cuda and type(x) is torch.Tensor and torch._C._functorch.peek_interpreter_stack() is None \
+        and torch._C._has_storage(x) and torch.autograd.forward_ad._current_level < 0 \
+        and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+
+
+# Gradients of weight and bias, kernel / library, us on the device: 2 048 rows x 3072 x 1024 36 / 43, x 1024 x 1024 29 / 33 (no
+# faster with their launches), 4 096 rows 42 / 61 and 32 / 48, 24 192 rows 130 / 279 and 62 / 206.
+def linear_wgrad_pays(rows: int) -> bool:
+    return rows >= 4096
+
+
+class _LinearFn(torch.autograd.Function):
+    """``F.linear`` whose parameters' gradients come from :func:`linear_wgrad`; keeps what ``F.linear`` keeps."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias):
+        ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, weight if ctx.needs_input_grad[0] else None)
+        return torch.nn.functional.linear(x, weight, bias)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        dx = dw = db = None
+        dy2 = dy.reshape(-1, dy.shape[-1])
+        if ctx.needs_input_grad[0]:
+            dx = (dy2 @ weight).view(*dy.shape[:-1], weight.shape[1])
+        if ctx.needs_input_grad[1] and not torch.is_grad_enabled() and ordinary(dy):   # (a derivative of the backward itself: torch's)
+            got = linear_wgrad(dy2, x.reshape(-1, x.shape[-1]), ctx.needs_input_grad[2])
+            if got is not None:
+                return dx, *got
+        if ctx.needs_input_grad[1]:
+            dw = dy2.t() @ x.reshape(-1, x.shape[-1])
+        if ctx.needs_input_grad[2]:
+            db = dy2.sum(0)
+        return dx, dw, db
+
+
+def autocast_once(x: torch.Tensor) -> torch.Tensor:
+    """``x`` as autocast hands it to several products: one copy in its dtype where it keeps the copy (of a leaf that wants a
+    gradient) or no gradient tells one copy from several."""
+    if torch.is_autocast_enabled("cuda") and x.dtype == torch.float32 and (
+            not x.requires_grad or (x.is_leaf and not x._is_view() and torch.is_autocast_cache_enabled())):
+        return x.to(torch.get_autocast_dtype("cuda"))
+    return x
+
+
+def linear_autograd(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    """``F.linear(x, weight, bias)`` with autocast's casts, differentiable, with the parameters' gradients from one kernel."""
+    if torch.is_autocast_enabled("cuda"):
+        dtype = torch.get_autocast_dtype("cuda")
+        x, weight, bias = (t if t is None else t.to(dtype) for t in (x, weight, bias))
+    return _LinearFn.apply(x, weight, bias)
+
+
+def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, bias: bool):
+    """``(dy^T x, dy.sum(0) or None)`` of dy ``[M,N]`` and x ``[M,C]``: gradients of a linear layer's parameters, summed in fp32.
+
+    Returns None where the library has no kernel (bf16/fp16, N and C multiples of 8, with the bias C > 768, rows of
+    adjacent values, 16-byte aligned)."""
+    (m, n), c = dy.shape, x.shape[1]
+    if dy.dtype not in (torch.bfloat16, torch.float16) or x.dtype != dy.dtype or x.device != dy.device or x.shape[0] != m or n % 8 or c % 8 \
+            or m == 0 or n * c == 0 or (bias and c <= 768) or max(n, c) > 1 << 20:
+        return None
+    for t in (dy, x):
+        if t.stride(1) != 1 or t.stride(0) % 8 or not t.shape[1] <= t.stride(0) < 1 << 21 or t.data_ptr() % 16:
+            return None
+    ld = max(dy.stride(0), x.stride(0))
+    if m > 64 * (0x7f000000 // (2 * ld) - 128):
+        return None
+    dw, db = dy.new_empty((n, c)), dy.new_empty((n,)) if bias else None
+    with _on(dy.device):
+        lib = _lib.lib()
+        ws = torch.empty((lib.s3r_linear_wgrad_workspace(m, n, c, dy.stride(0), x.stride(0)),), dtype=torch.float32, device=dy.device)
+        rc = lib.s3r_linear_wgrad(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), db.data_ptr() if bias else None, ws.data_ptr(), m, n, c,
+                                  dy.stride(0), x.stride(0), _code(dy), _stream(dy))
+    _lib.check(rc, "s3r_linear_wgrad")
+    return dw, db
+
+
 def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], num_heads: int, block: int, positions: torch.Tensor,
                 cos_tab: torch.Tensor, sin_tab: torch.Tensor, q_ln=None, k_ln=None, eps: float = 1e-5, *, pooled: bool,
                 inv_freq: Optional[torch.Tensor] = None, gate: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None):

@@ -1,0 +1,113 @@
+"""Gradients of linear layers' parameters (``s3r_linear_wgrad``) against float64 at the edges of their tiles and ranges of tokens, and
+the calls that keep torch's own graph."""
+import pytest
+import torch
+import torch.nn.functional as F
+from torch import nn
+
+from speed3r_amd.layers.sparse_attention import linear, linear_trains
+from speed3r_amd.sparse_attn import ops
+
+DEV = "cuda"
+ROWS = 4096   # the fewest that the layers hand to the kernel
+
+
+def test_function_has_the_gradients_of_linear():
+    x, w, b = (torch.randn(s, dtype=torch.float64, requires_grad=True) for s in ((2, 3, 4), (5, 4), (5,)))
+    assert torch.equal(ops._LinearFn.apply(x, w, b), F.linear(x, w, b))
+    assert torch.autograd.gradcheck(ops._LinearFn.apply, (x, w, b), check_batched_grad=True)
+    assert torch.autograd.gradgradcheck(ops._LinearFn.apply, (x, w, b))
+    assert torch.autograd.gradcheck(lambda w: ops._LinearFn.apply(x.detach(), w, None), (w,))
+    assert torch.autograd.gradcheck(lambda x, b: ops._LinearFn.apply(x, w.detach(), b), (x, b))
+
+
+# rows below, at and beyond the pairs of steps; outputs and inputs around 16, 128 and 256; one range of tokens, and many
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,c", [(1, 8, 8), (127, 32, 1024), (128, 256, 256), (385, 264, 776), (1000, 32, 1024), (4097, 1032, 1032), (9000, 136, 520), (20161, 3072, 1024)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wgrad_matches_float64(m, n, c, dtype):
+    gen = torch.Generator(device=DEV).manual_seed(m + n)
+    dy = torch.randn(m, n + 8, generator=gen, device=DEV).to(dtype)[:, :n]   # (rows of their own strides)
+    x = torch.randn(m, c + 16, generator=gen, device=DEV).to(dtype)[:, 8:8 + c]
+    bias = c > 768
+    dw, db = ops.linear_wgrad(dy, x, bias)
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11   # half a step of the type, relative to the value
+    for got, a, b in ((dw, dy, x), (db, dy, torch.ones_like(x[:, :1]))) if bias else ((dw, dy, x),):
+        want = a.double().t() @ b.double()
+        room = (a.double().abs().t() @ b.double().abs()) * m * 2.0 ** -24   # a rounding of the sum of magnitudes per token
+        assert got.dtype == dtype and got.is_contiguous()
+        assert ((got.double() - want.view_as(got)).abs() <= half * want.abs().view_as(got) * (1 + half) + room.view_as(got) + 2.0 ** -25).all()
+    assert torch.equal(dw, ops.linear_wgrad(dy, x, bias)[0])
+
+
+@pytest.mark.gpu
+def test_wgrad_refuses_what_it_is_not_built_for():
+    x, dy = torch.randn(256, 512, device=DEV).bfloat16(), torch.randn(256, 64, device=DEV).bfloat16()
+    assert ops.linear_wgrad(dy, x, True) is None                       # sums of dY with few inputs
+    assert ops.linear_wgrad(dy[:, :60], x, False) is None and ops.linear_wgrad(dy[:, 4:12], x, False) is None
+    assert ops.linear_wgrad(dy.float(), x.float(), False) is None and ops.linear_wgrad(dy, x.half(), False) is None
+    assert ops.linear_wgrad(dy, x.t().contiguous().t(), False) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("autocast", [False, True])
+def test_layers_train_through_the_kernel(autocast):
+    master = torch.float32 if autocast else torch.bfloat16
+    m = nn.Linear(1024, 32, device=DEV, dtype=master)
+    x = torch.randn(2, ROWS // 2 + 3, 1024, device=DEV, dtype=master, requires_grad=True)
+    wrt = (x, m.weight, m.bias)
+    dy = torch.randn(*x.shape[:2], 32, device=DEV).bfloat16()
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        assert linear_trains(m, x)
+        got, want = linear(m, x), m(x)
+    assert torch.equal(got, want) and type(got.grad_fn).__name__ == "_LinearFnBackward"
+    a, b = (torch.autograd.grad(t, wrt, dy, retain_graph=True) for t in (got, want))
+    assert torch.equal(a[0], b[0])
+    for g, w, mag in zip(a[1:], b[1:], (dy.double().abs().flatten(0, 1).t() @ x.double().abs().flatten(0, 1), dy.double().abs().sum((0, 1)))):
+        assert g.dtype == w.dtype == master
+        # both within half a bf16 step of the value, and each within one fp32 rounding per token of the sum of magnitudes
+        assert ((g.double() - w.double()).abs() <= 2.0 ** -7 * w.double().abs() + 2 * mag * x.shape[1] * 2 * 2.0 ** -24).all()
+    second = torch.autograd.grad(got.float().square().sum(), m.weight, create_graph=True)[0]
+    assert torch.autograd.grad(second.float().sum(), x)[0].shape == x.shape
+
+
+@pytest.mark.gpu
+def test_other_calls_keep_their_graph():
+    x = torch.randn(ROWS, 256, device=DEV, dtype=torch.bfloat16)
+    m = nn.Linear(256, 128, device=DEV, dtype=torch.bfloat16)
+    assert linear_trains(m, x) and not linear_trains(m, x[1:]) and not linear_trains(m, x.cpu())
+    with torch.no_grad():
+        assert not linear_trains(m, x)
+    assert torch.func.vmap(lambda t: torch.tensor(linear_trains(m, t)))(x[None]).logical_not().all()
+    seen = []
+
+    class Probe(torch.autograd.Function):   # what a backward is given where several gradients come at once
+        forward = staticmethod(lambda ctx, t: t.clone())
+        backward = staticmethod(lambda ctx, g: (seen.append(ops.ordinary(g)), g)[1])
+
+    leaf = x.float().requires_grad_()
+    torch.autograd.grad(Probe.apply(leaf), leaf, torch.ones(2, ROWS, 256, device=DEV), is_grads_batched=True)
+    assert seen == [False]
+    with torch.autograd.forward_ad.dual_level():
+        assert not linear_trains(m, torch.autograd.forward_ad.make_dual(x, x))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not linear_trains(m, x.double())
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(DEV)):
+        out = linear(m, x)
+    out.sum().backward()
+    assert m.weight.grad.shape == m.weight.shape
+    m.register_full_backward_hook(lambda *a: None)
+    assert not linear_trains(m, x)
+
+
+@pytest.mark.gpu
+def test_autocast_makes_one_copy_where_it_keeps_it():
+    x = torch.randn(8, 8, device=DEV)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert ops.autocast_once(x).dtype == torch.bfloat16
+        x.requires_grad_()
+        assert ops.autocast_once(x).dtype == torch.bfloat16
+        assert ops.autocast_once(x * 1.0).dtype == torch.float32   # two copies, whose gradients meet in fp32
+    with torch.autocast("cuda", dtype=torch.bfloat16, cache_enabled=False):
+        assert ops.autocast_once(x).dtype == torch.float32
+    assert ops.autocast_once(x) is x
