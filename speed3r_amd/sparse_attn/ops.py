@@ -475,11 +475,11 @@ def add_layer_norm(x: torch.Tensor, a: torch.Tensor, gamma: Optional[torch.Tenso
     return s, y
 
 
-# Where the layers leave a product to the library (us on the device, library / kernel): few rows, a handful of tiles
-# (256 x 1024 x 1024 5.5 / 8.7, 1 041 x 1024 x 1024 9.0 / 9.2, 2 016 x 1024 x 1024 10.4 / 9.7), and a long K with fewer tiles than
-# CUs, which the library splits (2 016 x 1024 x 4096 28 / 40, 4 032 x 1024 x 4096 43.5 / 43.7).
+# Where the layers leave a product to the library (us on the device, library / kernel): a long K with fewer tiles than CUs, which
+# the library splits (2 016 x 1024 x 4096 28 / 40, 4 032 x 1024 x 4096 43.5 / 43.7).  Few rows are no faster here on the device
+# (256 x 1024 x 1024 5.5 / 8.7, 1 041 9.0 / 9.2, 2 016 10.4 / 9.7) but on the host, which they wait for.
 def linear_pays(rows: int, n: int, k: int) -> bool:
-    return rows >= 1024 and (k <= 1024 or -(-rows // 128) * -(-n // 128) >= 256)
+    return k <= 1024 or -(-rows // 128) * -(-n // 128) >= 256
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], gelu: bool = False) -> Optional[torch.Tensor]:
