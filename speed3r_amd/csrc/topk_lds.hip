@@ -1,4 +1,4 @@
-// Exact top-k block indices of the compressed branch for up to 2496 pooled keys (flash_attention_topk.py:101-157): the scores
+// Exact top-k block indices of the compressed branch for up to 1216 pooled keys (flash_attention_topk.py:101-157): the scores
 // of 16 query rows against all keys stay in LDS, and a row is selected by one wave that sees all of it.
 //
 // The two-sweep kernel (compressed_mfma.hip) meets at a barrier per 64 keys and folds queues of survivors into register lists;

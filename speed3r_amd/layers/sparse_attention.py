@@ -5,12 +5,14 @@ Same constructor arguments, same parameter names (``qkv``, ``proj``, ``q_norm``,
 same ``forward(x, attn_bias=None, xpos=None)``, so a reference checkpoint loads with ``load_state_dict``.
 Differences, all on the host side of the operator boundary:
 
-* q, k, v are handed to the kernels as strided views of the packed projection (no ``.contiguous()`` copies),
-  pooling reads the packed projection directly, and the gated merge runs in the selection kernel's epilogue
-  (or in its own kernel where that is not built), writing ``[B, N, C]`` for ``proj``;
+* for inference the projection, qk-norm, RoPE and the block means are one kernel (:func:`project`) and ``proj`` is another
+  (:func:`linear`); where these are not built or do not pay, q, k, v are strided views of the packed projection (no
+  ``.contiguous()`` copies), which one pass reads directly;
+* the gated merge runs in the selection kernel's epilogue (or in its own kernel where that is not built), writing
+  ``[B, N, C]`` for ``proj``;
 * when a gradient is wanted (grad mode on and the input or a parameter requires grad) the layer runs as projections
   around one differentiable operator with a backward of kernels (bf16/fp16, head_dim 64, blocks of 64 or 16 tokens; see
-  ``_forward_with_grad`` for the rest);
+  ``_forward_with_grad`` for the rest), the gradients of the projections' parameters by a kernel of their own;
 * ``N`` need not be a multiple of the block: the last block pools its valid tokens, its keys beyond ``N`` are
   masked and its query rows beyond ``N`` do not exist (the reference raises for such ``N``);
 * the top-k count, 32 in the reference, is a constructor argument.
