@@ -61,13 +61,17 @@ def linear_trains(m: nn.Linear, x: Tensor) -> bool:
     """Whether ``ops.linear_autograd`` may stand in for ``m(x)``: an ordinary call, with or without autocast, in a 16-bit type, of
     a module that would run ``nn.Linear.forward`` and nothing else, on so many rows that the kernel for the weight's gradient
     is the faster one."""
-    if not torch.is_grad_enabled():
+    if not torch.is_grad_enabled() or not ops.linear_wgrad_pays(x.numel() // max(x.shape[-1], 1)):   # (first: few rows wait for the host)
         return False
     dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
     return calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter and m.weight.requires_grad \
         and dtype in (torch.bfloat16, torch.float16) and x.shape[-1] == m.weight.shape[1] and ops.ordinary(x) \
-        and all(t is None or t.dtype in (torch.float32, torch.bfloat16, torch.float16) for t in (x, m.weight, m.bias)) \
-        and ops.linear_wgrad_pays(x.numel() // max(x.shape[-1], 1))
+        and all(t is None or t.dtype in (torch.float32, torch.bfloat16, torch.float16) for t in (x, m.weight, m.bias))
+
+
+def linear_with_grad(m: nn.Linear, x: Tensor) -> Tensor:
+    """``m(x)`` in training: with a kernel for the parameters' gradients where :func:`linear_trains` says so."""
+    return ops.linear_autograd(x, m.weight, m.bias) if linear_trains(m, x) else m(x)
 
 
 def linear(m: nn.Linear, x: Tensor, gelu: bool = False) -> Tensor:
@@ -222,11 +226,12 @@ class SparseFlashAttentionRope(nn.Module):
         b, n, c = x.shape
         h = self.num_heads
         block = self.block_size ** 2
-        plain_gate = self._plain_gate()
-        if plain_gate and linear_trains(self.qkv, x) and linear_trains(self.gate[0], x):
+        if linear_trains(self.qkv, x) and self._plain_gate() and linear_trains(self.gate[0], x):
             x = ops.autocast_once(x)
-        qkv = linear(self.qkv, x)
-        gate = torch.sigmoid(linear(self.gate[0], x)) if plain_gate else self.gate(x)
+            qkv = ops.linear_autograd(x, self.qkv.weight, self.qkv.bias)
+            gate = torch.sigmoid(ops.linear_autograd(x, self.gate[0].weight, self.gate[0].bias))
+        else:
+            qkv, gate = linear_with_grad(self.qkv, x), self.gate(x)
         gate = gate.view(b, n, h, 2).permute(0, 2, 1, 3)                      # [B, H, N, 2]
         use_pos = xpos is not None and self.rope is not None
         fused = fused_qk_args(self, qkv, xpos if use_pos else None, n_pos, training=True)
@@ -239,12 +244,12 @@ class SparseFlashAttentionRope(nn.Module):
                 if self.keep_topk_idx:
                     self.last_topk_idx = idx
                 if len(branches) == 1:
-                    return self.proj_drop(linear(self.proj, branches[0]))
+                    return self.proj_drop(linear_with_grad(self.proj, branches[0]))
         o_c, o_s = branches if branches is not None else self._branches_with_grad(qkv, xpos if use_pos else None)
         blk = torch.arange(n, device=x.device) // block
         out = gate[..., 0:1] * o_c[:, :, blk] + gate[..., 1:2] * o_s           # [B, H, N, D]
         out = out.permute(0, 2, 1, 3).reshape(b, n, c)
-        return self.proj_drop(linear(self.proj, out))
+        return self.proj_drop(linear_with_grad(self.proj, out))
 
     def _branches_with_grad(self, qkv: Tensor, xpos: Optional[Tensor]):
         """Outputs of the two attention branches as a composition of torch expressions around the attention operators."""
