@@ -22,7 +22,9 @@
 //
 // Up to kMostKeys keys two workgroups fit a CU (78 KB each).  With more keys one does, and the two phases have nobody to hide
 // behind: 2 016 keys, top-32, 95 / 112.  With more than kMostGroups workgroups the two-sweep kernel, which shares its key tiles
-// among more rows, is no longer bound by latency: 24 heads of 1 041 47 / 48, 32 of them 53 / 58, 48 of 756 44 / 46.
+// among more rows, is no longer bound by latency: 24 heads of 1 041 47 / 48, 32 of them 53 / 58, 48 of 756 44 / 46.  Up to
+// top-8 its folds are short, and it is as good from fewer keys on (whole operator, us, top-8: 537 keys 182 / 172, 1 009 287 /
+// 286, 1 201 336 / 344; top-4: 537 145 / 142, 814 191 / 192, 1 009 225 / 230; top-1: 537 136 / 119, 814 156 / 163).
 #include "select_common.h"
 #include "attn_params.h"
 
@@ -259,7 +261,9 @@ template <typename E> static int launch(const AttnParams& p, hipStream_t st) {
 
 constexpr int64_t kMostGroups = 1536;
 
-bool topk_lds_pays(const AttnParams& p) { return p.Lk <= kMostKeys && (p.Lq + tkl::kRows - 1) / tkl::kRows * p.B * p.H <= kMostGroups; }
+bool topk_lds_pays(const AttnParams& p) {
+  return p.Lk <= (p.K <= 4 ? 640 : p.K <= 8 ? 1024 : kMostKeys) && (p.Lq + tkl::kRows - 1) / tkl::kRows * p.B * p.H <= kMostGroups;
+}
 
 int launch_topk_lds(const AttnParams& p, int dtype, void* stream) {
   return dtype == S3R_BF16 ? tkl::launch<bf16_t>(p, (hipStream_t)stream) : tkl::launch<f16_t>(p, (hipStream_t)stream);
