@@ -994,16 +994,22 @@ def _two_kernel_compressed(q: torch.Tensor, topk: int, block: int = 1) -> bool:
 
 # Pooled rows (B * H * blocks) from which the index kernel goes on a stream of its own.  The two events and the change of
 # stream cost the host 60 to 80 us and the kernels behind them a wait between queues; what there is to hide is the dense
-# sweep's 12 to 16 us and the norm/RoPE pass.  us per call, two streams / one, 16 heads: layer, two views at 16-token blocks
-# (126 pooled tokens) 259 / 183, eight views (504) 286 / 253, 16 (1 008) 384 / 400, 32 (2 016) 701 / 747; operators, one view
-# (63) 118 / 61, eight (504) 131 / 122, 16 (1 008) 147 / 146; at 64-token blocks 8 frames (130) 127 / 94, 32 (518) 259 / 254.
-SIDE_STREAM_ROWS = 16 * 512
+# sweep's 12 to 16 us.  Up to 1216 pooled tokens (top-8: 1024, top-4 and less: 640) the indices come from the short kernel, which has too
+# little to gain; the line lies there for 16 heads.  us per call, two streams / one, 16 heads: layer at 16-token blocks, 504 pooled tokens 221 / 186, 1 008
+# 335 / 328, 2 016 714 / 721; at 64-token blocks, 394 378 / 365, 814 806 / 802, 1 074 1 054 / 1 047, 1 627 1 570 / 1 592; operators, 504
+# pooled tokens 122 / 95, 1 008 161 / 148, at 64-token blocks 537 227 / 222, 1 041 418 / 413, 1 172 451 / 441, 1 627 612 / 611,
+# 2 082 766 / 778, 4 164 1 532 / 1 551; top-8, 1 188 328 / 331.
+SIDE_STREAM_ROWS = 16 * 1216
+
+
+def _side_stream_rows(topk: int) -> int:
+    return SIDE_STREAM_ROWS if topk > 8 else 16 * (1024 if topk > 4 else 640)
 
 
 def _indices_beside(q: torch.Tensor, topk: int, block: int = 1) -> bool:
     """True where the index kernel runs on the side stream (arguments as for :func:`_two_kernel_compressed`)."""
     rows = q.shape[0] * q.shape[1] * -(-q.shape[2] // block)
-    return rows > SIDE_STREAM_ROWS and _two_kernel_compressed(q, topk, block)
+    return rows > _side_stream_rows(topk) and _two_kernel_compressed(q, topk, block)
 
 
 def topk_indices_on_side_stream(qc: torch.Tensor, kc: torch.Tensor, topk: int, softmax_scale: Optional[float] = None):
