@@ -25,7 +25,8 @@ struct LinearParams {
 
 // x/2 (1 + erf(x / sqrt 2)).  With t = 1 / (1 + p |x| / sqrt 2) the complementary error function is t times a polynomial
 // of degree 4 in t times exp(-x^2 / 2), absolute error 1.5e-7 (Abramowitz and Stegun, 7.1.26); the negative side is taken
-// from the complement itself, so that nothing cancels there.
+// from the complement itself, so that nothing cancels there.  From 16 on the correction is zero: +inf stays itself (and -inf
+// gives NaN, as x/2 (1 + erf) does).
 __device__ __forceinline__ float gelu(float x) {
   const float a = fabsf(x);
   const float t = __builtin_amdgcn_rcpf(fmaf(a, 0.3275911f * 0.70710678f, 1.f));
@@ -34,7 +35,7 @@ __device__ __forceinline__ float gelu(float x) {
   q = fmaf(t, q, 0.5f * 1.421413741f);
   q = fmaf(t, q, 0.5f * -0.284496736f);
   q = fmaf(t, q, 0.5f * 0.254829592f);
-  return fmaf(-a, q * t * e, fmaxf(x, 0.f));
+  return fmaf(-fabsf(fminf(x, 16.f)), q * t * e, fmaxf(x, 0.f));
 }
 
 template <typename E, int T, bool GELU, int WPS>

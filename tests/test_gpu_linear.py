@@ -35,6 +35,15 @@ def test_linear_matches_float64(m, n, k, dtype):
             assert ((got.double() - want).abs() <= bound).all()
 
 
+def test_gelu_of_infinities_and_nan():
+    x, w = torch.ones(6, 128, device=DEV).bfloat16(), torch.ones(8, 128, device=DEV).bfloat16()
+    x[1], x[2, 5], x[3, 5], x[4, 5], x[5] = 3e38, float("inf"), float("-inf"), float("nan"), -3e38   # (rows 1 and 5: infinite sums)
+    want = F.gelu(F.linear(x, w))
+    assert want[1:3].isposinf().all() and want[3:].isnan().all()
+    got = ops.linear(x, w, None, gelu=True)
+    assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isnan(), want.isnan()) and torch.equal(got[0], want[0])
+
+
 def test_linear_writes_inside_its_rows_only():
     x, w = torch.randn(300, 256, device=DEV).bfloat16(), torch.randn(264, 256, device=DEV).bfloat16()
     from speed3r_amd import _lib
