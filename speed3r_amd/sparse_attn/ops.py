@@ -17,6 +17,7 @@ import os
 from typing import Optional, Tuple
 
 import torch
+from torch.utils._device import DeviceContext
 
 from .. import _lib
 
@@ -504,10 +505,17 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     return out
 
 
+def _seen_by_modes() -> bool:
+    """Whether a mode (``make_fx``, flop counters, selective checkpointing, function modes) is to see the torch operations;
+    ``torch.device`` as a context and the default device concern factory functions only."""
+    return torch._C._len_torch_dispatch_stack() > 0 or any(
+        type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+
+
 def ordinary(x: torch.Tensor) -> bool:
-    """Whether a call on ``x`` is an ordinary one: a tensor on the GPU, without tracing, compilation or a transform (vmap,
+    """Whether a call on ``x`` is an ordinary one: a tensor on the GPU, without tracing, compilation, a mode or a transform (vmap,
     forward-mode derivatives) that has to see the torch operations."""
-    return x.is_cuda and type(x) is torch.Tensor and torch._C._functorch.peek_interpreter_stack() is None \
+    return x.is_cuda and not _seen_by_modes() and type(x) is torch.Tensor and torch._C._functorch.peek_interpreter_stack() is None \
         and torch._C._has_storage(x) and torch.autograd.forward_ad._current_level < 0 \
         and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
 
