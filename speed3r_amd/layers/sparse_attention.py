@@ -43,6 +43,11 @@ def takes_kernels(x: Tensor) -> bool:
     return not torch.is_autocast_enabled("cuda") and ops.ordinary(x)
 
 
+def sizes_are_known(x: Tensor) -> bool:
+    """Whether the sizes of ``x`` may choose a path: not where a call is traced, compiled or exported for any sizes."""
+    return type(x) is Tensor and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+
+
 # Calls with less work keep torch's products and the passes over them.  A layer of few rows is bound by the host: 400 to 1 020 tokens of
 # 1024 channels take 162 us with those, 137 with the projection in one launch, 126 with both products here (2 016 tokens: 180 / 126).
 def enough_work(x: Tensor) -> bool:
@@ -52,7 +57,7 @@ def enough_work(x: Tensor) -> bool:
 def linear_takes(m: nn.Linear, x: Tensor) -> bool:
     """Whether a kernel may stand in for ``m(x)``: an ordinary call for inference of a module that would run
     ``nn.Linear.forward`` and nothing else, on enough rows (asked first: few rows wait for the host)."""
-    return enough_work(x) and calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter \
+    return sizes_are_known(x) and enough_work(x) and calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter \
         and x.shape[-1] == m.weight.shape[1] and takes_kernels(x) \
         and not (torch.is_grad_enabled() and (x.requires_grad or m.weight.requires_grad or (m.bias is not None and m.bias.requires_grad)))
 
@@ -61,7 +66,7 @@ def linear_trains(m: nn.Linear, x: Tensor) -> bool:
     """Whether ``ops.linear_autograd`` may stand in for ``m(x)``: an ordinary call, with or without autocast, in a 16-bit type, of
     a module that would run ``nn.Linear.forward`` and nothing else, on so many rows that the kernel for the weight's gradient
     is the faster one."""
-    if not torch.is_grad_enabled() or not ops.linear_wgrad_pays(x.numel() // max(x.shape[-1], 1)):   # (first: few rows wait for the host)
+    if not torch.is_grad_enabled() or not sizes_are_known(x) or not ops.linear_wgrad_pays(x.numel() // max(x.shape[-1], 1)):   # (first: few rows wait for the host)
         return False
     dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
     return calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter and m.weight.requires_grad \

@@ -49,7 +49,10 @@ class Mlp(nn.Module):
         self.fc2 = nn.Linear(hidden, dim)
 
     def forward(self, x: Tensor) -> Tensor:
-        return linear(self.fc2, linear(self.fc1, x, gelu=True))
+        if torch.jit.is_scripting():
+            return self.fc2(F.gelu(self.fc1(x)))
+        else:   # (not compiled by TorchScript)
+            return linear(self.fc2, linear(self.fc1, x, gelu=True))
 
 
 class LayerScale(nn.Module):
