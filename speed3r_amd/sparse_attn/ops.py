@@ -532,7 +532,9 @@ class _LinearFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
         ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, weight if ctx.needs_input_grad[0] else None)
-        return torch.nn.functional.linear(x, weight, bias)
+        out = torch.nn.functional.linear(x, weight, bias)
+        # (of a batch it is a view of the product's rows: views that are made in here may not be changed in place)
+        return torch.ops.aten._unsafe_view(out, out.shape) if out._is_view() else out
 
     @staticmethod
     def backward(ctx, dy):

@@ -21,6 +21,19 @@ def test_function_has_the_gradients_of_linear():
     assert torch.autograd.gradcheck(lambda x, b: ops._LinearFn.apply(x, w.detach(), b), (x, b))
 
 
+@pytest.mark.parametrize("lead", [(6,), (2, 3)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_output_may_be_changed_in_place(lead, bias):
+    x, w, b = (torch.randn(s, requires_grad=True) for s in ((*lead, 4), (5, 4), (5,)))
+    wrt = (x, w, b) if bias else (x, w)
+    got, want = (f(x, w, b if bias else None) for f in (ops.linear_autograd, F.linear))
+    for out in (got, want):
+        out.mul_(2.0)
+        out[..., 1:3].add_(1.0)
+    assert torch.equal(got, want)
+    assert all(torch.equal(g, e) for g, e in zip(torch.autograd.grad(got.sum(), wrt), torch.autograd.grad(want.sum(), wrt)))
+
+
 # rows below, at and beyond the pairs of steps; outputs and inputs around 16, 128 and 256; one range of tokens, and many
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,c", [(1, 8, 8), (127, 32, 1024), (128, 256, 256), (385, 264, 776), (1000, 32, 1024), (4097, 1032, 1032), (9000, 136, 520), (20161, 3072, 1024)])
