@@ -554,20 +554,25 @@ class _LinearFn(torch.autograd.Function):
         return dx, dw, db
 
 
+def _cast(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """``t`` as autocast hands it to a product: the copy that it keeps for a leaf in this region, else a new one.  (Autocast casts
+    the operands of einsum too; of one operand in its own order einsum makes a view.)"""
+    return t if t is None or t.dtype == torch.get_autocast_dtype("cuda") else torch.einsum("...i->...i", t)
+
+
 def autocast_once(x: torch.Tensor) -> torch.Tensor:
     """``x`` as autocast hands it to several products: one copy in its dtype where it keeps the copy (of a leaf that wants a
     gradient) or no gradient tells one copy from several."""
     if torch.is_autocast_enabled("cuda") and x.dtype == torch.float32 and (
             not x.requires_grad or (x.is_leaf and not x._is_view() and torch.is_autocast_cache_enabled())):
-        return x.to(torch.get_autocast_dtype("cuda"))
+        return _cast(x)
     return x
 
 
 def linear_autograd(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
     """``F.linear(x, weight, bias)`` with autocast's casts, differentiable, with the parameters' gradients from one kernel."""
     if torch.is_autocast_enabled("cuda"):
-        dtype = torch.get_autocast_dtype("cuda")
-        x, weight, bias = (t if t is None else t.to(dtype) for t in (x, weight, bias))
+        x, weight, bias = _cast(x), _cast(weight), _cast(bias)
     return _LinearFn.apply(x, weight, bias)
 
 

@@ -124,3 +124,20 @@ def test_autocast_makes_one_copy_where_it_keeps_it():
     with torch.autocast("cuda", dtype=torch.bfloat16, cache_enabled=False):
         assert ops.autocast_once(x).dtype == torch.float32
     assert ops.autocast_once(x) is x
+
+
+@pytest.mark.gpu
+def test_calls_in_one_autocast_region_share_the_cast_weights():
+    m, x = nn.Linear(1024, 32, device=DEV), torch.randn(2, 8, 1024, device=DEV)
+    for cache in (True, False):
+        kept, grads = [], []
+        for f in (lambda t: ops.linear_autograd(t, m.weight, m.bias), m):
+            saved = set()
+            with torch.autocast("cuda", dtype=torch.bfloat16, cache_enabled=cache), torch.autograd.graph.saved_tensors_hooks(
+                    lambda t: (saved.add(t.untyped_storage().data_ptr()) if t.shape[0] in (32, 1024) else None, t)[1], lambda t: t):
+                out = sum(f(t.requires_grad_()).float().square().sum() for t in (x.clone(), x + 1))
+                kept.append(len(saved))
+            grads.append(torch.autograd.grad(out, (m.weight, m.bias)))
+        assert kept == ([1, 1] if cache else [2, 2])
+        for g, e in zip(*grads):   # (other sums of the same products: a rounding to bf16 of the value, twice)
+            assert g.dtype == torch.float32 and (g - e).abs().max() <= 2.0 ** -7 * e.abs().max()
