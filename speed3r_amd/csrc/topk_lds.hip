@@ -9,11 +9,14 @@
 //     eight waves share the key tiles; operands come straight from memory (each is used once per workgroup), four tiles in
 //     flight per wave.
 //   * Selection: a wave reads a row, 4 neighbouring columns per lane and 256-column piece, into registers.  The K-th largest of
-//     256 group maxima (a lane's four columns modulo 4: neighbours in different groups, since large scores come in runs) is a
+//     256 group maxima (a lane's four columns modulo 4: neighbours in different groups, since large scores come in runs; the lanes
+//     turned from piece to piece, since they come at one place of every frame of a still scene) is a
 //     lower bound of the row's K-th largest score; the search for it looks at the upper 24 bits of the sortable pattern only (its result may only be lower).  Scores at or above it, K to 1.4 K of them as a
 //     rule, are gathered in the row's own LDS space, one per lane, and ranked by counting: lane l compares its key with every
 //     other one.  No chain of exchanges, no sort.
-//   * More than 64 candidates (ties; a row of equal scores): K times the largest key below the last one, from the registers.
+//   * More than 64 candidates (a looser bound, equal scores): the bound is raised by halving the range of patterns, and of columns
+//     with one pattern, until 64 or fewer are left.  1 041 keys, top-32: 36 us as a rule, 65 where all scores are equal (two-sweep
+//     kernel 61 / 84); still scenes of 64 blocks a frame, 1 024 and 1 216 keys 27 and 37 (58 and 65; without turned lanes 37 and 51).
 // Order, fillers and NaN as in the two-sweep kernel: descending (sortable score, lowest column first), NaN never chosen, Lk - 1
 // in slots that nothing fills.
 //
@@ -122,6 +125,9 @@ __global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, 
 
   // ---- selection ----
   const int K = p.K;
+  // A lane's columns in piece i: turned against the other pieces, so that places 256 columns apart (or one place of several frames)
+  // lie in different lanes' groups
+  auto first_col = [&](int i) { return i * 256 + ((lane + (i * (i + 9) >> 1)) & 63) * 4; };
   constexpr int G = 4;               // groups of scores per lane: neighbouring columns in different ones
   constexpr int R = kRows / kWaves;  // rows of a wave, side by side: each hides the other's waits
   float v[R][NC][4];
@@ -137,7 +143,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, 
     for (int e = 0; e < G; e++) mx[e] = -INFINITY;
 #pragma unroll
     for (int i = 0; i < NC; i++) {
-      const int col = (i * 64 + lane) * 4;
+      const int col = first_col(i);
       const float4 x = *reinterpret_cast<const float4*>(row[r] + (col < Lk ? col : 0));
       v[r][i][0] = x.x; v[r][i][1] = x.y; v[r][i][2] = x.z; v[r][i][3] = x.w;
       if (i * 256 + 256 > Lk) {  // beyond the keys: NaN, which no comparison lets pass
@@ -161,6 +167,20 @@ __global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, 
       for (int e = 0; e < G; e++) cnt += (int)__popcll(__ballot(gk[r][e] >= cand));
       t[r] = cnt >= K ? cand : t[r];
     }
+  // lanes' counts -> what the lanes below have; the sum of all
+  auto prefix = [](int& own, int& all) {
+    int s = own;  // inclusive sum over the lanes below: rows of 16, then across them
+#define S3R_STEP(ctrl, rows_on) s += __builtin_amdgcn_update_dpp(0, s, ctrl, rows_on, 0xF, false)
+    S3R_STEP(0x111, 0xF);  // row_shr:1
+    S3R_STEP(0x112, 0xF);  // row_shr:2
+    S3R_STEP(0x114, 0xF);  // row_shr:4
+    S3R_STEP(0x118, 0xF);  // row_shr:8
+    S3R_STEP(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+    S3R_STEP(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+#undef S3R_STEP
+    all = __builtin_amdgcn_readlane(s, 63);
+    own = s - own;
+  };
   // candidates, packed to the front of the row's space (its scores are in registers): pattern and column
   float bound[R];
   int mine[R], n[R];  // where a lane's first one goes; the number of all
@@ -172,17 +192,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, 
     for (int i = 0; i < NC; i++)
 #pragma unroll
       for (int e = 0; e < 4; e++) mine[r] += v[r][i][e] >= bound[r] ? 1 : 0;
-    int s = mine[r];  // inclusive sum over the lanes below: rows of 16, then across them
-#define S3R_STEP(ctrl, rows_on) s += __builtin_amdgcn_update_dpp(0, s, ctrl, rows_on, 0xF, false)
-    S3R_STEP(0x111, 0xF);  // row_shr:1
-    S3R_STEP(0x112, 0xF);  // row_shr:2
-    S3R_STEP(0x114, 0xF);  // row_shr:4
-    S3R_STEP(0x118, 0xF);  // row_shr:8
-    S3R_STEP(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
-    S3R_STEP(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
-#undef S3R_STEP
-    n[r] = __builtin_amdgcn_readlane(s, 63);
-    mine[r] = s - mine[r];
+    prefix(mine[r], n[r]);
   }
 #pragma unroll
   for (int r = 0; r < R; r++)
@@ -192,7 +202,58 @@ __global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, 
       for (int i = 0; i < NC; i++)
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          if (v[r][i][e] >= bound[r]) *at++ = make_uint2(__float_as_uint(v[r][i][e]), (uint32_t)((i * 64 + lane) * 4 + e));
+          if (v[r][i][e] >= bound[r]) *at++ = make_uint2(__float_as_uint(v[r][i][e]), (uint32_t)(first_col(i) + e));
+    } else if (wave * R + r < rows) {
+      // More than fit the lanes: large scores share groups (256 columns apart, or four frames of 64 blocks: the same place in a still
+      // scene), or many are equal.  Halve the range of patterns until K to 64 lie at or above its lower end, or it is one
+      // pattern; of its columns then the range of those that are needed.
+      uint32_t x[NC][4];  // sortable patterns; NaN below all
+#pragma unroll
+      for (int i = 0; i < NC; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[i][e] = v[r][i][e] >= bound[r] ? sortable_key(v[r][i][e]) : 0;
+      uint32_t most = 0;
+#pragma unroll
+      for (int e = 0; e < G; e++) most = max(most, gk[r][e]);
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) most = max(most, (uint32_t)__shfl_xor((int)most, off));
+      most = __builtin_amdgcn_readfirstlane(most);
+      uint32_t lo = bound[r] == -INFINITY ? 0x007FFFFFu : t[r], hi = most + 1;  // as many at or above as n, none
+      int cols = Lk, cnt = n[r];  // columns below `cols` of those with the pattern `lo`
+      auto count = [&](auto takes) {
+        int c = 0, all;
+#pragma unroll
+        for (int i = 0; i < NC; i++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) c += takes(x[i][e], first_col(i) + e) ? 1 : 0;
+        prefix(c, all);
+        mine[r] = c;
+        return all;
+      };
+      while (cnt > 64 && hi - lo > 1) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        const int c = count([&](uint32_t k, int) { return k >= mid; });
+        if (c >= K) { lo = mid; cnt = c; }
+        else hi = mid;
+      }
+      if (cnt > 64) {
+        int below = 0;  // too few columns
+        while (cols - below > 1) {
+          const int mid = below + (cols - below) / 2;
+          const int c = count([&](uint32_t k, int col) { return k > lo || (k == lo && col < mid); });
+          if (c >= K) cols = mid;
+          else below = mid;
+        }
+      }
+      n[r] = count([&](uint32_t k, int col) { return k > lo || (k == lo && col < cols); });
+      uint2* at = reinterpret_cast<uint2*>(row[r]) + mine[r];
+#pragma unroll
+      for (int i = 0; i < NC; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int col = first_col(i) + e;
+          if (x[i][e] > lo || (x[i][e] == lo && col < cols)) *at++ = make_uint2(__float_as_uint(sortable_to_float(x[i][e])), (uint32_t)col);
+        }
     }
   uint64_t key[R];
   uint32_t col[R];
@@ -204,44 +265,22 @@ __global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, 
   }
 #pragma unroll
   for (int r = 0; r < R; r++)
-    if (n[r] <= 64 && wave * R + r < rows) reinterpret_cast<uint64_t*>(row[r])[lane] = key[r];
+    if (wave * R + r < rows) reinterpret_cast<uint64_t*>(row[r])[lane] = key[r];
 #pragma unroll
   for (int r = 0; r < R; r++) {
     if (wave * R + r >= rows) break;
     int32_t* const out = p.topk_idx + ((int64_t)bh * p.Lq + q0 + wave * R + r) * K;
-    if (n[r] <= 64) {
-      int rank = 0;
-      for (int j = 0; j < n[r]; j += 8) {  // (keys behind the last one are 0: above nothing)
-        const ulonglong2* const o = reinterpret_cast<const ulonglong2*>(row[r]) + j / 2;
-        ulonglong2 w[4];
+    int rank = 0;
+    for (int j = 0; j < n[r]; j += 8) {  // (keys behind the last one are 0: above nothing)
+      const ulonglong2* const o = reinterpret_cast<const ulonglong2*>(row[r]) + j / 2;
+      ulonglong2 w[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) w[u] = o[u];
+      for (int u = 0; u < 4; u++) w[u] = o[u];
 #pragma unroll
-        for (int u = 0; u < 4; u++) rank += (w[u].x > key[r] ? 1 : 0) + (w[u].y > key[r] ? 1 : 0);
-      }
-      if (lane < n[r] && rank < K) out[rank] = (int32_t)col[r];
-      if (lane >= n[r] && lane < K) out[lane] = Lk - 1;
-    } else {
-      uint64_t last = ~0ull;
-#pragma unroll 1
-      for (int k = 0; k < K; k++) {
-        uint64_t best = 0;
-#pragma unroll
-        for (int i = 0; i < NC; i++)
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const uint64_t x = ((uint64_t)sortable_key(v[r][i][e]) << 32) | (uint32_t)(Lk - 1 - ((i * 64 + lane) * 4 + e));
-            best = v[r][i][e] >= bound[r] && x < last && x > best ? x : best;
-          }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const uint64_t other = ((uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)(best >> 32), off) << 32) | (uint32_t)__shfl_xor((int)(uint32_t)best, off);
-          best = other > best ? other : best;
-        }
-        last = best;
-        if (lane == 0) out[k] = Lk - 1 - (int)(uint32_t)best;
-      }
+      for (int u = 0; u < 4; u++) rank += (w[u].x > key[r] ? 1 : 0) + (w[u].y > key[r] ? 1 : 0);
     }
+    if (lane < n[r] && rank < K) out[rank] = (int32_t)col[r];
+    if (lane >= n[r] && lane < K) out[lane] = Lk - 1;
   }
 }
 

@@ -35,6 +35,22 @@ def test_indices_match_the_selection_on_stored_scores(b, h, lq, lk, dtype):
             assert torch.equal(got, want), topk
 
 
+# still scenes: the same blocks in every frame, with a little of their own or none (equal scores), so that a query's best keys lie at
+# one place of every frame: in few of the groups whose maxima bound the selection
+@pytest.mark.parametrize("per,frames", [(64, 16), (64, 19), (16, 76), (256, 4), (96, 12), (1, 1216), (2, 300), (5, 240)])
+@pytest.mark.parametrize("noise", [0.0, 0.1])
+def test_still_scenes(per, frames, noise):
+    gen = torch.Generator(device=DEV).manual_seed(per)
+    randn = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    x = (randn(1, 2, 1, per, 64) + noise * randn(1, 2, frames, per, 64)).reshape(1, 2, -1, 64)
+    for dtype in (torch.bfloat16, torch.float16):
+        q, k = x.to(dtype), (x + 0.1 * noise * randn(*x.shape)).to(dtype)
+        for topk in (1, 8, 16, 32):
+            for sign in (1, -1):   # scores above and below zero
+                got, want, _ = _same(q, sign * k, topk)
+                assert torch.equal(got, want), topk
+
+
 def test_infinite_scores_and_strided_rows():
     q, k = torch.randn(1, 2, 40, 128, device=DEV).bfloat16(), torch.randn(1, 2, 100, 192, device=DEV).bfloat16()
     q, k = q[..., 64:], k[..., 64:128]                      # rows 128 and 192 values apart
