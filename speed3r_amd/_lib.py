@@ -45,6 +45,7 @@ SIGNATURES = {
     "s3r_layer_prepass": (c_int, [c_void_p, c_void_p]),
     "s3r_layer_prepass_bwd": (c_int, [c_void_p] * 12 + [c_int, c_void_p]),
     "s3r_gated_merge_bwd": (c_int, [c_void_p] * 9 + [c_int, c_int, c_int64, c_int, c_int, *_i64x3, c_int, c_void_p]),
+    "s3r_topk_in_lds": (c_int, [c_int64, c_int64, c_int64, c_int]),
     "s3r_linear": (c_int, [c_void_p] * 4 + [c_int64, c_int, c_int, *_i64x3, c_int, c_int, c_void_p]),
     "s3r_linear_wgrad_workspace": (c_int64, [c_int64, c_int, c_int, c_int64, c_int64]),
     "s3r_linear_wgrad": (c_int, [c_void_p] * 5 + [c_int64, c_int, c_int, c_int64, c_int64, c_int, c_void_p]),

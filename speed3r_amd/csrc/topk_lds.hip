@@ -300,12 +300,22 @@ template <typename E> static int launch(const AttnParams& p, hipStream_t st) {
 
 constexpr int64_t kMostGroups = 1536;
 
-bool topk_lds_pays(const AttnParams& p) {
-  return p.Lk <= (p.K <= 4 ? 640 : p.K <= 8 ? 1024 : kMostKeys) && (p.Lq + tkl::kRows - 1) / tkl::kRows * p.B * p.H <= kMostGroups;
+// Few keys and a short list: the two-sweep kernel's folds are fewer than the steps of the search here.  16 heads, as many rows as keys,
+// two-sweep / this: top-1 16 keys 4.7 / 6.7, 96 6.9 / 7.1, 126 7.4 / 7.2; top-4 16 5.1 / 6.8, 64 6.2 / 7.0, 65 8.1 / 7.1; top-8 64 6.6 /
+// 7.0, 65 8.4 / 7.2; top-16 16 6.1 / 7.0, 33 7.0 / 7.2, 48 8.0 / 7.3; top-32 32 9.5 / 7.3.
+static bool short_lists(int64_t BH, int64_t Lq, int64_t Lk, int K) {
+  return Lk > (K <= 2 ? 96 : K <= 8 ? 64 : K <= 16 ? 40 : 0) && Lk <= (K <= 4 ? 640 : K <= 8 ? 1024 : kMostKeys) &&
+         (Lq + tkl::kRows - 1) / tkl::kRows * BH <= kMostGroups;
 }
+
+bool topk_lds_pays(const AttnParams& p) { return short_lists((int64_t)p.B * p.H, p.Lq, p.Lk, p.K); }
 
 int launch_topk_lds(const AttnParams& p, int dtype, void* stream) {
   return dtype == S3R_BF16 ? tkl::launch<bf16_t>(p, (hipStream_t)stream) : tkl::launch<f16_t>(p, (hipStream_t)stream);
 }
 
 }  // namespace s3r
+
+extern "C" int s3r_topk_in_lds(int64_t batch_heads, int64_t Lq, int64_t Lk, int K) {
+  return batch_heads > 0 && Lq > 0 && Lk > 0 && K > 0 && batch_heads <= s3r::kMostGroups && Lq <= (1 << 20) && s3r::short_lists(batch_heads, Lq, Lk, K);
+}

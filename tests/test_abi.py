@@ -109,3 +109,12 @@ def test_reference_signature_asserts():
         s3r.topk_blocksparse_attention(x, x, x, torch.zeros((1, 1, 1, 1), dtype=torch.int64), 64)   # idx dtype
     with pytest.raises(AssertionError):
         s3r.topk_blocksparse_attention(x, x, x, torch.zeros((1, 1, 1, 1), dtype=torch.int32), 48)   # block size
+
+
+def test_which_kernel_selects_the_indices():
+    """Few keys and a short list, many keys, many rows: not the kernel that keeps the scores in LDS."""
+    rule = lambda bh, lq, lk, k: bool(_lib.lib().s3r_topk_in_lds(bh, lq, lk, k))
+    for k, few, most in ((1, 96, 640), (2, 96, 640), (4, 64, 640), (8, 64, 1024), (16, 40, 1216), (32, 0, 1216)):
+        for n, want in ((few, False), (few + 1, True), (most, True), (most + 1, False)):
+            assert n == 0 or rule(2, n, n, k) is want, (k, n)
+    assert rule(16, 1536, 700, 32) and not rule(16, 1537, 700, 32) and not rule(1 << 40, 1, 700, 32) and not rule(1, 0, 700, 32)

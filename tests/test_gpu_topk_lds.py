@@ -35,6 +35,13 @@ def test_indices_match_the_selection_on_stored_scores(b, h, lq, lk, dtype):
             assert torch.equal(got, want), topk
 
 
+@pytest.mark.parametrize("topk,keys", [(1, 96), (2, 97), (4, 64), (4, 65), (8, 64), (8, 65), (16, 40), (16, 41), (4, 641), (8, 1025)])
+def test_both_sides_of_the_rule(topk, keys):
+    q, k = (torch.randn(1, 2, keys, 64, generator=torch.Generator(device=DEV).manual_seed(s), device=DEV).bfloat16() for s in (topk, keys))
+    got, want, _ = _same(q, k, topk)
+    assert torch.equal(got, want)
+
+
 # still scenes: the same blocks in every frame, with a little of their own or none (equal scores), so that a query's best keys lie at
 # one place of every frame: in few of the groups whose maxima bound the selection
 @pytest.mark.parametrize("per,frames", [(64, 16), (64, 19), (16, 76), (256, 4), (96, 12), (1, 1216), (2, 300), (5, 240)])
