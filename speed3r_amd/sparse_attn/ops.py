@@ -1007,24 +1007,30 @@ def _two_kernel_compressed(q: torch.Tensor, topk: int, block: int = 1) -> bool:
             and -(-q.shape[2] // block) <= (1 << 21) and _lib.lib_has_fused_topk())
 
 
-# Pooled rows (B * H * blocks) from which the index kernel goes on a stream of its own.  The two events and the change of
-# stream cost the host 60 to 80 us and the kernels behind them a wait between queues; what there is to hide is the dense
-# sweep's 12 to 16 us.  Up to 1216 pooled tokens (top-8: 1024, top-4 and less: 640) the indices come from the short kernel, which has too
-# little to gain; the line lies there for 16 heads.  us per call, two streams / one, 16 heads: layer at 16-token blocks, 504 pooled tokens 221 / 186, 1 008
-# 335 / 328, 2 016 714 / 721; at 64-token blocks, 394 378 / 365, 814 806 / 802, 1 074 1 054 / 1 047, 1 627 1 570 / 1 592; operators, 504
-# pooled tokens 122 / 95, 1 008 161 / 148, at 64-token blocks 537 227 / 222, 1 041 418 / 413, 1 172 451 / 441, 1 627 612 / 611,
-# 2 082 766 / 778, 4 164 1 532 / 1 551; top-8, 1 188 328 / 331.
+# When the index kernel goes on a stream of its own.  The two events and the change of stream cost the host up to 40 us and the kernels
+# behind them a wait between queues; what there is to hide is the dense sweep's 12 to 16 us.  The kernel for short lists of keys has
+# too little to gain.  The two-sweep kernel pays from 19 456 pooled rows (B * H * blocks) on; long lists over few heads, whose chain is long and
+# leaves most of the chip idle, from 8192.  us per call, two streams / one: short lists, 2 x 16 heads of 620 pooled tokens, operators 238 / 228,
+# layer 416 / 404, 32 heads of 600 235 / 226 and 538 / 535, top-1 over 16 heads of 700 125 / 85 and 253 / 204; two sweeps, 16 heads,
+# 16-token blocks, layer 2 016 pooled tokens 714 / 721, top-4 over 1 200 318 / 309, over 1 300 332 / 338; 64-token blocks, layer 1 627
+# 1 570 / 1 592, operators 1 041 418 / 413, 2 082 766 / 778, 4 164 1 532 / 1 551; 2 x 16 heads of 1 300 at 16-token blocks 481 / 504 and 883 / 894;
+# 8 heads of 2 016 at 16- / 64-token blocks, layer 366 / 363 and 983 / 989, operators 265 / 269 and 671 / 671; of 2 432 443 / 433; of 2 600
+# 467 / 467 and 334 / 342; 4 heads of 4 000 404 / 407 and 329 / 342; 2 heads of 5 000 379 / 391 and 339 / 354, top-4 over 4 200
+# 213 / 204 and 164 / 177.
 SIDE_STREAM_ROWS = 16 * 1216
+SIDE_STREAM_ROWS_OF_LONG_LISTS = 8192
 
 
-def _side_stream_rows(topk: int) -> int:
-    return SIDE_STREAM_ROWS if topk > 8 else 16 * (1024 if topk > 4 else 640)
+def _side_stream_pays(heads: int, blocks: int, topk: int) -> bool:
+    """``heads``: those of all sequences; ``blocks``: pooled tokens of each."""
+    rows = heads * blocks
+    return (rows > SIDE_STREAM_ROWS or (topk > 8 and blocks > 2432 and rows > SIDE_STREAM_ROWS_OF_LONG_LISTS)) \
+        and not _lib.lib().s3r_topk_in_lds(heads, blocks, blocks, topk)
 
 
 def _indices_beside(q: torch.Tensor, topk: int, block: int = 1) -> bool:
     """True where the index kernel runs on the side stream (arguments as for :func:`_two_kernel_compressed`)."""
-    rows = q.shape[0] * q.shape[1] * -(-q.shape[2] // block)
-    return rows > _side_stream_rows(topk) and _two_kernel_compressed(q, topk, block)
+    return _side_stream_pays(q.shape[0] * q.shape[1], -(-q.shape[2] // block), topk) and _two_kernel_compressed(q, topk, block)
 
 
 def topk_indices_on_side_stream(qc: torch.Tensor, kc: torch.Tensor, topk: int, softmax_scale: Optional[float] = None):
@@ -1057,7 +1063,7 @@ def sparse_global_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g
     The merge runs in the selection kernel's epilogue where the library offers it (same bits either way);
     ``return_parts`` needs the selection output and therefore runs the two operators separately.
 
-    ``overlap`` (default: on from ``SIDE_STREAM_ROWS`` pooled rows; True: wherever it applies): the indices need pooled q and k only, the compressed attention output
+    ``overlap`` (default: where :func:`_side_stream_pays` says so; True: wherever it applies): the indices need pooled q and k only, the compressed attention output
     is not read before the merge.  Where the two come from different kernels (no score buffer), the index kernel runs
     on a second stream next to the pooling of v and the compressed attention (same kernels, same results; only the
     schedule differs).  The index kernel alone leaves most of the chip idle below a few thousand pooled tokens (one

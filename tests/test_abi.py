@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from speed3r_amd import _lib
+from speed3r_amd.sparse_attn import ops
 
 ROOT = Path(__file__).resolve().parent.parent
 HEADER = (ROOT / "include" / "speed3r_hip.h").read_text()
@@ -118,3 +119,10 @@ def test_which_kernel_selects_the_indices():
         for n, want in ((few, False), (few + 1, True), (most, True), (most + 1, False)):
             assert n == 0 or rule(2, n, n, k) is want, (k, n)
     assert rule(16, 1536, 700, 32) and not rule(16, 1537, 700, 32) and not rule(1 << 40, 1, 700, 32) and not rule(1, 0, 700, 32)
+
+
+def test_second_stream_follows_the_index_kernel():
+    pays = ops._side_stream_pays
+    assert not pays(32, 620, 32) and not pays(32, 768, 16) and not pays(16, 700, 1)   # short lists: one kernel of a few microseconds
+    assert pays(32, 769, 32) and pays(16, 1217, 16) and pays(16, 1217, 1) and not pays(16, 1216, 1)
+    assert pays(4, 4000, 32) and not pays(4, 4000, 8) and not pays(8, 2432, 32) and pays(8, 2433, 16) and not pays(2, 4000, 32)
