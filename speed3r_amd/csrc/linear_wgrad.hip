@@ -5,8 +5,9 @@
 // the tokens leaves the chip idle.  Here each tile's tokens are dealt out over enough workgroups to fill the chip once; their
 // partial tiles meet in a workspace and a second kernel adds them.  The sums of dY over the tokens (the bias's gradient) take one
 // more product by ones in 64: the tiles that share dY's columns share them out.  bf16, us, the library's product and its sum of
-// dY / here: 24 192 tokens 3072 x 1024 240 + 39 / 130 (1.17 PFLOP/s), 1024 x 1024 179 + 27 / 62, 32 x 1024 78 + 10 / 37; 8 192
-// tokens 79 + 25 / 59 and 53 + 20 / 38; 50 000 tokens 3072 x 1024 402 + 70 / 311.  Bound by the matrix cores' power where tiles
+// dY / here: 24 192 tokens 3072 x 1024 246 + 41 / 137 (1.11 PFLOP/s), 1024 x 1024 181 + 29 / 63, 32 x 1024 79 + 10 / 28; 8 192
+// tokens 85 + 26 / 62 and 53 + 20 / 38; 50 000 tokens 3072 x 1024 418 + 74 / 267.  The last rows, fewer than 128, come as a
+// pair of steps filled up with zeros (added by the second kernel one by one, 64 of them made 24 000 tokens 160 us instead of 125).  Bound by the matrix cores' power where tiles
 // are many, by the way of the partial tiles where they are few (64 MB each way for 1024 x 1024).
 //
 // The tile is linear_tile.h's (four waves of 128 x 128 values in all accumulator registers, operands a half step ahead, transfers
@@ -25,13 +26,19 @@ struct WgradParams {
   float* ws;      // [splits][N][C], then with db [splits][N]
   int64_t M, lddy, ldx;
   int N, C, nt, ct, splits;
-  int64_t units;  // whole pairs of steps: 128 tokens each
+  int64_t units;  // pairs of steps, 128 tokens each, the last one perhaps fewer
 };
 
 __device__ __forceinline__ constexpr int unit_swizzle(int row) { return (row & 3) | (((row >> 3) & 1) << 2); }
 
 __device__ __forceinline__ s16x4 read_tr(const void* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)p);
+}
+
+// 16 bytes per lane from base + off to dst + 16 lane; zeros where `off` is not below `bytes`
+__device__ __forceinline__ void rows_to_lds(const char* base, int bytes, void* dst, uint32_t off) {
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes > 0 ? bytes : 0, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
 }
 
 template <typename E> struct TokenTile {
@@ -41,20 +48,23 @@ template <typename E> struct TokenTile {
   uint32_t xoff[T], yoff[T];   // the lane's pieces of a step's rows
   uint32_t fx[T], fy[T];       // where the wave's tiles lie in a buffer's first rows
   const char *bx, *by;
-  uint32_t sx, sy;             // bytes from step to step
+  int sx, sy;                  // bytes from step to step
+  int nx, ny;                  // bytes of the range's rows: what lies beyond is read as zeros
   struct Frag8 { V8 x[T], y[T], b; } P, Q;
   uint32_t fb;                 // the tile of dY whose sums this wave takes (b)
   V8 ones;
   f32x4 sums;                  // lane: out-channel lane % 16, four times
   f32x4 acc[T][T];             // [out][in]: lane: in-channels 4 (lane / 16) .. + 3 of out-channel lane % 16
 
-  __device__ __forceinline__ void init(const E* x, int64_t ldx, int xcols, const E* dy, int64_t ldy, int ycols, int sum_tile) {
+  __device__ __forceinline__ void init(const E* x, int64_t ldx, int xcols, const E* dy, int64_t ldy, int ycols, int rows, int sum_tile) {
     wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     lane = threadIdx.x & 63;
     bx = reinterpret_cast<const char*>(x);
     by = reinterpret_cast<const char*>(dy);
-    sx = (uint32_t)(ldx * 128);
-    sy = (uint32_t)(ldy * 128);
+    sx = (int)(ldx * 128);
+    sy = (int)(ldy * 128);
+    nx = rows * (int)(ldx * 2);
+    ny = rows * (int)(ldy * 2);
 #pragma unroll
     for (int i = 0; i < T; i++) {
       const int row = 16 * wave + 2 * i + (lane >> 5);
@@ -76,8 +86,9 @@ template <typename E> struct TokenTile {
     sums = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   template <typename P8> __device__ __forceinline__ void move(P8* lx, P8* ly, uint32_t step, int i) {
-    if (i < T) to_lds16(bx, lx + (16 * wave + 2 * i) * 512, xoff[i], step * sx);
-    else to_lds16(by, ly + (16 * wave + 2 * (i - T)) * 512, yoff[i - T], step * sy);
+    const int px = (int)step * sx, py = (int)step * sy;
+    if (i < T) rows_to_lds(bx + px, nx - px, lx + (16 * wave + 2 * i) * 512, xoff[i]);
+    else rows_to_lds(by + py, ny - py, ly + (16 * wave + 2 * (i - T)) * 512, yoff[i - T]);
   }
   template <typename P8> __device__ __forceinline__ void read(Frag8& f, P8* lx, P8* ly, int half, int r) {  // fragment r: y0, x0 .., y1 ..
     union { s16x4 s[2]; V8 v; } g;
@@ -135,7 +146,7 @@ template <typename E> __global__ __launch_bounds__(256, 1) void wgrad_kernel(Wgr
   const int64_t u0 = p.units * s / p.splits, u1 = p.units * (s + 1) / p.splits;
   Tl tl;
   tl.init((const E*)p.x + u0 * 128 * p.ldx + c0, p.ldx, p.C - c0 < 256 ? p.C - c0 : 256, (const E*)p.dy + u0 * 128 * p.lddy + n0, p.lddy,
-          p.N - n0 < 256 ? p.N - n0 : 256, __builtin_amdgcn_readfirstlane(sum_tile));
+          p.N - n0 < 256 ? p.N - n0 : 256, (int)(u1 * 128 < p.M ? (u1 - u0) * 128 : p.M - u0 * 128), __builtin_amdgcn_readfirstlane(sum_tile));
   const uint32_t steps = (uint32_t)(u1 - u0) * 2;
   if (steps == 0) return;  // (never: as many splits as units at most)
 #pragma unroll
@@ -178,32 +189,20 @@ template <typename E> __global__ __launch_bounds__(256, 1) void wgrad_kernel(Wgr
   __builtin_amdgcn_s_waitcnt(0x0070);  // no transfer may still write LDS when the wave ends
 }
 
-// dW = sum of the partial tiles and of the last tokens (fewer than 128, which fill no pair of steps): HBM bound
+// dW = sum of the partial tiles: HBM bound
 template <typename E> __global__ __launch_bounds__(256) void wgrad_sum_kernel(WgradParams p) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= (int64_t)p.N * p.C) {
     const int64_t n = i / 4 - (int64_t)p.N * p.C / 4;  // behind the weights: one thread per bias
     if (!p.db || n >= p.N) return;
     float a = 0.f;
-    if (p.units > 0)
-      for (int s = 0; s < p.splits; s++) a += p.ws[(int64_t)p.splits * p.N * p.C + (int64_t)s * p.N + n];
-    for (int64_t m = p.units * 128; m < p.M; m++) a += (float)((const E*)p.dy)[m * p.lddy + n];
+    for (int s = 0; s < p.splits; s++) a += p.ws[(int64_t)p.splits * p.N * p.C + (int64_t)s * p.N + n];
     ((E*)p.db)[n] = (E)a;
     return;
   }
   f32x4 a = {0.f, 0.f, 0.f, 0.f};
-  if (p.units > 0) {
 #pragma unroll 8
-    for (int s = 0; s < p.splits; s++) a += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.ws + (int64_t)s * p.N * p.C + i));
-  }
-  const int n = (int)(i / p.C), c = (int)(i - (int64_t)n * p.C);
-  for (int64_t m = p.units * 128; m < p.M; m++) {
-    const float d = (float)((const E*)p.dy)[m * p.lddy + n];
-    union { uint2 u; E e[4]; } x;
-    x.u = *reinterpret_cast<const uint2*>((const E*)p.x + m * p.ldx + c);
-#pragma unroll
-    for (int k = 0; k < 4; k++) a[k] = fmaf(d, (float)x.e[k], a[k]);
-  }
+  for (int s = 0; s < p.splits; s++) a += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.ws + (int64_t)s * p.N * p.C + i));
   union { E e[4]; uint2 u; } o;
 #pragma unroll
   for (int k = 0; k < 4; k++) o.e[k] = (E)a[k];
@@ -213,7 +212,7 @@ template <typename E> __global__ __launch_bounds__(256) void wgrad_sum_kernel(Wg
 // Ranges of tokens: the fewest microseconds of rounds of workgroups (1.5 a step of 64 tokens, 6 to fill the pipeline and write a
 // partial tile) and of the partial tiles' way through memory, and a range's rows inside 32-bit byte offsets.
 static int wgrad_splits(int64_t M, int N, int C, int64_t ld) {
-  const int64_t tiles = (int64_t)((N + 255) / 256) * ((C + 255) / 256), units = M / 128;
+  const int64_t tiles = (int64_t)((N + 255) / 256) * ((C + 255) / 256), units = (M + 127) / 128;
   int best = 1;
   double least = 1e30;
   for (int64_t s = 1; s <= 64 && s <= units; s++) {
@@ -247,17 +246,15 @@ extern "C" int s3r_linear_wgrad(const void* dy, const void* x, void* dw, void* d
   if (M > 64 * (0x7f000000LL / (2 * ld) - 128)) return fail(S3R_ERR_UNSUPPORTED, "s3r_linear_wgrad: 64 ranges of %lld rows are not enough", (long long)M);
   if (!aligned16(dy) || !aligned16(x) || !aligned16(dw) || !aligned16(workspace) || lddy % 8 || ldx % 8)
     return fail(S3R_ERR_BAD_ARG, "s3r_linear_wgrad: pointers and rows must be multiples of 16 bytes");
-  lin::WgradParams p = {dy, x, dw, db, workspace, M, lddy, ldx, N, C, (N + 255) / 256, (C + 255) / 256, 0, M / 128};
+  lin::WgradParams p = {dy, x, dw, db, workspace, M, lddy, ldx, N, C, (N + 255) / 256, (C + 255) / 256, 0, (M + 127) / 128};
   p.splits = lin::wgrad_splits(M, N, C, ld);
   const int64_t wgs = (int64_t)p.nt * p.ct * p.splits, sums = ((int64_t)N * C / 4 + N + 255) / 256;
   if (wgs > 0x7fffffffLL || sums > 0x7fffffffLL) return fail(S3R_ERR_UNSUPPORTED, "s3r_linear_wgrad: tensor too large for one launch");
   hipStream_t st = (hipStream_t)stream;
-  if (p.units > 0) {
-    if (dtype == S3R_BF16) hipLaunchKernelGGL((lin::wgrad_kernel<bf16_t>), dim3((unsigned)wgs), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((lin::wgrad_kernel<f16_t>), dim3((unsigned)wgs), dim3(256), 0, st, p);
-    const int rc = check_launch("wgrad_kernel");
-    if (rc != S3R_OK) return rc;
-  }
+  if (dtype == S3R_BF16) hipLaunchKernelGGL((lin::wgrad_kernel<bf16_t>), dim3((unsigned)wgs), dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((lin::wgrad_kernel<f16_t>), dim3((unsigned)wgs), dim3(256), 0, st, p);
+  const int rc = check_launch("wgrad_kernel");
+  if (rc != S3R_OK) return rc;
   if (dtype == S3R_BF16) hipLaunchKernelGGL((lin::wgrad_sum_kernel<bf16_t>), dim3((unsigned)sums), dim3(256), 0, st, p);
   else hipLaunchKernelGGL((lin::wgrad_sum_kernel<f16_t>), dim3((unsigned)sums), dim3(256), 0, st, p);
   return check_launch("wgrad_sum_kernel");

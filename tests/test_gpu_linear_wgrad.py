@@ -53,6 +53,23 @@ def test_wgrad_matches_float64(m, n, c, dtype):
     assert torch.equal(dw, ops.linear_wgrad(dy, x, bias)[0])
 
 
+# rows around the steps of 64 and the pairs of them, in one range and in many; around them, and in what the same workgroups worked on
+# before, values that would show
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 15, 63, 64, 65, 127, 129, 191, 193, 4100, 4159, 4161])
+def test_wgrad_takes_its_rows_only(m):
+    nan = float("nan")
+    dy, x = (torch.full((m + 256, c), nan, device=DEV).bfloat16() for c in (136, 1032))
+    dy[128:128 + m], x[128:128 + m] = torch.randn(m, 136, device=DEV).bfloat16(), torch.randn(m, 1032, device=DEV).bfloat16()
+    ops.linear_wgrad(torch.full_like(dy, nan), torch.full_like(x, nan), True)
+    a, b = dy[128:128 + m], x[128:128 + m]
+    dw, db = ops.linear_wgrad(a, b, True)
+    for got, t in ((dw, b), (db, torch.ones_like(b[:, :1]))):
+        want, room = a.double().t() @ t.double(), (a.double().abs().t() @ t.double().abs()) * m * 2.0 ** -24
+        # half a bf16 step of the value, a rounding of the sum of magnitudes per token
+        assert ((got.double() - want.view_as(got)).abs() <= 2.0 ** -8 * want.abs().view_as(got) * (1 + 2.0 ** -8) + room.view_as(got) + 2.0 ** -25).all()
+
+
 @pytest.mark.gpu
 def test_wgrad_refuses_what_it_is_not_built_for():
     x, dy = torch.randn(256, 512, device=DEV).bfloat16(), torch.randn(256, 64, device=DEV).bfloat16()
