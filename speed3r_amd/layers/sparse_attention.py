@@ -70,7 +70,9 @@ def linear_trains(m: nn.Linear, x: Tensor) -> bool:
         return False
     dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
     return calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter and m.weight.requires_grad \
-        and dtype in (torch.bfloat16, torch.float16) and x.shape[-1] == m.weight.shape[1] and ops.ordinary(x) \
+        and dtype in (torch.bfloat16, torch.float16) and x.shape[-1] == m.weight.shape[1] \
+        and ops.linear_wgrad_takes(*m.weight.shape) \
+        and ops.ordinary(x) \
         and all(t is None or t.dtype in (torch.float32, torch.bfloat16, torch.float16) for t in (x, m.weight, m.bias))
 
 

@@ -526,6 +526,11 @@ def linear_wgrad_pays(rows: int) -> bool:
     return rows >= 4096
 
 
+def linear_wgrad_takes(n: int, c: int) -> bool:
+    """Whether the kernel is built for ``n`` outputs and ``c`` inputs."""
+    return n % 8 == 0 and c % 8 == 0 and 0 < n <= 1 << 20 and 0 < c <= 1 << 20
+
+
 class _LinearFn(torch.autograd.Function):
     """``F.linear`` whose parameters' gradients come from :func:`linear_wgrad`; keeps what ``F.linear`` keeps."""
 
@@ -544,9 +549,11 @@ class _LinearFn(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dx = (dy2 @ weight).view(*dy.shape[:-1], weight.shape[1])
         if ctx.needs_input_grad[1] and not torch.is_grad_enabled() and ordinary(dy):   # (a derivative of the backward itself: torch's)
-            got = linear_wgrad(dy2, x.reshape(-1, x.shape[-1]), ctx.needs_input_grad[2])
+            want_db = ctx.needs_input_grad[2]
+            inside = want_db and x.shape[-1] > 768   # (the kernel sums dy beside enough inputs only)
+            got = linear_wgrad(dy2, x.reshape(-1, x.shape[-1]), inside)
             if got is not None:
-                return dx, *got
+                return dx, got[0], dy2.sum(0) if want_db and not inside else got[1]
         if ctx.needs_input_grad[1]:
             dw = dy2.t() @ x.reshape(-1, x.shape[-1])
         if ctx.needs_input_grad[2]:
@@ -582,8 +589,8 @@ def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, bias: bool):
     Returns None where the library has no kernel (bf16/fp16, N and C multiples of 8, with the bias C > 768, rows of
     adjacent values, 16-byte aligned)."""
     (m, n), c = dy.shape, x.shape[1]
-    if dy.dtype not in (torch.bfloat16, torch.float16) or x.dtype != dy.dtype or x.device != dy.device or x.shape[0] != m or n % 8 or c % 8 \
-            or m == 0 or n * c == 0 or (bias and c <= 768) or max(n, c) > 1 << 20:
+    if dy.dtype not in (torch.bfloat16, torch.float16) or x.dtype != dy.dtype or x.device != dy.device or x.shape[0] != m or m == 0 \
+            or not linear_wgrad_takes(n, c) or (bias and c <= 768):
         return None
     for t in (dy, x):
         if t.stride(1) != 1 or t.stride(0) % 8 or not t.shape[1] <= t.stride(0) < 1 << 21 or t.data_ptr() % 16:

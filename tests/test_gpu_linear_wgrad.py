@@ -158,3 +158,25 @@ def test_calls_in_one_autocast_region_share_the_cast_weights():
         assert kept == ([1, 1] if cache else [2, 2])
         for g, e in zip(*grads):   # (other sums of the same products: a rounding to bf16 of the value, twice)
             assert g.dtype == torch.float32 and (g - e).abs().max() <= 2.0 ** -7 * e.abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c,bias", [(256, True), (256, False), (768, True), (776, True)])
+def test_weights_of_few_inputs_train_through_the_kernel(c, bias, monkeypatch):
+    calls = []
+    kernel = ops.linear_wgrad
+    monkeypatch.setattr(ops, "linear_wgrad", lambda *a: (calls.append(kernel(*a)), calls[-1])[1])
+    m = nn.Linear(c, 64, bias=bias, device=DEV, dtype=torch.bfloat16)
+    x, dy = torch.randn(ROWS, c, device=DEV).bfloat16(), torch.randn(ROWS, 64, device=DEV).bfloat16()
+    wrt = tuple(m.parameters())
+    got, want = torch.autograd.grad(linear(m, x), wrt, dy), torch.autograd.grad(m(x), wrt, dy)
+    assert len(calls) == 1 and calls[0] is not None and calls[0][0] is got[0]
+    mags = (dy.double().abs().t() @ x.double().abs(), dy.double().abs().sum(0))
+    for g, w, mag in zip(got, want, mags):   # as above: half a bf16 step each, an fp32 rounding per token each
+        assert ((g.double() - w.double()).abs() <= 2.0 ** -7 * w.double().abs() + 2 * mag * ROWS * 2.0 ** -24).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,c", [(60, 1024), (64, 100)])
+def test_weights_without_a_kernel_keep_their_graph(n, c):
+    assert not linear_trains(nn.Linear(c, n, device=DEV, dtype=torch.bfloat16), torch.randn(ROWS, c, device=DEV).bfloat16())
