@@ -44,6 +44,12 @@ def test_gelu_of_infinities_and_nan():
     assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isnan(), want.isnan()) and torch.equal(got[0], want[0])
 
 
+@torch.no_grad()
+def test_linear_without_inputs():
+    m, x = nn.Linear(0, 8, device=DEV, dtype=torch.bfloat16), torch.empty(5, 0, device=DEV, dtype=torch.bfloat16)
+    assert torch.equal(linear(m, x), m(x)) and torch.equal(linear(m, x[:0]), m(x[:0]))
+
+
 def test_linear_writes_inside_its_rows_only():
     x, w = torch.randn(300, 256, device=DEV).bfloat16(), torch.randn(264, 256, device=DEV).bfloat16()
     from speed3r_amd import _lib
