@@ -54,10 +54,12 @@ def enough_work(x: Tensor) -> bool:
     return x.numel() >= max(1, min(1024 * x.shape[-1], 384 * 1024))
 
 
-def linear_takes(m: nn.Linear, x: Tensor) -> bool:
+def linear_takes(m: nn.Linear, x: Tensor, gelu: Optional[bool] = None) -> bool:
     """Whether a kernel may stand in for ``m(x)``: an ordinary call for inference of a module that would run
-    ``nn.Linear.forward`` and nothing else, on enough rows (asked first: few rows wait for the host)."""
-    return sizes_are_known(x) and enough_work(x) and calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter \
+    ``nn.Linear.forward`` and nothing else, on enough rows (asked first: few rows wait for the host) and, unless ``gelu`` is None,
+    where ``ops.linear`` with it or without is the faster one."""
+    return sizes_are_known(x) and enough_work(x) and type(m) is nn.Linear \
+        and (gelu is None or ops.linear_pays(x.numel() // x.shape[-1], *m.weight.shape, gelu)) and calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter \
         and x.shape[-1] == m.weight.shape[1] and takes_kernels(x) \
         and not (torch.is_grad_enabled() and (x.requires_grad or m.weight.requires_grad or (m.bias is not None and m.bias.requires_grad)))
 
@@ -87,7 +89,7 @@ def linear(m: nn.Linear, x: Tensor, gelu: bool = False) -> Tensor:
     if linear_trains(m, x):
         out = ops.linear_autograd(x, m.weight, m.bias)
         return nn.functional.gelu(out) if gelu else out
-    if linear_takes(m, x) and ops.linear_pays(x.numel() // x.shape[-1], *m.weight.shape):
+    if linear_takes(m, x, gelu):
         out = ops.linear(x, m.weight, m.bias, gelu)
         if out is not None:
             return out

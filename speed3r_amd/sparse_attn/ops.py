@@ -476,11 +476,17 @@ def add_layer_norm(x: torch.Tensor, a: torch.Tensor, gamma: Optional[torch.Tenso
     return s, y
 
 
-# Where the layers leave a product to the library (us on the device, library / kernel): a long K with fewer tiles than CUs, which
-# the library splits (2 016 x 1024 x 4096 28 / 40, 4 032 x 1024 x 4096 43.5 / 43.7).  Few rows are no faster here on the device
-# (256 x 1024 x 1024 5.5 / 8.7, 1 041 9.0 / 9.2, 2 016 10.4 / 9.7) but on the host, which they wait for.
-def linear_pays(rows: int, n: int, k: int) -> bool:
-    return k <= 1024 or -(-rows // 128) * -(-n // 128) >= 256
+# Where the layers leave a product to the library (us on the device, library / kernel).  Inputs of 1024 and fewer: nowhere; few rows are no
+# faster here on the device (256 x 1024 x 1024 5.5 / 8.7, 1 041 9.0 / 9.2, 2 016 10.4 / 9.7) but on the host, which they wait for.  More
+# inputs: the library splits them where tiles are few (2 016 x 1024 x 4096 26 / 39) and reaches 1.4 to 1.5 PFLOP/s where they are many
+# (32 256 x 2048 x 8192 705 / 795, 16 128 x 1536 x 6144 230 / 244, 8 064 x 3072 x 12288 435 / 528, 8 064 x 4608 x 1536 97 / 101), except
+# where one round of 128-wide tiles, two per CU, is full (8 064 x 1024 x 4096 58 / 55, 6 000 x 1280 x 5120 69 / 67, 4 032 x 2048 x 2048 33 / 30);
+# with GELU in the epilogue there is a pass less (8 064 x 5120 x 1280 145 / 107, 2 016 x 8192 x 2048 73 / 57, 400 x 12288 x 3072 45 / 39).
+def linear_pays(rows: int, n: int, k: int, gelu: bool = False) -> bool:
+    if k <= 1024:
+        return True
+    tiles = -(-rows // 128) * -(-n // 128)
+    return tiles >= 256 if gelu else 400 < tiles <= 512
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], gelu: bool = False) -> Optional[torch.Tensor]:

@@ -50,6 +50,19 @@ def test_linear_without_inputs():
     assert torch.equal(linear(m, x), m(x)) and torch.equal(linear(m, x[:0]), m(x[:0]))
 
 
+@torch.no_grad()
+@pytest.mark.parametrize("rows,n,k,gelu,kernel", [(2016, 1024, 4096, False, False), (8064, 1024, 4096, False, True), (2016, 8192, 2048, False, False),
+                                                  (2016, 8192, 2048, True, True), (400, 1536, 1536, True, False), (1024, 1024, 1024, False, True)])
+def test_long_products_stay_with_the_library_where_it_is_faster(rows, n, k, gelu, kernel, monkeypatch):
+    calls = []
+    own = ops.linear
+    monkeypatch.setattr(ops, "linear", lambda *a: (calls.append(1), own(*a))[1])
+    m, x = nn.Linear(k, n, device=DEV, dtype=torch.bfloat16), torch.randn(rows, k, device=DEV, dtype=torch.bfloat16)
+    out, want = linear(m, x, gelu), F.gelu(m(x)) if gelu else m(x)
+    assert (len(calls) == 1) is kernel and torch.allclose(out.float(), want.float(), atol=2e-2, rtol=2e-2)
+    assert torch.equal(linear(nn.Identity(), x), x)
+
+
 def test_linear_writes_inside_its_rows_only():
     x, w = torch.randn(300, 256, device=DEV).bfloat16(), torch.randn(264, 256, device=DEV).bfloat16()
     from speed3r_amd import _lib
