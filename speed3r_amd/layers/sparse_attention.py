@@ -78,15 +78,31 @@ def linear_trains(m: nn.Linear, x: Tensor) -> bool:
         and all(t is None or t.dtype in (torch.float32, torch.bfloat16, torch.float16) for t in (x, m.weight, m.bias))
 
 
+# The function in the place of F.linear costs the host 15 us a product without autocast and 40 with it, what its kernel saves of the device
+# counts where the step waits for the device.  Multiply-adds of a product from which that is so: an MLP's (its two products, us a step, torch's /
+# here, under autocast: 8 320 rows of 768 channels 491 / 552, 12 032 697 / 568, 16 000 of 512 554 / 546, 4 160 of 1024 413 / 413, 8 320 707 / 607;
+# without: 8 320 of 512 331 / 361, 12 032 414 / 361, 4 160 of 1024 366 / 325), and an attention layer's projection, whose step has more to do on the
+# host (autocast: 12 032 rows of 1024 channels 1 170 / 1 286, 16 000 1 277 / 1 306, 24 000 1 772 / 1 445, 8 320 of 1536 1 224 / 1 324, 12 032
+# 1 631 / 1 415; without: 12 032 of 1024 975 / 829 on a fast host, 1 044 / 1 110 on another, 16 000 1 184 / 970, 16 000 of 768 1 076 / 1 094,
+# 24 000 1 450 / 1 185).
+def training_pays(x: Tensor, m: nn.Module, layer: bool) -> bool:
+    """Whether the gradients of ``m``'s parameters, those of an attention layer's projection or another product, are enough work
+    for :func:`linear_with_grad` in the place of ``m(x)``."""
+    if not sizes_are_known(x) or type(m) is not nn.Linear:
+        return False
+    work = x.numel() * m.weight.shape[0]
+    return work >= ((6e10 if layer else 2e10) if torch.is_autocast_enabled("cuda") else (4e10 if layer else 1.2e10))
+
+
 def linear_with_grad(m: nn.Linear, x: Tensor) -> Tensor:
     """``m(x)`` in training: with a kernel for the parameters' gradients where :func:`linear_trains` says so."""
     return ops.linear_autograd(x, m.weight, m.bias) if linear_trains(m, x) else m(x)
 
 
-def linear(m: nn.Linear, x: Tensor, gelu: bool = False) -> Tensor:
+def linear(m: nn.Linear, x: Tensor, gelu: bool = False, trains: Optional[bool] = None) -> Tensor:
     """``m(x)``, with ``gelu`` followed by ``F.gelu``: one kernel where :func:`linear_takes` says so, the product with a kernel for
-    the parameters' gradients where :func:`linear_trains` does, else the modules."""
-    if linear_trains(m, x):
+    the parameters' gradients where :func:`linear_trains` does (and ``trains``, where it is given), else the modules."""
+    if trains is not False and linear_trains(m, x):
         out = ops.linear_autograd(x, m.weight, m.bias)
         return nn.functional.gelu(out) if gelu else out
     if linear_takes(m, x, gelu):
@@ -235,12 +251,13 @@ class SparseFlashAttentionRope(nn.Module):
         b, n, c = x.shape
         h = self.num_heads
         block = self.block_size ** 2
-        if linear_trains(self.qkv, x) and self._plain_gate() and linear_trains(self.gate[0], x):
+        product = linear_with_grad if training_pays(x, self.qkv, layer=True) else lambda m, t: m(t)
+        if product is linear_with_grad and linear_trains(self.qkv, x) and self._plain_gate() and linear_trains(self.gate[0], x):
             x = ops.autocast_once(x)
             qkv = ops.linear_autograd(x, self.qkv.weight, self.qkv.bias)
             gate = torch.sigmoid(ops.linear_autograd(x, self.gate[0].weight, self.gate[0].bias))
         else:
-            qkv, gate = linear_with_grad(self.qkv, x), self.gate(x)
+            qkv, gate = product(self.qkv, x), self.gate(x)
         gate = gate.view(b, n, h, 2).permute(0, 2, 1, 3)                      # [B, H, N, 2]
         use_pos = xpos is not None and self.rope is not None
         fused = fused_qk_args(self, qkv, xpos if use_pos else None, n_pos, training=True)
@@ -253,12 +270,12 @@ class SparseFlashAttentionRope(nn.Module):
                 if self.keep_topk_idx:
                     self.last_topk_idx = idx
                 if len(branches) == 1:
-                    return self.proj_drop(linear_with_grad(self.proj, branches[0]))
+                    return self.proj_drop(product(self.proj, branches[0]))
         o_c, o_s = branches if branches is not None else self._branches_with_grad(qkv, xpos if use_pos else None)
         blk = torch.arange(n, device=x.device) // block
         out = gate[..., 0:1] * o_c[:, :, blk] + gate[..., 1:2] * o_s           # [B, H, N, D]
         out = out.permute(0, 2, 1, 3).reshape(b, n, c)
-        return self.proj_drop(linear_with_grad(self.proj, out))
+        return self.proj_drop(product(self.proj, out))
 
     def _branches_with_grad(self, qkv: Tensor, xpos: Optional[Tensor]):
         """Outputs of the two attention branches as a composition of torch expressions around the attention operators."""

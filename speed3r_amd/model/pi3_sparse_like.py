@@ -37,9 +37,14 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from ..layers import RoPE2D, SparseFlashAttentionRope
-from ..layers.sparse_attention import calls_forward_only, fused_qk_args, linear, norm_rope_fused_or_eager, project
+from ..layers.sparse_attention import calls_forward_only, fused_qk_args, linear, norm_rope_fused_or_eager, project, training_pays
 from ..sparse_attn import ops
 from .token_order import tile_major, tile_major_inverse
+
+
+def product(m: nn.Module, x: Tensor, gelu: bool = False, layer: bool = False) -> Tensor:
+    """``linear``, in training where the product is enough work for it (``layer``: an attention layer's projection)."""
+    return linear(m, x, gelu, trains=torch.is_grad_enabled() and training_pays(x, m, layer))
 
 
 class Mlp(nn.Module):
@@ -52,7 +57,7 @@ class Mlp(nn.Module):
         if torch.jit.is_scripting():
             return self.fc2(F.gelu(self.fc1(x)))
         else:   # (not compiled by TorchScript)
-            return linear(self.fc2, linear(self.fc1, x, gelu=True))
+            return product(self.fc2, product(self.fc1, x, gelu=True))
 
 
 class LayerScale(nn.Module):
@@ -112,7 +117,7 @@ class DenseAttentionRope(nn.Module):
         pos = xpos if self.rope is not None else None
         projected = project(self, x, pos, n_pos, 64, False) if not torch.is_grad_enabled() else None
         if projected is None:
-            qkv = linear(self.qkv, x)
+            qkv = product(self.qkv, x, layer=True)
             fused = fused_qk_args(self, qkv, pos, n_pos) if not torch.is_grad_enabled() else None
             if fused is not None and (pos is not None or fused[4] is not None):   # one pass over the projection for q and k
                 projected = ops.qkv_prepass(qkv, h, 64, *fused[:3], *fused[4:], pooled=None, inv_freq=fused[3])
@@ -125,7 +130,7 @@ class DenseAttentionRope(nn.Module):
             # the package's dense flash kernel (the compressed branch's attention), written straight into [B,N,H,D]
             o = torch.empty((b, n, h, c // h), dtype=x.dtype, device=x.device)
             ops.compressed_attn_topk(q, k, v, None, out=o.permute(0, 2, 1, 3))
-            return linear(self.proj, o.view(b, n, c))
+            return product(self.proj, o.view(b, n, c), layer=True)
         o = F.scaled_dot_product_attention(q, k, v)
         return self.proj(o.transpose(1, 2).reshape(b, n, c))
 
@@ -214,7 +219,7 @@ class HeadDecoder(nn.Module):
         self.linear_out = nn.Linear(dim, out_dim)
 
     def forward(self, x: Tensor, xpos: Tensor, n_pos: Optional[int] = None) -> Tensor:
-        return linear(self.linear_out, run_blocks(self.blocks, linear(self.project, x), None, xpos=xpos, n_pos=n_pos)[0])
+        return product(self.linear_out, run_blocks(self.blocks, product(self.project, x), None, xpos=xpos, n_pos=n_pos)[0])
 
 
 class PixelShuffleHead(nn.Module):

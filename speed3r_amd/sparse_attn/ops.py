@@ -526,8 +526,8 @@ def ordinary(x: torch.Tensor) -> bool:
         and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
 
 
-# Gradients of weight and bias, kernel / library, us on the device: 2 048 rows x 3072 x 1024 36 / 43, x 1024 x 1024 29 / 33 (no
-# faster with their launches), 4 096 rows 42 / 61 and 32 / 48, 24 192 rows 130 / 279 and 62 / 206.
+# Gradients of weight and bias, kernel / library, us on the device: 2 048 rows x 3072 x 1024 36 / 44, x 1024 x 1024 30 / 30 (no
+# faster with their launches), 4 096 rows 42 / 64 and 32 / 50, 24 000 rows 125 / 262 and 61 / 185.
 def linear_wgrad_pays(rows: int) -> bool:
     return rows >= 4096
 
@@ -570,7 +570,9 @@ class _LinearFn(torch.autograd.Function):
 def _cast(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """``t`` as autocast hands it to a product: the copy that it keeps for a leaf in this region, else a new one.  (Autocast casts
     the operands of einsum too; of one operand in its own order einsum makes a view.)"""
-    return t if t is None or t.dtype == torch.get_autocast_dtype("cuda") else torch.einsum("...i->...i", t)
+    if t is None or t.dtype == torch.get_autocast_dtype("cuda"):
+        return t
+    return torch.einsum("...i->...i", t) if t.is_leaf and t.requires_grad else t.to(torch.get_autocast_dtype("cuda"))
 
 
 def autocast_once(x: torch.Tensor) -> torch.Tensor:

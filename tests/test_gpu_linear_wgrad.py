@@ -6,6 +6,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from speed3r_amd.layers.sparse_attention import linear, linear_trains
+from speed3r_amd.model.pi3_sparse_like import Mlp
 from speed3r_amd.sparse_attn import ops
 
 DEV = "cuda"
@@ -180,3 +181,15 @@ def test_weights_of_few_inputs_train_through_the_kernel(c, bias, monkeypatch):
 @pytest.mark.parametrize("n,c", [(60, 1024), (64, 100)])
 def test_weights_without_a_kernel_keep_their_graph(n, c):
     assert not linear_trains(nn.Linear(c, n, device=DEV, dtype=torch.bfloat16), torch.randn(ROWS, c, device=DEV).bfloat16())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,c,autocast,kernel", [(ROWS, 512, False, False), (16000, 512, False, True), (8320, 768, True, False), (12032, 768, True, True)])
+def test_small_steps_keep_the_products_of_torch(rows, c, autocast, kernel, monkeypatch):
+    calls = []
+    own = ops.linear_autograd
+    monkeypatch.setattr(ops, "linear_autograd", lambda *a: (calls.append(1), own(*a))[1])
+    m = Mlp(c, 4 * c).to(DEV, torch.float32 if autocast else torch.bfloat16)
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        m(torch.randn(rows, c, device=DEV, dtype=m.fc1.weight.dtype)).float().sum().backward()
+    assert len(calls) == (2 if kernel else 0) and all(p.grad is not None for p in m.parameters())
