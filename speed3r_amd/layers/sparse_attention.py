@@ -116,9 +116,11 @@ def project(attn: nn.Module, x: Tensor, pos: Optional[Tensor], n_pos: Optional[i
     """The projection of an attention layer with all that follows it row by row, and the layer's gate (weight, bias) beside it
     (``ops.qkv_project``), or None where the kernel does not take the layer or does not stand in for its modules (then:
     ``linear`` and the passes over its result)."""
-    if pos is None or not linear_takes(attn.qkv, x) or pos.is_floating_point():
+    # (asked before the tables are, which the passes over the projection ask for again and a rope of another kind looks at the positions for)
+    if pos is None or not linear_takes(attn.qkv, x) or pos.is_floating_point() or x.dim() != 3 \
+            or not ops.qkv_project_takes(x, attn.num_heads, block, pooled, isinstance(attn.q_norm, nn.LayerNorm)):
         return None
-    fused = fused_qk_args(attn, x, pos, n_pos, takes=x.dim() == 3 and x.shape[-1] == 64 * attn.num_heads)
+    fused = fused_qk_args(attn, x, pos, n_pos, takes=True)
     if fused is None or fused[0].shape != (*x.shape[:2], 2):
         return None
     return ops.qkv_project(x, attn.qkv.weight, attn.qkv.bias, attn.num_heads, block, *fused[:3], *fused[4:], pooled=pooled, inv_freq=fused[3],

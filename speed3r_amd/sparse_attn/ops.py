@@ -616,6 +616,14 @@ def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, bias: bool):
     return dw, db
 
 
+def qkv_project_takes(x: torch.Tensor, num_heads: int, block: int, pooled: bool, norms: bool) -> bool:
+    """Whether the library has a kernel for :func:`qkv_project` of these tokens (``norms``: with them)."""
+    b, n, c = x.shape
+    return x.dtype in (torch.bfloat16, torch.float16) and c == 64 * num_heads and num_heads % 2 == 0 and 0 < c <= 1 << 18 and 0 < b * n <= 1 << 30 \
+        and x.is_contiguous() and (not pooled or (norms and block in (16, 64))) \
+        and (b == 1 or (n >= 256 and num_heads * n * 128 <= 0x70000000 and not (pooled and n % block)))
+
+
 def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], num_heads: int, block: int, positions: torch.Tensor,
                 cos_tab: torch.Tensor, sin_tab: torch.Tensor, q_ln=None, k_ln=None, eps: float = 1e-5, *, pooled: bool,
                 inv_freq: Optional[torch.Tensor] = None, gate: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None):
@@ -625,7 +633,7 @@ def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     :func:`gate`, whose result ``[B,N,O]`` is then the last one, or None where its outputs are not a multiple of 4 up to 32 or
     the kernel has no idle time for it.
 
-    Returns None where the library has no kernel: bf16/fp16, head_dim 64, an even number of heads, contiguous 16-byte
+    Returns None where the library has no kernel (:func:`qkv_project_takes`): bf16/fp16, head_dim 64, an even number of heads, contiguous 16-byte
     aligned tensors of one dtype; means with norms and over blocks of 16 or 64 tokens only; several sequences of 256 tokens or
     more each, with means a multiple of the block."""
     _need_device(x)
@@ -633,12 +641,9 @@ def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     b, n, c = x.shape
     h = num_heads
     ts = [t for t in (x, weight, bias) if t is not None]
-    if x.dtype not in (torch.bfloat16, torch.float16) or c != 64 * h or h % 2 or c > 1 << 18 or x.numel() == 0 or b * n > 1 << 30 \
-            or weight.shape != (3 * c, c) or (bias is not None and bias.shape != (3 * c,)):
+    if not qkv_project_takes(x, h, block, pooled, q_ln is not None) or weight.shape != (3 * c, c) or (bias is not None and bias.shape != (3 * c,)):
         return None
     if any(t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
-        return None
-    if pooled and (q_ln is None or block not in (16, 64)) or b > 1 and (n < 256 or h * n * 128 > 0x70000000 or pooled and n % block):
         return None
     a, keep = _prepass_args(x, h, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq)
     q, k, v = x.new_empty((3, b, h, n, 64)).unbind(0)

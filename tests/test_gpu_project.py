@@ -5,7 +5,7 @@ import torch
 import torch.nn.functional as F
 
 from speed3r_amd import _lib
-from speed3r_amd.layers import RoPE2D
+from speed3r_amd.layers import RoPE2D, SparseFlashAttentionRope
 from speed3r_amd.sparse_attn import ops
 
 pytestmark = pytest.mark.gpu
@@ -153,3 +153,19 @@ def test_project_refuses_what_it_is_not_built_for():
     x, w, bias, pos, ln = _case(1, 64, 2, torch.bfloat16)
     assert ops.qkv_project(x, w, bias, 2, 64, pos, cos, sin, None, None, pooled=True) is None
     assert ops.qkv_project(x, w, bias.float(), 2, 64, pos, cos, sin, *ln, 1e-6, pooled=True) is None
+
+
+@pytest.mark.parametrize("heads,block_size,norm", [(3, 4, True), (4, 16, True), (4, 8, False), (4, 8, True)])
+def test_layers_lay_out_tables_once(heads, block_size, norm):
+    class Rope(RoPE2D):
+        asked = 0
+
+        def fused_tables(self, *args, **kwargs):
+            self.asked += 1
+            return super().fused_tables(*args, **kwargs)
+
+    c, rope = 64 * heads, Rope(100.0)
+    layer = SparseFlashAttentionRope(c, num_heads=heads, qk_norm=norm, rope=rope, block_size=block_size, topk=2).to(DEV, torch.bfloat16)
+    with torch.no_grad():
+        layer(torch.randn(1, 2048, c, device=DEV).bfloat16(), xpos=torch.randint(0, 30, (1, 2048, 2), device=DEV), n_pos=40)
+    assert rope.asked == 1
