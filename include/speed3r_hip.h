@@ -328,7 +328,8 @@ int s3r_linear_wgrad(const void* dy, const void* x, void* dw, void* db, float* w
  * q and k after LayerNorm and RoPE2D, v, and the finished block means (sparse_attention.py:93-110,115-124).
  *   x: [B*N, C] rows of stride ldx, w: [3*C, C] of stride ldw, bias: [3*C] or NULL, C = 64 H; v_out: contiguous [B,H,N,64];
  *   a: as for s3r_layer_prepass (q, k, v and the strides are not read): q_out, k_out, positions and tables are required,
- *   the three means and the norms optional; means only with norms, `finish_pooled` and without q_raw, k_raw.
+ *   the three means and the norms optional; means only with norms, `finish_pooled` and without q_raw, k_raw; not with inv_freq and
+ *   signed_positions.
  * bf16 / fp16, an even number of heads, block 16 or 64; several sequences: 256 tokens or more each, with means a multiple of
  * the block.  gate_out (or NULL): [B*N, gate_outputs], what s3r_gate gives for x, gate_w ([gate_outputs, C]) and gate_bias (or
  * NULL); a multiple of 4 outputs up to 32.  Rounding: the projection to the I/O dtype, then once at the end (s3r_layer_prepass also rounds in between).

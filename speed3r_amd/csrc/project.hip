@@ -539,6 +539,8 @@ extern "C" int s3r_qkv_project(const void* x, const void* w, const void* bias, i
   if ((a->dtype != S3R_BF16 && a->dtype != S3R_F16) || a->head_dim != 64 || C % 128 || C > (1 << 20) / 3 || M > (1 << 30))
     return fail(S3R_ERR_UNSUPPORTED, "s3r_qkv_project: dtype %d, head_dim %d, %d heads, %lld rows (built for 16-bit types, head_dim 64, an even "
                 "number of heads)", a->dtype, a->head_dim, a->H, (long long)M);
+  if (a->inv_freq != nullptr && a->signed_positions)
+    return fail(S3R_ERR_UNSUPPORTED, "s3r_qkv_project: angles of their own for positions below zero (built for positions that are clamped to zero)");
   // a tile of rows reaches into one more sequence at most; its rows are addressed by 32-bit byte offsets
   if (a->B > 1 && (a->N < 256 || (int64_t)a->H * a->N * 128 > 0x70000000LL))
     return fail(S3R_ERR_UNSUPPORTED, "s3r_qkv_project: %d sequences of %lld tokens (built for 256 tokens or more each)", a->B, (long long)a->N);
@@ -548,7 +550,7 @@ extern "C" int s3r_qkv_project(const void* x, const void* w, const void* bias, i
                 "that end with each sequence of a batch)", a->block);
   if (ldx < C || ldw < C || ldx >= (1 << 21) || ldw >= (1 << 21))
     return fail(S3R_ERR_BAD_ARG, "s3r_qkv_project: rows overlap or lie 2^21 elements or more apart");
-  const void* ptrs[] = {x, w, a->q_out, a->k_out, v_out, a->q_pool, a->k_pool, a->v_pool};
+  const void* ptrs[] = {x, w, a->q_out, a->k_out, v_out, a->q_pool, a->k_pool, a->v_pool, a->cos_table, a->sin_table};
   for (const void* ptr : ptrs)
     if (!aligned16(ptr)) return fail(S3R_ERR_BAD_ARG, "s3r_qkv_project: pointers must be multiples of 16 bytes");
   if (ldx % 8 || ldw % 8 || (reinterpret_cast<uintptr_t>(bias) & 7u))

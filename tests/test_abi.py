@@ -90,6 +90,23 @@ def test_backward_entry_points_validate_on_the_host():
     assert b"s3r_key_block_lists" in L.s3r_last_error()
 
 
+def test_projection_refuses_on_the_host():
+    L = _lib.lib()
+    one = ctypes.c_void_p(16)   # (never dereferenced: every call here is refused)
+
+    def project(**fields):
+        a = _lib.PrepassArgs(q_out=16, k_out=16, positions=16, cos_table=16, sin_table=16, inv_freq=16, N=64, pos_stride_b=128, pos_stride_n=2, B=1, H=2,
+                             head_dim=64, block=64, table_rows=40, dtype=_lib.S3R_BF16, eps=1e-6)
+        for name, value in fields.items():
+            setattr(a, name, value)
+        return L.s3r_qkv_project(one, one, None, 128, 128, one, ctypes.byref(a), None, None, None, 0, None)
+
+    assert project(signed_positions=1) == _lib.S3R_ERR_UNSUPPORTED   # angles of their own below zero are the pass's
+    assert b"below zero" in L.s3r_last_error()
+    assert project(cos_table=24) == _lib.S3R_ERR_BAD_ARG and project(sin_table=24) == _lib.S3R_ERR_BAD_ARG
+    assert project(H=3) == _lib.S3R_ERR_UNSUPPORTED and project(k_out=None) == _lib.S3R_ERR_BAD_ARG
+
+
 def test_operators_refuse_cpu_tensors():
     import speed3r_amd as s3r
 
