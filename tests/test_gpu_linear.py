@@ -63,6 +63,15 @@ def test_long_products_stay_with_the_library_where_it_is_faster(rows, n, k, gelu
     assert torch.equal(linear(nn.Identity(), x), x)
 
 
+def test_linear_beyond_two_to_the_31():
+    """x beyond 2^31 bytes, y beyond 2^31 values: the same bits as pieces of it (which test_linear_matches_float64 checks)."""
+    m, n, k = 1100001, 3072, 1024
+    x, w, b = torch.randn(m, k, device=DEV, dtype=torch.bfloat16), torch.randn(n, k, device=DEV, dtype=torch.bfloat16), torch.randn(n, device=DEV, dtype=torch.bfloat16)
+    y = ops.linear(x, w, b)
+    for at in (0, 2 ** 31 // n - 100, 2 ** 31 // (2 * k) - 100, 2 ** 32 // (2 * n) - 100, m - 200):
+        assert torch.equal(y[at:at + 200], ops.linear(x[at:at + 200], w, b)), at
+
+
 def test_linear_writes_inside_its_rows_only():
     x, w = torch.randn(300, 256, device=DEV).bfloat16(), torch.randn(264, 256, device=DEV).bfloat16()
     from speed3r_amd import _lib

@@ -72,6 +72,23 @@ def test_wgrad_takes_its_rows_only(m):
 
 
 @pytest.mark.gpu
+def test_wgrad_beyond_two_to_the_31():
+    m, n, c = 1100001, 64, 1032   # x beyond 2^31 bytes
+    gen = torch.Generator(device=DEV).manual_seed(0)
+    dy, x = torch.randn(m, n, generator=gen, device=DEV, dtype=torch.bfloat16), torch.randn(m, c, generator=gen, device=DEV, dtype=torch.bfloat16)
+    dw, db = ops.linear_wgrad(dy, x, True)
+    want, mag = torch.zeros(n, c, device=DEV, dtype=torch.float64), torch.zeros(n, c, device=DEV, dtype=torch.float64)
+    for a, b in zip(dy.split(100000), x.split(100000)):
+        want += a.double().t() @ b.double()
+        mag += a.double().abs().t() @ b.double().abs()
+    # half a bf16 step of the value; an fp32 rounding of the sum of magnitudes per 16 tokens of one of 64 ranges, and per range (what a
+    # tenth of the tokens adds is some 300)
+    chain = (m / 64 / 16 + 64) * 2.0 ** -24
+    assert ((dw.double() - want).abs() <= 2.0 ** -8 * want.abs() * 1.01 + chain * mag).all() and (chain * mag).max() < 100
+    assert ((db.double() - dy.double().sum(0)).abs() <= 2.0 ** -8 * dy.double().sum(0).abs() * 1.01 + chain * dy.double().abs().sum(0)).all()
+
+
+@pytest.mark.gpu
 def test_wgrad_refuses_what_it_is_not_built_for():
     x, dy = torch.randn(256, 512, device=DEV).bfloat16(), torch.randn(256, 64, device=DEV).bfloat16()
     assert ops.linear_wgrad(dy, x, True) is None                       # sums of dY with few inputs

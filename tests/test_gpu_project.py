@@ -169,3 +169,42 @@ def test_layers_lay_out_tables_once(heads, block_size, norm):
     with torch.no_grad():
         layer(torch.randn(1, 2048, c, device=DEV).bfloat16(), xpos=torch.randint(0, 30, (1, 2048, 2), device=DEV), n_pos=40)
     assert rope.asked == 1
+
+
+# several sequences whose borders lie inside tiles of 128 and of 256 tokens (then with two heads a wave), at any row where there are no
+# means; the sizes take the large tile where the second number says so
+@pytest.mark.parametrize("b,n,h,pooled,block", [(3, 1041, 2, False, 64), (8, 1041, 16, False, 64), (5, 257, 2, False, 64), (2, 2576, 16, True, 16), (2, 2624, 16, True, 64),
+                                                (3, 272, 2, True, 16)])
+def test_project_across_the_borders_of_sequences(b, n, h, pooled, block):
+    x, w, bias, pos, ln = _case(b, n, h, torch.bfloat16, seed=n)
+    rope = RoPE2D(100.0)
+    cos, sin, inv_freq = rope.fused_tables(64, None, x.device, x.dtype, bounded=True)
+    near = pos.clone()
+    for i in range(b):   # on both sides of a border: beyond the staged rows, beyond the tables, below zero
+        pos[i, 0], pos[i, 1], pos[i, n - 1], pos[i, n - 2], pos[i, n // 2] = (torch.tensor(p) for p in ([70, 3], [5, 100000], [2, 90], [100001, 66], [-3, 4]))
+    for p in (near, pos):
+        got = ops.qkv_project(x, w, bias, h, block, p, cos, sin, *ln, 1e-6, pooled=pooled, inv_freq=inv_freq)
+        for i in range(b):   # each sequence on its own: no border, the same sums
+            one = ops.qkv_project(x[i:i + 1], w, bias, h, block, p[i:i + 1], cos, sin, *ln, 1e-6, pooled=pooled, inv_freq=inv_freq)
+            assert all(torch.equal(g[i:i + 1], e) for g, e in zip(got, one))
+    tok, means = _want(x, w, bias, near, ln, h, block, rope, 40)
+    got = ops.qkv_project(x, w, bias, h, block, near, cos, sin, *ln, 1e-6, pooled=pooled, inv_freq=inv_freq)
+    for name, g, e in zip("q k v qc kc vc".split(), got, tok + means):   # bounds: test_project_matches_float64
+        assert ((g.double() - e).abs() <= 2.0 ** -7 * (0.5 * e.abs() + 8 * (1 + e.abs()))).all(), name
+
+
+@pytest.mark.parametrize("b,n", [(1, 1100032), (2, 600064)])
+def test_project_beyond_two_to_the_31(b, n):
+    """x and every output beyond 2^31 bytes, all outputs together beyond 2^31 values: the same bits as pieces of it."""
+    h, block = 16, 64
+    x, w, bias, _, ln = _case(b, 64, h, torch.bfloat16)
+    x = x.repeat(1, n // 64, 1).add_(torch.arange(n, device=DEV)[None, :, None] % 251 / 251)
+    pos = torch.randint(0, 40, (b, n, 2), device=DEV)
+    cos, sin = RoPE2D(100.0).tables(64, 40, x.device, x.dtype)
+    got = ops.qkv_project(x, w, bias, h, block, pos, cos, sin, *ln, 1e-6, pooled=True)
+    for i in range(b):
+        for at in (0, n // 128 * 64, 2 ** 31 // 2048 - 128 if b == 1 else 2 ** 31 // 4096, n - 320):
+            one = ops.qkv_project(x[i:i + 1, at:at + 320].contiguous(), w, bias, h, block, pos[i:i + 1, at:at + 320], cos, sin, *ln, 1e-6, pooled=True)
+            for g, e in zip(got, one):
+                part = g[i:i + 1, :, at:at + 320] if g.shape[2] == n else g[i:i + 1, :, at // block:(at + 320) // block]
+                assert torch.equal(part, e), (i, at)
