@@ -38,14 +38,9 @@ def calls_forward_only(m: nn.Module, kind: type) -> bool:
         or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks)
 
 
-def takes_kernels(x: Tensor) -> bool:
-    """Whether a call on ``x`` is an ordinary one (:func:`ops.ordinary`), without autocast."""
-    return not torch.is_autocast_enabled("cuda") and ops.ordinary(x)
-
-
 def sizes_are_known(x: Tensor) -> bool:
     """Whether the sizes of ``x`` may choose a path: not where a call is traced, compiled or exported for any sizes."""
-    return type(x) is Tensor and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+    return type(x) is Tensor and not torch.compiler.is_compiling() and not torch._C._is_tracing()
 
 
 # Calls with less work keep torch's products and the passes over them.  A layer of few rows is bound by the host: 400 to 1 020 tokens of
@@ -60,7 +55,7 @@ def linear_takes(m: nn.Linear, x: Tensor, gelu: Optional[bool] = None) -> bool:
     where ``ops.linear`` with it or without is the faster one."""
     return sizes_are_known(x) and enough_work(x) and type(m) is nn.Linear \
         and (gelu is None or ops.linear_pays(x.numel() // x.shape[-1], *m.weight.shape, gelu)) and calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter \
-        and x.shape[-1] == m.weight.shape[1] and takes_kernels(x) \
+        and x.shape[-1] == m.weight.shape[1] and not torch.is_autocast_enabled("cuda") and ops.unchanged_here(x) \
         and not (torch.is_grad_enabled() and (x.requires_grad or m.weight.requires_grad or (m.bias is not None and m.bias.requires_grad)))
 
 
@@ -74,7 +69,7 @@ def linear_trains(m: nn.Linear, x: Tensor) -> bool:
     return calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter and m.weight.requires_grad \
         and dtype in (torch.bfloat16, torch.float16) and x.shape[-1] == m.weight.shape[1] \
         and ops.linear_wgrad_takes(*m.weight.shape) \
-        and ops.ordinary(x) \
+        and ops.unchanged_here(x) \
         and all(t is None or t.dtype in (torch.float32, torch.bfloat16, torch.float16) for t in (x, m.weight, m.bias))
 
 
@@ -124,7 +119,7 @@ def project(attn: nn.Module, x: Tensor, pos: Optional[Tensor], n_pos: Optional[i
     if fused is None or fused[0].shape != (*x.shape[:2], 2):
         return None
     return ops.qkv_project(x, attn.qkv.weight, attn.qkv.bias, attn.num_heads, block, *fused[:3], *fused[4:], pooled=pooled, inv_freq=fused[3],
-                           gate=gate)
+                           gate=gate, takes=True)
 
 
 def norm_rope_fused_or_eager(t: Tensor, norm: nn.Module, rope, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:

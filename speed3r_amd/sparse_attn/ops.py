@@ -497,12 +497,12 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     _need_device(x)
     _forward_only(x, weight)
     k, n = x.shape[-1], weight.shape[0]
-    ts = [t for t in (x, weight, bias) if t is not None]
     if x.dtype not in (torch.bfloat16, torch.float16) or k % 128 or n % 8 or x.numel() == 0 or weight.shape != (n, k) or k > 1 << 20 or n > 1 << 20 \
             or (bias is not None and bias.shape != (n,)):
         return None
-    if any(t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
-        return None
+    for t in (x, weight, bias):
+        if t is not None and (t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16):
+            return None
     out = x.new_empty((*x.shape[:-1], n))
     with _on(x.device):
         rc = _lib.lib().s3r_linear(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
@@ -511,19 +511,20 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     return out
 
 
-def _seen_by_modes() -> bool:
-    """Whether a mode (``make_fx``, flop counters, selective checkpointing, function modes) is to see the torch operations;
-    ``torch.device`` as a context and the default device concern factory functions only."""
-    return torch._C._len_torch_dispatch_stack() > 0 or any(
-        type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+def unchanged_here(x: torch.Tensor) -> bool:
+    """Whether a call on ``x`` is seen by nobody but torch itself: a tensor on the GPU, without a transform (vmap, forward-mode
+    derivatives) or a mode (``make_fx``, flop counters, selective checkpointing, function modes) that has to see the torch
+    operations; ``torch.device`` as a context and the default device concern factory functions only."""
+    c = torch._C
+    return x.is_cuda and c._len_torch_dispatch_stack() == 0 and c._functorch.peek_interpreter_stack() is None \
+        and c._has_storage(x) and torch.autograd.forward_ad._current_level < 0 \
+        and (c._len_torch_function_stack() == 0
+             or all(type(c._get_function_stack_at(i)) is DeviceContext for i in range(c._len_torch_function_stack())))
 
 
 def ordinary(x: torch.Tensor) -> bool:
-    """Whether a call on ``x`` is an ordinary one: a tensor on the GPU, without tracing, compilation, a mode or a transform (vmap,
-    forward-mode derivatives) that has to see the torch operations."""
-    return x.is_cuda and not _seen_by_modes() and type(x) is torch.Tensor and torch._C._functorch.peek_interpreter_stack() is None \
-        and torch._C._has_storage(x) and torch.autograd.forward_ad._current_level < 0 \
-        and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+    """Whether a call on ``x`` is an ordinary one: :func:`unchanged_here`, and neither traced nor compiled."""
+    return type(x) is torch.Tensor and unchanged_here(x) and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
 
 
 # Gradients of weight and bias, kernel / library, us on the device: 2 048 rows x 3072 x 1024 36 / 44, x 1024 x 1024 30 / 30 (no
@@ -626,12 +627,12 @@ def qkv_project_takes(x: torch.Tensor, num_heads: int, block: int, pooled: bool,
 
 def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], num_heads: int, block: int, positions: torch.Tensor,
                 cos_tab: torch.Tensor, sin_tab: torch.Tensor, q_ln=None, k_ln=None, eps: float = 1e-5, *, pooled: bool,
-                inv_freq: Optional[torch.Tensor] = None, gate: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None):
+                inv_freq: Optional[torch.Tensor] = None, gate: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None, takes: Optional[bool] = None):
     """:func:`linear` with the weights of the packed projection and :func:`qkv_prepass` of its result (``pooled``: with
     ``pooled="final"``, else without means) in one kernel: ``(q, k, v[, q_c, k_c, v_c][, gates])``, all contiguous.  The projection
     is rounded, then once at the end (the pass rounds after the norm and inside the rotation too).  ``gate``: (weight, bias) of
     :func:`gate`, whose result ``[B,N,O]`` is then the last one, or None where its outputs are not a multiple of 4 up to 32 or
-    the kernel has no idle time for it.
+    the kernel has no idle time for it.  ``takes``: what :func:`qkv_project_takes` says, where the caller has asked.
 
     Returns None where the library has no kernel (:func:`qkv_project_takes`): bf16/fp16, head_dim 64, an even number of heads, contiguous 16-byte
     aligned tensors of one dtype; means with norms and over blocks of 16 or 64 tokens only; several sequences of 256 tokens or
@@ -640,11 +641,11 @@ def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     _forward_only(x, weight)
     b, n, c = x.shape
     h = num_heads
-    ts = [t for t in (x, weight, bias) if t is not None]
-    if not qkv_project_takes(x, h, block, pooled, q_ln is not None) or weight.shape != (3 * c, c) or (bias is not None and bias.shape != (3 * c,)):
+    if not (qkv_project_takes(x, h, block, pooled, q_ln is not None) if takes is None else takes) or weight.shape != (3 * c, c) or (bias is not None and bias.shape != (3 * c,)):
         return None
-    if any(t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
-        return None
+    for t in (x, weight, bias):
+        if t is not None and (t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16):
+            return None
     a, keep = _prepass_args(x, h, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq)
     q, k, v = x.new_empty((3, b, h, n, 64)).unbind(0)
     a.q_out, a.k_out = q.data_ptr(), k.data_ptr()
