@@ -16,7 +16,9 @@
 // (the pass rounds after the norm and after each product of the rotation as well).  The means keep the pass's points.
 //
 // Bound: the matrix cores inside the sweep over K; behind it about 280 vector instructions per 16 tokens and head of q or k
-// with one wave per SIMD, 30 % of the time of a 256 x 256 tile at K = 1024.  Tried without gain: fp32 tables in LDS instead of
+// with one wave per SIMD, 30 % of the time of a 256 x 256 tile at K = 1024.  The registers are full: the 256-wide instances spill 112 to 120
+// scalar registers to lanes of vector registers with means, 62 to 72 without, and none to 4 vector registers to memory; the 128-wide
+// ones 42 to 66 scalar ones, fp16 with 64-token means 2 vector ones.  Tried without gain: fp32 tables in LDS instead of
 // packed pairs (16 instructions less, 4 % slower), both heads of a wave in one pass, 128 x 128 tiles throughout (809 against 742).
 #include "linear_tile.h"
 #include "prepass.h"
@@ -171,8 +173,8 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
       const int wr = tl.wm * WROWS, c16 = lane & 15, g4 = lane >> 4;
       auto row_offset = [&](int row) { return (uint32_t)row * 128u + (row >= cross ? jump : 0u); };
       const int2* const pos = &lpos[par][wr];
-      // Rare: some token of the tile lies outside of the staged rows.  The pairs of all the wave's tokens then go through memory: 64
-      // pairs are a row's 128 bytes, and they take the rows that the results of its last head overwrite, group by group, each
+      // Rare: some token of the tile lies outside of the staged rows.  The pairs of all the wave's tokens then go through memory: 32
+      // pairs of four bytes are a row's 128, and they take the rows that the results of its last head overwrite, group by group, each
       // after its pairs have been read.
       bool far = false;
       char* const scratch = reinterpret_cast<char*>(out + (int64_t)(HD - 1) * p.N * 64);

@@ -2,12 +2,12 @@
 // of 16 query rows against all keys stay in LDS, and a row is selected by one wave that sees all of it.
 //
 // The two-sweep kernel (compressed_mfma.hip) meets at a barrier per 64 keys and folds queues of survivors into register lists;
-// with few tiles its chains of barriers, LDS round trips and folds are all there is (63 tiles, top-32: 124 us, 2 % of the
-// matrix rate).  Here:
+// with few tiles its chains of barriers, LDS round trips and folds are all there is (1 041 keys, 33 tiles of 32, 16 heads, top-32, alone
+// on the chip: 61 us, 3 % of the matrix rate).  Here:
 //   * Scores: S^T = K Q^T with v_mfma_f32_32x32x16 as there, same operands in the same order, so the scores are the same bits.  A
 //     workgroup has 16 rows, so half of the 32 query columns repeat the other half: the products are a fiftieth of the work.  The
-//     eight waves share the key tiles; operands come straight from memory (each is used once per workgroup), four tiles in
-//     flight per wave.
+//     eight waves share the key tiles; all of a wave's keys, up to five tiles, are on their way at once and go through the columns of
+//     LDS that the scores will fill into operand order (each is used once per workgroup).
 //   * Selection: a wave reads a row, 4 neighbouring columns per lane and 256-column piece, into registers.  The K-th largest of
 //     256 group maxima (a lane's four columns modulo 4: neighbours in different groups, since large scores come in runs; the lanes
 //     turned from piece to piece, since they come at one place of every frame of a still scene) is a
@@ -20,8 +20,9 @@
 // Order, fillers and NaN as in the two-sweep kernel: descending (sortable score, lowest column first), NaN never chosen, Lk - 1
 // in slots that nothing fills.
 //
-// us on the device, two-sweep kernel / this, 16 heads, as many rows as keys: 126 keys, top-32 16 / 8; 504, top-32 40 / 13; 1 041,
-// top-16 46 / 35; 1 200, top-32 66 / 39.  Bound: the vector instructions of the selection, about 700 per row at 1 041 keys.
+// us alone on the chip, two-sweep kernel / this, 16 heads, as many rows as keys: 126 keys, top-32 16 / 8; 504, top-32 40 / 13; 1 041,
+// top-16 46 / 34; 1 200, top-32 66 / 38.  Bound: the vector instructions of the selection, about 700 per row at 1 041 keys.  The instance of
+// five pieces spills 20 scalar registers to lanes of vector registers, the others none.
 //
 // Up to kMostKeys keys two workgroups fit a CU (78 KB each).  With more keys one does, and the two phases have nobody to hide
 // behind: 2 016 keys, top-32, 95 / 112.  With more than kMostGroups workgroups the two-sweep kernel, which shares its key tiles

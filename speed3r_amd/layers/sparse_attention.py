@@ -44,7 +44,9 @@ def sizes_are_known(x: Tensor) -> bool:
 
 
 # Calls with less work keep torch's products and the passes over them.  A layer of few rows is bound by the host: 400 to 1 020 tokens of
-# 1024 channels take 162 us with those, 137 with the projection in one launch, 126 with both products here (2 016 tokens: 180 / 126).
+# 1024 channels take 162 us with those, 137 with the projection in one launch, 126 with both products here (2 016 tokens: 180 / 126).  Other
+# widths, with those / here, 16-token blocks: 1 024 tokens of 128 channels 201 / 129, 512 of 768 177 / 130, 272 to 1 024 of 2048 199 / 178; the
+# kernels alone 70 / 55, 76 / 68, 91 / 90 to 119 / 107.
 def enough_work(x: Tensor) -> bool:
     return x.numel() >= max(1, min(1024 * x.shape[-1], 384 * 1024))
 
@@ -219,7 +221,8 @@ class SparseFlashAttentionRope(nn.Module):
         self.keep_topk_idx = False   # debugging aid: keep the last forward's block indices in ``last_topk_idx``
         self.last_topk_idx = None
         self.last_prepass = None     # whether the last forward took q, k and the block means from one launch over the packed projection
-        self.last_passes = None      # its launches over the projection: 1, 2 (block means, then q and k) or 0 (kernels per tensor)
+        self.last_passes = None      # the launches that made these: 1 (a pass over the projection, or the projection's own kernel), 2 (block
+                                     # means, then q and k) or 0 (kernels per tensor)
         self.last_path = None        # which route the last forward took: "fused-merge", "two-operators" or "autograd"
 
     def _norm_rope(self, t: Tensor, norm: nn.Module, pos: Optional[Tensor], n_pos: Optional[int] = None) -> Tensor:
