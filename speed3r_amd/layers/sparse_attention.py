@@ -38,6 +38,9 @@ def calls_forward_only(m: nn.Module, kind: type) -> bool:
         or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks)
 
 
+LINEAR_FORWARD = nn.Linear.forward   # what the kernels stand in for: not a forward that was put in its place for all layers
+
+
 def sizes_are_known(x: Tensor) -> bool:
     """Whether the sizes of ``x`` may choose a path: not where a call is traced, compiled or exported for any sizes."""
     return type(x) is Tensor and not torch.compiler.is_compiling() and not torch._C._is_tracing()
@@ -56,7 +59,8 @@ def linear_takes(m: nn.Linear, x: Tensor, gelu: Optional[bool] = None) -> bool:
     ``nn.Linear.forward`` and nothing else, on enough rows (asked first: few rows wait for the host) and, unless ``gelu`` is None,
     where ``ops.linear`` with it or without is the faster one."""
     return sizes_are_known(x) and enough_work(x) and type(m) is nn.Linear \
-        and (gelu is None or ops.linear_pays(x.numel() // x.shape[-1], *m.weight.shape, gelu)) and calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter \
+        and (gelu is None or ops.linear_pays(x.numel() // x.shape[-1], *m.weight.shape, gelu)) \
+        and calls_forward_only(m, nn.Linear) and nn.Linear.forward is LINEAR_FORWARD and type(m.weight) is nn.Parameter \
         and x.shape[-1] == m.weight.shape[1] and not torch.is_autocast_enabled("cuda") and ops.unchanged_here(x) \
         and not (torch.is_grad_enabled() and (x.requires_grad or m.weight.requires_grad or (m.bias is not None and m.bias.requires_grad)))
 
@@ -65,10 +69,11 @@ def linear_trains(m: nn.Linear, x: Tensor) -> bool:
     """Whether ``ops.linear_autograd`` may stand in for ``m(x)``: an ordinary call, with or without autocast, in a 16-bit type, of
     a module that would run ``nn.Linear.forward`` and nothing else, on so many rows that the kernel for the weight's gradient
     is the faster one."""
-    if not torch.is_grad_enabled() or not sizes_are_known(x) or not ops.linear_wgrad_pays(x.numel() // max(x.shape[-1], 1)):   # (first: few rows wait for the host)
+    # (first: few rows wait for the host)
+    if not torch.is_grad_enabled() or not sizes_are_known(x) or not ops.linear_wgrad_pays(x.numel() // max(x.shape[-1], 1)):
         return False
     dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
-    return calls_forward_only(m, nn.Linear) and type(m.weight) is nn.Parameter and m.weight.requires_grad \
+    return calls_forward_only(m, nn.Linear) and nn.Linear.forward is LINEAR_FORWARD and type(m.weight) is nn.Parameter and m.weight.requires_grad \
         and dtype in (torch.bfloat16, torch.float16) and x.shape[-1] == m.weight.shape[1] \
         and ops.linear_wgrad_takes(*m.weight.shape) \
         and ops.unchanged_here(x) \

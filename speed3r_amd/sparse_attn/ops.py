@@ -641,7 +641,9 @@ def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     _forward_only(x, weight)
     b, n, c = x.shape
     h = num_heads
-    if not (qkv_project_takes(x, h, block, pooled, q_ln is not None) if takes is None else takes) or weight.shape != (3 * c, c) or (bias is not None and bias.shape != (3 * c,)):
+    if takes is None:
+        takes = qkv_project_takes(x, h, block, pooled, q_ln is not None)
+    if not takes or weight.shape != (3 * c, c) or (bias is not None and bias.shape != (3 * c,)):
         return None
     for t in (x, weight, bias):
         if t is not None and (t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16):
@@ -658,10 +660,11 @@ def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     if gate is not None:
         gw, gb = gate
         gts = [t for t in gate if t is not None]
-        takes = _lib.lib().s3r_qkv_project_gate_rides(b * n, h) and gw.shape[0] % 4 == 0 and gw.shape[0] <= 32 and gw.shape[1:] == (c,) and (gb is None or gb.shape == gw.shape[:1]) \
+        rides = _lib.lib().s3r_qkv_project_gate_rides(b * n, h) and gw.shape[0] % 4 == 0 and gw.shape[0] <= 32 and gw.shape[1:] == (c,) \
+            and (gb is None or gb.shape == gw.shape[:1]) \
             and all(t.dtype == x.dtype and t.device == x.device and t.is_contiguous() for t in gts) and gw.data_ptr() % 16 == 0
-        gates = (x.new_empty((b, n, gw.shape[0])) if takes else None,)
-        if takes:
+        gates = (x.new_empty((b, n, gw.shape[0])) if rides else None,)
+        if rides:
             gate_args = (gw.data_ptr(), gb.data_ptr() if gb is not None else None, gates[0].data_ptr(), gw.shape[0])
     with _on(x.device):
         rc = _lib.lib().s3r_qkv_project(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, c, c, v.data_ptr(),
