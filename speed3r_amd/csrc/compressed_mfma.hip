@@ -13,8 +13,8 @@
 // fp32, P rounded to the I/O dtype, O^T += V^T P^T with V^T fragments from ds_read_b64_tr_b16.
 //
 // Selection without a score buffer (the top-k-only instance, KTOP > 0): two sweeps over the key tiles, K tiles by
-// direct transfers into an LDS ring.  Sweep 1 keeps, per lane, the K largest of its half-tile maxima; the K-th
-// largest of the two lanes' lists is a lower bound of the row's K-th largest score.  Sweep 2 recomputes the scores
+// direct transfers into an LDS ring.  Sweep 1 deals every s-th key out to 128 groups per row (64 registers in each of the
+// row's two lanes) and keeps each group's maximum; the K-th largest of them is a lower bound of the row's K-th largest score.  Sweep 2 recomputes the scores
 // and appends every score >= that threshold to a small per-lane queue in LDS (no branch).  Every lane keeps the
 // exact top-K of the keys IT sees (half of each tile): a descending sorted list of K keys,
 // key = (sortable(bits(score)), Lk-1-col) in lexicographic order, in registers.  When some lane's queue is nearly
@@ -99,6 +99,36 @@ template <int N, int NF = 0> __device__ __forceinline__ void merge_top_desc(key_
 #pragma unroll
   for (int i = NF; i < N; i++) a[i] = __builtin_fmax(a[i], b[N - 1 - i]);  // half-cleaner: a is now bitonic
   bitonic_merge_desc<N>(a);
+}
+// The same on scores (no order among equal values, NaN loses to every number).
+template <int N> __device__ __forceinline__ void bitonic_merge_desc(float (&x)[N]) {
+#pragma unroll
+  for (int d = N / 2; d >= 1; d >>= 1)
+#pragma unroll
+    for (int i = 0; i < N; i++)
+      if ((i & d) == 0) {
+        const float hi = fmaxf(x[i], x[i | d]), lo = fminf(x[i], x[i | d]);
+        x[i] = hi;
+        x[i | d] = lo;
+      }
+}
+template <int N> __device__ __forceinline__ void sort_desc(float (&x)[N]) {
+  if constexpr (N > 1) {  // both halves descending, the second one turned round: a bitonic sequence
+    float a[N / 2], b[N / 2];
+#pragma unroll
+    for (int i = 0; i < N / 2; i++) {
+      a[i] = x[i];
+      b[i] = x[N / 2 + i];
+    }
+    sort_desc<N / 2>(a);
+    sort_desc<N / 2>(b);
+#pragma unroll
+    for (int i = 0; i < N / 2; i++) {
+      x[i] = a[i];
+      x[N - 1 - i] = b[i];
+    }
+    bitonic_merge_desc<N>(x);
+  }
 }
 // Sorting network for the 13 entries a lane's queue can hold (descending, entries 0..12 of x): Batcher's odd-even
 // merge sort for 16 inputs without the comparators that touch inputs 13..15, 48 compare-exchanges against the 80
@@ -245,7 +275,7 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
 #pragma unroll
   for (int i = 0; i < KL; i++) list[i] = 0;
   float thr = -INFINITY;   // survivors are the scores >= thr
-  float thr0 = -INFINITY;  // the row's threshold from the group maxima; thr never drops below it
+  float thr0 = -INFINITY;  // the row's threshold from the first sweep; thr never drops below it
   int qn = 0;
   uint2* qlane = FUSED ? &queue[wave][0][lane] : nullptr;  // entry e at qlane[e * 64]
   const uint32_t lkm1 = (uint32_t)(Lk - 1);
@@ -295,10 +325,6 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
   };
 
   const int ntiles = (int)((Lk + 63) / 64);
-  // Fused selection, first sweep: per lane the K largest half-tile maxima, descending
-  float top[KL];
-#pragma unroll
-  for (int i = 0; i < KL; i++) top[i] = -INFINITY;
   if constexpr (!FUSED) {
   fetch(0);
   stash(0);
@@ -443,21 +469,22 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
     uint32_t dl_off[4] = {0, 0, 0, 0};  // NI of them are used
 #pragma unroll
     for (int i = 0; i < NI; i++) dl_off[i] = (uint32_t)(dl_row + 8 * i) * krow_bytes + dl_chunk[i & 1];
-    auto dma_tile = [&](int t, int buf) {  // tiles past the end repeat the last one (never read)
-      const int tt = t < ntiles ? t : ntiles - 1;
-      const int64_t start = (int64_t)tt * 64;
-      const int rem = (int)(Lk - 1 - start);
+    // Tile t of a sweep holds keys 64 t s, (64 t + 1) s, ...: every key (s = 1) or, in the first sweep, every s-th one.
+    auto dma_tile = [&](int t, int buf, const int s, const int nt) {  // tiles past the end repeat the last one (never read)
+      const int tt = t < nt ? t : nt - 1;
+      const int64_t start = (int64_t)tt * 64 * s;
+      const int rem = (int)((uint32_t)(Lk - 1 - start) / (uint32_t)s);
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(kp + start * p.skn), 0, 0x7fffffff, 0x00020000);
       char* dst = reinterpret_cast<char*>(&Ks[buf][0]) + wave_u * (NI * 1024);
       uint32_t off[4] = {0, 0, 0, 0};  // the per-lane offsets of a full tile never change
 #pragma unroll
-      for (int i = 0; i < NI; i++) off[i] = dl_off[i];
+      for (int i = 0; i < NI; i++) off[i] = s == 1 ? dl_off[i] : (uint32_t)(dl_row + 8 * i) * (krow_bytes * (uint32_t)s) + dl_chunk[i & 1];
       if (__builtin_expect(rem < 63, 0)) {       // ragged last tile: rows beyond the end re-read the last row
 #pragma unroll
         for (int i = 0; i < NI; i++) {
           int r = dl_row + 8 * i;
           r = r < rem ? r : rem;
-          off[i] = (uint32_t)r * krow_bytes + dl_chunk[i & 1];
+          off[i] = (uint32_t)r * (krow_bytes * (uint32_t)s) + dl_chunk[i & 1];
           asm volatile("" : "+v"(off[i]));       // stays inside this branch
         }
       }
@@ -467,20 +494,21 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
     };
     const uint32_t lds_k = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)reinterpret_cast<char*>(&Ks[0][0]);
     const uint32_t kr_off = lds_k + (uint32_t)(c * 128 + ((hh ^ k_swizzle(c)) << 4));  // A operand: lane = key row, chunk hh + 2 ks
-    auto sweep = [&](auto filter_tag, const int stride) {  // tiles 0, stride, 2 stride, ...
+    float best[FUSED ? 2 : 1][2][16];  // first sweep: per register the largest score of the even and of the odd tiles
+    auto sweep = [&](auto filter_tag, const int keystep) {  // every keystep-th key
       constexpr bool FILTER = decltype(filter_tag)::value;
-      const int nsteps = (ntiles + stride - 1) / stride;
-      for (int i = 0; i < NB - 1; i++) dma_tile(i * stride, i);
+      const int s = FILTER ? 1 : keystep;
+      const int nsteps = FILTER ? ntiles : (int)((Lk + 64 * s - 1) / (64 * s));
+      for (int i = 0; i < NB - 1; i++) dma_tile(i, i, s, nsteps);
       int buf = 0, fill = NB - 1;  // ring positions of step i's tile and of step i + NB - 1's
       for (int i = 0; i < nsteps; i++) {
-        const int t = i * stride;
         // this wave's share of tile t has landed (transfers complete in order, NI per tile, NB - 2 tiles younger) ...
         __builtin_amdgcn_s_waitcnt(0x0F70 | (NI * (NB - 2)));
         __builtin_amdgcn_s_barrier();  // ... and everybody's; all waves are done with tile t - 1, whose buffer is refilled now
-        dma_tile((i + NB - 1) * stride, fill);
+        dma_tile(i + NB - 1, fill, s, nsteps);
         {
-          const int64_t start = (int64_t)t * 64;
-          const bool partial = start + 64 > Lk;
+          const int64_t start = (int64_t)i * 64 * s;
+          const bool partial = start + 63 * s >= Lk;
           u32x4 kf[2][4];
           const uint32_t kb = kr_off + (uint32_t)buf * (kTile * (uint32_t)sizeof(E));
           lds_read_kfrags(kb, kf);
@@ -499,7 +527,8 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
           buf = buf + 1 == NB ? 0 : buf + 1;
           fill = fill + 1 == NB ? 0 : fill + 1;
           if (partial) {  // last tile only: keys beyond Lk get a score that neither raises a maximum nor passes the filter
-            const int lim = (int)(Lk - start) - 4 * hh;  // register r of tile kt holds key kt*32 + 4hh + 8(r/4) + r%4
+            // register r of tile kt holds row kt*32 + 4hh + 8(r/4) + r%4 of the tile
+            const int lim = (int)((uint32_t)(Lk - 1 - start) / (uint32_t)s) + 1 - 4 * hh;
 #pragma unroll
             for (int kt = 0; kt < 2; kt++)
 #pragma unroll
@@ -507,19 +536,17 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
                 if (kt * 32 + 8 * (r >> 2) + (r & 3) >= lim) st[kt][r] = FILTER ? __uint_as_float(0x7FC00000u) : -INFINITY;
           }
           if constexpr (!FILTER) {
-            float mx = st[0][0];
+            // ordinary VALU reads of both accumulators first: the compiler pads the distance from the MFMAs that wrote
+            // them for these instructions, not for inline assembly
+            const float s0 = fmaxf(st[0][0], st[0][15]), s1 = fmaxf(st[1][0], st[1][15]);
+            asm volatile("" ::"v"(s0), "v"(s1));
+            auto raise = [&](float (&g)[2][16]) {
 #pragma unroll
-            for (int kt = 0; kt < 2; kt++)
+              for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-              for (int r = 0; r < 16; r++) mx = fmaxf(mx, st[kt][r]);
-            // this lane's maximum over its 32 keys of the tile goes into its descending list of the K largest such
-            // maxima (NaN never enters: fmaxf/fminf drop it)
-#pragma unroll
-            for (int i = 0; i < KL; i++) {
-              const float hi = fmaxf(top[i], mx);
-              mx = fminf(top[i], mx);
-              top[i] = hi;
-            }
+                for (int r = 0; r < 16; r++) asm("v_max_f32 %0, %0, %1" : "+v"(g[kt][r]) : "v"(st[kt][r]));  // (NaN loses)
+            };
+            if (i & 1) raise(best[FUSED ? 1 : 0]); else raise(best[0]);
           } else {
             const uint32_t col0 = (uint32_t)start + 4 * hh;
             const uint32_t qbase = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)reinterpret_cast<char*>(qlane);
@@ -594,16 +621,51 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
       }
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the transfers issued past the last tile are done too
     };
-    // First sweep: every lane keeps the K largest of its half-tile maxima (maxima over 32 different keys each).
-    // A sample of the tiles is enough: the K-th largest maximum over any subset of the keys is still a lower bound.
-    // With fewer sampled tiles the bound is looser (more survivors in the second sweep) but the sweep shorter;
-    // about 20 sampled tiles balance the two (measured at 66 and 261 tiles; 16 to 22 are within 1 % of each other, 32
-    // and 12 are 2-3 % slower for lists of 16).
-    const int stride1 = ntiles >= 64 ? (ntiles / 20 < 12 ? ntiles / 20 : 12) : 1;
+    // First sweep: a lower bound of each row's K-th largest score from a sample of the keys, every stride1-th of them.  Sample m
+    // goes to row m % 64 of tile m / 64; each of a lane's 32 registers keeps its largest score over the even and over the odd
+    // tiles, and the K-th largest of the row's 2 x 64 maxima is the bound.  Both the sample and the groups are spread over the
+    // sequence on purpose: a query's best keys lie side by side (the blocks of one frame), and with groups of 32 neighbours
+    // in every stride1-th tile, as this kernel had them before, a frame was one or two groups and was often missed:
+    // Pooled blocks of a video x 16 heads, us before / now: 16 656 keys, top-32 851 / 738; 16 266, top-16 759 / 681; 4 164 114 / 96;
+    // 2 016, top-32 91 / 54; 1 627 55 / 38.  Scores without such neighbours: within 4 % either way (16 266 keys 1 271 / 1 256,
+    // 3 024 147 / 141, 4 164 top-8 131 / 136).  The sweep itself got cheaper too: 32 maxima per tile in place of 31 and an
+    // insertion into a sorted list.
+    // About 24 sampled tiles balance the sweep against the survivors that a looser bound lets through (20 and 30 are within
+    // 1 %; every second key from 32 tiles on: 4 032 keys of a video 95 -> 81, but 3 024 keys without neighbours 140 -> 154).
+    const int far = (int)(0x7fffffffu / (64u * krow_bytes));  // a sampled tile's rows lie within 2^31 bytes
+    int stride1 = ntiles >= 64 ? (ntiles / 24 < 10 ? ntiles / 24 : 10) : 1;
+    stride1 = stride1 < far ? stride1 : far;
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) best[g][kt][r] = -INFINITY;
     sweep(std::false_type{}, stride1);
-    // Threshold: the K-th largest of the row's half-tile maxima, i.e. of the union of the two lanes' lists.  K
-    // different scores (one per half tile) are at least that large, so a score below it is not among the K
-    // largest, whatever the tie-break.  With fewer than K half tiles it stays -inf and every score is a candidate.
+    // the K largest of the lane's 64 maxima, descending (pieces sorted and merged: once per wave)
+    float top[KL];
+    {
+      constexpr int PIECE = KL < 4 ? 4 : KL;
+      float all[64];
+#pragma unroll
+      for (int g = 0; g < 64; g++) all[g] = best[g >> 5][(g >> 4) & 1][g & 15];
+      float run[PIECE];
+#pragma unroll
+      for (int pc = 0; pc < 64 / PIECE; pc++) {
+        float x[PIECE];
+#pragma unroll
+        for (int i = 0; i < PIECE; i++) x[i] = all[pc * PIECE + i];
+        sort_desc<PIECE>(x);
+#pragma unroll
+        for (int i = 0; i < PIECE; i++) run[i] = pc == 0 ? x[i] : fmaxf(run[i], x[PIECE - 1 - i]);
+        if (pc != 0) bitonic_merge_desc<PIECE>(run);
+      }
+#pragma unroll
+      for (int i = 0; i < KL; i++) top[i] = run[i];
+    }
+    // Threshold: the K-th largest of the row's group maxima, i.e. of the union of the two lanes' lists.  K
+    // different scores (one per group) are at least that large, so a score below it is not among the K
+    // largest, whatever the tie-break.  With fewer than K groups that hold a key it stays -inf and every score is a candidate.
     // The K-th largest of two descending lists a, b is the largest min(a[i-1], b[K-i-1]) over the splits i.
     {
       float tau = fmaxf(top[KL - 1], __uint_as_float(xh_swap(__float_as_uint(top[KL - 1]))));  // splits i = K and i = 0
