@@ -371,15 +371,14 @@ int s3r_gated_merge(const void* o_cmp, const void* o_sel, const void* gate, void
  * s3r_attn_bwd_delta:  delta[b,h,n] = sum_d o[b,h,n,d] * dout[b,h,n,d]  (fp32, contiguous [B,H,N]).
  * s3r_attn_bwd: with P = exp(scale * q k^T - lse) over the keys the forward attended to,
  *   dv = P^T dout,  dS = scale * P * (dout v^T - delta),  dq = dS k,  dk = dS^T q;
- *   P and dS are rounded to the I/O dtype before the products, accumulation is fp32 (for dk in bf16 with 64-token
- *   blocks the rounded factor is dS / scale and the scale multiplies the fp32 sum: the same relative rounding).
+ *   P and dS are rounded to the I/O dtype before the products, accumulation is fp32 (for dk in bf16 the
+ *   rounded factor is dS / scale and the scale multiplies the fp32 sum: the same relative rounding).
  *   lse: the forward's optional output (natural log, scaled scores), fp32 [B,H,Lq] contiguous.
  *   idx: the forward's block indices [B,H,ceil(Lq/block),K] (strides sib,sih,sim), or NULL for dense attention.
  *   kq_list, kq_off (needed for dk/dv when idx is given): for every (b,h) the query-block ids that list key block j,
  *     one entry per occurrence, ascending, are kq_list[(b*H+h)*list_stride + kq_off[(b*H+h)*(nkb+1) + j] ...
  *     kq_off[... + j+1]), nkb = ceil(Lk/block); entries of idx that are < 0 or >= nkb appear in no list
- *     (reference count_query_fixedlen / reorder_topk_idx_fixedlen, :423-554).  With block 16 the dk/dv kernel merges
- *     neighbouring lists and relies on every list being ascending, as s3r_key_block_lists leaves it.
+ *     (reference count_query_fixedlen / reorder_topk_idx_fixedlen, :423-554).  The kernels add up in the order of the list.
  *   dq (layout strides sdq*), dk, dv (sdk*, sdv*): I/O dtype; dq == NULL or dk == dv == NULL skips that kernel.
  *   Every row of dq, dk, dv inside the tensors is written (zeros where nothing attends).
  */

@@ -25,15 +25,6 @@
 //     dV^T += dO^T P and dK^T += Q^T dS read their A operands transposed from the same buffers.
 // Query rows beyond Lq have lse = +inf (P = 0), keys beyond Lk are masked (P = 0); rows past the end of a tensor are
 // never read (transfers re-read the last valid row).
-//
-// 16-token blocks (BLK = 16, the reference layer's own block size) run through the same kernels: a 32-row half tile
-// is then two 16-row blocks, and neighbouring blocks name mostly the same partners, so both kernels walk UNIONS of
-// lists (distinct blocks from a 512-slot hash table in LDS, with a count byte per list: how often that list names the
-// block; a product's quadrant whose count is 0 gets P = 0, one listed twice counts twice).  dQ kernel: the union of
-// the index rows of the wave's four query blocks, two distinct key blocks per half tile against all 64 queries.
-// dK/dV kernel: the workgroup's 64 keys are four neighbouring key blocks; it walks the union of their four
-// query-block lists, four entries per 64-row tile, with the tile code of the 64-token blocks; the union is built a
-// chunk of the (ascending) lists at a time.
 #include "select_common.h"
 #include "attn_bwd.h"
 
@@ -42,9 +33,6 @@ namespace bwd {
 using namespace sel;
 
 constexpr int kHalfBytes = 32 * 128;  // one half tile: 32 rows of 64 two-byte values
-// dK/dV at 16-token blocks: list entries per chunk of the union of four neighbouring key blocks' lists (a quarter from
-// each list; the union's hash table has 512 slots)
-constexpr int kMergeMax = 384;
 constexpr float kLog2e = 1.4426950408889634f;
 
 typedef std::integral_constant<int, 0> H0;
@@ -95,25 +83,6 @@ __device__ __forceinline__ void dma_rows(const E* base, uint32_t rowbytes, int f
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds_half + i * 1024), 16,
                                                (uint32_t)row * rowbytes + (uint32_t)(chunk * 16), 0, 0, 0);
     }
-  }
-}
-
-// The same for a half tile made of two 16-row blocks: instructions 0, 1 move block A, 2, 3 block B; rows are clamped
-// to last_a / last_b (relative to the block's first row).
-template <typename E, bool VSW>
-__device__ __forceinline__ void dma_rows16(const E* base_a, const E* base_b, uint32_t rowbytes, int last_a, int last_b, char* lds_half, int lane) {
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)base_a, 0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)base_b, 0, 0x7fffffff, 0x00020000);
-  const int lr = lane >> 3;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int ldsrow = 8 * i + lr;
-    const int last = i < 2 ? last_a : last_b;
-    int row = ldsrow & 15;
-    row = row < last ? row : last;
-    const int chunk = (lane & 7) ^ k_swizzle(ldsrow);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(i < 2 ? ra : rb, (__attribute__((address_space(3))) void*)(lds_half + i * 1024), 16,
-                                             (uint32_t)row * rowbytes + (uint32_t)(chunk * 16), 0, 0, 0);
   }
 }
 
@@ -247,7 +216,7 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[2], E* rowptr, bo
 }
 
 // ---- dQ ----------------------------------------------------------------------------------------------------------
-template <typename E, bool DENSE, int BLK>
+template <typename E, bool DENSE>
 __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, int nqg, int total_wg) {
   typedef typename Mma<E>::V8 V8;
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[4 * kHalfBytes];
@@ -314,116 +283,26 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
       for (int r = 0; r < 16; r++) dqt[qt][dt][r] = 0.f;
 
   // key tiles of this query block
-  static_assert(BLK == 64 || (BLK == 16 && !DENSE), "blocks of 64 tokens, or of 16 with an index list");
   int32_t my_idx = -1;
   uint64_t todo = 0;
   int ntiles;
   int dense_next = 0;
-  // BLK 16: the wave's 64 queries are four query blocks with a list each; neighbouring lists name mostly the same key
-  // blocks, so the wave walks the UNION of the four lists.  Entry n of the walk list (LDS) is a distinct key block and
-  // four count bytes (how often query block j lists it; 0: not at all, above 1: a duplicated entry, which weighs the
-  // block that often, as the forward pass does).  A tile is four entries: two per 32-key half.
-  __shared__ __attribute__((aligned(16))) int2 lds_walk[BLK == 16 ? 4 : 1][BLK == 16 ? 264 : 1];
-  int2* const walk = lds_walk[BLK == 16 ? wave : 0];
-  int n_union = 0;
-  bool dup = false;  // some list names a block more than once (wave-uniform)
   if constexpr (DENSE) {
     ntiles = (int)((Lk + 63) >> 6);
-  } else if constexpr (BLK == 64) {
+  } else {
     const int32_t* idx_row = p.idx + (int64_t)b * p.sib + (int64_t)h * p.sih + (int64_t)qb * p.sim;
     my_idx = lane < p.K ? idx_row[lane] : -1;
     todo = __ballot(my_idx >= 0 && (int64_t)my_idx * 64 < Lk);
     ntiles = __popcll(todo);
-  } else {
-    const int64_t nqb16 = (Lq + 15) >> 4;
-    int32_t my16[4] = {-1, -1, -1, -1};  // entry `lane` of the four lists
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      const int64_t qb16 = (int64_t)qb * 4 + s;
-      if (qb16 < nqb16 && lane < p.K) {
-        const int32_t v = (p.idx + (int64_t)b * p.sib + (int64_t)h * p.sih + qb16 * p.sim)[lane];
-        my16[s] = (v >= 0 && (int64_t)v * 16 < Lk) ? v : -1;
-      }
-    }
-    // Distinct blocks and their counts through a hash table in LDS (512 slots in this wave's first K buffer, which no
-    // transfer touches before the list is complete): every lane inserts its entry of list j with a compare-and-swap on
-    // the key (linear probing; at most 4 x 64 distinct blocks) and adds 1 << 8j to the slot's count; the occupied
-    // slots are then compacted into the list, eight slots per lane, positions from ballots.
-    int32_t* const hkey = reinterpret_cast<int32_t*>(k_buf[0]);          // [512]
-    uint32_t* const hcnt = reinterpret_cast<uint32_t*>(k_buf[0] + 2048);  // [512]
-    reinterpret_cast<int4*>(hkey)[lane] = make_int4(-1, -1, -1, -1);
-    reinterpret_cast<int4*>(hkey)[lane + 64] = make_int4(-1, -1, -1, -1);
-    reinterpret_cast<int4*>(hcnt)[lane] = make_int4(0, 0, 0, 0);
-    reinterpret_cast<int4*>(hcnt)[lane + 64] = make_int4(0, 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int32_t e = my16[j];
-      bool active = e >= 0;
-      uint32_t slot = ((uint32_t)e * 0x9E3779B1u) >> 23;
-      while (active) {
-        const int32_t old = atomicCAS(hkey + slot, -1, e);
-        if (old == -1 || old == e) {
-          atomicAdd(hcnt + slot, 1u << (8 * j));
-          active = false;
-        } else {
-          slot = (slot + 1) & 511u;
-        }
-      }
-    }
-    const int4 k0 = reinterpret_cast<const int4*>(hkey)[2 * lane], k1 = reinterpret_cast<const int4*>(hkey)[2 * lane + 1];
-    const int4 c0 = reinterpret_cast<const int4*>(hcnt)[2 * lane], c1 = reinterpret_cast<const int4*>(hcnt)[2 * lane + 1];
-    const int32_t ks8[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-    const int32_t cs8[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-    uint32_t pos = 0;  // occupied slots of the lanes below
-    uint32_t cnt_bits = 0;
-#pragma unroll
-    for (int s8 = 0; s8 < 8; s8++) {
-      const uint64_t m = __ballot(ks8[s8] >= 0);
-      pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, pos));
-      n_union += __popcll(m);
-      cnt_bits |= (uint32_t)cs8[s8];
-    }
-#pragma unroll
-    for (int s8 = 0; s8 < 8; s8++)
-      if (ks8[s8] >= 0) walk[pos++] = make_int2(ks8[s8], cs8[s8]);
-    if (lane < 4) walk[n_union + lane] = make_int2(-1, 0);  // the last tile's missing entries
-    dup = __any((cnt_bits & 0xfefefefeu) != 0);
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the table is read and the list written before the first transfer
-    ntiles = (n_union + 3) >> 2;
   }
-  auto pop = [&]() -> int64_t {  // start row of the next tile, BLK 16: its list position (callers pop exactly ntiles times)
+  auto pop = [&]() -> int64_t {  // start row of the next tile (callers pop exactly ntiles times)
     if constexpr (DENSE) {
       return (int64_t)(dense_next++) * 64;
-    } else if constexpr (BLK == 64) {
+    } else {
       const int t = __ffsll((unsigned long long)todo) - 1;
       todo &= todo - 1;
       return (int64_t)__builtin_amdgcn_readlane(my_idx, t) * 64;
-    } else {
-      return (int64_t)(dense_next++);
     }
-  };
-  // BLK 16: the four entries (key block, four count bytes; -1: none) of the tile being computed and of the tile whose
-  // first half is fetched meanwhile, read from the walk list once per tile (a hand-written read, like the fragments')
-  // and kept in scalar registers
-  struct Entries16 { int32_t blk[4] = {-1, -1, -1, -1}; uint32_t cnt[4] = {0, 0, 0, 0}; };
-  struct NoEntries {};
-  typedef std::conditional_t<BLK == 16, Entries16, NoEntries> TileEntries;
-  TileEntries ent_cur, ent_nxt;
-  auto read_entries = [&](int64_t t, Entries16& e) {
-    const uint32_t a = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)reinterpret_cast<const char*>(walk + 4 * t);
-    u32x4 v0, v1;
-    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:16\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v0), "=&v"(v1) : "v"(a));
-    e.blk[0] = __builtin_amdgcn_readfirstlane((int32_t)v0[0]); e.cnt[0] = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)v0[1]);
-    e.blk[1] = __builtin_amdgcn_readfirstlane((int32_t)v0[2]); e.cnt[1] = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)v0[3]);
-    e.blk[2] = __builtin_amdgcn_readfirstlane((int32_t)v1[0]); e.cnt[2] = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)v1[1]);
-    e.blk[3] = __builtin_amdgcn_readfirstlane((int32_t)v1[2]); e.cnt[3] = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)v1[3]);
-  };
-  // first key row, number of valid rows and the count bytes of entry `s` (0..3) of a tile (none: row 0, no counts)
-  auto sub_block = [&](const Entries16& e, int s, int64_t& start, int& nv, uint32_t& counts) {
-    const int32_t blk = e.blk[s];
-    counts = e.cnt[s];
-    start = blk >= 0 ? (int64_t)blk * 16 : 0;
-    nv = blk >= 0 ? (int)(Lk - start < 16 ? Lk - start : 16) : 0;
   };
 
   const float scale = p.scale;
@@ -431,35 +310,15 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
   const uint32_t krow = (uint32_t)p.skn * (uint32_t)sizeof(E), vrow = (uint32_t)p.svn * (uint32_t)sizeof(E);
   const int tr_off = tr_offset(lane);
 
-  auto fetch = [&](int64_t start, auto hf, int buf, const TileEntries& ent) {  // half HF of the tile at `start` -> buffers `buf`
+  auto fetch = [&](int64_t start, auto hf, int buf) {  // half HF of the tile at `start` -> buffers `buf`
     constexpr int HF = decltype(hf)::value;
-    if constexpr (BLK == 64) {
-      const int last = (int)((Lk - start < 64 ? Lk - start : 64) - 1);
-      dma_rows<E, true>(kp + start * p.skn, krow, 32 * HF, last, k_buf[buf], lane, 0, 4);
-      dma_rows<E, false>(vp + start * p.svn, vrow, 32 * HF, last, v_buf[buf], lane, 0, 4);
-    } else {
-      int64_t sa, sb;
-      int na, nb;
-      uint32_t ca, cb;
-      sub_block(ent, 2 * HF, sa, na, ca);
-      sub_block(ent, 2 * HF + 1, sb, nb, cb);
-      const int la = na > 0 ? na - 1 : 0, lb = nb > 0 ? nb - 1 : 0;
-      dma_rows16<E, true>(kp + sa * p.skn, kp + sb * p.skn, krow, la, lb, k_buf[buf], lane);
-      dma_rows16<E, false>(vp + sa * p.svn, vp + sb * p.svn, vrow, la, lb, v_buf[buf], lane);
-    }
+    const int last = (int)((Lk - start < 64 ? Lk - start : 64) - 1);
+    dma_rows<E, true>(kp + start * p.skn, krow, 32 * HF, last, k_buf[buf], lane, 0, 4);
+    dma_rows<E, false>(vp + start * p.svn, vrow, 32 * HF, last, v_buf[buf], lane, 0, 4);
   };
-  auto compute = [&](int64_t start, auto hf, int buf, const TileEntries& ent) {
+  auto compute = [&](int64_t start, auto hf, int buf) {
     constexpr int HF = decltype(hf)::value;
-    int nvalid = 64;
-    int na = 16, nb = 16;      // BLK 16: valid keys of the half's two blocks A (rows 0..15) and B (16..31)
-    uint32_t ca = 0, cb = 0;   // and how often each of the four query blocks lists them
-    if constexpr (BLK == 64) {
-      nvalid = (int)(Lk - start < 64 ? Lk - start : 64);
-    } else {
-      int64_t sa, sb;
-      sub_block(ent, 2 * HF, sa, na, ca);
-      sub_block(ent, 2 * HF + 1, sb, nb, cb);
-    }
+    const int nvalid = (int)(Lk - start < 64 ? Lk - start : 64);
     const bool ragged = nvalid < 64;
     V8 ak[4], av[4];
     {
@@ -482,32 +341,12 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
       for (int ks = 0; ks < 4; ks++) st = Mma<E>::mma(ak[ks], bq[qt][ks], st);
 #pragma unroll
       for (int ks = 0; ks < 4; ks++) dp = Mma<E>::mma(av[ks], bg[qt][ks], dp);
-      if constexpr (BLK == 64) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) st[r] = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, -lse2[qt]));  // P^T
-        if (ragged) {  // keys beyond Lk carry no probability
+      for (int r = 0; r < 16; r++) st[r] = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, -lse2[qt]));  // P^T
+      if (ragged) {  // keys beyond Lk carry no probability
 #pragma unroll
-          for (int r = 0; r < 16; r++)
-            if (32 * HF + 4 * hh + 8 * (r >> 2) + (r & 3) >= nvalid) st[r] = 0.f;
-        }
-      } else {
-        // registers 0..7 are keys of block A, 8..15 of block B; this lane's query block lists each 0, 1 or more times,
-        // and a probability counts that often: the count goes into the exponent (lse - log2(count); 0 times: +inf),
-        // two values per lane instead of a test per score
-        const int sh = 8 * (2 * qt + (c >> 4));
-        const uint32_t wa = (ca >> sh) & 0xffu, wb = (cb >> sh) & 0xffu;
-        float la = wa != 0 ? lse2[qt] : INFINITY, lb = wb != 0 ? lse2[qt] : INFINITY;
-        if (dup) {
-          la -= __builtin_amdgcn_logf((float)(wa > 1 ? wa : 1));
-          lb -= __builtin_amdgcn_logf((float)(wb > 1 ? wb : 1));
-        }
-#pragma unroll
-        for (int r = 0; r < 16; r++) st[r] = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, -(r < 8 ? la : lb)));  // P^T
-        if (na < 16 || nb < 16) {  // (wave-uniform) a block cut short by the end of the sequence, or none
-#pragma unroll
-          for (int r = 0; r < 16; r++)
-            if (4 * hh + 8 * ((r >> 2) & 1) + (r & 3) >= (r < 8 ? na : nb)) st[r] = 0.f;
-        }
+        for (int r = 0; r < 16; r++)
+          if (32 * HF + 4 * hh + 8 * (r >> 2) + (r & 3) >= nvalid) st[r] = 0.f;
       }
 #pragma unroll
       for (int r = 0; r < 16; r++) ds[qt][r >> 3][r & 7] = (E)(st[r] * fmaf(dp[r], scale, -dlts[qt]));  // scale * P * (dP - delta)
@@ -531,28 +370,23 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
 
   if (ntiles > 0) {
     int64_t cur = pop();
-    if constexpr (BLK == 16) read_entries(cur, ent_cur);
-    fetch(cur, H0{}, 0, ent_cur);
+    fetch(cur, H0{}, 0);
     for (int t = 0; t < ntiles; t++) {
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads of buffer 1 (previous tile) are done
-      fetch(cur, H1{}, 1, ent_cur);
+      fetch(cur, H1{}, 1);
       __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): half 0 has landed
-      compute(cur, H0{}, 0, ent_cur);
+      compute(cur, H0{}, 0);
       const bool more = t + 1 < ntiles;
       const int64_t nxt = more ? pop() : cur;
-      if constexpr (BLK == 16) {
-        if (more) read_entries(nxt, ent_nxt);
-      }
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads of buffer 0 are done
       if (more) {
-        fetch(nxt, H0{}, 0, ent_nxt);
+        fetch(nxt, H0{}, 0);
         __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): half 1 has landed
       } else {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
       }
-      compute(cur, H1{}, 1, ent_cur);
+      compute(cur, H1{}, 1);
       cur = nxt;
-      ent_cur = ent_nxt;
     }
   }
 
@@ -565,7 +399,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
 }
 
 // ---- dK, dV ------------------------------------------------------------------------------------------------------
-template <typename E, bool DENSE, int BLK>
+template <typename E, bool DENSE>
 __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, int nqb_all, int total_wg) {
   typedef typename Mma<E>::V8 V8;
   constexpr int kTileBytes = 2 * kHalfBytes;  // a 64-row query tile
@@ -573,14 +407,10 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
   __shared__ __attribute__((aligned(1024))) unsigned char lds_q1[kTileBytes];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_g0[kTileBytes];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_g1[kTileBytes];
-  // per-query scalars of a tile: [0,64) lse, [64,128) delta.  BLK 16: four such pairs kVar floats apart, one per key
-  // block of the workgroup, each with its own variant of lse (delta is repeated, so that a lane finds both values of
-  // a query at a fixed distance and reads them with one instruction)
-  constexpr int kVar = 136;
+  // per-query scalars of a tile: [0,64) lse, [64,128) delta
   constexpr int kDeltaAt = 64;
-  __shared__ __attribute__((aligned(256))) float lds_s0[BLK == 16 ? 4 * kVar : 128];
-  __shared__ __attribute__((aligned(256))) float lds_s1[BLK == 16 ? 4 * kVar : 128];
-  __shared__ __attribute__((aligned(16))) int2 lds_union[BLK == 16 ? kMergeMax + 8 : 1];  // BLK 16: the current chunk's union of the four lists
+  __shared__ __attribute__((aligned(256))) float lds_s0[128];
+  __shared__ __attribute__((aligned(256))) float lds_s1[128];
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -602,16 +432,8 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
 
   const int64_t Lq = p.Lq, Lk = p.Lk;
   if constexpr (!DENSE) {
-    const int64_t nkbl = (Lk + BLK - 1) / BLK;
-    const int32_t* off = p.kq_off + ((int64_t)b * p.H + h) * (nkbl + 1);
-    int len;
-    if constexpr (BLK == 64) {
-      len = off[kb + 1] - off[kb];
-    } else {  // the workgroup walks the lists of its four key blocks one after the other, four entries per step
-      const int64_t ka = (int64_t)kb * 4;
-      const int64_t kz = ka + 4 < nkbl ? ka + 4 : nkbl;
-      len = (off[kz] - off[ka]) / 4;
-    }
+    const int32_t* off = p.kq_off + ((int64_t)b * p.H + h) * (nkb + 1);
+    int len = off[kb + 1] - off[kb];
     len = __builtin_amdgcn_readfirstlane(len);
     if ((len > 4 * p.K) != long_pass) return;
   }
@@ -622,8 +444,7 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
   const float* lsep = p.lse + ((int64_t)b * p.H + h) * Lq;
   const float* dlp = p.delta + ((int64_t)b * p.H + h) * Lq;
 
-  // B operands K and V of this wave's 32 keys (lane = key, head_dim chunk hh + 2 ks).  BLK 16: these are two
-  // neighbouring key blocks, the workgroup's 64 keys four.
+  // B operands K and V of this wave's 32 keys (lane = key, head_dim chunk hh + 2 ks)
   const int64_t key = (int64_t)kb * 64 + wave * 32 + c;
   V8 bk[4], bv[4];
   f32x16 dkt[2], dvt[2];  // dK^T, dV^T [dt]: lane = key, registers = head_dim
@@ -648,27 +469,16 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
   load_keys();
 
   // query blocks that attend to this key block
-  static_assert(BLK == 64 || (BLK == 16 && !DENSE), "blocks of 64 tokens, or of 16 with key-centric lists");
   int n_lists;
   const int32_t* list = nullptr;
-  const int32_t* off16 = nullptr;  // BLK 16: the list offsets of this (b, h); `list` then points at the head's whole list array
   if constexpr (DENSE) {
     n_lists = nqb_all;
-  } else if constexpr (BLK == 64) {
+  } else {
     const int32_t* off = p.kq_off + ((int64_t)b * p.H + h) * (nkb + 1);
     const int32_t lo = off[kb], hi = off[kb + 1];
     n_lists = hi - lo;
     list = p.kq_list + ((int64_t)b * p.H + h) * p.list_stride + lo;
-  } else {
-    const int64_t nkb16 = (Lk + 15) >> 4;
-    const int32_t* off = p.kq_off + ((int64_t)b * p.H + h) * (nkb16 + 1);
-    n_lists = 0;  // set per key block below
-    list = p.kq_list + ((int64_t)b * p.H + h) * p.list_stride;
-    off16 = off;
   }
-  // BLK 16: how often each of the workgroup's four key blocks lists the two query blocks this wave fetches for the
-  // tile in flight (a byte per key block), set by block_of for the fetch that follows it
-  uint32_t ent_cnt_a = 0, ent_cnt_b = 0;
   // List entries come 64 at a time (lane l holds entry base + l), so the latency of the list read is paid once per
   // 64 tiles and not in front of every tile's transfers.  The lists are walked front to back.
   int32_t held_a = -1;
@@ -683,45 +493,35 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
   auto block_of = [&](int i) -> int64_t {
     if constexpr (DENSE) {
       return (int64_t)i;
-    } else if constexpr (BLK == 64) {
+    } else {
       return (int64_t)entry(list, n_lists, held_a, base_a, i);
-    } else {  // tile i of the chunk: entries 4i .. 4i+3 of the union, this wave fetches 4i + 2 wave and the next one
-      const int4 v = *reinterpret_cast<const int4*>(lds_union + 4 * i + 2 * wave);
-      const int32_t q0 = __builtin_amdgcn_readfirstlane(v.x), q1 = __builtin_amdgcn_readfirstlane(v.z);
-      ent_cnt_a = (uint32_t)__builtin_amdgcn_readfirstlane(v.y);
-      ent_cnt_b = (uint32_t)__builtin_amdgcn_readfirstlane(v.w);
-      return (int64_t)(uint32_t)q0 | ((int64_t)q1 << 32);  // packed for `fetch`; -1: none
     }
   };
 
   const float scale = p.scale;
   const float sl2 = scale * kLog2e;
   // The per-query terms ride in the accumulators instead of in the vector slots.  The accumulator of S starts at
-  // -lse / scale (16-token blocks: the variant of the lane's key block, its count folded in), so P = exp2(scale * log2(e) *
-  // accumulator); the accumulator of dP starts at -delta, so dS / scale = P * accumulator.  No slot then begins with an
-  // LDS read of per-query values in front of the arithmetic that needs them: the start values come with four
-  // ds_read_b128 per accumulator ahead of the half's products (those of the second half's dP a quarter per slot, next
-  // to the fragments of its products: the 16-token instance has no register to spare for all of them at once).  bf16
-  // also puts the softmax scale onto dK once at the end (the rounding of dS to the I/O type is relative and
-  // does not care for the factor): per score a multiplication, an exponential and a multiplication instead of two fused
-  // multiply-adds, an exponential and a multiplication; fp16, with its narrow range, scales every dS.  bf16, 266 496
-  // tokens: 64-token blocks, top-16: 2.88 -> 2.79 (delta) -> 2.62 ms (lse); 16-token blocks, top-32: 3.74 -> 3.67 ms.
+  // -lse / scale, so P = exp2(scale * log2(e) * accumulator); the accumulator of dP starts at -delta, so
+  // dS / scale = P * accumulator.  No slot then begins with an LDS read of per-query values in front of the arithmetic
+  // that needs them: the start values come with four ds_read_b128 per accumulator ahead of the half's products (those of
+  // the second half's dP a quarter per slot, next to the fragments of its products).  bf16 also puts the softmax scale
+  // onto dK once at the end (the rounding of dS to the I/O type is relative and does not care for the factor): per score
+  // a multiplication, an exponential and a multiplication instead of two fused multiply-adds, an exponential and a
+  // multiplication; fp16, with its narrow range, scales every dS.  bf16, 266 496 tokens, top-16: 2.88 -> 2.79 (delta) ->
+  // 2.62 ms (lse).
   const float inv_scale = 1.0f / scale;
   constexpr bool FOLD = true;  // (kept as a switch: the other form reads lse and delta from LDS inside the vector slots)
   constexpr bool LATE_SCALE = std::is_same<E, bf16_t>::value;  // the softmax scale goes onto dK at the end
   const uint32_t qrow = (uint32_t)p.sqm * (uint32_t)sizeof(E), grow = (uint32_t)p.sgm * (uint32_t)sizeof(E);
   const int tr_off = tr_offset(lane);
-  const int lse_at = BLK == 16 ? (2 * wave + (c >> 4)) * kVar : 0;
   // (one per parity of the instruction inside its half tile: the chunk map of rows 8..15 differs from that of rows 0..7)
   const uint32_t q_voff[2] = {(uint32_t)(lane >> 3) * qrow + (uint32_t)(((lane & 7) ^ k_swizzle(lane >> 3)) * 16),
                               (uint32_t)(lane >> 3) * qrow + (uint32_t)(((lane & 7) ^ k_swizzle((lane >> 3) + 8)) * 16)};
   const uint32_t g_voff[2] = {(uint32_t)(lane >> 3) * grow + (uint32_t)(((lane & 7) ^ k_swizzle(lane >> 3)) * 16),
                               (uint32_t)(lane >> 3) * grow + (uint32_t)(((lane & 7) ^ k_swizzle((lane >> 3) + 8)) * 16)};
 
-  float staged = 0.f;          // this lane's lse or delta value of the tile in flight, as loaded (BLK 64: wave 0 lse,
-                               // wave 1 delta; BLK 16: lanes 0..31 lse, 32..63 delta of the wave's 32 queries)
-  bool staged_inf = false;     // rows past the end of the tensor or of a block publish lse = +inf
-  uint32_t staged_cnt = 0;     // BLK 16: the count bytes of the row's query block
+  float staged = 0.f;          // this lane's lse or delta value of the tile in flight, as loaded (wave 0 lse, wave 1 delta)
+  bool staged_inf = false;     // rows past the end of the tensor publish lse = +inf
   int staged_buf = -1;         // (wave-uniform) the buffer it goes to; -1: nothing staged
   // One query tile (64 rows of Q and dO, 64 lse and delta values) -> buffer BUF; each wave moves half of every
   // operand (instructions 2*wave, 2*wave+1 of both 32-row halves), wave 0 the lse values, wave 1 delta.
@@ -729,57 +529,37 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
     constexpr int BUF = decltype(bufc)::value;
     char* qb = reinterpret_cast<char*>(BUF == 0 ? lds_q0 : lds_q1);
     char* gb = reinterpret_cast<char*>(BUF == 0 ? lds_g0 : lds_g1);
-    if constexpr (BLK == 64) {
-      const int64_t start = qblk * 64;
-      const int last = (int)((Lq - start < 64 ? Lq - start : 64) - 1);
-      if (last >= 63) {
-        // (wave-uniform) a full tile: per-lane offsets (row lane/8 and its chunk) that do not depend on the tile, the
-        // instruction's rows ride in the scalar offset
-        const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)(qp + start * p.sqm), 0, 0x7fffffff, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void*)(gp + start * p.sgm), 0, 0x7fffffff, 0x00020000);
+    const int64_t start = qblk * 64;
+    const int last = (int)((Lq - start < 64 ? Lq - start : 64) - 1);
+    if (last >= 63) {
+      // (wave-uniform) a full tile: per-lane offsets (row lane/8 and its chunk) that do not depend on the tile, the
+      // instruction's rows ride in the scalar offset
+      const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)(qp + start * p.sqm), 0, 0x7fffffff, 0x00020000);
+      const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void*)(gp + start * p.sgm), 0, 0x7fffffff, 0x00020000);
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++)
+      for (int hf = 0; hf < 2; hf++)
 #pragma unroll
-          for (int ii = 0; ii < 2; ii++) {
-            const int i = 2 * wave + ii;
-            const uint32_t rows = (uint32_t)(32 * hf + 8 * i);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (__attribute__((address_space(3))) void*)(qb + hf * kHalfBytes + i * 1024), 16,
-                                                     q_voff[ii], rows * qrow, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (__attribute__((address_space(3))) void*)(gb + hf * kHalfBytes + i * 1024), 16,
-                                                     g_voff[ii], rows * grow, 0, 0);
-          }
-      } else {
-#pragma unroll
-        for (int hf = 0; hf < 2; hf++) {
-          dma_rows<E, true>(qp + start * p.sqm, qrow, 32 * hf, last, qb + hf * kHalfBytes, lane, 2 * wave, 2 * wave + 2);
-          dma_rows<E, true>(gp + start * p.sgm, grow, 32 * hf, last, gb + hf * kHalfBytes, lane, 2 * wave, 2 * wave + 2);
+        for (int ii = 0; ii < 2; ii++) {
+          const int i = 2 * wave + ii;
+          const uint32_t rows = (uint32_t)(32 * hf + 8 * i);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (__attribute__((address_space(3))) void*)(qb + hf * kHalfBytes + i * 1024), 16,
+                                                   q_voff[ii], rows * qrow, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (__attribute__((address_space(3))) void*)(gb + hf * kHalfBytes + i * 1024), 16,
+                                                   g_voff[ii], rows * grow, 0, 0);
         }
-      }
-      // per-query scalars pass through a register and are stored to LDS by `publish` before the barrier that opens
-      // the tile
-      const int r = lane < last ? lane : last;
-      staged = ((wave == 0 ? lsep : dlp) + start)[r];
-      staged_inf = wave == 0 && lane > last;  // query rows beyond Lq: lse = +inf, no probability
-      staged_buf = BUF;
     } else {
-      // this wave's half of the tile: the 16 queries of each of the step's two query blocks (none: any rows,
-      // lse = +inf); lanes 0..31 fetch the 32 lse values, lanes 32..63 the delta values
-      const int32_t ea = (int32_t)(qblk & 0xffffffffLL), eb = (int32_t)(qblk >> 32);  // the step's two query blocks (-1: none)
-      const int64_t sa = ea >= 0 ? (int64_t)ea * 16 : 0, sbk = eb >= 0 ? (int64_t)eb * 16 : 0;
-      const int na = ea >= 0 ? (int)(Lq - sa < 16 ? Lq - sa : 16) : 0;
-      const int nb = eb >= 0 ? (int)(Lq - sbk < 16 ? Lq - sbk : 16) : 0;
-      const int la = na > 0 ? na - 1 : 0, lb = nb > 0 ? nb - 1 : 0;
-      dma_rows16<E, true>(qp + sa * p.sqm, qp + sbk * p.sqm, qrow, la, lb, qb + wave * kHalfBytes, lane);
-      dma_rows16<E, true>(gp + sa * p.sgm, gp + sbk * p.sgm, grow, la, lb, gb + wave * kHalfBytes, lane);
-      const int j = lane & 31, j16 = j & 15;
-      const bool second = (j >> 4) != 0;
-      const int nmine = second ? nb : na;
-      const int64_t row = (second ? sbk : sa) + (j16 < nmine ? j16 : 0);
-      staged = (hh == 0 ? lsep : dlp)[row];
-      staged_inf = hh == 0 && j16 >= nmine;
-      staged_cnt = second ? ent_cnt_b : ent_cnt_a;
-      staged_buf = BUF;
+#pragma unroll
+      for (int hf = 0; hf < 2; hf++) {
+        dma_rows<E, true>(qp + start * p.sqm, qrow, 32 * hf, last, qb + hf * kHalfBytes, lane, 2 * wave, 2 * wave + 2);
+        dma_rows<E, true>(gp + start * p.sgm, grow, 32 * hf, last, gb + hf * kHalfBytes, lane, 2 * wave, 2 * wave + 2);
+      }
     }
+    // per-query scalars pass through a register and are stored to LDS by `publish` before the barrier that opens
+    // the tile
+    const int r = lane < last ? lane : last;
+    staged = ((wave == 0 ? lsep : dlp) + start)[r];
+    staged_inf = wave == 0 && lane > last;  // query rows beyond Lq: lse = +inf, no probability
+    staged_buf = BUF;
   };
   // The loaded value is first touched here, a whole tile of work after its load: any arithmetic on it inside `fetch`
   // would make the wave wait for the load there, and with it (the counter is in order) for the tile transfers issued
@@ -787,32 +567,9 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
   auto publish = [&]() {
     if (staged_buf < 0) return;
     float* const sb = staged_buf == 0 ? lds_s0 : lds_s1;
-    if constexpr (BLK == 64) {
-      // scaled once here (lse to base 2, delta by the softmax scale) instead of once per score
-      if constexpr (FOLD) sb[64 * wave + lane] = staged_inf ? -INFINITY : wave == 0 ? -staged * inv_scale : -staged;
-      else sb[64 * wave + lane] = staged_inf ? INFINITY : staged * (wave == 0 ? kLog2e : scale);
-    } else {
-      // P of (query, key) counts as often as the key's block lists the query's block: the count goes into the
-      // exponent (lse - log2(count); 0 times: lse = +inf), one variant of the query's value per key block
-      const bool is_lse = hh == 0;
-      const float base = FOLD ? (staged_inf ? -INFINITY : is_lse ? -staged * inv_scale : -staged)
-                              : (staged_inf ? INFINITY : staged * (is_lse ? kLog2e : scale));
-      const bool plain = __ballot(is_lse && (staged_cnt & 0xfefefefeu) != 0) == 0;  // (wave-uniform) no block listed twice
-      float* const to = sb + (is_lse ? 0 : kDeltaAt) + 32 * wave + (lane & 31);
-#pragma unroll
-      for (int kk = 0; kk < 4; kk++) {
-        const uint32_t wgt = (staged_cnt >> (8 * kk)) & 0xffu;
-        float vkk;
-        if constexpr (FOLD) {  // start value of the S accumulator: -(lse - ln(count)) / scale
-          vkk = is_lse && wgt == 0 ? -INFINITY : base;
-          if (!plain && is_lse) vkk += __builtin_amdgcn_logf((float)(wgt > 1 ? wgt : 1)) * (1.0f / sl2);
-        } else {
-          vkk = is_lse && wgt == 0 ? INFINITY : base;
-          if (!plain && is_lse) vkk -= __builtin_amdgcn_logf((float)(wgt > 1 ? wgt : 1));
-        }
-        to[kk * kVar] = vkk;
-      }
-    }
+    // scaled once here (lse to base 2, delta by the softmax scale) instead of once per score
+    if constexpr (FOLD) sb[64 * wave + lane] = staged_inf ? -INFINITY : wave == 0 ? -staged * inv_scale : -staged;
+    else sb[64 * wave + lane] = staged_inf ? INFINITY : staged * (wave == 0 ? kLog2e : scale);
     staged_buf = -1;
   };
   // One tile in three stages per 32-query half (A = row reads + S, dP; B = P and dS from the per-query scalars; C =
@@ -826,7 +583,6 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
     const char* qb = reinterpret_cast<const char*>(BUF == 0 ? lds_q0 : lds_q1);
     const char* gb = reinterpret_cast<const char*>(BUF == 0 ? lds_g0 : lds_g1);
     const float* sb = BUF == 0 ? lds_s0 : lds_s1;
-    const float* sl = sb + lse_at;  // BLK 16: the lse variant of this lane's key block
     f32x16 sc[2], dpv[2];   // S and dP of the two halves
     V8 pbv[2][2], dbv[2][2];  // P and dS as B operands [half][jj]
     V8 aq[4], ag[4];          // row fragments of Q, dO (A operands of the scores)
@@ -846,7 +602,7 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
       if constexpr (FOLD) {
 #pragma unroll
         for (int g4 = 0; g4 < 4; g4++) {
-          const float4 l4 = *reinterpret_cast<const float4*>(sl + 32 * HF + 4 * hh + 8 * g4);
+          const float4 l4 = *reinterpret_cast<const float4*>(sb + 32 * HF + 4 * hh + 8 * g4);
           sc[HF][4 * g4] = l4.x;
           sc[HF][4 * g4 + 1] = l4.y;
           sc[HF][4 * g4 + 2] = l4.z;
@@ -857,7 +613,7 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
     auto delta_init_piece = [&](auto hf_tag, auto g_tag) {  // registers 4g .. 4g+3 of the half's dP accumulator
       constexpr int HF = decltype(hf_tag)::value, g4 = decltype(g_tag)::value;
       if constexpr (FOLD) {
-        const float4 d4 = *reinterpret_cast<const float4*>(sl + kDeltaAt + 32 * HF + 4 * hh + 8 * g4);
+        const float4 d4 = *reinterpret_cast<const float4*>(sb + kDeltaAt + 32 * HF + 4 * hh + 8 * g4);
         dpv[HF][4 * g4] = d4.x;
         dpv[HF][4 * g4 + 1] = d4.y;
         dpv[HF][4 * g4 + 2] = d4.z;
@@ -885,10 +641,10 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
         e0 = LATE_SCALE ? p0 * dh[r] : p0 * (dh[r] * scale);
         e1 = LATE_SCALE ? p1 * dh[r + 1] : p1 * (dh[r + 1] * scale);
       } else {
-        const float2 l2 = *reinterpret_cast<const float2*>(sl + 32 * HF + 4 * hh + 8 * (j >> 1) + 2 * (j & 1));
+        const float2 l2 = *reinterpret_cast<const float2*>(sb + 32 * HF + 4 * hh + 8 * (j >> 1) + 2 * (j & 1));
         p0 = __builtin_amdgcn_exp2f(fmaf(sh[r], sl2, -l2.x));
         p1 = __builtin_amdgcn_exp2f(fmaf(sh[r + 1], sl2, -l2.y));
-        const float2 d2 = *reinterpret_cast<const float2*>(sl + kDeltaAt + 32 * HF + 4 * hh + 8 * (j >> 1) + 2 * (j & 1));
+        const float2 d2 = *reinterpret_cast<const float2*>(sb + kDeltaAt + 32 * HF + 4 * hh + 8 * (j >> 1) + 2 * (j & 1));
         e0 = p0 * fmaf(dh[r], scale, -d2.x);
         e1 = p1 * fmaf(dh[r + 1], scale, -d2.y);
       }
@@ -899,19 +655,8 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
       dv[r & 7] = (E)e0;
       dv[(r & 7) + 1] = (E)e1;
     };
-    if constexpr (BLK == 64) {
-      read_rows<E, true>(qb, c, hh, aq);
-      read_rows<E, true>(gb, c, hh, ag);
-    } else {  // all eight fragments requested at once and waited for by hand: left to itself the compiler, short of
-      // registers further down the tile, reads them one at a time in this instance, each in front of its product
-      u32x4 qw[4], gw[4];
-      read_rows2_sync(qb, gb, c, hh, qw, gw);
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) {
-        aq[ks] = frag_of<E>(qw[ks]);
-        ag[ks] = frag_of<E>(gw[ks]);
-      }
-    }
+    read_rows<E, true>(qb, c, hh, aq);
+    read_rows<E, true>(gb, c, hh, ag);
     delta_init(H0{});
     static_for<8>([&](auto i_tag) { mma_a(H0{}, i_tag); });
     __builtin_amdgcn_sched_barrier(0);
@@ -935,25 +680,9 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
       vec(H1{}, j_tag);
       __builtin_amdgcn_sched_barrier(0);
     });
-    if constexpr (BLK == 64) {
-      read_transposed<E>(gb + kHalfBytes, tr_off, gt);
-      read_transposed<E>(qb + kHalfBytes, tr_off, qt);
-      static_for<8>([&](auto i_tag) { mma_c(H1{}, i_tag); });
-    } else {
-      u32x2 gw[2][2][2], qw[2][2][2];
-      read_transposed_sync(gb + kHalfBytes, tr_off, gw);
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++)
-#pragma unroll
-        for (int dt = 0; dt < 2; dt++) gt[jj][dt] = frag_of<E>(gw[jj][dt][0], gw[jj][dt][1]);
-      static_for<4>([&](auto i_tag) { mma_c(H1{}, i_tag); });
-      read_transposed_sync(qb + kHalfBytes, tr_off, qw);
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++)
-#pragma unroll
-        for (int dt = 0; dt < 2; dt++) qt[jj][dt] = frag_of<E>(qw[jj][dt][0], qw[jj][dt][1]);
-      static_for<4>([&](auto i_tag) { mma_c(H1{}, std::integral_constant<int, decltype(i_tag)::value + 4>{}); });
-    }
+    read_transposed<E>(gb + kHalfBytes, tr_off, gt);
+    read_transposed<E>(qb + kHalfBytes, tr_off, qt);
+    static_for<8>([&](auto i_tag) { mma_c(H1{}, i_tag); });
   };
   // this wave's part of the tile has landed, its reads of the other buffer are done; after the barrier both hold
   // for both waves
@@ -985,129 +714,15 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
   };
   E* dkp = (E*)p.dk + (int64_t)b * p.sdkb + (int64_t)h * p.sdkh;
   E* dvp = (E*)p.dv + (int64_t)b * p.sdvb + (int64_t)h * p.sdvh;
-  if constexpr (BLK == 64) {
-    walk();
-    if constexpr (LATE_SCALE) {
+  walk();
+  if constexpr (LATE_SCALE) {
 #pragma unroll
-      for (int dt = 0; dt < 2; dt++)
+    for (int dt = 0; dt < 2; dt++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) dkt[dt][r] *= scale;
-    }
-    store_rows<E>(dkt, dkp + key * p.sdkn, key < Lk, hh);
-    store_rows<E>(dvt, dvp + key * p.sdvn, key < Lk, hh);
-  } else {
-    // The workgroup's 64 keys are FOUR neighbouring key blocks, whose lists name mostly the same query blocks (at
-    // 266 496 tokens, top-32, the union of the four lists is half as long as the lists together), and the workgroup walks
-    // that union, four distinct query blocks per 64-row tile, with the 64-token kernel's tile code: a probability counts
-    // as often as its key block's list names its query block (`publish`).  The union is built a chunk at a time from
-    // the (ascending) lists: every list offers a window of its next kWin entries; tau = the smallest value that follows
-    // a window; the chunk takes the window entries below tau (the list that sets tau gives its whole window, so the
-    // walk advances; entries at or above tau may have partners in other lists that are not in their windows yet).
-    // Each wave inserts two of the lists into a 512-slot hash table in an idle tile buffer: compare-and-swap on the query
-    // block, linear probing, 1 added to the list's byte of the slot's count; wave 0 then compacts the occupied slots into
-    // lds_union, eight slots per lane, positions from ballots.  Tiles come in the table's order (fp32 summation order
-    // only).  Every list entry is in exactly one chunk, so whatever the chunks' borders, every (query block, key block)
-    // pair is counted as often as listed.
-    constexpr int kWin = kMergeMax / 4;
-    static_assert(kWin > 64 && kWin <= 128, "a window is read with two loads per lane; a query block repeats at most 64 times in a list");
-    const int64_t nkb16 = (Lk + 15) >> 4;
-    const int32_t* lp[4];
-    int llen[4], lpos[4];
-#pragma unroll
-    for (int i4 = 0; i4 < 4; i4++) {
-      const int64_t kblk = (int64_t)kb * 4 + i4;
-      const bool there = kblk < nkb16;
-      const int32_t o0 = there ? __builtin_amdgcn_readfirstlane(off16[kblk]) : 0;
-      const int32_t o1 = there ? __builtin_amdgcn_readfirstlane(off16[kblk + 1]) : 0;
-      lp[i4] = list + o0;
-      llen[i4] = o1 - o0;
-      lpos[i4] = 0;
-    }
-    int32_t* const hkey = reinterpret_cast<int32_t*>(lds_q0);          // [512]
-    uint32_t* const hcnt = reinterpret_cast<uint32_t*>(lds_q0 + 2048);  // [512]
-    auto insert = [&](bool active, int32_t e, uint32_t one) {
-      uint32_t slot = ((uint32_t)e * 0x9E3779B1u) >> 23;
-      while (active) {
-        const int32_t old = atomicCAS(hkey + slot, -1, e);
-        if (old == -1 || old == e) {
-          atomicAdd(hcnt + slot, one);
-          active = false;
-        } else {
-          slot = (slot + 1) & 511u;
-        }
-      }
-    };
-    auto build_chunk = [&]() -> bool {  // false: the lists are exhausted.  Both waves take the same decisions.
-      // all eight loads in one round trip: lane kWin - 64 of a list's second load fetches the value after the window
-      int32_t ev[4][2];
-#pragma unroll
-      for (int i4 = 0; i4 < 4; i4++) {
-        const int i0 = lpos[i4] + lane, i1 = lpos[i4] + 64 + lane;
-        ev[i4][0] = i0 < llen[i4] ? lp[i4][i0] : 0x7fffffff;
-        ev[i4][1] = lane <= kWin - 64 && i1 < llen[i4] ? lp[i4][i1] : 0x7fffffff;
-      }
-      int32_t tau = 0x7fffffff;
-#pragma unroll
-      for (int i4 = 0; i4 < 4; i4++) {
-        const int32_t nextv = __builtin_amdgcn_readlane(ev[i4][1], kWin - 64);
-        tau = nextv < tau ? nextv : tau;
-        if (lane == kWin - 64) ev[i4][1] = 0x7fffffff;  // not part of the window
-      }
-      int taken[4], total = 0;
-#pragma unroll
-      for (int i4 = 0; i4 < 4; i4++) {
-        taken[i4] = __popcll(__ballot(ev[i4][0] < tau)) + __popcll(__ballot(ev[i4][1] < tau));  // a prefix: the list is ascending
-        total += taken[i4];
-      }
-      if (total == 0) return false;
-      __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0): this wave is through the previous chunk's tiles
-      __syncthreads();                      // ... and so is the other one: the table's buffer and the list are free
-      reinterpret_cast<int4*>(hkey)[threadIdx.x] = make_int4(-1, -1, -1, -1);
-      reinterpret_cast<int4*>(hcnt)[threadIdx.x] = make_int4(0, 0, 0, 0);
-      __syncthreads();
-#pragma unroll
-      for (int i4 = 0; i4 < 4; i4++) {
-        if ((i4 >> 1) == wave) {  // (wave-uniform) this wave's two lists
-          insert(ev[i4][0] < tau, ev[i4][0], 1u << (8 * i4));
-          insert(ev[i4][1] < tau, ev[i4][1], 1u << (8 * i4));
-        }
-        lpos[i4] += taken[i4];
-      }
-      __syncthreads();
-      if (wave == 0) {
-        const int4 k0 = reinterpret_cast<const int4*>(hkey)[2 * lane], k1 = reinterpret_cast<const int4*>(hkey)[2 * lane + 1];
-        const int4 c0 = reinterpret_cast<const int4*>(hcnt)[2 * lane], c1 = reinterpret_cast<const int4*>(hcnt)[2 * lane + 1];
-        const int32_t ks8[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-        const int32_t cs8[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-        uint32_t at = 0;  // occupied slots of the lanes below
-        int n_union = 0;
-#pragma unroll
-        for (int s8 = 0; s8 < 8; s8++) {
-          const uint64_t m = __ballot(ks8[s8] >= 0);
-          at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, at));
-          n_union += __popcll(m);
-        }
-#pragma unroll
-        for (int s8 = 0; s8 < 8; s8++)
-          if (ks8[s8] >= 0) lds_union[at++] = make_int2(ks8[s8], cs8[s8]);
-        if (lane < 4) lds_union[n_union + lane] = make_int2(-1, 0);  // the last tile's missing entries
-        if (lane == 0) lds_union[kMergeMax + 7] = make_int2(n_union, 0);
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the table is read before the first transfer lands on it
-      }
-      __syncthreads();
-      n_lists = (__builtin_amdgcn_readfirstlane(lds_union[kMergeMax + 7].x) + 3) >> 2;  // tiles of this chunk
-      return true;
-    };
-    while (build_chunk()) walk();
-    if constexpr (LATE_SCALE) {
-#pragma unroll
-      for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) dkt[dt][r] *= scale;
-    }
-    store_rows<E>(dkt, dkp + key * p.sdkn, key < Lk, hh);
-    store_rows<E>(dvt, dvp + key * p.sdvn, key < Lk, hh);
+      for (int r = 0; r < 16; r++) dkt[dt][r] *= scale;
   }
+  store_rows<E>(dkt, dkp + key * p.sdkn, key < Lk, hh);
+  store_rows<E>(dvt, dvp + key * p.sdvn, key < Lk, hh);
 }
 
 }  // namespace bwd
@@ -1115,6 +730,7 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
 int launch_attn_bwd(const BwdParams& p, int dtype, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   const bool dense = p.idx == nullptr;
+  if (!dense && p.block == 16) return launch_attn_bwd16(p, dtype, stream);
   const int64_t nqb = (p.Lq + 63) / 64, nkb = (p.Lk + 63) / 64;
   const int64_t nqg = (nqb + 3) / 4;
   const int64_t total_q = nqg * p.B * p.H, total_k = nkb * p.B * p.H;
@@ -1124,14 +740,12 @@ int launch_attn_bwd(const BwdParams& p, int dtype, void* stream) {
 #define S3R_BWD_LAUNCH(E)                                                                                                       \
   do {                                                                                                                          \
     if (p.dq != nullptr) {                                                                                                      \
-      if (dense) hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, true, 64>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);     \
-      else if (p.block == 16) hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, false, 16>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q); \
-      else hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, false, 64>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);          \
+      if (dense) hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, true>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);     \
+      else hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, false>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);          \
     }                                                                                                                           \
     if (p.dk != nullptr) {                                                                                                      \
-      if (dense) hipLaunchKernelGGL((bwd::bwd_dkdv_kernel<E, true, 64>), gk, bk, 0, st, p, (int)nkb, (int)nqb, (int)total_k);   \
-      else if (p.block == 16) hipLaunchKernelGGL((bwd::bwd_dkdv_kernel<E, false, 16>), gk, bk, 0, st, p, (int)nkb, (int)nqb, (int)total_k); \
-      else hipLaunchKernelGGL((bwd::bwd_dkdv_kernel<E, false, 64>), gk, bk, 0, st, p, (int)nkb, (int)nqb, (int)total_k);        \
+      if (dense) hipLaunchKernelGGL((bwd::bwd_dkdv_kernel<E, true>), gk, bk, 0, st, p, (int)nkb, (int)nqb, (int)total_k);   \
+      else hipLaunchKernelGGL((bwd::bwd_dkdv_kernel<E, false>), gk, bk, 0, st, p, (int)nkb, (int)nqb, (int)total_k);        \
     }                                                                                                                           \
   } while (0)
   if (dtype == S3R_BF16) S3R_BWD_LAUNCH(bf16_t);

@@ -760,10 +760,8 @@ def key_block_lists(idx: torch.Tensor, n_key_blocks: int) -> Tuple[torch.Tensor,
 
 def key_lists_ascending(lists: torch.Tensor, offs: torch.Tensor) -> bool:
     """Whether every group of ``lists`` ([B,H,L] int32, groups delimited by ``offs`` [B,H,n_key_blocks+1]) is ascending,
-    as :func:`key_block_lists` builds them.  The dK/dV kernel for 16-token blocks merges the lists of four neighbouring
-    key blocks and relies on that order: on a list that is not ascending it skips entries and the gradients come out
-    incomplete WITHOUT an error.  Works on CPU and GPU tensors (on the GPU: a few small kernels and one
-    synchronisation)."""
+    as :func:`key_block_lists` builds them.  The dK/dV kernels add up in the order of a list, so that another order gives
+    other roundings.  Works on CPU and GPU tensors (on the GPU: a few small kernels and one synchronisation)."""
     b, h, length = lists.shape
     if length < 2:
         return True
@@ -797,8 +795,8 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     """Gradients ``(dq, dk, dv)`` of an attention forward with output ``o`` and log-sum-exp ``lse``:
     selection attention over the blocks of ``idx`` ([B,H,Nq_blocks,K] int32), or dense attention (``idx=None``).
     ``delta`` (:func:`attn_bwd_delta`) and ``key_lists`` (:func:`key_block_lists`) are computed here unless given.
-    Caller-built ``key_lists`` must be ascending within every group (see :func:`key_lists_ascending`: with 16-token
-    blocks anything else gives silently incomplete dk, dv); ``check_lists=True`` (default: the environment variable
+    Caller-built ``key_lists`` must be ascending within every group (see :func:`key_lists_ascending`);
+    ``check_lists=True`` (default: the environment variable
     ``S3R_CHECK_LISTS=1``) verifies that here, at the price of a device synchronisation."""
     _need_device(q, k, v, o, dout, lse)
     assert bwd_supported(q, block), "attention backward: built for bf16/fp16, head_dim 64, block 64 or 16"
