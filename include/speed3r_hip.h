@@ -340,6 +340,20 @@ int s3r_qkv_project(const void* x, const void* w, const void* bias, int64_t ldx,
 int s3r_qkv_project_gate_rides(int64_t rows, int H);
 
 /*
+ * The attention layer's inference (pi3/models/layers/sparse_attention.py:90-141) in one call: s3r_qkv_project with its gate,
+ * s3r_compressed_attn_topk with indices, s3r_gate where that does not ride, s3r_select_attn_merge and, with proj_w, s3r_linear, one after
+ * the other on `stream`: the same results.  Few tokens wait for the host, which makes one call instead of five.
+ *   a: as for s3r_qkv_project with means and norms, but its outputs (q_out .. v_pool) are not read: they lie in `workspace`,
+ *   s3r_attention_layer_workspace bytes at a multiple of 256; gate_w: [2 H, C]; proj_w: [C, C] or NULL (out is then the merged
+ *   branches); out: contiguous [B*N, C]; all weights contiguous, 16-byte aligned, in a->dtype.
+ * K: 1, 2, 4, 8, 16 or 32.  The gate: 2 H outputs a multiple of 4 up to 32 that ride, or H a multiple of 4 up to 16.
+ */
+int64_t s3r_attention_layer_workspace(int B, int H, int64_t N, int block, int K, int with_projection);
+int s3r_attention_layer(const void* x, const void* qkv_w, const void* qkv_bias, const void* gate_w, const void* gate_bias,
+                        const void* proj_w, const void* proj_bias, void* out, void* workspace, int64_t workspace_bytes,
+                        const struct s3r_prepass_args* a, int K, float softmax_scale, void* stream);
+
+/*
  * The layer's gate  out[r,:] = sigmoid(x[r,:] W^T + bias)  (pi3/models/layers/sparse_attention.py:88,127); fp32 sums, the
  * product with its bias and the sigmoid each rounded to the I/O dtype.
  *   x: contiguous [rows, C], w: contiguous [O, C], bias: [O] or NULL, out: contiguous [rows, O]; bf16 / fp16, C a multiple of

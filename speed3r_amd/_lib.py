@@ -50,6 +50,8 @@ SIGNATURES = {
     "s3r_linear_wgrad_workspace": (c_int64, [c_int64, c_int, c_int, c_int64, c_int64]),
     "s3r_linear_wgrad": (c_int, [c_void_p] * 5 + [c_int64, c_int, c_int, c_int64, c_int64, c_int, c_void_p]),
     "s3r_qkv_project": (c_int, [c_void_p] * 3 + [c_int64, c_int64] + [c_void_p] * 5 + [c_int, c_void_p]),
+    "s3r_attention_layer_workspace": (c_int64, [c_int, c_int, c_int64, c_int, c_int, c_int]),
+    "s3r_attention_layer": (c_int, [c_void_p] * 9 + [c_int64, c_void_p, c_int, c_float, c_void_p]),
     "s3r_qkv_project_gate_rides": (c_int, [c_int64, c_int]),
     "s3r_gate": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
     "s3r_add_layer_norm": (c_int, [c_void_p] * 7 + [c_float, c_int64, c_int, c_int, c_void_p]),

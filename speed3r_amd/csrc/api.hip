@@ -282,3 +282,69 @@ extern "C" int s3r_attn_bwd(const void* q, const void* k, const void* v, const v
   p.scale = softmax_scale;
   return launch_attn_bwd(p, dtype, stream);
 }
+
+// ---- the attention layer in one call ------------------------------------------------------------------------------
+// What the layer holds between its kernels, in the order of its workspace (each part at a multiple of 256 bytes).
+namespace {
+struct LayerParts {
+  int64_t q, k, v, qc, kc, vc, oc, idx, gate, merged, bytes;
+};
+LayerParts layer_parts(int64_t B, int64_t H, int64_t N, int block, int K, bool merged) {
+  LayerParts l;
+  int64_t at = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t here = at;
+    at += (bytes + 255) / 256 * 256;
+    return here;
+  };
+  const int64_t tokens = B * H * N * 128, means = B * H * ((N + block - 1) / block) * 128;
+  l.q = take(tokens); l.k = take(tokens); l.v = take(tokens);
+  l.qc = take(means); l.kc = take(means); l.vc = take(means); l.oc = take(means);
+  l.idx = take(means / 32 * K);
+  l.gate = take(B * N * H * 4);
+  l.merged = take(merged ? tokens : 0);
+  l.bytes = at;
+  return l;
+}
+}  // namespace
+
+extern "C" int64_t s3r_attention_layer_workspace(int B, int H, int64_t N, int block, int K, int with_projection) {
+  if (B <= 0 || H <= 0 || N <= 0 || block <= 0 || K <= 0) return 0;
+  return layer_parts(B, H, N, block, K, with_projection != 0).bytes;
+}
+
+extern "C" int s3r_attention_layer(const void* x, const void* qkv_w, const void* qkv_bias, const void* gate_w, const void* gate_bias,
+                                   const void* proj_w, const void* proj_bias, void* out, void* workspace, int64_t workspace_bytes,
+                                   const s3r_prepass_args* a, int K, float softmax_scale, void* stream) {
+  if (!a || !x || !gate_w || !out || !workspace) return fail(S3R_ERR_BAD_ARG, "s3r_attention_layer: null pointer");
+  if (a->B <= 0 || a->H <= 0 || a->N <= 0 || K <= 0) return fail(S3R_ERR_BAD_ARG, "s3r_attention_layer: non-positive size");
+  if ((a->block != 16 && a->block != 64) || !compressed_fused_topk_available(K))
+    return fail(S3R_ERR_UNSUPPORTED, "s3r_attention_layer: blocks of %d tokens, top-k %d (built for 16 or 64 and powers of two up to 32)", a->block, K);
+  const int B = a->B, H = a->H, C = 64 * H, O = 2 * H;
+  const int64_t N = a->N, M = (int64_t)B * N, Nc = (N + a->block - 1) / a->block;
+  // (everything that a later kernel may refuse is refused before the first one runs)
+  const bool rides = s3r_qkv_project_gate_rides(M, H) && O % 4 == 0 && O <= 32;
+  if (!rides && (C % 256 || C > 1024 || O > 32)) return fail(S3R_ERR_UNSUPPORTED, "s3r_attention_layer: a gate of %d heads", H);
+  if (Nc > (1 << 21) || (proj_w != nullptr && !aligned16(proj_w)) || !aligned16(gate_w) || (reinterpret_cast<uintptr_t>(proj_bias) & 15u))
+    return fail(S3R_ERR_UNSUPPORTED, "s3r_attention_layer: more than 2^21 blocks, or weights that are no multiples of 16 bytes");
+  const LayerParts l = layer_parts(B, H, N, a->block, K, proj_w != nullptr);
+  if (workspace_bytes < l.bytes || (reinterpret_cast<uintptr_t>(workspace) & 255u) || !aligned16(out))
+    return fail(S3R_ERR_BAD_ARG, "s3r_attention_layer: the workspace needs %lld bytes at a multiple of 256", (long long)l.bytes);
+  char* const ws = (char*)workspace;
+  void *q = ws + l.q, *k = ws + l.k, *v = ws + l.v, *oc = ws + l.oc, *gate = ws + l.gate, *merged = proj_w != nullptr ? ws + l.merged : out;
+  int32_t* const idx = (int32_t*)(ws + l.idx);
+  s3r_prepass_args pa = *a;
+  pa.q_out = q; pa.k_out = k; pa.q_pool = ws + l.qc; pa.k_pool = ws + l.kc; pa.v_pool = ws + l.vc; pa.finish_pooled = 1;
+  const int64_t hb = H * N * 64, hc = H * Nc * 64;
+  int rc = s3r_qkv_project(x, qkv_w, qkv_bias, C, C, v, &pa, rides ? gate_w : nullptr, rides ? gate_bias : nullptr, rides ? gate : nullptr,
+                           rides ? O : 0, stream);
+  if (rc == S3R_OK)
+    rc = s3r_compressed_attn_topk(pa.q_pool, pa.k_pool, pa.v_pool, oc, nullptr, idx, nullptr, B, H, (int)Nc, (int)Nc, 64, K, hc, Nc * 64, 64,
+                                  hc, Nc * 64, 64, hc, Nc * 64, 64, hc, Nc * 64, 64, softmax_scale, a->dtype, stream);
+  if (rc == S3R_OK && !rides) rc = s3r_gate(x, gate_w, gate_bias, gate, M, C, O, a->dtype, stream);
+  if (rc == S3R_OK)
+    rc = s3r_select_attn_merge(q, k, v, idx, oc, gate, merged, B, H, N, 64, a->block, K, hb, N * 64, 64, hb, N * 64, 64, hb, N * 64, 64,
+                               H * Nc * K, Nc * K, K, hc, Nc * 64, 64, N * O, 2, O, softmax_scale, a->dtype, stream);
+  if (rc == S3R_OK && proj_w != nullptr) rc = s3r_linear(merged, proj_w, proj_bias, out, M, C, C, C, C, C, 0, a->dtype, stream);
+  return rc;
+}

@@ -43,5 +43,6 @@ constexpr int64_t kMostKeys = 1216;
 bool topk_lds_pays(const AttnParams& p);  // top-k indices alone: neither too few nor too many keys for the list, at most kMostKeys, and not too many rows
 int launch_topk_lds(const AttnParams& p, int dtype, void* stream);
 int launch_compressed_mfma(const AttnParams& p, int dtype, void* stream);
+bool compressed_fused_topk_available(int K);
 
 }  // namespace s3r

@@ -114,16 +114,21 @@ def linear(m: nn.Linear, x: Tensor, gelu: bool = False, trains: Optional[bool] =
     return nn.functional.gelu(m(x)) if gelu else m(x)
 
 
-def project(attn: nn.Module, x: Tensor, pos: Optional[Tensor], n_pos: Optional[int], block: int, pooled: bool, gate=None):
-    """The projection of an attention layer with all that follows it row by row, and the layer's gate (weight, bias) beside it
-    (``ops.qkv_project``), or None where the kernel does not take the layer or does not stand in for its modules (then:
-    ``linear`` and the passes over its result)."""
+def project_args(attn: nn.Module, x: Tensor, pos: Optional[Tensor], n_pos: Optional[int], block: int, pooled: bool):
+    """:func:`fused_qk_args` of a layer's projection with all that follows it row by row, or None where the kernel does not take the
+    layer or does not stand in for its modules (then: ``linear`` and the passes over its result)."""
     # (asked before the tables are, which the passes over the projection ask for again and a rope of another kind looks at the positions for)
     if pos is None or not linear_takes(attn.qkv, x) or pos.is_floating_point() or x.dim() != 3 \
             or not ops.qkv_project_takes(x, attn.num_heads, block, pooled, isinstance(attn.q_norm, nn.LayerNorm)):
         return None
     fused = fused_qk_args(attn, x, pos, n_pos, takes=True)
-    if fused is None or fused[0].shape != (*x.shape[:2], 2):
+    return fused if fused is not None and fused[0].shape == (*x.shape[:2], 2) else None
+
+
+def project(attn: nn.Module, x: Tensor, fused, block: int, pooled: bool, gate=None):
+    """The projection of an attention layer with what :func:`project_args` said, and the layer's gate (weight, bias) beside it
+    (``ops.qkv_project``); None where there is nothing to say."""
+    if fused is None:
         return None
     return ops.qkv_project(x, attn.qkv.weight, attn.qkv.bias, attn.num_heads, block, *fused[:3], *fused[4:], pooled=pooled, inv_freq=fused[3],
                            gate=gate, takes=True)
@@ -339,7 +344,18 @@ class SparseFlashAttentionRope(nn.Module):
         gate = None
         projected = None
         if pos is not None and enough_work(x):
-            projected = project(self, x, pos, n_pos, block, True, (self.gate[0].weight, self.gate[0].bias) if self._plain_gate() else None)
+            args = project_args(self, x, pos, n_pos, block, True)
+            gate_args = (self.gate[0].weight, self.gate[0].bias) if args is not None and self._plain_gate() else None
+            if gate_args is not None and not self.keep_topk_idx:
+                # all of the layer in one call where the kernels follow each other on this stream: 2 016 tokens of 1024 channels
+                # wait for the host, 126 us with a call a kernel, 81 with one
+                with_proj = linear_takes(self.proj, x, False)
+                out = ops.attention_layer(x, (self.qkv.weight, self.qkv.bias), gate_args, (self.proj.weight, self.proj.bias) if with_proj else None,
+                                          h, block, self.topk, *args[:3], *args[4:], args[3])
+                if out is not None:
+                    self.last_prepass, self.last_passes, self.last_path = True, 1, "fused-merge"
+                    return self.proj_drop(out if with_proj else linear(self.proj, out))
+            projected = project(self, x, args, block, True, gate_args)
         if projected is None:
             qkv = linear(self.qkv, x)                                  # [B, N, 3C], layout (qkv h d)
             fused = fused_qk_args(self, qkv, pos, n_pos)

@@ -37,7 +37,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from ..layers import RoPE2D, SparseFlashAttentionRope
-from ..layers.sparse_attention import calls_forward_only, fused_qk_args, linear, norm_rope_fused_or_eager, project, training_pays
+from ..layers.sparse_attention import calls_forward_only, fused_qk_args, linear, norm_rope_fused_or_eager, project, project_args, training_pays
 from ..sparse_attn import ops
 from .token_order import tile_major, tile_major_inverse
 
@@ -115,7 +115,7 @@ class DenseAttentionRope(nn.Module):
         b, n, c = x.shape
         h = self.num_heads
         pos = xpos if self.rope is not None else None
-        projected = project(self, x, pos, n_pos, 64, False) if not torch.is_grad_enabled() else None
+        projected = project(self, x, project_args(self, x, pos, n_pos, 64, False), 64, False) if not torch.is_grad_enabled() else None
         if projected is None:
             qkv = product(self.qkv, x, layer=True)
             fused = fused_qk_args(self, qkv, pos, n_pos) if not torch.is_grad_enabled() else None

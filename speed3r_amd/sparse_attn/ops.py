@@ -673,6 +673,43 @@ def qkv_project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     return (q, k, v, *means, *gates)
 
 
+def attention_layer(x: torch.Tensor, qkv, gate, proj, num_heads: int, block: int, topk: int, positions: torch.Tensor, cos_tab: torch.Tensor,
+                    sin_tab: torch.Tensor, q_ln, k_ln, eps: float, inv_freq: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """The layer's inference in one call of the library: :func:`qkv_project` with means and the gate, :func:`compressed_attn_topk`,
+    :func:`gate` where it does not ride, :func:`select_attn_merge` and, unless ``proj`` is None, :func:`linear`: the same kernels in the
+    same order, the same results.  ``qkv``, ``gate``, ``proj``: (weight, bias).  For tokens that :func:`qkv_project_takes` (with means and
+    norms), on the calling stream alone (not where :func:`_side_stream_pays`).
+
+    Returns None where the library has no kernels: top-k a power of two up to 32, contiguous 16-byte aligned weights of one dtype,
+    a gate of 2 outputs per head that one of its kernels takes."""
+    b, n, c = x.shape
+    h = num_heads
+    if topk not in (1, 2, 4, 8, 16, 32) or _side_stream_pays(b * h, -(-n // block), topk):
+        return None
+    dtype, device = x.dtype, x.device
+    for lin, rows in ((qkv, 3 * c), (gate, 2 * h), (proj, c)):
+        if lin is None:
+            continue
+        w, bias = lin
+        if w.shape != (rows, c) or w.dtype != dtype or w.device != device or not w.is_contiguous() or w.data_ptr() % 16:
+            return None
+        if bias is not None and (bias.shape != (rows,) or bias.dtype != dtype or bias.device != device or not bias.is_contiguous()
+                                 or bias.data_ptr() % 16):
+            return None
+    if x.data_ptr() % 16 or c % 256 or c > 1024:
+        return None
+    a, keep = _prepass_args(x, h, block, positions, cos_tab, sin_tab, q_ln, k_ln, float(eps), inv_freq)
+    lib = _lib.lib()
+    out = torch.empty_like(x)
+    size = lib.s3r_attention_layer_workspace(b, h, n, block, topk, proj is not None)
+    with _on(device):
+        ws = torch.empty((size,), dtype=torch.uint8, device=device)
+        rc = lib.s3r_attention_layer(x.data_ptr(), *(t.data_ptr() if t is not None else None for t in (*qkv, *gate, *(proj or (None, None)))),
+                                     out.data_ptr(), ws.data_ptr(), size, ctypes.byref(a), topk, 0.125, _stream(x))
+    _lib.check(rc, "s3r_attention_layer")
+    return out
+
+
 def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """``sigmoid(F.linear(x, weight, bias))`` for the few outputs of the layer's gate, in one pass over ``x`` (inference).
 
