@@ -3,9 +3,14 @@
 //
 // Bound: the fp32 matrix instructions (v_mfma_f32_16x16x4_f32: 64 FLOP per cycle and SIMD, 157 TFLOP/s; a product of
 // 8192 x 8192 matrices by the library reaches 154).  At 8 328 tokens x 16 heads, 16 blocks of 64 (3.5e10 FLOP, 0.23 ms)
-// the generic kernel, whose vector FMAs wait for one LDS read per four products, takes 1.36 ms, this one 0.34 ms; at
-// 16-token blocks, top-32, 4.8 and 0.24 ms.  What is left: 38 us per 1 041 tokens = 73 % of the matrix rate (the vector
-// instructions of the softmax do not overlap with it fully) plus 45 us for the last wave of a SIMD.
+// the generic kernel, whose vector FMAs wait for one LDS read per four products, takes 1.36 ms, this one 0.29 ms; at
+// 16-token blocks, top-32, 4.8 and 0.22 ms.  The vector instructions of the softmax hardly overlap with these products (they
+// share the SIMD's FMA units), so what a probability costs beside its products is what is lost.  Base 2 with one constant
+// (scale log2(e)): a fused multiply-add, an exponential and an addition, in place of exp(x) from exp2 with the rounding of
+// x log2(e) put back (ten instructions): 342 -> 316 us.  A reference that moves only when a score exceeds it by
+// kSlack, in place of the running maximum, whose exchange between lanes every stage waited for: 316 -> 307.  Error against 64 bits
+// over 5 scales of the inputs: 0.65e-6 to 2.34e-6 before and after.  Half blocks at the end of a launch (launch_t): 307 ->
+// 292.  What is left: 33 us per 1 041 tokens = 86 % of the matrix rate, and 28 us beside them (the first loads, a SIMD's last waves).
 //
 // One wave owns 16 query rows: S^T = K Q^T puts one query per lane (column c = lane % 16) and four keys of every
 // 16-key group (4 g + r, g = lane / 16), so the probabilities are already the B operand of O^T = V^T P^T and never
@@ -25,44 +30,48 @@ namespace s3r {
 namespace f32 {
 using namespace sel;
 
+constexpr float kLn2 = 0.693147182f, kLn2Lo = -1.90465421e-9f;  // ln 2 = their sum
 constexpr int kRow = 256;  // bytes of a K or V row
 
-// exp(x) for x <= 0 to about one unit in the last place: exp2 of the product x log2(e), corrected by what its rounding
-// left out (without the correction the error grows with |x|).  Arguments below -200 (exp is 0 from -104 on) give 0.
-__device__ __forceinline__ float exp_nonpos(float x) {
-  constexpr float kHi = 1.44269502f, kLo = 1.92596303e-8f, kLn2 = 0.693147181f;  // log2(e) = kHi + kLo
-  x = x < -200.f ? -200.f : x;
-  const float t = x * kHi;
-  const float e = fmaf(x, kLo, fmaf(x, kHi, -t));
-  const float y = __builtin_amdgcn_exp2f(t);
-  return fmaf(y, e * kLn2, y);
+// Base-2 units by which a score may exceed the row's reference: probabilities and sums scale with 2^kSlack, their
+// relative errors do not.
+constexpr float kSlack = 4.f;
+// ln(l 2^m): the exponent of l joins m, so that the logarithm of what is left is small and the sum is rounded once
+__device__ __forceinline__ float log_sum(float m, float l) {
+  if (!(l > 0.f)) return -INFINITY;
+  const float e = m + (float)__builtin_amdgcn_frexp_expf(l);
+  return fmaf(e, kLn2, fmaf(e, kLn2Lo, logf(__builtin_amdgcn_frexp_mantf(l))));
 }
-
 // W waves share a workgroup's 16 W query rows and its stages of KS keys.  SELECT: the rows are one query block of 16 W
-// tokens, the stages the parts of its listed key blocks; otherwise every key.
-template <int W, int KS, int BLK>
-__global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int ngrp, int total) {
+// tokens, the stages the parts of its listed key blocks; otherwise every key.  SPLIT: workgroups from number `whole` on take half
+// a block's rows each; two waves share 16 rows, each takes one half of every stage, and the first adds up what the two have.
+template <int W, int KS, int BLK, bool SPLIT>
+__global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int ngrp, int total, int whole) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[KS * kRow], lds_k1[KS * kRow];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_v0[KS * kRow], lds_v1[KS * kRow];
   constexpr bool SELECT = BLK > 0;
   constexpr int SUB = SELECT ? BLK / KS : 1, NG = KS / 16, NI = KS / (4 * W);
   static_assert(!SELECT || (BLK % KS == 0 && BLK % (16 * W) == 0), "a block is a whole number of stages and of workgroups");
+  static_assert(!SPLIT || (SELECT && W == 4 && NG == 2), "four waves as two row groups and two halves of a stage");
   static_assert(NI * 4 * W == KS, "every wave moves the same number of 1 KB pieces");
 
   const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
   // each XCD takes a contiguous range of query blocks: neighbours list mostly the same key blocks
-  const int w = blockIdx.x;
-  const int xcd = w & 7, per = total >> 3, rem = total & 7;
-  const int vid = xcd * per + (xcd < rem ? xcd : rem) + (w >> 3);
+  const bool half = SPLIT && (int)blockIdx.x >= whole;  // this workgroup takes half a block's rows
+  const int w = half ? blockIdx.x - whole : blockIdx.x, items = half ? 2 * (total - whole) : SPLIT ? whole : total;
+  const int xcd = w & 7, per = items >> 3, rem = items & 7;
+  const int item = xcd * per + (xcd < rem ? xcd : rem) + (w >> 3);
+  const int vid = half ? whole + (item >> 1) : item;
   const int bh = vid / ngrp;
   const int64_t row0 = (int64_t)(vid - bh * ngrp) * (16 * W);
+  const int rows_at = half ? (item & 1) * 32 + (wave & 1) * 16 : wave * 16, part = half ? wave >> 1 : 0;
   const int b = bh / p.H;
   const int h = bh - b * p.H;
 
   const int64_t N = p.Lk;
-  const int64_t qrow = row0 + wave * 16 + c;
+  const int64_t qrow = row0 + rows_at + c;
   const bool live = qrow < p.Lq;
   const float* qp = (const float*)p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh;
   const float* kp = (const float*)p.k + (int64_t)b * p.skb + (int64_t)h * p.skh;
@@ -115,6 +124,8 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
 #pragma unroll
   for (int s = 0; s < 16; s++) q[s] = live ? qp[qrow * p.sqm + 4 * s + g] : 0.f;
 
+  const float sl2 = (float)((double)p.scale * 1.4426950408889634);
+
   f32x4 o[4];
 #pragma unroll
   for (int dg = 0; dg < 4; dg++)
@@ -122,8 +133,9 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
     for (int r = 0; r < 4; r++) o[dg][r] = 0.f;
   float m_i = -INFINITY, l_i = 0.f;
 
-  auto compute = [&](int64_t s0, const unsigned char* kb, const unsigned char* vb) {
-    const int nvalid = (int)(N - s0 < KS ? N - s0 : KS);
+  auto compute = [&](auto groups, int64_t s0, const unsigned char* kb, const unsigned char* vb) {
+    constexpr int NG = decltype(groups)::value, KC = 16 * NG;
+    const int nvalid = (int)(N - s0 < KC ? N - s0 : KC);
     f32x4 st[NG];
 #pragma unroll
     for (int kg = 0; kg < NG; kg++)
@@ -146,7 +158,7 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
             if (kg * 16 + 4 * g + r < nvalid) srow[kg * 16 + 4 * g + r] = st[kg][r];
       }
     }
-    if (nvalid < KS) {  // (wave-uniform) the ragged end of the sequence
+    if (nvalid < KC) {  // (wave-uniform) the ragged end of the sequence
 #pragma unroll
       for (int kg = 0; kg < NG; kg++)
 #pragma unroll
@@ -158,23 +170,23 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
     for (int kg = 0; kg < NG; kg++)
 #pragma unroll
       for (int r = 0; r < 4; r++) mx = fmaxf(mx, st[kg][r]);
-    mx = xh_max(fmaxf(mx, lane_xor<16>(mx))) * p.scale;  // scale > 0: the maximum of the scaled scores
-    const float m_new = fmaxf(m_i, mx);
-    if (__any(m_new != m_i)) {
-      const float alpha = m_i == -INFINITY ? 0.f : exp_nonpos(m_i - m_new);
+    if (__any(mx * sl2 > m_i + kSlack)) {  // scale > 0
+      mx = xh_max(fmaxf(mx, lane_xor<16>(mx))) * sl2;
+      const float m_new = fmaxf(m_i, mx);
+      const float alpha = m_i == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_i - m_new);
       l_i *= alpha;
 #pragma unroll
       for (int dg = 0; dg < 4; dg++)
 #pragma unroll
         for (int r = 0; r < 4; r++) o[dg][r] *= alpha;
+      m_i = m_new;
     }
-    m_i = m_new;
-    const float m_neg = m_new == -INFINITY ? 0.f : -m_new;
+    const float m_neg = m_i == -INFINITY ? 0.f : -m_i;
 #pragma unroll
     for (int kg = 0; kg < NG; kg++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const float pv = exp_nonpos(fmaf(st[kg][r], p.scale, m_neg));
+        const float pv = __builtin_amdgcn_exp2f(fmaf(st[kg][r], sl2, m_neg));
         l_i += pv;
         const float4 vf = *reinterpret_cast<const float4*>(vb + (kg * 16 + 4 * g + r) * kRow + c * 16);
         o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf.x, pv, o[0], 0, 0, 0);
@@ -193,22 +205,56 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
     if constexpr (W > 1) __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  first();
-  if (start >= 0) {
-    request(start, lds_k0, lds_v0);
+  auto sweep = [&](auto groups) __attribute__((always_inline)) {
+    const int at = part * (16 * kRow);
     while (true) {
       int64_t cur = start;
       advance();
       ready();
       if (start >= 0) request(start, lds_k1, lds_v1);
-      compute(cur, lds_k0, lds_v0);
+      compute(groups, cur + 16 * part, lds_k0 + at, lds_v0 + at);
       if (start < 0) break;
       cur = start;
       advance();
       ready();
       if (start >= 0) request(start, lds_k0, lds_v0);
-      compute(cur, lds_k1, lds_v1);
+      compute(groups, cur + 16 * part, lds_k1 + at, lds_v1 + at);
       if (start < 0) break;
+    }
+  };
+  first();
+  if (start >= 0) {
+    request(start, lds_k0, lds_v0);
+    if constexpr (SPLIT) {
+      if (half) sweep(std::integral_constant<int, 1>{});
+      else sweep(std::integral_constant<int, NG>{});
+    } else {
+      sweep(std::integral_constant<int, NG>{});
+    }
+  }
+  if constexpr (SPLIT) {
+    if (half) {  // the waves of the stages' second halves hand over to those of the first ones
+      __syncthreads();
+      float* const to = reinterpret_cast<float*>((wave & 1) ? lds_k1 : lds_k0);
+      float* const stat = reinterpret_cast<float*>(lds_v0) + (wave & 1) * 128;
+      if (part == 1) {
+#pragma unroll
+        for (int dg = 0; dg < 4; dg++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) to[(dg * 4 + r) * 64 + lane] = o[dg][r];
+        stat[lane] = m_i;
+        stat[64 + lane] = l_i;
+      }
+      __syncthreads();
+      if (part == 1) return;
+      const float m1 = stat[lane], m_new = fmaxf(m_i, m1);
+      const float a0 = m_i == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_i - m_new), a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - m_new);
+      m_i = m_new;
+      l_i = l_i * a0 + stat[64 + lane] * a1;
+#pragma unroll
+      for (int dg = 0; dg < 4; dg++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) o[dg][r] = o[dg][r] * a0 + to[(dg * 4 + r) * 64 + lane] * a1;
     }
   }
 
@@ -219,15 +265,22 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
 #pragma unroll
     for (int r = 0; r < 4; r++)
       *reinterpret_cast<float4*>(op + 4 * r) = make_float4(o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv);
-    if (p.lse != nullptr && g == 0) p.lse[((int64_t)b * p.H + h) * p.Lq + qrow] = l > 0.f ? m_i + logf(l) : -INFINITY;
+    if (p.lse != nullptr && g == 0) p.lse[((int64_t)b * p.H + h) * p.Lq + qrow] = log_sum(m_i, l);
   }
 }
 
-template <int W, int KS, int BLK> static int launch_t(const AttnParams& p, hipStream_t st) {
+template <int W, int KS, int BLK, bool SPLIT = false> static int launch_t(const AttnParams& p, hipStream_t st) {
   const int64_t ngrp = (p.Lq + 16 * W - 1) / (16 * W);
   const int64_t total = ngrp * p.B * p.H;
-  if (total > 0x7fffffffLL) return fail(S3R_ERR_UNSUPPORTED, "attention: grid too large");
-  hipLaunchKernelGGL((attn_f32_kernel<W, KS, BLK>), dim3((unsigned)total), dim3(64 * W), 0, st, p, (int)ngrp, (int)total);
+  // Blocks over a whole number per CU (256) make one CU in a few work a block longer than the others: where they are so
+  // few that their halves still fit one to a CU, they go in halves.  16 heads, us without and with: 1 041 tokens (16
+  // blocks over) 77 / 62, 1 500 (128 over) 79 / 64, 4 164 (32) 177 / 163, 8 328 (48) 307 / 292; 2 600 (144 over) 111.8 / 112.9,
+  // 700 tokens (176 blocks in all) 36.6 / 37.0.  All blocks in halves: 8 328 tokens 325.
+  const int64_t over = total & 255;
+  const int64_t whole = SPLIT && over <= 128 ? total - over : total;
+  const int64_t grid = whole + 2 * (total - whole);
+  if (grid > 0x7fffffffLL) return fail(S3R_ERR_UNSUPPORTED, "attention: grid too large");
+  hipLaunchKernelGGL((attn_f32_kernel<W, KS, BLK, SPLIT>), dim3((unsigned)grid), dim3(64 * W), 0, st, p, (int)ngrp, (int)total, (int)whole);
   return check_launch("attn_f32_kernel");
 }
 
@@ -236,7 +289,7 @@ template <int W, int KS, int BLK> static int launch_t(const AttnParams& p, hipSt
 int launch_attn_f32(const AttnParams& p, bool select, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   if (select) {
-    if (p.block == 64) return f32::launch_t<4, 32, 64>(p, st);
+    if (p.block == 64) return f32::launch_t<4, 32, 64, true>(p, st);
     if (p.block == 32) return f32::launch_t<2, 32, 32>(p, st);
     return f32::launch_t<1, 16, 16>(p, st);
   }
