@@ -1,0 +1,29 @@
+"""GPU: key-block lists of every length at which their sort changes (one entry per lane, networks of 128, 256 and 512, the workgroup's
+sort beyond), with repeated entries, against a stable sort on the host.  Whole numbers: equal."""
+import pytest
+import torch
+
+from speed3r_amd.sparse_attn import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513])
+def test_lists_of_length(n):
+    gen = torch.Generator().manual_seed(n)
+    nqb, k, nkb = 600, 4, 9
+    idx = torch.full((2, 1, nqb * k), nkb, dtype=torch.int32)      # (beyond the last block: in no list)
+    for b in range(2):                                              # block 3 n times, its neighbours once more and once less
+        where = torch.randperm(nqb * k, generator=gen)
+        idx[b, 0, where[:n]] = 3
+        idx[b, 0, where[n:2 * n + 1]] = 4
+        idx[b, 0, where[2 * n + 1:3 * n]] = 7
+    idx = idx.view(2, 1, nqb, k)
+    lists, off = (t.cpu() for t in ops.key_block_lists(idx.cuda(), nkb))
+    for b in range(2):
+        at = 0
+        for j in range(nkb):
+            want = (idx[b, 0] == j).nonzero()[:, 0]                 # row by row: ascending, a row once per entry
+            assert off[b, 0, j] == at and torch.equal(lists[b, 0, at:at + len(want)].long(), want)
+            at += len(want)
+        assert off[b, 0, nkb] == at
