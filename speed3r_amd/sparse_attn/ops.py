@@ -998,8 +998,9 @@ class _LayerCoreFn(torch.autograd.Function):
         full = attn_bwd(q, k, v, o_s, d_os, lse, idx, block, delta=delta_s)
         q_ln, k_ln = ((q_w, q_b), (k_w, k_b)) if q_w is not None else (None, None)
         d_qkv, d_norm = qkv_prepass_bwd(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, (q_raw, k_raw), (*full, *pooled), inv_freq, signed=True)
-        # (tensors of their own: autograd keeps what it is given as .grad)
-        params = [d_norm[i].to(t.dtype, copy=True) if t is not None else None for i, t in enumerate((q_w, q_b, k_w, k_b))]
+        # (tensors of their own, autograd keeps what it is given as .grad: by one launch, not a copy each)
+        own = iter(torch._foreach_mul([d_norm[i] for i, t in enumerate((q_w, q_b, k_w, k_b)) if t is not None], 1.0) if q_w is not None else ())
+        params = [next(own).to(t.dtype) if t is not None else None for t in (q_w, q_b, k_w, k_b)]
         return d_qkv, d_gate, *params, *([None] * 8)
 
 
