@@ -81,8 +81,9 @@ int s3r_compressed_attn_topk(const void* q, const void* k, const void* v,
                              int64_t svb, int64_t svh, int64_t svn,
                              int64_t sob, int64_t soh, int64_t som,
                              float softmax_scale, int dtype, void* stream);
-/* Whether the indices without a score buffer come from the kernel for short lists of keys, which keeps a row's scores in LDS (else
- * from the one that sweeps over the keys twice); the same indices either way.  batch_heads = B*H. */
+/* Whether the indices without a score buffer come from the kernel for short lists of keys, which keeps a row's scores in LDS, and the
+ * attention output with them in one launch (else from the one that sweeps over the keys twice, and a dense sweep); the same indices
+ * either way.  batch_heads = B*H. */
 int s3r_topk_in_lds(int64_t batch_heads, int64_t Lq, int64_t Lk, int K);
 
 /*

@@ -40,7 +40,7 @@ int launch_attn_f32(const AttnParams& p, bool select, void* stream);  // fp32, h
 int launch_select_pipe(const AttnParams& p, int dtype, void* stream);
 int launch_select_b16(const AttnParams& p, int dtype, void* stream);  // block 16
 constexpr int64_t kMostKeys = 1216;
-bool topk_lds_pays(const AttnParams& p);  // top-k indices alone: neither too few nor too many keys for the list, at most kMostKeys, and not too many rows
+bool topk_lds_pays(const AttnParams& p);  // indices, with the attention output or without: neither too few nor too many keys for the list, at most kMostKeys, and not too many rows
 int launch_topk_lds(const AttnParams& p, int dtype, void* stream);
 int launch_compressed_mfma(const AttnParams& p, int dtype, void* stream);
 bool compressed_fused_topk_available(int K);

@@ -769,6 +769,7 @@ int launch_compressed_mfma(const AttnParams& p, int dtype, void* stream) {
     return fail(S3R_ERR_UNSUPPORTED, "s3r_compressed_attn_topk: fused selection is built for top-k in {1,2,4,8,16,32}; pass a scores buffer");
   if (p.topk_idx != nullptr && (p.Lk > (1 << 21) || p.skn >= (1 << 24)))
     return fail(S3R_ERR_UNSUPPORTED, "s3r_compressed_attn_topk: fused selection is built for Lk <= 2^21 and key strides < 2^24; pass a scores buffer");
+  if (p.topk_idx != nullptr && topk_lds_pays(p)) return launch_topk_lds(p, dtype, stream);  // both in one launch
   if (p.o != nullptr) {
     int rc;
     if (p.Lq == p.Lk && p.sqm > 0 && p.skn > 0 && p.svn > 0 && p.sqm < (1 << 20) && p.skn < (1 << 20) && p.svn < (1 << 20)) {
@@ -785,7 +786,6 @@ int launch_compressed_mfma(const AttnParams& p, int dtype, void* stream) {
     }
     if (rc != S3R_OK) return rc;
   }
-  if (p.topk_idx != nullptr && topk_lds_pays(p)) return launch_topk_lds(p, dtype, stream);
   if (p.topk_idx != nullptr) return dtype == S3R_BF16 ? cmp::launch_e<bf16_t>(p, true, st) : cmp::launch_e<f16_t>(p, true, st);
   return S3R_OK;
 }

@@ -1,5 +1,6 @@
-// Exact top-k block indices of the compressed branch for up to 1216 pooled keys (flash_attention_topk.py:101-157): the scores
-// of 16 query rows against all keys stay in LDS, and a row is selected by one wave that sees all of it.
+// Compressed branch for up to 1216 pooled keys (flash_attention_topk.py:101-157): exact top-k block indices, and in the same launch, by
+// workgroups of their own, the attention output (attend below).  The scores of
+// 16 query rows against all keys stay in LDS, and a row is selected by one wave that sees all of it.
 //
 // The two-sweep kernel (compressed_mfma.hip) meets at a barrier per 64 keys and folds queues of survivors into register lists;
 // with few tiles its chains of barriers, LDS round trips and folds are all there is (1 041 keys, 33 tiles of 32, 16 heads, top-32, alone
@@ -21,15 +22,15 @@
 // in slots that nothing fills.
 //
 // us alone on the chip, two-sweep kernel / this, 16 heads, as many rows as keys: 126 keys, top-32 16 / 8; 504, top-32 40 / 13; 1 041,
-// top-16 46 / 34; 1 200, top-32 66 / 38.  Bound: the vector instructions of the selection, about 700 per row at 1 041 keys.  The instance of
-// five pieces spills 20 scalar registers to lanes of vector registers, the others none.
+// top-16 46 / 34; 1 200, top-32 66 / 38.  Bound: the vector instructions of the selection, about 700 per row at 1 041 keys.  The instances
+// of three to five pieces spill 15 to 32 scalar registers to lanes of vector registers, the others none.
 //
-// Up to kMostKeys keys two workgroups fit a CU (78 KB each).  With more keys one does, and the two phases have nobody to hide
+// Up to kMostKeys keys two workgroups fit a CU (78 KB each; up to 512 keys three, by registers too).  With more keys one does, and the two phases have nobody to hide
 // behind: 2 016 keys, top-32, 95 / 112.  With more than kMostGroups workgroups the two-sweep kernel, which shares its key tiles
 // among more rows, is no longer bound by latency: 24 heads of 1 041 47 / 48, 32 of them 53 / 58, 48 of 756 44 / 46.  Up to
 // top-8 its folds are short, and it is as good from fewer keys on (whole operator, us, top-8: 537 keys 182 / 172, 1 009 287 /
 // 286, 1 201 336 / 344; top-4: 537 145 / 142, 814 191 / 192, 1 009 225 / 230; top-1: 537 136 / 119, 814 156 / 163).
-#include "select_common.h"
+#include "block16.h"
 #include "attn_params.h"
 
 namespace s3r {
@@ -37,22 +38,140 @@ namespace tkl {
 using namespace sel;
 
 constexpr int kRows = 16, kWaves = 8;
+constexpr int kAttnRows = 16 * kWaves;  // query rows of an attention workgroup
+
+// The attention itself, by workgroups of their own in front of the others' grid: 16 query rows a wave, 64 keys and their values at a
+// time through LDS (`lds`: 16 KB), the next step's requested while it computes; 16 x 16 products as in the kernels for 16-token
+// blocks, scaled fp32 scores, running maximum (exchanged between the lanes only in steps that raise it).  As a launch of its own (the
+// selection kernel's dense sweep) a chain of waits with the chip idle around it; here it runs beside the selection.  Attention and
+// indices, us, two launches / one (the indices alone): 16 heads, top-32, 126 pooled tokens 15.0 / 8.0 (7.9), 504 22.6 / 16.9 (12.9), 756
+// 32.1 / 25.3 (20.8), 1 200 52.4 / 46.0 (38.1); top-8 393 20.8 / 13.3; 2 heads 1 200 26.4 / 22.7; 2 x 16 heads 756 45.4 / 44.2.  Bound: the
+// vector instructions that it adds to the selection's.  Two or four waves to a row's keys, for shorter chains: 504 18.9, 1 041 51 against
+// 40.  Error of the output against 64 bits, bf16, scores of standard deviation 0.25 to 9, 126 to 1 041 tokens: 1.6e-3 to 2.4e-3 (before
+// 1.6e-3 to 3.7e-3: queries scaled in bf16), with the log-sum-exp before 1.7e-3 to 2.4e-3; fp16 2.1e-4 to 3.0e-4 (2.1e-4 to 5.2e-4).
+template <typename E> __device__ __forceinline__ void attend(const AttnParams& p, int vid, int groups, unsigned char* lds) {
+  using namespace b16x;
+  typedef typename Mma<E>::V8 V8;
+  typedef typename Mma4<E>::V4 V4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int bh = vid / groups, b = bh / p.H, h = bh - b * p.H;
+  const int row = (vid - bh * groups) * kAttnRows + wave * 16 + c, Lk = (int)p.Lk;
+  const bool live = row < (int)p.Lq;
+  const E* const qp = (const E*)p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh + (int64_t)(live ? row : (int)p.Lq - 1) * p.sqm + 8 * g;
+  V8 bq[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++) bq[ks] = frag_of<E>(*reinterpret_cast<const u32x4*>(qp + 32 * ks));
+  const E* const kp = (const E*)p.k + (int64_t)b * p.skb + (int64_t)h * p.skh + (tid & 7) * 8;
+  const E* const vp = (const E*)p.v + (int64_t)b * p.svb + (int64_t)h * p.svh + (tid & 7) * 8;
+  u32x4 kv, vv;  // this thread's piece of the next step
+  auto fetch = [&](int first) {
+    const int at = first + (tid >> 3), key = at < Lk ? at : Lk - 1;
+    kv = *reinterpret_cast<const u32x4*>(kp + (int64_t)key * p.skn);
+    vv = *reinterpret_cast<const u32x4*>(vp + (int64_t)key * p.svn);
+    if (at >= Lk) vv = (u32x4){0, 0, 0, 0};  // (0 times what the last row holds may be NaN)
+  };
+  const int r16 = (tid >> 3) & 15;
+  unsigned char* const put = lds + (tid >> 7) * 2048 + r16 * 128 + (((tid & 7) ^ swz(r16)) << 4);
+  const int row_off = c * 128 + ((g ^ swz(c)) << 4);
+  const int tr_row = 4 * g + (c >> 2), tr_off = 8192 + tr_row * 128 + ((((c & 3) >> 1) ^ swz(tr_row)) << 4) + (c & 1) * 8;
+  const float sl2 = p.scale * kLog2e;
+  float m = -INFINITY, l = 0.f;  // reference in base 2 (the same in a query's four lanes), sum of this lane's probabilities
+  f32x4 o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; dt++) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  fetch(0);
+  for (int first = 0; first < Lk; first += 64) {
+    *reinterpret_cast<u32x4*>(put) = kv;
+    *reinterpret_cast<u32x4*>(put + 8192) = vv;
+    if (first + 64 < Lk) fetch(first + 64);
+    __syncthreads();
+    f32x4 st[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      st[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      st[t] = mma16<E>(frag_of<E>(*reinterpret_cast<const u32x4*>(lds + row_off + t * 2048)), bq[0], st[t]);
+      st[t] = mma16<E>(frag_of<E>(*reinterpret_cast<const u32x4*>(lds + (row_off ^ 64) + t * 2048)), bq[1], st[t]);
+    }
+    asm volatile("s_nop 7" : "+v"(st[0]), "+v"(st[1]), "+v"(st[2]), "+v"(st[3]));  // (a rare branch behind products, see settle)
+    if (first + 64 > Lk) {
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) st[t][r] = first + 16 * t + 4 * g + r < Lk ? st[t][r] : -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 4; t++) mx = fmaxf(mx, fmaxf(fmaxf(st[t][0], st[t][1]), fmaxf(st[t][2], st[t][3])));
+    mx *= sl2;            // sl2 > 0: the maximum of the scaled scores
+    if (__any(mx > m)) {  // (the first step: unless all of its scores are -inf)
+      mx = fmaxf(m, xh_max(fmaxf(mx, lane_xor<16>(mx))));
+      const float alpha = __builtin_amdgcn_exp2f(m - (mx == -INFINITY ? 0.f : mx));  // 0 while there is none
+      m = mx;
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 4; dt++) o[dt] *= alpha;
+    }
+    const float use = m == -INFINITY ? 0.f : m;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      float x[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) x[r] = __builtin_amdgcn_exp2f(fmaf(st[t][r], sl2, -use));
+      l += (x[0] + x[1]) + (x[2] + x[3]);
+      const V4 pr = pack4<E>(x);
+#pragma unroll
+      for (int dt = 0; dt < 4; dt++) {
+        const s16x4 vt = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(lds + t * 2048 + (tr_off ^ (32 * dt))));
+        o[dt] = Mma4<E>::mma(__builtin_bit_cast(u32x2, vt), pr, o[dt]);
+      }
+    }
+    __syncthreads();  // the step's rows are read
+  }
+  const float sum = xh_sum(l + lane_xor<16>(l));
+  const float inv = sum == 0.f ? 0.f : 1.f / sum;
+  E* const op = (E*)p.o + (int64_t)b * p.sob + (int64_t)h * p.soh + (int64_t)row * p.som;
+#pragma unroll
+  for (int dp = 0; dp < 2; dp++) {  // (the exchange and the stores of the kernels for 16-token blocks)
+    float y[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) y[t][r] = o[2 * dp + t][r] * inv;
+    const u32x2 wa = __builtin_bit_cast(u32x2, pack4<E>(y[0])), wb = __builtin_bit_cast(u32x2, pack4<E>(y[1]));
+    union { uint32_t w[4]; uint4 u; } pc;
+#pragma unroll
+    for (int wi = 0; wi < 2; wi++) {
+      const auto r = __builtin_amdgcn_permlane16_swap(wa[wi], wb[wi], false, false);
+      pc.w[wi] = r[0];
+      pc.w[2 + wi] = r[1];
+    }
+    if (live) *reinterpret_cast<uint4*>(op + 16 * (2 * dp + (g & 1)) + 8 * (g >> 1)) = pc.u;
+  }
+  if (live && p.lse != nullptr && g == 0) p.lse[((int64_t)b * p.H + h) * p.Lq + row] = (m + __builtin_amdgcn_logf(sum)) * 0.6931471805599453f;
+}
 
 __device__ __forceinline__ float sortable_to_float(uint32_t k) {  // the inverse of sortable_key
   return __uint_as_float(k ^ ((k & 0x80000000u) ? 0x80000000u : 0xFFFFFFFFu));
 }
 
 template <typename E, int NC>  // NC: pieces of 256 columns
-__global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, int groups, int total) {
+__global__ __launch_bounds__(64 * kWaves, NC <= 2 ? 6 : 4) void topk_lds_kernel(AttnParams p, int groups, int total, int attn_groups, int attn_total, int attn_wgs) {
   typedef typename Mma<E>::V8 V8;
   // rows of the scores, 4 mod 64 values apart: what 16 lanes on 16 rows touch lies in different banks
   constexpr int stride = (NC == 5 ? (int)kMostKeys : 256 * NC) + 4;
-  __shared__ __attribute__((aligned(16))) float sc[kRows * stride];
+  __shared__ __attribute__((aligned(1024))) float sc[kRows * stride];
+  static_assert(sizeof(sc) >= 16384, "a step of the attention");
+  // the workgroups of a head run on one XCD, whose L2 then holds its keys (attn_wgs is a multiple of 8)
+  const int xcd = blockIdx.x & 7;
+  auto item = [&](int w, int all) { return xcd * (all >> 3) + (xcd < (all & 7) ? xcd : (all & 7)) + (w >> 3); };
+  if ((int)blockIdx.x < attn_wgs) {
+    if ((int)(blockIdx.x >> 3) < (attn_total >> 3) + (xcd < (attn_total & 7) ? 1 : 0))
+      attend<E>(p, item(blockIdx.x, attn_total), attn_groups, reinterpret_cast<unsigned char*>(sc));
+    return;
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int hh = lane >> 5, c = lane & 31;
-  // the row groups of a head run on one XCD, whose L2 then holds its keys
-  const int xcd = blockIdx.x & 7, per = total >> 3, rem = total & 7;
-  const int vid = xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  const int vid = item((int)blockIdx.x - attn_wgs, total);
   const int bh = vid / groups, g = vid - bh * groups;
   const int b = bh / p.H, h = bh - b * p.H;
   const int Lk = (int)p.Lk, q0 = g * kRows;
@@ -287,7 +406,10 @@ __global__ __launch_bounds__(64 * kWaves, 4) void topk_lds_kernel(AttnParams p, 
 
 template <typename E> static int launch(const AttnParams& p, hipStream_t st) {
   const int64_t groups = (p.Lq + kRows - 1) / kRows, total = groups * p.B * p.H;
-#define S3R_TKL(NC) hipLaunchKernelGGL((topk_lds_kernel<E, NC>), dim3((unsigned)total), dim3(64 * kWaves), 0, st, p, (int)groups, (int)total)
+  const int64_t attn_groups = p.o != nullptr ? (p.Lq + kAttnRows - 1) / kAttnRows : 0, attn = attn_groups * p.B * p.H, attn_wgs = (attn + 7) / 8 * 8;
+#define S3R_TKL(NC)                                                                                                                         \
+  hipLaunchKernelGGL((topk_lds_kernel<E, NC>), dim3((unsigned)(attn_wgs + total)), dim3(64 * kWaves), 0, st, p, (int)groups, (int)total, \
+                     (int)attn_groups, (int)attn, (int)attn_wgs)
   if (p.Lk <= 256) S3R_TKL(1);
   else if (p.Lk <= 512) S3R_TKL(2);
   else if (p.Lk <= 768) S3R_TKL(3);

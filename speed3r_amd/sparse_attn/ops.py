@@ -1061,10 +1061,13 @@ def _side_stream(device: torch.device) -> "torch.cuda.Stream":
 
 
 def _two_kernel_compressed(q: torch.Tensor, topk: int, block: int = 1) -> bool:
-    """True where the compressed branch is two independent kernels (attention, indices without a score buffer).
+    """True where the compressed branch is two independent kernels (attention, indices without a score buffer): not for short lists of
+    keys, whose indices and attention are one launch.
     ``q``: the pooled queries (``block`` = 1) or the full tokens that will be pooled over ``block`` tokens."""
+    blocks = -(-q.shape[2] // block)
     return (q.dtype != torch.float32 and q.shape[-1] == 64 and topk in (1, 2, 4, 8, 16, 32)
-            and -(-q.shape[2] // block) <= (1 << 21) and _lib.lib_has_fused_topk())
+            and blocks <= (1 << 21) and _lib.lib_has_fused_topk()
+            and not _lib.lib().s3r_topk_in_lds(q.shape[0] * q.shape[1], blocks, blocks, topk))
 
 
 # When the index kernel goes on a stream of its own.  The two events and the change of stream cost the host up to 40 us and the kernels
