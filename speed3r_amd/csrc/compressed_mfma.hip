@@ -196,16 +196,20 @@ __device__ __forceinline__ void lds_read_queue13(uint32_t addr, u32x2 (&r)[13]) 
 // workgroup; with few workgroups (one round, nothing else on the SIMD to fill the gap) pairs lose less than quads.
 // Two waves per workgroup double the K tile transfers per query row and use a ring of two tiles (30 KB of LDS with the
 // queues, five workgroups per CU).
-template <typename E, int KTOP /* 0: attention (+ scores); > 0: top-k only */, int WAVES>
-__global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(AttnParams p) {
+// PARTS = 2 (four waves): two pairs of waves own the same 64 rows and take every other key tile each, from a ring of three tiles of
+// their own; they exchange their bounds between the sweeps and their lists at the end (see launch_e).
+template <typename E, int KTOP /* 0: attention (+ scores); > 0: top-k only */, int WAVES, int PARTS = 1>
+__global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compressed_mfma_kernel(AttnParams p) {
   typedef typename Mma<E>::V8 V8;
   constexpr bool FUSED = KTOP > 0;
   static_assert(WAVES == 4 || (WAVES == 2 && FUSED), "two waves per workgroup: top-k-only kernel");
   constexpr int KL = FUSED ? KTOP : 1;  // list length per lane
   constexpr int kQSlots = TopkCfg<KTOP>::kQSlots;
+  static_assert(PARTS == 1 || (PARTS == 2 && WAVES == 4 && FUSED), "two parts: pairs of a top-k-only workgroup");
+  constexpr int PW = WAVES / PARTS;  // waves that share their tiles
   constexpr int NB = WAVES == 2 ? 2 : TopkCfg<KTOP>::kRing;
-  constexpr int NI = 8 / WAVES;  // transfer instructions (8 rows each) per wave and tile
-  __shared__ __attribute__((aligned(1024))) E Ks[NB][kTile];
+  constexpr int NI = 8 / PW;  // transfer instructions (8 rows each) per wave and tile
+  __shared__ __attribute__((aligned(1024))) E Ks[NB * PARTS][kTile];
   __shared__ __attribute__((aligned(1024))) E Vs[FUSED ? 1 : 2][FUSED ? 8 : kTile];  // the top-k-only kernel stages K tiles alone
   __shared__ __attribute__((aligned(16))) uint2 queue[FUSED ? WAVES : 1][kQSlots][64];
   __shared__ __attribute__((aligned(16))) float sstage[FUSED ? 1 : 4][FUSED ? 4 : 32 * 64];  // score-store staging (unfused launches)
@@ -218,7 +222,7 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
   const int b = blockIdx.y / p.H;
   const int h = blockIdx.y - b * p.H;
   const int64_t Lq = p.Lq, Lk = p.Lk;
-  const int64_t q0 = (int64_t)blockIdx.x * (32 * WAVES) + wave * 32;
+  const int64_t q0 = (int64_t)blockIdx.x * (32 * PW) + (wave % PW) * 32;
 
   const E* qp = (const E*)p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh;
   const E* kp = (const E*)p.k + (int64_t)b * p.skb + (int64_t)h * p.skh;
@@ -463,7 +467,8 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
     // (row, c') holds head_dim chunk c' ^ k_swizzle(row).  Rows beyond Lk re-read the last row (they are masked).
     const uint32_t krow_bytes = (uint32_t)p.skn * (uint32_t)sizeof(E);
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);  // the LDS destination of a transfer is a scalar (M0)
-    const int dl_row = wave_u * (8 * NI) + (lane >> 3);
+    const int pair_wave = wave_u % PW, part = wave_u / PW;
+    const int dl_row = pair_wave * (8 * NI) + (lane >> 3);
     // (the chunk map repeats every 16 rows: instructions of equal parity share it)
     const uint32_t dl_chunk[2] = {(uint32_t)(((lane & 7) ^ k_swizzle(lane >> 3)) * 16), (uint32_t)(((lane & 7) ^ k_swizzle((lane >> 3) + 8)) * 16)};
     uint32_t dl_off[4] = {0, 0, 0, 0};  // NI of them are used
@@ -475,7 +480,7 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
       const int64_t start = (int64_t)tt * 64 * s;
       const int rem = (int)((uint32_t)(Lk - 1 - start) / (uint32_t)s);
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(kp + start * p.skn), 0, 0x7fffffff, 0x00020000);
-      char* dst = reinterpret_cast<char*>(&Ks[buf][0]) + wave_u * (NI * 1024);
+      char* dst = reinterpret_cast<char*>(&Ks[part * NB + buf][0]) + pair_wave * (NI * 1024);
       uint32_t off[4] = {0, 0, 0, 0};  // the per-lane offsets of a full tile never change
 #pragma unroll
       for (int i = 0; i < NI; i++) off[i] = s == 1 ? dl_off[i] : (uint32_t)(dl_row + 8 * i) * (krow_bytes * (uint32_t)s) + dl_chunk[i & 1];
@@ -493,21 +498,21 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, off[i], 0, 0, 0);
     };
     const uint32_t lds_k = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)reinterpret_cast<char*>(&Ks[0][0]);
-    const uint32_t kr_off = lds_k + (uint32_t)(c * 128 + ((hh ^ k_swizzle(c)) << 4));  // A operand: lane = key row, chunk hh + 2 ks
+    const uint32_t kr_off = lds_k + (uint32_t)part * (NB * kTile * (uint32_t)sizeof(E)) + (uint32_t)(c * 128 + ((hh ^ k_swizzle(c)) << 4));  // A operand: lane = key row, chunk hh + 2 ks
     float best[FUSED ? 2 : 1][2][16];  // first sweep: per register the largest score of the even and of the odd tiles
     auto sweep = [&](auto filter_tag, const int keystep) {  // every keystep-th key
       constexpr bool FILTER = decltype(filter_tag)::value;
       const int s = FILTER ? 1 : keystep;
-      const int nsteps = FILTER ? ntiles : (int)((Lk + 64 * s - 1) / (64 * s));
-      for (int i = 0; i < NB - 1; i++) dma_tile(i, i, s, nsteps);
+      const int all = FILTER ? ntiles : (int)((Lk + 64 * s - 1) / (64 * s)), nsteps = (all + PARTS - 1) / PARTS;
+      for (int i = 0; i < NB - 1; i++) dma_tile(i * PARTS + part, i, s, all);
       int buf = 0, fill = NB - 1;  // ring positions of step i's tile and of step i + NB - 1's
       for (int i = 0; i < nsteps; i++) {
         // this wave's share of tile t has landed (transfers complete in order, NI per tile, NB - 2 tiles younger) ...
         __builtin_amdgcn_s_waitcnt(0x0F70 | (NI * (NB - 2)));
         __builtin_amdgcn_s_barrier();  // ... and everybody's; all waves are done with tile t - 1, whose buffer is refilled now
-        dma_tile(i + NB - 1, fill, s, nsteps);
+        dma_tile((i + NB - 1) * PARTS + part, fill, s, all);
         {
-          const int64_t start = (int64_t)i * 64 * s;
+          const int64_t start = (int64_t)(i * PARTS + part) * 64 * s;
           const bool partial = start + 63 * s >= Lk;
           u32x4 kf[2][4];
           const uint32_t kb = kr_off + (uint32_t)buf * (kTile * (uint32_t)sizeof(E));
@@ -526,9 +531,9 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
           }
           buf = buf + 1 == NB ? 0 : buf + 1;
           fill = fill + 1 == NB ? 0 : fill + 1;
-          if (partial) {  // last tile only: keys beyond Lk get a score that neither raises a maximum nor passes the filter
+          if (partial) {  // last tile only (or, of the second part, none left): keys beyond Lk get a score that neither raises a maximum nor passes the filter
             // register r of tile kt holds row kt*32 + 4hh + 8(r/4) + r%4 of the tile
-            const int lim = (int)((uint32_t)(Lk - 1 - start) / (uint32_t)s) + 1 - 4 * hh;
+            const int lim = (PARTS > 1 && start >= Lk ? 0 : (int)((uint32_t)(Lk - 1 - start) / (uint32_t)s) + 1) - 4 * hh;
 #pragma unroll
             for (int kt = 0; kt < 2; kt++)
 #pragma unroll
@@ -668,11 +673,30 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
     // largest, whatever the tie-break.  With fewer than K groups that hold a key it stays -inf and every score is a candidate.
     // The K-th largest of two descending lists a, b is the largest min(a[i-1], b[K-i-1]) over the splits i.
     {
-      float tau = fmaxf(top[KL - 1], __uint_as_float(xh_swap(__float_as_uint(top[KL - 1]))));  // splits i = K and i = 0
+      float tau;
+      if constexpr (PARTS == 1) {
+        tau = fmaxf(top[KL - 1], __uint_as_float(xh_swap(__float_as_uint(top[KL - 1]))));  // splits i = K and i = 0
 #pragma unroll
-      for (int i = 1; i < KL; i++) {
-        const float bi = __uint_as_float(xh_swap(__float_as_uint(top[KL - i - 1])));
-        tau = fmaxf(tau, fminf(top[i - 1], bi));
+        for (int i = 1; i < KL; i++) {
+          const float bi = __uint_as_float(xh_swap(__float_as_uint(top[KL - i - 1])));
+          tau = fmaxf(tau, fminf(top[i - 1], bi));
+        }
+      } else {  // the two lanes' K largest, descending in both, and the same of the other part, through the queues' space
+        float both[KL];
+#pragma unroll
+        for (int i = 0; i < KL; i++) both[i] = fmaxf(top[i], __uint_as_float(xh_swap(__float_as_uint(top[KL - 1 - i]))));
+        if constexpr (KL > 1) bitonic_merge_desc<KL>(both);
+        static_assert(KL * 32 * 4 <= (int)sizeof(queue[0]), "a wave's queues hold its rows' bounds");
+        float* const mine = reinterpret_cast<float*>(&queue[wave][0][0]) + c;
+        const float* const other = reinterpret_cast<const float*>(&queue[wave ^ PW][0][0]) + c;
+        if (hh == 0) {
+#pragma unroll
+          for (int i = 0; i < KL; i++) mine[i * 32] = both[i];
+        }
+        __syncthreads();
+        tau = fmaxf(both[KL - 1], other[(KL - 1) * 32]);
+#pragma unroll
+        for (int i = 1; i < KL; i++) tau = fmaxf(tau, fminf(both[i - 1], other[(KL - i - 1) * 32]));
       }
       thr0 = qvalid ? tau : INFINITY;  // rows beyond Lq (all-zero scores) must not flood the queue
       thr = thr0;
@@ -702,6 +726,22 @@ __global__ __launch_bounds__(256, KTOP > 0 ? 3 : 2) void compressed_mfma_kernel(
       }
       bitonic_merge_desc<KL>(list);
     }
+    if constexpr (PARTS == 2) {  // the second part's lists to the first's waves, through the tiles' space
+      __syncthreads();           // every wave is done with its tiles
+      static_assert(PW * KL * 32 * 8 <= (int)sizeof(Ks), "the tiles' space holds the lists of a part");
+      key_t* const lists = reinterpret_cast<key_t*>(&Ks[0][0]) + (wave % PW) * (KL * 32) + c;
+      if (wave >= PW) {
+        if (hh == 0) {
+#pragma unroll
+          for (int i = 0; i < KL; i++) lists[i * 32] = list[i];
+        }
+      }
+      __syncthreads();
+      if (wave >= PW) return;
+#pragma unroll
+      for (int i = 0; i < KL; i++) list[i] = __builtin_fmax(list[i], lists[(KL - 1 - i) * 32]);
+      if constexpr (KL > 1) bitonic_merge_desc<KL>(list);
+    }
     if (qvalid && hh == 0) {
       int32_t* irow = p.topk_idx + (((int64_t)b * p.H + h) * Lq + qrow) * KL;
 #pragma unroll
@@ -726,13 +766,20 @@ static int launch_e(const AttnParams& p, bool fused, hipStream_t st) {
   // (16 266 tokens: pairs +7 %), with fewer the transfers' latency does (1 041 tokens: pairs +2 .. 15 %).
   const int64_t pairs = ((p.Lq + 63) / 64) * (int64_t)p.B * p.H;
   const bool two = pairs > 3 * 256 && pairs <= 5 * 256;
-  const int waves = two ? 2 : 4;
-  const int64_t nqg = (p.Lq + 32 * waves - 1) / (32 * waves);
+  // Few rows (quads that leave every SIMD one wave or none): two waves share the keys of 32 rows, twice the waves and half the chain of
+  // each; two workgroups of 76 KB fit a CU.  us alone on the chip, quads / parts, random keys (keys of which 16 neighbours are alike): 16
+  // heads, top-16 1 217 keys 52 / 38 (52 / 27), 1 627 62 / 43 (62 / 31); 2 016 top-32 95 / 63 (105 / 54), top-4 50 / 36 (44 / 27), 2 048
+  // top-1 39 / 30 (28 / 25); 8 heads, 4 000 top-16 115 / 77 (110 / 58); 2 heads, 5 000 top-32 193 / 103 (194 / 93); 1 head, 16 384
+  // top-16 369 / 216 (332 / 182).  Beyond 512 workgroups a second round of them: 2 200 keys stay with quads.
+  const bool parts = pairs <= 2 * 256;
+  const int waves = two ? 2 : 4, rows = two || parts ? 64 : 128;
+  const int64_t nqg = (p.Lq + rows - 1) / rows;
   if (nqg > 0x7fffffffLL) return fail(S3R_ERR_UNSUPPORTED, "s3r_compressed_attn_topk: grid too large");
   dim3 grid((unsigned)nqg, (unsigned)(p.B * p.H)), blk(64 * waves);
 #define S3R_LAUNCH_TOPK(K)                                                              \
   case K:                                                                               \
-    if (two) hipLaunchKernelGGL((compressed_mfma_kernel<E, K, 2>), grid, blk, 0, st, p); \
+    if (parts) hipLaunchKernelGGL((compressed_mfma_kernel<E, K, 4, 2>), grid, blk, 0, st, p); \
+    else if (two) hipLaunchKernelGGL((compressed_mfma_kernel<E, K, 2>), grid, blk, 0, st, p); \
     else hipLaunchKernelGGL((compressed_mfma_kernel<E, K, 4>), grid, blk, 0, st, p);     \
     break;
   switch (p.K) {
