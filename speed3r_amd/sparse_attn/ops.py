@@ -678,13 +678,17 @@ def attention_layer(x: torch.Tensor, qkv, gate, proj, num_heads: int, block: int
     """The layer's inference in one call of the library: :func:`qkv_project` with means and the gate, :func:`compressed_attn_topk`,
     :func:`gate` where it does not ride, :func:`select_attn_merge` and, unless ``proj`` is None, :func:`linear`: the same kernels in the
     same order, the same results.  ``qkv``, ``gate``, ``proj``: (weight, bias).  For tokens that :func:`qkv_project_takes` (with means and
-    norms), on the calling stream alone (not where :func:`_side_stream_pays`).
+    norms), on the calling stream alone (not where :func:`_side_stream_pays`, unless two waves of the index kernel share a row's keys:
+    at most 512 workgroups of 64 pooled rows.  These leave no LDS for a kernel beside them: 16 heads, us, two streams / this: 2 016
+    blocks of 16 tokens 618 / 585, 1 260 387 / 379; 1 627 of 64 1 539 / 1 537, 1 302 1 220 / 1 224; beyond, 4 164 4 295 / 4 360, 6 489 of
+    16 2 368 / 2 415).
 
     Returns None where the library has no kernels: top-k a power of two up to 32, contiguous 16-byte aligned weights of one dtype,
     a gate of 2 outputs per head that one of its kernels takes."""
     b, n, c = x.shape
     h = num_heads
-    if topk not in (1, 2, 4, 8, 16, 32) or _side_stream_pays(b * h, -(-n // block), topk):
+    blocks = -(-n // block)
+    if topk not in (1, 2, 4, 8, 16, 32) or (b * h * -(-blocks // 64) > 512 and _side_stream_pays(b * h, blocks, topk)):
         return None
     dtype, device = x.dtype, x.device
     for lin, rows in ((qkv, 3 * c), (gate, 2 * h), (proj, c)):
