@@ -174,14 +174,14 @@ int s3r_select_attn(const void* q, const void* k, const void* v, const int32_t* 
  * Selection-branch attention with the gated merge in its epilogue: the selection output never
  * goes to memory; the kernel writes
  *   out[b,n,h*D+d] = gate[b,h,n,0]*o_cmp[b,h,n/block,d] + gate[b,h,n,1]*o_sel[b,h,n,d]
- * 16-token blocks: with the rounding points of s3r_gated_merge (o_sel, each product and the sum rounded to the I/O
- * dtype), so the result equals s3r_select_attn followed by s3r_gated_merge bit for bit.  64-token blocks: the expression
+ * 16-token blocks, and fp32: with the rounding points of s3r_gated_merge (o_sel, each product and the sum rounded to the I/O
+ * dtype), so the result equals s3r_select_attn followed by s3r_gated_merge bit for bit.  64-token blocks of 16-bit types: the expression
  * is evaluated in fp32 on the unrounded selection output and rounded ONCE (at most four rounding steps of the I/O dtype,
  * taken on |gate0 o_cmp| + |gate1 o_sel|, away from the two-call result, on the side of the exact value).
  * Replaces topk_blocksparse_attention (pi3/models/sparse_attn/topk_blocksparse_attention.py:1093-1121)
  * together with the merge expression of pi3/models/layers/sparse_attention.py:127-136.
  * Arguments as in s3r_select_attn and s3r_gated_merge; out is contiguous [B,N,H*D].
- * Only for the MFMA paths (bf16/fp16, D == 64, block == 64 or 16, 16-byte aligned tensors); other
+ * Only for the MFMA paths (D == 64, block == 64 or 16, fp32 also 32, 16-byte aligned tensors); other
  * shapes return S3R_ERR_UNSUPPORTED and the caller runs the two operators one after the other.
  */
 int s3r_select_attn_merge(const void* q, const void* k, const void* v, const int32_t* idx,

@@ -261,6 +261,30 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
   const float l = xh_sum(l_i + lane_xor<16>(l_i));
   if (live) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
+    if constexpr (SELECT) {
+      // The gated merge (rounded as s3r_gated_merge does: each product, then the sum) in place of the output: a pass over it less,
+      // 8 328 tokens x 16 heads 357 -> 344 us for the whole path.
+      if (p.merge_out != nullptr) {
+#pragma clang fp contract(off)
+        const float* const gp = (const float*)p.merge_gate + (int64_t)b * p.sgb + (int64_t)h * p.sgh + qrow * p.sgn;
+        const float* const oc = (const float*)p.merge_oc + (int64_t)b * p.scb + (int64_t)h * p.sch + (qrow / BLK) * p.scm + 16 * g;
+        float* const to = (float*)p.merge_out + (((int64_t)b * p.Lq + qrow) * p.H + h) * 64 + 16 * g;
+        const float g0 = gp[0], g1 = gp[1];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float4 c4 = *reinterpret_cast<const float4*>(oc + 4 * r);
+          const float x[4] = {c4.x, c4.y, c4.z, c4.w};
+          float y[4];
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float s = o[e][r] * inv, a0 = g0 * x[e], a1 = g1 * s;
+            y[e] = a0 + a1;
+          }
+          *reinterpret_cast<float4*>(to + 4 * r) = make_float4(y[0], y[1], y[2], y[3]);
+        }
+        return;
+      }
+    }
     float* op = (float*)p.o + (int64_t)b * p.sob + (int64_t)h * p.soh + qrow * p.som + 16 * g;
 #pragma unroll
     for (int r = 0; r < 4; r++)

@@ -396,7 +396,7 @@ class SparseFlashAttentionRope(nn.Module):
         if self.keep_topk_idx:
             self.last_topk_idx = idx
 
-        out = ops.select_attn_merge(q, k, v, idx, o_c, gate, block)
+        out = ops._select_attn_merge(q, k, v, idx, o_c, gate, block)
         self.last_path = "fused-merge"
         if out is None:
             self.last_path = "two-operators"

@@ -739,8 +739,13 @@ def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) ->
 def select_attn_merge(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, idx: torch.Tensor, o_cmp: torch.Tensor,
                       gate: torch.Tensor, block: int, softmax_scale: Optional[float] = None) -> Optional[torch.Tensor]:
     """``select_attn`` with ``gated_merge`` in its epilogue -> ``[B,N,H*D]``; bit-identical to the two calls, without the
-    round trip of the selection output through memory.  Returns ``None`` when the library has no fused kernel for the
-    shape (the caller then runs the two operators)."""
+    round trip of the selection output through memory.  Returns ``None`` for fp32 and when the library has no fused kernel for
+    the shape (the caller then runs the two operators)."""
+    return _select_attn_merge(q, k, v, idx, o_cmp, gate, block, softmax_scale, (torch.bfloat16, torch.float16))
+
+
+def _select_attn_merge(q, k, v, idx, o_cmp, gate, block, softmax_scale=None, dtypes=(torch.bfloat16, torch.float16, torch.float32)):
+    """:func:`select_attn_merge` in fp32 too (the bits of the two operators)."""
     _need_device(q, k, v, idx, o_cmp, gate)
     _forward_only(q, k, v, o_cmp, gate)
     q, k, v, idx, o_cmp, gate = (_last_contig(t) for t in (q, k, v, idx, o_cmp, gate))
@@ -755,7 +760,7 @@ def select_attn_merge(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, idx: to
     if block in (128, 256):  # 64-row query blocks share their parent's list and its row of the compressed output
         o_cmp = o_cmp.repeat_interleave(block // 64, dim=2)[:, :, :-(-n // 64)].contiguous()
         idx, block = _as_64_token_blocks(idx, block, n), 64
-    if q.dtype == torch.float32 or d != 64 or block not in (64, 16) or idx.shape[3] > 64:
+    if q.dtype not in dtypes or d != 64 or block not in ((64, 32, 16) if q.dtype == torch.float32 else (64, 16)) or idx.shape[3] > 64:
         return None
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
     out = torch.empty((b, n, h * d), dtype=q.dtype, device=q.device)
@@ -1160,7 +1165,7 @@ def sparse_global_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g
         o_cmp, idx = compressed_attn_topk(qc, kc, vc, topk, softmax_scale, materialize_scores=materialize_scores)
     mark("select")
     if fuse_merge and not return_parts:
-        out = select_attn_merge(q, k, v, idx, o_cmp, gate, block, softmax_scale)
+        out = _select_attn_merge(q, k, v, idx, o_cmp, gate, block, softmax_scale)
         if out is not None:
             mark("end")
             return out
