@@ -5,7 +5,12 @@
 // holds the ids of the query blocks whose index row names j, one entry per occurrence, ascending; off[j] .. off[j+1]
 // delimit it.  Entries of idx that are < 0 or >= nkb appear in no list.
 //
-// Five small kernels, no workspace besides the two outputs:
+// Up to kHeadEntries index entries per head (count, scan and fill in one kernel, then sort): workgroup (p, head) reads all of the head's
+// entries and owns the key blocks lo .. hi: it counts theirs in LDS and, in a register, the entries of the blocks below, which gives the
+// start of its first list without a word from the others; then it reads the entries again and writes those of its blocks.  us, five kernels
+// without their sorts / this: 2 x 16 heads of 756 rows of 32 46 / 16, 16 heads of 4 164 rows of 16 43 / 26; with the sorts 2 x 16 x 756 x 32 60 / 30,
+// 16 x 4 096 x 32 90 / 75, 16 x 16 000 x 8 139 / 95.  Bound: the passes over the entries, eight loads in flight a thread.
+// More entries: five small kernels.  No workspace besides the two outputs either way:
 //   zero     off[*] = 0
 //   count    histogram of the index entries, block j counted at off[j + 2] (pre-aggregated per workgroup in LDS)
 //   scan     inclusive prefix sum per (b, h): off[j + 1] = first position of block j's list
@@ -78,6 +83,73 @@ __global__ __launch_bounds__(1024) void gather_kernel(const int32_t* __restrict_
     __syncthreads();
     if (j >= 0) list[bh * list_stride + base[slot] + rank] = m;
   }
+}
+
+constexpr int64_t kHeadEntries = 1 << 17;
+constexpr int kMostSpan = 1 << 14;  // key blocks of a workgroup
+
+__global__ __launch_bounds__(1024) void head_lists_kernel(const int32_t* __restrict__ idx, int32_t* __restrict__ off, int32_t* __restrict__ list,
+                                                           int H, int nqb, int K, int nkb, int span, int64_t sib, int64_t sih,
+                                                           int64_t sim, int64_t list_stride) {
+  extern __shared__ int32_t cnt[];  // of the workgroup's key blocks; later where the next entry of each goes
+  __shared__ int32_t part[1024], below_of[16];
+  const int t = threadIdx.x, lo = blockIdx.x * span, hi = lo + span < nkb ? lo + span : nkb;
+  if (lo >= nkb) return;
+  const int64_t bh = blockIdx.y, hh = bh % H, bb = bh / H;
+  const int32_t* const rows = idx + bb * sib + hh * sih;
+  for (int i = t; i < hi - lo; i += 1024) cnt[i] = 0;
+  __syncthreads();
+  // a thread stays in one column: 1024 / K rows at a time
+  const int step = 1024 / K, first = t / K;
+  const int32_t* const own = rows + (int64_t)first * sim + (t - first * K);
+  const int end = first < step ? nqb : 0;
+  int below = 0;
+  auto walk = [&](auto take) {  // eight entries on their way at once
+    const int32_t* from = own;
+    for (int m = first; m < end; m += 8 * step) {
+      int32_t j[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        j[u] = m + u * step < end ? *from : -1;
+        from += step * sim;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++) take(m + u * step, j[u]);
+    }
+  };
+  walk([&](int, int32_t j) {
+    below += j >= 0 && j < lo ? 1 : 0;
+    if (j >= lo && j < hi) atomicAdd(&cnt[j - lo], 1);
+  });
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) below += __shfl_xor(below, d);
+  if ((t & 63) == 0) below_of[t >> 6] = below;
+  __syncthreads();
+  const int per = (hi - lo + 1023) / 1024, b0 = t * per, b1 = b0 + per < hi - lo ? b0 + per : hi - lo;
+  int32_t sum = 0;
+  for (int i = b0; i < b1; i++) sum += cnt[i];
+  part[t] = sum;
+  __syncthreads();
+  for (int d = 1; d < 1024; d <<= 1) {  // Hillis-Steele over the 1024 partial sums
+    const int32_t v = t >= d ? part[t - d] : 0;
+    __syncthreads();
+    part[t] += v;
+    __syncthreads();
+  }
+  int32_t at = t > 0 ? part[t - 1] : 0;
+#pragma unroll
+  for (int w = 0; w < 16; w++) at += below_of[w];
+  int32_t* const starts = off + bh * (nkb + 1);
+  for (int i = b0; i < b1; i++) {
+    const int32_t n = cnt[i];
+    cnt[i] = starts[lo + i] = at;
+    at += n;
+  }
+  if (hi == nkb && b0 < b1 && b1 == hi - lo) starts[nkb] = at;
+  __syncthreads();
+  walk([&](int m, int32_t j) {
+    if (j >= lo && j < hi) list[bh * list_stride + atomicAdd(&cnt[j - lo], 1)] = m;
+  });
 }
 
 // one workgroup of 1024 per (b, h): in-place inclusive scan of n values
@@ -242,11 +314,18 @@ int launch_key_block_lists(const int32_t* idx, int32_t* kq_list, int32_t* kq_off
   const int64_t g_off = (noff + 255) / 256, g_ent = (total + 255) / 256, g_short = (nseg * 64 + 255) / 256;
   if (g_off > 0x7fffffffLL || g_ent > 0x7fffffffLL || g_short > 0x7fffffffLL || bh > 65535)
     return fail(S3R_ERR_UNSUPPORTED, "s3r_key_block_lists: tensor too large for one launch");
-  hipLaunchKernelGGL(kl::zero_kernel, dim3((unsigned)g_off), dim3(256), 0, st, kq_off, noff);
-  const dim3 g_gather((unsigned)((nqb * K + 1023) / 1024), (unsigned)bh);
-  hipLaunchKernelGGL(kl::gather_kernel<false>, g_gather, dim3(1024), 0, st, idx, kq_off, kq_list, H, nqb, K, nkb, sib, sih, sim, list_stride);
-  hipLaunchKernelGGL(kl::scan_kernel, dim3((unsigned)bh), dim3(1024), 0, st, kq_off, nkb + 1);
-  hipLaunchKernelGGL(kl::gather_kernel<true>, g_gather, dim3(1024), 0, st, idx, kq_off, kq_list, H, nqb, K, nkb, sib, sih, sim, list_stride);
+  // workgroups for every CU once; each reads all of a head's entries
+  const int64_t parts = bh >= 256 ? 1 : 256 / bh < nkb ? 256 / bh : nkb, span = (nkb + parts - 1) / parts;
+  if (nqb * K <= kl::kHeadEntries && K <= 1024 && span <= kl::kMostSpan) {
+    hipLaunchKernelGGL(kl::head_lists_kernel, dim3((unsigned)parts, (unsigned)bh), dim3(1024), (unsigned)(span * 4), st, idx, kq_off, kq_list, H,
+                       (int)nqb, K, (int)nkb, (int)span, sib, sih, sim, list_stride);
+  } else {
+    hipLaunchKernelGGL(kl::zero_kernel, dim3((unsigned)g_off), dim3(256), 0, st, kq_off, noff);
+    const dim3 g_gather((unsigned)((nqb * K + 1023) / 1024), (unsigned)bh);
+    hipLaunchKernelGGL(kl::gather_kernel<false>, g_gather, dim3(1024), 0, st, idx, kq_off, kq_list, H, nqb, K, nkb, sib, sih, sim, list_stride);
+    hipLaunchKernelGGL(kl::scan_kernel, dim3((unsigned)bh), dim3(1024), 0, st, kq_off, nkb + 1);
+    hipLaunchKernelGGL(kl::gather_kernel<true>, g_gather, dim3(1024), 0, st, idx, kq_off, kq_list, H, nqb, K, nkb, sib, sih, sim, list_stride);
+  }
   hipLaunchKernelGGL(kl::sort_short_kernel, dim3((unsigned)g_short), dim3(256), 0, st, kq_list, kq_off, nkb, list_stride, nseg);
   const int64_t g_long = nseg < 4096 ? nseg : 4096;
   hipLaunchKernelGGL(kl::sort_long_kernel, dim3((unsigned)g_long), dim3(256), 0, st, kq_list, kq_off, nkb, list_stride, nseg);

@@ -27,3 +27,22 @@ def test_lists_of_length(n):
             assert off[b, 0, j] == at and torch.equal(lists[b, 0, at:at + len(want)].long(), want)
             at += len(want)
         assert off[b, 0, nkb] == at
+
+
+# entries per head on both sides of the line between the kernels that make the lists; key blocks that the workgroups of a head share unevenly,
+# fewer of them than workgroups, more heads than CUs; strided index rows, entries that are skipped
+@pytest.mark.parametrize("bh,nqb,k,nkb", [(1, 4096, 32, 4096), (1, 4097, 32, 300), (3, 1000, 5, 1), (2, 777, 16, 3), (16, 130, 8, 131), (300, 20, 4, 20),
+                                          (1, 50, 2, 70000), (2, 100, 64, 20000)])
+def test_lists_of_heads(bh, nqb, k, nkb):
+    gen = torch.Generator().manual_seed(nqb)
+    wide = torch.randint(-2, nkb + 2, (1, bh, nqb, k + 3), generator=gen, dtype=torch.int32)
+    wide = torch.where(torch.rand(wide.shape, generator=gen) < 0.2, wide.clamp(max=nkb // 3), wide)
+    idx = wide.cuda()[..., :k]
+    lists, off = (t.cpu()[0] for t in ops.key_block_lists(idx, nkb))
+    for b in range(bh):
+        e = wide[0, b, :, :k].reshape(-1).long()
+        ok = (e >= 0) & (e < nkb)
+        order = torch.sort(e[ok], stable=True)
+        rows = torch.arange(nqb).repeat_interleave(k)[ok][order.indices]
+        assert torch.equal(off[b].long(), torch.cat((torch.zeros(1, dtype=torch.long), torch.bincount(e[ok], minlength=nkb).cumsum(0))))
+        assert torch.equal(lists[b, :len(rows)].long(), rows)
