@@ -52,6 +52,10 @@ int s3r_pool_mean(const void* x, void* y, int B, int H, int64_t N, int D, int bl
                   int64_t sxb, int64_t sxh, int64_t sxn,
                   int64_t syb, int64_t syh, int64_t syn,
                   int dtype, void* stream);
+/* The same for q, k and v of one shape in one launch; y: contiguous [3,B,H,ceil(N/block),D]. */
+int s3r_pool_means3(const void* q, const void* k, const void* v, void* y, int B, int H, int64_t N, int D, int block,
+                    int64_t sqb, int64_t sqh, int64_t sqn, int64_t skb, int64_t skh, int64_t skn,
+                    int64_t svb, int64_t svh, int64_t svn, int dtype, void* stream);
 
 /*
  * Compressed-branch attention with top-k block selection.

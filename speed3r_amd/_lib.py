@@ -22,6 +22,7 @@ SIGNATURES = {
     "s3r_last_error": (c_char_p, []),
     "s3r_capabilities": (c_int, []),
     "s3r_pool_mean": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int64, c_int, c_int, *_i64x3, *_i64x3, c_int, c_void_p]),
+    "s3r_pool_means3": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int, c_int, *_i64x3, *_i64x3, *_i64x3, c_int, c_void_p]),
     "s3r_compressed_attn_topk": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                          c_int, c_int, c_int, c_int, c_int, c_int,
                                          *_i64x3, *_i64x3, *_i64x3, *_i64x3, c_float, c_int, c_void_p]),

@@ -32,10 +32,19 @@ template <int VEC> __device__ __forceinline__ void fold_mean(float (&acc)[VEC], 
   }
 }
 
+// up to three tensors of one shape, blockIdx.y says which
+struct PoolSet {
+  const void* x[3];
+  void* y[3];
+  int64_t sxb[3], sxh[3], sxn[3];
+  int64_t syb, syh, syn;
+};
+
 template <typename T, int U>
-__global__ __launch_bounds__(256) void pool_mean_kernel(
-    const T* __restrict__ x, T* __restrict__ y, int H, int64_t N, int D, int block, int64_t Nc,
-    int64_t total, int64_t sxb, int64_t sxh, int64_t sxn, int64_t syb, int64_t syh, int64_t syn) {
+__global__ __launch_bounds__(256) void pool_mean_kernel(PoolSet s, int H, int64_t N, int D, int block, int64_t Nc, int64_t total) {
+  const T* const x = (const T*)s.x[blockIdx.y];
+  T* const y = (T*)s.y[blockIdx.y];
+  const int64_t sxb = s.sxb[blockIdx.y], sxh = s.sxh[blockIdx.y], sxn = s.sxn[blockIdx.y];
   constexpr int VEC = 16 / sizeof(T);
   const int lane = threadIdx.x & 63;
   const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -82,7 +91,7 @@ __global__ __launch_bounds__(256) void pool_mean_kernel(
     T* e = reinterpret_cast<T*>(&raw);
 #pragma unroll
     for (int i = 0; i < VEC; i++) e[i] = from_f32<T>(acc[i]);
-    *reinterpret_cast<uint4*>(y + b * syb + h * syh + j * syn + dc * VEC) = raw;
+    *reinterpret_cast<uint4*>(y + b * s.syb + h * s.syh + j * s.syn + dc * VEC) = raw;
   }
 }
 
@@ -90,9 +99,11 @@ __global__ __launch_bounds__(256) void pool_mean_kernel(
 // loads in flight as for the large blocks (with one block per wave only 2 KB per wave are in flight and the kernel
 // runs at 5.0 instead of 6.6 TB/s at 16-token blocks).
 template <typename T, int U, int G>
-__global__ __launch_bounds__(256) void pool_mean_group_kernel(
-    const T* __restrict__ x, T* __restrict__ y, int H, int64_t N, int D, int block, int64_t Nc, int64_t ngrp,
-    int64_t total, int64_t sxb, int64_t sxh, int64_t sxn, int64_t syb, int64_t syh, int64_t syn) {
+__global__ __launch_bounds__(256) void pool_mean_group_kernel(PoolSet s, int H, int64_t N, int D, int block, int64_t Nc, int64_t ngrp,
+                                                               int64_t total) {
+  const T* const x = (const T*)s.x[blockIdx.y];
+  T* const y = (T*)s.y[blockIdx.y];
+  const int64_t sxb = s.sxb[blockIdx.y], sxh = s.sxh[blockIdx.y], sxn = s.sxn[blockIdx.y];
   constexpr int VEC = 16 / sizeof(T);
   const int lane = threadIdx.x & 63;
   const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -139,7 +150,7 @@ __global__ __launch_bounds__(256) void pool_mean_group_kernel(
       T* e = reinterpret_cast<T*>(&out);
 #pragma unroll
       for (int i = 0; i < VEC; i++) e[i] = from_f32<T>(acc[i]);
-      *reinterpret_cast<uint4*>(y + b * syb + h * syh + (jg * G + g) * syn + dc * VEC) = out;
+      *reinterpret_cast<uint4*>(y + b * s.syb + h * s.syh + (jg * G + g) * s.syn + dc * VEC) = out;
     }
   }
 }
@@ -183,10 +194,9 @@ __global__ __launch_bounds__(256) void gated_merge_kernel(
 
 using namespace s3r;
 
-extern "C" int s3r_pool_mean(const void* x, void* y, int B, int H, int64_t N, int D, int block,
-                             int64_t sxb, int64_t sxh, int64_t sxn, int64_t syb, int64_t syh, int64_t syn,
-                             int dtype, void* stream) {
-  if (!x || !y) return fail(S3R_ERR_BAD_ARG, "s3r_pool_mean: null pointer");
+static int pool_impl(const PoolSet& s, int count, int B, int H, int64_t N, int D, int block, int dtype, void* stream) {
+  for (int i = 0; i < count; i++)
+    if (!s.x[i] || !s.y[i]) return fail(S3R_ERR_BAD_ARG, "s3r_pool_mean: null pointer");
   if (B <= 0 || H <= 0 || N <= 0 || D <= 0 || block <= 0) return fail(S3R_ERR_BAD_ARG, "s3r_pool_mean: non-positive size");
   if (dtype != S3R_F32 && dtype != S3R_BF16 && dtype != S3R_F16) return fail(S3R_ERR_UNSUPPORTED, "s3r_pool_mean: dtype %d", dtype);
   const int es = elt_size(dtype);
@@ -194,22 +204,23 @@ extern "C" int s3r_pool_mean(const void* x, void* y, int B, int H, int64_t N, in
   const int lpr = D / vec;
   if (D % vec != 0 || lpr > 64 || (lpr & (lpr - 1)) != 0)
     return fail(S3R_ERR_UNSUPPORTED, "s3r_pool_mean: head_dim %d (row bytes must be a power-of-two multiple of 16, <= 1024)", D);
-  if (!aligned16(x) || !aligned16(y) || (sxb * es) % 16 || (sxh * es) % 16 || (sxn * es) % 16 || (syb * es) % 16 ||
-      (syh * es) % 16 || (syn * es) % 16)
-    return fail(S3R_ERR_BAD_ARG, "s3r_pool_mean: pointers and strides must be 16-byte aligned");
+  for (int i = 0; i < count; i++)
+    if (!aligned16(s.x[i]) || !aligned16(s.y[i]) || (s.sxb[i] * es) % 16 || (s.sxh[i] * es) % 16 || (s.sxn[i] * es) % 16 || (s.syb * es) % 16 ||
+        (s.syh * es) % 16 || (s.syn * es) % 16)
+      return fail(S3R_ERR_BAD_ARG, "s3r_pool_mean: pointers and strides must be 16-byte aligned");
   const int64_t Nc = (N + block - 1) / block;
   const int64_t total = (int64_t)B * H * Nc;
   const int64_t nwg = (total + 3) / 4;
   if (nwg > 0x7fffffffLL) return fail(S3R_ERR_UNSUPPORTED, "s3r_pool_mean: too many blocks");
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid((unsigned)nwg), blk(256);
+  dim3 grid((unsigned)nwg, (unsigned)count), blk(256);
   const int loads = (block * lpr + 63) / 64;  // wave-wide loads that cover one block
-#define S3R_POOL(T, U) hipLaunchKernelGGL((pool_mean_kernel<T, U>), grid, blk, 0, st, (const T*)x, (T*)y, H, N, D, block, Nc, total, sxb, sxh, sxn, syb, syh, syn)
+#define S3R_POOL(T, U) hipLaunchKernelGGL((pool_mean_kernel<T, U>), grid, blk, 0, st, s, H, N, D, block, Nc, total)
 #define S3R_POOL_G(T, U, G)                                                                                                  \
   do {                                                                                                                       \
     const int64_t ngrp = (Nc + G - 1) / G, tot = (int64_t)B * H * ngrp;                                                      \
-    hipLaunchKernelGGL((pool_mean_group_kernel<T, U, G>), dim3((unsigned)((tot + 3) / 4)), blk, 0, st, (const T*)x, (T*)y, H, N, D, \
-                       block, Nc, ngrp, tot, sxb, sxh, sxn, syb, syh, syn);                                                  \
+    hipLaunchKernelGGL((pool_mean_group_kernel<T, U, G>), dim3((unsigned)((tot + 3) / 4), (unsigned)count), blk, 0, st, s, H, N, D, \
+                       block, Nc, ngrp, tot);                                                  \
   } while (0)
 #define S3R_POOL_T(T)                                       \
   do {                                                      \
@@ -227,6 +238,33 @@ extern "C" int s3r_pool_mean(const void* x, void* y, int B, int H, int64_t N, in
 #undef S3R_POOL_G
 #undef S3R_POOL
   return check_launch("s3r_pool_mean");
+}
+
+extern "C" int s3r_pool_mean(const void* x, void* y, int B, int H, int64_t N, int D, int block,
+                             int64_t sxb, int64_t sxh, int64_t sxn, int64_t syb, int64_t syh, int64_t syn,
+                             int dtype, void* stream) {
+  PoolSet s = {};
+  s.x[0] = x; s.y[0] = y; s.sxb[0] = sxb; s.sxh[0] = sxh; s.sxn[0] = sxn;
+  s.syb = syb; s.syh = syh; s.syn = syn;
+  return pool_impl(s, 1, B, H, N, D, block, dtype, stream);
+}
+
+extern "C" int s3r_pool_means3(const void* q, const void* k, const void* v, void* y, int B, int H, int64_t N, int D, int block,
+                               int64_t sqb, int64_t sqh, int64_t sqn, int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh,
+                               int64_t svn, int dtype, void* stream) {
+  if (!y) return fail(S3R_ERR_BAD_ARG, "s3r_pool_means3: null pointer");
+  if (B <= 0 || H <= 0 || N <= 0 || D <= 0 || block <= 0) return fail(S3R_ERR_BAD_ARG, "s3r_pool_means3: non-positive size");
+  const int64_t Nc = (N + block - 1) / block, one = (int64_t)B * H * Nc * D * elt_size(dtype);
+  PoolSet s = {};
+  const void* const from[3] = {q, k, v};
+  const int64_t strides[3][3] = {{sqb, sqh, sqn}, {skb, skh, skn}, {svb, svh, svn}};
+  for (int i = 0; i < 3; i++) {
+    s.x[i] = from[i];
+    s.y[i] = (char*)y + i * one;
+    s.sxb[i] = strides[i][0]; s.sxh[i] = strides[i][1]; s.sxn[i] = strides[i][2];
+  }
+  s.syb = (int64_t)H * Nc * D; s.syh = Nc * D; s.syn = D;
+  return pool_impl(s, 3, B, H, N, D, block, dtype, stream);
 }
 
 extern "C" int s3r_gated_merge(const void* o_cmp, const void* o_sel, const void* gate, void* out,

@@ -82,6 +82,23 @@ def pool_mean(x: torch.Tensor, block: int) -> torch.Tensor:
     return y
 
 
+def _pool_means(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, block: int):
+    """:func:`pool_mean` of q, k and v, in one launch where they share shape, type and device (the same bits)."""
+    if not (q.shape == k.shape == v.shape and q.dtype == k.dtype == v.dtype and q.device == k.device == v.device):
+        return pool_mean(q, block), pool_mean(k, block), pool_mean(v, block)
+    _need_device(q, k, v)
+    _forward_only(q, k, v)
+    q, k, v = (_last_contig(t) for t in (q, k, v))
+    b, h, n, d = q.shape
+    y = torch.empty((3, b, h, -(-n // block), d), dtype=q.dtype, device=q.device)
+    with _on(q.device):
+        rc = _lib.lib().s3r_pool_means3(q.data_ptr(), k.data_ptr(), v.data_ptr(), y.data_ptr(), b, h, n, d, block, q.stride(0), q.stride(1),
+                                        q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
+                                        _code(q), _stream(q))
+    _lib.check(rc, "s3r_pool_means3")
+    return y.unbind(0)
+
+
 def pool_qkv_packed(qkv: torch.Tensor, num_heads: int, block: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Pool the packed projection ``[B, N, 3*H*D]`` (layout ``(qkv h d)``) in one launch.
 
@@ -1160,7 +1177,7 @@ def sparse_global_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g
         o_cmp, _ = compressed_attn_topk(qc, kc, vc, None, softmax_scale)
         join()
     else:
-        qc, kc, vc = pool_mean(q, block), pool_mean(k, block), pool_mean(v, block)
+        qc, kc, vc = _pool_means(q, k, v, block)
         mark("pooled")
         o_cmp, idx = compressed_attn_topk(qc, kc, vc, topk, softmax_scale, materialize_scores=materialize_scores)
     mark("select")
