@@ -1097,15 +1097,12 @@ def _two_kernel_compressed(q: torch.Tensor, topk: int, block: int = 1) -> bool:
 
 
 # When the index kernel goes on a stream of its own.  The two events and the change of stream cost the host up to 40 us and the kernels
-# behind them a wait between queues; what there is to hide is the dense sweep's 12 to 16 us.  The kernel for short lists of keys has
-# too little to gain.  The two-sweep kernel pays from 19 456 pooled rows (B * H * blocks) on; long lists over few heads, whose chain is long and
-# leaves most of the chip idle, from 8192.  us per call, two streams / one: short lists, 2 x 16 heads of 620 pooled tokens, operators 238 / 228,
-# layer 416 / 404, 32 heads of 600 235 / 226 and 538 / 535, top-1 over 16 heads of 700 125 / 85 and 253 / 204; two sweeps, 16 heads,
-# 16-token blocks, layer 2 016 pooled tokens 714 / 721, top-4 over 1 200 318 / 309, over 1 300 332 / 338; 64-token blocks, layer 1 627
-# 1 570 / 1 592, operators 1 041 418 / 413, 2 082 766 / 778, 4 164 1 532 / 1 551; 2 x 16 heads of 1 300 at 16-token blocks 481 / 504 and 883 / 894;
-# 8 heads of 2 016 at 16- / 64-token blocks, layer 366 / 363 and 983 / 989, operators 265 / 269 and 671 / 671; of 2 432 443 / 433; of 2 600
-# 467 / 467 and 334 / 342; 4 heads of 4 000 404 / 407 and 329 / 342; 2 heads of 5 000 379 / 391 and 339 / 354, top-4 over 4 200
-# 213 / 204 and 164 / 177.
+# behind them a wait between queues; what there is to hide is the dense sweep (and the pooling of v, or a layer's gate).  Short lists of keys
+# are one launch with the attention.  The two-sweep kernel pays from 19 456 pooled rows (B * H * blocks) on; long lists over few heads, whose
+# chain is long and leaves most of the chip idle, from 8192.  Operators, us per call, two streams / one, 16 heads: 16-token blocks, top-32,
+# 1 512 pooled tokens 185 / 188, 2 016 235 / 237, 3 780 438 / 441; 64-token blocks, top-16, 1 302 480 / 482, 1 952 701 / 702, 2 603 938 / 953, 4 164
+# 1 532 / 1 551.  Layers: 2 520 blocks of 16 798 / 792, 3 780 1 193 / 1 165, 5 040 1 711 / 1 665, 6 489 2 368 / 2 415, 12 600 5 410 / 5 630; 4 164 of 64
+# 4 295 / 4 360; 3 x 16 heads of 1 008 798 / 812 (up to 512 workgroups of 64 pooled rows: see attention_layer).
 SIDE_STREAM_ROWS = 16 * 1216
 SIDE_STREAM_ROWS_OF_LONG_LISTS = 8192
 
