@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64, 4) void bwd16_dq_kernel(BwdParams p, int nqb, i
           st = mma16<E>(frag_of<E>(kw[ks]), bq[j][ks], st);
           dp = mma16<E>(frag_of<E>(vw[ks]), bg[j][ks], dp);
         }
-        settle2(st, dp);
+        settle(st, dp);
         float nl = nlse[j];
         if (__builtin_expect(rare, 0)) {
           nl += __builtin_amdgcn_logf((float)w);  // a block listed w times weighs w times

@@ -148,6 +148,9 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
         const float a = *reinterpret_cast<const float*>(kb + (kg * 16 + c) * kRow + ((s ^ c) << 4) + g * 4);
         st[kg] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, q[s], st[kg], 0, 0, 0);
       }
+    static_assert(NG <= 2, "every group's product is waited for");
+    if constexpr (NG == 2) settle_f32(st[0], st[1]);
+    else settle_f32(st[0]);
     if constexpr (!SELECT) {
       if (p.scores != nullptr && live) {
         float* srow = p.scores + (((int64_t)b * p.H + h) * p.Lq + qrow) * p.Lk + s0;

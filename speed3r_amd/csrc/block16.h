@@ -8,6 +8,7 @@ namespace b16x {
 using sel::Frag;
 using sel::as_v8;
 using sel::Mma;
+using sel::settle;
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kPair = 32 * 128;  // bytes of two 16-row blocks
@@ -15,12 +16,6 @@ constexpr int kPair = 32 * 128;  // bytes of two 16-row blocks
 template <typename E> __device__ __forceinline__ f32x4 mma16(typename Mma<E>::V8 a, typename Mma<E>::V8 b, f32x4 c);
 template <> __device__ __forceinline__ f32x4 mma16<bf16_t>(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 template <> __device__ __forceinline__ f32x4 mma16<f16_t>(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-
-// Eight wait states behind the matrix instruction that wrote x.  The compiler pads this distance by itself, but where a rare
-// branch leaves right behind the instruction and joins again it has counted the way through the branch only (seen in a
-// listing: three states on the straight way, and wrong values).
-__device__ __forceinline__ void settle(f32x4& x) { asm volatile("s_nop 7" : "+v"(x)); }
-__device__ __forceinline__ void settle2(f32x4& x, f32x4& y) { asm volatile("s_nop 7" : "+v"(x), "+v"(y)); }
 
 // 16 x 16 x 16: four values of K per lane, rows 4 (lane / 16) .. + 3
 template <typename E> struct Mma4;

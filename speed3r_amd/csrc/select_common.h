@@ -51,6 +51,16 @@ __device__ __forceinline__ float xh_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Wait states behind the matrix instructions that wrote the operands.  The compiler pads this distance by itself, but where a
+// branch leaves right behind a product and joins again it has counted one of the two ways only (seen in listings: three states
+// on the straight way of a 16-bit product, and wrong values; one behind an fp32 product).  It stands behind every product with
+// a branch or inline assembly in front of its first reader.  16 x 16 of 16-bit types: eight.
+__device__ __forceinline__ void settle(f32x4& x) { asm volatile("s_nop 7" : "+v"(x)); }
+__device__ __forceinline__ void settle(f32x4& x, f32x4& y) { asm volatile("s_nop 7" : "+v"(x), "+v"(y)); }
+// 16 x 16 of fp32: ten
+__device__ __forceinline__ void settle_f32(f32x4& x) { asm volatile("s_nop 7\n\ts_nop 1" : "+v"(x)); }
+__device__ __forceinline__ void settle_f32(f32x4& x, f32x4& y) { asm volatile("s_nop 7\n\ts_nop 1" : "+v"(x), "+v"(y)); }
+
 template <typename F, int... I> __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>{}), ...);
 }

@@ -43,3 +43,18 @@ def test_scores_that_rise_along_the_list(step):
     k[..., 0] = (torch.arange(400) // 64) * step
     idx = torch.arange(7, dtype=torch.int32).expand(1, 40, 7, 7).contiguous()
     _check(q, k, v, idx, 1e-5 + 4 * 6 * step * 2.0 ** -23)
+
+
+@pytest.mark.parametrize("n,h", [(400, 40), (450, 32), (384, 47)])   # 280 query blocks (24 in halves), 256 (none), 282 (26, all of them full)
+@pytest.mark.parametrize("dims", [slice(60, 61), slice(63, 64), slice(60, 64)])
+def test_scores_that_rise_in_the_last_dimensions(dims, n, h):
+    """The same, hundreds of units a block in the head dimensions that the last products of a score add: the reference of the softmax
+    is read from finished sums.  A score is at most 6 * 400 units: its rounding, 2^-23 of it twice over, moves the result by as much."""
+    g = torch.Generator().manual_seed(2)
+    q, k, v = (torch.randn((1, h, n, 64), generator=g) for _ in range(3))
+    width = dims.stop - dims.start
+    q[..., dims] = 8.0
+    k[..., dims] = (torch.arange(n) // 64)[:, None] * (400.0 / width)
+    nb = -(-n // 64)
+    order = torch.stack([torch.randperm(nb, generator=g) for _ in range(h * nb)]).view(1, h, nb, nb)   # (rising, falling and mixed)
+    _check(q, k, v, order.int().contiguous(), 1e-5 + 4 * 2400 * 2.0 ** -23)
