@@ -23,13 +23,12 @@
 // the end the two lanes of a query merge their lists and lane < 32 writes the K indices in descending key order.
 // The filter is conservative (anything that could enter passes), the network compares full keys, so the result is
 // the same unique top-K as a sort of the whole row.
-#include "s3r_common.h"
+#include "select_common.h"
 #include "attn_params.h"
-#include <type_traits>
-#include <utility>
 
 namespace s3r {
 namespace cmp {
+using sel::settle;
 
 template <typename E> struct Mma;
 template <> struct Mma<bf16_t> {
@@ -355,6 +354,7 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
         st[kt] = Mma<E>::mma(as_v8<E>(f), bq[ks], st[kt]);
       }
     }
+    settle(st);
 
     if (p.scores != nullptr) {
       float* sbase = p.scores + (((int64_t)b * p.H + h) * Lq + q0) * Lk + start;  // row 0 of this wave, column 0 of the tile
@@ -529,6 +529,7 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
               st[kt] = Mma<E>::mma(as_v8<E>(f), bq[ks], st[kt]);
             }
           }
+          settle(st);
           buf = buf + 1 == NB ? 0 : buf + 1;
           fill = fill + 1 == NB ? 0 : fill + 1;
           if (partial) {  // last tile only (or, of the second part, none left): keys beyond Lk get a score that neither raises a maximum nor passes the filter
@@ -541,10 +542,6 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
                 if (kt * 32 + 8 * (r >> 2) + (r & 3) >= lim) st[kt][r] = FILTER ? __uint_as_float(0x7FC00000u) : -INFINITY;
           }
           if constexpr (!FILTER) {
-            // ordinary VALU reads of both accumulators first: the compiler pads the distance from the MFMAs that wrote
-            // them for these instructions, not for inline assembly
-            const float s0 = fmaxf(st[0][0], st[0][15]), s1 = fmaxf(st[1][0], st[1][15]);
-            asm volatile("" ::"v"(s0), "v"(s1));
             auto raise = [&](float (&g)[2][16]) {
 #pragma unroll
               for (int kt = 0; kt < 2; kt++)
@@ -561,10 +558,6 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
             // branch each (top-16: 0.754 -> 0.710 ms; 16 656 keys, top-32: 0.887 -> 0.828 ms).
             bool tile_hit;
             {
-              // ordinary VALU reads of both accumulators first: the compiler pads the distance from the MFMAs that
-              // wrote them for these instructions, not for inline assembly
-              const float s0 = fmaxf(st[0][0], st[0][15]), s1 = fmaxf(st[1][0], st[1][15]);
-              asm volatile("" ::"v"(s0), "v"(s1));
               float ma, mb, mt;
               asm("v_max3_f32 %0, %1, %2, %3\n\tv_max3_f32 %0, %0, %4, %5\n\tv_max3_f32 %0, %0, %6, %7\n\tv_max3_f32 %0, %0, %8, %9\n\t"
                   "v_max3_f32 %0, %0, %10, %11\n\tv_max3_f32 %0, %0, %12, %13\n\tv_max3_f32 %0, %0, %14, %15\n\tv_max_f32 %0, %0, %16"
@@ -582,12 +575,6 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
             if (tile_hit)
 #pragma unroll
             for (int g = 0; g < 32 / kGroup; g++) {  // a group of scores, then a drain check
-              if ((g % (16 / kGroup)) == 0) {
-                // an ordinary VALU read of the accumulator before the hand-written block below: the compiler pads
-                // the distance from the MFMA that wrote it for this instruction, not for inline assembly
-                const float settled = fmaxf(st[g / (16 / kGroup)][0], st[g / (16 / kGroup)][15]);
-                asm volatile("" ::"v"(settled));
-              }
               {  // No survivor among the group's 4 x 64 scores (NaNs of masked keys drop out of the maxima): next group, for
                  // two maxima, one compare and one branch instead of four of each.  With K wanted out of several thousand keys,
                  // three groups in four end here (16 266 keys, top-16: 1.11 -> 0.92 ms; 4 164 keys: 0.166 -> 0.152 ms); a

@@ -53,10 +53,15 @@ __device__ __forceinline__ float xh_sum(float x) {
 
 // Wait states behind the matrix instructions that wrote the operands.  The compiler pads this distance by itself, but where a
 // branch leaves right behind a product and joins again it has counted one of the two ways only (seen in listings: three states
-// on the straight way of a 16-bit product, and wrong values; one behind an fp32 product).  It stands behind every product with
-// a branch or inline assembly in front of its first reader.  16 x 16 of 16-bit types: eight.
+// on the straight way of a 16-bit product, and wrong values; one behind an fp32 product), and for inline assembly that reads the
+// result it counts nothing.  So these stand where a rare branch or inline assembly comes between a product and its readers (a
+// test walks the built code for all products).  16 x 16 of 16-bit types: eight.
 __device__ __forceinline__ void settle(f32x4& x) { asm volatile("s_nop 7" : "+v"(x)); }
 __device__ __forceinline__ void settle(f32x4& x, f32x4& y) { asm volatile("s_nop 7" : "+v"(x), "+v"(y)); }
+__device__ __forceinline__ void settle(f32x4 (&x)[4]) { asm volatile("s_nop 7" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3])); }
+// 32 x 32 x 16 of 16-bit types: twelve
+__device__ __forceinline__ void settle(f32x16& x) { asm volatile("s_nop 7\n\ts_nop 3" : "+v"(x)); }
+__device__ __forceinline__ void settle(f32x16 (&x)[2]) { asm volatile("s_nop 7\n\ts_nop 3" : "+v"(x[0]), "+v"(x[1])); }
 // 16 x 16 of fp32: ten
 __device__ __forceinline__ void settle_f32(f32x4& x) { asm volatile("s_nop 7\n\ts_nop 1" : "+v"(x)); }
 __device__ __forceinline__ void settle_f32(f32x4& x, f32x4& y) { asm volatile("s_nop 7\n\ts_nop 1" : "+v"(x), "+v"(y)); }

@@ -92,7 +92,7 @@ template <typename E> __device__ __forceinline__ void attend(const AttnParams& p
       st[t] = mma16<E>(frag_of<E>(*reinterpret_cast<const u32x4*>(lds + row_off + t * 2048)), bq[0], st[t]);
       st[t] = mma16<E>(frag_of<E>(*reinterpret_cast<const u32x4*>(lds + (row_off ^ 64) + t * 2048)), bq[1], st[t]);
     }
-    asm volatile("s_nop 7" : "+v"(st[0]), "+v"(st[1]), "+v"(st[2]), "+v"(st[3]));  // (a rare branch behind products, see settle)
+    settle(st);
     if (first + 64 > Lk) {
 #pragma unroll
       for (int t = 0; t < 4; t++)
@@ -233,6 +233,7 @@ __global__ __launch_bounds__(64 * kWaves, NC <= 2 ? 6 : 4) void topk_lds_kernel(
         for (int r = 0; r < 16; r++) acc[r] = 0.f;
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) acc = Mma<E>::mma(__builtin_bit_cast(V8, kf[ks]), as_v8<E>(qf[ks]), acc);
+        settle(acc);
         if (c < kRows) {
           float* const dst = sc + c * stride + t * 32 + 4 * hh;  // rows 8 j + 4 hh + i of the tile
 #pragma unroll
