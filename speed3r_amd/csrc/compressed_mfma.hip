@@ -624,9 +624,8 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
     // insertion into a sorted list.
     // About 24 sampled tiles balance the sweep against the survivors that a looser bound lets through (20 and 30 are within
     // 1 %; every second key from 32 tiles on: 4 032 keys of a video 95 -> 81, but 3 024 keys without neighbours 140 -> 154).
-    const int far = (int)(0x7fffffffu / (64u * krow_bytes));  // a sampled tile's rows lie within 2^31 bytes
     int stride1 = ntiles >= 64 ? (ntiles / 24 < 10 ? ntiles / 24 : 10) : 1;
-    stride1 = stride1 < far ? stride1 : far;
+    while (stride1 > 1 && (uint64_t)(64 * stride1) * krow_bytes > 0x7fffffffu) stride1--;  // a sampled tile's rows lie within 2^31 bytes
 #pragma unroll
     for (int g = 0; g < 2; g++)
 #pragma unroll

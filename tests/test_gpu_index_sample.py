@@ -46,3 +46,14 @@ def test_rows_too_far_apart_for_a_sampled_tile():
     q = k[:, :, :70].contiguous()
     want = ops.compressed_attn_topk(q, k.contiguous(), None, 16)[1]
     assert torch.equal(ops.compressed_attn_topk(q, k, None, 16)[1], want)
+
+
+@pytest.mark.parametrize("keys", [4032, 4100])   # without and with a sample
+def test_one_key_seen_many_times(keys):
+    """An expanded k (token stride 0): every score of a row is the same, the first blocks are the choice."""
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    q, k = (torch.randn((1, 2, n, 64), generator=gen, device=DEV).bfloat16() for n in (130, 1))
+    for topk in (1, 16):
+        idx = ops.compressed_attn_topk(q, k.expand(1, 2, keys, 64), None, topk)[1]
+        assert torch.equal(idx, torch.arange(topk, dtype=torch.int32, device=DEV).expand_as(idx))
+        _check(q, k.expand(1, 2, keys, 64), topk)
