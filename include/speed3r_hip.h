@@ -351,7 +351,8 @@ int s3r_qkv_project_gate_rides(int64_t rows, int H);
  *   a: as for s3r_qkv_project with means and norms, but its outputs (q_out .. v_pool) are not read: they lie in `workspace`,
  *   s3r_attention_layer_workspace bytes at a multiple of 256; gate_w: [2 H, C]; proj_w: [C, C] or NULL (out is then the merged
  *   branches); out: contiguous [B*N, C]; all weights contiguous, 16-byte aligned, in a->dtype.
- * K: 1, 2, 4, 8, 16 or 32.  The gate: 2 H outputs a multiple of 4 up to 32 that ride, or H a multiple of 4 up to 16.
+ * K: 1, 2, 4, 8, 16 or 32; softmax_scale > 0; B H up to 65535.  The gate: 2 H outputs a multiple of 4 up to 32 that ride, or H a
+ * multiple of 4 up to 16.
  */
 int64_t s3r_attention_layer_workspace(int B, int H, int64_t N, int block, int K, int with_projection);
 int s3r_attention_layer(const void* x, const void* qkv_w, const void* qkv_bias, const void* gate_w, const void* gate_bias,

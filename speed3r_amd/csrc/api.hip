@@ -326,6 +326,9 @@ extern "C" int s3r_attention_layer(const void* x, const void* qkv_w, const void*
   // (everything that a later kernel may refuse is refused before the first one runs)
   const bool rides = s3r_qkv_project_gate_rides(M, H) && O % 4 == 0 && O <= 32;
   if (!rides && (C % 256 || C > 1024 || O > 32)) return fail(S3R_ERR_UNSUPPORTED, "s3r_attention_layer: a gate of %d heads", H);
+  if (!(softmax_scale > 0.f) || (int64_t)B * H > 65535)
+    return fail(S3R_ERR_UNSUPPORTED, "s3r_attention_layer: softmax scale %g, %lld heads in all (built for a positive scale, up to 65535)", softmax_scale,
+                (long long)B * H);
   if (Nc > (1 << 21) || (proj_w != nullptr && !aligned16(proj_w)) || !aligned16(gate_w) || (reinterpret_cast<uintptr_t>(proj_bias) & 15u))
     return fail(S3R_ERR_UNSUPPORTED, "s3r_attention_layer: more than 2^21 blocks, or weights that are no multiples of 16 bytes");
   const LayerParts l = layer_parts(B, H, N, a->block, K, proj_w != nullptr);

@@ -17,12 +17,12 @@ def test_refused_before_anything_is_launched():
     L = _lib.lib()
     one, far = ctypes.c_void_p(4096), ctypes.c_void_p(8192)   # (never dereferenced: every call here is refused)
 
-    def call(x=one, gate=one, out=one, ws=far, size=1 << 40, k=16, proj=one, **fields):
+    def call(x=one, gate=one, out=one, ws=far, size=1 << 40, k=16, proj=one, scale=0.125, **fields):
         a = _lib.PrepassArgs(positions=4096, cos_table=4096, sin_table=4096, q_norm_weight=4096, k_norm_weight=4096, N=2048, B=1, H=16, head_dim=64,
                              block=16, table_rows=37, dtype=_lib.S3R_BF16, pos_stride_b=4096, pos_stride_n=2)
         for name, value in fields.items():
             setattr(a, name, value)
-        return L.s3r_attention_layer(x, one, None, gate, None, proj, None, out, ws, size, ctypes.byref(a), k, 0.125, None)
+        return L.s3r_attention_layer(x, one, None, gate, None, proj, None, out, ws, size, ctypes.byref(a), k, scale, None)
 
     for name in ("x", "gate", "out", "ws"):
         assert call(**{name: None}) == _lib.S3R_ERR_BAD_ARG
@@ -30,6 +30,10 @@ def test_refused_before_anything_is_launched():
     assert call(k=3) == _lib.S3R_ERR_UNSUPPORTED and call(k=64) == _lib.S3R_ERR_UNSUPPORTED and call(block=32) == _lib.S3R_ERR_UNSUPPORTED
     assert call(H=18) == _lib.S3R_ERR_UNSUPPORTED                                  # a gate that no kernel takes
     assert call(proj=ctypes.c_void_p(4104)) == _lib.S3R_ERR_UNSUPPORTED
+    # what the index kernels would refuse behind the projection
+    for scale in (0.0, -0.125, float("nan")):
+        assert call(scale=scale) == _lib.S3R_ERR_UNSUPPORTED and b"s3r_attention_layer" in L.s3r_last_error()
+    assert call(B=4096, N=256, size=1 << 50) == _lib.S3R_ERR_UNSUPPORTED and b"s3r_attention_layer" in L.s3r_last_error()
     need = L.s3r_attention_layer_workspace(1, 16, 2048, 16, 16, 1)
     assert need >= 4 * 2048 * 1024 * 2 and call(size=need - 1) == _lib.S3R_ERR_BAD_ARG
     assert call(ws=ctypes.c_void_p(8192 + 128)) == _lib.S3R_ERR_BAD_ARG and call(out=ctypes.c_void_p(4104)) == _lib.S3R_ERR_BAD_ARG
