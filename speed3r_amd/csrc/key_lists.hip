@@ -5,7 +5,7 @@
 // holds the ids of the query blocks whose index row names j, one entry per occurrence, ascending; off[j] .. off[j+1]
 // delimit it.  Entries of idx that are < 0 or >= nkb appear in no list.
 //
-// Up to kHeadEntries index entries per head (count, scan and fill in one kernel, then sort): workgroup (p, head) reads all of the head's
+// Up to kHeadEntries index entries per head, with one exception at the launch (count, scan and fill in one kernel, then sort): workgroup (p, head) reads all of the head's
 // entries and owns the key blocks lo .. hi: it counts theirs in LDS and, in a register, the entries of the blocks below, which gives the
 // start of its first list without a word from the others; then it reads the entries again and writes those of its blocks.  us, five kernels
 // without their sorts / this: 2 x 16 heads of 756 rows of 32 46 / 16, 16 heads of 4 164 rows of 16 43 / 26; with the sorts 2 x 16 x 756 x 32 60 / 30,
@@ -316,7 +316,11 @@ int launch_key_block_lists(const int32_t* idx, int32_t* kq_list, int32_t* kq_off
     return fail(S3R_ERR_UNSUPPORTED, "s3r_key_block_lists: tensor too large for one launch");
   // workgroups for every CU once; each reads all of a head's entries
   const int64_t parts = bh >= 256 ? 1 : 256 / bh < nkb ? 256 / bh : nkb, span = (nkb + parts - 1) / parts;
-  if (nqb * K <= kl::kHeadEntries && K <= 1024 && span <= kl::kMostSpan) {
+  // One head alone: all 256 workgroups read all of its entries, and with many of them the five kernels are as good while the scan is short
+  // and the lists too (us, five kernels / one, entries x key blocks: 98 304 x 8 192 32.6 / 32.7, 131 072 x 4 096 39.9 / 39.6, x 6 144 36.2 / 39.3,
+  // x 8 192 35.4 / 39.4, x 9 216 43.3 / 40.1; two heads of 131 072 x 8 192 48.3 / 43.1).
+  const bool crowded = bh == 1 && nqb * K > 98304 && nkb > 4096 && nkb <= 8192;
+  if (nqb * K <= kl::kHeadEntries && K <= 1024 && span <= kl::kMostSpan && !crowded) {
     hipLaunchKernelGGL(kl::head_lists_kernel, dim3((unsigned)parts, (unsigned)bh), dim3(1024), (unsigned)(span * 4), st, idx, kq_off, kq_list, H,
                        (int)nqb, K, (int)nkb, (int)span, sib, sih, sim, list_stride);
   } else {

@@ -30,9 +30,13 @@ def test_lists_of_length(n):
 
 
 # entries per head on both sides of the line between the kernels that make the lists; key blocks that the workgroups of a head share unevenly,
-# fewer of them than workgroups, more heads than CUs; strided index rows, entries that are skipped
+# fewer of them than workgroups, more heads than CUs; strided index rows, entries that are skipped; a workgroup's key blocks with one counter
+# a thread and with more, up to the most that it takes (64 KB of counters) and one beyond; one head's many entries over the block counts that the
+# two ways share
 @pytest.mark.parametrize("bh,nqb,k,nkb", [(1, 4096, 32, 4096), (1, 4097, 32, 300), (3, 1000, 5, 1), (2, 777, 16, 3), (16, 130, 8, 131), (300, 20, 4, 20),
-                                          (1, 50, 2, 70000), (2, 100, 64, 20000)])
+                                          (1, 50, 2, 70000), (2, 100, 64, 20000), (256, 40, 4, 1024), (256, 40, 4, 1025), (257, 40, 3, 2047),
+                                          (128, 90, 7, 5000), (256, 90, 5, 16384), (256, 90, 5, 16385), (1, 6144, 16, 8192), (1, 6145, 16, 8192),
+                                          (1, 6145, 16, 8193), (1, 6145, 16, 4096)])
 def test_lists_of_heads(bh, nqb, k, nkb):
     gen = torch.Generator().manual_seed(nqb)
     wide = torch.randint(-2, nkb + 2, (1, bh, nqb, k + 3), generator=gen, dtype=torch.int32)
