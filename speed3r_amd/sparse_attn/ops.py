@@ -993,6 +993,14 @@ def qkv_prepass_bwd(qkv: torch.Tensor, num_heads: int, block: int, positions, co
     return d_qkv, d_norm
 
 
+def _norm_grads(d_norm: Optional[torch.Tensor], params):
+    """Rows of ``d_norm`` in the types of ``params`` (None: none), tensors of their own: autograd keeps what it is given as .grad.  Those of
+    its own type by one launch, not a copy each; the others' conversion is a copy."""
+    same = [i for i, t in enumerate(params) if t is not None and t.dtype == d_norm.dtype]
+    own = dict(zip(same, torch._foreach_mul([d_norm[i] for i in same], 1.0))) if same else {}
+    return [None if t is None else own[i] if i in own else d_norm[i].to(t.dtype) for i, t in enumerate(params)]
+
+
 class _LayerCoreFn(torch.autograd.Function):
     """Everything of the layer between its projections, ``(packed qkv, gate, qk-norm parameters) -> ([B,N,C], indices)``
     (pi3/models/layers/sparse_attention.py:97-136): the forward kernels of the inference route with their log-sum-exps,
@@ -1024,10 +1032,7 @@ class _LayerCoreFn(torch.autograd.Function):
         full = attn_bwd(q, k, v, o_s, d_os, lse, idx, block, delta=delta_s)
         q_ln, k_ln = ((q_w, q_b), (k_w, k_b)) if q_w is not None else (None, None)
         d_qkv, d_norm = qkv_prepass_bwd(qkv, heads, block, xpos, cos, sin, q_ln, k_ln, eps, (q_raw, k_raw), (*full, *pooled), inv_freq, signed=True)
-        # (tensors of their own, autograd keeps what it is given as .grad: by one launch, not a copy each)
-        own = iter(torch._foreach_mul([d_norm[i] for i, t in enumerate((q_w, q_b, k_w, k_b)) if t is not None], 1.0) if q_w is not None else ())
-        params = [next(own).to(t.dtype) if t is not None else None for t in (q_w, q_b, k_w, k_b)]
-        return d_qkv, d_gate, *params, *([None] * 8)
+        return d_qkv, d_gate, *_norm_grads(d_norm, (q_w, q_b, k_w, k_b)), *([None] * 8)
 
 
 def layer_core_autograd(qkv: torch.Tensor, gate: torch.Tensor, heads: int, block: int, topk: int, xpos, cos, sin, inv_freq, q_ln, k_ln, eps: float):
