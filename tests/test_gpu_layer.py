@@ -5,6 +5,7 @@ import torch
 import oracle
 from helpers import max_abs
 from speed3r_amd.layers import RoPE2D, SparseFlashAttentionRope
+from speed3r_amd.sparse_attn import ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -252,16 +253,58 @@ def test_layer_takes_the_one_pass_route_where_it_is_built():
         assert m3.last_prepass is False and m3.last_path == "fused-merge"
 
 
-@pytest.mark.parametrize("n,block,topk", [(8192, 16, 32), (8193, 16, 32), (8207, 16, 4), (100, 64, 2)])
-def test_operators_give_the_same_bits_on_one_stream_and_on_two(n, block, topk):
-    """Around the line where the index kernel moves to a stream of its own (512 blocks x 16 heads), and below it."""
+# (heads, tokens, block, top-k, indices and attention are two kernels, the index kernel has a stream of its own by default): short lists of keys up to
+# 1216 (640 for top-4), two waves to a row's keys up to 2 048 blocks of 16 heads, few heads and long lists from 2 433 blocks on
+STREAMS = [(16, 16 * 1216, 16, 32, False, False), (16, 16 * 1217, 16, 32, True, True), (16, 16 * 2048 - 3, 16, 32, True, True),
+           (16, 16 * 2049, 16, 32, True, True), (16, 16 * 640, 16, 4, False, False), (16, 16 * 641, 16, 4, True, False),
+           (4, 16 * 2432, 16, 16, True, False), (4, 16 * 2433 - 5, 16, 16, True, True), (16, 64 * 1300 - 9, 64, 16, True, True),
+           (16, 100, 64, 2, True, False)]
+
+
+@pytest.mark.parametrize("h,n,block,topk,two_kernels,beside", STREAMS)
+def test_operators_give_the_same_bits_on_one_stream_and_on_two(h, n, block, topk, two_kernels, beside):
+    """Around the lines where the index kernel is one launch with the attention and where it moves to a stream of its own."""
     import speed3r_amd as s3r
 
-    g = torch.Generator().manual_seed(n)
-    q, k, v = (torch.randn((1, 16, n, 64), generator=g).to(torch.bfloat16).cuda() for _ in range(3))
-    gate = torch.rand((1, 16, n, 2), generator=g).to(torch.bfloat16).cuda()
-    got = [s3r.sparse_global_attention(q, k, v, gate, block, topk, overlap=o) for o in (None, True, False)]
-    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    g = torch.Generator(device=DEV).manual_seed(n)
+    q, k, v = (torch.randn((1, h, n, 64), generator=g, device=DEV).to(torch.bfloat16) for _ in range(3))
+    gate = torch.rand((1, h, n, 2), generator=g, device=DEV).to(torch.bfloat16)
+    assert ops._two_kernel_compressed(q, topk, block) is two_kernels and ops._indices_beside(q, topk, block) is beside
+    want = s3r.sparse_global_attention(q, k, v, gate, block, topk, overlap=False)
+    for overlap in (None, True) * 3:                                              # (a hole in the order would have a chance to show)
+        assert torch.equal(s3r.sparse_global_attention(q, k, v, gate, block, topk, overlap=overlap), want)
+
+
+@pytest.mark.parametrize("blocks,one_call", [(1217, True), (2048, True), (2049, False)])
+def test_layer_gives_the_same_bits_on_one_stream_and_on_two(monkeypatch, blocks, one_call):
+    """16-token blocks on both sides of the line where the layer is one call on one stream."""
+    torch.manual_seed(blocks)
+    with torch.device(DEV):
+        m = SparseFlashAttentionRope(dim=1024, num_heads=16, qkv_bias=True, qk_norm=True, rope=RoPE2D(100.0), block_size=4, topk=32)
+    m = m.to(torch.bfloat16).eval()
+    x = torch.randn(1, 16 * blocks, 1024, device=DEV).to(torch.bfloat16)
+    pos = torch.randint(0, 36, (1, 16 * blocks, 2), device=DEV)
+    calls = {"one call": 0, "second stream": 0}
+
+    def counted(name, fn):
+        def call(*args, **kwargs):
+            out = fn(*args, **kwargs)
+            calls[name] += out is not None
+            return out
+        return call
+
+    monkeypatch.setattr(ops, "attention_layer", counted("one call", ops.attention_layer))
+    monkeypatch.setattr(ops, "topk_indices_on_side_stream", counted("second stream", ops.topk_indices_on_side_stream))
+    with torch.no_grad():
+        plain = [m(x, xpos=pos) for _ in range(3)]
+        assert calls == ({"one call": 3, "second stream": 0} if one_call else {"one call": 0, "second stream": 3})
+        m.keep_topk_idx = True                                                    # (which takes the kernels one by one)
+        beside = [m(x, xpos=pos) for _ in range(3)]
+        assert calls["second stream"] == (3 if one_call else 6)
+        monkeypatch.setattr(ops, "_indices_beside", lambda *a: False)
+        want = m(x, xpos=pos)
+        assert calls["second stream"] == (3 if one_call else 6)
+    assert all(torch.equal(t, want) for t in plain + beside)
 
 
 def _layer_and_input(block_size, rope, n=200, seed=0, dim=256):
