@@ -13,9 +13,9 @@
 // fp32, P rounded to the I/O dtype, O^T += V^T P^T with V^T fragments from ds_read_b64_tr_b16.
 //
 // Selection without a score buffer (the top-k-only instance, KTOP > 0): two sweeps over the key tiles, K tiles by
-// direct transfers into an LDS ring.  Sweep 1 deals every s-th key out to 128 groups per row (64 registers in each of the
-// row's two lanes) and keeps each group's maximum; the K-th largest of them is a lower bound of the row's K-th largest score.  Sweep 2 recomputes the scores
-// and appends every score >= that threshold to a small per-lane queue in LDS (no branch).  Every lane keeps the
+// direct transfers into an LDS ring.  Sweep 1 deals every s-th key out to 32 to 128 groups per row (by K; registers of the
+// row's two lanes, twice as many where two waves share a row) and keeps each group's maximum; the K-th largest of them is a lower
+// bound of the row's K-th largest score.  Sweep 2 recomputes the scores and appends every score >= that threshold to a small per-lane queue in LDS (no branch).  Every lane keeps the
 // exact top-K of the keys IT sees (half of each tile): a descending sorted list of K keys,
 // key = (sortable(bits(score)), Lk-1-col) in lexicographic order, in registers.  When some lane's queue is nearly
 // full, all lanes merge their queues into their lists with a register-resident bitonic network (no divergence:
@@ -471,25 +471,36 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
     const int dl_row = pair_wave * (8 * NI) + (lane >> 3);
     // (the chunk map repeats every 16 rows: instructions of equal parity share it)
     const uint32_t dl_chunk[2] = {(uint32_t)(((lane & 7) ^ k_swizzle(lane >> 3)) * 16), (uint32_t)(((lane & 7) ^ k_swizzle((lane >> 3) + 8)) * 16)};
-    uint32_t dl_off[4] = {0, 0, 0, 0};  // NI of them are used
+    // Tile t of a sweep holds keys 64 t s, (64 t + 1) s, ...: every key (s = 1) or, in the first sweep, every s-th one.  All tiles but the
+    // last are full; the last one's rows are counted once per sweep (a division by s per tile stood in every tile's chain:
+    // 16 heads of 2 200 keys, top-1, 54.9 us with it, 50.8 without).
+    struct Tiles {
+      int s, count, last;      // spacing of the keys; tiles; last row of the last one
+      uint32_t off[4];         // per-lane offsets of a full tile, NI of them
+    };
+    auto tiles_of = [&](const int s) {
+      Tiles w;
+      w.s = s;
+      w.count = s == 1 ? ntiles : (int)((uint32_t)(ntiles + s - 1) / (uint32_t)s);
+      const int left = (int)Lk - 1 - (w.count - 1) * 64 * s;
+      w.last = s == 1 ? left : (int)((uint32_t)left / (uint32_t)s);
 #pragma unroll
-    for (int i = 0; i < NI; i++) dl_off[i] = (uint32_t)(dl_row + 8 * i) * krow_bytes + dl_chunk[i & 1];
-    // Tile t of a sweep holds keys 64 t s, (64 t + 1) s, ...: every key (s = 1) or, in the first sweep, every s-th one.
-    auto dma_tile = [&](int t, int buf, const int s, const int nt) {  // tiles past the end repeat the last one (never read)
-      const int tt = t < nt ? t : nt - 1;
-      const int64_t start = (int64_t)tt * 64 * s;
-      const int rem = (int)((uint32_t)(Lk - 1 - start) / (uint32_t)s);
-      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(kp + start * p.skn), 0, 0x7fffffff, 0x00020000);
+      for (int i = 0; i < 4; i++) w.off[i] = i < NI ? (uint32_t)(dl_row + 8 * i) * (krow_bytes * (uint32_t)s) + dl_chunk[i & 1] : 0u;
+      return w;
+    };
+    auto dma_tile = [&](int t, int buf, const Tiles& w) {  // tiles past the end repeat the last one (never read)
+      const int tt = t < w.count ? t : w.count - 1;
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(kp + (int64_t)tt * 64 * w.s * p.skn), 0, 0x7fffffff, 0x00020000);
       char* dst = reinterpret_cast<char*>(&Ks[part * NB + buf][0]) + pair_wave * (NI * 1024);
-      uint32_t off[4] = {0, 0, 0, 0};  // the per-lane offsets of a full tile never change
+      uint32_t off[4] = {0, 0, 0, 0};
 #pragma unroll
-      for (int i = 0; i < NI; i++) off[i] = s == 1 ? dl_off[i] : (uint32_t)(dl_row + 8 * i) * (krow_bytes * (uint32_t)s) + dl_chunk[i & 1];
-      if (__builtin_expect(rem < 63, 0)) {       // ragged last tile: rows beyond the end re-read the last row
+      for (int i = 0; i < NI; i++) off[i] = w.off[i];
+      if (__builtin_expect(tt == w.count - 1 && w.last < 63, 0)) {  // ragged last tile: rows beyond the end re-read the last row
 #pragma unroll
         for (int i = 0; i < NI; i++) {
           int r = dl_row + 8 * i;
-          r = r < rem ? r : rem;
-          off[i] = (uint32_t)r * (krow_bytes * (uint32_t)s) + dl_chunk[i & 1];
+          r = r < w.last ? r : w.last;
+          off[i] = (uint32_t)r * (krow_bytes * (uint32_t)w.s) + dl_chunk[i & 1];
           asm volatile("" : "+v"(off[i]));       // stays inside this branch
         }
       }
@@ -499,21 +510,24 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
     };
     const uint32_t lds_k = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)reinterpret_cast<char*>(&Ks[0][0]);
     const uint32_t kr_off = lds_k + (uint32_t)part * (NB * kTile * (uint32_t)sizeof(E)) + (uint32_t)(c * 128 + ((hh ^ k_swizzle(c)) << 4));  // A operand: lane = key row, chunk hh + 2 ks
-    float best[FUSED ? 2 : 1][2][16];  // first sweep: per register the largest score of the even and of the odd tiles
+    // first sweep: the lane's largest scores of each group.  Short lists need few groups: one per pair of registers up to top-4, one per
+    // register at top-8, beyond one per register in the even and one in the odd tiles
+    constexpr int SETS = KL > 16 ? 2 : 1, HALVES = KL <= 4 ? 1 : 2, GROUPS = SETS * HALVES * 16;
+    float best[SETS][HALVES][16];
     auto sweep = [&](auto filter_tag, const int keystep) {  // every keystep-th key
       constexpr bool FILTER = decltype(filter_tag)::value;
-      const int s = FILTER ? 1 : keystep;
-      const int all = FILTER ? ntiles : (int)((Lk + 64 * s - 1) / (64 * s)), nsteps = (all + PARTS - 1) / PARTS;
-      for (int i = 0; i < NB - 1; i++) dma_tile(i * PARTS + part, i, s, all);
+      const Tiles w = tiles_of(FILTER ? 1 : keystep);
+      const int nsteps = (w.count + PARTS - 1) / PARTS;
+      for (int i = 0; i < NB - 1; i++) dma_tile(i * PARTS + part, i, w);
       int buf = 0, fill = NB - 1;  // ring positions of step i's tile and of step i + NB - 1's
       for (int i = 0; i < nsteps; i++) {
         // this wave's share of tile t has landed (transfers complete in order, NI per tile, NB - 2 tiles younger) ...
         __builtin_amdgcn_s_waitcnt(0x0F70 | (NI * (NB - 2)));
         __builtin_amdgcn_s_barrier();  // ... and everybody's; all waves are done with tile t - 1, whose buffer is refilled now
-        dma_tile((i + NB - 1) * PARTS + part, fill, s, all);
+        dma_tile((i + NB - 1) * PARTS + part, fill, w);
         {
-          const int64_t start = (int64_t)(i * PARTS + part) * 64 * s;
-          const bool partial = start + 63 * s >= Lk;
+          const int tile = i * PARTS + part;
+          const bool partial = tile == w.count - 1 ? w.last < 63 : PARTS > 1 && tile >= w.count;
           u32x4 kf[2][4];
           const uint32_t kb = kr_off + (uint32_t)buf * (kTile * (uint32_t)sizeof(E));
           lds_read_kfrags(kb, kf);
@@ -534,7 +548,7 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
           fill = fill + 1 == NB ? 0 : fill + 1;
           if (partial) {  // last tile only (or, of the second part, none left): keys beyond Lk get a score that neither raises a maximum nor passes the filter
             // register r of tile kt holds row kt*32 + 4hh + 8(r/4) + r%4 of the tile
-            const int lim = (PARTS > 1 && start >= Lk ? 0 : (int)((uint32_t)(Lk - 1 - start) / (uint32_t)s) + 1) - 4 * hh;
+            const int lim = (PARTS > 1 && tile >= w.count ? 0 : w.last + 1) - 4 * hh;
 #pragma unroll
             for (int kt = 0; kt < 2; kt++)
 #pragma unroll
@@ -542,15 +556,18 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
                 if (kt * 32 + 8 * (r >> 2) + (r & 3) >= lim) st[kt][r] = FILTER ? __uint_as_float(0x7FC00000u) : -INFINITY;
           }
           if constexpr (!FILTER) {
-            auto raise = [&](float (&g)[2][16]) {
+            auto raise = [&](float (&g)[HALVES][16]) {  // (NaN loses)
 #pragma unroll
-              for (int kt = 0; kt < 2; kt++)
+              for (int kt = 0; kt < HALVES; kt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) asm("v_max_f32 %0, %0, %1" : "+v"(g[kt][r]) : "v"(st[kt][r]));  // (NaN loses)
+                for (int r = 0; r < 16; r++) {
+                  if constexpr (HALVES == 1) asm("v_max3_f32 %0, %0, %1, %2" : "+v"(g[0][r]) : "v"(st[0][r]), "v"(st[1][r]));
+                  else asm("v_max_f32 %0, %0, %1" : "+v"(g[kt][r]) : "v"(st[kt][r]));
+                }
             };
-            if (i & 1) raise(best[FUSED ? 1 : 0]); else raise(best[0]);
+            if (SETS == 2 && (i & 1)) raise(best[SETS - 1]); else raise(best[0]);
           } else {
-            const uint32_t col0 = (uint32_t)start + 4 * hh;
+            const uint32_t col0 = (uint32_t)(tile * 64 + 4 * hh);
             const uint32_t qbase = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)reinterpret_cast<char*>(qlane);
             // One test for the whole tile first: the largest of the lane's 32 scores (two chains of three-way maxima, no
             // branch between them; a masked key's NaN loses either way) against the threshold.  Six tiles in seven hold no
@@ -614,78 +631,78 @@ __global__ __launch_bounds__(256, KTOP > 0 && PARTS == 1 ? 3 : 2) void compresse
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the transfers issued past the last tile are done too
     };
     // First sweep: a lower bound of each row's K-th largest score from a sample of the keys, every stride1-th of them.  Sample m
-    // goes to row m % 64 of tile m / 64; each of a lane's 32 registers keeps its largest score over the even and over the odd
-    // tiles, and the K-th largest of the row's 2 x 64 maxima is the bound.  Both the sample and the groups are spread over the
-    // sequence on purpose: a query's best keys lie side by side (the blocks of one frame), and with groups of 32 neighbours
-    // in every stride1-th tile, as this kernel had them before, a frame was one or two groups and was often missed:
-    // Pooled blocks of a video x 16 heads, us before / now: 16 656 keys, top-32 851 / 738; 16 266, top-16 759 / 681; 4 164 114 / 96;
-    // 2 016, top-32 91 / 54; 1 627 55 / 38.  Scores without such neighbours: within 4 % either way (16 266 keys 1 271 / 1 256,
-    // 3 024 147 / 141, 4 164 top-8 131 / 136).  The sweep itself got cheaper too: 32 maxima per tile in place of 31 and an
-    // insertion into a sorted list.
+    // goes to row m % 64 of tile m / 64, and the registers of a lane keep the largest scores of groups of such rows (best); the K-th largest
+    // of the row's maxima is the bound.  Both the sample and the groups are spread over the sequence on purpose: a query's best keys lie
+    // side by side (the blocks of one frame), and with groups of 32 neighbours in every stride1-th tile a frame was one or two groups
+    // and was often missed.  us, 16 heads, groups of neighbours / spread ones, pooled blocks of a video (keys without such neighbours):
+    // 16 266 keys, top-16 769 / 653 (1 307 / 1 225), top-1 582 / 511 (735 / 654); 4 164, top-32 182 / 116 (222 / 202), top-4 78 / 69 (110 / 100);
+    // 3 000, top-16 90 / 61 (102 / 103), top-1 48 / 49 (60 / 58); 2 200, top-4 44 / 39 (56 / 57).  128 groups a row for every K: 2 200 keys,
+    // top-1 36 -> 41, top-16 48 -> 52 (the registers' sort is a chain of its own).
     // About 24 sampled tiles balance the sweep against the survivors that a looser bound lets through (20 and 30 are within
     // 1 %; every second key from 32 tiles on: 4 032 keys of a video 95 -> 81, but 3 024 keys without neighbours 140 -> 154).
     int stride1 = ntiles >= 64 ? (ntiles / 24 < 10 ? ntiles / 24 : 10) : 1;
     while (stride1 > 1 && (uint64_t)(64 * stride1) * krow_bytes > 0x7fffffffu) stride1--;  // a sampled tile's rows lie within 2^31 bytes
-#pragma unroll
-    for (int g = 0; g < 2; g++)
-#pragma unroll
-      for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) best[g][kt][r] = -INFINITY;
-    sweep(std::false_type{}, stride1);
-    // the K largest of the lane's 64 maxima, descending (pieces sorted and merged: once per wave)
-    float top[KL];
-    {
-      constexpr int PIECE = KL < 4 ? 4 : KL;
-      float all[64];
-#pragma unroll
-      for (int g = 0; g < 64; g++) all[g] = best[g >> 5][(g >> 4) & 1][g & 15];
-      float run[PIECE];
-#pragma unroll
-      for (int pc = 0; pc < 64 / PIECE; pc++) {
-        float x[PIECE];
-#pragma unroll
-        for (int i = 0; i < PIECE; i++) x[i] = all[pc * PIECE + i];
-        sort_desc<PIECE>(x);
-#pragma unroll
-        for (int i = 0; i < PIECE; i++) run[i] = pc == 0 ? x[i] : fmaxf(run[i], x[PIECE - 1 - i]);
-        if (pc != 0) bitonic_merge_desc<PIECE>(run);
-      }
-#pragma unroll
-      for (int i = 0; i < KL; i++) top[i] = run[i];
-    }
-    // Threshold: the K-th largest of the row's group maxima, i.e. of the union of the two lanes' lists.  K
-    // different scores (one per group) are at least that large, so a score below it is not among the K
-    // largest, whatever the tie-break.  With fewer than K groups that hold a key it stays -inf and every score is a candidate.
-    // The K-th largest of two descending lists a, b is the largest min(a[i-1], b[K-i-1]) over the splits i.
-    {
-      float tau;
-      if constexpr (PARTS == 1) {
-        tau = fmaxf(top[KL - 1], __uint_as_float(xh_swap(__float_as_uint(top[KL - 1]))));  // splits i = K and i = 0
-#pragma unroll
-        for (int i = 1; i < KL; i++) {
-          const float bi = __uint_as_float(xh_swap(__float_as_uint(top[KL - i - 1])));
-          tau = fmaxf(tau, fminf(top[i - 1], bi));
-        }
-      } else {  // the two lanes' K largest, descending in both, and the same of the other part, through the queues' space
-        float both[KL];
-#pragma unroll
-        for (int i = 0; i < KL; i++) both[i] = fmaxf(top[i], __uint_as_float(xh_swap(__float_as_uint(top[KL - 1 - i]))));
-        if constexpr (KL > 1) bitonic_merge_desc<KL>(both);
-        static_assert(KL * 32 * 4 <= (int)sizeof(queue[0]), "a wave's queues hold its rows' bounds");
-        float* const mine = reinterpret_cast<float*>(&queue[wave][0][0]) + c;
-        const float* const other = reinterpret_cast<const float*>(&queue[wave ^ PW][0][0]) + c;
-        if (hh == 0) {
-#pragma unroll
-          for (int i = 0; i < KL; i++) mine[i * 32] = both[i];
-        }
-        __syncthreads();
-        tau = fmaxf(both[KL - 1], other[(KL - 1) * 32]);
-#pragma unroll
-        for (int i = 1; i < KL; i++) tau = fmaxf(tau, fminf(both[i - 1], other[(KL - i - 1) * 32]));
-      }
-      thr0 = qvalid ? tau : INFINITY;  // rows beyond Lq (all-zero scores) must not flood the queue
+    // One or two tiles: every score goes through the queue (32 heads of 1 000 rows, us with a first sweep / without: 100 keys,
+    // top-32 21.7 / 14.2, top-16 15.1 / 10.9; 200 keys, top-16 18.1 / 16.4).
+    if (ntiles <= (KL >= 8 ? 2 : 1)) {
+      thr0 = qvalid ? -INFINITY : INFINITY;
       thr = thr0;
+    } else {
+#pragma unroll
+      for (int g = 0; g < SETS; g++)
+#pragma unroll
+        for (int kt = 0; kt < HALVES; kt++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) best[g][kt][r] = -INFINITY;
+      sweep(std::false_type{}, stride1);
+      // the K largest of the lane's maxima, descending (pieces sorted and merged: once per wave)
+      float top[KL];
+#pragma unroll
+      for (int pc = 0; pc < GROUPS / KL; pc++) {
+        float x[KL];
+#pragma unroll
+        for (int i = 0; i < KL; i++) {
+          const int g = pc * KL + i;
+          x[i] = best[g / (16 * HALVES)][g / 16 % HALVES][g % 16];
+        }
+        sort_desc<KL>(x);
+#pragma unroll
+        for (int i = 0; i < KL; i++) top[i] = pc == 0 ? x[i] : fmaxf(top[i], x[KL - 1 - i]);
+        if (pc != 0) bitonic_merge_desc<KL>(top);
+      }
+      // Threshold: the K-th largest of the row's group maxima, i.e. of the union of the two lanes' lists.  K
+      // different scores (one per group) are at least that large, so a score below it is not among the K
+      // largest, whatever the tie-break.  With fewer than K groups that hold a key it stays -inf and every score is a candidate.
+      // The K-th largest of two descending lists a, b is the largest min(a[i-1], b[K-i-1]) over the splits i.
+      {
+        float tau;
+        if constexpr (PARTS == 1) {
+          tau = fmaxf(top[KL - 1], __uint_as_float(xh_swap(__float_as_uint(top[KL - 1]))));  // splits i = K and i = 0
+#pragma unroll
+          for (int i = 1; i < KL; i++) {
+            const float bi = __uint_as_float(xh_swap(__float_as_uint(top[KL - i - 1])));
+            tau = fmaxf(tau, fminf(top[i - 1], bi));
+          }
+        } else {  // the two lanes' K largest, descending in both, and the same of the other part, through the queues' space
+          float both[KL];
+#pragma unroll
+          for (int i = 0; i < KL; i++) both[i] = fmaxf(top[i], __uint_as_float(xh_swap(__float_as_uint(top[KL - 1 - i]))));
+          if constexpr (KL > 1) bitonic_merge_desc<KL>(both);
+          static_assert(KL * 32 * 4 <= (int)sizeof(queue[0]), "a wave's queues hold its rows' bounds");
+          float* const mine = reinterpret_cast<float*>(&queue[wave][0][0]) + c;
+          const float* const other = reinterpret_cast<const float*>(&queue[wave ^ PW][0][0]) + c;
+          if (hh == 0) {
+#pragma unroll
+            for (int i = 0; i < KL; i++) mine[i * 32] = both[i];
+          }
+          __syncthreads();
+          tau = fmaxf(both[KL - 1], other[(KL - 1) * 32]);
+#pragma unroll
+          for (int i = 1; i < KL; i++) tau = fmaxf(tau, fminf(both[i - 1], other[(KL - i - 1) * 32]));
+        }
+        thr0 = qvalid ? tau : INFINITY;  // rows beyond Lq (all-zero scores) must not flood the queue
+        thr = thr0;
+      }
     }
     // Second sweep: the scores again (same MFMA sequence, same bits), filtered against the threshold; survivors go
     // through the lane's queue into its exact list.
@@ -757,7 +774,7 @@ static int launch_e(const AttnParams& p, bool fused, hipStream_t st) {
   // heads, top-16 1 217 keys 52 / 38 (52 / 27), 1 627 62 / 43 (62 / 31); 2 016 top-32 95 / 63 (105 / 54), top-4 50 / 36 (44 / 27), 2 048
   // top-1 39 / 30 (28 / 25); 8 heads, 4 000 top-16 115 / 77 (110 / 58); 2 heads, 5 000 top-32 193 / 103 (194 / 93); 1 head, 16 384
   // top-16 369 / 216 (332 / 182).  Beyond 512 workgroups a second round of them: 2 200 keys stay with quads.
-  const bool parts = pairs <= 2 * 256;
+  const bool parts = pairs <= 2 * 256 && p.Lk > 64;  // (one tile has nothing to share: 32 heads of 1 000 rows, 64 keys, top-16 10.8 / 7.8)
   const int waves = two ? 2 : 4, rows = two || parts ? 64 : 128;
   const int64_t nqg = (p.Lq + rows - 1) / rows;
   if (nqg > 0x7fffffffLL) return fail(S3R_ERR_UNSUPPORTED, "s3r_compressed_attn_topk: grid too large");
