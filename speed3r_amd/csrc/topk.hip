@@ -1,15 +1,17 @@
 // Exact row-wise top-k of materialised fp32 scores: one wavefront per row, HBM-streaming.
 //
-// The wave reads its row 256 columns at a time (16 bytes per lane, two loads in flight).  Lane p
-// keeps the p-th largest 64-bit key seen so far, key = sortable(bits(score)) << 32 | (cols-1-col),
-// so the lanes together hold a descending sorted list and lane K-1 holds the admission
-// threshold.  Each score is first compared, as a float, against the threshold's score (one
-// VALU compare; the test is conservative: ties, signed zeros and NaNs pass); only if some lane
-// of the wave has a candidate are exact keys formed, and candidates beating the threshold key
-// are inserted one at a time with a single-lane shift of the list.  Keys are unique per row,
-// so the result is the unique top-k under the reference's order: descending score, equal
-// scores lowest column first, +0.0 above -0.0, NaNs by bit pattern.  Unfilled slots keep key
-// 0, which decodes to column cols-1, the reference's filler when cols < K.
+// Keys: sortable(bits(score)) << 32 | (cols-1-col), unique per row, so the result is the unique top-k under the reference's order:
+// descending score, equal scores lowest column first, +0.0 above -0.0, NaNs by bit pattern.  Slots that nothing fills keep key 0,
+// which decodes to column cols-1, the reference's filler when cols < K.
+//
+// Rows of up to 1024 columns: the wave holds the row in registers, finds a lower bound of its K-th largest score from the maxima of
+// 256 groups of columns, and ranks what lies at or above it by counting, one candidate per lane (up to 64 of them; few columns
+// are all candidates).  Longer rows, and those with more candidates: 4096 columns at a time in registers, each with such a bound; lane
+// p keeps the p-th largest key seen so far, so the lanes together hold a descending sorted list and lane K-1 holds the admission
+// threshold.  Each score is first compared, as a float, against bound and threshold (one VALU compare; the test is conservative:
+// ties, signed zeros and NaNs pass); only if some lane of the wave has a candidate are exact keys formed, and candidates
+// beating the threshold key are inserted one at a time with a single-lane shift of the list.  Long rows that cannot be read 16 bytes at
+// a time: the same, 64 columns at a time and without the bound.
 #include "s3r_common.h"
 
 namespace s3r {
@@ -58,7 +60,9 @@ struct RowTopK {
 
 // SEG: 256 columns each that a wave holds at once.  A row that fits one segment has its candidates, K to 1.4 K as a rule, ranked by
 // counting, one per lane, in place of an insertion each (us, before / now: 2 096 rows of 132
-// scores, top-16 8.8 / 5.5, of 131, which are not at 16 bytes, 13 / 6; 8 064 of 504, top-32 25.0 / 14.5; 16 000 of 1 024 49.9 / 26.4).
+// scores, top-16 8.8 / 5.5, of 131, which are not at 16 bytes, 13 / 6; 8 064 of 504, top-32 25.0 / 14.5; 16 000 of 1 024 49.9 / 26.4).  Few
+// columns are ranked without a search for a bound first (20 000 rows, insertions / search / neither: 1 column 6.6 / 14.8 / 4.2, 9, top-16 11.5 /
+// 16.3 / 5.5, 31 25.4 / 19.5 / 11.0; 16 rows of 63, top-64 5.9 / 6.6 / 5.0).
 template <int SEG>
 __global__ __launch_bounds__(256) void topk_rows_kernel(const float* __restrict__ scores, int32_t* __restrict__ idx,
                                                         int64_t rows, int cols_all, int64_t row_stride, int K, int vec_ok,
@@ -76,6 +80,14 @@ __global__ __launch_bounds__(256) void topk_rows_kernel(const float* __restrict_
   RowTopK st;
   st.init(K, lane);
   const uint32_t last = (uint32_t)(cols - 1);
+  if (SEG == 1 && (cols <= 32 || (cols <= 64 && 2 * K >= cols))) {  // every score is a candidate, one per lane
+    const uint64_t key = lane < cols ? ((uint64_t)sortable_key(row[lane]) << 32) | (last - (uint32_t)lane) : 0;
+    int rank = 0;
+    for (int u = 0; u < cols; u++) rank += readlane_u64(key, u) > key ? 1 : 0;
+    if (lane < cols && rank < K) idx[w * K + rank] = lane;
+    if (lane >= cols && lane < K) idx[w * K + lane] = (int32_t)last;
+    return;
+  }
 
   int c0 = 0;
   if (vec_ok || SEG <= 4) {
