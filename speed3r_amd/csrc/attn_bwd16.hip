@@ -13,8 +13,9 @@
 // Rows go global -> LDS by direct transfers, two steps in flight: a step reads all its operands into registers, requests
 // the step after next into the same buffers and computes meanwhile; nothing else is pipelined, the other waves of the
 // SIMD fill the gaps.
-// Bound: the vector cache's path into the LDS (about 20 cycles of the CU per KB, 60 to 70 % busy) and the LDS itself (a step
-// of dK/dV moves 8 KB in and reads 18 KB, 200 cycles), not the matrix cores (20 %).
+// Bound: the address unit on the way from the vector cache into the LDS.  Counters, layer features, 2 x 12 096 tokens, 16 heads, top-32,
+// dQ / dK/dV: that unit busy 81 / 74 %, vector port 38 / 29 %, matrix cores 26 / 19 %, LDS reads 21 / 23 %, 90 / 83 % of the requests
+// served by the L2.
 // us, 16 heads, top-32, before / now: layer features, 24 192 tokens: dQ 304 / 141, dK/dV 504 / 234; 4 032 tokens 74 / 34 and
 // 115 / 62; video (lists of neighbours that agree), 96 768 tokens: 577 / 467 and 1 317 / 863, 24 192: 160 / 113 and 381 / 229.
 #include "block16.h"
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(64, 4) void bwd16_dq_kernel(BwdParams p, int nqb, i
   const E* qp = (const E*)p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh + 8 * g;
   const E* gp = (const E*)p.dout + (int64_t)b * p.sgb + (int64_t)h * p.sgh + 8 * g;
   const int64_t stat = ((int64_t)b * p.H + h) * p.Lq;
-  V8 bq[kNQ][2], bg[kNQ][2];  // B operands of the four query blocks: lane = query, head dimensions 32 ks + 8 g ..
+  V8 bq[kNQ][2], bg[kNQ][2];  // B operands of the query blocks: lane = query, head dimensions 32 ks + 8 g ..
   float nlse[kNQ], dls[kNQ];
 #pragma unroll
   for (int j = 0; j < kNQ; j++) {

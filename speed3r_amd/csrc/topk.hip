@@ -61,8 +61,8 @@ struct RowTopK {
 // SEG: 256 columns each that a wave holds at once.  A row that fits one segment has its candidates, K to 1.4 K as a rule, ranked by
 // counting, one per lane, in place of an insertion each (us, before / now: 2 096 rows of 132
 // scores, top-16 8.8 / 5.5, of 131, which are not at 16 bytes, 13 / 6; 8 064 of 504, top-32 25.0 / 14.5; 16 000 of 1 024 49.9 / 26.4).  Few
-// columns are ranked without a search for a bound first (20 000 rows, insertions / search / neither: 1 column 6.6 / 14.8 / 4.2, 9, top-16 11.5 /
-// 16.3 / 5.5, 31 25.4 / 19.5 / 11.0; 16 rows of 63, top-64 5.9 / 6.6 / 5.0).
+// columns are ranked without a search for a bound first (20 000 rows, insertions / search / neither: 1 column 6.6 / 14.8 / 3.4, 9, top-16 11.5 /
+// 16.3 / 5.5, 13 14.1 / 16.9 / 6.4; 16 rows of 63, top-64 5.9 / 6.6 / 5.0).
 template <int SEG>
 __global__ __launch_bounds__(256) void topk_rows_kernel(const float* __restrict__ scores, int32_t* __restrict__ idx,
                                                         int64_t rows, int cols_all, int64_t row_stride, int K, int vec_ok,

@@ -129,9 +129,9 @@ def compressed_attn_topk(q: torch.Tensor, k: torch.Tensor, v: Optional[torch.Ten
     head_dim 64, top-k a power of two up to 32): the scores never leave the chip.  Otherwise the scores
     go through HBM (attention kernel, then the row-wise top-k kernel).
 
-    ``v=None`` asks for the indices alone (``o`` is returned as ``None``; fused selection only): the
-    attention output and the indices come from two different kernels, and a caller with two streams runs
-    them side by side, see :func:`sparse_global_attention`.
+    ``v=None`` asks for the indices alone (``o`` is returned as ``None``; fused selection only).  Short lists of
+    keys (``s3r_topk_in_lds``) give attention output and indices in one launch; beyond, they come from two
+    different kernels, and a caller with two streams runs them side by side, see :func:`sparse_global_attention`.
 
     ``out``: a ``[B,H,Lq,D]`` tensor (or view, any strides on the first three dimensions, e.g. the
     ``permute(0, 2, 1, 3)`` of a ``[B,Lq,H,D]`` buffer) that receives the attention output instead of a fresh one.
@@ -755,14 +755,16 @@ def gate(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) ->
 
 def select_attn_merge(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, idx: torch.Tensor, o_cmp: torch.Tensor,
                       gate: torch.Tensor, block: int, softmax_scale: Optional[float] = None) -> Optional[torch.Tensor]:
-    """``select_attn`` with ``gated_merge`` in its epilogue -> ``[B,N,H*D]``; bit-identical to the two calls, without the
-    round trip of the selection output through memory.  Returns ``None`` for fp32 and when the library has no fused kernel for
-    the shape (the caller then runs the two operators)."""
+    """``select_attn`` with ``gated_merge`` in its epilogue -> ``[B,N,H*D]``, without the round trip of the selection output
+    through memory: the bits of the two calls for 16-token blocks; for 64-token blocks (and 128, 256) the expression is evaluated
+    in fp32 and rounded once.  Returns ``None`` when the library has no fused kernel for the shape (the caller then runs the two
+    operators), and for fp32, which it has always left to them: programs and tests rely on that answer, and the bits are the
+    same (the whole path and the layer, which run either way themselves, use the kernel's fp32 merge)."""
     return _select_attn_merge(q, k, v, idx, o_cmp, gate, block, softmax_scale, (torch.bfloat16, torch.float16))
 
 
 def _select_attn_merge(q, k, v, idx, o_cmp, gate, block, softmax_scale=None, dtypes=(torch.bfloat16, torch.float16, torch.float32)):
-    """:func:`select_attn_merge` in fp32 too (the bits of the two operators)."""
+    """:func:`select_attn_merge` in fp32 too (the bits of the two operators), for this package's own paths."""
     _need_device(q, k, v, idx, o_cmp, gate)
     _forward_only(q, k, v, o_cmp, gate)
     q, k, v, idx, o_cmp, gate = (_last_contig(t) for t in (q, k, v, idx, o_cmp, gate))
@@ -1106,8 +1108,9 @@ def _two_kernel_compressed(q: torch.Tensor, topk: int, block: int = 1) -> bool:
 # are one launch with the attention.  The two-sweep kernel pays from 19 456 pooled rows (B * H * blocks) on; long lists over few heads, whose
 # chain is long and leaves most of the chip idle, from 8192.  Operators, us per call, two streams / one, 16 heads: 16-token blocks, top-32,
 # 1 512 pooled tokens 185 / 188, 2 016 235 / 237, 3 780 438 / 441; 64-token blocks, top-16, 1 302 480 / 482, 1 952 701 / 702, 2 603 938 / 953, 4 164
-# 1 532 / 1 551.  Layers: 2 520 blocks of 16 798 / 792, 3 780 1 193 / 1 165, 5 040 1 711 / 1 665, 6 489 2 368 / 2 415, 12 600 5 410 / 5 630; 4 164 of 64
-# 4 295 / 4 360; 3 x 16 heads of 1 008 798 / 812 (up to 512 workgroups of 64 pooled rows: see attention_layer).
+# 1 532 / 1 551.  Layers, up to 512 workgroups of 64 pooled rows: see attention_layer; beyond, 6 489 blocks of 16 2 368 / 2 415, 12 600
+# 5 410 / 5 630, 4 164 of 64 4 295 / 4 360, 3 x 16 heads of 1 008 of 16 798 / 812.  The line is too early for layers of 2 049 to some 5 500
+# blocks of 16 (16 heads), which would be 1 to 3 % faster in one call: 2 520 798 / 792, 3 780 1 193 / 1 165, 5 040 1 711 / 1 665.
 SIDE_STREAM_ROWS = 16 * 1216
 SIDE_STREAM_ROWS_OF_LONG_LISTS = 8192
 
@@ -1151,15 +1154,15 @@ def sparse_global_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g
                             fuse_merge: bool = True, overlap: Optional[bool] = None, timeline: Optional[dict] = None):
     """The whole path on post-norm/RoPE q, k, v ``[B,H,N,D]`` and gate ``[B,H,N,2]``:
     pool -> compressed attention + top-k -> selection attention -> gated merge -> ``[B,N,H*D]``.
-    The merge runs in the selection kernel's epilogue where the library offers it (same bits either way);
+    The merge runs in the selection kernel's epilogue where the library offers it (same bits either way but for 64-token
+    blocks of 16-bit types, which are then rounded once, see :func:`select_attn_merge`);
     ``return_parts`` needs the selection output and therefore runs the two operators separately.
 
     ``overlap`` (default: where :func:`_side_stream_pays` says so; True: wherever it applies): the indices need pooled q and k only, the compressed attention output
-    is not read before the merge.  Where the two come from different kernels (no score buffer), the index kernel runs
-    on a second stream next to the pooling of v and the compressed attention (same kernels, same results; only the
-    schedule differs).  The index kernel alone leaves most of the chip idle below a few thousand pooled tokens (one
-    workgroup per 128 pooled rows and head); measured at 266 496 tokens: 0.51 against 0.55 ms for everything in front
-    of the selection kernel.  ``overlap=False`` runs the kernels one after the other on the calling stream.
+    is not read before the merge.  Where the two come from different kernels (no score buffer, more keys than one launch
+    takes for both: :func:`_two_kernel_compressed`), the index kernel runs on a second stream next to the pooling of v and the
+    compressed attention (same kernels, same results; only the schedule differs).  Both sides measured: at
+    ``SIDE_STREAM_ROWS``.  ``overlap=False`` runs the kernels one after the other on the calling stream.
 
     ``timeline``: a dict that receives timing events of the calling stream under "start", "pooled" (sequential
     schedule only), "select" (everything before the selection kernel is done) and "end".

@@ -301,7 +301,7 @@ def test_selection_backward_with_blocks_of_128_and_256_tokens(n, block, kk):
 
 def test_caller_built_lists_that_are_not_ascending_are_refused_on_request():
     """ops.attn_bwd(check_lists=True): lists from key_block_lists pass; the same lists with one group reversed raise
-    (without the check the 16-token dK/dV kernel would skip entries and return incomplete gradients silently)."""
+    (without the check the kernels would add up in that order, with other roundings)."""
     import pytest as _pytest
     from speed3r_amd.sparse_attn import ops
     g = torch.Generator().manual_seed(3)

@@ -1,7 +1,6 @@
-"""The order the 16-token dK/dV kernel requires of caller-built key-centric lists, and the host-side check of it
-(``ops.key_lists_ascending``, used by ``ops.attn_bwd(check_lists=True)`` / ``S3R_CHECK_LISTS=1``).  The kernel merges
-the lists of four neighbouring key blocks a window at a time and treats the entries below a threshold as a prefix of
-each list: a list that is not ascending makes it skip entries, and dk / dv come out incomplete without any error."""
+"""The order of key-centric lists that ``ops.key_block_lists`` builds and ``ops.attn_bwd`` documents for caller-built ones, and the host-side
+check of it (``ops.key_lists_ascending``, used by ``ops.attn_bwd(check_lists=True)`` / ``S3R_CHECK_LISTS=1``).  The dK/dV kernels add up
+in the order of a list: another order names the same query blocks and gives other roundings."""
 import torch
 
 from speed3r_amd.sparse_attn.ops import key_lists_ascending
