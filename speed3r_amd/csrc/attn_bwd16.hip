@@ -14,7 +14,7 @@
 // the step after next into the same buffers and computes meanwhile; nothing else is pipelined, the other waves of the
 // SIMD fill the gaps.
 // Bound: the address unit on the way from the vector cache into the LDS.  Counters, layer features, 2 x 12 096 tokens, 16 heads, top-32,
-// dQ / dK/dV: that unit busy 81 / 74 %, vector port 38 / 29 %, matrix cores 26 / 19 %, LDS reads 21 / 23 %, 90 / 83 % of the requests
+// dQ / dK/dV: that unit busy 81 / 74 %, vector port 38 / 28 %, matrix cores 26 / 19 %, LDS reads 21 / 23 %, 90 / 83 % of the requests
 // served by the L2.
 // us, 16 heads, top-32, before / now: layer features, 24 192 tokens: dQ 304 / 141, dK/dV 504 / 234; 4 032 tokens 74 / 34 and
 // 115 / 62; video (lists of neighbours that agree), 96 768 tokens: 577 / 467 and 1 317 / 863, 24 192: 160 / 113 and 381 / 229.

@@ -10,7 +10,7 @@
 // after next into the same slot and computes meanwhile; the other waves of the SIMD fill the gaps.  One wave per workgroup
 // (unions differ in size, a workgroup holds its slots until its slowest wave ends).
 // Bound (counters, 16 heads, top-32, NQ 4): lists that share little (layer features, 2 x 12 096 tokens) the address unit on the way
-// from the vector cache into the LDS, busy 73 % (vector port 36 %, matrix cores 23 %); lists of neighbours that agree (video, 266 496
+// from the vector cache into the LDS, busy 73 % (vector port 36 %, matrix cores 22 %); lists of neighbours that agree (video, 266 496
 // tokens) the vector port, 67 %, beside it (65 %; matrix cores 40 %).
 // NQ, us, 16 heads (the kernel before this one, 32 x 32 products over unions of four lists / 1 / 2 / 4): layer features, top-32,
 // 2 016 tokens 40 / 18.5 / 26 / 41, 4 032 42 / 28 / 30.5 / 45, 8 064 63 / 52 / 50 / 58, 16 128 111 / 97 / 86 / 105, 24 192 152 / 136 / 120 /
