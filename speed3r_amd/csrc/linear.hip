@@ -87,20 +87,13 @@ __global__ __launch_bounds__(256, WPS) void linear_kernel(LinearParams p) {
 #pragma unroll
   for (int i = 0; i < Tl::NL; i++) tl.move(lx1, lw1, kb, i);
   tl.begin(lx0, lw0);
+  bool fresh = true;
   for (;;) {
     uint2 cb[T];  // this tile's bias (nb moves on to the next tile's)
 #pragma unroll
     for (int c = 0; c < T; c++) cb[c] = nb[c];
-    tl.clear();
-    tl.before_products();
-    int left = p.K >> 6;  // even
-    do {
-      advance();
-      tl.step(lx0, lw0, lx1, lw1, kb);
-      advance();
-      tl.step(lx1, lw1, lx0, lw0, kb);
-      left -= 2;
-    } while (left > 0);
+    tl.template sweep<T * (16 * 2 * T / 64)>(lx0, lw0, lx1, lw1, p.K >> 6, fresh, kb, advance);
+    fresh = false;
     tl.after_products();
 
     // A lane holds 4 channels of a token in each tile; 16 tokens at a time go through LDS so that consecutive lanes store

@@ -36,12 +36,17 @@ __device__ __forceinline__ void store16_if(void* base, uint32_t bytes, uint32_t 
 
 // Accumulators in the AGPR half of the register file where they fill it (with two waves per SIMD the compiler would split
 // the file in halves for 64 of them).
-template <typename E, bool AGPR> __device__ __forceinline__ void mma_acc(typename Mma<E>::V8 a, typename Mma<E>::V8 b, f32x4& c) {
+template <typename E, bool AGPR, bool FIRST = false> __device__ __forceinline__ void mma_acc(typename Mma<E>::V8 a, typename Mma<E>::V8 b, f32x4& c) {
+  // (FIRST: an operand all the same, so that a tile's first products take the registers of the ones that follow)
   if constexpr (std::is_same<E, bf16_t>::value) {
-    if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    if constexpr (AGPR && FIRST) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "+a"(c) : "v"(a), "v"(b));
+    else if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    else if constexpr (FIRST) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "+v"(c) : "v"(a), "v"(b));
     else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
   } else {
-    if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    if constexpr (AGPR && FIRST) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "+a"(c) : "v"(a), "v"(b));
+    else if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    else if constexpr (FIRST) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "+v"(c) : "v"(a), "v"(b));
     else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
   }
 }
@@ -141,18 +146,24 @@ template <typename E, int TT, int TC> struct Tile {
     for (int r = 0; r < NL; r++) read(P, x0, w0, 0, r);
   }
   // One step on the buffer (lx, lw), whose first half is in P; leaves the first half of the other buffer (ox, ow) in P and
-  // the step at kb requested into (lx, lw).
-  template <typename P8> __device__ __forceinline__ void step(P8* lx, P8* lw, P8* ox, P8* ow, int kb) {
+  // the step at kb requested into (lx, lw).  A tile's first step starts its sums (FIRST) instead of adding to cleared ones.
+  template <bool FIRST, typename P8> __device__ __forceinline__ void first_half(P8* lx, P8* lw) {
 #pragma unroll
     for (int j = 0; j < NM; j++) {
 #pragma unroll
       for (int r = 0; r < NL; r++)
         if (r * kRead1 / 16 == j) read(Q, lx, lw, 1, r);
-      mma_acc<E, kAgpr>(P.w[j / TT], P.x[j % TT], acc[j / TT][j % TT]);
+      mma_acc<E, kAgpr, FIRST>(P.w[j / TT], P.x[j % TT], acc[j / TT][j % TT]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    // the buffer's last reads are in registers and the other buffer's transfers have landed, in every wave
-    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+  }
+  // the buffer's last reads are in registers and the other buffer's transfers have landed, in every wave; LEFT: what the wave has
+  // requested or stored behind those transfers may still be under way
+  template <int LEFT = 0> __device__ __forceinline__ void turn() {
+    static_assert(LEFT < 64, "what the counter holds");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (LEFT & 15) | ((LEFT >> 4) << 14));  // vmcnt(LEFT) lgkmcnt(0)
+  }
+  template <typename P8> __device__ __forceinline__ void second_half(P8* lx, P8* lw, P8* ox, P8* ow, int kb) {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -162,24 +173,44 @@ template <typename E, int TT, int TC> struct Tile {
         if (r * kMove2 / 16 == j) move(lx, lw, kb, r);
         if (r * kRead2 / 16 + kRead2At == j) read(P, ox, ow, 0, r);
       }
-      mma_acc<E, kAgpr>(Q.w[j / TT], Q.x[j % TT], acc[j / TT][j % TT]);
+      mma_acc<E, kAgpr, false>(Q.w[j / TT], Q.x[j % TT], acc[j / TT][j % TT]);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  __device__ __forceinline__ void clear() {
+  // A tile: its K / 64 steps (an even number), two at a time, `advance` in front of each of them.  STORES: of the tile before, at most; they
+  // were issued behind the transfers that the first step waits for (`fresh`: there is no such tile).
+  template <int STORES, typename P8, typename F> __device__ __forceinline__ void sweep(P8* x0, P8* w0, P8* x1, P8* w1, int steps, bool fresh, const int& kb, F&& advance) {
+    start();
+    advance();
+    first_half<true>(x0, w0);
+    if (fresh) turn<0>();
+    else turn<STORES>();
+    second_half(x0, w0, x1, w1, kb);
+    advance();
+    step(x1, w1, x0, w0, kb);
+    for (steps -= 2; steps > 0; steps -= 2) {
+      advance();
+      step(x0, w0, x1, w1, kb);
+      advance();
+      step(x1, w1, x0, w0, kb);
+    }
+  }
+  template <typename P8> __device__ __forceinline__ void step(P8* lx, P8* lw, P8* ox, P8* ow, int kb) {
+    first_half<false>(lx, lw);
+    turn<0>();
+    second_half(lx, lw, ox, ow, kb);
+  }
+  __device__ __forceinline__ void start() {  // (whatever the registers hold: a tile's first products do not read it)
 #pragma unroll
     for (int c = 0; c < TC; c++)
 #pragma unroll
-      for (int t = 0; t < TT; t++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc[c][t][i] = 0.f;
+      for (int t = 0; t < TT; t++) {
+        if constexpr (kAgpr) asm volatile("" : "=a"(acc[c][t]));
+        else asm volatile("" : "=v"(acc[c][t]));
+      }
   }
-  // Around the products written out the compiler knows of no hazards: accumulators written by vector instructions are given
-  // time before the first product reads them, the last products time before vector instructions read theirs.
-  __device__ __forceinline__ void before_products() {
-    touch();
-    asm volatile("s_nop 7");
-  }
+  // Around the products written out the compiler knows of no hazards: the last products are given time before vector
+  // instructions read their accumulators.  (The first ones of a tile take no accumulators, and write what has been read.)
   __device__ __forceinline__ void after_products() {
     asm volatile("s_nop 15\n s_nop 15");
     touch();

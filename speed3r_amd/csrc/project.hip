@@ -144,17 +144,9 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
   for (int i = 0; i < Tl::NL; i++) tl.move(lx1, lw1, kb, i);
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the tables, and what has been handed out
   tl.begin(lx0, lw0);
+  bool fresh = true;
   for (;; par ^= 1) {
-    tl.clear();
-    tl.before_products();
-    int left = p.K >> 6;  // even
-    do {
-      advance();
-      tl.step(lx0, lw0, lx1, lw1, kb);
-      advance();
-      tl.step(lx1, lw1, lx0, lw0, kb);
-      left -= 2;
-    } while (left > 0);
+    tl.template sweep<T * HD * 2>(lx0, lw0, lx1, lw1, p.K >> 6, fresh, kb, advance);
     tl.after_products();
 
     // ---- epilogue ----
@@ -379,6 +371,7 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
     };
     if (which < 2) finish(std::true_type{});
     else if (which == 2) finish(std::false_type{});
+    fresh = which > 2;  // (a wave beyond the last column has stored nothing)
     walk.at += walk.slots;
     if (walk.at >= walk.count) break;
     walk.locate(walk.at, m, n);
@@ -403,13 +396,9 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
 #pragma unroll
     for (int t = 0; t < Gt::NL; t++) gt.move(lx1, lw1, 128, t);
     gt.begin(lx0, lw0);
-    gt.clear();
-    gt.before_products();
     const int last = p.K * 2 - 128;
-    for (int kb = 256; kb < p.K * 2 + 256; kb += 256) {  // (beyond the end the last step is requested again)
-      gt.step(lx0, lw0, lx1, lw1, kb < last ? kb : last);
-      gt.step(lx1, lw1, lx0, lw0, kb + 128 < last ? kb + 128 : last);
-    }
+    int at = 128;
+    gt.template sweep<0>(lx0, lw0, lx1, lw1, p.K >> 6, true, at, [&]() { at = at + 128 < last ? at + 128 : last; });  // (beyond the end the last step is requested again)
     gt.after_products();
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the requests beyond the end have landed
     const int o = gt.wn * 16 + 4 * gt.g4;
