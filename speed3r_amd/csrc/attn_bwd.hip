@@ -25,7 +25,7 @@
 //     dV^T += dO^T P and dK^T += Q^T dS read their A operands transposed from the same buffers.
 // Query rows beyond Lq have lse = +inf (P = 0), keys beyond Lk are masked (P = 0); rows past the end of a tensor are
 // never read (transfers re-read the last valid row).
-#include "select_common.h"
+#include "block16.h"
 #include "attn_bwd.h"
 
 namespace s3r {
@@ -134,53 +134,6 @@ __device__ __forceinline__ typename Mma<E>::V8 read_transposed_frag(const char* 
   return as_v8<E>(f);
 }
 
-// The same reads written by hand, each group one asm statement that ends with its own wait: the compiler neither sees an
-// LDS access nor adds a wait of its own, and no register of an outstanding read is left to the register allocator.  A
-// compiler-visible LDS read that follows direct transfers into LDS makes the compiler wait for every transfer that it
-// cannot tell apart from the buffer being read, here also those of the NEXT half tile, which have just been issued.
-// Row fragments of two half tiles (K and V, or Q and dO): lane = row c, k-step ks: head_dim chunk 2ks + hh.
-__device__ __forceinline__ void read_rows2_sync(const char* half_a, const char* half_b, int c, int hh, u32x4 (&a)[4], u32x4 (&b)[4]) {
-  // one address per tile: row and the chunk of k-step 0; the k-step flips chunk bits 1..2 (tiles are 1 KB aligned).
-  // The empty asm keeps the eight addresses from being computed ahead of the loop and held in registers.
-  const uint32_t off = (uint32_t)(c * 128 + ((hh ^ k_swizzle(c)) << 4));
-  uint32_t a0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)half_a + off;
-  uint32_t b0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)half_b + off;
-  asm volatile("" : "+v"(a0), "+v"(b0));
-  asm volatile(
-      "ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\tds_read_b128 %2, %10\n\tds_read_b128 %3, %11\n\t"
-      "ds_read_b128 %4, %12\n\tds_read_b128 %5, %13\n\tds_read_b128 %6, %14\n\tds_read_b128 %7, %15\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3])
-      : "v"(a0), "v"(a0 ^ 32u), "v"(a0 ^ 64u), "v"(a0 ^ 96u), "v"(b0), "v"(b0 ^ 32u), "v"(b0 ^ 64u), "v"(b0 ^ 96u)
-      : "memory");
-}
-// Transposed fragments of one half tile: dst[jj][dt][rows 0-7 | 8-15 of the 16-row group jj].
-__device__ __forceinline__ void read_transposed_sync(const char* half, int tr_off, u32x2 (&dst)[2][2][2]) {
-  uint32_t t0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)half + (uint32_t)tr_off;
-  asm volatile("" : "+v"(t0));
-  const uint32_t t8 = t0 ^ (uint32_t)(k_swizzle(8) << 4);  // rows 8 further down: chunk map ^ k_swizzle(8)
-  asm volatile(
-      "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %10 offset:1024\n\t"
-      "ds_read_b64_tr_b16 %2, %9\n\tds_read_b64_tr_b16 %3, %11 offset:1024\n\t"
-      "ds_read_b64_tr_b16 %4, %8 offset:2048\n\tds_read_b64_tr_b16 %5, %10 offset:3072\n\t"
-      "ds_read_b64_tr_b16 %6, %9 offset:2048\n\tds_read_b64_tr_b16 %7, %11 offset:3072\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(dst[0][0][0]), "=&v"(dst[0][0][1]), "=&v"(dst[0][1][0]), "=&v"(dst[0][1][1]), "=&v"(dst[1][0][0]), "=&v"(dst[1][0][1]),
-        "=&v"(dst[1][1][0]), "=&v"(dst[1][1][1])
-      : "v"(t0), "v"(t0 ^ 64u), "v"(t8), "v"(t8 ^ 64u)
-      : "memory");
-}
-template <typename E> __device__ __forceinline__ typename Mma<E>::V8 frag_of(u32x4 w) {
-  Frag f;
-  f.u = make_uint4(w[0], w[1], w[2], w[3]);
-  return as_v8<E>(f);
-}
-template <typename E> __device__ __forceinline__ typename Mma<E>::V8 frag_of(u32x2 lo, u32x2 hi) {
-  Frag f;
-  f.u = make_uint4(lo[0], lo[1], hi[0], hi[1]);
-  return as_v8<E>(f);
-}
-
 __device__ __forceinline__ int tr_offset(int lane) {
   const int hh = lane >> 5;
   const int i16 = lane & 15;
@@ -216,9 +169,24 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[2], E* rowptr, bo
 }
 
 // ---- dQ ----------------------------------------------------------------------------------------------------------
+// One wave per 64-row query block.  The unit of its pipeline is 32 keys x 16 queries, twelve products of 16 x 16; in the phase of unit u
+// the wave issues, one per slot,
+//     dQ^T of unit u-1 (4),  S^T and dP^T of unit u+1 (8)
+// and between them the vector work of unit u, cut into pairs of scores (two fused multiply-adds, two exponentials, two multiplications, one
+// conversion over three slots), so that nothing waits for a product or an exponential of its own slot.  The wave's key tile is read in halves of 32 keys:
+// row fragments of K and V and transposed fragments of K, each requested from LDS eight products ahead of its first use, into the registers
+// that the half before has just left.
+//   * dS = P (dP - delta) with the softmax scale inside P: P = exp2(scale log2(e) S - lse log2(e) + log2(scale)), and the accumulator
+//     of dP starts at -delta (a tuple per 16 queries that stays in registers): per score one fused multiply-add, one exponential, one
+//     multiplication and half a conversion, against two multiply-adds, one exponential, one multiplication and half a conversion before.
+//   * 16 x 16 x 32 products: a lane's tuple is four scores, so a unit is small enough to be pipelined in registers (32 x 32 products
+//     with both halves of the queries in flight did not fit, and the compiler's order left matrix cores and vector unit taking turns).
+// us, before / now: 266 496 tokens x 16 heads, top-16 1 902 / 1 531 (1.1 PFLOP/s: matrix cores and vector unit have the same work, 1 536
+// cycles each per tile, and the chip runs below 2 GHz under it), dense over 4 164 tokens 212 / 161.
 template <typename E, bool DENSE>
 __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, int nqg, int total_wg) {
   typedef typename Mma<E>::V8 V8;
+  typedef typename Mma<E>::V2 V2;
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[4 * kHalfBytes];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k1[4 * kHalfBytes];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_v0[4 * kHalfBytes];
@@ -226,8 +194,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int hh = lane >> 5;
-  const int c = lane & 31;
+  const int g = lane >> 4;
+  const int c = lane & 15;
 
   const int w = blockIdx.x;  // workgroup w -> work item: each XCD walks a contiguous range of query blocks of one head
   const int xcd = w & 7, slot = w >> 3;
@@ -249,152 +217,253 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
   const float* lsep = p.lse + ((int64_t)b * p.H + h) * Lq;
   const float* dlp = p.delta + ((int64_t)b * p.H + h) * Lq;
 
-  char* k_buf[2] = {reinterpret_cast<char*>(lds_k0) + wave * kHalfBytes, reinterpret_cast<char*>(lds_k1) + wave * kHalfBytes};
-  char* v_buf[2] = {reinterpret_cast<char*>(lds_v0) + wave * kHalfBytes, reinterpret_cast<char*>(lds_v1) + wave * kHalfBytes};
-
-  // B operands Q and dO (lane = query row, head_dim chunk hh + 2 ks), per-query lse (base 2) and delta
-  V8 bq[2][4], bg[2][4];
-  float lse2[2], dlts[2];  // log-sum-exp in base 2, delta times the softmax scale
+  // the list first: it heads the longest chain of the start
+  int32_t my_idx = -1;
+  if constexpr (!DENSE) {
+    const int32_t* idx_row = p.idx + (int64_t)b * p.sib + (int64_t)h * p.sih + (int64_t)qb * p.sim;
+    if (lane < p.K) my_idx = idx_row[lane];
+  }
+  // B operands Q and dO: lane = query 16 qt + c, head dimensions 32 ks + 8 g ..
+  V8 bq[4][2], bg[4][2];
+  float nl[4];    // log2(scale) - lse log2(e)
+  f32x4 nd[4];    // -delta, what the products of dP^T start from
+  const float log2_scale = __builtin_amdgcn_logf(p.scale);
 #pragma unroll
-  for (int qt = 0; qt < 2; qt++) {
-    const int64_t row = q0 + qt * 32 + c;
+  for (int qt = 0; qt < 4; qt++) {
+    const int64_t row = q0 + qt * 16 + c;
     const bool live = row < Lq;
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++) {
-      Frag f, g;
+    for (int ks = 0; ks < 2; ks++) {
+      Frag f, d;
       f.u = make_uint4(0, 0, 0, 0);
-      g.u = make_uint4(0, 0, 0, 0);
+      d.u = make_uint4(0, 0, 0, 0);
       if (live) {
-        f.u = *reinterpret_cast<const uint4*>(qp + row * p.sqm + ks * 16 + hh * 8);
-        g.u = *reinterpret_cast<const uint4*>(gp + row * p.sgm + ks * 16 + hh * 8);
+        f.u = *reinterpret_cast<const uint4*>(qp + row * p.sqm + ks * 32 + g * 8);
+        d.u = *reinterpret_cast<const uint4*>(gp + row * p.sgm + ks * 32 + g * 8);
       }
       bq[qt][ks] = as_v8<E>(f);
-      bg[qt][ks] = as_v8<E>(g);
+      bg[qt][ks] = as_v8<E>(d);
     }
-    lse2[qt] = live ? lsep[row] * kLog2e : INFINITY;
-    dlts[qt] = live ? dlp[row] * p.scale : 0.f;
+    nl[qt] = live ? fmaf(lsep[row], -kLog2e, log2_scale) : -INFINITY;
+    const float m = live ? -dlp[row] : 0.f;
+    nd[qt] = (f32x4){m, m, m, m};
   }
-  f32x16 dqt[2][2];  // dQ^T accumulators [qt][dt]: lane = query, registers = head_dim
+  f32x4 dq[4][4];  // dQ^T [qt][dt]: lane = query, registers = head dimensions 16 dt + 4 g ..
 #pragma unroll
-  for (int qt = 0; qt < 2; qt++)
+  for (int qt = 0; qt < 4; qt++)
 #pragma unroll
-    for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) dqt[qt][dt][r] = 0.f;
+    for (int dt = 0; dt < 4; dt++) dq[qt][dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  // key tiles of this query block
-  int32_t my_idx = -1;
+  // key tiles of this query block: full ones go through the pipeline, occurrences of the ragged last one come after it
+  const int32_t ragged_blk = (Lk & 63) ? (int32_t)(Lk >> 6) : -1;
   uint64_t todo = 0;
-  int ntiles;
+  int n_full, n_ragged;
   int dense_next = 0;
   if constexpr (DENSE) {
-    ntiles = (int)((Lk + 63) >> 6);
+    n_full = (int)(Lk >> 6);
+    n_ragged = (Lk & 63) ? 1 : 0;
   } else {
-    const int32_t* idx_row = p.idx + (int64_t)b * p.sib + (int64_t)h * p.sih + (int64_t)qb * p.sim;
-    my_idx = lane < p.K ? idx_row[lane] : -1;
-    todo = __ballot(my_idx >= 0 && (int64_t)my_idx * 64 < Lk);
-    ntiles = __popcll(todo);
+    const bool valid = my_idx >= 0 && (int64_t)my_idx * 64 < Lk;
+    todo = __ballot(valid && my_idx != ragged_blk);
+    n_ragged = __popcll(__ballot(valid && my_idx == ragged_blk));
+    n_full = __popcll(todo);
   }
-  auto pop = [&]() -> int64_t {  // start row of the next tile (callers pop exactly ntiles times)
+  int64_t last_start = 0;
+  auto pop_or_last = [&]() -> int64_t {  // first row of the next full tile, or the last one again
     if constexpr (DENSE) {
-      return (int64_t)(dense_next++) * 64;
+      last_start = (int64_t)(dense_next < n_full ? dense_next : n_full - 1) * 64;
+      dense_next++;
     } else {
-      const int t = __ffsll((unsigned long long)todo) - 1;
+      const bool any = todo != 0;
+      const int t = any ? __ffsll((unsigned long long)todo) - 1 : 0;
+      const int64_t s = (int64_t)__builtin_amdgcn_readlane(my_idx, t) * 64;
       todo &= todo - 1;
-      return (int64_t)__builtin_amdgcn_readlane(my_idx, t) * 64;
+      last_start = any ? s : last_start;
     }
+    return last_start;
   };
 
-  const float scale = p.scale;
-  const float sl2 = scale * kLog2e;
+  const float sl2 = p.scale * kLog2e;
   const uint32_t krow = (uint32_t)p.skn * (uint32_t)sizeof(E), vrow = (uint32_t)p.svn * (uint32_t)sizeof(E);
-  const int tr_off = tr_offset(lane);
-
-  auto fetch = [&](int64_t start, auto hf, int buf) {  // half HF of the tile at `start` -> buffers `buf`
-    constexpr int HF = decltype(hf)::value;
-    const int last = (int)((Lk - start < 64 ? Lk - start : 64) - 1);
-    dma_rows<E, true>(kp + start * p.skn, krow, 32 * HF, last, k_buf[buf], lane, 0, 4);
-    dma_rows<E, false>(vp + start * p.svn, vrow, 32 * HF, last, v_buf[buf], lane, 0, 4);
+  typedef __attribute__((address_space(3))) void* Lds;
+  // every buffer is named through one array: the compiler then knows that a read of one does not wait for transfers into another
+  auto k_buf = [&](auto hf) -> char* { return reinterpret_cast<char*>(decltype(hf)::value == 0 ? lds_k0 : lds_k1) + wave * kHalfBytes; };
+  auto v_buf = [&](auto hf) -> char* { return reinterpret_cast<char*>(decltype(hf)::value == 0 ? lds_v0 : lds_v1) + wave * kHalfBytes; };
+  // transfer i of a half tile moves its rows 8 i .. 8 i + 7 (chunk c of row r at c ^ swz(r), the same for all four)
+  const uint32_t chunk = (uint32_t)(((lane & 7) ^ b16x::swz(lane >> 3)) * 16);
+  const uint32_t k_voff = (uint32_t)(lane >> 3) * krow + chunk, v_voff = (uint32_t)(lane >> 3) * vrow + chunk;
+  auto dma_k = [&](auto hf, auto i_tag, int64_t start) {
+    constexpr int HF = decltype(hf)::value, i = decltype(i_tag)::value;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(kp + (start + 32 * HF) * p.skn), 0, 0x7fffffff, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (Lds)(k_buf(hf) + i * 1024), 16, k_voff, 8u * i * krow, 0, 0);
   };
-  auto compute = [&](int64_t start, auto hf, int buf) {
-    constexpr int HF = decltype(hf)::value;
-    const int nvalid = (int)(Lk - start < 64 ? Lk - start : 64);
-    const bool ragged = nvalid < 64;
-    V8 ak[4], av[4];
-    {
-      u32x4 kw[4], vw[4];
-      read_rows2_sync(k_buf[buf], v_buf[buf], c, hh, kw, vw);
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) {
-        ak[ks] = frag_of<E>(kw[ks]);
-        av[ks] = frag_of<E>(vw[ks]);
-      }
-    }
-    V8 ds[2][2];  // dS^T as B operand [qt][jj]
-    constexpr int QT0 = 0, QT1 = 2;
-#pragma unroll
-    for (int qt = QT0; qt < QT1; qt++) {
-      f32x16 st, dp;
-#pragma unroll
-      for (int r = 0; r < 16; r++) { st[r] = 0.f; dp[r] = 0.f; }
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) st = Mma<E>::mma(ak[ks], bq[qt][ks], st);
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) dp = Mma<E>::mma(av[ks], bg[qt][ks], dp);
-#pragma unroll
-      for (int r = 0; r < 16; r++) st[r] = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, -lse2[qt]));  // P^T
-      if (ragged) {  // keys beyond Lk carry no probability
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-          if (32 * HF + 4 * hh + 8 * (r >> 2) + (r & 3) >= nvalid) st[r] = 0.f;
-      }
-#pragma unroll
-      for (int r = 0; r < 16; r++) ds[qt][r >> 3][r & 7] = (E)(st[r] * fmaf(dp[r], scale, -dlts[qt]));  // scale * P * (dP - delta)
-    }
-    V8 kt[2][2];
-    {
-      u32x2 tw[2][2][2];
-      read_transposed_sync(k_buf[buf], tr_off, tw);
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++)
-#pragma unroll
-        for (int dt = 0; dt < 2; dt++) kt[jj][dt] = frag_of<E>(tw[jj][dt][0], tw[jj][dt][1]);
-    }
-#pragma unroll
-    for (int jj = 0; jj < 2; jj++)
-#pragma unroll
-      for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-        for (int qt = QT0; qt < QT1; qt++) dqt[qt][dt] = Mma<E>::mma(kt[jj][dt], ds[qt][jj], dqt[qt][dt]);
+  auto dma_v = [&](auto hf, auto i_tag, int64_t start) {
+    constexpr int HF = decltype(hf)::value, i = decltype(i_tag)::value;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(vp + (start + 32 * HF) * p.svn), 0, 0x7fffffff, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (Lds)(v_buf(hf) + i * 1024), 16, v_voff, 8u * i * vrow, 0, 0);
   };
-
-  if (ntiles > 0) {
-    int64_t cur = pop();
-    fetch(cur, H0{}, 0);
-    for (int t = 0; t < ntiles; t++) {
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads of buffer 1 (previous tile) are done
-      fetch(cur, H1{}, 1);
-      __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): half 0 has landed
-      compute(cur, H0{}, 0);
-      const bool more = t + 1 < ntiles;
-      const int64_t nxt = more ? pop() : cur;
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads of buffer 0 are done
-      if (more) {
-        fetch(nxt, H0{}, 0);
-        __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): half 1 has landed
-      } else {
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  const int row_off = c * 128 + ((g ^ b16x::swz(c)) << 4);
+  const int tr_row = 4 * g + (c >> 2);
+  const int tr_off = tr_row * 128 + ((((c & 3) >> 1) ^ b16x::swz(tr_row)) << 4) + (c & 1) * 8;
+  V8 ak[2][2], av[2][2];  // row fragments [16 keys][ks]
+  V8 kt[4];               // K^T [dt]: head dimension 16 dt + c, keys 4 g .. of either 16
+  auto read_rows16 = [&](const char* half, V8 (&dst)[2][2]) {
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        Frag f;
+        f.u = *reinterpret_cast<const uint4*>(half + t * 2048 + (row_off ^ (ks << 6)));
+        dst[t][ks] = as_v8<E>(f);
       }
-      compute(cur, H1{}, 1);
-      cur = nxt;
+  };
+  auto read_kt = [&](const char* half) {
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) {
+      const char* a = half + (tr_off ^ (dt << 5));
+      Frag f;
+      f.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(a));
+      f.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(a + 2048));
+      kt[dt] = as_v8<E>(f);
     }
+  };
+  f32x4 st[2][2], dp[2][2];  // S^T and dP^T [parity of the unit][16 keys]
+  V8 ds;                     // dS^T of the unit before
+  auto score = [&](auto i_tag, auto qt_tag) {  // product i of 8 of the scores of 16 queries
+    constexpr int i = decltype(i_tag)::value, QT = decltype(qt_tag)::value, t = i & 1, ks = (i >> 1) & 1, B = QT & 1;
+    if constexpr (i < 4) st[B][t] = b16x::mma16<E>(ak[t][ks], bq[QT][ks], ks ? st[B][t] : (f32x4){0.f, 0.f, 0.f, 0.f});
+    else dp[B][t] = b16x::mma16<E>(av[t][ks], bg[QT][ks], ks ? dp[B][t] : nd[QT]);
+  };
+  auto pair_of = [&](float a, float b2) -> uint32_t {
+    V2 v;
+    v[0] = (E)a;
+    v[1] = (E)b2;
+    return __builtin_bit_cast(uint32_t, v);
+  };
+  // Phase of unit (half HF of the tile, queries 16 QT ..).  Transfers: V of the next tile's half HF while QT = 0 (V's last reads of the buffer
+  // went into registers a unit ago), K of it while QT = 1 (behind the products that took kt), in this order, so that eight transfers are
+  // younger than what is read from the other half's buffers while QT = 2 and 3.
+  auto phase = [&](auto hf, auto qt_tag, int64_t next) {
+    constexpr int HF = decltype(hf)::value, QT = decltype(qt_tag)::value, B = QT & 1;
+    typedef std::integral_constant<int, HF ^ 1> HO;
+    typedef std::integral_constant<int, (QT + 1) & 3> NQ;
+    constexpr int PQ = (QT + 3) & 3;
+    float x0 = 0.f, x1 = 0.f, e0 = 0.f, e1 = 0.f;
+    u32x4 dn;
+    static_for<12>([&](auto j_tag) {
+      constexpr int j = decltype(j_tag)::value;
+      if constexpr (QT == 0 && j == 4) read_kt(k_buf(hf));
+      if constexpr (QT == 0 && j >= 6 && j < 10) dma_v(hf, std::integral_constant<int, (j - 6) & 3>{}, next);
+      if constexpr (QT == 1 && j >= 4 && j < 8) dma_k(hf, std::integral_constant<int, j & 3>{}, next);
+      if constexpr (QT == 2 && j == 8) {
+        __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): the other half of K and of V have landed
+        read_rows16(k_buf(HO{}), ak);
+      }
+      if constexpr (QT == 3 && j == 0) read_rows16(v_buf(HO{}), av);
+      if constexpr (j < 4) dq[PQ][j] = b16x::mma16<E>(kt[j], ds, dq[PQ][j]);
+      else score(std::integral_constant<int, (j + 8) % 12>{}, NQ{});
+      {
+        constexpr int pr = j / 3, s = j % 3, t = pr >> 1, r = 2 * (pr & 1);
+        if constexpr (s == 0) {
+          asm volatile("" : "+v"(st[B][t]));
+          x0 = fmaf(st[B][t][r], sl2, nl[QT]);
+          x1 = fmaf(st[B][t][r + 1], sl2, nl[QT]);
+          e0 = __builtin_amdgcn_exp2f(x0);
+          asm volatile("" : "+v"(x1), "+v"(e0));
+        } else if constexpr (s == 1) {
+          e1 = __builtin_amdgcn_exp2f(x1);
+          e0 *= dp[B][t][r];
+          asm volatile("" : "+v"(e0), "+v"(e1));
+        } else {
+          e1 *= dp[B][t][r + 1];
+          uint32_t wd = pair_of(e0, e1);
+          asm volatile("" : "+v"(wd));
+          dn[pr] = wd;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    ds = b16x::frag_of<E>(dn);
+  };
+  typedef std::integral_constant<int, 2> I2;
+  typedef std::integral_constant<int, 3> I3;
+
+  if (n_full > 0) {
+    int64_t cur = pop_or_last(), next = pop_or_last();
+    static_for<4>([&](auto i) { dma_v(H0{}, i, cur); });
+    static_for<4>([&](auto i) { dma_k(H0{}, i, cur); });
+    static_for<4>([&](auto i) { dma_v(H1{}, i, cur); });
+    static_for<4>([&](auto i) { dma_k(H1{}, i, cur); });
+    __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): half 0
+    read_rows16(k_buf(H0{}), ak);
+    read_rows16(v_buf(H0{}), av);
+    static_for<8>([&](auto i) { score(i, H0{}); });
+    const u32x4 zero = {0, 0, 0, 0};
+    ds = b16x::frag_of<E>(zero);  // nothing for the first phase to add
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) kt[dt] = b16x::frag_of<E>(zero);
+    for (int i = n_full; i > 0; i--) {  // past the last tile its rows are requested and scored again, for nothing
+      phase(H0{}, H0{}, next);
+      phase(H0{}, H1{}, next);
+      phase(H0{}, I2{}, next);
+      phase(H0{}, I3{}, next);
+      phase(H1{}, H0{}, next);
+      phase(H1{}, H1{}, next);
+      phase(H1{}, I2{}, next);
+      phase(H1{}, I3{}, next);
+      next = pop_or_last();
+    }
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) dq[3][dt] = b16x::mma16<E>(kt[dt], ds, dq[3][dt]);
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0): no transfer is on its way, nothing is read any more
+  }
+  for (; n_ragged > 0; n_ragged--) {  // the ragged last tile: rows beyond Lk re-read the last one and carry no probability
+    const int64_t start = (int64_t)ragged_blk * 64;
+    const int nvalid = (int)(Lk - start);
+    static_for<2>([&](auto hf) {
+      constexpr int HF = decltype(hf)::value;
+      const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)(kp + start * p.skn), 0, 0x7fffffff, 0x00020000);
+      const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)(vp + start * p.svn), 0, 0x7fffffff, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        int row = 32 * HF + 8 * i + (lane >> 3);
+        row = row < nvalid ? row : nvalid - 1;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (Lds)(k_buf(hf) + i * 1024), 16, (uint32_t)row * krow + chunk, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (Lds)(v_buf(hf) + i * 1024), 16, (uint32_t)row * vrow + chunk, 0, 0, 0);
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+      read_rows16(k_buf(hf), ak);
+      read_rows16(v_buf(hf), av);
+      read_kt(k_buf(hf));
+      static_for<4>([&](auto qt_tag) {
+        constexpr int QT = decltype(qt_tag)::value, B = QT & 1;
+        static_for<8>([&](auto i) { score(i, qt_tag); });
+        u32x4 dn;
+#pragma unroll
+        for (int pr = 0; pr < 4; pr++) {
+          const int t = pr >> 1, r = 2 * (pr & 1), key = 32 * HF + 16 * t + 4 * g + r;
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(st[B][t][r], sl2, nl[QT])), p1 = __builtin_amdgcn_exp2f(fmaf(st[B][t][r + 1], sl2, nl[QT]));
+          dn[pr] = pair_of((key < nvalid ? p0 : 0.f) * dp[B][t][r], (key + 1 < nvalid ? p1 : 0.f) * dp[B][t][r + 1]);
+        }
+        ds = b16x::frag_of<E>(dn);
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) dq[QT][dt] = b16x::mma16<E>(kt[dt], ds, dq[QT][dt]);
+      });
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): read before the next occurrence's transfers
+    });
   }
 
   E* dqp = (E*)p.dq + (int64_t)b * p.sdqb + (int64_t)h * p.sdqh;
 #pragma unroll
-  for (int qt = 0; qt < 2; qt++) {
-    const int64_t row = q0 + qt * 32 + c;
-    store_rows<E>(dqt[qt], dqp + row * p.sdqm, row < Lq, hh);
+  for (int qt = 0; qt < 4; qt++) {
+    const int64_t row = q0 + qt * 16 + c;
+    if (row < Lq) {
+#pragma unroll
+      for (int dt = 0; dt < 4; dt++) {
+        const u32x2 o = {pair_of(dq[qt][dt][0], dq[qt][dt][1]), pair_of(dq[qt][dt][2], dq[qt][dt][3])};
+        *reinterpret_cast<u32x2*>(dqp + row * p.sdqm + 16 * dt + 4 * g) = o;
+      }
+    }
   }
 }
 
