@@ -20,9 +20,8 @@
 //   * bwd_dkdv_kernel: one workgroup of two waves per 64-key block, each wave owns 32 keys (one KEY per lane:
 //     S = Q K^T, dP = dO V^T with K, V fragments in registers as B operands) and walks the query blocks that
 //     selected the key block (key-centric lists built by the host from the index tensor, reference :423-554).
-//     Q and dO tiles (64 queries) and the matching lse / delta values go global -> LDS, shared by the two waves,
-//     double buffered (the next tile's transfers fly during a whole tile of work), one barrier per tile;
-//     dV^T += dO^T P and dK^T += Q^T dS read their A operands transposed from the same buffers.
+//     Q and dO half tiles (32 queries) go global -> LDS, shared by the two waves, three half tiles ahead, one barrier
+//     per half tile; dV^T += dO^T P and dK^T += Q^T dS read their A operands transposed from the same buffers.
 // Query rows beyond Lq have lse = +inf (P = 0), keys beyond Lk are masked (P = 0); rows past the end of a tensor are
 // never read (transfers re-read the last valid row).
 #include "block16.h"
@@ -62,110 +61,6 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const E* __restrict__ o,
 #pragma unroll
   for (int off = 1; off < 8; off <<= 1) s += __shfl_xor(s, off);
   if (live && part == 0) delta[rr] = s;
-}
-
-// ---- shared pieces of the two MFMA kernels -----------------------------------------------------------------------
-// Transfer of rows [8*i0*.., ...) of a 32-row half tile: instruction i moves rows 8i .. 8i+7 (16 bytes per lane).
-// LDS chunk (row, c') holds head_dim chunk c' ^ k_swizzle(row) in every tile: 16-byte row reads and
-// ds_read_b64_tr_b16 reads both run without bank conflicts with it.  (VSW marks the tiles that are also read
-// transposed; the map is the same.)  Rows are clamped to `last` (relative to `base`'s row 0).
-template <typename E, bool VSW>
-__device__ __forceinline__ void dma_rows(const E* base, uint32_t rowbytes, int first_row, int last, char* lds_half, int lane, int i_begin, int i_end) {
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0x7fffffff, 0x00020000);
-  const int lr = lane >> 3;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if (i >= i_begin && i < i_end) {
-      const int ldsrow = 8 * i + lr;
-      int row = first_row + ldsrow;
-      row = row < last ? row : last;
-      const int chunk = (lane & 7) ^ k_swizzle(ldsrow);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds_half + i * 1024), 16,
-                                               (uint32_t)row * rowbytes + (uint32_t)(chunk * 16), 0, 0, 0);
-    }
-  }
-}
-
-// A operand from row reads of a half tile: lane = row c, k-step ks: head_dim chunk 2ks + hh.
-template <typename E, bool VSW>
-__device__ __forceinline__ void read_rows(const char* half, int c, int hh, typename Mma<E>::V8 (&dst)[4]) {
-  const int sw = k_swizzle(c);
-#pragma unroll
-  for (int ks = 0; ks < 4; ks++) {
-    Frag f;
-    f.u = *reinterpret_cast<const uint4*>(half + c * 128 + (((2 * ks + hh) ^ sw) << 4));
-    dst[ks] = as_v8<E>(f);
-  }
-}
-
-template <typename E, bool VSW>
-__device__ __forceinline__ typename Mma<E>::V8 read_row_frag(const char* half, int c, int hh, int ks) {
-  const int sw = k_swizzle(c);
-  Frag f;
-  f.u = *reinterpret_cast<const uint4*>(half + c * 128 + (((2 * ks + hh) ^ sw) << 4));
-  return as_v8<E>(f);
-}
-
-// A operand X^T from transposed reads of a half tile staged with VSW: fragment [jj][dt] holds, for head_dim row
-// dt*32 + c, the 8 rows 16jj + {4hh..4hh+3, 8+4hh..8+4hh+3} of the half: the order in which a 32x32 accumulator
-// with one column per lane hands over its registers 8jj .. 8jj+7.
-template <typename E>
-__device__ __forceinline__ void read_transposed(const char* half, int tr_off, typename Mma<E>::V8 (&dst)[2][2]) {
-#pragma unroll
-  for (int jj = 0; jj < 2; jj++)
-#pragma unroll
-    for (int dt = 0; dt < 2; dt++) {
-      const char* a0 = half + (tr_off ^ (dt * 64)) + (jj * 16) * 128;
-      const char* a8 = half + (tr_off ^ (dt * 64) ^ (k_swizzle(8) << 4)) + (jj * 16 + 8) * 128;  // rows 8 further down: chunk map ^ k_swizzle(8)
-      Frag f;
-      f.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(a0));
-      f.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(a8));
-      dst[jj][dt] = as_v8<E>(f);
-    }
-}
-
-template <typename E>
-__device__ __forceinline__ typename Mma<E>::V8 read_transposed_frag(const char* half, int tr_off, int jj, int dt) {
-  const char* a0 = half + (tr_off ^ (dt * 64)) + (jj * 16) * 128;
-  const char* a8 = half + (tr_off ^ (dt * 64) ^ (k_swizzle(8) << 4)) + (jj * 16 + 8) * 128;
-  Frag f;
-  f.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(a0));
-  f.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(a8));
-  return as_v8<E>(f);
-}
-
-__device__ __forceinline__ int tr_offset(int lane) {
-  const int hh = lane >> 5;
-  const int i16 = lane & 15;
-  const int tr_row = 4 * hh + (i16 >> 2);
-  const int tr_chunk = (((lane >> 4) & 1) * 2 + ((i16 & 3) >> 1)) ^ k_swizzle(tr_row);
-  return tr_row * 128 + tr_chunk * 16 + (i16 & 1) * 8;
-}
-
-// Store of a transposed 64 x 64 accumulator pair acc[dt] (lane = row of the output, registers = head_dim values
-// dt*32 + 8*(r/4) + 4*hh + r%4): one exchange with lane ^ 32 per packed word gives every lane 8 consecutive values.
-template <typename E>
-__device__ __forceinline__ void store_rows(const f32x16 (&acc)[2], E* rowptr, bool live, int hh) {
-#pragma unroll
-  for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-    for (int gp = 0; gp < 2; gp++) {
-      union { E e[8]; uint32_t w[4]; uint4 u; } pc;
-      union { E e[2]; uint32_t w; } t;
-#pragma unroll
-      for (int wi = 0; wi < 2; wi++) {
-        t.e[0] = (E)acc[dt][8 * gp + 2 * wi];
-        t.e[1] = (E)acc[dt][8 * gp + 2 * wi + 1];
-        const uint32_t a = t.w;
-        t.e[0] = (E)acc[dt][8 * gp + 4 + 2 * wi];
-        t.e[1] = (E)acc[dt][8 * gp + 4 + 2 * wi + 1];
-        const uint32_t bw = t.w;
-        const auto r = __builtin_amdgcn_permlane32_swap(a, bw, false, false);
-        pc.w[wi] = r[0];
-        pc.w[2 + wi] = r[1];
-      }
-      if (live) *reinterpret_cast<uint4*>(rowptr + dt * 32 + 8 * (2 * gp + hh)) = pc.u;
-    }
 }
 
 // ---- dQ ----------------------------------------------------------------------------------------------------------
@@ -223,8 +118,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
     const int32_t* idx_row = p.idx + (int64_t)b * p.sib + (int64_t)h * p.sih + (int64_t)qb * p.sim;
     if (lane < p.K) my_idx = idx_row[lane];
   }
-  // B operands Q and dO: lane = query 16 qt + c, head dimensions 32 ks + 8 g ..
-  V8 bq[4][2], bg[4][2];
   float nl[4];    // log2(scale) - lse log2(e)
   f32x4 nd[4];    // -delta, what the products of dP^T start from
   const float log2_scale = __builtin_amdgcn_logf(p.scale);
@@ -232,18 +125,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
   for (int qt = 0; qt < 4; qt++) {
     const int64_t row = q0 + qt * 16 + c;
     const bool live = row < Lq;
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      Frag f, d;
-      f.u = make_uint4(0, 0, 0, 0);
-      d.u = make_uint4(0, 0, 0, 0);
-      if (live) {
-        f.u = *reinterpret_cast<const uint4*>(qp + row * p.sqm + ks * 32 + g * 8);
-        d.u = *reinterpret_cast<const uint4*>(gp + row * p.sgm + ks * 32 + g * 8);
-      }
-      bq[qt][ks] = as_v8<E>(f);
-      bg[qt][ks] = as_v8<E>(d);
-    }
     nl[qt] = live ? fmaf(lsep[row], -kLog2e, log2_scale) : -INFINITY;
     const float m = live ? -dlp[row] : 0.f;
     nd[qt] = (f32x4){m, m, m, m};
@@ -305,6 +186,40 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
   const int row_off = c * 128 + ((g ^ b16x::swz(c)) << 4);
   const int tr_row = 4 * g + (c >> 2);
   const int tr_off = tr_row * 128 + ((((c & 3) >> 1) ^ b16x::swz(tr_row)) << 4) + (c & 1) * 8;
+  // B operands Q and dO: lane = query 16 qt + c, head dimensions 32 ks + 8 g ..; through the K and V buffers, whose map the transfers and
+  // the reads share (rows beyond Lq re-read the last one, never stored).  Loaded in the operands' own pattern, they took the address unit
+  // four times as long.
+  V8 bq[4][2], bg[4][2];
+  {
+    const uint32_t qrow = (uint32_t)p.sqm * (uint32_t)sizeof(E), grow = (uint32_t)p.sgm * (uint32_t)sizeof(E);
+    const int left = (int)(Lq - q0 < 64 ? Lq - q0 : 64) - 1;
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)(qp + q0 * p.sqm), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void*)(gp + q0 * p.sgm), 0, 0x7fffffff, 0x00020000);
+    static_for<2>([&](auto hf) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        int row = 32 * decltype(hf)::value + 8 * i + (lane >> 3);
+        row = row < left ? row : left;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (Lds)(k_buf(hf) + i * 1024), 16, (uint32_t)row * qrow + chunk, 0, 0, 2 /* nt: read once */);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (Lds)(v_buf(hf) + i * 1024), 16, (uint32_t)row * grow + chunk, 0, 0, 2);
+      }
+    });
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    static_for<4>([&](auto qt_tag) {
+      constexpr int QT = decltype(qt_tag)::value;
+      typedef std::integral_constant<int, (QT >> 1)> HF;
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        Frag f, d;
+        f.u = *reinterpret_cast<const uint4*>(k_buf(HF{}) + (QT & 1) * 2048 + (row_off ^ (ks << 6)));
+        d.u = *reinterpret_cast<const uint4*>(v_buf(HF{}) + (QT & 1) * 2048 + (row_off ^ (ks << 6)));
+        bq[QT][ks] = as_v8<E>(f);
+        bg[QT][ks] = as_v8<E>(d);
+      }
+    });
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): read before the first tile is requested
+    asm volatile("" ::: "memory");
+  }
   V8 ak[2][2], av[2][2];  // row fragments [16 keys][ks]
   V8 kt[4];               // K^T [dt]: head dimension 16 dt + c, keys 4 g .. of either 16
   auto read_rows16 = [&](const char* half, V8 (&dst)[2][2]) {
@@ -365,19 +280,18 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
       {
         constexpr int pr = j / 3, s = j % 3, t = pr >> 1, r = 2 * (pr & 1);
         if constexpr (s == 0) {
-          asm volatile("" : "+v"(st[B][t]));
           x0 = fmaf(st[B][t][r], sl2, nl[QT]);
           x1 = fmaf(st[B][t][r + 1], sl2, nl[QT]);
           e0 = __builtin_amdgcn_exp2f(x0);
-          asm volatile("" : "+v"(x1), "+v"(e0));
+          asm volatile("" ::"v"(x1), "v"(e0));
         } else if constexpr (s == 1) {
           e1 = __builtin_amdgcn_exp2f(x1);
           e0 *= dp[B][t][r];
-          asm volatile("" : "+v"(e0), "+v"(e1));
+          asm volatile("" ::"v"(e0), "v"(e1));
         } else {
           e1 *= dp[B][t][r + 1];
           uint32_t wd = pair_of(e0, e1);
-          asm volatile("" : "+v"(wd));
+          asm volatile("" ::"v"(wd));
           dn[pr] = wd;
         }
       }
@@ -468,330 +382,357 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
 }
 
 // ---- dK, dV ------------------------------------------------------------------------------------------------------
+// A workgroup of two waves per 64-key block, 32 keys a wave: K and V of its keys as B operands (32 registers), dK^T and dV^T (64) and the
+// fragments of 32 queries (64).  The unit of the pipeline is 32 queries x 16 keys: S and dP (8 products of 16 x 16 x 32), P and dS of
+// eight scores a lane, dV^T and dK^T (8).  In the phase of unit u a wave issues, one product per slot,
+//     dV^T and dK^T of unit u-1,  S and dP of unit u+1
+// and between them the vector work of unit u, a pair of scores over four slots.  Fragments are requested from LDS twelve products ahead,
+// into the registers that the half tile before has just left.  Tiles of 64 queries go global -> LDS once for both waves (each moves half of
+// every half tile), three half tiles ahead, with one barrier per half tile: behind it both waves' parts of the next half tile have landed
+// and nobody reads the one before this any more, whose buffers are then requested again.
+// The per-query terms ride in the accumulators: S starts at -lse / scale, so P = exp2(scale log2(e) S), and dP at -delta, so dS / scale =
+// P dP; bf16 puts the scale onto dK once at the end, fp16, with its narrow range, onto every dS.
+// us, before (32 x 32 products, two tiles, the scores of a tile's first half and the products of its second one with nothing beside them) /
+// now: 266 496 tokens x 16 heads, top-16 2 532 / 2 336, dense over 8 192 x 16 537 / 472, 4 164 x 16 208 / 188.  Dense it runs at 1.17 PFLOP/s, the rate of
+// a large library product (the chip's power: on zeros the same instructions take 384); with lists a workgroup's start and end, 1.1 GB each
+// of K and V, Q and dO, dK and dV, take 0.4 ms beside it.  Tried: one wave a SIMD with 64 keys (half the LDS reads, but a lone wave issues a vector
+// instruction every eight cycles, two of them one every four: 2 478).
 template <typename E, bool DENSE>
-__global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, int nqb_all, int total_wg) {
+__global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, int nqb_all, int total) {
   typedef typename Mma<E>::V8 V8;
-  constexpr int kTileBytes = 2 * kHalfBytes;  // a 64-row query tile
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_q0[kTileBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_q1[kTileBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_g0[kTileBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_g1[kTileBytes];
-  // per-query scalars of a tile: [0,64) lse, [64,128) delta
-  constexpr int kDeltaAt = 64;
-  __shared__ __attribute__((aligned(256))) float lds_s0[128];
-  __shared__ __attribute__((aligned(256))) float lds_s1[128];
+  typedef typename Mma<E>::V2 V2;
+  typedef __attribute__((address_space(3))) void* Lds;
+  // half tiles [tile parity][half]; separate arrays: a read of one does not wait for transfers into another
+  __shared__ __attribute__((aligned(1024))) unsigned char lds_q00[kHalfBytes], lds_q01[kHalfBytes], lds_q10[kHalfBytes], lds_q11[kHalfBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds_g00[kHalfBytes], lds_g01[kHalfBytes], lds_g10[kHalfBytes], lds_g11[kHalfBytes];
+  __shared__ __attribute__((aligned(256))) float lds_s[2][64];  // per wave, of a half tile: [0, 32) -lse / scale, [32, 64) -delta
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int hh = lane >> 5;
-  const int c = lane & 31;
+  const int g = lane >> 4;
+  const int c = lane & 15;
 
-  // With lists the grid has two passes over the key blocks: the first (workgroups [0, total_wg)) takes the blocks whose
+  // With lists the grid has two passes over the key blocks: the first (workgroups [0, total)) takes the blocks whose
   // lists are long, the second the others, so the longest lists of a skewed index tensor start first instead of
   // wherever their key block falls in the launch order.
-  const bool long_pass = DENSE || (int)blockIdx.x < total_wg;
-  const int w = (int)blockIdx.x < total_wg ? (int)blockIdx.x : (int)blockIdx.x - total_wg;
-  const int xcd = w & 7, slot = w >> 3;
-  const int per = total_wg >> 3, rem = total_wg & 7;
-  const int vid = xcd * per + (xcd < rem ? xcd : rem) + slot;
-  const int bh = vid / nkb;
-  const int kb = vid - bh * nkb;
-  const int b = bh / p.H;
+  const bool long_pass = DENSE || (int)blockIdx.x < total;
+  const int vid = b16x::work_item((int)blockIdx.x < total ? (int)blockIdx.x : (int)blockIdx.x - total, total);
+  const int bh = __builtin_amdgcn_readfirstlane(vid / nkb);
+  const int kb = __builtin_amdgcn_readfirstlane(vid - bh * nkb);
+  const int b = __builtin_amdgcn_readfirstlane(bh / p.H);
   const int h = bh - b * p.H;
 
   const int64_t Lq = p.Lq, Lk = p.Lk;
-  if constexpr (!DENSE) {
+  // query blocks that attend to this key block
+  int n;
+  const int32_t* list = nullptr;
+  if constexpr (DENSE) {
+    n = nqb_all;
+  } else {
     const int32_t* off = p.kq_off + ((int64_t)b * p.H + h) * (nkb + 1);
-    int len = off[kb + 1] - off[kb];
-    len = __builtin_amdgcn_readfirstlane(len);
-    if ((len > 4 * p.K) != long_pass) return;
+    const int32_t lo = off[kb], hi = off[kb + 1];
+    n = __builtin_amdgcn_readfirstlane(hi - lo);
+    if ((n > 4 * p.K) != long_pass) return;
+    list = p.kq_list + ((int64_t)b * p.H + h) * p.list_stride + lo;
   }
   const E* qp = (const E*)p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh;
   const E* kp = (const E*)p.k + (int64_t)b * p.skb + (int64_t)h * p.skh;
   const E* vp = (const E*)p.v + (int64_t)b * p.svb + (int64_t)h * p.svh;
   const E* gp = (const E*)p.dout + (int64_t)b * p.sgb + (int64_t)h * p.sgh;
-  const float* lsep = p.lse + ((int64_t)b * p.H + h) * Lq;
-  const float* dlp = p.delta + ((int64_t)b * p.H + h) * Lq;
-
-  // B operands K and V of this wave's 32 keys (lane = key, head_dim chunk hh + 2 ks)
-  const int64_t key = (int64_t)kb * 64 + wave * 32 + c;
-  V8 bk[4], bv[4];
-  f32x16 dkt[2], dvt[2];  // dK^T, dV^T [dt]: lane = key, registers = head_dim
-  auto load_keys = [&]() {
+  const int64_t key0 = (int64_t)kb * 64 + wave * 32 + c;
+  E* dkp = (E*)p.dk + (int64_t)b * p.sdkb + (int64_t)h * p.sdkh + 4 * g;
+  E* dvp = (E*)p.dv + (int64_t)b * p.sdvb + (int64_t)h * p.sdvh + 4 * g;
+  if (n == 0) {  // nobody attends to these keys
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++) {
-      Frag f, g;
-      f.u = make_uint4(0, 0, 0, 0);
-      g.u = make_uint4(0, 0, 0, 0);
+    for (int kt = 0; kt < 2; kt++) {
+      const int64_t key = key0 + 16 * kt;
       if (key < Lk) {
-        f.u = *reinterpret_cast<const uint4*>(kp + key * p.skn + ks * 16 + hh * 8);
-        g.u = *reinterpret_cast<const uint4*>(vp + key * p.svn + ks * 16 + hh * 8);
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) {
+          *reinterpret_cast<u32x2*>(dkp + key * p.sdkn + 16 * dt) = (u32x2){0, 0};
+          *reinterpret_cast<u32x2*>(dvp + key * p.sdvn + 16 * dt) = (u32x2){0, 0};
+        }
       }
-      bk[ks] = as_v8<E>(f);
-      bv[ks] = as_v8<E>(g);
     }
-#pragma unroll
-    for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) { dkt[dt][r] = 0.f; dvt[dt][r] = 0.f; }
-  };
-  load_keys();
-
-  // query blocks that attend to this key block
-  int n_lists;
-  const int32_t* list = nullptr;
-  if constexpr (DENSE) {
-    n_lists = nqb_all;
-  } else {
-    const int32_t* off = p.kq_off + ((int64_t)b * p.H + h) * (nkb + 1);
-    const int32_t lo = off[kb], hi = off[kb + 1];
-    n_lists = hi - lo;
-    list = p.kq_list + ((int64_t)b * p.H + h) * p.list_stride + lo;
+    return;
   }
+  const float* const stat = (lane < 32 ? p.lse : p.delta) + ((int64_t)b * p.H + h) * Lq;
+
   // List entries come 64 at a time (lane l holds entry base + l), so the latency of the list read is paid once per
-  // 64 tiles and not in front of every tile's transfers.  The lists are walked front to back.
-  int32_t held_a = -1;
-  int base_a = -64;
-  auto entry = [&](const int32_t* lst, int len, int32_t& held, int& base, int i) -> int32_t {
+  // 64 tiles and not in front of every tile's transfers.
+  int32_t held = -1;
+  int base = -64;
+  auto block_of = [&](int i) -> int32_t {
+    if constexpr (DENSE) return i;
     if (i >= base + 64) {
       base = i & ~63;
-      held = base + lane < len ? lst[base + lane] : -1;
+      held = base + lane < n ? list[base + lane] : -1;
+      asm volatile("" : "+v"(held));  // (waited for here: behind the branch every tile would wait)
     }
     return __builtin_amdgcn_readlane(held, i - base);
-  };
-  auto block_of = [&](int i) -> int64_t {
-    if constexpr (DENSE) {
-      return (int64_t)i;
-    } else {
-      return (int64_t)entry(list, n_lists, held_a, base_a, i);
-    }
   };
 
   const float scale = p.scale;
   const float sl2 = scale * kLog2e;
-  // The per-query terms ride in the accumulators instead of in the vector slots.  The accumulator of S starts at
-  // -lse / scale, so P = exp2(scale * log2(e) * accumulator); the accumulator of dP starts at -delta, so
-  // dS / scale = P * accumulator.  No slot then begins with an LDS read of per-query values in front of the arithmetic
-  // that needs them: the start values come with four ds_read_b128 per accumulator ahead of the half's products (those of
-  // the second half's dP a quarter per slot, next to the fragments of its products).  bf16 also puts the softmax scale
-  // onto dK once at the end (the rounding of dS to the I/O type is relative and does not care for the factor): per score
-  // a multiplication, an exponential and a multiplication instead of two fused multiply-adds, an exponential and a
-  // multiplication; fp16, with its narrow range, scales every dS.  bf16, 266 496 tokens, top-16: 2.88 -> 2.79 (delta) ->
-  // 2.62 ms (lse).
-  const float inv_scale = 1.0f / scale;
-  constexpr bool FOLD = true;  // (kept as a switch: the other form reads lse and delta from LDS inside the vector slots)
+  const float factor = lane < 32 ? -1.0f / scale : -1.0f;
   constexpr bool LATE_SCALE = std::is_same<E, bf16_t>::value;  // the softmax scale goes onto dK at the end
   const uint32_t qrow = (uint32_t)p.sqm * (uint32_t)sizeof(E), grow = (uint32_t)p.sgm * (uint32_t)sizeof(E);
-  const int tr_off = tr_offset(lane);
-  // (one per parity of the instruction inside its half tile: the chunk map of rows 8..15 differs from that of rows 0..7)
-  const uint32_t q_voff[2] = {(uint32_t)(lane >> 3) * qrow + (uint32_t)(((lane & 7) ^ k_swizzle(lane >> 3)) * 16),
-                              (uint32_t)(lane >> 3) * qrow + (uint32_t)(((lane & 7) ^ k_swizzle((lane >> 3) + 8)) * 16)};
-  const uint32_t g_voff[2] = {(uint32_t)(lane >> 3) * grow + (uint32_t)(((lane & 7) ^ k_swizzle(lane >> 3)) * 16),
-                              (uint32_t)(lane >> 3) * grow + (uint32_t)(((lane & 7) ^ k_swizzle((lane >> 3) + 8)) * 16)};
+  const uint32_t chunk = (uint32_t)(((lane & 7) ^ b16x::swz(lane >> 3)) * 16);
+  const uint32_t q_voff = (uint32_t)(lane >> 3) * qrow + chunk, g_voff = (uint32_t)(lane >> 3) * grow + chunk;
+  const int row_off = c * 128 + ((g ^ b16x::swz(c)) << 4);
+  const int tr_row = 4 * g + (c >> 2);
+  const int tr_off = tr_row * 128 + ((((c & 3) >> 1) ^ b16x::swz(tr_row)) << 4) + (c & 1) * 8;
+  auto q_buf = [&](auto par, auto hf) -> char* {
+    if constexpr (decltype(par)::value == 0) return reinterpret_cast<char*>(decltype(hf)::value == 0 ? lds_q00 : lds_q01);
+    else return reinterpret_cast<char*>(decltype(hf)::value == 0 ? lds_q10 : lds_q11);
+  };
+  auto g_buf = [&](auto par, auto hf) -> char* {
+    if constexpr (decltype(par)::value == 0) return reinterpret_cast<char*>(decltype(hf)::value == 0 ? lds_g00 : lds_g01);
+    else return reinterpret_cast<char*>(decltype(hf)::value == 0 ? lds_g10 : lds_g11);
+  };
 
-  float staged = 0.f;          // this lane's lse or delta value of the tile in flight, as loaded (wave 0 lse, wave 1 delta)
-  bool staged_inf = false;     // rows past the end of the tensor publish lse = +inf
-  int staged_buf = -1;         // (wave-uniform) the buffer it goes to; -1: nothing staged
-  // One query tile (64 rows of Q and dO, 64 lse and delta values) -> buffer BUF; each wave moves half of every
-  // operand (instructions 2*wave, 2*wave+1 of both 32-row halves), wave 0 the lse values, wave 1 delta.
-  auto fetch = [&](int64_t qblk, auto bufc) {
-    constexpr int BUF = decltype(bufc)::value;
-    char* qb = reinterpret_cast<char*>(BUF == 0 ? lds_q0 : lds_q1);
-    char* gb = reinterpret_cast<char*>(BUF == 0 ? lds_g0 : lds_g1);
-    const int64_t start = qblk * 64;
-    const int last = (int)((Lq - start < 64 ? Lq - start : 64) - 1);
-    if (last >= 63) {
-      // (wave-uniform) a full tile: per-lane offsets (row lane/8 and its chunk) that do not depend on the tile, the
-      // instruction's rows ride in the scalar offset
-      const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)(qp + start * p.sqm), 0, 0x7fffffff, 0x00020000);
-      const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void*)(gp + start * p.sgm), 0, 0x7fffffff, 0x00020000);
-#pragma unroll
-      for (int hf = 0; hf < 2; hf++)
-#pragma unroll
-        for (int ii = 0; ii < 2; ii++) {
-          const int i = 2 * wave + ii;
-          const uint32_t rows = (uint32_t)(32 * hf + 8 * i);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (__attribute__((address_space(3))) void*)(qb + hf * kHalfBytes + i * 1024), 16,
-                                                   q_voff[ii], rows * qrow, 0, 0);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (__attribute__((address_space(3))) void*)(gb + hf * kHalfBytes + i * 1024), 16,
-                                                   g_voff[ii], rows * grow, 0, 0);
-        }
+  // A half tile's requests: of a wave four transfers (number i of 0, 1 of Q, 2, 3 of dO: rows 8 (2 wave + i % 2) .. + 7) and one load of lse
+  // or delta per lane.  The tile that ends the tensor early issues the same four without records, which fetch nothing, and then transfers whose
+  // rows beyond the end re-read the last one: the waits count the requests behind the one they need, and more of them only wait for more.
+  float staged[2][2];  // lse or delta as loaded [tile parity][half]
+  int end[2][2];       // (scalar) last row of its tile
+  int last[2];         // (scalar) last row of the tile that is being requested
+  int64_t first[2];    // (scalar) its first row
+  const int32_t ragged_blk = (Lq & 63) ? (int32_t)(Lq >> 6) : -1;
+  auto aim = [&](auto par, int32_t blk) {
+    constexpr int PAR = decltype(par)::value;
+    first[PAR] = (int64_t)blk * 64;
+    last[PAR] = blk == ragged_blk ? (int)(Lq & 63) - 1 : 63;
+  };
+  auto request = [&](auto par, auto hf, auto i_tag) {
+    constexpr int PAR = decltype(par)::value, HF = decltype(hf)::value, i = decltype(i_tag)::value;
+    const uint32_t part = (uint32_t)(2 * wave + (i & 1)), r = 32 * HF + 8 * part;
+    int32_t rec, some;
+    b16x::records(last[PAR] - 63, rec, some);
+    if constexpr (i < 2) {
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(qp + first[PAR] * p.sqm), 0, rec, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (Lds)(q_buf(par, hf) + part * 1024), 16, q_voff, r * qrow, 0, 0);
     } else {
-#pragma unroll
-      for (int hf = 0; hf < 2; hf++) {
-        dma_rows<E, true>(qp + start * p.sqm, qrow, 32 * hf, last, qb + hf * kHalfBytes, lane, 2 * wave, 2 * wave + 2);
-        dma_rows<E, true>(gp + start * p.sgm, grow, 32 * hf, last, gb + hf * kHalfBytes, lane, 2 * wave, 2 * wave + 2);
-      }
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(gp + first[PAR] * p.sgm), 0, rec, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (Lds)(g_buf(par, hf) + part * 1024), 16, g_voff, r * grow, 0, 0);
     }
-    // per-query scalars pass through a register and are stored to LDS by `publish` before the barrier that opens
-    // the tile
-    const int r = lane < last ? lane : last;
-    staged = ((wave == 0 ? lsep : dlp) + start)[r];
-    staged_inf = wave == 0 && lane > last;  // query rows beyond Lq: lse = +inf, no probability
-    staged_buf = BUF;
-  };
-  // The loaded value is first touched here, a whole tile of work after its load: any arithmetic on it inside `fetch`
-  // would make the wave wait for the load there, and with it (the counter is in order) for the tile transfers issued
-  // just before, which is the tile that should be in flight during the current tile's work.
-  auto publish = [&]() {
-    if (staged_buf < 0) return;
-    float* const sb = staged_buf == 0 ? lds_s0 : lds_s1;
-    // scaled once here (lse to base 2, delta by the softmax scale) instead of once per score
-    if constexpr (FOLD) sb[64 * wave + lane] = staged_inf ? -INFINITY : wave == 0 ? -staged * inv_scale : -staged;
-    else sb[64 * wave + lane] = staged_inf ? INFINITY : staged * (wave == 0 ? kLog2e : scale);
-    staged_buf = -1;
-  };
-  // One tile in three stages per 32-query half (A = row reads + S, dP; B = P and dS from the per-query scalars; C =
-  // transposed reads + dV^T, dK^T) with every instruction placed by hand, as in the forward kernel.  The vector work of
-  // a 32-query half (16 scores per lane: P, dS, their roundings) is cut into eight slots of two scores; each slot also
-  // issues one matrix product of another stage: the scores of half 1 run under the vector work of half 0, the dV / dK
-  // products of half 0 under the vector work of half 1.  Only the scores of half 0 and the products of half 1 have no
-  // vector work to hide behind.  Query rows beyond Lq need no masks: their lse is +inf.
-  auto tile64 = [&](auto bufc) {
-    constexpr int BUF = decltype(bufc)::value;
-    const char* qb = reinterpret_cast<const char*>(BUF == 0 ? lds_q0 : lds_q1);
-    const char* gb = reinterpret_cast<const char*>(BUF == 0 ? lds_g0 : lds_g1);
-    const float* sb = BUF == 0 ? lds_s0 : lds_s1;
-    f32x16 sc[2], dpv[2];   // S and dP of the two halves
-    V8 pbv[2][2], dbv[2][2];  // P and dS as B operands [half][jj]
-    V8 aq[4], ag[4];          // row fragments of Q, dO (A operands of the scores)
-    V8 gt[2][2], qt[2][2];    // transposed fragments of dO, Q (A operands of dV^T, dK^T)
-    auto mma_a = [&](auto hf_tag, auto i_tag) {  // product i of 8 of a half's scores: 0-3 S, 4-7 dP
-      constexpr int HF = decltype(hf_tag)::value, i = decltype(i_tag)::value, ks = i & 3;
-      f32x16 z;
+    if constexpr (i == 3) {
+      if (__builtin_expect(last[PAR] < 63, 0)) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): behind the ones that fetch nothing
+        const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)(qp + first[PAR] * p.sqm), 0, 0x7fffffff, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void*)(gp + first[PAR] * p.sgm), 0, 0x7fffffff, 0x00020000);
 #pragma unroll
-      for (int r = 0; r < 16; r++) z[r] = 0.f;
-      if constexpr (i < 4) sc[HF] = Mma<E>::mma(aq[ks], bk[ks], ks == 0 && !FOLD ? z : sc[HF]);
-      else dpv[HF] = Mma<E>::mma(ag[ks], bv[ks], ks == 0 && !FOLD ? z : dpv[HF]);
-    };
-    // FOLD: the accumulator of a half's dP starts at minus delta of its queries (registers 4g .. 4g+3 hold the queries
-    // 4hh + 8g .. + 3 of the half)
-    auto lse_init = [&](auto hf_tag) {
-      constexpr int HF = decltype(hf_tag)::value;
-      if constexpr (FOLD) {
-#pragma unroll
-        for (int g4 = 0; g4 < 4; g4++) {
-          const float4 l4 = *reinterpret_cast<const float4*>(sb + 32 * HF + 4 * hh + 8 * g4);
-          sc[HF][4 * g4] = l4.x;
-          sc[HF][4 * g4 + 1] = l4.y;
-          sc[HF][4 * g4 + 2] = l4.z;
-          sc[HF][4 * g4 + 3] = l4.w;
+        for (int k = 0; k < 2; k++) {
+          int row = 32 * HF + 8 * (2 * wave + k) + (lane >> 3);
+          row = row < last[PAR] ? row : last[PAR];
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (Lds)(q_buf(par, hf) + (2 * wave + k) * 1024), 16, (uint32_t)row * qrow + chunk, 0, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (Lds)(g_buf(par, hf) + (2 * wave + k) * 1024), 16, (uint32_t)row * grow + chunk, 0, 0, 0);
         }
       }
-    };
-    auto delta_init_piece = [&](auto hf_tag, auto g_tag) {  // registers 4g .. 4g+3 of the half's dP accumulator
-      constexpr int HF = decltype(hf_tag)::value, g4 = decltype(g_tag)::value;
-      if constexpr (FOLD) {
-        const float4 d4 = *reinterpret_cast<const float4*>(sb + kDeltaAt + 32 * HF + 4 * hh + 8 * g4);
-        dpv[HF][4 * g4] = d4.x;
-        dpv[HF][4 * g4 + 1] = d4.y;
-        dpv[HF][4 * g4 + 2] = d4.z;
-        dpv[HF][4 * g4 + 3] = d4.w;
-      }
-    };
-    auto delta_init = [&](auto hf_tag) {
-      lse_init(hf_tag);
-      static_for<4>([&](auto g_tag) { delta_init_piece(hf_tag, g_tag); });
-    };
-    auto mma_c = [&](auto hf_tag, auto i_tag) {  // product i of 8 of a half's dV^T / dK^T updates
-      constexpr int HF = decltype(hf_tag)::value, i = decltype(i_tag)::value, jj = (i >> 1) & 1, dt = i & 1;
-      if constexpr (i < 4) dvt[dt] = Mma<E>::mma(gt[jj][dt], pbv[HF][jj], dvt[dt]);
-      else dkt[dt] = Mma<E>::mma(qt[jj][dt], dbv[HF][jj], dkt[dt]);
-    };
-    auto vec = [&](auto hf_tag, auto j_tag) {  // scores 2j, 2j+1 of the half: P, dS, both rounded
-      constexpr int HF = decltype(hf_tag)::value, j = decltype(j_tag)::value, r = 2 * j;
-      // queries 4hh + 8(j/2) + 2(j%2) + {0, 1} of the half
-      f32x16& sh = sc[HF];
-      f32x16& dh = dpv[HF];
-      float p0, p1, e0, e1;
-      if constexpr (FOLD) {
-        p0 = __builtin_amdgcn_exp2f(sh[r] * sl2);
-        p1 = __builtin_amdgcn_exp2f(sh[r + 1] * sl2);
-        e0 = LATE_SCALE ? p0 * dh[r] : p0 * (dh[r] * scale);
-        e1 = LATE_SCALE ? p1 * dh[r + 1] : p1 * (dh[r + 1] * scale);
-      } else {
-        const float2 l2 = *reinterpret_cast<const float2*>(sb + 32 * HF + 4 * hh + 8 * (j >> 1) + 2 * (j & 1));
-        p0 = __builtin_amdgcn_exp2f(fmaf(sh[r], sl2, -l2.x));
-        p1 = __builtin_amdgcn_exp2f(fmaf(sh[r + 1], sl2, -l2.y));
-        const float2 d2 = *reinterpret_cast<const float2*>(sb + kDeltaAt + 32 * HF + 4 * hh + 8 * (j >> 1) + 2 * (j & 1));
-        e0 = p0 * fmaf(dh[r], scale, -d2.x);
-        e1 = p1 * fmaf(dh[r + 1], scale, -d2.y);
-      }
-      V8& pv = pbv[HF][r >> 3];
-      V8& dv = dbv[HF][r >> 3];
-      pv[r & 7] = (E)p0;
-      pv[(r & 7) + 1] = (E)p1;
-      dv[r & 7] = (E)e0;
-      dv[(r & 7) + 1] = (E)e1;
-    };
-    read_rows<E, true>(qb, c, hh, aq);
-    read_rows<E, true>(gb, c, hh, ag);
-    delta_init(H0{});
-    static_for<8>([&](auto i_tag) { mma_a(H0{}, i_tag); });
-    __builtin_amdgcn_sched_barrier(0);
-    // the fragments of a region's second four products are requested four slots ahead, one per slot, so that at most
-    // five fragments are in registers at a time
-    read_rows<E, true>(qb + kHalfBytes, c, hh, aq);
-    lse_init(H1{});
-    static_for<8>([&](auto j_tag) {
-      constexpr int j = decltype(j_tag)::value;
-      if constexpr (j < 4) ag[j] = read_row_frag<E, true>(gb + kHalfBytes, c, hh, j);
-      if constexpr (j < 4) delta_init_piece(H1{}, j_tag);  // (a quarter per slot: needed from the fifth product on)
-      mma_a(H1{}, j_tag);
-      vec(H0{}, j_tag);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    read_transposed<E>(gb, tr_off, gt);
-    static_for<8>([&](auto j_tag) {
-      constexpr int j = decltype(j_tag)::value;
-      if constexpr (j < 4) qt[(j >> 1) & 1][j & 1] = read_transposed_frag<E>(qb, tr_off, (j >> 1) & 1, j & 1);
-      mma_c(H0{}, j_tag);
-      vec(H1{}, j_tag);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    read_transposed<E>(gb + kHalfBytes, tr_off, gt);
-    read_transposed<E>(qb + kHalfBytes, tr_off, qt);
-    static_for<8>([&](auto i_tag) { mma_c(H1{}, i_tag); });
-  };
-  // this wave's part of the tile has landed, its reads of the other buffer are done; after the barrier both hold
-  // for both waves
-  auto sync = [&]() {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    publish();
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-  };
-
-  auto walk = [&]() {  // all tiles of the current list, double buffered
-    if (n_lists > 0) {
-      int64_t cur = block_of(0);
-      fetch(cur, H0{});
-      for (int t = 0; t < n_lists; t += 2) {
-        sync();
-        const bool more1 = t + 1 < n_lists;
-        const int64_t nxt1 = more1 ? block_of(t + 1) : cur;
-        if (more1) fetch(nxt1, H1{});
-        tile64(H0{});
-        if (!more1) break;
-        sync();
-        const bool more2 = t + 2 < n_lists;
-        cur = more2 ? block_of(t + 2) : nxt1;
-        if (more2) fetch(cur, H0{});
-        tile64(H1{});
-      }
+      end[PAR][HF] = last[PAR];
+      const int row = 32 * HF + (lane & 31);
+      staged[PAR][HF] = (stat + first[PAR])[row < last[PAR] ? row : last[PAR]];
     }
   };
-  E* dkp = (E*)p.dk + (int64_t)b * p.sdkb + (int64_t)h * p.sdkh;
-  E* dvp = (E*)p.dv + (int64_t)b * p.sdvb + (int64_t)h * p.sdvh;
-  walk();
-  if constexpr (LATE_SCALE) {
+  auto request_all = [&](auto par, auto hf) { static_for<4>([&](auto i) { request(par, hf, i); }); };
+  // The loaded value is first touched when its half tile's transfers have been waited for (the counter is in order).
+  auto publish = [&](auto par, auto hf) {
+    constexpr int PAR = decltype(par)::value, HF = decltype(hf)::value;
+    const bool live = 32 * HF + (lane & 31) <= end[PAR][HF];  // query rows beyond Lq: no probability
+    lds_s[wave][lane] = live ? staged[PAR][HF] * factor : lane < 32 ? -INFINITY : 0.f;
+  };
+  V8 aq[2][2], ag[2][2];   // row fragments of Q, dO [16 queries][ks]: A operands of S, dP
+  V8 qt[4], gt[4];         // Q^T, dO^T [dt]: head dimension 16 dt + c, queries 4 g .. of either 16
+  f32x4 lse4[2], delta4[2];  // what S and dP start from [16 queries]
+  auto read_rows16 = [&](const char* half, V8 (&dst)[2][2]) {
 #pragma unroll
-    for (int dt = 0; dt < 2; dt++)
+    for (int t = 0; t < 2; t++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) dkt[dt][r] *= scale;
+      for (int ks = 0; ks < 2; ks++) {
+        Frag f;
+        f.u = *reinterpret_cast<const uint4*>(half + t * 2048 + (row_off ^ (ks << 6)));
+        dst[t][ks] = as_v8<E>(f);
+      }
+  };
+  auto read_cols = [&](const char* half, V8 (&dst)[4]) {
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) {
+      const char* a = half + (tr_off ^ (dt << 5));
+      Frag f;
+      f.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(a));
+      f.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(a + 2048));
+      dst[dt] = as_v8<E>(f);
+    }
+  };
+  auto read_terms = [&](f32x4 (&dst)[2], int at) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) dst[t] = *reinterpret_cast<const f32x4*>(&lds_s[wave][at + 16 * t + 4 * g]);
+  };
+  V8 bk[2][2], bv[2][2];     // K, V as B operands: lane = key 16 kt + c, head dimensions 32 ks + 8 g ..
+  f32x4 st[2][2], dp[2][2];  // S, dP [parity of the unit][16 queries]
+  f32x4 dk[2][4], dv[2][4];  // dK^T, dV^T [kt][dt]: lane = key, registers = head dimensions 16 dt + 4 g ..
+  V8 pf, ds;                 // P, dS of the unit before
+  auto score = [&](auto i_tag, auto kt_tag) {  // product i of 8 of the scores of 16 keys
+    constexpr int i = decltype(i_tag)::value, KT = decltype(kt_tag)::value, t = i & 1, ks = (i >> 1) & 1, B = KT & 1;
+    if constexpr (i < 4) st[B][t] = b16x::mma16<E>(aq[t][ks], bk[KT][ks], ks ? st[B][t] : lse4[t]);
+    else dp[B][t] = b16x::mma16<E>(ag[t][ks], bv[KT][ks], ks ? dp[B][t] : delta4[t]);
+  };
+  auto pair_of = [&](float x, float y) -> uint32_t {
+    V2 v;
+    v[0] = (E)x;
+    v[1] = (E)y;
+    return __builtin_bit_cast(uint32_t, v);
+  };
+  // the requests of a half tile have landed in both waves, LEFT of this wave's being younger; nobody reads the half tile two before any more
+  auto meet = [&](auto left) {
+    constexpr int LEFT = decltype(left)::value;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | LEFT);  // vmcnt(LEFT)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // Phase of unit (half HF of the tile, keys 16 KT ..).  KT = 0: transposed fragments of this half tile behind the last products of the one
+  // before; then the barrier and row fragments of the next one, and requests of the half tile three further on into the buffers of the
+  // one before this.
+  auto phase = [&](auto par, auto hf, auto kt_tag) {
+    constexpr int PAR = decltype(par)::value, HF = decltype(hf)::value, KT = decltype(kt_tag)::value, B = KT;
+    typedef std::integral_constant<int, HF == 0 ? PAR : PAR ^ 1> NPar;  // the next half tile
+    typedef std::integral_constant<int, HF ^ 1> NHf;
+    typedef std::integral_constant<int, HF == 0 ? PAR ^ 1 : PAR> LPar;  // the half tile before, and the one three further on
+    typedef std::integral_constant<int, KT ^ 1> NK;
+    constexpr int PK = KT ^ 1;
+    float x1 = 0.f, e0 = 0.f, e1 = 0.f, d0 = 0.f, d1 = 0.f;
+    u32x4 pn, dn;
+    static_for<16>([&](auto j_tag) {
+      constexpr int j = decltype(j_tag)::value;
+      if constexpr (KT == 0 && j == 4) read_cols(g_buf(par, hf), gt);
+      if constexpr (KT == 0 && j == 8) read_cols(q_buf(par, hf), qt);
+      if constexpr (KT == 0 && j == 12) {
+        meet(std::integral_constant<int, 5>{});
+        publish(NPar{}, NHf{});
+        read_terms(lse4, 0);
+        read_rows16(q_buf(NPar{}, NHf{}), aq);
+      }
+      if constexpr (KT == 1 && j == 0) {
+        read_terms(delta4, 32);
+        read_rows16(g_buf(NPar{}, NHf{}), ag);
+      }
+      if constexpr (KT == 1 && j >= 4 && j < 8) request(LPar{}, NHf{}, std::integral_constant<int, j & 3>{});
+      if constexpr (j < 4) dv[PK][j] = b16x::mma16<E>(gt[j], pf, dv[PK][j]);
+      else if constexpr (j < 8) dk[PK][j - 4] = b16x::mma16<E>(qt[j - 4], ds, dk[PK][j - 4]);
+      else score(std::integral_constant<int, j & 7>{}, NK{});
+      {
+        constexpr int pr = j >> 2, s = j & 3, t = pr >> 1, r = 2 * (pr & 1);
+        if constexpr (s == 0) {
+          e0 = __builtin_amdgcn_exp2f(st[B][t][r] * sl2);
+          x1 = st[B][t][r + 1] * sl2;
+          asm volatile("" ::"v"(e0), "v"(x1));
+        } else if constexpr (s == 1) {
+          e1 = __builtin_amdgcn_exp2f(x1);
+          d0 = LATE_SCALE ? e0 * dp[B][t][r] : e0 * (dp[B][t][r] * scale);
+          asm volatile("" ::"v"(e1), "v"(d0));
+        } else if constexpr (s == 2) {
+          d1 = LATE_SCALE ? e1 * dp[B][t][r + 1] : e1 * (dp[B][t][r + 1] * scale);
+          uint32_t wd = pair_of(e0, e1);
+          asm volatile("" ::"v"(wd), "v"(d1));
+          pn[pr] = wd;
+        } else {
+          uint32_t wd = pair_of(d0, d1);
+          asm volatile("" ::"v"(wd));
+          dn[pr] = wd;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    pf = b16x::frag_of<E>(pn);
+    ds = b16x::frag_of<E>(dn);
+  };
+
+  // K and V of the wave's keys, on their way through the buffers of the second tile (rows beyond Lk re-read the last one, never stored)
+  {
+    const uint32_t krow = (uint32_t)p.skn * (uint32_t)sizeof(E), vrow = (uint32_t)p.svn * (uint32_t)sizeof(E);
+    const int64_t k0 = (int64_t)kb * 64;
+    const int left = (int)(Lk - k0 < 64 ? Lk - k0 : 64) - 1;
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)(kp + k0 * p.skn), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)(vp + k0 * p.svn), 0, 0x7fffffff, 0x00020000);
+    char* const kl = wave == 0 ? q_buf(H1{}, H0{}) : q_buf(H1{}, H1{});
+    char* const vl = wave == 0 ? g_buf(H1{}, H0{}) : g_buf(H1{}, H1{});
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      int row = 32 * wave + 8 * i + (lane >> 3);
+      row = row < left ? row : left;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (Lds)(kl + i * 1024), 16, (uint32_t)row * krow + chunk, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (Lds)(vl + i * 1024), 16, (uint32_t)row * vrow + chunk, 0, 0, 0);
+    }
   }
-  store_rows<E>(dkt, dkp + key * p.sdkn, key < Lk, hh);
-  store_rows<E>(dvt, dvp + key * p.sdvn, key < Lk, hh);
+  int next = 0;
+  auto next_block = [&]() -> int32_t {  // past the end the last one again
+    const int i = next < n ? next : n - 1;
+    next++;
+    return block_of(i);
+  };
+  aim(H0{}, next_block());
+  request_all(H0{}, H0{});
+  request_all(H0{}, H1{});
+  aim(H1{}, next_block());
+  __builtin_amdgcn_s_waitcnt(0x0F7A);  // vmcnt(10): K and V
+  if (wave == 0) {
+    read_rows16(q_buf(H1{}, H0{}), bk);
+    read_rows16(g_buf(H1{}, H0{}), bv);
+  } else {
+    read_rows16(q_buf(H1{}, H1{}), bk);
+    read_rows16(g_buf(H1{}, H1{}), bv);
+  }
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  meet(std::integral_constant<int, 5>{});  // the first half tile; both waves have read K and V
+  request_all(H1{}, H0{});
+  publish(H0{}, H0{});
+  read_terms(lse4, 0);
+  read_terms(delta4, 32);
+  read_rows16(q_buf(H0{}, H0{}), aq);
+  read_rows16(g_buf(H0{}, H0{}), ag);
+  static_for<8>([&](auto i) { score(i, H0{}); });
+  const u32x4 zero = {0, 0, 0, 0};  // nothing for the first phase to add
+  pf = ds = b16x::frag_of<E>(zero);
+#pragma unroll
+  for (int dt = 0; dt < 4; dt++) qt[dt] = gt[dt] = b16x::frag_of<E>(zero);
+#pragma unroll
+  for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) dk[kt][dt] = dv[kt][dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  auto tile = [&](auto par) {  // the tile behind it comes into the other parity's buffers, its second half while this one's first is worked on
+    phase(par, H0{}, H0{});
+    phase(par, H0{}, H1{});
+    aim(par, next_block());
+    phase(par, H1{}, H0{});
+    phase(par, H1{}, H1{});
+  };
+  for (int left = n >> 1; left > 0; left--) {
+    tile(H0{});
+    tile(H1{});
+  }
+  if (n & 1) tile(H0{});
+#pragma unroll
+  for (int dt = 0; dt < 4; dt++) {
+    dv[1][dt] = b16x::mma16<E>(gt[dt], pf, dv[1][dt]);
+    dk[1][dt] = b16x::mma16<E>(qt[dt], ds, dk[1][dt]);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): no transfer may still write LDS when the wave ends
+  const float after = LATE_SCALE ? scale : 1.f;
+#pragma unroll
+  for (int kt = 0; kt < 2; kt++) {
+    const int64_t key = key0 + 16 * kt;
+    if (key < Lk) {
+#pragma unroll
+      for (int dt = 0; dt < 4; dt++) {
+        const f32x4 a = dk[kt][dt], d = dv[kt][dt];
+        const u32x2 ko = {pair_of(a[0] * after, a[1] * after), pair_of(a[2] * after, a[3] * after)};
+        const u32x2 vo = {pair_of(d[0], d[1]), pair_of(d[2], d[3])};
+        *reinterpret_cast<u32x2*>(dkp + key * p.sdkn + 16 * dt) = ko;
+        *reinterpret_cast<u32x2*>(dvp + key * p.sdvn + 16 * dt) = vo;
+      }
+    }
+  }
 }
 
 }  // namespace bwd
