@@ -563,7 +563,9 @@ class _LinearFn(torch.autograd.Function):
         ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, weight if ctx.needs_input_grad[0] else None)
         # The product itself, us on the device, library / kernel: 1024 inputs, 3 072 outputs, 8 104 rows 52.9 / 47.2, 24 192 129.5 / 128.1, 33 345 219 /
         # 175, 50 016 309 / 253; 1 024 outputs 18.9 / 16.6, 45.7 / 49.5, 66.2 / 70.7, 93.1 / 94.3; the gate's 32 18.5 / 8.6 (the host's share), 21.6 / 15.0.
-        out = linear(x, weight, bias) if x.numel() != 0 and linear_pays(x.numel() // x.shape[-1], *weight.shape) else None
+        out = None
+        if ordinary(x) and x.numel() != 0 and weight.dim() == 2 and linear_pays(x.numel() // x.shape[-1], *weight.shape):
+            out = linear(x, weight, bias)
         if out is None:
             out = torch.nn.functional.linear(x, weight, bias)
         # (of a batch it is a view of the product's rows: views that are made in here may not be changed in place)
