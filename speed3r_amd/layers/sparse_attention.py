@@ -80,20 +80,25 @@ def linear_trains(m: nn.Linear, x: Tensor) -> bool:
         and all(t is None or t.dtype in (torch.float32, torch.bfloat16, torch.float16) for t in (x, m.weight, m.bias))
 
 
-# The function in the place of F.linear costs the host 15 us a product without autocast and 40 with it, what its kernel saves of the device
-# counts where the step waits for the device.  Multiply-adds of a product from which that is so: an MLP's (its two products, us a step, torch's /
-# here, under autocast: 8 320 rows of 768 channels 491 / 552, 12 032 697 / 568, 16 000 of 512 554 / 546, 4 160 of 1024 413 / 413, 8 320 707 / 607;
-# without: 8 320 of 512 331 / 361, 12 032 414 / 361, 4 160 of 1024 366 / 325), and an attention layer's projection, whose step has more to do on the
-# host (autocast: 12 032 rows of 1024 channels 1 170 / 1 286, 16 000 1 277 / 1 306, 24 000 1 772 / 1 445, 8 320 of 1536 1 224 / 1 324, 12 032
-# 1 631 / 1 415; without: 12 032 of 1024 975 / 829 on a fast host, 1 044 / 1 110 on another, 16 000 1 184 / 970, 16 000 of 768 1 076 / 1 094,
-# 24 000 1 450 / 1 185).
+# The function in the place of F.linear costs the host up to 40 us a product under autocast, what its kernels save of the device counts where
+# the step waits for the device.  Multiply-adds of a product from which that is so (and, of a layer under autocast, rows: with fewer the step
+# waits for the host), us a step, torch's / here.  An MLP (its two products) under autocast: 4 160 rows of 1024 channels 384 / 470, 6 016 479 /
+# 475, 8 320 663 / 557; 8 320 of 768 488 / 483; 12 032 of 512 424 / 341; without: 6 016 of 512 273 / 309, 8 320 301 / 229, 4 160 of 768 263 / 231,
+# 2 048 of 1024 275 / 275.  A layer (its projection, which gives its other products their way too) under autocast: 8 064 rows of 1024 channels
+# 1 022 / 1 017, 12 096 1 136 / 1 021, 16 128 1 366 / 1 135; 12 096 of 768 1 123 / 1 142, 24 192 1 708 / 1 415; 6 048 of 1536 1 046 / 1 157, 8 064
+# 1 178 / 1 154, 12 096 1 701 / 1 482; without: 6 048 of 768 965 / 932, 4 032 of 1024 903 / 906, 6 048 895 / 832, 8 064 905 / 831, 12 096
+# 1 085 / 879.
 def training_pays(x: Tensor, m: nn.Module, layer: bool) -> bool:
     """Whether the gradients of ``m``'s parameters, those of an attention layer's projection or another product, are enough work
     for :func:`linear_with_grad` in the place of ``m(x)``."""
     if not sizes_are_known(x) or type(m) is not nn.Linear:
         return False
     work = x.numel() * m.weight.shape[0]
-    return work >= ((6e10 if layer else 2e10) if torch.is_autocast_enabled("cuda") else (4e10 if layer else 1.2e10))
+    if not torch.is_autocast_enabled("cuda"):
+        return work >= (1e10 if layer else 8.5e9)
+    if not layer:
+        return work >= 2e10
+    return work >= 6e10 or (work >= 3.5e10 and x.numel() >= 10000 * x.shape[-1])
 
 
 def linear_with_grad(m: nn.Linear, x: Tensor) -> Tensor:
