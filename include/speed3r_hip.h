@@ -401,6 +401,8 @@ int s3r_gated_merge(const void* o_cmp, const void* o_sel, const void* gate, void
  *     (reference count_query_fixedlen / reorder_topk_idx_fixedlen, :423-554).  The kernels add up in the order of the list.
  *   dq (layout strides sdq*), dk, dv (sdk*, sdv*): I/O dtype; dq == NULL or dk == dv == NULL skips that kernel.
  *   Every row of dq, dk, dv inside the tensors is written (zeros where nothing attends).
+ * s3r_attn_bwd_from_output: the same with delta computed on the way, from the forward's output o (layout strides so*): delta is
+ *   [B,H,Lq] fp32 that the call fills.  dq is required; dense attention and blocks of 64.
  */
 /*
  * Key-centric lists for s3r_attn_bwd from the forward's index tensor.
@@ -426,6 +428,16 @@ int s3r_attn_bwd(const void* q, const void* k, const void* v, const void* dout, 
                  int64_t sdqb, int64_t sdqh, int64_t sdqm, int64_t sdkb, int64_t sdkh, int64_t sdkn,
                  int64_t sdvb, int64_t sdvh, int64_t sdvn, int64_t sib, int64_t sih, int64_t sim,
                  float softmax_scale, int dtype, void* stream);
+int s3r_attn_bwd_from_output(const void* q, const void* k, const void* v, const void* dout, const float* lse,
+                             const void* o, int64_t sob, int64_t soh, int64_t som, float* delta,
+                             const int32_t* idx, const int32_t* kq_list, const int32_t* kq_off, int64_t list_stride,
+                             void* dq, void* dk, void* dv,
+                             int B, int H, int64_t Lq, int64_t Lk, int D, int block, int K,
+                             int64_t sqb, int64_t sqh, int64_t sqm, int64_t skb, int64_t skh, int64_t skn,
+                             int64_t svb, int64_t svh, int64_t svn, int64_t sgb, int64_t sgh, int64_t sgm,
+                             int64_t sdqb, int64_t sdqh, int64_t sdqm, int64_t sdkb, int64_t sdkh, int64_t sdkn,
+                             int64_t sdvb, int64_t sdvh, int64_t sdvn, int64_t sib, int64_t sih, int64_t sim,
+                             float softmax_scale, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -251,6 +251,46 @@ extern "C" int s3r_key_block_lists(const int32_t* idx, int32_t* kq_list, int32_t
   return launch_key_block_lists(idx, kq_list, kq_off, B, H, nqb, K, nkb, sib, sih, sim, list_stride, stream);
 }
 
+// o: nullptr, or the forward's output (strides so*), from which delta is computed
+static int attn_bwd_impl(const char* name, const void* o, int64_t sob, int64_t soh, int64_t som,
+                         const void* q, const void* k, const void* v, const void* dout, const float* lse, float* delta,
+                            const int32_t* idx, const int32_t* kq_list, const int32_t* kq_off, int64_t list_stride,
+                            void* dq, void* dk, void* dv,
+                            int B, int H, int64_t Lq, int64_t Lk, int D, int block, int K,
+                            int64_t sqb, int64_t sqh, int64_t sqm, int64_t skb, int64_t skh, int64_t skn,
+                            int64_t svb, int64_t svh, int64_t svn, int64_t sgb, int64_t sgh, int64_t sgm,
+                            int64_t sdqb, int64_t sdqh, int64_t sdqm, int64_t sdkb, int64_t sdkh, int64_t sdkn,
+                            int64_t sdvb, int64_t sdvh, int64_t sdvn, int64_t sib, int64_t sih, int64_t sim,
+                            float softmax_scale, int dtype, void* stream) {
+  if (!q || !k || !v || !dout || !lse || !delta) return fail(S3R_ERR_BAD_ARG, "%s: null pointer", name);
+  if (!dq && !dk && !dv) return fail(S3R_ERR_BAD_ARG, "%s: no gradient requested", name);
+  if ((dk == nullptr) != (dv == nullptr)) return fail(S3R_ERR_BAD_ARG, "%s: dk and dv come together", name);
+  if (idx != nullptr && dk != nullptr && (!kq_list || !kq_off)) return fail(S3R_ERR_BAD_ARG, "%s: dk/dv of the selection branch need the key-centric lists", name);
+  if (B <= 0 || H <= 0 || Lq <= 0 || Lk <= 0 || (idx != nullptr && K <= 0)) return fail(S3R_ERR_BAD_ARG, "%s: non-positive size", name);
+  if ((dtype != S3R_BF16 && dtype != S3R_F16) || D != 64 || (idx != nullptr && block != 64 && block != 16) || K > 64 || !(softmax_scale > 0.f))
+    return fail(S3R_ERR_UNSUPPORTED, "%s: built for bf16/fp16, head_dim 64, block 64 or 16, top-k <= 64, positive scale", name);
+  const int64_t lim = 1 << 20;
+  if (sqm <= 0 || skn <= 0 || svn <= 0 || sgm <= 0 || sqm >= lim || skn >= lim || svn >= lim || sgm >= lim)
+    return fail(S3R_ERR_UNSUPPORTED, "%s: row strides must be positive and below 2^20 elements", name);
+  if (o && (!dq || (idx != nullptr && block != 64)))
+    return fail(S3R_ERR_UNSUPPORTED, "%s: delta comes out of the dq kernel of dense attention and of blocks of 64", name);
+  if (o && (som <= 0 || som >= lim)) return fail(S3R_ERR_UNSUPPORTED, "%s: row strides must be positive and below 2^20 elements", name);
+  if (o && !vec_ok(o, 2, sob, soh, som)) return fail(S3R_ERR_BAD_ARG, "%s: pointers and strides must be multiples of 16 bytes", name);
+  if (!vec_ok(q, 2, sqb, sqh, sqm) || !vec_ok(k, 2, skb, skh, skn) || !vec_ok(v, 2, svb, svh, svn) || !vec_ok(dout, 2, sgb, sgh, sgm) ||
+      (dq && !vec_ok(dq, 2, sdqb, sdqh, sdqm)) || (dk && (!vec_ok(dk, 2, sdkb, sdkh, sdkn) || !vec_ok(dv, 2, sdvb, sdvh, sdvn))))
+    return fail(S3R_ERR_BAD_ARG, "%s: pointers and strides must be multiples of 16 bytes", name);
+  BwdParams p = {};
+  p.q = q; p.k = k; p.v = v; p.dout = dout; p.lse = lse; p.delta = delta; p.o = o; p.delta_out = delta; p.dq = dq; p.dk = dk; p.dv = dv;
+  p.idx = idx; p.kq_list = kq_list; p.kq_off = kq_off; p.list_stride = list_stride;
+  p.B = B; p.H = H; p.Lq = Lq; p.Lk = Lk; p.K = K; p.block = idx != nullptr ? block : 64;
+  p.sqb = sqb; p.sqh = sqh; p.sqm = sqm; p.skb = skb; p.skh = skh; p.skn = skn; p.svb = svb; p.svh = svh; p.svn = svn;
+  p.sob = sob; p.soh = soh; p.som = som;
+  p.sgb = sgb; p.sgh = sgh; p.sgm = sgm; p.sdqb = sdqb; p.sdqh = sdqh; p.sdqm = sdqm; p.sdkb = sdkb; p.sdkh = sdkh; p.sdkn = sdkn;
+  p.sdvb = sdvb; p.sdvh = sdvh; p.sdvn = sdvn; p.sib = sib; p.sih = sih; p.sim = sim;
+  p.scale = softmax_scale;
+  return launch_attn_bwd(p, dtype, stream);
+}
+
 extern "C" int s3r_attn_bwd(const void* q, const void* k, const void* v, const void* dout, const float* lse, const float* delta,
                             const int32_t* idx, const int32_t* kq_list, const int32_t* kq_off, int64_t list_stride,
                             void* dq, void* dk, void* dv,
@@ -260,28 +300,26 @@ extern "C" int s3r_attn_bwd(const void* q, const void* k, const void* v, const v
                             int64_t sdqb, int64_t sdqh, int64_t sdqm, int64_t sdkb, int64_t sdkh, int64_t sdkn,
                             int64_t sdvb, int64_t sdvh, int64_t sdvn, int64_t sib, int64_t sih, int64_t sim,
                             float softmax_scale, int dtype, void* stream) {
-  if (!q || !k || !v || !dout || !lse || !delta) return fail(S3R_ERR_BAD_ARG, "s3r_attn_bwd: null pointer");
-  if (!dq && !dk && !dv) return fail(S3R_ERR_BAD_ARG, "s3r_attn_bwd: no gradient requested");
-  if ((dk == nullptr) != (dv == nullptr)) return fail(S3R_ERR_BAD_ARG, "s3r_attn_bwd: dk and dv come together");
-  if (idx != nullptr && dk != nullptr && (!kq_list || !kq_off)) return fail(S3R_ERR_BAD_ARG, "s3r_attn_bwd: dk/dv of the selection branch need the key-centric lists");
-  if (B <= 0 || H <= 0 || Lq <= 0 || Lk <= 0 || (idx != nullptr && K <= 0)) return fail(S3R_ERR_BAD_ARG, "s3r_attn_bwd: non-positive size");
-  if ((dtype != S3R_BF16 && dtype != S3R_F16) || D != 64 || (idx != nullptr && block != 64 && block != 16) || K > 64 || !(softmax_scale > 0.f))
-    return fail(S3R_ERR_UNSUPPORTED, "s3r_attn_bwd: built for bf16/fp16, head_dim 64, block 64 or 16, top-k <= 64, positive scale");
-  const int64_t lim = 1 << 20;
-  if (sqm <= 0 || skn <= 0 || svn <= 0 || sgm <= 0 || sqm >= lim || skn >= lim || svn >= lim || sgm >= lim)
-    return fail(S3R_ERR_UNSUPPORTED, "s3r_attn_bwd: row strides must be positive and below 2^20 elements");
-  if (!vec_ok(q, 2, sqb, sqh, sqm) || !vec_ok(k, 2, skb, skh, skn) || !vec_ok(v, 2, svb, svh, svn) || !vec_ok(dout, 2, sgb, sgh, sgm) ||
-      (dq && !vec_ok(dq, 2, sdqb, sdqh, sdqm)) || (dk && (!vec_ok(dk, 2, sdkb, sdkh, sdkn) || !vec_ok(dv, 2, sdvb, sdvh, sdvn))))
-    return fail(S3R_ERR_BAD_ARG, "s3r_attn_bwd: pointers and strides must be multiples of 16 bytes");
-  BwdParams p = {};
-  p.q = q; p.k = k; p.v = v; p.dout = dout; p.lse = lse; p.delta = delta; p.dq = dq; p.dk = dk; p.dv = dv;
-  p.idx = idx; p.kq_list = kq_list; p.kq_off = kq_off; p.list_stride = list_stride;
-  p.B = B; p.H = H; p.Lq = Lq; p.Lk = Lk; p.K = K; p.block = idx != nullptr ? block : 64;
-  p.sqb = sqb; p.sqh = sqh; p.sqm = sqm; p.skb = skb; p.skh = skh; p.skn = skn; p.svb = svb; p.svh = svh; p.svn = svn;
-  p.sgb = sgb; p.sgh = sgh; p.sgm = sgm; p.sdqb = sdqb; p.sdqh = sdqh; p.sdqm = sdqm; p.sdkb = sdkb; p.sdkh = sdkh; p.sdkn = sdkn;
-  p.sdvb = sdvb; p.sdvh = sdvh; p.sdvn = sdvn; p.sib = sib; p.sih = sih; p.sim = sim;
-  p.scale = softmax_scale;
-  return launch_attn_bwd(p, dtype, stream);
+  // (without o delta is only read)
+  return attn_bwd_impl("s3r_attn_bwd", nullptr, 0, 0, 0, q, k, v, dout, lse, const_cast<float*>(delta), idx, kq_list, kq_off, list_stride,
+                       dq, dk, dv, B, H, Lq, Lk, D, block, K, sqb, sqh, sqm, skb, skh, skn, svb, svh, svn, sgb, sgh, sgm,
+                       sdqb, sdqh, sdqm, sdkb, sdkh, sdkn, sdvb, sdvh, sdvn, sib, sih, sim, softmax_scale, dtype, stream);
+}
+
+extern "C" int s3r_attn_bwd_from_output(const void* q, const void* k, const void* v, const void* dout, const float* lse,
+                            const void* o, int64_t sob, int64_t soh, int64_t som, float* delta,
+                            const int32_t* idx, const int32_t* kq_list, const int32_t* kq_off, int64_t list_stride,
+                            void* dq, void* dk, void* dv,
+                            int B, int H, int64_t Lq, int64_t Lk, int D, int block, int K,
+                            int64_t sqb, int64_t sqh, int64_t sqm, int64_t skb, int64_t skh, int64_t skn,
+                            int64_t svb, int64_t svh, int64_t svn, int64_t sgb, int64_t sgh, int64_t sgm,
+                            int64_t sdqb, int64_t sdqh, int64_t sdqm, int64_t sdkb, int64_t sdkh, int64_t sdkn,
+                            int64_t sdvb, int64_t sdvh, int64_t sdvn, int64_t sib, int64_t sih, int64_t sim,
+                            float softmax_scale, int dtype, void* stream) {
+  if (!o) return fail(S3R_ERR_BAD_ARG, "s3r_attn_bwd_from_output: null pointer");
+  return attn_bwd_impl("s3r_attn_bwd_from_output", o, sob, soh, som, q, k, v, dout, lse, delta, idx, kq_list, kq_off, list_stride,
+                       dq, dk, dv, B, H, Lq, Lk, D, block, K, sqb, sqh, sqm, skb, skh, skn, svb, svh, svn, sgb, sgh, sgm,
+                       sdqb, sdqh, sdqm, sdkb, sdkh, sdkn, sdvb, sdvh, sdvn, sib, sih, sim, softmax_scale, dtype, stream);
 }
 
 // ---- the attention layer in one call ------------------------------------------------------------------------------

@@ -12,6 +12,8 @@ struct BwdParams {
   const void* dout;        // gradient of the attention output, layout of q
   const float* lse;        // [B,H,Lq] natural-log log-sum-exp of the scaled scores (forward output)
   const float* delta;      // [B,H,Lq] rowsum(dout * out)
+  const void* o;           // nullptr, or the attention output: the dQ kernel computes delta from it and stores it to delta_out (= delta)
+  float* delta_out;
   void* dq;                // nullptr: skip the dQ kernel
   void* dk;                // nullptr: skip the dK/dV kernel
   void* dv;
@@ -27,6 +29,7 @@ struct BwdParams {
   int64_t skb, skh, skn;
   int64_t svb, svh, svn;
   int64_t sgb, sgh, sgm;   // dout
+  int64_t sob, soh, som;   // o
   int64_t sdqb, sdqh, sdqm;
   int64_t sdkb, sdkh, sdkn;
   int64_t sdvb, sdvh, sdvn;

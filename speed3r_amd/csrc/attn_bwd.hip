@@ -10,7 +10,7 @@
 // (reference :683-690, :826-838).
 //
 // Three kernels:
-//   * bwd_delta_kernel: delta[b,h,n] = sum_d o * dO in fp32 (HBM bound).
+//   * bwd_delta_kernel: delta[b,h,n] = sum_d o * dO in fp32 (HBM bound), where the dQ kernel does not compute it on its way.
 //   * bwd_dq_kernel: one wavefront per 64-row query block, four independent waves per workgroup; walks the block's
 //     selected key tiles (or all of them).  Everything is computed transposed, as in the forward kernels:
 //     S^T = K Q^T and dP^T = V dO^T put one QUERY per lane, so lse and delta are per-lane scalars;
@@ -76,9 +76,12 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const E* __restrict__ o,
 //     multiplication and half a conversion, against two multiply-adds, one exponential, one multiplication and half a conversion before.
 //   * 16 x 16 x 32 products: a lane's tuple is four scores, so a unit is small enough to be pipelined in registers (32 x 32 products
 //     with both halves of the queries in flight did not fit, and the compiler's order left matrix cores and vector unit taking turns).
+//   * DELTA: delta comes from O, whose rows a wave reads beside the dO that it holds in LDS anyway, instead of from a kernel of its own that
+//     reads both (171 us at 266 496 tokens): two operators with gradients at that size 5 842 / 5 742.  One sum of eight values per lane, in
+//     the order of that kernel.
 // us, before / now: 266 496 tokens x 16 heads, top-16 1 902 / 1 531 (1.1 PFLOP/s: matrix cores and vector unit have the same work, 1 536
 // cycles each per tile, and the chip runs below 2 GHz under it), dense over 4 164 tokens 212 / 161.
-template <typename E, bool DENSE>
+template <typename E, bool DENSE, bool DELTA>
 __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, int nqg, int total_wg) {
   typedef typename Mma<E>::V8 V8;
   typedef typename Mma<E>::V2 V2;
@@ -126,8 +129,10 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
     const int64_t row = q0 + qt * 16 + c;
     const bool live = row < Lq;
     nl[qt] = live ? fmaf(lsep[row], -kLog2e, log2_scale) : -INFINITY;
-    const float m = live ? -dlp[row] : 0.f;
-    nd[qt] = (f32x4){m, m, m, m};
+    if constexpr (!DELTA) {
+      const float m = live ? -dlp[row] : 0.f;
+      nd[qt] = (f32x4){m, m, m, m};
+    }
   }
   f32x4 dq[4][4];  // dQ^T [qt][dt]: lane = query, registers = head dimensions 16 dt + 4 g ..
 #pragma unroll
@@ -195,6 +200,17 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
     const int left = (int)(Lq - q0 < 64 ? Lq - q0 : 64) - 1;
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)(qp + q0 * p.sqm), 0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void*)(gp + q0 * p.sgm), 0, 0x7fffffff, 0x00020000);
+    u32x4 out[8];  // DELTA: the forward's output, the same chunks of the same rows that the lane's transfers move of dO
+    if constexpr (DELTA) {
+      const E* const op = (const E*)p.o + (int64_t)b * p.sob + (int64_t)h * p.soh;
+      const uint32_t orow = (uint32_t)p.som * (uint32_t)sizeof(E);
+      const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void*)(op + q0 * p.som), 0, 0x7fffffff, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int row = 8 * i + (lane >> 3);
+        out[i] = __builtin_amdgcn_raw_buffer_load_b128(ro, (uint32_t)(row < left ? row : left) * orow + chunk, 0, 2 /* nt: read once */);
+      }
+    }
     static_for<2>([&](auto hf) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -217,6 +233,27 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(BwdParams p, int nqb, in
         bg[QT][ks] = as_v8<E>(d);
       }
     });
+    if constexpr (DELTA) {
+      float s = 0.f;  // of row 8 (lane % 8) + lane / 8
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const u32x4 gv = *reinterpret_cast<const u32x4*>((i < 4 ? v_buf(H0{}) : v_buf(H1{})) + (i & 3) * 1024 + lane * 16);
+        const E* const oe = reinterpret_cast<const E*>(&out[i]);
+        const E* const ge = reinterpret_cast<const E*>(&gv);
+        float t = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) t = fmaf((float)oe[e], (float)ge[e], t);
+        t = group_sum<8>(t);
+        s = (lane & 7) == i ? t : s;
+      }
+      const int64_t row = q0 + 8 * (lane & 7) + (lane >> 3);
+      if (row < Lq) p.delta_out[((int64_t)b * p.H + h) * Lq + row] = s;
+#pragma unroll
+      for (int qt = 0; qt < 4; qt++) {
+        const float m = -__int_as_float(__builtin_amdgcn_ds_bpermute(((c & 7) * 8 + 2 * qt + (c >> 3)) * 4, __float_as_int(s)));
+        nd[qt] = (f32x4){m, m, m, m};
+      }
+    }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): read before the first tile is requested
     asm volatile("" ::: "memory");
   }
@@ -739,7 +776,7 @@ __global__ __launch_bounds__(128, 2) void bwd_dkdv_kernel(BwdParams p, int nkb, 
 
 int launch_attn_bwd(const BwdParams& p, int dtype, void* stream) {
   hipStream_t st = (hipStream_t)stream;
-  const bool dense = p.idx == nullptr;
+  const bool dense = p.idx == nullptr, own = p.o != nullptr;
   if (!dense && p.block == 16) return launch_attn_bwd16(p, dtype, stream);
   const int64_t nqb = (p.Lq + 63) / 64, nkb = (p.Lk + 63) / 64;
   const int64_t nqg = (nqb + 3) / 4;
@@ -750,8 +787,10 @@ int launch_attn_bwd(const BwdParams& p, int dtype, void* stream) {
 #define S3R_BWD_LAUNCH(E)                                                                                                       \
   do {                                                                                                                          \
     if (p.dq != nullptr) {                                                                                                      \
-      if (dense) hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, true>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);     \
-      else hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, false>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);          \
+      if (dense && own) hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, true, true>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);   \
+      else if (dense) hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, true, false>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);    \
+      else if (own) hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, false, true>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);      \
+      else hipLaunchKernelGGL((bwd::bwd_dq_kernel<E, false, false>), gq, bq, 0, st, p, (int)nqb, (int)nqg, (int)total_q);              \
     }                                                                                                                           \
     if (p.dk != nullptr) {                                                                                                      \
       if (dense) hipLaunchKernelGGL((bwd::bwd_dkdv_kernel<E, true>), gk, bk, 0, st, p, (int)nkb, (int)nqb, (int)total_k);   \

@@ -876,7 +876,12 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     b, h, lq, d = q.shape
     lk = k.shape[2]
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
-    if delta is None:
+    # (a kernel that walks the queries reads the output beside the gradient that it reads anyway)
+    inside = delta is None and need_dq and (idx is None or block == 64) and o.shape == q.shape and o.dtype == dout.dtype == q.dtype \
+        and 0 < o.stride(2) < 1 << 20
+    if inside:
+        delta = torch.empty((b, h, lq), dtype=torch.float32, device=q.device)
+    elif delta is None:
         delta = attn_bwd_delta(o, dout)
     dq = torch.empty_like(q, memory_format=torch.contiguous_format) if need_dq else None
     dk = torch.empty_like(k, memory_format=torch.contiguous_format) if need_dkv else None
@@ -898,10 +903,7 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     def st(t):
         return (t.stride(0), t.stride(1), t.stride(2)) if t is not None else (0, 0, 0)
 
-    with _on(q.device):
-        rc = _lib.lib().s3r_attn_bwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), lse.data_ptr(), delta.data_ptr(),
-            idx.data_ptr() if idx is not None else None,
+    rest = (idx.data_ptr() if idx is not None else None,
             lists.data_ptr() if lists is not None else None, offs.data_ptr() if offs is not None else None,
             lists.shape[-1] if lists is not None else 0,
             dq.data_ptr() if dq is not None else None, dk.data_ptr() if dk is not None else None,
@@ -909,6 +911,12 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
             b, h, lq, lk, d, block, kk,
             *st(q), *st(k), *st(v), *st(dout), *st(dq), *st(dk), *st(dv), *st(idx),
             scale, _code(q), _stream(q))
+    first = (q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), lse.data_ptr())
+    with _on(q.device):
+        if inside:
+            rc = _lib.lib().s3r_attn_bwd_from_output(*first, o.data_ptr(), *st(o), delta.data_ptr(), *rest)
+        else:
+            rc = _lib.lib().s3r_attn_bwd(*first, delta.data_ptr(), *rest)
     _lib.check(rc, "s3r_attn_bwd")
     return dq, dk, dv
 

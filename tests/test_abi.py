@@ -61,6 +61,21 @@ def test_host_side_validation_returns_error_codes():
     assert causal(k=12) == _lib.S3R_ERR_UNSUPPORTED and causal(d=128) == _lib.S3R_ERR_UNSUPPORTED
 
 
+def test_backward_from_the_output_validates_on_the_host():
+    L = _lib.lib()
+    one, st = ctypes.c_void_p(16), (64 * 64, 64 * 64, 64)
+
+    def bwd(o=one, o_st=st, delta=one, dq=one, idx=None, block=64):
+        return L.s3r_attn_bwd_from_output(one, one, one, one, one, o, *o_st, delta, idx, one, one, 0, dq, one, one, 1, 1, 64, 64, 64, block, 4,
+                                          *st, *st, *st, *st, *st, *st, *st, 0, 0, 0, 0.125, _lib.S3R_BF16, None)
+
+    assert bwd(o=None) == _lib.S3R_ERR_BAD_ARG and bwd(delta=None) == _lib.S3R_ERR_BAD_ARG
+    assert bwd(dq=None) == _lib.S3R_ERR_UNSUPPORTED and bwd(idx=one, block=16) == _lib.S3R_ERR_UNSUPPORTED   # dq's kernel of 64-token blocks
+    assert bwd(o_st=(64 * 64, 64 * 64, 0)) == _lib.S3R_ERR_UNSUPPORTED and bwd(o_st=(0, 0, 1 << 20)) == _lib.S3R_ERR_UNSUPPORTED
+    assert bwd(o_st=(64 * 64, 64 * 64, 68)) == _lib.S3R_ERR_BAD_ARG and bwd(o=ctypes.c_void_p(8)) == _lib.S3R_ERR_BAD_ARG
+    assert b"s3r_attn_bwd_from_output" in L.s3r_last_error()
+
+
 def test_backward_entry_points_validate_on_the_host():
     L = _lib.lib()
     z3 = (0, 0, 0)

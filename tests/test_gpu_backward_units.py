@@ -18,13 +18,26 @@ def _check(got, want, room, unit, floor, what):
     assert worst <= 1.0, (what, worst)
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("n,lists,scale", [
+CASES = [
     (1, [[0]], 0.125), (15, [[0, 0]], 0.125), (17, [[0]], 0.3), (64, [[0]], 0.125), (64, [[0, 0, 0]], 0.125), (65, [[1], [0]], 0.125),
     (79, [[1, 1], [1, 0]], 0.125), (112, [[0, 1], [1, 0]], 1.0), (128, [[1], [0]], 0.125), (129, [[2, 0, 1], [1, 2, 2], [0, 0, 1]], 0.125),
     (200, [[3, 2, 1, 0], [-1, 3, -1, 2], [0, 1, 2, 9], [3, -1, -1, -1]], 0.07), (320, None, 0.125), (333, None, 0.125), (1090, None, 0.125),
-])
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,lists,scale", CASES)
 def test_gradients_of_one_tile_more_or_less(dtype, n, lists, scale):
+    _gradients(dtype, n, lists, scale, False)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,lists,scale", CASES)
+def test_delta_from_the_output_on_the_way(dtype, n, lists, scale):
+    _gradients(dtype, n, lists, scale, True)
+
+
+def _gradients(dtype, n, lists, scale, inside):
     gen = torch.Generator().manual_seed(n)
     heads, nb = 2, -(-n // 64)
     wide = [torch.randn((1, n, heads, 72), generator=gen).mul_(0.6).to(dtype)[..., :64].permute(0, 2, 1, 3) for _ in range(4)]
@@ -36,8 +49,11 @@ def test_gradients_of_one_tile_more_or_less(dtype, n, lists, scale):
     else:
         o, lse = s3r.select_attn(q, k, v, idx, 64, return_lse=True, softmax_scale=scale)
         times = torch.stack([(torch.tensor(lists) == j).sum(1) for j in range(nb)], dim=1).double()   # how often a list names a block
+    if inside:                                             # (a wider row stride for the output too)
+        wide_o = torch.full((1, n, heads, 72), float("nan"), dtype=dtype, device=DEV)
+        o = wide_o[..., :64].copy_(o.permute(0, 2, 1, 3)).permute(0, 2, 1, 3)
     delta = ops.attn_bwd_delta(o, g)
-    dq, dk, dv = ops.attn_bwd(q, k, v, o, g, lse, idx, softmax_scale=scale, delta=delta)
+    dq, dk, dv = ops.attn_bwd(q, k, v, o, g, lse, idx, softmax_scale=scale, delta=None if inside else delta)
 
     qf, kf, vf, gf = (t.double() for t in wide)
     times = times.repeat_interleave(64, 0)[:n].repeat_interleave(64, 1)[:, :n]
