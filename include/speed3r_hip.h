@@ -402,7 +402,7 @@ int s3r_gated_merge(const void* o_cmp, const void* o_sel, const void* gate, void
  *   dq (layout strides sdq*), dk, dv (sdk*, sdv*): I/O dtype; dq == NULL or dk == dv == NULL skips that kernel.
  *   Every row of dq, dk, dv inside the tensors is written (zeros where nothing attends).
  * s3r_attn_bwd_from_output: the same with delta computed on the way, from the forward's output o (layout strides so*): delta is
- *   [B,H,Lq] fp32 that the call fills.  dq is required; dense attention and blocks of 64.
+ *   [B,H,Lq] fp32 that the call fills.  dq is required.
  */
 /*
  * Key-centric lists for s3r_attn_bwd from the forward's index tensor.

@@ -272,8 +272,7 @@ static int attn_bwd_impl(const char* name, const void* o, int64_t sob, int64_t s
   const int64_t lim = 1 << 20;
   if (sqm <= 0 || skn <= 0 || svn <= 0 || sgm <= 0 || sqm >= lim || skn >= lim || svn >= lim || sgm >= lim)
     return fail(S3R_ERR_UNSUPPORTED, "%s: row strides must be positive and below 2^20 elements", name);
-  if (o && (!dq || (idx != nullptr && block != 64)))
-    return fail(S3R_ERR_UNSUPPORTED, "%s: delta comes out of the dq kernel of dense attention and of blocks of 64", name);
+  if (o && !dq) return fail(S3R_ERR_UNSUPPORTED, "%s: delta comes out of the dq kernel", name);
   if (o && (som <= 0 || som >= lim)) return fail(S3R_ERR_UNSUPPORTED, "%s: row strides must be positive and below 2^20 elements", name);
   if (o && !vec_ok(o, 2, sob, soh, som)) return fail(S3R_ERR_BAD_ARG, "%s: pointers and strides must be multiples of 16 bytes", name);
   if (!vec_ok(q, 2, sqb, sqh, sqm) || !vec_ok(k, 2, skb, skh, skn) || !vec_ok(v, 2, svb, svh, svn) || !vec_ok(dout, 2, sgb, sgh, sgm) ||

@@ -877,8 +877,7 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
     lk = k.shape[2]
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
     # (a kernel that walks the queries reads the output beside the gradient that it reads anyway)
-    inside = delta is None and need_dq and (idx is None or block == 64) and o.shape == q.shape and o.dtype == dout.dtype == q.dtype \
-        and 0 < o.stride(2) < 1 << 20
+    inside = delta is None and need_dq and o.shape == q.shape and o.dtype == dout.dtype == q.dtype and 0 < o.stride(2) < 1 << 20
     if inside:
         delta = torch.empty((b, h, lq), dtype=torch.float32, device=q.device)
     elif delta is None:

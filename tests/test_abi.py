@@ -70,7 +70,7 @@ def test_backward_from_the_output_validates_on_the_host():
                                           *st, *st, *st, *st, *st, *st, *st, 0, 0, 0, 0.125, _lib.S3R_BF16, None)
 
     assert bwd(o=None) == _lib.S3R_ERR_BAD_ARG and bwd(delta=None) == _lib.S3R_ERR_BAD_ARG
-    assert bwd(dq=None) == _lib.S3R_ERR_UNSUPPORTED and bwd(idx=one, block=16) == _lib.S3R_ERR_UNSUPPORTED   # dq's kernel of 64-token blocks
+    assert bwd(dq=None) == _lib.S3R_ERR_UNSUPPORTED                         # delta comes out of dq's kernel
     assert bwd(o_st=(64 * 64, 64 * 64, 0)) == _lib.S3R_ERR_UNSUPPORTED and bwd(o_st=(0, 0, 1 << 20)) == _lib.S3R_ERR_UNSUPPORTED
     assert bwd(o_st=(64 * 64, 64 * 64, 68)) == _lib.S3R_ERR_BAD_ARG and bwd(o=ctypes.c_void_p(8)) == _lib.S3R_ERR_BAD_ARG
     assert b"s3r_attn_bwd_from_output" in L.s3r_last_error()
