@@ -1,0 +1,71 @@
+"""fp32 selection attention in blocks of 64 on the 16-bit matrix instructions (needs an MI355X), 512 blocks and more: ragged last blocks, lists that repeat, skip or
+lack entries, strided and odd-aligned queries, values that three bf16 parts do not hold."""
+import pytest
+import torch
+
+import speed3r_amd as s3r
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _reference(q, k, v, idx, scale):
+    """Output, log-sum-exp and an error bound of the output, in 64 bits on the CPU."""
+    q, k, v, idx = (t.cpu().double() if t.is_floating_point() else t.cpu() for t in (q, k, v, idx))
+    out, lse, bound = torch.zeros_like(q), torch.full(q.shape[:3], -float("inf"), dtype=torch.float64), torch.zeros_like(q)
+    n = q.shape[2]
+    for h in range(q.shape[1]):
+        for i in range(idx.shape[2]):
+            cols = [torch.arange(j * 64, min(n, j * 64 + 64)) for j in idx[0, h, i].tolist() if 0 <= j * 64 < n]
+            if not cols:
+                continue
+            cols, rows = torch.cat(cols), slice(i * 64, min(n, i * 64 + 64))
+            s = scale * q[0, h, rows] @ k[0, h, cols].T
+            p = torch.softmax(s, -1)
+            out[0, h, rows] = p @ v[0, h, cols]
+            lse[0, h, rows] = torch.logsumexp(s, -1)
+            # 64 + 16 roundings of 2^-24 in a score, as many in the exponent's product, then 40 in sums and quotient
+            ds = 2.0 ** -24 * (80 * scale * q[0, h, rows].abs() @ k[0, h, cols].abs().T + 2 * s.abs()).amax(-1, keepdim=True)
+            bound[0, h, rows] = (2 * ds + 40 * 2.0 ** -24) * (p @ v[0, h, cols].abs())
+    return out, lse, bound
+
+
+def _inputs(heads, n, seed, size=1.0):
+    gen = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn((1, heads, n, 64), generator=gen).mul_(size).to(DEV) for _ in range(3))
+    nb = -(-n // 64)
+    idx = torch.randint(-1, nb + 1, (1, heads, nb, 5), generator=gen).int().to(DEV)   # (some skipped, some twice)
+    return q, k, v, idx
+
+
+@pytest.mark.parametrize("heads,n,scale", [(512, 1, 0.125), (512, 31, 0.125), (513, 33, 0.125), (512, 64, 1.0), (256, 65, 0.125), (171, 161, 0.3), (64, 512, 0.125)])
+def test_against_64_bits(heads, n, scale):
+    q, k, v, idx = _inputs(heads, n, n)
+    idx[0, 0, 0] = -1                                                                 # nothing listed
+    want, lse_want, bound = _reference(q, k, v, idx, scale)
+    odd = torch.empty(heads * n * 65 + 1, device=DEV)[1:].view(1, n, heads, 65)[..., :64].copy_(q.permute(0, 2, 1, 3)).permute(0, 2, 1, 3)
+    for query in (q, odd):
+        o, lse = s3r.select_attn(query, k, v, idx, 64, scale, return_lse=True)
+        assert ((o.double().cpu() - want).abs() <= bound + 1e-30).all()
+        far = torch.isinf(lse_want)
+        assert torch.equal(torch.isinf(lse).cpu(), far) and ((lse.double().cpu() - lse_want).abs()[~far] <= 2e-5).all()
+
+
+@pytest.mark.parametrize("what,value", [("k", 3.39e38), ("k", 1e-30), ("v", 1e-30), ("q", 1e-30), ("k", -float("inf")), ("v", float("inf")), ("q", float("nan")), ("v", float("nan"))])
+def test_values_beyond_three_parts(what, value):
+    t = dict(zip("qkvi", _inputs(256, 100, 3)))
+    t["i"][0, :, 0] = torch.tensor([0, 1, 0, 1, 1], device=DEV)
+    t["i"][0, 0, 1] = 0                                                               # (block 1's rows of head 0 do not see row 70)
+    if abs(value) < 1:
+        t[what].mul_(value)
+    else:
+        t[what][0, 0, 70, 5] = value
+    if value == 3.39e38:
+        t["q"][..., 5] = 2e-38                                                        # (finite scores)
+    want, _, bound = _reference(t["q"], t["k"], t["v"], t["i"], 0.125)
+    o = s3r.select_attn(t["q"], t["k"], t["v"], t["i"], 64).double().cpu()
+    clean = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(o), clean) and torch.equal(torch.isinf(o), torch.isinf(want))
+    bound = torch.nan_to_num(bound, nan=0.0, posinf=0.0)
+    sure = clean & (bound > 0)
+    assert ((o - want).abs()[sure] <= bound[sure] + 1e-44).all()
