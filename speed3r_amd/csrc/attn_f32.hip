@@ -1,7 +1,7 @@
 // fp32 attention on the matrix cores (head_dim 64): the selection branch for blocks of 64, 32 and 16 tokens and the
 // compressed branch with its fp32 scores.
 //
-// Blocks of 64 go to attn_f32_split_kernel from 512 of them on (launch_64); what follows is about attn_f32_kernel.
+// Blocks of 64 go to attn_f32_split_kernel from 385 of them on (launch_64); what follows is about attn_f32_kernel.
 //
 // Bound: the fp32 matrix instructions (v_mfma_f32_16x16x4_f32: 64 FLOP per cycle and SIMD, 157 TFLOP/s; a product of
 // 8192 x 8192 matrices by the library reaches 154).  At 8 328 tokens x 16 heads, 16 blocks of 64 (3.5e10 FLOP, 0.23 ms)
@@ -614,12 +614,12 @@ template <int W, int KS, int BLK, bool SPLIT = false> static int launch_t(const 
   return check_launch("attn_f32_kernel");
 }
 
-// Blocks of 64.  With fewer than two of them to a CU the workgroups of the split values wait for one another's units too little: 16 heads, us, fp32
-// instructions / split values: 333 tokens (96 blocks) 16.2 / 19.6, 500 (128) 21.4 / 26.7, 700 (176) 38.8 / 35.0, 1 041 (272) 62.9 / 61.3, 1 500
-// (384) 66.5 / 63.1, 2 600 (656) 118 / 82.
+// Blocks of 64.  Up to 384 of them the fp32 instructions, half blocks in the last round, are faster or within 10 %, and keep the score bits of a
+// chain of fp32 products; then they take a second whole round.  16 heads, us, fp32 instructions / split values: 333 tokens (96 blocks) 16.2 /
+// 19.6, 500 (128) 21.4 / 26.7, 700 (176) 38.8 / 35.0, 1 041 (272) 62.9 / 61.3, 1 500 (384) 66.5 / 63.1, 1 900 (480) 84.8 / 63.8, 2 600 (656) 118 / 82.
 static int launch_64(const AttnParams& p, hipStream_t st) {
   const int64_t ngrp = (p.Lq + 63) / 64, total = ngrp * p.B * p.H;
-  if (total < 512) return launch_t<4, 32, 64, true>(p, st);
+  if (total <= 384) return launch_t<4, 32, 64, true>(p, st);
   if (total > 0x7fffffffLL) return fail(S3R_ERR_UNSUPPORTED, "attention: grid too large");
   hipLaunchKernelGGL(attn_f32_split_kernel, dim3((unsigned)total), dim3(256), 0, st, p, (int)ngrp, (int)total);
   return check_launch("attn_f32_split_kernel");
