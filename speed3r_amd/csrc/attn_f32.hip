@@ -312,7 +312,7 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
 // by the four waves, 44 that of the probabilities), and with four waves to a SIMD the two units overlap by half: without a third
 // of the products 176 us, without the splitting 221.  K and V come through registers, a stage ahead, into one LDS buffer of
 // 24 KB (two barriers a stage): with two buffers only three waves fit a SIMD, 235 us.
-// Where something does not split (infinities, values next to the end of the range at either side) the workgroup starts over on the
+// Where something does not split (infinities, values from 2^60 on, values next to the lower end of the range) the workgroup starts over on the
 // fp32 instructions, operands from memory.
 __device__ __forceinline__ uint32_t pair_bf16(float a, float b) {  // (by hand: the compiler converts once more for each part it takes out)
   uint32_t o;
@@ -336,9 +336,10 @@ __device__ __forceinline__ float largest(const float4& a, const float4& b) {
       : "=&v"(x) : "v"(a.x), "v"(a.y), "v"(a.z), "v"(a.w), "v"(b.x), "v"(b.y), "v"(b.z), "v"(b.w));
   return x;
 }
-// Do three parts hold them?  Beyond 3.3e38 the first part may round to infinity; where the largest is below 2^-90, third parts fall out of
-// the normal range.
-__device__ __forceinline__ bool splits(float largest) { return largest < 3.3e38f && !(largest > 0.f && largest < 8.1e-28f); }
+// Do three parts hold them, and their products?  From 2^60 on a score's or an output's partial sums may leave the range (64 products of two values
+// below it reach 2^126), and what cancels in a chain of whole products does not in the parts': infinities of either sign, a NaN
+// where the chain has a score of -inf.  Where the largest is below 2^-90, third parts fall out of the normal range.
+__device__ __forceinline__ bool splits(float largest) { return largest < 0x1p60f && !(largest > 0.f && largest < 8.1e-28f); }
 typedef float Any4 __attribute__((ext_vector_type(4), aligned(4)));
 struct Parts {
   u32x4 p[3];

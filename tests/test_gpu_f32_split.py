@@ -69,3 +69,17 @@ def test_values_beyond_three_parts(what, value):
     bound = torch.nan_to_num(bound, nan=0.0, posinf=0.0)
     sure = clean & (bound > 0)
     assert ((o - want).abs()[sure] <= bound[sure] + 1e-44).all()
+
+
+# A chain of fp32 products gives such a score -inf or a number that far down, and its key no weight; the products of parts have either sign.  Bound: 2^-24 for
+# each of 64 roundings in the scores, which are at most 10, and of 40 in sums and quotient.  A key with any weight more would be 1e-2 of the result.
+@pytest.mark.parametrize("size", [1e18, 1e19, 1e21, 1e25, 1e30])
+@pytest.mark.parametrize("channels", [slice(5, 6), slice(8, 16), slice(0, 64)])
+def test_scores_beyond_the_range(size, channels):
+    q, k, v, idx = _inputs(256, 100, 5)
+    idx[..., 0], idx[..., 1] = 0, 1
+    q[..., channels], k[..., channels] = size, 0.0
+    k[:, :, 70, channels] = -size                                                     # (one key far below the others, which are ordinary)
+    want, lse_want, _ = _reference(q, k, v, idx, 0.125)
+    o, lse = s3r.select_attn(q, k, v, idx, 64, 0.125, return_lse=True)
+    assert bool((o.double().cpu() - want).norm() <= 4e-5 * want.norm()) and bool((lse.double().cpu() - lse_want).abs().max() <= 4e-5)
