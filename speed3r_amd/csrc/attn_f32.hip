@@ -312,8 +312,9 @@ __global__ __launch_bounds__(64 * W, 4) void attn_f32_kernel(AttnParams p, int n
 // by the four waves, 44 that of the probabilities), and with four waves to a SIMD the two units overlap by half: without a third
 // of the products 176 us, without the splitting 221.  K and V come through registers, a stage ahead, into one LDS buffer of
 // 24 KB (two barriers a stage): with two buffers only three waves fit a SIMD, 235 us.
-// Where something does not split (infinities, values from 2^60 on, values next to the lower end of the range) the workgroup starts over on the
-// fp32 instructions, operands from memory.
+// Where something does not split (infinities, values from 2^60 on, values of V next to the lower end of the range) the workgroup starts over on
+// the fp32 instructions, operands from memory.  Probabilities below 2^-112 of the row's reference keep fewer than 24 bits, those below
+// 2^-126 are lost on both paths: 2.9e-6 / 3.4e-6 at 2^-112, 2.9e-6 / 1.6e-5 at 2^-117, 2.9e-6 / 3.2e-4 at 2^-122 (seen where the keys above have values of zero).
 __device__ __forceinline__ uint32_t pair_bf16(float a, float b) {  // (by hand: the compiler converts once more for each part it takes out)
   uint32_t o;
   asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b));
@@ -336,10 +337,21 @@ __device__ __forceinline__ float largest(const float4& a, const float4& b) {
       : "=&v"(x) : "v"(a.x), "v"(a.y), "v"(a.z), "v"(a.w), "v"(b.x), "v"(b.y), "v"(b.z), "v"(b.w));
   return x;
 }
-// Do three parts hold them, and their products?  From 2^60 on a score's or an output's partial sums may leave the range (64 products of two values
+// Do three parts hold their products too?  From 2^60 on a score's or an output's partial sums may leave the range (64 products of two values
 // below it reach 2^126), and what cancels in a chain of whole products does not in the parts': infinities of either sign, a NaN
-// where the chain has a score of -inf.  Where the largest is below 2^-90, third parts fall out of the normal range.
-__device__ __forceinline__ bool splits(float largest) { return largest < 0x1p60f && !(largest > 0.f && largest < 8.1e-28f); }
+// where the chain has a score of -inf.
+__device__ __forceinline__ bool bounded(float largest) { return largest < 0x1p60f; }
+// At the other end a part that is a subnormal bf16 number (kept by conversion and product) ends at 2^-133: three hold every value from 2^-110 on.
+// Values of V: an output column may hold nothing larger, so the smallest of them counts, zeros apart.  Of queries and keys a score loses
+// 2^-134 2^60 a product, which the softmax scale does not bring back up to 2^30 (launch_64).
+constexpr float kSmallest = 0x1p-110f;
+__device__ __forceinline__ float smallest(const float4& a, const float4& b) {  // (zeros count, a NaN does not)
+  float x;
+  asm("v_min3_f32 %0, |%1|, |%2|, |%3|\n\tv_min3_f32 %0, %0, |%4|, |%5|\n\tv_min3_f32 %0, %0, |%6|, |%7|\n\tv_min_f32 %0, %0, |%8|"
+      : "=&v"(x) : "v"(a.x), "v"(a.y), "v"(a.z), "v"(a.w), "v"(b.x), "v"(b.y), "v"(b.z), "v"(b.w));
+  return x;
+}
+__device__ __forceinline__ bool too_small(float x) { return x != 0.f && fabsf(x) < kSmallest; }
 typedef float Any4 __attribute__((ext_vector_type(4), aligned(4)));
 struct Parts {
   u32x4 p[3];
@@ -420,7 +432,7 @@ __global__ __launch_bounds__(256, 4) void attn_f32_split_kernel(AttnParams p, in
     // (a row of q may begin at any value: 4-byte alignment)
     const float4 x = __builtin_bit_cast(float4, *reinterpret_cast<const Any4*>(qp + 16 * ks + 4 * g));
     const float4 y = __builtin_bit_cast(float4, *reinterpret_cast<const Any4*>(qp + 32 + 16 * ks + 4 * g));
-    plain = plain && splits(largest(x, y));
+    plain = plain && bounded(largest(x, y));
     const Parts q = split8(x, y);
 #pragma unroll
     for (int i = 0; i < 3; i++) bq[ks][i] = b16x::frag_of<bf16_t>(q.p[i]);
@@ -476,7 +488,11 @@ __global__ __launch_bounds__(256, 4) void attn_f32_split_kernel(AttnParams p, in
   for (int buf = 0; start >= 0; buf ^= 1) {
     const int nvalid = (int)(N - start < 32 ? N - start : 32);
     {
-      fits = fits && splits(largest(kr[0], kr[1])) && splits(largest(vr[0], vr[1]));
+      fits = fits && bounded(largest(kr[0], kr[1])) && bounded(largest(vr[0], vr[1]));
+      if (__any(!(smallest(vr[0], vr[1]) >= kSmallest))) {  // (zeros, mostly)
+#pragma unroll
+        for (int i = 0; i < 2; i++) fits = fits && !(too_small(vr[i].x) || too_small(vr[i].y) || too_small(vr[i].z) || too_small(vr[i].w));
+      }
       if (lane == 0) wide[buf][wave] = 0;
       if (!__all(fits) && lane == 0) wide[buf][wave] = 1;
       const Parts k3 = split8(kr[0], kr[1]), v3 = split8(vr[0], vr[1]);
@@ -620,7 +636,7 @@ template <int W, int KS, int BLK, bool SPLIT = false> static int launch_t(const 
 // 19.6, 500 (128) 21.4 / 26.7, 700 (176) 38.8 / 35.0, 1 041 (272) 62.9 / 61.3, 1 500 (384) 66.5 / 63.1, 1 900 (480) 84.8 / 63.8, 2 600 (656) 118 / 82.
 static int launch_64(const AttnParams& p, hipStream_t st) {
   const int64_t ngrp = (p.Lq + 63) / 64, total = ngrp * p.B * p.H;
-  if (total <= 384) return launch_t<4, 32, 64, true>(p, st);
+  if (total <= 384 || p.scale > 0x1p30f) return launch_t<4, 32, 64, true>(p, st);
   if (total > 0x7fffffffLL) return fail(S3R_ERR_UNSUPPORTED, "attention: grid too large");
   hipLaunchKernelGGL(attn_f32_split_kernel, dim3((unsigned)total), dim3(256), 0, st, p, (int)ngrp, (int)total);
   return check_launch("attn_f32_split_kernel");

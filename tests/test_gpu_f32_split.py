@@ -83,3 +83,29 @@ def test_scores_beyond_the_range(size, channels):
     want, lse_want, _ = _reference(q, k, v, idx, 0.125)
     o, lse = s3r.select_attn(q, k, v, idx, 64, 0.125, return_lse=True)
     assert bool((o.double().cpu() - want).norm() <= 4e-5 * want.norm()) and bool((lse.double().cpu() - lse_want).abs().max() <= 4e-5)
+
+
+# Equal scores, so that only the values' parts and sums count: 80 sums of four products (the fp32 instructions'; split values have fewer) and the quotient round
+# by 2^-24 of the sum of magnitudes.  Three bf16 parts of values of 1e-35 keep 18 bits, of 1e-36 14.
+@pytest.mark.parametrize("size", [1.0, 1e-31, 1e-33, 1e-34, 1e-35, 1e-36, 1e-37])
+def test_small_columns_beside_ordinary_ones(size):
+    q, k, v, idx = _inputs(256, 100, 7)
+    idx[..., 0] = 0
+    q.zero_()
+    v[..., [5, 40]] *= size
+    v[:, :, 3], v[..., 41] = 0.0, 0.0
+    want, _, _ = _reference(q, k, v, idx, 0.125)
+    mags, _, _ = _reference(q, k, v.abs(), idx, 0.125)
+    o = s3r.select_attn(q, k, v, idx, 64, 0.125).double().cpu()
+    assert bool(((o - want).abs() <= 84 * 2.0 ** -24 * mags).all())
+
+
+@pytest.mark.parametrize("heads", [128, 512])
+def test_scales_that_bring_small_scores_back(heads):
+    """Queries whose lowest bits three parts do not hold, keys as large, and the scale that makes a score of both (bound: of the 64-bit test)."""
+    q, k, v, idx = _inputs(heads, 64, 11)
+    q, k, scale = q * 2.0 ** -122, k * 2.0 ** 57, 2.0 ** 65
+    want, lse_want, bound = _reference(q, k, v, idx, scale)
+    o, lse = s3r.select_attn(q, k, v, idx, 64, scale, return_lse=True)
+    far = torch.isinf(lse_want)
+    assert bool(((o.double().cpu() - want).abs() <= bound).all()) and bool(((lse.double().cpu() - lse_want).abs()[~far] <= 2e-5).all())
