@@ -43,6 +43,7 @@ __global__ __launch_bounds__(256, WPS) void linear_kernel(LinearParams p) {
   typedef Tile<E, T, T> Tl;
   typedef typename Mma<E>::V2 V2;
   constexpr int BM = Tl::BM, BN = Tl::BN, kStage = 16 * 32 * T;  // kStage: 16 tokens x the wave's channels
+  constexpr int PC = 2 * T, RPI = 64 / PC, NS = 16 / RPI;        // 16-byte pieces per row, rows per store, stores per 16 tokens
   __shared__ __attribute__((aligned(1024))) unsigned char lx0[BM * 128];
   __shared__ __attribute__((aligned(1024))) unsigned char lx1[BM * 128];
   __shared__ __attribute__((aligned(1024))) unsigned char lw0[BN * 128];
@@ -92,13 +93,12 @@ __global__ __launch_bounds__(256, WPS) void linear_kernel(LinearParams p) {
     uint2 cb[T];  // this tile's bias (nb moves on to the next tile's)
 #pragma unroll
     for (int c = 0; c < T; c++) cb[c] = nb[c];
-    tl.template sweep<T * (16 * 2 * T / 64)>(lx0, lw0, lx1, lw1, p.K >> 6, fresh, kb, advance);
+    tl.template sweep<T * NS>(lx0, lw0, lx1, lw1, p.K >> 6, fresh, kb, advance);
     fresh = false;
     tl.after_products();
 
     // A lane holds 4 channels of a token in each tile; 16 tokens at a time go through LDS so that consecutive lanes store
     // consecutive 16-byte pieces of a row (64-byte runs of four lanes sixteen apart: 8 % of the whole kernel at K = 1024).
-    constexpr int PC = 2 * T, RPI = 64 / PC;  // 16-byte pieces per row, rows per store
     const int64_t r0 = (int64_t)m * BM;
     const uint32_t row_bytes = (uint32_t)(p.ldy * 2);
     const uint32_t bytes = (uint32_t)(p.M - r0 < BM ? p.M - r0 : BM) * row_bytes;
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256, WPS) void linear_kernel(LinearParams p) {
         *reinterpret_cast<uint2*>(buf + tl.c16 * (32 * T) + (((c * 2 + (tl.g4 >> 1)) ^ (tl.c16 & (PC - 1))) << 4) + (tl.g4 & 1) * 8) = o.u;
       }
 #pragma unroll
-      for (int i = 0; i < 16 / RPI; i++) {
+      for (int i = 0; i < NS; i++) {
         const int r = i * RPI + pr;
         const uint4 v = *reinterpret_cast<const uint4*>(buf + r * (32 * T) + ((pc ^ (r & (PC - 1))) << 4));
         store16_if((E*)p.y + r0 * p.ldy, bytes, yo + (uint32_t)(t * 16 + i * RPI) * row_bytes, v);

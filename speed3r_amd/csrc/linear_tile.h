@@ -28,7 +28,8 @@ __device__ __forceinline__ void to_lds16(const void* base, void* dst, uint32_t v
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
 }
 // 16 bytes to base + off unless that lies at or beyond `bytes`; non-temporal, so that what is written does not push the X and W
-// rows of the tiles to come out of the L2 (104 100 x 3072 x 1024: 546 -> 520 us; the projection with its epilogue 722 -> 697)
+// rows of the tiles to come out of the L2 (104 100 x 3072 x 1024: 546 -> 520 us; the projection with its epilogue 722 -> 697).  Issued, and
+// counted, whether anything is written or not: a tile's stores are counted on by the next one's first wait (sweep).
 __device__ __forceinline__ void store16_if(void* base, uint32_t bytes, uint32_t off, const uint4& v) {
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
   __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4*>(&v), rs, off, 0, 2);
@@ -157,8 +158,8 @@ template <typename E, int TT, int TC> struct Tile {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  // the buffer's last reads are in registers and the other buffer's transfers have landed, in every wave; LEFT: what the wave has
-  // requested or stored behind those transfers may still be under way
+  // the buffer's last reads are in registers and the other buffer's transfers have landed, in every wave, if the wave has issued LEFT or more
+  // requests and stores behind those transfers (with fewer the wait would pass while some of them are still under way)
   template <int LEFT = 0> __device__ __forceinline__ void turn() {
     static_assert(LEFT < 64, "what the counter holds");
     __builtin_amdgcn_s_waitcnt(0x0070 | (LEFT & 15) | ((LEFT >> 4) << 14));  // vmcnt(LEFT) lgkmcnt(0)
@@ -177,8 +178,9 @@ template <typename E, int TT, int TC> struct Tile {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  // A tile: its K / 64 steps (an even number), two at a time, `advance` in front of each of them.  STORES: of the tile before, at most; they
-  // were issued behind the transfers that the first step waits for (`fresh`: there is no such tile).
+  // A tile: its K / 64 steps (an even number), two at a time, `advance` in front of each of them.  STORES: every wave has issued at least so
+  // many for the tile before, behind the transfers that the first step waits for, so that these have landed when as many operations are left.
+  // None of them may depend on a branch; a wave that has issued fewer, or has no tile before, says `fresh` and waits for all.
   template <int STORES, typename P8, typename F> __device__ __forceinline__ void sweep(P8* x0, P8* w0, P8* x1, P8* w1, int steps, bool fresh, const int& kb, F&& advance) {
     start();
     advance();

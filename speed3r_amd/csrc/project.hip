@@ -75,7 +75,7 @@ template <typename E, int T, bool NORM, int POOL, int WPS>
 __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
   typedef Tile<E, T, T> Tl;
   typedef typename Mma<E>::V2 V2;
-  constexpr int BM = Tl::BM, BN = Tl::BN, HD = T / 4;  // HD: heads of a wave
+  constexpr int BM = Tl::BM, BN = Tl::BN, HD = T / 4, NS = 2;  // HD: heads of a wave, NS: stores per head and 16 tokens
   constexpr int WROWS = 16 * T;                        // its tokens
   constexpr int BLOCKS = POOL ? WROWS / (POOL ? POOL : 1) : 0, SETS = (BLOCKS + 3) / 4;
   __shared__ __attribute__((aligned(1024))) unsigned char lx0[BM * 128];
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
   tl.begin(lx0, lw0);
   bool fresh = true;
   for (;; par ^= 1) {
-    tl.template sweep<T * HD * 2>(lx0, lw0, lx1, lw1, p.K >> 6, fresh, kb, advance);
+    tl.template sweep<T * HD * NS>(lx0, lw0, lx1, lw1, p.K >> 6, fresh, kb, advance);
     tl.after_products();
 
     // ---- epilogue ----
@@ -254,10 +254,10 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
 #pragma unroll
           for (int i = 0; i < 4; i++) pv[s][i] = 0.f;
         u32x4 pr[2];
-        uint4 st[2];  // the group before, on its way out
+        uint4 st[NS];  // the group before, on its way out
         auto put = [&](int t) {
 #pragma unroll
-          for (int i = 0; i < 2; i++) {
+          for (int i = 0; i < NS; i++) {
             const int row = wr + t * 16 + i * 8 + (lane >> 3);
             store16_if(dst, 0x80000000u, row < rows ? row_offset(row) + (lane & 7) * 16 : 0x80000000u, st[i]);
           }
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(256, WPS) void project_kernel(ProjectParams p) {
           // a group is stored behind the work on the next one, when its rows have come back from LDS
           if (t > 0) put(t - 1);
 #pragma unroll
-          for (int i = 0; i < 2; i++) {
+          for (int i = 0; i < NS; i++) {
             const int r = i * 8 + (lane >> 3);
             st[i] = *reinterpret_cast<const uint4*>(mine + r * 128 + (((lane & 7) ^ row_swizzle(r)) << 4));
           }
