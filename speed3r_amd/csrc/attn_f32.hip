@@ -1,7 +1,7 @@
 // fp32 attention on the matrix cores (head_dim 64): the selection branch for blocks of 64, 32 and 16 tokens and the
 // compressed branch with its fp32 scores.
 //
-// Blocks of 64 go to attn_f32_split_kernel from 385 of them on (launch_64); what follows is about attn_f32_kernel.
+// Blocks of 64 go to attn_f32_split_kernel from 385 of them on, up to a softmax scale of 2^30 (launch_64); what follows is about attn_f32_kernel.
 //
 // Bound: the fp32 matrix instructions (v_mfma_f32_16x16x4_f32: 64 FLOP per cycle and SIMD, 157 TFLOP/s; a product of
 // 8192 x 8192 matrices by the library reaches 154).  At 8 328 tokens x 16 heads, 16 blocks of 64 (3.5e10 FLOP, 0.23 ms)
@@ -622,7 +622,7 @@ template <int W, int KS, int BLK, bool SPLIT = false> static int launch_t(const 
   const int64_t total = ngrp * p.B * p.H;
   // Blocks over a whole number per CU (256) make one CU in a few work a block longer than the others: where they are so
   // few that their halves still fit one to a CU, they go in halves.  16 heads, us without and with: 1 041 tokens (16
-  // blocks over) 77 / 62, 1 500 (128 over) 79 / 64, 4 164 (32) 177 / 163, 700 tokens (176 blocks in all) 36.6 / 37.0.
+  // blocks over) 77 / 62, 1 500 (128 over) 79 / 64; 700 tokens (176 blocks in all, whole) 36.6 / 37.0.
   const int64_t over = total & 255;
   const int64_t whole = SPLIT && over <= 128 ? total - over : total;
   const int64_t grid = whole + 2 * (total - whole);
@@ -631,8 +631,8 @@ template <int W, int KS, int BLK, bool SPLIT = false> static int launch_t(const 
   return check_launch("attn_f32_kernel");
 }
 
-// Blocks of 64.  Up to 384 of them the fp32 instructions, half blocks in the last round, are faster or within 10 %, and keep the score bits of a
-// chain of fp32 products; then they take a second whole round.  16 heads, us, fp32 instructions / split values: 333 tokens (96 blocks) 16.2 /
+// Blocks of 64.  Up to 128 of them the fp32 instructions are the faster ones; at 176 to 384, with half blocks in the last round, they are 3 to 11 %
+// slower, and stay for their scores' bits, those of a chain of fp32 products; then they take a second whole round.  16 heads, us, fp32 instructions / split values: 333 tokens (96 blocks) 16.2 /
 // 19.6, 500 (128) 21.4 / 26.7, 700 (176) 38.8 / 35.0, 1 041 (272) 62.9 / 61.3, 1 500 (384) 66.5 / 63.1, 1 900 (480) 84.8 / 63.8, 2 600 (656) 118 / 82.
 static int launch_64(const AttnParams& p, hipStream_t st) {
   const int64_t ngrp = (p.Lq + 63) / 64, total = ngrp * p.B * p.H;

@@ -47,6 +47,8 @@ def test_against_64_bits(heads, n, scale):
     for query in (q, odd):
         o, lse = s3r.select_attn(query, k, v, idx, 64, scale, return_lse=True)
         assert ((o.double().cpu() - want).abs() <= bound + 1e-30).all()
+        # as a whole: a score's sum rounds some 16 times by 2^-24 of its own size, 8 x scale, in either direction (two parts would give 3e-6 and more)
+        assert bool((o.double().cpu() - want).norm() <= 2.0 ** -24 * (4 + 16 ** 0.5 * 8 * scale) * want.norm())
         far = torch.isinf(lse_want)
         assert torch.equal(torch.isinf(lse).cpu(), far) and ((lse.double().cpu() - lse_want).abs()[~far] <= 2e-5).all()
 
@@ -109,3 +111,53 @@ def test_scales_that_bring_small_scores_back(heads):
     o, lse = s3r.select_attn(q, k, v, idx, 64, scale, return_lse=True)
     far = torch.isinf(lse_want)
     assert bool(((o.double().cpu() - want).abs() <= bound).all()) and bool(((lse.double().cpu() - lse_want).abs()[~far] <= 2e-5).all())
+
+
+def _whole_bound(score):
+    """Of output and log-sum-exp: 1e-5, and the rounding of a score by 2^-24 of it with each of 64 products (a large one may come first), with
+    the scale and in the exponent, twice for output and reference."""
+    return 1e-5 + 2 * 66 * score * 2.0 ** -24
+
+
+@pytest.mark.parametrize("step", [0.5, 3.0, 30.0])
+@pytest.mark.parametrize("n,h", [(400, 60), (250, 128)])
+def test_scores_that_rise_along_the_list(step, n, h):
+    """Every listed block's scores lie ``step`` natural units above the ones before it: below and above what the reference lets pass."""
+    gen, nb = torch.Generator().manual_seed(1), -(-n // 64)
+    q, k, v = (torch.randn((1, h, n, 64), generator=gen) for _ in range(3))
+    q[..., 0] = 8.0
+    k[..., 0] = (torch.arange(n) // 64) * step
+    idx = torch.arange(nb, dtype=torch.int32).expand(1, h, nb, nb).contiguous()
+    want, lse_want, _ = _reference(q, k, v, idx, 0.125)
+    o, lse = s3r.select_attn(*(t.to(DEV) for t in (q, k, v, idx)), 64, 0.125, return_lse=True)
+    for got, exact in ((o, want), (lse, lse_want)):
+        assert bool(((got.double().cpu() - exact).abs() <= _whole_bound((nb - 1) * step)).all())
+
+
+@pytest.mark.parametrize("dims", [slice(0, 1), slice(31, 32), slice(32, 33), slice(60, 61), slice(63, 64), slice(60, 64)])
+def test_scores_that_rise_in_some_dimensions(dims):
+    """The same, hundreds of units a block in dimensions that the first or the last products of a score add, along lists in any order: the
+    reference of the softmax is read from finished sums."""
+    gen, n, h = torch.Generator().manual_seed(2), 450, 57
+    q, k, v = (torch.randn((1, h, n, 64), generator=gen) for _ in range(3))
+    width = dims.stop - dims.start
+    q[..., dims] = 8.0
+    k[..., dims] = (torch.arange(n) // 64)[:, None] * (400.0 / width)
+    nb = -(-n // 64)
+    idx = torch.stack([torch.randperm(nb, generator=gen) for _ in range(h * nb)]).view(1, h, nb, nb).int().contiguous()
+    want, lse_want, _ = _reference(q, k, v, idx, 0.125)
+    o, lse = s3r.select_attn(*(t.to(DEV) for t in (q, k, v, idx)), 64, 0.125, return_lse=True)
+    for got, exact in ((o, want), (lse, lse_want)):
+        assert bool(((got.double().cpu() - exact).abs() <= _whole_bound((nb - 1) * 400)).all())
+
+
+def test_last_parts_of_values_count():
+    """Equal scores, and values of which neighbours leave 2^-18 of each other.  Some 32 roundings of 2^-24 of a value or two in either direction
+    against a sum of 64 such remainders: 0.7 %; values in two parts, off by up to 2^-18 themselves, would be off by most of it."""
+    q, k, v, idx = _inputs(256, 128, 9)
+    idx[...] = torch.tensor([0, 1, -1, -1, -1], device=DEV)
+    q.zero_()
+    v[:, :, 1::2] = -v[:, :, ::2] * (1 + 2.0 ** -18)
+    want, _, _ = _reference(q, k, v, idx, 0.125)
+    o = s3r.select_attn(q, k, v, idx, 64, 0.125).double().cpu()
+    assert bool((o - want).norm() <= 0.03 * want.norm())

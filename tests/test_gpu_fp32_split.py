@@ -1,4 +1,5 @@
-"""The fp32 selection kernel where the last query blocks are computed in halves, and its softmax reference, against the oracle."""
+"""The fp32 selection kernel where the last query blocks are computed in halves (up to 384 blocks in all), and its softmax reference, against
+the oracle."""
 import pytest
 import torch
 
@@ -18,7 +19,8 @@ def _check(q, k, v, idx, tol):
     assert torch.equal(torch.isfinite(lse.cpu()), fin) and max_abs(lse.cpu()[fin], lse_ref[fin]) <= tol
 
 
-# query blocks: 1, 128 (all in halves), 129 (none), 255, 256, 257, 384 (the last 128), 385 (none), 513; last key blocks of 5, 17 and 64 keys
+# query blocks: 1, 128 (all in halves), 129 (none), 255, 256, 257, 384 (the last 128); 385 and 513, which go to the kernel of split values; last
+# key blocks of 5, 17 and 64 keys
 @pytest.mark.parametrize("h,n,kk", [(1, 40, 1), (64, 69, 2), (43, 145, 3), (85, 133, 2), (64, 256, 4), (257, 17, 1), (128, 133, 3), (77, 261, 2),
                                     (57, 517, 6)])
 def test_blocks_in_halves_match_the_oracle(h, n, kk):
