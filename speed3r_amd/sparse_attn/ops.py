@@ -550,20 +550,6 @@ def linear_wgrad_pays(rows: int) -> bool:
     return rows >= 4096
 
 
-# A training step's product, us on the device, library / kernel (the host's share, which ``linear_pays`` counts, is behind the device's there).
-# 1024 inputs, 1 024 outputs: 8 192 rows 21.9 / 18.1, 9 760 24.0 / 25.8, 12 096 23.8 / 24.3, 20 160 39.1 / 41.3, 24 192 45.9 / 47.2, on another card
-# 45.7 / 49.5 and inside a step 50 / 55, 33 345 63.9 / 69.7, 41 008 95.3 / 79.6, 50 016 92.3 / 92.7, 80 000 150 / 130 (the other way round on another
-# card: 16 208 30.5 / 30.2, 32 224 58.6 / 56.6); 3 072 outputs: 8 104 49.8 / 44.1, 24 192 129 / 127, 33 345 213 / 172, 50 016 301 / 251; 4 096: 10 240
-# 95 / 78, 24 192 182 / 159; 2 048: 6 096 27.3 / 28.3, 12 192 51.5 / 47.8, 24 192 91 / 80; 512: 20 160 21.7 / 23.0, 39 056 45.9 / 43.3, 80 000
-# 90 / 75; the gate's 32: 24 192 21.7 / 15.1, 80 000 37.9 / 32.6.  896 inputs, 1 024 outputs: 9 760 22.3 / 23.6, 16 208 28.2 / 27.8; 768 and 768: 24 192
-# 46.8 / 31.5; 512 and 1 536: 16 000 39.2 / 25.2.
-def training_product_pays(rows: int, n: int, k: int) -> bool:
-    """Whether the kernel takes a product of a training step, ``rows`` of ``k`` inputs and ``n`` outputs."""
-    if 768 < k <= 1024 and 768 < n <= 1024 and 9e6 <= rows * n < 3.5e7:
-        return False
-    return linear_pays(rows, n, k)
-
-
 def linear_wgrad_takes(n: int, c: int) -> bool:
     """Whether the kernel is built for ``n`` outputs and ``c`` inputs."""
     return n % 8 == 0 and c % 8 == 0 and 0 < n <= 1 << 20 and 0 < c <= 1 << 20
@@ -575,8 +561,10 @@ class _LinearFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
         ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, weight if ctx.needs_input_grad[0] else None)
+        # The product itself, us on the device, library / kernel: 1024 inputs, 3 072 outputs, 8 104 rows 52.9 / 47.2, 24 192 129.5 / 128.1, 33 345 219 /
+        # 175, 50 016 309 / 253; 1 024 outputs 18.9 / 16.6, 45.7 / 49.5, 66.2 / 70.7, 93.1 / 94.3; the gate's 32 18.5 / 8.6 (the host's share), 21.6 / 15.0.
         out = None
-        if ordinary(x) and x.numel() != 0 and weight.dim() == 2 and training_product_pays(x.numel() // x.shape[-1], *weight.shape):
+        if ordinary(x) and x.numel() != 0 and weight.dim() == 2 and linear_pays(x.numel() // x.shape[-1], *weight.shape):
             out = linear(x, weight, bias)
         if out is None:
             out = torch.nn.functional.linear(x, weight, bias)
