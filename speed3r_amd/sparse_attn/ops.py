@@ -561,8 +561,11 @@ class _LinearFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
         ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, weight if ctx.needs_input_grad[0] else None)
-        # The product itself, us on the device, library / kernel: 1024 inputs, 3 072 outputs, 8 104 rows 52.9 / 47.2, 24 192 129.5 / 128.1, 33 345 219 /
-        # 175, 50 016 309 / 253; 1 024 outputs 18.9 / 16.6, 45.7 / 49.5, 66.2 / 70.7, 93.1 / 94.3; the gate's 32 18.5 / 8.6 (the host's share), 21.6 / 15.0.
+        # The product alone, us on the device, library / kernel: 1024 inputs, 3 072 outputs, 8 104 rows 49.8 / 44.1, 24 192 129 / 127, 33 345 213 / 172, 50 016
+        # 301 / 251; 4 096: 8 104 54 / 57, 10 240 95 / 78, 24 192 182 / 159; 2 048: 6 096 27.3 / 28.3, 12 192 51.5 / 47.8, 24 192 91 / 80; 1 024: 8 192 21.9 /
+        # 18.1, 9 760 24.0 / 25.8, 24 192 45.9 / 47.2, 33 345 63.9 / 69.7, 41 008 95.3 / 79.6, 80 000 150 / 130; the gate's 32: 24 192 21.7 / 15.1.  Where the
+        # library is the faster one alone, a whole step is not with it: a layer's output projection of 16 128 to 33 312 rows by the library / here, 24 192 rows
+        # under autocast 1 645 / 1 647, 16 128 without 1 121 / 1 115, 22 settings 0.02 % apart on average.
         out = None
         if ordinary(x) and x.numel() != 0 and weight.dim() == 2 and linear_pays(x.numel() // x.shape[-1], *weight.shape):
             out = linear(x, weight, bias)

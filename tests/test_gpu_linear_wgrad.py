@@ -210,3 +210,24 @@ def test_small_steps_keep_the_products_of_torch(rows, c, autocast, kernel, monke
     with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
         m(torch.randn(rows, c, device=DEV, dtype=m.fc1.weight.dtype)).float().sum().backward()
     assert len(calls) == (2 if kernel else 0) and all(p.grad is not None for p in m.parameters())
+
+
+# one tile and less, ragged last tiles, both tile sizes; more inputs than the kernel is faster for, outputs, inputs, a type and a row stride that it does not
+# take
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,k,dtype,kernel", [(1, 8, 128, torch.bfloat16, True), (4099, 136, 1024, torch.bfloat16, True), (8104, 3072, 1024, torch.float16, True),
+                                                   (8104, 1024, 1024, torch.bfloat16, True), (4099, 1024, 2048, torch.bfloat16, False), (300, 60, 1024, torch.bfloat16, False), (300, 64, 200, torch.bfloat16, False),
+                                                   (300, 64, 256, torch.float32, False)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_forward_of_the_function(rows, n, k, dtype, kernel, bias, monkeypatch):
+    own, calls = ops.linear, []
+    monkeypatch.setattr(ops, "linear", lambda *a: (calls.append(own(*a)), calls[-1])[1])
+    x, w, b = (torch.randn(s, device=DEV).to(dtype).requires_grad_() for s in ((rows, k), (n, k), (n,)))
+    got = ops._LinearFn.apply(x, w, b if bias else None)
+    assert (len(calls) == 1 and calls[0] is not None) == kernel and got.requires_grad
+    want = x.double() @ w.double().t() + (b.double() if bias else 0)
+    # half a step of the type, and an fp32 rounding for each of the products' sums
+    mag = x.double().abs() @ w.double().abs().t() + b.double().abs()
+    assert bool(((got.double() - want).abs() <= torch.finfo(dtype).eps / 2 * want.abs() + (k + 2) * 2.0 ** -24 * mag).all())
+    strided = torch.randn(rows, 2, k, device=DEV, dtype=dtype)[:, 0]
+    assert torch.equal(ops._LinearFn.apply(strided, w, None), F.linear(strided, w)) or rows == 1
